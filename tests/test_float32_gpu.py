@@ -1,0 +1,101 @@
+"""The float32 engine's kernels on the matrix instructions and for single tokens, against 64-bit arithmetic, at the edges of
+their tiles. Bounds: a sum of n float32 products in any order is off by at most n 2^-24 times the sum of their magnitudes
+(first order; 2 covers the rest)."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _gen(seed):
+    return torch.Generator(device=DEV).manual_seed(seed)
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 5, 4), (1, 1000, 1028), (2, 64, 260), (3, 1024, 4096), (4, 20000, 512), (8, 100, 2052),
+                                   (16, 20000, 260), (17, 48, 32), (64, 64, 64), (65, 100, 96), (101, 2048, 2048),
+                                   (129, 50, 512), (180, 1024, 4096), (401, 2048, 1024), (513, 4100, 320), (40, 7, 1056)])
+def test_float32_product(m, n, k):
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g = HipOps(torch.float32, DEV), _gen(m + n + k)
+    x = torch.randn(m, k, device=DEV, generator=g)
+    w = torch.randn(n, k, device=DEV, generator=g)
+    bias, res = torch.randn(n, device=DEV, generator=g), torch.randn(m, n, device=DEV, generator=g)
+    exact = x.double() @ w.double().T
+    bound = 2 * (k + 2) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T + bias.abs() + res.abs())
+    for b, r, act in ((None, None, None), (bias, None, "relu"), (bias, res, None)):
+        got = hip.linear(x, w, b, act=act, residual=r, out_f32=True).double()
+        want = exact + (b.double() if b is not None else 0)
+        want = want.relu() if act else want
+        want = want + (r.double() if r is not None else 0)
+        assert bool(((got - want).abs() <= bound).all())
+    # a row that is not finite is its own alone
+    x[m // 2, k // 2] = float("inf")
+    got = hip.linear(x, w, out_f32=True)
+    assert not bool(torch.isfinite(got[m // 2]).any())
+    rest = torch.arange(m, device=DEV) != m // 2
+    assert bool(torch.isfinite(got[rest]).all())
+
+
+def _step(runs, cached, page, seed):
+    from transformers_neuronx_amd.engine.batch import StepEntry, build_context
+    from transformers_neuronx_amd.kernels.attention_plan import attention_plan
+    width = max(-(-(c + r) // page) for c, r in zip(cached, runs))
+    order = torch.randperm(len(runs) * width, generator=torch.Generator().manual_seed(seed)).view(len(runs), width)
+    table = order.to(torch.int32).numpy()
+    entries = [StepEntry(i, [0] * r, [r - 1]) for i, r in enumerate(runs)]
+    return build_context(entries, list(cached), list(range(len(runs))), {"full": table}, page, DEV,
+                         {"attention": attention_plan}), len(runs) * width
+
+
+@pytest.mark.parametrize("heads,kv,hs", [(4, 4, 64), (8, 2, 80), (2, 1, 128), (3, 3, 16), (4, 2, 48)])
+@pytest.mark.parametrize("page", [16, 48, 64])
+@pytest.mark.parametrize("window", [None, 37])
+def test_float32_attention(heads, kv, hs, page, window):
+    """Portions of prompts behind a cache, single tokens, whole short prompts, in one step; what lies behind a request's last
+    token in its pages is not a number."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g = HipOps(torch.float32, DEV), _gen(heads * hs + page)
+    runs, cached = [70, 1, 33, 1, 2, 1, 129], [45, 0, 0, 700, 31, 64, 0]
+    ctx, pages = _step(runs, cached, page, seed=hs)
+    view = ctx.groups["full"]
+    kp = torch.full((pages, kv, page, hs), float("nan"), device=DEV)
+    vp = torch.full((pages, kv, hs, page), float("nan"), device=DEV)
+    q = torch.randn(sum(runs), heads * hs, device=DEV, generator=g) * hs ** -0.5
+    want, bound, at = torch.empty(sum(runs), heads, hs, dtype=torch.float64, device=DEV), None, 0
+    for r, (n, c) in enumerate(zip(runs, cached)):
+        total = c + n
+        keys = torch.randn(kv, total, hs, device=DEV, generator=g)
+        vals = torch.randn(kv, total, hs, device=DEV, generator=g)
+        for b in range(-(-total // page)):
+            p, rows = int(view.block_table[r, b]), slice(b * page, min(total, (b + 1) * page))
+            kp[p, :, :rows.stop - rows.start] = keys[:, rows]
+            vp[p, :, :, :rows.stop - rows.start] = vals[:, rows].transpose(1, 2)
+        qr = q[at:at + n].double().view(n, heads, hs).transpose(0, 1)
+        s = qr @ keys.double().repeat_interleave(heads // kv, 0).transpose(1, 2)
+        i, j = torch.arange(c, total, device=DEV)[:, None], torch.arange(total, device=DEV)[None]
+        hidden = (j > i) | ((i - j >= window) if window else (j > i))
+        want[at:at + n] = (torch.softmax(s.masked_fill(hidden, float("-inf")), -1)
+                           @ vals.double().repeat_interleave(heads // kv, 0)).transpose(0, 1)
+        at += n
+    got = hip.attention(q, heads, kv, hs, ctx, view, kp, vp, window)
+    # weights of scores up to 8 or so: off by their scores' error (hs + 2 roundings of at most 8) and their sums' (760 keys)
+    torch.testing.assert_close(got.double(), want.reshape(sum(runs), -1), rtol=0, atol=5 * (8 * hs + 760) * 2.0 ** -24)
+
+
+def test_float32_attention_keeps_a_value_that_is_no_number_to_its_readers():
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g = HipOps(torch.float32, DEV), _gen(3)
+    heads, hs, page, n = 2, 64, 64, 50
+    ctx, pages = _step([n], [0], page, seed=1)
+    kp = torch.randn(pages, heads, page, hs, device=DEV, generator=g)
+    vp = torch.randn(pages, heads, hs, page, device=DEV, generator=g)
+    q = torch.randn(n, heads * hs, device=DEV, generator=g) * 0.1
+    clean = hip.attention(q, heads, heads, hs, ctx, ctx.groups["full"], kp, vp)
+    vp[int(ctx.groups["full"].block_table[0, 0]), 1, 5, 21] = float("inf")
+    got = hip.attention(q, heads, heads, hs, ctx, ctx.groups["full"], kp, vp).view(n, heads, hs)
+    clean = clean.view(n, heads, hs).clone()
+    assert bool(torch.isinf(got[21:, 1, 5]).all())
+    got[21:, 1, 5] = clean[21:, 1, 5] = 0
+    torch.testing.assert_close(got, clean, rtol=1e-5, atol=1e-5)

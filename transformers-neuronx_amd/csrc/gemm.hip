@@ -1,5 +1,6 @@
 // Matrix products `out[M, N] = act(x[M, K] w[N, K]^T + bias[N]) + residual[M, N]` with float32 accumulation.
-//   gemm_f32        float32 operands, plain FMA (no matrix-core mode of reduced precision)
+//   gemm_f32        float32 operands, on the float32 matrix instructions (nothing is rounded to fewer bits), on plain
+//                   FMA for few rows and for sizes that are no multiples of 32 in K
 //   gemm_bf16       bfloat16 operands on MFMA, many rows (prompts): 256x256x64 tiles, operands straight from
 //                   global memory into two LDS stages, four waves of 128x128 (sizes in whole 64-steps of K);
 //                   128x128 tiles staged through registers for every other size
@@ -126,14 +127,19 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const 
 // Few rows in float32 (decoding): the product is the weight read once. A wave makes 4 columns of the output
 // for up to MR rows of `x`; its lanes share K four floats at a time, so a row of the weight is read in runs
 // of 1 KB, and the 64 partial sums of every output meet in a butterfly at the end. K is a multiple of 4.
-template <int MR>
+// SPLIT: the block's four waves make the same 4 columns and take steps of 256 of K in turn, their sums meet in LDS; where
+// the columns are few, four times the blocks read the weight and a wave's chain of waits is a quarter as long. UNROLL steps
+// are asked for together: what bounds a narrow matrix is how often a wave waits for memory, not the bytes. Measured at 3
+// rows, a wave for every 4 columns against four: 1,024 columns of K 4,096 13.8 us against 7.7, 4,096 of 1,024 9.8 against 8.3.
+template <int MR, bool SPLIT, int UNROLL>
 __global__ void __launch_bounds__(256)
 gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                        const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
                        int N, int K) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int n0 = (blockIdx.x * 4 + wave) * 4;
-  if (n0 >= N) return;
+  __shared__ float sums[SPLIT ? 4 : 1][4 * MR];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n0 = (SPLIT ? blockIdx.x : blockIdx.x * 4 + wave) * 4;
+  if (n0 >= N) return;                 // (SPLIT: the whole block)
   const float* wrow[4];
 #pragma unroll
   for (int c = 0; c < 4; ++c) wrow[c] = w + (size_t)min(n0 + c, N - 1) * K;
@@ -146,27 +152,32 @@ gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
 #pragma unroll
     for (int m = 0; m < MR; ++m) acc[c][m] = 0.f;
   const int k_last = K - 4;
-  for (int k0 = 0; k0 < K; k0 += 256) {
-    // lanes beyond K read the last four floats again and add nothing
-    const int k = min(k0 + 4 * lane, k_last);
-    const float keep = k0 + 4 * lane < K ? 1.f : 0.f;
-    f32x4 wv[4], xv[MR];
+  constexpr int STRIDE = SPLIT ? 1024 : 256;
+  for (int k0 = SPLIT ? 256 * wave : 0; k0 < K; k0 += STRIDE * UNROLL) {
+    f32x4 wv[UNROLL][4], xv[UNROLL][MR];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) wv[c] = *(const f32x4*)(wrow[c] + k);
+    for (int u = 0; u < UNROLL; ++u) {
+      // lanes beyond K read the last four floats again and add nothing
+      const int k = min(k0 + u * STRIDE + 4 * lane, k_last);
 #pragma unroll
-    for (int m = 0; m < MR; ++m) xv[m] = *(const f32x4*)(xrow[m] + k);
+      for (int c = 0; c < 4; ++c) wv[u][c] = *(const f32x4*)(wrow[c] + k);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-      const f32x4 wk = wv[c] * keep;
+      for (int m = 0; m < MR; ++m) xv[u][m] = *(const f32x4*)(xrow[m] + k);
+    }
 #pragma unroll
-      for (int m = 0; m < MR; ++m) {
-        float a = acc[c][m];
-        a = fmaf(wk[0], xv[m][0], a);
-        a = fmaf(wk[1], xv[m][1], a);
-        a = fmaf(wk[2], xv[m][2], a);
-        a = fmaf(wk[3], xv[m][3], a);
-        acc[c][m] = a;
-      }
+    for (int u = 0; u < UNROLL; ++u) {
+      if (k0 + u * STRIDE + 4 * lane >= K) continue;
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+          float a = acc[c][m];
+          a = fmaf(wv[u][c][0], xv[u][m][0], a);
+          a = fmaf(wv[u][c][1], xv[u][m][1], a);
+          a = fmaf(wv[u][c][2], xv[u][m][2], a);
+          a = fmaf(wv[u][c][3], xv[u][m][3], a);
+          acc[c][m] = a;
+        }
     }
   }
 #pragma unroll
@@ -175,25 +186,234 @@ gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
     for (int m = 0; m < MR; ++m) {
       const float a = wave_sum(acc[c][m]);
       // every lane has the sum; lane c * MR + m (modulo the wave) writes it
-      if (lane == ((c * MR + m) & 63) && n0 + c < N && m < M)
-        epilogue_store(a, m, n0 + c, N, bias, residual, out, out_dtype, act);
+      if (lane == ((c * MR + m) & 63)) {
+        if (SPLIT) sums[wave][c * MR + m] = a;
+        else if (n0 + c < N && m < M) epilogue_store(a, m, n0 + c, N, bias, residual, out, out_dtype, act);
+      }
     }
+  if (SPLIT) {
+    __syncthreads();
+    for (int i = threadIdx.x; i < 4 * MR; i += 256) {
+      const int c = i / MR, m = i % MR;
+      if (n0 + c < N && m < M)
+        epilogue_store((sums[0][i] + sums[1][i]) + (sums[2][i] + sums[3][i]), m, n0 + c, N, bias, residual, out, out_dtype, act);
+    }
+  }
 }
 
+template <int MR>
+static void launch_f32_skinny(const float* x, const float* w, const float* bias, const float* residual, void* out,
+                              int out_dtype, int act, int M, int N, int K, hipStream_t stream) {
+  // Steps asked for together: as many as the rows leave registers for.
+  constexpr int MOST = MR <= 4 ? 4 : MR <= 8 ? 2 : 1;
+  // A wave for every 4 columns gives N / 16 blocks; below four blocks a compute unit the waves of a block share K instead.
+  if ((N + 15) / 16 < 4 * tnx_compute_units()) {
+    const dim3 grid((N + 3) / 4);
+    if (K > 1024 && MOST > 1)
+      gemm_f32_skinny_kernel<MR, true, MOST><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+    else
+      gemm_f32_skinny_kernel<MR, true, 1><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+  } else {
+    gemm_f32_skinny_kernel<MR, false, (MOST > 2 ? 2 : MOST)><<<dim3((N + 15) / 16), 256, 0, stream>>>(x, w, bias, residual,
+                                                                                          out, out_dtype, act, M, N, K);
+  }
+}
+
+// Many rows in float32, on the float32 matrix instructions (32x32x2: products and sums in float32, no operand is
+// rounded): tiles of 64 MI rows of `x` by 64 NI of `w`, four waves (2 x 2) of 32 MI x 32 NI each. What bounds the product is
+// these instructions' rate (256 flops a cycle and unit: 157 TFLOP/s), 16 times below bfloat16's, so a plain pipeline feeds
+// them: tiles of 32 floats of K go straight into LDS, NSTAGE deep, 16-byte chunks swizzled by row; a lane reads four floats
+// of K of its row at once, which serve four instructions (which two places of K an instruction joins is free, as long as
+// both operands agree: here k and k + 4). The share of K that a block takes (gridDim.y of them) keeps the units busy where
+// the result has few tiles; its sums then go to `partial` and are added by `gemm_mid_sum_kernel`.
+// Measured at 401 rows, us (TFLOP/s), with these tiles and with the tiles of 64 x 64 on plain FMA that served such sizes
+// before: 8,192 columns of K 2,048: 159 (85) against 446; 6,144 of 2,048: 142 (71) against 372; 2,048 of 2,048 and of 8,192:
+// 52 (65) and 144 (93, with the sum of four shares) against 561 on average. Its error against 64 bits is the smaller one.
+template <int MI, int NI, int NSTAGE>
+__global__ void __launch_bounds__(256)
+gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+                      const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act,
+                      float* __restrict__ partial, int M, int N, int K, int tiles_m, int steps_per_share) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int TM = 64 * MI, TN = 64 * NI, STAGE = (TM + TN) * 128;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int l32 = lane & 31, half = lane >> 5;
+  const int wm = (wave & 1) * 32 * MI, wn = (wave >> 1) * 32 * NI;
+  // blocks of one XCD (every eighth) take neighbouring tiles, those of the same columns of `w` first
+  const int nb = gridDim.x, xcd = blockIdx.x & 7, each = nb >> 3, more_of = nb & 7;
+  const int bid = xcd * each + min(xcd, more_of) + (blockIdx.x >> 3);
+  const int m0 = bid % tiles_m * TM, n0 = bid / tiles_m * TN;
+  const int first = blockIdx.y * steps_per_share, steps = min(K / 32 - first, steps_per_share);
+
+  const int lrow = lane >> 3, lpos = lane & 7;
+  const float* xsrc[2 * MI];
+  const float* wsrc[2 * NI];
+#pragma unroll
+  for (int j = 0; j < 2 * MI; ++j) {
+    const int row = (2 * MI * wave + j) * 8 + lrow;
+    xsrc[j] = x + (size_t)min(m0 + row, M - 1) * K + 32 * first + 4 * (lpos ^ ((row >> 1) & 7));
+  }
+#pragma unroll
+  for (int j = 0; j < 2 * NI; ++j) {
+    const int row = (2 * NI * wave + j) * 8 + lrow;
+    wsrc[j] = w + (size_t)min(n0 + row, N - 1) * K + 32 * first + 4 * (lpos ^ ((row >> 1) & 7));
+  }
+  auto issue = [&](int t) {
+    char* a_dst = smem + (t % NSTAGE) * STAGE + 2 * MI * wave * 1024;
+    char* b_dst = smem + (t % NSTAGE) * STAGE + TM * 128 + 2 * NI * wave * 1024;
+#pragma unroll
+    for (int j = 0; j < 2 * MI; ++j) load_to_lds(xsrc[j] + 32 * t, lds_offset(a_dst + j * 1024));
+#pragma unroll
+    for (int j = 0; j < 2 * NI; ++j) load_to_lds(wsrc[j] + 32 * t, lds_offset(b_dst + j * 1024));
+  };
+  f32x16 acc[MI][NI];
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+#pragma unroll
+  for (int p = 0; p < NSTAGE - 1; ++p)
+    if (p < steps) issue(p);
+  const int swizzle = (l32 >> 1) & 7;
+  for (int t = 0; t < steps; ++t) {
+    // tile t has landed when at most the loads of the NSTAGE - 2 tiles behind it are still in flight
+    constexpr int L = 2 * MI + 2 * NI;
+    const int ahead = min(NSTAGE - 2, steps - 1 - t);
+    if (NSTAGE > 3 && ahead == 2) __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * L) & 15) | (((2 * L) >> 4) << 14));
+    else if (NSTAGE > 2 && ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | (L & 15) | ((L >> 4) << 14));
+    else __builtin_amdgcn_s_waitcnt(0x0F70);
+    __syncthreads();
+    if (t + NSTAGE - 1 < steps) issue(t + NSTAGE - 1);
+    const char* base = smem + (t % NSTAGE) * STAGE;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+      const int chunk = ((2 * s + half) ^ swizzle) * 16;
+      f32x4 a[MI], b[NI];
+#pragma unroll
+      for (int i = 0; i < MI; ++i) a[i] = *(const f32x4*)(base + (wm + 32 * i + l32) * 128 + chunk);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) b[j] = *(const f32x4*)(base + TM * 128 + (wn + 32 * j + l32) * 128 + chunk);
+#pragma unroll
+      for (int c = 0; c < 4; ++c)
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+          for (int j = 0; j < NI; ++j)
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][c], a[i][c], acc[i][j], 0, 0, 0);
+    }
+  }
+  // element e of a lane: row lane % 32, column 8 (e / 4) + 4 (lane / 32) + e % 4 of the 32 x 32
+#pragma unroll
+  for (int i = 0; i < MI; ++i) {
+    const int m = m0 + wm + 32 * i + l32;
+    if (m >= M) continue;
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = n0 + wn + 32 * j + 8 * g + 4 * half;
+        if (partial) {
+          // (N is a multiple of 4 here: four columns are inside or outside together)
+          if (n < N)
+            *(f32x4*)(partial + ((size_t)blockIdx.y * M + m) * N + n) =
+                (f32x4){acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (n + e < N) epilogue_store(acc[i][j][4 * g + e], m, n + e, N, bias, residual, out, out_dtype, act);
+        }
+      }
+  }
+}
+
+__global__ void gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__ bias,
+                                    const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
+                                    int N, int shares);
+
+template <int MI, int NI, int NSTAGE>
+static int launch_f32_tiles(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
+                            int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
+  constexpr int bytes = NSTAGE * (64 * MI + 64 * NI) * 128;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_tiles_kernel<MI, NI, NSTAGE>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "gemm_f32: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  const int tiles_m = (M + 64 * MI - 1) / (64 * MI), tiles_n = (N + 64 * NI - 1) / (64 * NI);
+  const int per = (K / 32 + shares - 1) / shares;
+  shares = (K / 32 + per - 1) / per;
+  gemm_f32_tiles_kernel<MI, NI, NSTAGE><<<dim3(tiles_m * tiles_n, shares), 256, bytes, stream>>>(
+      x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, M, N, K, tiles_m, per);
+  TNX_CHECK_LAUNCH("gemm_f32_tiles");
+  if (shares > 1) {
+    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
+                                                                                        act, M, N, shares);
+    TNX_CHECK_LAUNCH("gemm_mid_sum");
+  }
+  return 0;
+}
+
+// The most floats that the shares' sums of one product may take (32 MB).
+constexpr long long F32_SHARES_MOST = 8 << 20;
+
+// The tile and the shares of K: what the fullest compute unit has to do, in steps of 32 of K of a 64 x 64 tile (0.43 us at
+// the instructions' rate), a step in which a block fills and empties its pipeline, and the sum of the shares.
+static void choose_f32_tiles(int M, int N, int K, int& tile, int& shares) {
+  const int units = tnx_compute_units(), steps = K / 32;
+  const int sizes[3][2] = {{1, 1}, {2, 1}, {2, 2}};
+  const double cost_of_step[3] = {1.0, 1.9, 3.6};
+  double best = 1e30;
+  for (int i = 0; i < 3; ++i) {
+    const long long tiles = (long long)((M + 64 * sizes[i][0] - 1) / (64 * sizes[i][0])) * ((N + 64 * sizes[i][1] - 1) / (64 * sizes[i][1]));
+    for (int s = 1; s <= 8 && (s == 1 || (N % 4 == 0 && steps / s >= 4 && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
+      const int per = (steps + s - 1) / s;
+      const long long rounds = (tiles * s + units - 1) / units;
+      double cost = (double)rounds * (per * cost_of_step[i] + 3.0);
+      if (s > 1) cost += 8.0 + (double)M * N * (s + 1) * 4e-6 / 4.0 / 0.43;
+      if (cost < best) best = cost, tile = i, shares = s;
+    }
+  }
+}
+
+// How many floats of workspace `tnx_gemm_f32` wants for a product: those of the shares' sums, 0 where K is not shared out.
+extern "C" int tnx_gemm_f32_workspace(int M, int N, int K) {
+  if (M <= 16 || N <= 0 || K < 32 || K % 32 != 0) return 0;
+  int tile = 0, shares = 1;
+  choose_f32_tiles(M, N, K, tile, shares);
+  return shares > 1 ? shares * M * N : 0;
+}
+
+// `workspace`: as many floats as `tnx_gemm_f32_workspace` names for the sizes; with less, K is not shared out.
 extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, const float* residual, void* out,
-                            int out_dtype, int act, int M, int N, int K, hipStream_t stream) {
+                            int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
+                            hipStream_t stream) {
   TNX_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   if (M <= 16 && K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0) {
-    const dim3 grid((N + 15) / 16);
-    if (M <= 4)
-      gemm_f32_skinny_kernel<4><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+    if (M <= 1)
+      launch_f32_skinny<1>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
+    else if (M <= 2)
+      launch_f32_skinny<2>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
+    else if (M <= 4)
+      launch_f32_skinny<4>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
     else if (M <= 8)
-      gemm_f32_skinny_kernel<8><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+      launch_f32_skinny<8>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
     else
-      gemm_f32_skinny_kernel<16><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+      launch_f32_skinny<16>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
     TNX_CHECK_LAUNCH("gemm_f32_skinny");
     return 0;
+  }
+  if (K % 32 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) % 16 == 0) {
+    int tile = 0, shares = 1;
+    choose_f32_tiles(M, N, K, tile, shares);
+    if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
+#define F32_TILES(MI, NI, ST) launch_f32_tiles<MI, NI, ST>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
+    return tile == 0 ? F32_TILES(1, 1, 4) : tile == 1 ? F32_TILES(2, 1, 3) : F32_TILES(2, 2, 2);
+#undef F32_TILES
   }
   dim3 grid((N + F32_TILE - 1) / F32_TILE, (M + F32_TILE - 1) / F32_TILE);
   TNX_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d is too large", M);

@@ -38,7 +38,8 @@ _SIGNATURES = {
     },
     "gemm": {
         "tnx_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
-                         _c_int, _c_void_p],
+                         _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
+        "tnx_gemm_f32_workspace": [_c_int, _c_int, _c_int],
         "tnx_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gemm_bf16_qkv": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p,
@@ -76,6 +77,11 @@ _SIGNATURES = {
         "tnx_attention_decode_static": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int,
                                         _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                                         _c_int, _c_int, _c_void_p, _c_void_p],
+    },
+    "attention_f32": {
+        "tnx_attention_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
+                              _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int,
+                              _c_int, _c_int, _c_void_p],
     },
     "sampling": {
         "tnx_ban_tokens": [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p],
@@ -705,8 +711,10 @@ class HipOps:
             return out
         if w.dtype == torch.float32:
             xa = self.cast(x, torch.float32)
+            room = library("gemm").tnx_gemm_f32_workspace(m, n, k)
+            space = torch.empty(room, dtype=torch.float32, device=x.device) if room else None
             self._call("gemm", "tnx_gemm_f32", _ptr(xa), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out),
-                       _code(out_dtype), _ACT[act], m, n, k, _stream(),
+                       _code(out_dtype), _ACT[act], m, n, k, _ptr(space), room, _stream(),
                        work=self._product_work(m, n, k, 4, 4, out.element_size(), residual is not None))
         else:
             xa = self.cast(x, torch.bfloat16)
@@ -961,6 +969,14 @@ class HipOps:
             build._log(f"a page size of {view.page_size} is no power of two: steps with decoding requests run on the "
                        "general attention kernel (one wave a query), several times slower than the matrix-unit "
                        "kernels that pages of 16, 32, 64, ... tokens get")
+        if (self.dtype == torch.float32 and not self.force_plain_attention and head_size <= 128 and "tile_run" in ctx.plan
+                and _ptr(q) % 16 == 0):
+            tiles, singles = ctx.plan["tile_run"], ctx.plan["decode_runs"]
+            self._call("attention_f32", "tnx_attention_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.run_start),
+                       _ptr(ctx.cached_lens), _ptr(view.block_table), view.width, view.page_size, num_pages, _ptr(tiles),
+                       _ptr(ctx.plan["tile_start"]), tiles.numel(), QUERY_TILE, _ptr(singles), singles.numel(), _ptr(out),
+                       num_heads, num_kv_heads, head_size, window, pad, _stream())
+            return out
         if not fast:
             self._call("attention", "tnx_attention_any", _ptr(q), _code(self.dtype), _ptr(k_pages), _ptr(v_pages),
                        _ptr(ctx.positions), _ptr(ctx.token_request), _ptr(view.block_table), view.width,
