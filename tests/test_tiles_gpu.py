@@ -1,0 +1,64 @@
+"""Products by tiles of 64 and 128 rows against 64-bit arithmetic: the experts' over many pairs each, at the edges of tiles."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+
+
+def _apart(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+def _act(name, g, u, limit):
+    if name == "silu":
+        return torch.nn.functional.silu(g) * u
+    if name == "gelu_new":
+        return torch.nn.functional.gelu(g, approximate="tanh") * u
+    if name == "clamped_swiglu":
+        g, u = g.clamp(max=limit), u.clamp(-limit, limit)
+        return g * torch.sigmoid(1.702 * g) * (u + 1)
+    return {"relu": torch.relu, "relu2": lambda x: torch.relu(x) ** 2}[name](g)
+
+
+@pytest.mark.parametrize("counts", [[64, 0, 65, 127], [1, 128, 129, 300], [200, 31, 0, 1], [700, 513, 5, 64]])
+@pytest.mark.parametrize("width,f", [(64, 64), (192, 320), (256, 128)])
+@pytest.mark.parametrize("act,on,identity", [("silu", "input", 0), ("gelu_new", "output", 0), ("clamped_swiglu", "output", 2),
+                                             ("relu2", "output", 0), ("relu", "output", 1)])
+@pytest.mark.parametrize("rows", [64, 128])
+def test_experts_by_tiles(counts, width, f, act, on, identity, rows):
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops = HipOps(torch.bfloat16, DEV)
+    ops.expert_grouped_rows = 1
+    ops.expert_wide_tiles = 1 if rows == 128 else 1 << 30
+    g = torch.Generator(device=DEV).manual_seed(sum(counts) + width)
+    experts, gated = len(counts), act not in ("relu", "relu2")
+    flat = torch.repeat_interleave(torch.arange(experts, device=DEV), torch.tensor(counts, device=DEV))
+    flat = flat[torch.randperm(flat.numel(), device=DEV, generator=g)]
+    tokens = -(-flat.numel() // 2)
+    # the places left over: experts without tensors where there are some, else the first again
+    fill = torch.full((2 * tokens - flat.numel(),), experts if identity else 0, device=DEV)
+    chosen = torch.cat([flat, fill]).view(tokens, 2)
+    if identity:
+        chosen[::7, 1] = experts + identity - 1
+    weights = torch.rand(tokens, 2, device=DEV, generator=g) + 0.1
+    h = torch.randn(tokens, width, device=DEV, generator=g).bfloat16()
+    up = (torch.randn(experts, (2 if gated else 1) * f, width, device=DEV, generator=g) * width ** -0.5).bfloat16()
+    down = (torch.randn(experts, width, f, device=DEV, generator=g) * f ** -0.5).bfloat16()
+    residual = torch.randn(tokens, width, device=DEV, generator=g)
+    want = torch.zeros(tokens, width, dtype=torch.float64, device=DEV)
+    for c in range(2):
+        for e in range(experts):
+            at = (chosen[:, c] == e).nonzero().flatten()
+            x, s = h[at].double(), weights[at, c].double()[:, None]
+            z = (x * s if on == "input" else x) @ up[e].double().T
+            y = _act(act, z[:, :f], z[:, f:], 1.5) @ down[e].double().T
+            want[at] += y if on == "input" else s * y
+        same = chosen[:, c] >= experts
+        want[same] += weights[same, c].double()[:, None] * h[same].double()
+    for r in (residual, None):
+        got = ops.expert_mixture(h, chosen.int().contiguous(), weights, up, down, act, on, r,
+                                 limit=1.5 if act == "clamped_swiglu" else None, identity=identity)
+        # the inner values are rounded to bfloat16 (by 2^-8 of themselves at most), everything else is summed in float32
+        assert _apart(got - (r if r is not None else 0), want) < 2.0 ** -8

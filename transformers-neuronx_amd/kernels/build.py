@@ -1,7 +1,7 @@
 """Compiling the HIP sources and finding what is compiled.
 
 Each source under `csrc/` becomes one shared library named after the hash of
-its text (and of the shared header and the flags), so a library never outlives
+its text (and of the shared headers and the flags), so a library never outlives
 the source it was built from. A library is compiled when it is first needed and
 kept beside the sources; if that folder cannot be written, under the user's
 cache folder or the temporary folder. While hipcc runs a line is printed every
@@ -9,6 +9,7 @@ few seconds.
 """
 import hashlib
 import os
+import re
 import shutil
 import subprocess
 import sys
@@ -61,7 +62,10 @@ def source_hash(module: str) -> str:
     h = hashlib.sha256()
     src = _SOURCES[module]
     own_header = os.path.join(os.path.dirname(src), f"tnx_{module}.h")   # its entry points: not every module has one
-    for path in (src, os.path.join(CSRC, "common.h"), own_header):
+    with open(src) as fp:
+        shared = [os.path.join(CSRC, name) for name in re.findall(r'#include "(\w+\.h)"', fp.read())]
+    others = [p for p in shared if os.path.basename(p) not in ("common.h", os.path.basename(own_header)) and os.path.exists(p)]
+    for path in (src, os.path.join(CSRC, "common.h"), own_header, *others):
         if path == own_header and not os.path.exists(path):
             continue
         with open(path, "rb") as fp:

@@ -149,6 +149,9 @@ _SIGNATURES = {
         "tnx_expert_mixture": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p],
+        "tnx_expert_grouped": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                               _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_int, _c_int,
+                               _c_int, _c_void_p],
         "tnx_row_activation": [_c_void_p, _c_ll, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_ll, _c_void_p],
         "tnx_gated_activation": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_float, _c_void_p],
         "tnx_expert_order": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
@@ -1911,10 +1914,17 @@ class HipOps:
                    gate_ld, _stream(), work=(f"{t}x{f}", t * f * (4.0 + out.element_size()), 0.0))
         return out
 
-    # A step of this many (token, choice) pairs an expert or more, bfloat16, that is not being recorded: the host
-    # reads where each expert's pairs begin (one small copy that waits for the device) and every expert's two
-    # products go to the vendor library over its own rows, as the many-rows products of the other parts do. Below
-    # that, and in recorded steps, one launch of ours takes all experts and the host reads nothing. 0: never.
+    # From `expert_grouped_rows` (token, choice) pairs an expert on, bfloat16, sizes in 64s: the experts' products by tiles
+    # (two launches over all experts, the host reads nothing), of 128 pairs from `expert_wide_tiles` an expert on. Measured
+    # for 8 experts, two a token, us a layer, one launch of 16 pairs a tile or the library / tiles of 64 / of 128: 2,048 wide,
+    # 12 pairs an expert 57 / 65 / 69, 16: 73 / 66 / 71, 50: 132 / 73 / 77, 99: 520 / 95 / 91, 512: 504 / 207 / 213; 4,096 wide,
+    # 12: 155 / 216 / 212, 16: 216 / 214 / 221, 50: 463 / 221 / 219, 99: 492 / 272 / 232, 512: 804 / 681 / 632.
+    expert_grouped_rows = 16           # 0: never
+    expert_wide_tiles = 64
+    # Other sizes, from this many pairs an expert on, in a step that is not being recorded: the host reads where each
+    # expert's pairs begin (one small copy that waits for the device) and every expert's two products go to the vendor
+    # library over its own rows. Below that, and in recorded steps, one launch of ours with tiles of 16 pairs takes all
+    # experts and the host reads nothing. 0: never.
     expert_library_rows = 96
     expert_row_step = 128
     expert_plain_products = False      # tests set it: the kernel without the matrix unit in bfloat16 too
@@ -1940,6 +1950,20 @@ class HipOps:
         dev = h.device
         pairs = t * top
         out = torch.empty(t, width, dtype=torch.float32, device=dev)
+        if (self.expert_grouped_rows > 0 and self.expert_library_rows > 0 and pairs >= self.expert_grouped_rows * experts
+                and not self.expert_plain_products and h.dtype == torch.bfloat16 and width % 64 == 0 and f % 64 == 0
+                and (_ptr(h) | _ptr(w_gate_up) | _ptr(w_down)) % 16 == 0 and (residual is None or _ptr(residual) % 16 == 0)):
+            rows = 128 if pairs >= self.expert_wide_tiles * experts else 64
+            ints = torch.empty(experts + 2 + 2 * pairs + 2 * (pairs // rows + experts), dtype=torch.int32, device=dev)
+            inner = torch.empty(pairs, f, dtype=h.dtype, device=dev)
+            y = torch.empty(pairs, width, dtype=torch.float32, device=dev)
+            self._call("experts", "tnx_expert_grouped", _ptr(h), _ptr(chosen), _ptr(weights), _ptr(w_gate_up), _ptr(w_down),
+                       _ptr(ints), _ptr(inner), _ptr(y), _ptr(residual), _ptr(out), t, experts, top, width, f,
+                       (_ACT if ungated else _GATE_ACT)[activation], int(weight_on == "input"), float(limit or 0.0), int(identity),
+                       int(ungated), rows, _stream(),
+                       work=(f"{t}x{top} of {experts}", experts * (2.0 if ungated else 3.0) * f * width * 2 + t * width * 10.0,
+                             (4.0 if ungated else 6.0) * pairs * f * width))
+            return out
         if (may_wait and self.expert_library_rows > 0 and pairs >= self.expert_library_rows * experts
                 and self.dtype == torch.bfloat16 and h.dtype == torch.bfloat16 and width % 8 == 0 and f % 8 == 0
                 and self.library_direct and not debug.tapping()):
