@@ -324,7 +324,8 @@ def _ptr(t: Optional[torch.Tensor]):
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    """The current stream of the current device, by its address (a `torch.cuda.Stream` made to ask it takes 4 us)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _want(t: torch.Tensor, name: str, dtype=None, shape=None):
@@ -357,13 +358,17 @@ class HipOps:
         self._ints, self._ints_done, self._ints_turn = [None, None], [None, None], 0
 
     def _call(self, module: str, fn: str, *args, work=None):
-        """`work` = (what, bytes, flops) names the launch for a kernel timer: what it is (its sizes), what it has
-        to read and write once, and its multiply-adds times two."""
+        """`work() -> (what, bytes, flops)` names the launch for a kernel timer: what it is (its sizes), what it has
+        to read and write once, and its multiply-adds times two (asked for only where a timer runs)."""
         lib = library(module)
         timer = debug.timer()
         end = None
         if timer is not None:
-            end = timer.start(fn, 0, 0) if work is None else timer.start(f"{fn} {work[0]}", work[1], work[2])
+            if work is None:
+                end = timer.start(fn, 0, 0)
+            else:
+                what, nbytes, flops = work()
+                end = timer.start(f"{fn} {what}", nbytes, flops)
         rc = getattr(lib, fn)(*args)
         if end is not None:
             end.record()
@@ -524,7 +529,7 @@ class HipOps:
         out_cd = torch.empty(t, width, dtype=dtype, device=x.device) if (want_compute and not same) else None
         self._call("elementwise", "tnx_layernorm", _ptr(x), _ptr(weight), _ptr(bias), float(eps), _ptr(out_f32),
                    _ptr(out_cd), _code(dtype), t, width, int(bool(center)), _stream(),
-                   work=(f"{t}x{width}", t * width * (4 + (4 if out_f32 is not None else 0) + (2 if out_cd is not None else 0)), 0.0))
+                   work=lambda: (f"{t}x{width}", t * width * (4 + (4 if out_f32 is not None else 0) + (2 if out_cd is not None else 0)), 0.0))
         return (out_f32 if want_f32 else None), ((out_f32 if same else out_cd) if want_compute else None)
 
     # Steps of few rows: a LayerNorm that only a matrix product reads is done by that product (`fold_norm`,
@@ -640,7 +645,7 @@ class HipOps:
                 rows, shift = x.normalised(), folded.d_with(bias)     # held until the launch is made
                 self._call("gemm", "tnx_gemm_bf16", _ptr(rows), _ptr(w.tensor), _ptr(folded.tiles), _ptr(shift), None,
                            _ptr(out), _code(self.dtype), _ACT[act], m, n, k, int(force_tiled), _stream(),
-                           work=self._product_work(m, n, k))
+                           work=lambda: self._product_work(m, n, k))
                 return out
             else:
                 if act not in _ACT:
@@ -652,7 +657,7 @@ class HipOps:
                 out = torch.empty(m, n, dtype=self.dtype, device=x.x.device)
                 self._call("gemm", "tnx_gemm_bf16_normed", _ptr(x.x), _ptr(folded.tiles), _ptr(folded.c),
                            _ptr(folded.d), float(x.eps), _ptr(bias), _ptr(out), _code(self.dtype), _ACT[act], m, n, k,
-                           int(force_tiled), int(bool(x.center)), _stream(), work=self._product_work(m, n, k, x_item=4))
+                           int(force_tiled), int(bool(x.center)), _stream(), work=lambda: self._product_work(m, n, k, x_item=4))
                 return out
         tiles = None
         if isinstance(w, PreparedWeight):
@@ -678,7 +683,7 @@ class HipOps:
             space = self._library_workspace(x.device)
             self._call("gemm", "tnx_gemm_bf16_mid", _ptr(self.cast(x, torch.bfloat16)), _ptr(tiles), _ptr(bias),
                        _ptr(residual), _ptr(out), _code(out_dtype), _ACT[act], m, n, k, _ptr(space), space.numel() // 4,
-                       0, 0, _stream(), work=self._product_work(m, n, k, out_item=4, residual=residual is not None))
+                       0, 0, _stream(), work=lambda: self._product_work(m, n, k, out_item=4, residual=residual is not None))
             return out
         if (self._library_product(m, n, k, w, force_tiled) and (residual is not None or not out_f32)):
             # Many rows: the product goes to the vendor library (hipBLASLt), with what follows it where the
@@ -718,12 +723,12 @@ class HipOps:
             space = torch.empty(room, dtype=torch.float32, device=x.device) if room else None
             self._call("gemm", "tnx_gemm_f32", _ptr(xa), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out),
                        _code(out_dtype), _ACT[act], m, n, k, _ptr(space), room, _stream(),
-                       work=self._product_work(m, n, k, 4, 4, out.element_size(), residual is not None))
+                       work=lambda: self._product_work(m, n, k, 4, 4, out.element_size(), residual is not None))
         else:
             xa = self.cast(x, torch.bfloat16)
             self._call("gemm", "tnx_gemm_bf16", _ptr(xa), _ptr(w), _ptr(tiles), _ptr(bias), _ptr(residual),
                        _ptr(out), _code(out_dtype), _ACT[act], m, n, k, int(force_tiled), _stream(),
-                       work=self._product_work(m, n, k, out_item=out.element_size(), residual=residual is not None))
+                       work=lambda: self._product_work(m, n, k, out_item=out.element_size(), residual=residual is not None))
         return out
 
     library_direct = True   # many-rows products as calls of the vendor library itself, with what follows them
@@ -892,7 +897,7 @@ class HipOps:
                            view.page_size, num_pages, int(force_tiled), _ptr(turn_a), _ptr(turn_b), _ptr(turn_pos),
                            turn_rows, self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size,
                                                      view.page_size), int(bool(h.center)), _stream(),
-                           work=self._product_work(t, total, h.x.shape[1], x_item=4))
+                           work=lambda: self._product_work(t, total, h.x.shape[1], x_item=4))
                 return q
         tiles = None
         if isinstance(w, PreparedWeight):
@@ -927,7 +932,7 @@ class HipOps:
                    num_heads, num_kv_write, head_size, view.page_size, num_pages, int(force_tiled), _ptr(turn_a),
                    _ptr(turn_b), _ptr(turn_pos), turn_rows,
                    self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size, view.page_size), _stream(),
-                   work=self._product_work(t, total, h.shape[1]))
+                   work=lambda: self._product_work(t, total, h.shape[1]))
         return q
 
     def qkv_write(self, qkv, bias, num_heads, num_kv_write, head_size, scale, ctx, view, k_pages, v_pages, turn=None):
@@ -992,8 +997,7 @@ class HipOps:
                        view.page_size, num_pages, _ptr(ctx.plan["tile_run"]), _ptr(ctx.plan["tile_start"]), ctx.plan["tile_run"].numel(),
                        _ptr(out), num_heads, num_kv_heads, head_size, window,
                        int(self.prefill_direct) or self._prefill_sets(ctx, num_heads, window), QUERY_TILE, pad,
-                       _stream(), work=self._attention_work(ctx, "prompt", num_heads, num_kv_heads, head_size, window, 2)
-                       if debug.timer() is not None else None)
+                       _stream(), work=lambda: self._attention_work(ctx, "prompt", num_heads, num_kv_heads, head_size, window, 2))
         n_dec = ctx.plan["decode_runs"].numel()
         if n_dec:
             splits, waves = self._decode_splits(ctx, n_dec * self._decode_blocks(num_heads, num_kv_heads, head_size),
@@ -1007,8 +1011,7 @@ class HipOps:
                        view.page_size, num_pages, _ptr(ctx.plan["decode_runs"]), n_dec, _ptr(out), _ptr(part_o),
                        _ptr(part_ml), num_heads, num_kv_heads, head_size, window, splits, waves,
                        _ptr(ctx.plan["longest_decode"]), pad,
-                       _stream(), work=self._attention_work(ctx, "decode", num_heads, num_kv_heads, head_size, window, 2)
-                       if debug.timer() is not None else None)
+                       _stream(), work=lambda: self._attention_work(ctx, "decode", num_heads, num_kv_heads, head_size, window, 2))
         return out
 
     # What the choice between one and two sets of waves a block rests on: the time of one 64-key step of a
@@ -1130,7 +1133,7 @@ class HipOps:
                    kept_tokens.numel() if kept_tokens is not None else 0, _ptr(table), _ptr(pairs), _code(table.dtype),
                    table.shape[0], buckets, mul_prev, mul_cur, _ptr(ctx.positions), _ptr(ctx.token_request),
                    _ptr(ctx.run_start), _ptr(ctx.slots), _ptr(last_token), _ptr(out), t, table.shape[1],
-                   ctx.num_requests, _stream(), work=(f"{t}x{table.shape[1]}", t * table.shape[1] * (4 + 2 * table.element_size()), 0.0))
+                   ctx.num_requests, _stream(), work=lambda: (f"{t}x{table.shape[1]}", t * table.shape[1] * (4 + 2 * table.element_size()), 0.0))
         return out
 
     def norm_add(self, y, weight, bias, eps, center, residual, mult=1.0, out=None, want_compute=False):
@@ -1152,7 +1155,7 @@ class HipOps:
             copy = torch.empty(t, width, dtype=self.dtype, device=y.device)
         self._call("stream", "tnx_norm_add", _ptr(y), _ptr(weight), _ptr(bias), float(eps), int(bool(center)),
                    _ptr(residual), float(mult), _ptr(out), _ptr(copy), _code(self.dtype), t, width, _stream(),
-                   work=(f"{t}x{width}", t * width * (12 + (2 if copy is not None else 0)), 0.0))
+                   work=lambda: (f"{t}x{width}", t * width * (12 + (2 if copy is not None else 0)), 0.0))
         if not want_compute:
             return out
         return out, (copy if copy is not None else self.cast(out, self.dtype))
@@ -1177,7 +1180,7 @@ class HipOps:
         self._call("stream", "tnx_join_norm", _ptr(x), float(alpha), _ptr(ya), _ptr(wa), float(fa), _ptr(yb), _ptr(wb),
                    float(fb), part_eps.pop() if part_eps else 1.0, _ptr(weight), float(eps), _ptr(out), _ptr(copy), _code(dtype),
                    t, width, _stream(),
-                   work=(f"{t}x{width}x{len(results)}", t * width * (8.0 + 4.0 * len(results) + (2 if copy is not None else 0)), 0.0))
+                   work=lambda: (f"{t}x{width}x{len(results)}", t * width * (8.0 + 4.0 * len(results) + (2 if copy is not None else 0)), 0.0))
         return out, (copy if copy is not None else out)
 
     fuse_rows = 64       # up to this many rows the join, the norm and the convolution are one launch
@@ -1224,7 +1227,7 @@ class HipOps:
                    _ptr(x_out), _ptr(pw), _ptr(pb), int(bool(pc)), float(eps), _ptr(conv_w), mine, stride, taps,
                    _ptr(ctx.positions), _ptr(ctx.token_request), _ptr(ctx.run_start), _ptr(ctx.slots), _ptr(out),
                    _code(dtype), _ptr(keep), int(single), t, width, ctx.num_requests, _stream(),
-                   work=(f"{t}x{width}{' joined' if join is not None else ''}",
+                   work=lambda: (f"{t}x{width}{' joined' if join is not None else ''}",
                          t * width * (4 + out.element_size() + (8 if join is not None else 0)), 0.0))
         return (x_out if join is not None else x), out
 
@@ -1253,7 +1256,7 @@ class HipOps:
         out = torch.empty(t, width, dtype=dtype, device=h.device)
         self._call("stream", "tnx_input_conv", _ptr(h), _ptr(weight), mine, stride, taps, _ptr(ctx.positions),
                    _ptr(ctx.token_request), _ptr(ctx.run_start), _ptr(ctx.slots), _ptr(out), _code(dtype), t, width, ctx.num_requests, _stream(),
-                   work=(f"{t}x{width}", t * width * (4 + out.element_size()), 0.0))
+                   work=lambda: (f"{t}x{width}", t * width * (4 + out.element_size()), 0.0))
         return out
 
     def poly_norm(self, z, coeffs, eps):
@@ -1262,7 +1265,7 @@ class HipOps:
         _want(coeffs, "coefficients", torch.float32, (4,))
         out = torch.empty(z.shape, dtype=self.dtype, device=z.device)
         self._call("stream", "tnx_poly_norm", _ptr(z), _ptr(coeffs), float(eps), _ptr(out), _code(self.dtype),
-                   z.shape[0], z.shape[1], _stream(), work=(f"{z.shape[0]}x{z.shape[1]}", z.numel() * (4 + out.element_size()), 0.0))
+                   z.shape[0], z.shape[1], _stream(), work=lambda: (f"{z.shape[0]}x{z.shape[1]}", z.numel() * (4 + out.element_size()), 0.0))
         return out
 
     def mul_columns(self, g, rows, offset):
@@ -1282,7 +1285,7 @@ class HipOps:
             raise ValueError(f"weighted_sum of {count} slots: {history.shape[0]} are there, {weights.numel()} weights")
         out = torch.empty_like(history[0])
         self._call("stream", "tnx_weighted_sum", _ptr(history), _ptr(weights), count, history.stride(0), _ptr(out),
-                   out.numel(), _stream(), work=(f"{count}x{out.numel()}", (count + 1) * out.numel() * 4, 0.0))
+                   out.numel(), _stream(), work=lambda: (f"{count}x{out.numel()}", (count + 1) * out.numel() * 4, 0.0))
         return out
 
     def _latent_pages(self, latent_pages, rotated_pages, kv_rank, rot, page_size, across_pages=None):
@@ -1328,7 +1331,7 @@ class HipOps:
                    rotated_pages.stride(0) if kv_rank else 0, num_pages, view.page_size,
                    _ptr(across_pages) if kv_rank and across_pages is not None else None,
                    across_pages.stride(0) if kv_rank and across_pages is not None else 0, t, _stream(),
-                   work=(f"{t}x{q_rank}+{kv_rank}+{rot}", t * ((q_rank + kv_rank + rot) * 4 + (q_rank + 2 * kv_rank + rot) * 2), 0.0))
+                   work=lambda: (f"{t}x{q_rank}+{kv_rank}+{rot}", t * ((q_rank + kv_rank + rot) * 4 + (q_rank + 2 * kv_rank + rot) * 2), 0.0))
         return c_q
 
     batched_library_rows = 64      # from this many rows on a bfloat16 product per head goes to the vendor library (0: never)
@@ -1355,7 +1358,7 @@ class HipOps:
         out = torch.empty(t, heads, n, dtype=torch.float32 if out_f32 else self.dtype, device=x.device)
         self._call("latent", "tnx_batched_linear", _ptr(x), _code(x.dtype), x.stride(0), x.stride(1), _ptr(w),
                    _code(w.dtype), _ptr(out), _code(out.dtype), float(alpha), t, heads, n, k, _stream(),
-                   work=(f"{t}x{heads}x{n}x{k}", heads * n * k * w.element_size() + t * heads * (k + n) * 2,
+                   work=lambda: (f"{t}x{heads}x{n}x{k}", heads * n * k * w.element_size() + t * heads * (k + n) * 2,
                          2.0 * t * heads * n * k))
         return out
 
@@ -1400,7 +1403,7 @@ class HipOps:
         self._call("latent", "tnx_latent_gather", _ptr(latent_pages), _ptr(rotated_pages), latent_pages.stride(0),
                    rotated_pages.stride(0), view.page_size, num_pages, _ptr(view.block_table), view.width,
                    _ptr(row_run_d), _ptr(row_pos_d), _ptr(c_dense), _ptr(r_dense), kv_rank, rot, rows, _stream(),
-                   work=(f"{rows}x{kv_rank}+{rot}", rows * (kv_rank + rot) * 4, 0.0))
+                   work=lambda: (f"{rows}x{kv_rank}+{rot}", rows * (kv_rank + rot) * 4, 0.0))
         k_n = self.linear(c_dense, w_uk, None)                                   # [rows, H * n]
         uv = w_uv.tensor if isinstance(w_uv, PreparedWeight) else w_uv
         v_t = self.linear(uv, c_dense, None)                                     # [H * v, rows]: tokens side by side
@@ -1412,7 +1415,7 @@ class HipOps:
                    _ptr(ctx.plan["tile_start"]), tiles, QUERY_TILE, rows, _ptr(freqs), freqs.numel(), float(scale),
                    num_heads, head_size, rot, value_size, int(window or 0), *self._sink_and_gate(sink, gate, t, num_heads),
                    _stream(),
-                   work=(f"{tiles} tiles", rows * num_heads * (head_size + value_size) * 2.0,
+                   work=lambda: (f"{tiles} tiles", rows * num_heads * (head_size + value_size) * 2.0,
                          2.0 * num_heads * (head_size + rot + value_size) * float((lens * seen).sum())))
         return out
 
@@ -1470,7 +1473,7 @@ class HipOps:
                        _ptr(across_pages), latent_pages.stride(0), rotated_pages.stride(0), across_pages.stride(0),
                        _ptr(freqs), freqs.numel(), float(scale), num_heads, head_size, rot, kv_rank, int(window or 0),
                        _ptr(part), splits, per_split, int(self.latent_prompt_kind), *finish, _stream(),
-                       work=(f"{tiles} tiles {decodes} decodes", seen * (2 * kv_rank + rot) * 2,
+                       work=lambda: (f"{tiles} tiles {decodes} decodes", seen * (2 * kv_rank + rot) * 2,
                              2.0 * num_heads * (2 * kv_rank + rot) * float(
                                  (ctx.run_lens_host * np.minimum(ctx.cached_lens_host + (ctx.run_lens_host + 1) / 2,
                                                                  window or 1 << 30)).sum()))
@@ -1523,7 +1526,7 @@ class HipOps:
                    value_size, cache_head, int(bool(per_head)), -1 if values_at is None else int(values_at),
                    _ptr(head_scale), float(temperature[0]) if temperature else 0.0, int(temperature[1]) if temperature else 0,
                    _stream(),
-                   work=(f"{t}x{need}", t * (need * 4 + (num_heads + 2 * num_kv) * cache_head * q.element_size()), 0.0))
+                   work=lambda: (f"{t}x{need}", t * (need * 4 + (num_heads + 2 * num_kv) * cache_head * q.element_size()), 0.0))
         return q
 
     # ---------------------------------------------------------------- several copies of the stream
@@ -1538,7 +1541,7 @@ class HipOps:
         cd = torch.empty(t, width, dtype=dtype, device=src.device) if want_compute and dtype != torch.float32 else None
         self._call("hyper", "tnx_add_sinusoid", _ptr(src), _code(src.dtype), _ptr(positions), _ptr(freqs), _ptr(out),
                    _ptr(cd), _code(dtype), t, width, float(scale), _stream(),
-                   work=(f"{t}x{width}", t * width * (4 + src.element_size()), 0.0))
+                   work=lambda: (f"{t}x{width}", t * width * (4 + src.element_size()), 0.0))
         return out, ((cd if cd is not None else out) if want_compute else None)
 
     def _hyper(self, copies, pending, read, norm_weight, eps, h32, hcd, total):
@@ -1556,7 +1559,7 @@ class HipOps:
         moved = s * t * width * 4.0 * (2 if pending is not None else 1) + (t * width * 4.0 if pending is not None else 0)
         self._call("hyper", "tnx_hyper_step", _ptr(copies), _ptr(y), _ptr(mix), _ptr(out_w), _ptr(read), _ptr(norm_weight),
                    float(eps), _ptr(h32), _ptr(hcd), _code(hcd.dtype) if hcd is not None else 0, _ptr(total), s, t, width,
-                   _stream(), work=(f"{s}x{t}x{width}", moved + t * width * 4.0, 0.0))
+                   _stream(), work=lambda: (f"{s}x{t}x{width}", moved + t * width * 4.0, 0.0))
 
     def hyper_step(self, copies, pending, read, norm_weight, eps, dtype, want_f32, want_compute):
         """See `ReferenceOps.hyper_step`."""
@@ -1609,8 +1612,9 @@ class HipOps:
                 raise ValueError(f"the bias by distance is [heads, distances], got {tuple(distance_bias.shape)}")
             far = distance_bias.shape[1] - 1
         pad = self._page_pad(k_pages, num_kv_heads, head_size, view.page_size)
-        work = (self._scored_work(ctx, num_heads, num_kv_heads, head_size, window, chunk, q.element_size())
-                if debug.timer() is not None else None)
+        def work():
+            return self._scored_work(ctx, num_heads, num_kv_heads, head_size, window, chunk, q.element_size())
+
         if self.dtype == torch.bfloat16 and not self.force_plain_attention and "tile_run" in ctx.plan:
             # on the matrix unit: the runs of several tokens by tiles of queries (through LDS where the pages are a
             # power of two of keys), the runs of one token by key/value head
@@ -1689,7 +1693,7 @@ class HipOps:
         out_ld = self._rows_apart(out, "the result", self.dtype, t, inner)
         self._call("recurrent", "tnx_min_gru", _ptr(proj), 3 * inner, inner, _ptr(ctx.positions), _ptr(ctx.run_start),
                    _ptr(ctx.slots), _ptr(carried), _ptr(out), out_ld, _code(self.dtype), float(out_scale), t,
-                   ctx.num_requests, _stream(), work=(f"{t}x{inner}", t * inner * (12.0 + out.element_size()), 0.0))
+                   ctx.num_requests, _stream(), work=lambda: (f"{t}x{inner}", t * inner * (12.0 + out.element_size()), 0.0))
         return out
 
     def channel_conv(self, x, weight, bias, ctx, state):
@@ -1706,7 +1710,7 @@ class HipOps:
         self._call("recurrent", "tnx_channel_conv", _ptr(x), ld, _ptr(self._taps_first(weight)), _ptr(bias),
                    _ptr(state) if taps > 1 else None, taps, _ptr(ctx.positions), _ptr(ctx.token_request),
                    _ptr(ctx.run_start), _ptr(ctx.slots), _ptr(out), _ptr(cd), _code(self.dtype), t, channels,
-                   ctx.num_requests, _stream(), work=(f"{t}x{channels}", t * channels * 10.0, 0.0))
+                   ctx.num_requests, _stream(), work=lambda: (f"{t}x{channels}", t * channels * 10.0, 0.0))
         return out, (cd if cd is not None else out)
 
     def gated_linear_recurrence(self, gates, gate_bias, u, y, rate, ctx, carried, out=None, out_scale=1.0):
@@ -1728,7 +1732,7 @@ class HipOps:
         self._call("recurrent", "tnx_gated_linear_recurrence", _ptr(gates), _ptr(gate_bias), _ptr(u), _ptr(y), y_ld,
                    _ptr(rate), _ptr(ctx.positions), _ptr(ctx.run_start), _ptr(ctx.slots), _ptr(carried), _ptr(out), out_ld,
                    _code(self.dtype), float(out_scale), t, ctx.num_requests, blocks, w, _stream(),
-                   work=(f"{t}x{channels}", t * channels * (16.0 + out.element_size()), 0.0))
+                   work=lambda: (f"{t}x{channels}", t * channels * (16.0 + out.element_size()), 0.0))
         return out
 
     # ---------------------------------------------------------------- the matrix memory
@@ -1753,7 +1757,7 @@ class HipOps:
         self._call("memory", "tnx_matrix_memory", _ptr(proj), total, _ptr(ctx.run_start), _ptr(ctx.cached_lens),
                    _ptr(ctx.slots), _ptr(memory), _ptr(normalizer), _ptr(peak), slots, _ptr(raw), _ptr(gates), _ptr(norm_weight),
                    float(eps), _ptr(out), _code(self.dtype), t, ctx.num_requests, h, n, v, float(gate_cap), _stream(),
-                   work=(f"{t} tokens {ctx.num_requests} runs", state + t * total * 4.0, 4.0 * t * h * n * v))
+                   work=lambda: (f"{t} tokens {ctx.num_requests} runs", state + t * total * 4.0, 4.0 * t * h * n * v))
         return out
 
     # ---------------------------------------------------------------- linear memories
@@ -1782,7 +1786,7 @@ class HipOps:
                    _ptr(ctx.token_request), _ptr(ctx.run_start), _ptr(ctx.slots), int(size), int(count), int(scaled),
                    float(scale), _ptr(u), channels + 64, heads, int(dt_at), -1 if write_at is None else int(write_at), _ptr(rate),
                    _ptr(dt_bias), _ptr(gates[0]), _ptr(gates[1]), t, ctx.num_requests, _stream(),
-                   work=(f"{t}x{channels}", t * channels * 8.0 + ctx.num_requests * (taps - 1) * channels * 8.0, 0.0))
+                   work=lambda: (f"{t}x{channels}", t * channels * 8.0 + ctx.num_requests * (taps - 1) * channels * 8.0, 0.0))
         return u, gates[0], gates[1]
 
     def channel_decays(self, low, weight, bias, tau):
@@ -1795,7 +1799,7 @@ class HipOps:
         out = torch.empty(t, channels, dtype=torch.float32, device=low.device)
         self._call("linear_memory", "tnx_channel_decays", _ptr(low), low_ld, _ptr(weight), _code(weight.dtype), _ptr(bias),
                    1.0 / float(tau), _ptr(out), t, channels, rank, _stream(),
-                   work=(f"{t}x{channels}", t * channels * 4.0 + channels * rank * weight.element_size(), 2.0 * t * channels * rank))
+                   work=lambda: (f"{t}x{channels}", t * channels * 4.0 + channels * rank * weight.element_size(), 2.0 * t * channels * rank))
         return out
 
     def turn_heads(self, x, at, heads, n, freqs, interleaved, ctx):
@@ -1806,7 +1810,7 @@ class HipOps:
         ld = self._rows_apart(x, "projections", torch.float32, x.shape[0], x.shape[1])
         self._call("linear_memory", "tnx_turn_heads", _ptr(x), ld, int(at), int(heads), int(n), _ptr(freqs), freqs.numel(),
                    int(bool(interleaved)), _ptr(ctx.positions), x.shape[0], _stream(),
-                   work=(f"{x.shape[0]}x{heads}", x.shape[0] * heads * 2.0 * freqs.numel() * 8, 0.0))
+                   work=lambda: (f"{x.shape[0]}x{heads}", x.shape[0] * heads * 2.0 * freqs.numel() * 8, 0.0))
         return x
 
     def linear_memory(self, u, q_at, k_at, v_at, heads, groups, n, v, log_decay, write, ctx, memory, delta):
@@ -1825,8 +1829,11 @@ class HipOps:
         _want(memory, "memory", torch.float32, (memory.shape[0], 2, heads, v, n))
         out = torch.empty(t, heads * v, dtype=torch.float32, device=u.device)
         state = float(ctx.num_requests) * heads * n * v * 8
-        work = (f"{t} tokens {ctx.num_requests} runs", state + t * (u.shape[1] + heads * v + decay_ld) * 4.0,
-                (6.0 if delta else 4.0) * t * heads * n * v)
+
+        def work():
+            return (f"{t} tokens {ctx.num_requests} runs", state + t * (u.shape[1] + heads * v + decay_ld) * 4.0,
+                    (6.0 if delta else 4.0) * t * heads * n * v)
+
         by_chunks = ctx.plan.get("memory_long_run")
         longest = 0
         if by_chunks is not None and by_chunks.numel() and self.memory_by_chunks:
@@ -1870,7 +1877,7 @@ class HipOps:
         self._call("linear_memory", "tnx_gated_norm", _ptr(o), _ptr(gate), gate_ld, _ptr(weight), float(eps), int(parts),
                    int(bool(gate_first)), _ptr(factors), factors.numel() if factors is not None else 0, _ptr(x), x_ld, _ptr(out), out_ld,
                    float(out_scale), _code(self.dtype), t, width, _stream(),
-                   work=(f"{t}x{width}", t * width * (8.0 + (4 if skip is not None else 0) + out.element_size()), 0.0))
+                   work=lambda: (f"{t}x{width}", t * width * (8.0 + (4 if skip is not None else 0) + out.element_size()), 0.0))
         return out
 
     # ---------------------------------------------------------------- experts
@@ -1901,7 +1908,7 @@ class HipOps:
         out = torch.empty(t, two_f // 2, dtype=self.dtype, device=gate_up.device)
         self._call("experts", "tnx_gated_activation", _ptr(gate_up), _ptr(out), _code(self.dtype), t, two_f // 2,
                    _GATE_ACT[activation], _ptr(row_weights), float(limit or 0.0), _stream(),
-                   work=(f"{t}x{two_f // 2}", t * two_f * 4.0 + out.numel() * out.element_size(), 0.0))
+                   work=lambda: (f"{t}x{two_f // 2}", t * two_f * 4.0 + out.numel() * out.element_size(), 0.0))
         return out
 
     def row_activation(self, x, activation, row_gate=None):
@@ -1911,7 +1918,7 @@ class HipOps:
         gate_ld = self._rows_apart(row_gate, "the rows' gate", torch.float32, t, 1) if row_gate is not None else 0
         out = torch.empty(t, f, dtype=self.dtype, device=x.device)
         self._call("experts", "tnx_row_activation", _ptr(x), ld, _ptr(out), _code(self.dtype), t, f, _ACT[activation], _ptr(row_gate),
-                   gate_ld, _stream(), work=(f"{t}x{f}", t * f * (4.0 + out.element_size()), 0.0))
+                   gate_ld, _stream(), work=lambda: (f"{t}x{f}", t * f * (4.0 + out.element_size()), 0.0))
         return out
 
     # From `expert_grouped_rows` (token, choice) pairs an expert on, bfloat16, sizes in 64s: the experts' products by tiles
@@ -1961,7 +1968,7 @@ class HipOps:
                        _ptr(ints), _ptr(inner), _ptr(y), _ptr(residual), _ptr(out), t, experts, top, width, f,
                        (_ACT if ungated else _GATE_ACT)[activation], int(weight_on == "input"), float(limit or 0.0), int(identity),
                        int(ungated), rows, _stream(),
-                       work=(f"{t}x{top} of {experts}", experts * (2.0 if ungated else 3.0) * f * width * 2 + t * width * 10.0,
+                       work=lambda: (f"{t}x{top} of {experts}", experts * (2.0 if ungated else 3.0) * f * width * 2 + t * width * 10.0,
                              (4.0 if ungated else 6.0) * pairs * f * width))
             return out
         if (may_wait and self.expert_library_rows > 0 and pairs >= self.expert_library_rows * experts
@@ -1994,7 +2001,7 @@ class HipOps:
                 self.linear(inner, w_down[e], None, out_f32=True, f32_by_library=True, into=y[a:b])
             self._call("experts", "tnx_expert_combine", _ptr(y), _ptr(place), None if on_input else _ptr(weights),
                        _ptr(residual), _ptr(out), t, top, width, _ptr(h) if identity else None, _ptr(chosen), experts, _stream(),
-                       work=(f"{t}x{top}x{width}", (pairs + 2.0 * t) * width * 4, 0.0))
+                       work=lambda: (f"{t}x{top}x{width}", (pairs + 2.0 * t) * width * 4, 0.0))
             return out
         ints = torch.empty(experts + 1 + pairs, dtype=torch.int32, device=dev)
         inner = torch.empty(pairs, f, dtype=h.dtype, device=dev)
@@ -2006,7 +2013,7 @@ class HipOps:
                    _code(h.dtype), t, experts, top, width, f, (_ACT if ungated else _GATE_ACT)[activation],
                    int(weight_on == "input"), int(bool(self.expert_plain_products)), float(limit or 0.0), int(identity),
                    int(ungated), _stream(),
-                   work=(f"{t}x{top} of {experts}", used * (2.0 if ungated else 3.0) * f * width * item + t * width * (item + 8.0),
+                   work=lambda: (f"{t}x{top} of {experts}", used * (2.0 if ungated else 3.0) * f * width * item + t * width * (item + 8.0),
                          (4.0 if ungated else 6.0) * t * top * f * width))
         return out
 
