@@ -45,7 +45,8 @@ struct QkvScatter {
 
 // `v`: element n of token m's projections with its bias; `beside`: element n ^ 1 with its bias (read only
 // where the scatter turns pairs)
-__device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, const QkvScatter& sc) {
+// (`page`, `off`: what `token_page` and `token_off` say of token m)
+__device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, const QkvScatter& sc, int page, int off) {
   if (sc.turn_a && n < sc.nq + sc.nk) {
     const size_t at = (size_t)min(max(sc.positions[m], 0), sc.turn_rows - 1) * sc.head_size + n % sc.head_size;
     v = sc.turn_a[at] * v + sc.turn_b[at] * beside;
@@ -54,7 +55,6 @@ __device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, c
     sc.q_out[(size_t)m * sc.nq + n] = (bf16_t)(v * sc.scale);
     return;
   }
-  const int page = sc.token_page[m], off = sc.token_off[m];
   if (page < 0 || page >= sc.num_pages) return;
   int j = n - sc.nq;
   const bool is_key = j < sc.nk;
@@ -515,7 +515,7 @@ gemm_bf16_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, con
           if (QKV) {
             // (the element beside this one is the neighbouring lane's: N is even, so both are there or neither)
             const float v = acc[i][j][e] + (bias ? bias[n] : 0.f);
-            qkv_store(v, lane_dpp<TNX_DPP_XOR1>(v), m, n, sc);
+            qkv_store(v, lane_dpp<TNX_DPP_XOR1>(v), m, n, sc, sc.token_page[m], sc.token_off[m]);
           } else {
             epilogue_store(acc[i][j][e], m, n, N, bias, residual, out, out_dtype, act);
           }
@@ -818,6 +818,29 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     wrow[j] = SHUF ? w + (size_t)min((int)blockIdx.x * RT + j, N / 16 - 1) * 16 * K + (r * 4 + g) * 8
                    : w + (size_t)min(n0 + 16 * j + r, N - 1) * K + 8 * g;
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  // What the end of the kernel adds (bias, residual, the folded norm's vectors) is asked for first: there it would be one
+  // more time to reach memory after the last product. A thread's element q is (row, column) of `place(q)`.
+  constexpr int OUTS = MT * RT * 4 / WAVES;      // elements a thread makes: MT RT tiles of 256 by 64 WAVES threads
+  auto place = [&](int q, int& m, int& n) {
+    const int idx = tid + q * WAVES * 64, l = idx & 63, i = (idx >> 6) & 3, j = (idx >> 8) % RT, t = idx / (256 * RT);
+    m = t * 16 + (l & 15);
+    n = n0 + 16 * j + 4 * (l >> 4) + i;
+  };
+  constexpr bool EARLY = OUTS >= 1 && OUTS <= 4 && MT * RT * 4 % WAVES == 0;
+  float add[EARLY ? OUTS : 1], onto[EARLY ? OUTS : 1], fold_c[EARLY ? OUTS : 1], fold_d[EARLY ? OUTS : 1];
+  int page[EARLY ? OUTS : 1], off[EARLY ? OUTS : 1];
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int q = 0; q < OUTS; ++q) {
+      int m, n;
+      place(q, m, n);
+      m = min(m, M - 1), n = min(n, N - 1);
+      add[q] = bias ? bias[n] : 0.f;
+      if (NORMED) fold_c[q] = nf.c[n], fold_d[q] = nf.d[n];
+      onto[q] = !QKV && residual ? residual[(size_t)m * N + n] : 0.f;
+      if (QKV) page[q] = sc.token_page[m], off[q] = sc.token_off[m];
+    }
+  }
   f32x4 acc[MT][RT];
 #pragma unroll
   for (int t = 0; t < MT; ++t)
@@ -967,7 +990,7 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
   }
   __syncthreads();
   // acc[t][j][i] of lane l is output column n0 + 16*j + 4*(l/16) + i, row 16*t + l%16.
-  for (int idx = tid; idx < MT * RT * 256; idx += WAVES * 64) {
+  auto finish = [&](int idx, int q) {
     const int l = idx & 63, i = (idx >> 6) & 3, j = (idx >> 8) % RT, t = idx / (256 * RT);
     float v = 0.f;
 #pragma unroll
@@ -990,20 +1013,31 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
       const float mean = nf.center ? a1 / (float)K : 0.f;     // of x - x0
       const float var = fmaxf(a2 / (float)K - mean * mean, 0.f);
       const float rstd = rsqrtf(var + nf.eps);
-      v = rstd * (v - mean * nf.c[n]) + nf.d[n];
+      v = rstd * (v - mean * (EARLY ? fold_c[q] : nf.c[n])) + (EARLY ? fold_d[q] : nf.d[n]);
       if (pairs) beside = rstd * (beside - mean * nf.c[n ^ 1]) + nf.d[n ^ 1];
     }
     if (n < N && m < M) {
       if (QKV) {
         if (bias) {
-          v += bias[n];
+          v += EARLY ? add[q] : bias[n];
           if (pairs) beside += bias[n ^ 1];
         }
-        qkv_store(v, beside, m, n, sc);
+        qkv_store(v, beside, m, n, sc, EARLY ? page[q] : sc.token_page[m], EARLY ? off[q] : sc.token_off[m]);
+      } else if (EARLY) {
+        if (bias) v += add[q];
+        v = apply_act(v, act);
+        if (residual) v += onto[q];
+        store_any(out, out_dtype, (size_t)m * N + n, v);
       } else {
         epilogue_store(v, m, n, N, bias, residual, out, out_dtype, act);
       }
     }
+  };
+  if constexpr (EARLY) {
+#pragma unroll
+    for (int q = 0; q < OUTS; ++q) finish(tid + q * WAVES * 64, q);
+  } else {
+    for (int idx = tid; idx < MT * RT * 256; idx += WAVES * 64) finish(idx, 0);
   }
 }
 

@@ -812,15 +812,21 @@ class HipOps:
         shares = max(1, min(self.compute_units // column_blocks, k // 512))     # as the kernel shares K out
         return small or 4 * column_blocks * shares >= 3 * self.compute_units
 
-    def _library_product(self, m, n, k, w, force_tiled) -> bool:
+    def _library_product(self, m, n, k, w, force_tiled, scattered=False) -> bool:
+        """`scattered`: the fused projection of queries, keys and values, whose result the few-rows kernel puts in its
+        places itself (after the library's product a kernel of 6 to 7 us does that)."""
         if not (self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.library_rows > 0
                 and m >= self.library_rows and not force_tiled and n % 8 == 0 and k % 8 == 0):
             return False
         # small matrices at up to 32 rows: one launch of ours (5 to 10 us with its epilogue) beats the
         # library's product and the epilogue after it (11 to 15 us)
-        return not (m <= 32 and n * k <= self.small_matrix)
+        return not (m <= 32 and n * k <= (self.fused_matrix if scattered else self.small_matrix))
 
     small_matrix = 1 << 23
+    # Queries, keys and values at 17 to 32 rows, us, few-rows kernel with everything in one launch against the library's
+    # product and `qkv_write`: 24 rows 6,144 x 2,048 11.5 / 18.9, 32 rows 12.3 / 16.4, 7,680 x 2,560 14.0 / 20.0 and
+    # 15.1 / 20.4; 12,288 x 4,096 33.7 / 33 and 38.2 / 33.6.
+    fused_matrix = 20 << 20
 
     # ---------------------------------------------------------------- attention
 
@@ -869,7 +875,7 @@ class HipOps:
         if isinstance(h, DeferredNorm):
             folded = self._folded_for(h, w) if force_tiled != 1 else None
             if folded is not None and (ctx.num_tokens >= 128 or self._library_product(
-                    ctx.num_tokens, w.tensor.shape[0], w.tensor.shape[1], w.tensor, force_tiled)):
+                    ctx.num_tokens, w.tensor.shape[0], w.tensor.shape[1], w.tensor, force_tiled, True)):
                 folded = None
             if folded is None:
                 h = h.materialize()
@@ -904,7 +910,7 @@ class HipOps:
             w, tiles = w.tensor, w.tiles
         many = ctx.num_tokens >= 128 and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and not force_tiled
         if self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (many or self._library_product(
-                ctx.num_tokens, w.shape[0], w.shape[1], w, force_tiled)):
+                ctx.num_tokens, w.shape[0], w.shape[1], w, force_tiled, tiles is not None)):
             # many rows (the vendor library, or our wide-tile kernel where sizes allow): the bias joins the
             # product's float32 sums before they are rounded, once, as in the fused kernel below, so that keys
             # and values are cached with the same rounding whichever path a token took; the queries are
