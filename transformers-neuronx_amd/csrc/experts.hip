@@ -372,16 +372,18 @@ __global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p)
 }
 
 // ---------------------------------------------------------------- many pairs an expert
-// The same products where an expert has many pairs (prompts): tiles of 64 MI pairs by 128 of the matrix's rows on MFMA
-// 32x32x16 (`tiles.h`), one launch over all experts. UP_GATED: a wave takes 32 gate rows and the 32 up rows that go with
-// them, so that act(g) * u is made of its own sums; the tile makes 64 columns of `inner`. The pairs' rows are gathered by
-// the loads themselves: a lane's address in `h` is that of its pair's token. `inner` and the result lie in sorted order.
-// What bounds it is the matrix unit (a tile of 128 x 128 reads LDS at the full rate while it multiplies); an expert's last
-// tile may be nearly empty, so where an expert has fewer pairs the tiles are of 64.
+// The same products where an expert has many pairs (prompts): tiles of 64 or 128 pairs by 128 or 256 of the matrix's rows on
+// MFMA 32x32x16 (`tiles.h`), one launch over all experts. UP_GATED: a wave takes 32 gate rows and the 32 up rows that go with
+// them, so that act(g) * u is made of its own sums; the tile makes half as many columns of `inner`. The pairs' rows are
+// gathered by the loads themselves: a lane's address in `h` is that of its pair's token. `inner` and the result lie in sorted
+// order. What bounds it is how well a unit's waves keep its matrix cores at work between their meetings (two waves a core and
+// a wave's 64 x 64 of the tile: 60 % of the time); an expert's last tile may be nearly empty, so where an expert has fewer
+// pairs the tiles are of 64.
 // Blocks of an XCD take the tiles of one column block after the other, so that an expert's rows of the matrix are brought
 // from memory once and read again from that XCD's cache.
-// Measured at 2,048 tokens of two choices among 8 experts, a layer: 4,096 wide, inner 4,096, 632 us (650 TFLOP/s) against
-// 804 with sixteen products of the vendor library and a wait for the host between; 2,048 wide 207 against 504.
+// Measured at 2,048 tokens of two choices among 8 experts, a layer: 4,096 wide, inner 4,096, 543 us (760 TFLOP/s) against
+// 795 with sixteen products of the vendor library and a wait for the host between; 2,048 wide 175 against 422. With four
+// waves of 64 x 64 on 128 rows of the matrix, two blocks a unit: 632 and 207.
 struct GroupedArgs {
   const bf16_t* a;          // UP: h [T, K]; DOWN: inner [sorted pairs, K]
   const bf16_t* w;          // [E, N(, 2), K]
@@ -394,17 +396,17 @@ struct GroupedArgs {
   float limit;
 };
 
-template <int KIND, int MI, int ST>
-__global__ void __launch_bounds__(256) expert_tiles_kernel(GroupedArgs p) {
+template <int KIND, int MI, int ST, int WN>
+__global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
   constexpr bool GATED = KIND == UP_GATED, UP = KIND != DOWN;
-  typedef Tile<MI, 2, ST> Products;
+  typedef Tile<MI, 2, ST, 2, WN> Products;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int at = by_xcd(blockIdx.x, gridDim.x);
   const int2 tile = p.tiles[at % p.slots];
   const int e = tile.x;
   if (e < 0) return;
   const int begin = tile.y, count = min(Products::TM, p.first[e + 1] - begin);
-  const int n0 = at / p.slots * (GATED ? 64 : 128);
+  const int n0 = at / p.slots * (GATED ? Products::TN / 2 : Products::TN);
   Products t;
 #pragma unroll
   for (int j = 0; j < Products::LA; ++j) {
@@ -447,29 +449,31 @@ __global__ void __launch_bounds__(256) expert_tiles_kernel(GroupedArgs p) {
   }
 }
 
-template <int KIND, int MI, int ST>
+template <int KIND, int MI, int ST, int WN>
 int launch_tiles(const GroupedArgs& p, hipStream_t stream) {
-  constexpr int bytes = Tile<MI, 2, ST>::BYTES;
+  typedef Tile<MI, 2, ST, 2, WN> Products;
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)expert_tiles_kernel<KIND, MI, ST>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
-    TNX_REQUIRE(e == hipSuccess, "expert tiles: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    hipError_t e = hipFuncSetAttribute((const void*)expert_tiles_kernel<KIND, MI, ST, WN>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, Products::BYTES);
+    TNX_REQUIRE(e == hipSuccess, "expert tiles: cannot reserve %d bytes of LDS: %s", Products::BYTES, hipGetErrorString(e));
     configured = true;
   }
-  const int columns = KIND == UP_GATED ? 64 : 128;
-  expert_tiles_kernel<KIND, MI, ST><<<(p.n + columns - 1) / columns * p.slots, 256, bytes, stream>>>(p);
+  const int columns = KIND == UP_GATED ? Products::TN / 2 : Products::TN;
+  expert_tiles_kernel<KIND, MI, ST, WN><<<(p.n + columns - 1) / columns * p.slots, 128 * WN, Products::BYTES, stream>>>(p);
   TNX_CHECK_LAUNCH("expert tiles");
   return 0;
 }
 
+// Tiles of 128 pairs: eight waves over 256 of the matrix's rows, three stages (144 KB, one block a unit). Tiles of 64: four
+// waves over 128 rows; two stages, so that a unit holds three blocks, four where it has no more than one anyway (the slots
+// count an empty tile an expert too many, about half used).
 template <int KIND>
 int launch_tiles(const GroupedArgs& p, int tile_rows, hipStream_t stream) {
-  // four stages where a compute unit has one block anyway (slots count an empty tile an expert too many, about half used)
+  if (tile_rows == 128) return launch_tiles<KIND, 2, 3, 4>(p, stream);
   const int columns = KIND == UP_GATED ? 64 : 128;
   const bool deep = (long long)((p.n + columns - 1) / columns) * p.slots <= tnx_compute_units();
-  if (tile_rows == 64) return deep ? launch_tiles<KIND, 1, 4>(p, stream) : launch_tiles<KIND, 1, 2>(p, stream);
-  return deep ? launch_tiles<KIND, 2, 4>(p, stream) : launch_tiles<KIND, 2, 2>(p, stream);
+  return deep ? launch_tiles<KIND, 1, 4, 2>(p, stream) : launch_tiles<KIND, 1, 2, 2>(p, stream);
 }
 
 // (`place`: the row of y that holds pair t * top + c, where the rows lie in another order; `scale`: a factor a pair.

@@ -4,20 +4,21 @@
 #include "common.h"
 #include <type_traits>
 
-// A block of 2 x 2 waves, each of 32 MI rows by 32 NI columns as MI x NI MFMA 32x32x16 tiles: TM = 64 MI, TN = 64 NI.
+// A block of WM x WN waves, each of 32 MI rows by 32 NI columns as MI x NI MFMA 32x32x16 tiles: TM = 32 MI WM, TN = 32 NI WN.
 // Both operands go from global memory straight into LDS in steps of 64 of K, ST stages deep; the 16-byte chunks of a row
 // (8 of them, 128 bytes) lie swizzled by row, so that the fragment reads are free of bank conflicts.
-// MI = NI = 2 and two stages take 64 KB and leave room for a second block on the compute unit, whose products cover this
-// one's waits; where a unit has one block anyway, four stages (128 KB) do that instead.
-template <int MI, int NI, int ST>
+// Eight waves give every matrix core two: one multiplies while the other waits for LDS or for a load to be taken. Measured as a
+// plain product of 2,048 rows, 4,096 columns, K 16,384, us (TFLOP/s): four waves of 128 x 64 on 256 x 128, three stages, 264
+// (1,040); eight of 64 x 64 there 243 (1,130), with the next step's fragments read before the last products of a step 235
+// (1,170); four of 64 x 64 on 128 x 128, two stages and two blocks a unit, 306; 256 x 256, two stages, 263 at best.
+template <int MI, int NI, int ST, int WM = 2, int WN = 2>
 struct Tile {
-  static constexpr int TM = 64 * MI, TN = 64 * NI;
+  static constexpr int WAVES = WM * WN, TM = 32 * MI * WM, TN = 32 * NI * WN;
   static constexpr int STAGE = (TM + TN) * 128;                     // bytes
-  static constexpr int AHEAD = MI * NI <= 4 ? 4 : 2;
-  static constexpr int LA = 2 * MI, LB = 2 * NI;                    // loads a wave issues for a step of x, of w
+  static constexpr int LA = TM / 8 / WAVES, LB = TN / 8 / WAVES;    // loads a wave issues for a step of x, of w
   static constexpr int OUT_ROW = 32 * NI * 4 + 16;                  // bytes of a row of the result on its way out
   static constexpr int OUT = 32 * OUT_ROW;                          // bytes of LDS a wave uses for that
-  static constexpr int BYTES = ST * STAGE > 4 * OUT ? ST * STAGE : 4 * OUT;
+  static constexpr int BYTES = ST * STAGE > WAVES * OUT ? ST * STAGE : WAVES * OUT;
 
   // what this lane loads at step 0, as bytes from the operands' beginnings (operands of less than 4 GB): set by the
   // caller from `x_row` / `w_row` and `k_of`
@@ -30,20 +31,29 @@ struct Tile {
   static __device__ __forceinline__ int w_row(int j) { return (LB * wave() + j) * 8 + ((threadIdx.x & 63) >> 3); }
   static __device__ __forceinline__ int k_of(int row) { return 8 * ((threadIdx.x & 7) ^ ((row >> 1) & 7)); }
   // the first row and column of this wave within the tile
-  static __device__ __forceinline__ int row0() { return (wave() & 1) * 32 * MI; }
-  static __device__ __forceinline__ int col0() { return (wave() >> 1) * 32 * NI; }
+  static __device__ __forceinline__ int row0() { return (wave() % WM) * 32 * MI; }
+  static __device__ __forceinline__ int col0() { return (wave() / WM) * 32 * NI; }
 
-  // The sums over `steps` steps of 64 of K. A step's loads are issued one by one between the products of the step before:
-  // a load takes the unit's address path for 16 cycles, and a wave waits where it comes to one that the others' loads
-  // keep busy (all at the top of a step: 2 to 10 % slower).
+  // The sums over `steps` steps of 64 of K. A step is four products of 16 of K; its loads, for the step ST - 1 ahead, are
+  // issued one by one between them. The wait for the next step's operands and the block's meeting come before the last of
+  // the four, and so do the reads of the next step's first fragments: those products run while the fragments arrive, where
+  // after a meeting at the top of a step the matrix unit would stand until LDS has answered.
   __device__ __forceinline__ void run(char* smem, const bf16_t* x, const bf16_t* w, int steps) {
-    constexpr int L = LA + LB, P = 4 * MI * NI;                     // loads and products of a step
+    constexpr int L = LA + LB, P = 3 * MI * NI;                     // loads of a step, and the products they stand between
     const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
     const unsigned a_dst = lds_offset(smem) + LA * wave() * 1024, b_dst = lds_offset(smem) + TM * 128 + LB * wave() * 1024;
     auto load = [&](int t, int l) {
       const unsigned stage = (t % ST) * STAGE;
       if (l < LA) load_to_lds(x + (size_t)64 * t, xoff[l < LA ? l : 0], a_dst + stage + l * 1024);
       else load_to_lds(w + (size_t)64 * t, woff[l < LA ? 0 : l - LA], b_dst + stage + (l - LA) * 1024);
+    };
+    // step t has landed when at most the loads of the `behind` steps after it are still in flight
+    auto landed = [&](int behind) {
+      if (ST > 4 && behind >= 3) __builtin_amdgcn_s_waitcnt(0x0F70 | ((3 * L) & 15) | (((3 * L) >> 4) << 14));
+      else if (ST > 3 && behind == 2) __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * L) & 15) | (((2 * L) >> 4) << 14));
+      else if (ST > 2 && behind == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | (L & 15) | ((L >> 4) << 14));
+      else __builtin_amdgcn_s_waitcnt(0x0F70);
+      __syncthreads();
     };
 #pragma unroll
     for (int i = 0; i < MI; ++i)
@@ -59,29 +69,29 @@ struct Tile {
       }
     const int swizzle = (l32 >> 1) & 7;
     const int a0 = (row0() + l32) * 128, b0 = TM * 128 + (col0() + l32) * 128;
+    bf16x8 a[4][MI], b[4][NI];
+    auto frags = [&](int t, int s) {
+      const char* base = smem + (t % ST) * STAGE;
+      const int chunk = ((2 * s + half) ^ swizzle) * 16;
+#pragma unroll
+      for (int i = 0; i < MI; ++i) a[s][i] = *(const bf16x8*)(base + a0 + i * 4096 + chunk);
+#pragma unroll
+      for (int j = 0; j < NI; ++j) b[s][j] = *(const bf16x8*)(base + b0 + j * 4096 + chunk);
+    };
+    landed(min(ST - 2, steps - 1));
+    frags(0, 0);
     auto step = [&](int t, auto with_loads) {
       constexpr bool more = decltype(with_loads)::value;
-      // step t has landed when at most the loads of the ST - 2 steps behind it are still in flight
-      const int ahead = min(ST - 2, steps - 1 - t);
-      if (ST > 3 && ahead == 2) __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * L) & 15) | (((2 * L) >> 4) << 14));
-      else if (ST > 2 && ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | (L & 15) | ((L >> 4) << 14));
-      else __builtin_amdgcn_s_waitcnt(0x0F70);
-      __syncthreads();
-      const char* base = smem + (t % ST) * STAGE;
-      bf16x8 a[4][MI], b[4][NI];
-      auto frags = [&](int slot, int s) {
-        const int chunk = ((2 * s + half) ^ swizzle) * 16;
 #pragma unroll
-        for (int i = 0; i < MI; ++i) a[slot][i] = *(const bf16x8*)(base + a0 + i * 4096 + chunk);
-#pragma unroll
-        for (int j = 0; j < NI; ++j) b[slot][j] = *(const bf16x8*)(base + b0 + j * 4096 + chunk);
-      };
-#pragma unroll
-      for (int s = 0; s < AHEAD; ++s) frags(s, s);
+      for (int s = 1; s < 4; ++s) frags(t, s);
+      __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int s = 0; s < 4; ++s) {
-        if (s + AHEAD < 4) frags(s + AHEAD, s + AHEAD);      // later products' fragments arrive while these run
-        __builtin_amdgcn_sched_barrier(0);
+        if (s == 3 && (more || t + 1 < steps)) {
+          landed(more ? ST - 2 : min(ST - 2, steps - 2 - t));
+          frags(t + 1, 0);
+          __builtin_amdgcn_sched_barrier(0);
+        }
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
@@ -90,7 +100,7 @@ struct Tile {
             if constexpr (more) {
               const int q = (s * MI + i) * NI + j;
 #pragma unroll
-              for (int l = q * L / P; l < (q + 1) * L / P; ++l) {
+              for (int l = q * L / P; l < (q + 1) * L / P && l < L; ++l) {
                 __builtin_amdgcn_sched_barrier(0);
                 load(t + ST - 1, l);
                 __builtin_amdgcn_sched_barrier(0);

@@ -1930,10 +1930,10 @@ class HipOps:
     # From `expert_grouped_rows` (token, choice) pairs an expert on, bfloat16, sizes in 64s: the experts' products by tiles
     # (two launches over all experts, the host reads nothing), of 128 pairs from `expert_wide_tiles` an expert on. Measured
     # for 8 experts, two a token, us a layer, one launch of 16 pairs a tile or the library / tiles of 64 / of 128: 2,048 wide,
-    # 12 pairs an expert 57 / 65 / 69, 16: 73 / 66 / 71, 50: 132 / 73 / 77, 99: 520 / 95 / 91, 512: 504 / 207 / 213; 4,096 wide,
-    # 12: 155 / 216 / 212, 16: 216 / 214 / 221, 50: 463 / 221 / 219, 99: 492 / 272 / 232, 512: 804 / 681 / 632.
+    # 12 pairs an expert 57 / 67 / 77, 16: 75 / 68 / 77, 50: 132 / 73 / 82, 99: 432 / 97 / 91, 512: 422 / 205 / 175; 4,096 wide,
+    # 12: 199 / 218 / 209, 16: 218 / 216 / 208, 50: 469 / 224 / 209, 99: 449 / 283 / 220, 512: 795 / 688 / 543.
     expert_grouped_rows = 16           # 0: never
-    expert_wide_tiles = 64
+    expert_wide_tiles = 80
     # Other sizes, from this many pairs an expert on, in a step that is not being recorded: the host reads where each
     # expert's pairs begin (one small copy that waits for the device) and every expert's two products go to the vendor
     # library over its own rows. Below that, and in recorded steps, one launch of ours with tiles of 16 pairs takes all
