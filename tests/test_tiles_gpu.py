@@ -62,3 +62,42 @@ def test_experts_by_tiles(counts, width, f, act, on, identity, rows):
                                  limit=1.5 if act == "clamped_swiglu" else None, identity=identity)
         # the inner values are rounded to bfloat16 (by 2^-8 of themselves at most), everything else is summed in float32
         assert _apart(got - (r if r is not None else 0), want) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 64, 64), (33, 200, 64), (64, 72, 320), (65, 2048, 2048), (128, 136, 8192), (129, 128, 512),
+                                   (333, 264, 2048), (700, 520, 2112)])
+@pytest.mark.parametrize("tile,shares", [(1, 1), (1, 3), (2, 1), (2, 5)])
+def test_product_by_tiles(m, n, k, tile, shares):
+    """Every tile with and without shares of K, at sizes that end inside a tile."""
+    from transformers_neuronx_amd.kernels.hip import HipOps, _ptr, _stream
+    ops, g = HipOps(torch.bfloat16, DEV), torch.Generator(device=DEV).manual_seed(m + n + k)
+    x, w = torch.randn(m, k, device=DEV, generator=g).bfloat16(), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).bfloat16()
+    bias, res = torch.randn(n, device=DEV, generator=g), torch.randn(m, n, device=DEV, generator=g)
+    exact = x.double() @ w.double().T
+    space = torch.empty(shares * m * n, device=DEV)
+    magnitude = x.double().abs() @ w.double().abs().T + bias.abs() + res.abs()
+    for b, r, act, dtype in ((bias, None, 1, torch.bfloat16), (bias, res, 0, torch.float32), (None, None, 0, torch.float32)):
+        out = torch.full((m, n), float("nan"), device=DEV, dtype=dtype)
+        ops.call("gemm", "tnx_gemm_bf16_tiles", _ptr(x), _ptr(w), _ptr(b), _ptr(r), _ptr(out), int(dtype == torch.bfloat16), act,
+                 m, n, k, _ptr(space), space.numel(), tile, shares, _stream())
+        want = exact + (b.double() if b is not None else 0)
+        want = want.relu() if act else want
+        want = want + (r.double() if r is not None else 0)
+        # products of bfloat16 are exact in float32; a sum of k of them is off by k 2^-24 of the magnitudes at most, and a
+        # bfloat16 result (8 bits) by half a place, 2^-8 of it at most, more
+        bound = 2 * (k + 4) * 2.0 ** -24 * magnitude + (2.0 ** -8 * want.abs() if dtype == torch.bfloat16 else 0)
+        assert bool(((out.double() - want).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("m,n,k", [(40, 2048, 2048), (100, 6144, 2048), (333, 2048, 8192)])
+def test_products_that_the_tiles_take(m, n, k):
+    """`linear` takes the tiles there, with what the library's way gives up to the rounding of the result."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops, lib = HipOps(torch.bfloat16, DEV), HipOps(torch.bfloat16, DEV)
+    lib.tile_products = False
+    g = torch.Generator(device=DEV).manual_seed(n)
+    x, w = torch.randn(m, k, device=DEV, generator=g).bfloat16(), (torch.randn(n, k, device=DEV, generator=g) * k ** -0.5).bfloat16()
+    bias, res = torch.randn(n, device=DEV, generator=g), torch.randn(m, n, device=DEV, generator=g)
+    assert ops._tiles_room(m, n, k, x, w, None, False, False) >= 0
+    for kw in (dict(bias=bias, act="relu"), dict(bias=bias, act="gelu"), dict(residual=res, out_f32=True), dict()):
+        torch.testing.assert_close(ops.linear(x, w, **kw).float(), lib.linear(x, w, **kw).float(), rtol=1e-2, atol=2e-2)

@@ -6,7 +6,7 @@
 //                   128x128 tiles staged through registers for every other size
 //   gemm_bf16_skinny  bfloat16 operands on MFMA for M <= 64 (decoding): streams the weight once
 // bias and residual are float32 and optional; the output is float32 or bfloat16.
-#include "common.h"
+#include "tiles.h"
 #include <type_traits>
 
 TNX_DEFINE_ERROR_API
@@ -1478,6 +1478,160 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 #undef MID_HIGH
 #undef MID_LOW
 #undef MID
+}
+
+// ------------------------------------------------------------------------------------- bfloat16, tiles
+
+// out = act(x w^T + bias) + residual by tiles of 32 MI WM x 32 NI WN (`tiles.h`), K shared out over gridDim.y blocks where the
+// result has too few tiles to give every compute unit one; the shares' float32 sums then go to `partial` and
+// `gemm_mid_sum_kernel` adds them in their order. K is a multiple of 64, N of 8.
+template <int MI, int NI, int ST, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_tiles_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w,
+                                                              const float* __restrict__ bias, const float* __restrict__ residual,
+                                                              void* __restrict__ out, int out_dtype, int act,
+                                                              float* __restrict__ partial, int M, int N, int K, int tiles_m,
+                                                              int steps_per_share) {
+  typedef Tile<MI, NI, ST, WM, WN> Products;
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int at = by_xcd(blockIdx.x, gridDim.x);
+  const int m0 = at % tiles_m * Products::TM, n0 = at / tiles_m * Products::TN;
+  const int first = blockIdx.y * steps_per_share, steps = min(K / 64 - first, steps_per_share);
+  Products t;
+#pragma unroll
+  for (int j = 0; j < Products::LA; ++j) {
+    const int row = Products::x_row(j);
+    t.xoff[j] = 2u * ((unsigned)min(m0 + row, M - 1) * (unsigned)K + Products::k_of(row));
+  }
+#pragma unroll
+  for (int j = 0; j < Products::LB; ++j) {
+    const int row = Products::w_row(j);
+    t.woff[j] = 2u * ((unsigned)min(n0 + row, N - 1) * (unsigned)K + Products::k_of(row));
+  }
+  t.run(smem, x + 64 * first, w + 64 * first, steps);
+  const int mw = m0 + Products::row0(), nw = n0 + Products::col0();
+  if (partial) {
+    float* mine = partial + (size_t)blockIdx.y * M * N;
+    t.template hand_out<float, 32 * NI>(
+        smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
+        [&](int r, int c, f32x4 chunk) {
+          if (mw + r < M && nw + c < N) *(f32x4*)(mine + (size_t)(mw + r) * N + nw + c) = chunk;
+        });
+    return;
+  }
+  float added[NI][16];
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e)
+      added[j][e] = bias ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * (int)((threadIdx.x >> 5) & 1) + (e & 3), N - 1)] : 0.f;
+  auto value = [&](int i, int j, int e, int, int) { return apply_act(t.acc[i][j][e] + added[j][e], act); };
+  if (out_dtype == TNX_F32) {
+    t.template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
+      if (mw + r < M && nw + c < N) {
+        const size_t o = (size_t)(mw + r) * N + nw + c;
+        if (residual) chunk += *(const f32x4*)(residual + o);
+        *(f32x4*)((float*)out + o) = chunk;
+      }
+    });
+  } else {
+    t.template hand_out<bf16_t, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
+      if (mw + r < M && nw + c < N) *(f32x4*)((bf16_t*)out + (size_t)(mw + r) * N + nw + c) = chunk;
+    });
+  }
+}
+
+template <int MI, int NI, int ST, int WM, int WN>
+static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, const float* residual, void* out, int out_dtype,
+                        int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
+  constexpr int bytes = Tile<MI, NI, ST, WM, WN>::BYTES;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_tiles_kernel<MI, NI, ST, WM, WN>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "gemm_bf16_tiles: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  const int tiles_m = (M + 32 * MI * WM - 1) / (32 * MI * WM), tiles_n = (N + 32 * NI * WN - 1) / (32 * NI * WN);
+  const int per = (K / 64 + shares - 1) / shares;
+  shares = (K / 64 + per - 1) / per;
+  gemm_bf16_tiles_kernel<MI, NI, ST, WM, WN><<<dim3(tiles_m * tiles_n, shares), 64 * WM * WN, bytes, stream>>>(
+      x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, M, N, K, tiles_m, per);
+  TNX_CHECK_LAUNCH("gemm_bf16_tiles");
+  if (shares > 1) {
+    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
+                                                                                        act, M, N, shares);
+    TNX_CHECK_LAUNCH("gemm_mid_sum");
+  }
+  return 0;
+}
+
+// Which products these tiles take, and with which tile and how many shares of K (0: none, the vendor library is quicker).
+// Measured, us, library against tiles (which), bias and ReLU or residual included:
+//   long K, at least four times the columns, tiles of 128 x 128 and as many shares as give every unit a block: 100 rows 2,048
+//   (columns) x 8,192 (K) 20.4 / 18.4, 4,096 x 16,384 52.3 / 39.1; 333 rows 37.7 / 27.2 and 83.3 / 69.8; 640 rows 43.9 / 37.8
+//   and 120 / 109. Up to 768 rows: at 1,024 the library's larger tiles win (2,048 x 8,192 49 / 54).
+//   short K, up to 2,048, where tiles of 64 x 64 make at most one and a quarter a unit: 100 rows 6,144 x 2,048 14.3 / 13.3,
+//   8,192 x 2,048 16.7 / 15.2, 3,072 x 1,024 8.6 / 6.8; 333 rows 2,048 x 2,048 11.0 / 10.5, 3,072 x 1,024 10.4 / 8.5; or
+//   tiles of 128 x 128 at most one: 333 rows 6,144 x 2,048 25.2 / 20.7, 8,192 x 2,048 23.9 / 21.5; 640 rows 6,144 x 2,048
+//   24.8 / 23.7. Beyond (640 rows 8,192 x 2,048 27.3 / 32.3) the library.
+//   33 to 64 rows and K of 4,096, tiles of 64 x 64 with shares: 48 rows 4,096 x 4,096 16.2 / 13.2, 12,288 x 4,096 26.4 / 25.9.
+// Up to 32 rows half a tile would be padding (32 rows 10,240 x 2,560: 17.7 / 20), and other kernels stand ready.
+// A call of the library's takes the host some 13 us, a launch of ours 5: a step of 333 tokens waits for that, too.
+// What bounds these sizes is the time a unit takes for a step of its one block (0.55 us for 128 x 128 x 64, of which the
+// matrix cores work 0.24), not memory: shares of K are the way to keep all units at it.
+enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2 };
+static int choose_tiles(int M, int N, int K, int& shares) {
+  const int units = tnx_compute_units(), steps = K / 64;
+  const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64), large = (long long)((M + 127) / 128) * ((N + 127) / 128);
+  auto share_out = [&](long long tiles) {
+    int s = (int)(units / tiles);
+    s = s < 1 ? 1 : s > 8 ? 8 : s;
+    while (s > 1 && (steps / s < 4 || (long long)s * M * N > F32_SHARES_MOST)) --s;
+    return s;
+  };
+  shares = 1;
+  if (M <= 32 || M > 768) return TILES_NONE;
+  if (K >= 4ll * N && large <= units) {
+    shares = share_out(large);
+    return TILES_128;
+  }
+  if (K <= 2048 && 4 * small <= 5 * units) return TILES_64;
+  if (K <= 2048 && large <= units) return TILES_128;
+  if (M <= 64 && K <= 4096 && small <= units) {
+    shares = share_out(small);
+    return TILES_64;
+  }
+  return TILES_NONE;
+}
+
+// Whether `tnx_gemm_bf16_tiles` is the way for a product (-1: it is not), and how many floats of workspace it then wants.
+extern "C" int tnx_gemm_bf16_tiles_workspace(int M, int N, int K) {
+  if (M <= 0 || N <= 0 || N % 8 || K <= 0 || K % 64) return -1;
+  if ((long long)M * K >= (1ll << 31) || (long long)N * K >= (1ll << 31)) return -1;
+  int shares = 1;
+  if (choose_tiles(M, N, K, shares) == TILES_NONE) return -1;
+  return shares > 1 ? shares * M * N : 0;
+}
+
+// `workspace`: as many floats as `tnx_gemm_bf16_tiles_workspace` names for the sizes. `tile`, `shares` 0: chosen here.
+extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bias, const float* residual, void* out,
+                                   int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
+                                   int tile, int shares, hipStream_t stream) {
+  TNX_REQUIRE(M > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 64 == 0, "gemm_bf16_tiles: N in 8s and K in 64s, got M=%d N=%d K=%d", M, N, K);
+  TNX_REQUIRE((long long)M * K < (1ll << 31) && (long long)N * K < (1ll << 31), "gemm_bf16_tiles: operands of 4 GB or more");
+  TNX_REQUIRE(out_dtype == TNX_F32 || (out_dtype == TNX_BF16 && residual == nullptr), "gemm_bf16_tiles: a residual beside a float32 result");
+  TNX_REQUIRE(((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)residual | (uintptr_t)workspace) % 16 == 0,
+              "gemm_bf16_tiles: operands must be 16-byte aligned");
+  TNX_REQUIRE(tile >= 0 && tile <= TILES_128 && shares >= 0, "gemm_bf16_tiles: tiles 1 (64) and 2 (128)");
+  int chosen = 1;
+  if (tile == 0) tile = choose_tiles(M, N, K, chosen);
+  if (shares == 0) shares = chosen;
+  if (shares > K / 64) shares = K / 64;
+  if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
+  const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
+  if (tile == TILES_128)
+    return launch_tiles<2, 1, 4, 2, 4>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream);
+  return launch_tiles<1, 1, 4, 2, 2>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream);
 }
 
 // ------------------------------------------------------------------------------------- the vendor library

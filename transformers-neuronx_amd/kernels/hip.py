@@ -48,6 +48,9 @@ _SIGNATURES = {
         "tnx_gemm_skinny_tiles_per_block": [_c_int, _c_int],
         "tnx_gemm_bf16_mid": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                               _c_int, _c_void_p, ctypes.c_size_t, _c_int, _c_int, _c_void_p],
+        "tnx_gemm_bf16_tiles": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                _c_void_p, ctypes.c_size_t, _c_int, _c_int, _c_void_p],
+        "tnx_gemm_bf16_tiles_workspace": [_c_int, _c_int, _c_int],
         "tnx_gemm_library": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                              _c_int, _c_void_p, ctypes.c_size_t, _c_void_p, ctypes.c_size_t, _c_int, _c_void_p],
         "tnx_gemm_bf16_normed": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_void_p, _c_int,
@@ -354,6 +357,7 @@ class HipOps:
         self._conv_copies = {}
         self._later = []
         self._tiles_per_block = {}
+        self._tiles_rooms = {}
         self._landing, self._landing_turn = [None, None], 0
         self._ints, self._ints_done, self._ints_turn = [None, None], [None, None], 0
 
@@ -633,7 +637,7 @@ class HipOps:
         if isinstance(x, DeferredNorm):
             folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
             if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
-                                                              w.tensor, force_tiled):
+                                                              w.tensor, force_tiled, plain=True):
                 folded = None
             if folded is None:
                 x = x.materialize()
@@ -685,7 +689,18 @@ class HipOps:
                        _ptr(residual), _ptr(out), _code(out_dtype), _ACT[act], m, n, k, _ptr(space), space.numel() // 4,
                        0, 0, _stream(), work=lambda: self._product_work(m, n, k, out_item=4, residual=residual is not None))
             return out
-        if (self._library_product(m, n, k, w, force_tiled) and (residual is not None or not out_f32)):
+        room = self._tiles_room(m, n, k, x, w, residual, out_f32, force_tiled) if f32_by_library or residual is not None or not out_f32 else -1
+        if room >= 0:
+            out = torch.empty(m, n, dtype=out_dtype, device=x.device) if into is None else _want(into, "into", out_dtype, (m, n))
+            if _ptr(out) % 16 == 0:
+                xa = self.cast(x, torch.bfloat16)
+                space = torch.empty(room, dtype=torch.float32, device=x.device) if room else None
+                self._call("gemm", "tnx_gemm_bf16_tiles", _ptr(xa), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out), _code(out_dtype),
+                           _ACT[act], m, n, k, _ptr(space), room, 0, 0, _stream(),
+                           work=lambda: self._product_work(m, n, k, out_item=out.element_size(), residual=residual is not None))
+                return out
+        if (self._library_product(m, n, k, w, force_tiled, plain=tiles is not None and not out_f32)
+                and (residual is not None or not out_f32)):
             # Many rows: the product goes to the vendor library (hipBLASLt), with what follows it where the
             # library can do that itself: bias and ReLU before it rounds a bfloat16 result, or bias and the
             # residual added to its float32 sums for a float32 result. The float32 head keeps our kernel.
@@ -730,6 +745,19 @@ class HipOps:
                        _ptr(out), _code(out_dtype), _ACT[act], m, n, k, int(force_tiled), _stream(),
                        work=lambda: self._product_work(m, n, k, out_item=out.element_size(), residual=residual is not None))
         return out
+
+    tile_products = True    # products of 17 to 768 rows by tiles of ours where those are quicker than the vendor library
+
+    def _tiles_room(self, m, n, k, x, w, residual, out_f32, force_tiled) -> int:
+        """The floats of workspace that the product by tiles wants, -1 where it is not the way (the rule on sizes and what
+        it was measured by are with the kernel)."""
+        if not (self.tile_products and self._library_product(m, n, k, w, force_tiled) and (residual is None or out_f32)
+                and (_ptr(x) | _ptr(w) | (_ptr(residual) or 0)) % 16 == 0):
+            return -1
+        key = (m, n, k)
+        if key not in self._tiles_rooms:
+            self._tiles_rooms[key] = library("gemm").tnx_gemm_bf16_tiles_workspace(m, n, k)
+        return self._tiles_rooms[key]
 
     library_direct = True   # many-rows products as calls of the vendor library itself, with what follows them
     library_tune = 1        # and its algorithms timed once: 1, for products of few rows; 2, for every product
@@ -812,20 +840,21 @@ class HipOps:
         shares = max(1, min(self.compute_units // column_blocks, k // 512))     # as the kernel shares K out
         return small or 4 * column_blocks * shares >= 3 * self.compute_units
 
-    def _library_product(self, m, n, k, w, force_tiled, scattered=False) -> bool:
+    def _library_product(self, m, n, k, w, force_tiled, scattered=False, plain=False) -> bool:
         """`scattered`: the fused projection of queries, keys and values, whose result the few-rows kernel puts in its
-        places itself (after the library's product a kernel of 6 to 7 us does that)."""
+        places itself (after the library's product a kernel of 6 to 7 us does that). `plain`: a bfloat16 result."""
         if not (self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and self.library_rows > 0
                 and m >= self.library_rows and not force_tiled and n % 8 == 0 and k % 8 == 0):
             return False
         # small matrices at up to 32 rows: one launch of ours (5 to 10 us with its epilogue) beats the
         # library's product and the epilogue after it (11 to 15 us)
-        return not (m <= 32 and n * k <= (self.fused_matrix if scattered else self.small_matrix))
+        return not (m <= 32 and n * k <= (self.fused_matrix if scattered or (plain and m <= 24) else self.small_matrix))
 
     small_matrix = 1 << 23
     # Queries, keys and values at 17 to 32 rows, us, few-rows kernel with everything in one launch against the library's
     # product and `qkv_write`: 24 rows 6,144 x 2,048 11.5 / 18.9, 32 rows 12.3 / 16.4, 7,680 x 2,560 14.0 / 20.0 and
-    # 15.1 / 20.4; 12,288 x 4,096 33.7 / 33 and 38.2 / 33.6.
+    # 15.1 / 20.4; 12,288 x 4,096 33.7 / 33 and 38.2 / 33.6. The products of 17 to 24 rows with a bfloat16 result go the
+    # same way (24 rows 8,192 x 2,048 12.2 / 14.5 with the library), those of 32 have no clear winner.
     fused_matrix = 20 << 20
 
     # ---------------------------------------------------------------- attention
