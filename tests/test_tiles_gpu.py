@@ -101,3 +101,31 @@ def test_products_that_the_tiles_take(m, n, k):
     assert ops._tiles_room(m, n, k, x, w, None, False, False) >= 0
     for kw in (dict(bias=bias, act="relu"), dict(bias=bias, act="gelu"), dict(residual=res, out_f32=True), dict()):
         torch.testing.assert_close(ops.linear(x, w, **kw).float(), lib.linear(x, w, **kw).float(), rtol=1e-2, atol=2e-2)
+
+
+@pytest.mark.parametrize("tokens,top", [(1, 2), (3, 3), (8, 2), (9, 7), (32, 2), (33, 2), (16, 4)])
+@pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72)])
+@pytest.mark.parametrize("act,on", [("silu", "input"), ("relu2", "output")])
+def test_experts_of_few_pairs(tokens, top, experts, width, f, act, on):
+    """Up to 64 pairs (the blocks find theirs) and beyond, one set of waves or two, experts with no pair and with all."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    if top > experts:
+        pytest.skip("more choices than experts")
+    ops, g = HipOps(torch.bfloat16, DEV), torch.Generator(device=DEV).manual_seed(tokens * top + experts)
+    gated = act == "silu"
+    chosen = torch.stack([torch.randperm(experts, device=DEV, generator=g)[:top] for _ in range(tokens)])
+    chosen[:, 0] = experts - 1                      # one expert that every token has (perhaps twice: its rows are then added)
+    weights = torch.rand(tokens, top, device=DEV, generator=g) + 0.1
+    h = torch.randn(tokens, width, device=DEV, generator=g).bfloat16()
+    up = (torch.randn(experts, (2 if gated else 1) * f, width, device=DEV, generator=g) * width ** -0.5).bfloat16()
+    down = (torch.randn(experts, width, f, device=DEV, generator=g) * f ** -0.5).bfloat16()
+    residual = torch.randn(tokens, width, device=DEV, generator=g)
+    want = torch.zeros(tokens, width, dtype=torch.float64, device=DEV)
+    for t in range(tokens):
+        for c in range(top):
+            e, s, x = int(chosen[t, c]), weights[t, c].double(), h[t].double()
+            z = up[e].double() @ (x * s if on == "input" else x)
+            y = down[e].double() @ _act(act, z[:f], z[f:], None)
+            want[t] += y if on == "input" else s * y
+    got = ops.expert_mixture(h, chosen.int().contiguous(), weights, up, down, act, on, residual)
+    assert _apart(got - residual, want) < 2.0 ** -8

@@ -190,6 +190,7 @@ struct ProductArgs {
   int experts, top, n, k, act, weight_on_input, pairs;
   float limit;              // of the clamped activation
   int direct;               // DOWN: pair rows are the tokens' rows of the result, and take the residual
+  const int* chosen;        // [pairs], up to 64 pairs: the blocks find an expert's pairs in it themselves (no `first`, `order`)
 };
 
 template <typename T, int KIND>
@@ -279,8 +280,11 @@ __global__ void __launch_bounds__(256) expert_product_kernel(ProductArgs p) {
 // by side (512 bytes or more a row and instruction, marked as read once), all of a chunk's loads under way
 // together, and takes the operands from there; the pairs' rows come from the caches. The waves of a block never
 // wait for one another.
-template <int KIND>
-__global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p) {
+// PARTS: the waves of a block come in so many sets of four, each with its part of K; the sets' sums meet in LDS. Where a step
+// is a few tokens an expert has one tile and a unit one block: with two sets there are twice as many loads under way, and half
+// as many chunks one after the other (measured at `launch_products`).
+template <int KIND, int PARTS>
+__global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(ProductArgs p) {
   constexpr bool GATED = KIND == UP_GATED, UP = KIND != DOWN;
   constexpr int TM = 16;
   constexpr int ROWS = GATED ? 32 : 16;                   // rows of the matrix a wave holds
@@ -288,25 +292,39 @@ __global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p)
   constexpr int LD = KC + 8;                              // a row in LDS: 16 bytes more, so that rows lie in different banks
   constexpr int LPR = KC / 8, RPI = 64 / LPR;             // lanes a row, rows an instruction
   constexpr int LOADS = ROWS / RPI;
-  __shared__ __attribute__((aligned(16))) bf16_t staged[4][ROWS * LD];
-  int tile = blockIdx.y, e = 0, begin = 0, end = 0;
-  for (; e < p.experts; ++e) {
-    begin = p.first[e];
-    end = p.first[e + 1];
-    const int tiles = (end - begin + TM - 1) / TM;
-    if (tile < tiles) break;
-    tile -= tiles;
-  }
-  if (e >= p.experts) return;
-  begin += tile * TM;
-  const int count = min(TM, end - begin);
+  extern __shared__ __attribute__((aligned(16))) bf16_t staged[];     // [4 PARTS][ROWS * LD]
+  __shared__ int pairs_of[64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-  const int col0 = (blockIdx.x * 4 + wave) * 16;
-  if (col0 >= p.n) return;
-  const int pair = r < count ? p.order[begin + r] : -1;
+  const int part = wave >> 2, col0 = (blockIdx.x * 4 + (wave & 3)) * 16;
+  int e = 0, pair;
+  if (p.chosen) {
+    // block y is tile y / experts of expert y % experts: its pairs are the lanes whose choice it is
+    e = blockIdx.y % p.experts;
+    const bool its = lane < p.pairs && p.chosen[min(lane, p.pairs - 1)] == e;
+    const unsigned long long all = __ballot(its);
+    const int begin = blockIdx.y / p.experts * TM;
+    if (__popcll(all) <= begin) return;
+    // (every wave writes the same numbers; a wave's LDS operations keep their order)
+    if (its) pairs_of[__popcll(all & ((1ull << lane) - 1))] = lane;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    pair = begin + r < __popcll(all) ? pairs_of[begin + r] : -1;
+  } else {
+    int tile = blockIdx.y, begin = 0, end = 0;
+    for (; e < p.experts; ++e) {
+      begin = p.first[e];
+      end = p.first[e + 1];
+      const int tiles = (end - begin + TM - 1) / TM;
+      if (tile < tiles) break;
+      tile -= tiles;
+    }
+    if (e >= p.experts) return;
+    begin += tile * TM;
+    pair = begin + r < end ? p.order[begin + r] : -1;
+  }
+  const float weight = pair >= 0 ? p.weights[pair] : 0.f;
   const bf16_t* xrow = (const bf16_t*)p.a + (size_t)(pair < 0 ? 0 : (UP ? pair / p.top : pair)) * p.k;
   const bf16_t* W = (const bf16_t*)p.w + (size_t)e * (GATED ? 2 : 1) * p.n * p.k;
-  bf16_t* mine = staged[wave];
+  bf16_t* mine = staged + wave * (ROWS * LD);
   const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
   // load i of a chunk: row RPI i + lane / LPR of the wave's rows (the up rows behind the gate rows), elements 8 (lane % LPR) on
   const int lrow = lane / LPR, lcol = 8 * (lane % LPR);
@@ -317,6 +335,8 @@ __global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p)
     const int n = col0 + (row & 15);
     src[i] = n < p.n ? W + ((size_t)(row >> 4) * p.n + n) * p.k + lcol : nullptr;
   }
+  const int chunks = (p.k + KC - 1) / KC, per = (chunks + PARTS - 1) / PARTS;
+  const int k_begin = part * per * KC, k_end = min(p.k, k_begin + per * KC);
   f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acc_up = {0.f, 0.f, 0.f, 0.f};
   // a chunk's rows and the pair's elements that meet them are asked for while the chunk before is multiplied
   constexpr int STEPS = KC / 32;
@@ -330,14 +350,14 @@ __global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p)
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) got[i] = (src[i] != nullptr && k0 + lcol < p.k) ? load_once(src[i] + k0) : zero8;
   };
-  ask(0);
-  for (int k0 = 0; k0 < p.k; k0 += KC) {
+  if (k_begin < k_end) ask(k_begin);
+  for (int k0 = k_begin; k0 < k_end; k0 += KC) {
     bf16x8 x[STEPS];
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) x[s] = x_next[s];
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) *(bf16x8*)(mine + (RPI * i + lrow) * LD + lcol) = got[i];
-    if (k0 + KC < p.k) ask(k0 + KC);
+    if (k0 + KC < k_end) ask(k0 + KC);
 #pragma unroll
     for (int s = 0; s < STEPS; ++s) {
       if (k0 + 32 * s >= p.k) break;
@@ -350,25 +370,64 @@ __global__ void __launch_bounds__(256) expert_product_mfma_kernel(ProductArgs p)
       }
     }
   }
+  if (PARTS > 1) {
+    // the later sets leave their sums in their own place in LDS, the first adds them in their order
+    if (part > 0) {
+      ((f32x4*)mine)[lane] = acc;
+      if (GATED) ((f32x4*)mine)[64 + lane] = acc_up;
+    }
+    __syncthreads();
+    if (part > 0) return;
+#pragma unroll
+    for (int q = 1; q < PARTS; ++q) {
+      const f32x4* theirs = (const f32x4*)(staged + (wave + 4 * q) * (ROWS * LD));
+      acc += theirs[lane];
+      if (GATED) acc_up += theirs[64 + lane];
+    }
+  }
   if (pair < 0) return;
-  const float w = p.weights[pair];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int col = col0 + 4 * g + i;        // the lane holds columns 4 g .. 4 g + 3 of pair r
     if (col >= p.n) continue;
     if (GATED) {
       float gt = acc[i], up = acc_up[i];
-      if (p.weight_on_input) gt *= w, up *= w;
+      if (p.weight_on_input) gt *= weight, up *= weight;
       ((bf16_t*)p.out)[(size_t)pair * p.n + col] = (bf16_t)gated(gt, up, p.act, p.limit);
     } else if (UP) {
       ((bf16_t*)p.out)[(size_t)pair * p.n + col] = (bf16_t)apply_act(acc[i], p.act);
     } else {
       float y = acc[i];
-      if (!p.weight_on_input) y *= w;
+      if (!p.weight_on_input) y *= weight;
       if (p.direct && p.residual) y += p.residual[(size_t)pair * p.n + col];
       ((float*)p.out)[(size_t)pair * p.n + col] = y;
     }
   }
+}
+
+template <int KIND, int PARTS>
+int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
+  constexpr int bytes = 4 * PARTS * (KIND == UP_GATED ? 32 : 16) * (256 + 8) * 2;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void*)expert_product_mfma_kernel<KIND, PARTS>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "expert products: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  expert_product_mfma_kernel<KIND, PARTS><<<grid, 256 * PARTS, bytes, stream>>>(p);
+  return 0;
+}
+
+// Two sets of waves where K has two chunks for each and the blocks that find pairs are at most one a unit. Measured at two
+// choices among 8 experts, us a layer with one set and with two: 2,048 wide, 1 token 45.6 / 34.8, 8 tokens 56.2 / 47.1 (256
+// blocks), 32 tokens 56.4 / 49.4; 4,096 wide, 1 token (128 blocks) 75.1 / 61.6, 2 tokens (256) 89.5 / 89.6, 8 tokens (512)
+// 150.7 / 166.0.
+template <int KIND>
+int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
+  const long long blocks = (long long)grid.x * min(p.experts, p.pairs);
+  return p.k >= 1024 && blocks <= tnx_compute_units() ? launch_products<KIND, 2>(p, grid, stream)
+                                                       : launch_products<KIND, 1>(p, grid, stream);
 }
 
 // ---------------------------------------------------------------- many pairs an expert
@@ -592,14 +651,22 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
   TNX_REQUIRE(!identity || !weight_on_input, "expert_mixture: experts without tensors take their weight on the output");
   if (tokens == 0) return 0;
   const int pairs = tokens * top;
-  order_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(chosen, pairs, experts, first, order, nullptr, nullptr,
-                                                               top, nullptr, nullptr, nullptr, 0, 0);
-  TNX_CHECK_LAUNCH("expert order");
-  const int tiles = pairs / 16 + experts;       // the most tiles of 16 pairs: every expert may end in a part of one
+  const bool mfma = dtype == TNX_BF16 && width % 8 == 0 && f % 8 == 0 && !plain;
+  // Up to 64 pairs the products' blocks find their pairs themselves (a wave holds all choices), which saves the launch that
+  // orders them (3 to 4 us); a tile of 16 pairs an expert for every 16 pairs then, most of them empty.
+  const bool found = mfma && pairs <= 64 && (long long)experts * ((pairs + 15) / 16) <= 4096;
+  if (!found) {
+    order_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(chosen, pairs, experts, first, order, nullptr, nullptr, top,
+                                                                 nullptr, nullptr, nullptr, 0, 0);
+    TNX_CHECK_LAUNCH("expert order");
+  }
+  // the most tiles of 16 pairs: every expert may end in a part of one
+  const int tiles = found ? experts * ((pairs + 15) / 16) : pairs / 16 + experts;
+  const int* look = found ? chosen : nullptr;
   ProductArgs up{h, w_gate_up, first, order, weights, nullptr, inner, experts, top, f, width, act, weight_on_input, pairs,
-                 limit, 0};
+                 limit, 0, look};
   ProductArgs down{inner, w_down, first, order, weights, residual, direct ? out : pair_rows, experts, top, width, f,
-                   act, weight_on_input, pairs, limit, direct ? 1 : 0};
+                   act, weight_on_input, pairs, limit, direct ? 1 : 0, look};
   const dim3 grid_up((f + 63) / 64, tiles), grid_down((width + 63) / 64, tiles);
   if (dtype == TNX_F32) {
     if (ungated)
@@ -607,12 +674,9 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
     else
       expert_product_kernel<float, UP_GATED><<<grid_up, 256, 0, stream>>>(up);
     expert_product_kernel<float, DOWN><<<grid_down, 256, 0, stream>>>(down);
-  } else if (width % 8 == 0 && f % 8 == 0 && !plain) {
-    if (ungated)
-      expert_product_mfma_kernel<UP_PLAIN><<<grid_up, 256, 0, stream>>>(up);
-    else
-      expert_product_mfma_kernel<UP_GATED><<<grid_up, 256, 0, stream>>>(up);
-    expert_product_mfma_kernel<DOWN><<<grid_down, 256, 0, stream>>>(down);
+  } else if (mfma) {
+    if (int rc = ungated ? launch_products<UP_PLAIN>(up, grid_up, stream) : launch_products<UP_GATED>(up, grid_up, stream)) return rc;
+    if (int rc = launch_products<DOWN>(down, grid_down, stream)) return rc;
   } else {
     if (ungated)
       expert_product_kernel<bf16_t, UP_PLAIN><<<grid_up, 256, 0, stream>>>(up);
