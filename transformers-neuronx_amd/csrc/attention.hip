@@ -2067,11 +2067,15 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
     attention_decode_mfma_kernel<NDB, 4, true><<<grid, 256, 0, stream>>>(MFMA_ARGS);             \
   else                                                                                           \
     attention_decode_mfma_kernel<NDB, 4, false><<<grid, 256, 0, stream>>>(MFMA_ARGS)
-    // the registers are laid out for the next of these sizes; a smaller head repeats its last chunk there
+    // the registers are laid out for the next of these sizes; a smaller head repeats its last chunk there. 80 has a size
+    // of its own: laid out for 96 it reads its last sixth twice, 34.1 us against 34.8 for 32 requests of up to 700 tokens
+    // and 32 heads, 23.2 against 23.8 for 24 of them, 37.0 against 37.3 for 8 of 2,048.
     if (head_size <= 32) {
       LAUNCH_MFMA(2);
     } else if (head_size <= 64) {
       LAUNCH_MFMA(4);
+    } else if (head_size <= 80) {
+      LAUNCH_MFMA(5);
     } else if (head_size <= 96) {
       LAUNCH_MFMA(6);
     } else if (head_size <= 128) {
