@@ -5,6 +5,8 @@
 // Everything is float32. The state lies in two places by the parity of the position: the token at position p
 // reads place (p - 1) & 1 (nothing at p = 0) and writes place p & 1, so a step of single tokens that is run
 // twice reads the same both times.
+#include <type_traits>
+
 #include "common.h"
 
 TNX_DEFINE_ERROR_API
@@ -21,7 +23,8 @@ struct CellArgs {
   float* normalizer;      // [slots, 2, H, n]
   float* peak;            // [slots, 2, H]
   float* out;             // [T, H v], before the norm
-  int heads, n, v;
+  int heads, n, v, tokens;
+  int chunk_from;         // runs of so many tokens go by chunks, shorter ones token by token
   float cap, q_scale;
 };
 
@@ -58,13 +61,18 @@ __device__ __forceinline__ f32x4 load4(const float* p, int valid) {      // the 
   return r;
 }
 
-// grid: requests * heads blocks of one wave; 64 tokens a round, a token a lane, the running maximum a chain of
-// lane 0 between two rounds of side-by-side work.
-__global__ void __launch_bounds__(64) memory_gates_kernel(CellArgs a, float* __restrict__ keeps, float* __restrict__ takes,
-                                                          float* __restrict__ floors, float* __restrict__ aside) {
-  __shared__ float gis[64], gfs[64], ms[65];
+// grid: requests * heads blocks of W waves; W 64 tokens a round, a token a lane. The running maximum is a chain
+// m' = max(f + m, i) whose steps join: two neighbouring spans (F, I), m -> max(F + m, I), make one of
+// (F1 + F2, max(I1 + F2, I2)). A wave joins its lanes' steps in six rounds, the waves before it hand it their spans, and
+// every token's m is known at once. (Which m the state is scaled by is free as long as a token's factors name the same m
+// on both sides; the joined one differs from the chain's by roundings only.) 2,048 tokens, 32 heads: 102 us with a chain of
+// one lane over 64 tokens a round, 10 us so.
+template <int W>
+__global__ void __launch_bounds__(64 * W) memory_gates_kernel(CellArgs a, float* __restrict__ keeps, float* __restrict__ takes,
+                                                              float* __restrict__ floors, float* __restrict__ aside) {
+  __shared__ float spans[2][W][2];
   const int r = blockIdx.x / a.heads, head = blockIdx.x - r * a.heads;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int start = a.run_start[r], count = a.run_start[r + 1] - start;
   const int have = a.cached[r], slot = a.slots[r];
   const int hn = a.heads * a.n, hv = a.heads * a.v;
@@ -74,43 +82,295 @@ __global__ void __launch_bounds__(64) memory_gates_kernel(CellArgs a, float* __r
   {
     const float* np_ = a.normalizer + (head_at + (size_t)from * a.heads) * a.n;
     float* out = aside + (size_t)blockIdx.x * a.n;
-    for (int d = lane; d < a.n; d += 64) out[d] = have > 0 ? np_[d] : 0.f;
+    for (int d = threadIdx.x; d < a.n; d += 64 * W) out[d] = have > 0 ? np_[d] : 0.f;
   }
   float m = have > 0 ? a.peak[head_at + (size_t)from * a.heads] : 0.f;
-  for (int t0 = 0; t0 < count; t0 += 64) {
-    const int len = min(64, count - t0);
-    if (lane < len) {
-      const float* row = a.proj + (size_t)(start + t0 + lane) * a.ld + 2 * hn + 2 * hv;
-      gis[lane] = a.cap * tanhf(row[head] / a.cap);
-      gfs[lane] = log_sigmoid(a.cap * tanhf(row[a.heads + head] / a.cap));
+  int turn = 0;
+  for (int t0 = 0; t0 < count; t0 += 64 * W, turn ^= 1) {
+    const int t = t0 + threadIdx.x;
+    float gi = -INFINITY, gf = 0.f;               // (behind the run's end: a step that changes nothing)
+    if (t < count) {
+      const float* row = a.proj + (size_t)(start + t) * a.ld + 2 * hn + 2 * hv;
+      gi = a.cap * tanhf(row[head] / a.cap);
+      gf = log_sigmoid(a.cap * tanhf(row[a.heads + head] / a.cap));
     }
-    __syncthreads();
-    if (lane == 0) {
-      // (what the chain reads from LDS is read before it begins: a store into LDS between two loads would keep the
-      // second load from being under way with the first)
-      float gi_r[64], gf_r[64], after[64], peak = m;
+    float F = gf, I = gi;
 #pragma unroll
-      for (int t = 0; t < 64; ++t) gi_r[t] = t < len ? gis[t] : 0.f, gf_r[t] = t < len ? gfs[t] : 0.f;
-#pragma unroll
-      for (int t = 0; t < 64; ++t) after[t] = peak = t < len ? fmaxf(gf_r[t] + peak, gi_r[t]) : peak;
-      ms[0] = m;                                    // ms[t + 1]: the maximum after token t
-#pragma unroll
-      for (int t = 0; t < 64; ++t)
-        if (t < len) ms[t + 1] = after[t];
+    for (int off = 1; off < 64; off *= 2) {
+      const float F0 = __shfl_up(F, off), I0 = __shfl_up(I, off);
+      if (lane >= off) I = fmaxf(I0 + F, I), F = F0 + F;
     }
-    __syncthreads();
-    if (lane < len) {
-      const size_t at = (size_t)(start + t0 + lane) * a.heads + head;
-      keeps[at] = expf(gfs[lane] + ms[lane] - ms[lane + 1]);
-      takes[at] = expf(gis[lane] - ms[lane + 1]);
-      floors[at] = expf(-ms[lane + 1]);
+    float next = m;
+    if (W > 1) {
+      if (lane == 63) spans[turn][wave][0] = F, spans[turn][wave][1] = I;
+      __syncthreads();                            // (two places in turn: the next round writes the other)
+#pragma unroll
+      for (int w = 0; w < W; ++w) {
+        if (w == wave) m = next;
+        next = fmaxf(spans[turn][w][0] + next, spans[turn][w][1]);
+      }
     }
-    m = ms[len];
-    __syncthreads();
+    const float after = fmaxf(F + m, I);
+    float before = __shfl_up(after, 1);
+    if (lane == 0) before = m;
+    if (t < count) {
+      const size_t at = (size_t)head * a.tokens + start + t;
+      keeps[at] = expf(gf + before - after);
+      takes[at] = expf(gi - after);
+      floors[at] = expf(-after);
+    }
+    m = W > 1 ? next : __shfl(after, 63);
   }
-  if (lane == 0) a.peak[head_at + (size_t)to * a.heads] = m;
+  if (threadIdx.x == 0) a.peak[head_at + (size_t)to * a.heads] = m;
 }
 
+// ---------------------------------------------------------------- runs by chunks
+// Within a chunk of 64 tokens the recurrence is a sum, on the float32 matrix instructions: with P_t the product of the
+// chunk's keeps up to token t and D_tj that of the keeps behind token j up to t, times token j's take,
+//     S_t^T q_t = P_t S_0^T q_t + sum_{j <= t} (q_t . k_j) D_tj val_j,      S_64 = P_63 S_0 + sum_j D_63,j k_j val_j^T,
+// and the same with 1 for val_j for the normalizer. The products of keeps are made token by token, as the walk makes them:
+// nothing is divided and no logarithms are subtracted. `memory_weights_kernel` makes (q_t . k_j) D_tj, P_t and D_63,j for all
+// chunks side by side; `memory_chunks_kernel` goes through a run's chunks with 16 columns of S a block. The walk is a chain
+// of a few multiply-adds and four lane exchanges a token, whatever the matrix units could do. 2,048 tokens, 32 heads of 64
+// rows and 128 columns: 399 us by the walk, 132 us by chunks: 19 for the weights and
+// 113 for the chunks (3.5 us each, of which the matrix instructions take 0.65: one block of four waves a unit, which waits
+// for its operands). Against 64 bits: 4.2e-7 by the walk, 3.2e-7 by chunks.
+// (A token whose projections are not finite makes the chunk's earlier tokens not finite as well, not its later ones only.)
+typedef float f32x4v __attribute__((ext_vector_type(4)));
+
+// Chunk `b` of all chunks of 64 tokens of the runs that go by chunks: its run and its first token in it; false: there are fewer.
+__device__ __forceinline__ bool find_chunk(const CellArgs& a, int requests, int b, int* run, int* first) {
+  for (int r = 0; r < requests; ++r) {
+    const int count = a.run_start[r + 1] - a.run_start[r], chunks = count >= a.chunk_from ? (count + 63) >> 6 : 0;
+    if (b < chunks) {
+      *run = r, *first = 64 * b;
+      return true;
+    }
+    b -= chunks;
+  }
+  return false;
+}
+
+// grid: (chunks, heads), four waves. Wave w makes rows 16 w to 16 w + 15 of the chunk's [64, 64] weights: its 16 queries
+// against the keys up to its last row. The factors D: lane j carries token j's through the tokens, a multiplication each.
+// weights [H, T, 64], prefix and last [H, T]. NT: 16 NT rows of S hold n.
+template <int NT, bool ALIGNED>
+__global__ void __launch_bounds__(256) memory_weights_kernel(CellArgs a, int requests, const float* __restrict__ keeps,
+                                                             const float* __restrict__ takes, float* __restrict__ weights,
+                                                             float* __restrict__ prefix, float* __restrict__ last) {
+  constexpr int KD = 4 * NT;                        // elements of a query that a quarter of the lanes holds
+  __shared__ float decays[4][16][68];
+  int r, c0;
+  if (!find_chunk(a, requests, blockIdx.x, &r, &c0)) return;
+  const int head = blockIdx.y, lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
+  const int start = a.run_start[r] + c0, len = min(64, a.run_start[r + 1] - start);
+  const size_t at = (size_t)head * a.tokens + start;
+  const int hn = a.heads * a.n;
+  const float keep = lane < len ? keeps[at + lane] : 1.f, take = lane < len ? takes[at + lane] : 0.f;
+  const float* queries = a.proj + (size_t)start * a.ld + head * a.n + g * KD;
+  f32x4v acc[4] = {};
+  if (16 * wave < len) {
+    f32x4 q[NT];
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+      q[s] = load4<ALIGNED>(queries + (size_t)min(16 * wave + li, len - 1) * a.ld + 4 * s, a.n - g * KD - 4 * s);
+#pragma unroll
+    for (int jb = 0; jb < 4; ++jb)
+      if (jb <= wave) {
+        f32x4 k[NT];
+#pragma unroll
+        for (int s = 0; s < NT; ++s)
+          k[s] = load4<ALIGNED>(queries + hn + (size_t)min(16 * jb + li, len - 1) * a.ld + 4 * s, a.n - g * KD - 4 * s);
+#pragma unroll
+        for (int s = 0; s < KD; ++s) acc[jb] = __builtin_amdgcn_mfma_f32_16x16x4f32(q[s / 4][s % 4], k[s / 4][s % 4], acc[jb], 0, 0, 0);
+      }
+  }
+  float D = 0.f, P = 1.f;
+  for (int tb = 0; tb <= wave; ++tb) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int t = 16 * tb + i;
+      const float k = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(keep), t));
+      D = lane == t ? take : D * k;
+      P = lane >= t ? P * k : P;
+      if (tb == wave) decays[wave][i][lane] = D;
+    }
+  }
+  if (wave == 3 && lane < len) prefix[at + lane] = P, last[at + lane] = D;
+  __syncthreads();
+#pragma unroll
+  for (int jb = 0; jb < 4; ++jb)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int i = 4 * g + e, t = 16 * wave + i, j = 16 * jb + li;
+      if (t < len) weights[(at + t) * 64 + j] = j <= t ? acc[jb][e] * a.q_scale * decays[wave][i][j] : 0.f;
+    }
+}
+
+// grid: requests * heads * column blocks of 16, four waves. In a chunk wave w makes the outputs of tokens 16 w to 16 w + 15
+// and carries rows 16 (w + 4 u) on of S; S as the chunk begins goes round through LDS, in two places in turn, so that a chunk
+// has one barrier. Every other operand comes straight from memory in the matrix instruction's own order (a quarter of the
+// lanes takes a contiguous quarter of the summed index), a chunk ahead.
+template <int NT, bool ALIGNED>
+__global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(CellArgs a, const float* __restrict__ weights,
+                                                            const float* __restrict__ prefix, const float* __restrict__ last,
+                                                            const float* __restrict__ floors, const float* __restrict__ aside,
+                                                            int column_blocks) {
+  constexpr int KD = 4 * NT, NU = NT / 4;
+  __shared__ float begins[2][16 * NT * 16 + 64];          // S [row][column]; 16 places more after every quarter of the rows
+  __shared__ __attribute__((aligned(16))) float norms[2][16 * NT];
+  // A head's queries, keys and weights are read by all its column blocks: eight heads at a time, one an XCD, so that they
+  // come into one L2 once. (Blocks go round the XCDs in their order; heads beyond the last eight take theirs as they come.)
+  const int heads_by_xcd = gridDim.x / column_blocks & ~7, y = blockIdx.x >> 3;
+  const bool by_xcd = blockIdx.x < heads_by_xcd * column_blocks;
+  const int cb = (by_xcd ? y : blockIdx.x) % column_blocks;
+  const int rh = by_xcd ? 8 * (y / column_blocks) + (blockIdx.x & 7) : blockIdx.x / column_blocks;
+  const int r = rh / a.heads, head = rh - r * a.heads;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 15, g = lane >> 4;
+  const int start = a.run_start[r], count = a.run_start[r + 1] - start;
+  const int have = a.cached[r], slot = a.slots[r];
+  const int hn = a.heads * a.n, hv = a.heads * a.v;
+  if (count < a.chunk_from) return;
+  const int col = 16 * cb + li;
+  const bool col_ok = col < a.v;
+  const int from = (have - 1) & 1, to = (have + count - 1) & 1;
+  const size_t head_at = (size_t)slot * 2 * a.heads + head;        // + place * heads
+  f32x4v S[NU];
+  float nrm[NU];                                                   // row 16 (wave + 4 u) + li, the same in all quarters
+  {
+    const float* Sp = a.memory + ((head_at + (size_t)from * a.heads) * a.v + (col_ok ? col : 0)) * a.n;
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int d0 = 16 * (wave + 4 * u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = d0 + 4 * g + e;
+        S[u][e] = (have > 0 && d < a.n && col_ok) ? Sp[d] : 0.f;
+      }
+      nrm[u] = d0 + li < a.n ? aside[(size_t)rh * a.n + d0 + li] : 0.f;
+    }
+  }
+  f32x4 q[NT], w[4];
+  float k[NU][16], v[16], ends[16], mine, floor_, keep;
+  // (every load is made, of the run's last token's row behind its end and of the first column or row of S beyond the last
+  // one: what they bring is multiplied by a weight of zero or belongs to places that are not stored. A whole chunk's rows
+  // are a fixed distance apart.)
+  const int vcol = 2 * hn + head * a.v + (col_ok ? col : 0);
+  int krow[NU];
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int d = 16 * (wave + 4 * u) + li;
+    krow[u] = hn + head * a.n + (d < a.n ? d : 0);
+  }
+  auto fetch_rows = [&](int c0, int len, auto whole) __attribute__((always_inline)) {
+    const size_t at = (size_t)head * a.tokens + start + c0;
+    const float* rows = a.proj + (size_t)(start + c0) * a.ld;
+    const int t = whole ? 16 * wave + li : min(16 * wave + li, len - 1);
+#pragma unroll
+    for (int s = 0; s < NT; ++s)
+      q[s] = load4<ALIGNED>(rows + (size_t)t * a.ld + head * a.n + g * KD + 4 * s, a.n - g * KD - 4 * s);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) w[s] = *(const f32x4*)(weights + (at + t) * 64 + 16 * g + 4 * s);
+    mine = prefix[at + t], floor_ = floors[at + t], keep = prefix[at + len - 1];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      const int j = whole ? 16 * g + s : min(16 * g + s, len - 1);
+      const float* row = whole ? rows + (size_t)s * a.ld + 16 * g * a.ld : rows + (size_t)j * a.ld;
+      v[s] = row[vcol];
+      ends[s] = last[at + j];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) k[u][s] = row[krow[u]];
+    }
+  };
+  auto fetch = [&](int c0) __attribute__((always_inline)) {
+    const int len = count - c0;
+    if (len >= 64)
+      fetch_rows(c0, 64, std::true_type());
+    else
+      fetch_rows(c0, len, std::false_type());
+  };
+  fetch(0);
+  int turn = 0;
+  for (int c0 = 0; c0 < count; c0 += 64, turn ^= 1) {
+    const int len = min(64, count - c0);
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      const int d0 = 16 * (wave + 4 * u);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const int d = d0 + 4 * g + e;
+        begins[turn][16 * (d + d / KD) + li] = S[u][e];
+      }
+      if (g == 0) norms[turn][d0 + li] = nrm[u];
+    }
+    __syncthreads();
+    // this chunk's operands, made ready; then the next chunk's are asked for
+    f32x4 ww[4];
+    float qq[KD], kk[NU][16], vv[16];
+    const float scale = a.q_scale * mine, floor_now = floor_, keep_now = keep;
+#pragma unroll
+    for (int s = 0; s < KD; ++s) qq[s] = q[s / 4][s % 4] * scale;
+#pragma unroll
+    for (int s = 0; s < 4; ++s) ww[s] = w[s];
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      vv[s] = v[s];
+#pragma unroll
+      for (int u = 0; u < NU; ++u) kk[u][s] = 16 * g + s < len ? k[u][s] * ends[s] : 0.f;
+    }
+    if (c0 + 64 < count) fetch(c0 + 64);
+    f32x4v acc = {}, more = {};
+    float dot = 0.f;
+#pragma unroll
+    for (int s = 0; s < KD; ++s) {
+      const int d = g * KD + s;
+      acc = __builtin_amdgcn_mfma_f32_16x16x4f32(qq[s], begins[turn][16 * (d + g) + li], acc, 0, 0, 0);
+      dot += qq[s] * norms[turn][d];
+    }
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      more = __builtin_amdgcn_mfma_f32_16x16x4f32(ww[s / 4][s % 4], vv[s], more, 0, 0, 0);
+      dot += ww[s / 4][s % 4];
+    }
+#pragma unroll
+    for (int u = 0; u < NU; ++u) {
+      float sum = 0.f;
+      S[u] *= keep_now;
+#pragma unroll
+      for (int s = 0; s < 16; ++s) {
+        S[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[u][s], vv[s], S[u], 0, 0, 0);
+        sum += kk[u][s];
+      }
+      sum += __shfl_xor(sum, 16);
+      sum += __shfl_xor(sum, 32);
+      nrm[u] = keep_now * nrm[u] + sum;
+    }
+    dot += __shfl_xor(dot, 16);
+    dot += __shfl_xor(dot, 32);
+    // (the denominator is 1e-6 at least: its reciprocal, right to a unit in the last place, is no subnormal)
+    const float below = __builtin_amdgcn_rcpf(fmaxf(fabsf(dot), floor_now) + 1e-6f);
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int t = 16 * wave + 4 * g + e;
+      const float o = (acc[e] + more[e]) * __shfl(below, 4 * g + e);
+      if (t < len && col_ok) a.out[(size_t)(start + c0 + t) * hv + head * a.v + col] = o;
+    }
+  }
+#pragma unroll
+  for (int u = 0; u < NU; ++u) {
+    const int d0 = 16 * (wave + 4 * u);
+    if (col_ok) {
+      float* Sp = a.memory + ((head_at + (size_t)to * a.heads) * a.v + col) * a.n;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (d0 + 4 * g + e < a.n) Sp[d0 + 4 * g + e] = S[u][e];
+    }
+    if (cb == 0 && g == 0 && d0 + li < a.n)                        // the normalizer, once a head
+      a.normalizer[(head_at + (size_t)to * a.heads) * a.n + d0 + li] = nrm[u];
+  }
+}
+
+// ---------------------------------------------------------------- runs token by token
 // grid: requests * heads * column blocks; a block is four waves and 16 columns of S. In a wave the 16 lanes of a
 // row of lanes share a column (column 16 b + 4 w + lane / 16): lane % 16 holds its rows NR (lane % 16) + j, j < NR,
 // and the same rows of the normalizer; a column's sum over the rows is a sum over the 16 lanes of a row of lanes.
@@ -134,7 +394,7 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
   const int start = a.run_start[r], count = a.run_start[r + 1] - start;
   const int have = a.cached[r], slot = a.slots[r];
   const int hn = a.heads * a.n, hv = a.heads * a.v;
-  if (count <= 0) return;
+  if (count <= 0 || count >= a.chunk_from) return;
   const int col = 16 * cb + 4 * wave + (lane >> 4);
   const bool col_ok = col < a.v;
   float S[NR], nrm[NR];
@@ -161,7 +421,7 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
       const float* row = a.proj + (size_t)(start + t0 + (in ? t : 0)) * a.ld + head * a.n + d;
       rq[u] = load4<ALIGNED>(row, in ? a.n - d : 0);
       rk[u] = load4<ALIGNED>(row + hn, in ? a.n - d : 0);
-      rt[u] = in ? takes[(size_t)(start + t0 + t) * a.heads + head] : 0.f;
+      rt[u] = in ? takes[(size_t)head * a.tokens + start + t0 + t] : 0.f;
     }
     if (threadIdx.x < CH * 4) {                            // a token's 16 values: four pieces
       const int t = threadIdx.x >> 2, c = 16 * cb + 4 * (threadIdx.x & 3);
@@ -170,8 +430,8 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
     }
     if (threadIdx.x < CH) {
       const bool in = threadIdx.x < len;
-      rkeep = in ? keeps[(size_t)(start + t0 + threadIdx.x) * a.heads + head] : 1.f;
-      rfl = in ? floors[(size_t)(start + t0 + threadIdx.x) * a.heads + head] : 1.f;
+      rkeep = in ? keeps[(size_t)head * a.tokens + start + t0 + threadIdx.x] : 1.f;
+      rfl = in ? floors[(size_t)head * a.tokens + start + t0 + threadIdx.x] : 1.f;
     }
   };
   auto stash = [&]() {
@@ -286,10 +546,31 @@ void launch_cell(const CellArgs& a, const float* keeps, const float* takes, cons
     memory_cell_kernel<NR, false><<<grid, 256, 0, stream>>>(a, keeps, takes, floors, aside, column_blocks);
 }
 
+template <int NT>
+void launch_chunks(const CellArgs& a, const float* keeps, const float* takes, const float* floors, const float* aside,
+                   float* work, int requests, bool aligned, hipStream_t stream) {
+  const size_t th = (size_t)a.tokens * a.heads;
+  float *weights = work, *prefix = work + 64 * th, *last = work + 65 * th;
+  const dim3 chunks(a.tokens / 64 + requests, a.heads);
+  const int column_blocks = (a.v + 15) / 16;
+  const dim3 grid(requests * a.heads * column_blocks);
+  if (aligned) {
+    memory_weights_kernel<NT, true><<<chunks, 256, 0, stream>>>(a, requests, keeps, takes, weights, prefix, last);
+    memory_chunks_kernel<NT, true><<<grid, 256, 0, stream>>>(a, weights, prefix, last, floors, aside, column_blocks);
+  } else {
+    memory_weights_kernel<NT, false><<<chunks, 256, 0, stream>>>(a, requests, keeps, takes, weights, prefix, last);
+    memory_chunks_kernel<NT, false><<<grid, 256, 0, stream>>>(a, weights, prefix, last, floors, aside, column_blocks);
+  }
+}
+
 }  // namespace
 
+// `longest`, `shortest`: the tokens of the step's longest and shortest run. Runs of `chunk_from` tokens go by chunks
+// (query/key heads of up to 128 elements; `chunk_work`: 66 floats a token and head, 16 bytes aligned), shorter ones, and
+// all where `chunk_work` is null, token by token.
 extern "C" int tnx_matrix_memory(const float* proj, int ld, const int* run_start, const int* cached, const int* slots,
                                  float* memory, float* normalizer, float* peak, int num_slots, float* raw, float* gates,
+                                 int longest, int shortest, int chunk_from, float* chunk_work,
                                  const float* weight, float eps, void* out, int dtype, int tokens, int requests, int heads,
                                  int n, int v, float cap, hipStream_t stream) {
   TNX_REQUIRE(tokens >= 0 && requests >= 0 && heads > 0 && n > 0 && v > 0, "matrix_memory: bad sizes");
@@ -299,24 +580,41 @@ extern "C" int tnx_matrix_memory(const float* proj, int ld, const int* run_start
   TNX_REQUIRE(cap > 0.f, "matrix_memory: the gates' cap must be positive");
   TNX_REQUIRE(dtype == TNX_F32 || dtype == TNX_BF16, "matrix_memory: dtype %d", dtype);
   if (tokens == 0 || requests == 0) return 0;
-  CellArgs a{proj, ld, run_start, cached, slots, memory, normalizer, peak, raw, heads, n, v, cap, 1.f / sqrtf((float)n)};
-  float* keeps = gates;                             // [T, H] each
+  CellArgs a{proj, ld, run_start, cached, slots, memory, normalizer, peak, raw, heads, n, v, tokens,
+             chunk_work != nullptr ? (chunk_from > 1 ? chunk_from : 1) : 0x7fffffff, cap, 1.f / sqrtf((float)n)};
+  TNX_REQUIRE(chunk_work == nullptr || (n <= 128 && heads <= 65535 && (uintptr_t)chunk_work % 16 == 0),
+              "matrix_memory: by chunks: query/key heads of up to 128 elements, room at a multiple of 16 bytes");
+  float* keeps = gates;                             // [H, T] each
   float* takes = gates + (size_t)tokens * heads;
   float* floors = gates + 2 * (size_t)tokens * heads;
   float* aside = gates + 3 * (size_t)tokens * heads;      // [R, H, n]: the normalizers the runs begin with
   // rows and heads that begin at multiples of 16 bytes are loaded 16 bytes at a time
   const bool aligned = n % 4 == 0 && v % 4 == 0 && ld % 4 == 0 && (uintptr_t)proj % 16 == 0;
-  memory_gates_kernel<<<requests * heads, 64, 0, stream>>>(a, keeps, takes, floors, aside);
+  // as many waves as the longest run fills
+  if (longest <= 64)
+    memory_gates_kernel<1><<<requests * heads, 64, 0, stream>>>(a, keeps, takes, floors, aside);
+  else if (longest <= 256)
+    memory_gates_kernel<4><<<requests * heads, 256, 0, stream>>>(a, keeps, takes, floors, aside);
+  else
+    memory_gates_kernel<16><<<requests * heads, 1024, 0, stream>>>(a, keeps, takes, floors, aside);
   TNX_CHECK_LAUNCH("matrix_memory gates");
   const int rows16 = (n + 15) / 16;
-  if (rows16 <= 2)
-    launch_cell<2>(a, keeps, takes, floors, aside, requests, aligned, stream);
-  else if (rows16 <= 4)
-    launch_cell<4>(a, keeps, takes, floors, aside, requests, aligned, stream);
-  else if (rows16 <= 8)
-    launch_cell<8>(a, keeps, takes, floors, aside, requests, aligned, stream);
-  else
-    launch_cell<16>(a, keeps, takes, floors, aside, requests, aligned, stream);
+  if (longest >= a.chunk_from) {
+    if (rows16 <= 4)
+      launch_chunks<4>(a, keeps, takes, floors, aside, chunk_work, requests, aligned, stream);
+    else
+      launch_chunks<8>(a, keeps, takes, floors, aside, chunk_work, requests, aligned, stream);
+  }
+  if (shortest < a.chunk_from) {
+    if (rows16 <= 2)
+      launch_cell<2>(a, keeps, takes, floors, aside, requests, aligned, stream);
+    else if (rows16 <= 4)
+      launch_cell<4>(a, keeps, takes, floors, aside, requests, aligned, stream);
+    else if (rows16 <= 8)
+      launch_cell<8>(a, keeps, takes, floors, aside, requests, aligned, stream);
+    else
+      launch_cell<16>(a, keeps, takes, floors, aside, requests, aligned, stream);
+  }
   TNX_CHECK_LAUNCH("matrix_memory");
   const int pairs = tokens * heads;
   const int gate_at = 2 * heads * n + heads * v;

@@ -143,8 +143,8 @@ _SIGNATURES = {
     },
     "memory": {
         "tnx_matrix_memory": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
-                              _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
-                              _c_int, _c_float, _c_void_p],
+                              _c_int, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_float, _c_void_p,
+                              _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_float, _c_void_p],
     },
     "experts": {
         "tnx_route": [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float,
@@ -1772,6 +1772,14 @@ class HipOps:
 
     # ---------------------------------------------------------------- the matrix memory
 
+    # Runs of so many tokens go through the matrix memory by chunks of 64 (query/key heads of up to 128 elements), shorter
+    # ones token by token. us a layer of 32 heads of 64 rows, token by token / by chunks: 128 columns, one run of 24 tokens
+    # 15.6 / 17.8, 48: 19.7 / 19.0, 210: 56 / 34, 2,048: 426 / 159, eight runs of 48 58 / 49; 64 columns, 24: 14.7 / 16.8, 48:
+    # 18.8 / 18.0, 24 runs of 32 53 / 64. A step with shorter runs as well takes both ways, from a longer run on: beside 40
+    # runs of one token, 128 tokens 69 / 81, 600: 187 / 133.
+    memory_chunk_run = 48
+    memory_chunk_run_beside = 256
+
     def matrix_memory(self, proj, num_heads, head_size, value_size, gate_cap, eps, norm_weight, ctx, memory, normalizer,
                       peak):
         """See `ReferenceOps.matrix_memory`."""
@@ -1787,10 +1795,16 @@ class HipOps:
         raw = torch.empty(t, h * v, dtype=torch.float32, device=proj.device)
         # two factors and a floor a token, and the normalizer every run begins with
         gates = torch.empty(3 * t * h + ctx.num_requests * h * n, dtype=torch.float32, device=proj.device)
+        longest = ctx.max_run
+        shortest = int(ctx.run_lens_host.min())
+        by_chunks = n <= 128 and longest >= (self.memory_chunk_run if shortest >= self.memory_chunk_run
+                                             else self.memory_chunk_run_beside)
+        room = torch.empty(66 * t * h, dtype=torch.float32, device=proj.device) if by_chunks else None
         out = torch.empty(t, h * v, dtype=self.dtype, device=proj.device)
         state = float(ctx.num_requests) * h * n * v * 8
         self._call("memory", "tnx_matrix_memory", _ptr(proj), total, _ptr(ctx.run_start), _ptr(ctx.cached_lens),
-                   _ptr(ctx.slots), _ptr(memory), _ptr(normalizer), _ptr(peak), slots, _ptr(raw), _ptr(gates), _ptr(norm_weight),
+                   _ptr(ctx.slots), _ptr(memory), _ptr(normalizer), _ptr(peak), slots, _ptr(raw), _ptr(gates), longest,
+                   shortest, self.memory_chunk_run, _ptr(room), _ptr(norm_weight),
                    float(eps), _ptr(out), _code(self.dtype), t, ctx.num_requests, h, n, v, float(gate_cap), _stream(),
                    work=lambda: (f"{t} tokens {ctx.num_requests} runs", state + t * total * 4.0, 4.0 * t * h * n * v))
         return out
