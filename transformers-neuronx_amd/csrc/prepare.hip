@@ -35,6 +35,14 @@ struct PrepareArgs {
   const float* head_scale;  // [H] or null: a query head's elements times its number, beside `scale`
   float temp_coef;          // the queries of position p times 1 + temp_coef ln(floor((p + 1) / temp_every) + 1)
   int temp_every;           // 0: not
+  int tokens;
+  int fours;                // four neighbouring elements of the queries and keys a thread
+};
+
+typedef float f32x4p __attribute__((ext_vector_type(4)));
+template <typename T>
+struct Four {
+  typedef T type __attribute__((ext_vector_type(4)));
 };
 
 // what the token's queries are multiplied by, beside a head's own number
@@ -68,31 +76,81 @@ __device__ __forceinline__ float turned(const float* x, const float* w, float r,
   return first ? own * c - mate * s : own * c + mate * s;
 }
 
-// grid: (tokens, 3, shares): a block takes a share of a token's queries, keys or values; each of the three needs nothing
-// of the other two. (A norm over the whole projection is summed up by every block that shares it.)
+// Elements `e` to `e + 3` of head `head`, likewise (`fours`: turned by halves of a multiple of four elements, or not at all).
+__device__ __forceinline__ f32x4p turned4(const float* x, const float* w, float r, int head, int e, const PrepareArgs& a,
+                                          const float* cosines, const float* sines) {
+  const int at = head * a.n + e;
+  f32x4p own = *(const f32x4p*)(x + at) * r;
+  if (w) own *= *(const f32x4p*)(w + at);
+  if (a.freqs == nullptr || e >= 2 * a.half) return own;
+  const bool first = e < a.half;
+  const int i = first ? e : e - a.half, oat = first ? at + a.half : at - a.half;
+  f32x4p mate = *(const f32x4p*)(x + oat) * r;
+  if (w) mate *= *(const f32x4p*)(w + oat);
+  const f32x4p s = *(const f32x4p*)(sines + i), c = *(const f32x4p*)(cosines + i);
+  return first ? own * c - mate * s : own * c + mate * s;
+}
+
+// What a value's place in the cache holds: element `i` of `groups * d` of token `t`.
+__device__ __forceinline__ float value_of(const PrepareArgs& a, int t, int i, float lam) {
+  const int g = i / a.d, e = i - g * a.d;
+  if (e >= a.v) return 0.f;
+  const float val = a.proj[(size_t)t * a.ld + a.values_at + g * a.v + e];
+  return a.first != nullptr ? (1.f - lam) * val + lam * a.first[(size_t)t * a.first_ld + g * a.v + e] : val;
+}
+
+// Values of many tokens: a page holds an element's values of all its tokens side by side, so 64 tokens of 64 elements go
+// through LDS and a wave stores 64 tokens of one element. A token at a time every
+// value is a store of two bytes of its own.
 template <typename T>
+__device__ __forceinline__ void values_by_tiles(const PrepareArgs& a, int block, int blocks, float (*tile)[65]) {
+  const int count = a.groups * a.d, across = (count + 63) / 64, tiles = (a.tokens + 63) / 64 * across;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const float lam = a.first != nullptr ? a.mix_weight[0] : 0.f;
+  for (int at = block; at < tiles; at += blocks) {
+    const int t0 = at / across * 64, i0 = at % across * 64;
+    const int mine = t0 + lane;
+    const int page = mine < a.tokens ? a.token_page[mine] : -1, off = mine < a.tokens ? a.token_offset[mine] : 0;
+    if (i0 + lane < count) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int t = wave + 4 * k;
+        if (t0 + t < a.tokens) tile[lane][t] = value_of(a, t0 + t, i0 + lane, lam);
+      }
+    }
+    __syncthreads();
+    if (page >= 0 && page < a.num_pages) {         // the host checks that every token has a page
+      T* vp = (T*)a.v_pages + (size_t)page * a.page_stride + off;
+#pragma unroll
+      for (int k = 0; k < 16; ++k) {
+        const int i = wave + 4 * k;
+        if (i0 + i < count) vp[(size_t)(i0 + i) * a.page_size] = from_f32<T>(tile[i][lane]);
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Latency bounds it for few tokens, memory for many (2,048 tokens of 32 + 2 x 8 heads of 128: 76 MB). Elements one by one
+// and values a token at a time took 5.7 us for 8 tokens and 44.8 for 2,048; four at a time and by tiles 4.5 and 25.6.
+// grid: (tokens, 3, shares), values first: a block takes a share of a token's queries, keys or values; each of the three needs nothing
+// of the other two. (A norm over the whole projection is summed up by every block that shares it.)
+template <typename T, bool TILED>
 __global__ void __launch_bounds__(256) qkv_prepare_kernel(PrepareArgs a) {
   __shared__ float scratch[4];
-  __shared__ float cosines[128], sines[128];       // of the token's angles, once for all heads
-  const int t = blockIdx.x, part = blockIdx.y, share = blockIdx.z, shares = gridDim.z;
+  __shared__ __attribute__((aligned(16))) float cosines[128], sines[128];       // of the token's angles, once for all heads
+  __shared__ float tile[TILED ? 64 : 1][65];
+  const int t = blockIdx.x, part = 2 - blockIdx.y, share = blockIdx.z, shares = gridDim.z;
+  if (TILED && part == 2) return values_by_tiles<T>(a, t + a.tokens * share, a.tokens * shares, tile);
   const float* row = a.proj + (size_t)t * a.ld;
   const int nq = a.heads * a.n, nk = a.groups * a.n;
   const int page = a.token_page[t], off = a.token_offset[t];
   if (part > 0 && (page < 0 || page >= a.num_pages)) return;       // the host checks that every token has a page
   if (part == 2) {
-    const float* xv = row + a.values_at;
     T* vp = (T*)a.v_pages + (size_t)page * a.page_stride;
     const float lam = a.first != nullptr ? a.mix_weight[0] : 0.f;
-    const float* first = a.first != nullptr ? a.first + (size_t)t * a.first_ld : nullptr;
-    for (int i = threadIdx.x + 256 * share; i < a.groups * a.d; i += 256 * shares) {
-      const int g = i / a.d, e = i - g * a.d;
-      float val = 0.f;
-      if (e < a.v) {
-        val = xv[g * a.v + e];
-        if (first != nullptr) val = (1.f - lam) * val + lam * first[g * a.v + e];
-      }
-      vp[((size_t)g * a.d + e) * a.page_size + off] = from_f32<T>(val);
-    }
+    for (int i = threadIdx.x + 256 * share; i < a.groups * a.d; i += 256 * shares)
+      vp[(size_t)i * a.page_size + off] = from_f32<T>(value_of(a, t, i, lam));
     return;
   }
   const float scale = part == 0 ? query_scale(a, t) : 1.f;
@@ -127,11 +185,35 @@ __global__ void __launch_bounds__(256) qkv_prepare_kernel(PrepareArgs a) {
   float norm = 1.f;
   if (w != nullptr) {
     float s = 0.f;
-    for (int i = threadIdx.x; i < count; i += 256) s += x[i] * x[i];
+    if (a.fours) {
+      for (int i = threadIdx.x; i < count / 4; i += 256) {
+        const f32x4p z = ((const f32x4p*)x)[i];
+        s += z[0] * z[0] + z[1] * z[1] + z[2] * z[2] + z[3] * z[3];
+      }
+    } else {
+      for (int i = threadIdx.x; i < count; i += 256) s += x[i] * x[i];
+    }
     s = block_sum<4>(s, scratch);
     norm = 1.f / sqrtf(s / (float)count + a.eps);
   }
   __syncthreads();
+  if (a.fours) {
+    typedef typename Four<T>::type four;
+    T* out = part == 0 ? (T*)a.q_out + (size_t)t * a.heads * a.d
+                       : (T*)a.k_pages + (size_t)page * a.page_stride + (size_t)off * a.d;
+    const size_t apart = part == 0 ? a.d : (size_t)a.page_size * a.d;          // from a head to the next
+    const int per = a.d / 4;
+    for (int i = threadIdx.x + 256 * share; i < heads * per; i += 256 * shares) {
+      const int head = i / per, e = 4 * (i - head * per);
+      f32x4p val = {0.f, 0.f, 0.f, 0.f};
+      if (e < a.n) val = turned4(x, w, norm, head, e, a, cosines, sines) * (part == 0 && a.head_scale ? scale * a.head_scale[head] : scale);
+      four o;
+#pragma unroll
+      for (int c = 0; c < 4; ++c) o[c] = from_f32<T>(val[c]);
+      *(four*)(out + head * apart + e) = o;
+    }
+    return;
+  }
   if (part == 0) {
     T* q_out = (T*)a.q_out + (size_t)t * a.heads * a.d;
     for (int i = threadIdx.x + 256 * share; i < heads * a.d; i += 256 * shares) {
@@ -171,14 +253,26 @@ extern "C" int tnx_qkv_prepare(const float* proj, int ld, const float* q_weight,
   if (tokens == 0) return 0;
   PrepareArgs a{proj, ld, q_weight, k_weight, eps, freqs, half, interleaved, positions, scale, mix_weight, first, first_ld,
                 token_page, token_offset, q_out, k_pages, v_pages, page_stride, num_pages, page_size, heads, groups, n, v, d,
-                per_head, values_at, head_scale, temp_coef, temp_every};
+                per_head, values_at, head_scale, temp_coef, temp_every, tokens, 0};
+  // four neighbours at a time where heads, rows and places allow it (a row's start is its keys' start and a head's as well)
+  const uintptr_t ends = (uintptr_t)proj | (uintptr_t)q_weight | (uintptr_t)k_weight | (uintptr_t)q_out | (uintptr_t)k_pages;
+  a.fours = n % 4 == 0 && d % 4 == 0 && ld % 4 == 0 && page_stride % 4 == 0 && ends % 16 == 0 &&
+            (freqs == nullptr || (!interleaved && half % 4 == 0));
   // few tokens: a token's heads over several blocks
   int shares = 1;
   while (shares < 8 && 6ll * tokens * shares <= tnx_compute_units() && heads * d >= 1024 * shares) shares *= 2;
-  if (dtype == TNX_F32)
-    qkv_prepare_kernel<float><<<dim3(tokens, 3, shares), 256, 0, stream>>>(a);
-  else
-    qkv_prepare_kernel<bf16_t><<<dim3(tokens, 3, shares), 256, 0, stream>>>(a);
+  const dim3 grid(tokens, 3, shares);
+  // Values by tiles from 48 tiles on, fewer leave most units without one. us, a token at a time / by tiles, 32 query heads:
+  // 8 heads of 64, 256 tokens (32 tiles) 5.9 / 6.7, 400 (56) 6.8 / 6.8, 2,048 19.4 / 15.1; 8 of 128, 64 tokens (16) 6.3 / 6.8,
+  // 256 (64) 8.1 / 7.1, 2,048 30.6 / 25.6; 32 of 128, 128 tokens (128) 10.4 / 7.0, 2,048 81.7 / 40.4.
+  const bool tiled = ((long long)tokens + 63) / 64 * (((long long)groups * d + 63) / 64) >= 48;
+  if (dtype == TNX_F32) {
+    if (tiled) qkv_prepare_kernel<float, true><<<grid, 256, 0, stream>>>(a);
+    else qkv_prepare_kernel<float, false><<<grid, 256, 0, stream>>>(a);
+  } else {
+    if (tiled) qkv_prepare_kernel<bf16_t, true><<<grid, 256, 0, stream>>>(a);
+    else qkv_prepare_kernel<bf16_t, false><<<grid, 256, 0, stream>>>(a);
+  }
   TNX_CHECK_LAUNCH("qkv_prepare");
   return 0;
 }
