@@ -69,3 +69,32 @@ def test_memory_by_chunks(sizes, steps, gates, line):
             assert float((mem - plain[r][0]).norm() / plain[r][0].norm()) < 2e-5
             assert float((nrm - plain[r][1]).norm() / plain[r][1].norm()) < 2e-5
     assert float(state[0][1].min()) == 3.0 and float(state[0][4].min()) == 3.0       # slots of no one are not touched
+
+
+@pytest.mark.parametrize("column", ["query", "key", "value", "input gate", "forget gate"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_token_that_is_no_number_leaves_the_ones_before_it(column, bad):
+    """One projection of token 70 of 130 is no number: the tokens before it are what they are without it, to the bit, and the
+    head's tokens from it on (of a query: the token alone) are no numbers. A gate's cap makes a number of an infinite one."""
+    from transformers_neuronx_amd.kernels import make_ops
+    heads, n, v, at = 2, 64, 32, 70
+    hn, hv = heads * n, heads * v
+    ops = make_ops("hip", torch.float32, DEV)
+    ops.memory_chunk_run = 1
+    g = torch.Generator().manual_seed(8)
+    proj = torch.randn(130, 2 * hn + 2 * hv + 2 * heads, generator=g)
+    weight = torch.rand(hv, generator=g) + 0.5
+    made = []
+    for spoil in (False, True):
+        x = proj.clone()
+        if spoil:
+            x[at, {"query": n, "key": hn + n, "value": 2 * hn + v, "input gate": -heads + -heads + 1, "forget gate": -1}[column]] = bad
+        state = [torch.zeros(1, 2, heads, v, n, device=DEV), torch.zeros(1, 2, heads, n, device=DEV), torch.zeros(1, 2, heads, device=DEV)]
+        made.append(ops.matrix_memory(x.to(DEV), heads, n, v, 9.0, 1e-5, weight.to(DEV), _ctx([130], [0], [0]), *state).cpu())
+    clean, spoilt = made
+    assert torch.isfinite(clean).all()
+    assert torch.equal(clean[:at], spoilt[:at]) and torch.equal(clean[:, :v], spoilt[:, :v])      # (the head before: untouched)
+    if not ("gate" in column and bad == float("inf")):
+        last = at + 1 if column == "query" else 130
+        assert torch.isnan(spoilt[at:last, v:]).any(dim=1).all()
+        assert torch.equal(clean[last:, v:], spoilt[last:, v:])

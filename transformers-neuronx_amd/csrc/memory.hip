@@ -132,10 +132,9 @@ __global__ void __launch_bounds__(64 * W) memory_gates_kernel(CellArgs a, float*
 // nothing is divided and no logarithms are subtracted. `memory_weights_kernel` makes (q_t . k_j) D_tj, P_t and D_63,j for all
 // chunks side by side; `memory_chunks_kernel` goes through a run's chunks with 16 columns of S a block. The walk is a chain
 // of a few multiply-adds and four lane exchanges a token, whatever the matrix units could do. 2,048 tokens, 32 heads of 64
-// rows and 128 columns: 399 us by the walk, 132 us by chunks: 19 for the weights and
-// 113 for the chunks (3.5 us each, of which the matrix instructions take 0.65: one block of four waves a unit, which waits
-// for its operands). Against 64 bits: 4.2e-7 by the walk, 3.2e-7 by chunks.
-// (A token whose projections are not finite makes the chunk's earlier tokens not finite as well, not its later ones only.)
+// rows and 128 columns: 399 us by the walk, 124 us by chunks: 19 for the weights and 105 for the chunks (3.3 us each, of
+// which the matrix instructions take 0.65: one block of four waves a unit, which waits for its operands). Off from 64 bits
+// over 24 draws of 210 to 2,048 tokens, on average: 6.3e-7 of the result by the walk, 4.0e-7 by chunks.
 typedef float f32x4v __attribute__((ext_vector_type(4)));
 
 // Chunk `b` of all chunks of 64 tokens of the runs that go by chunks: its run and its first token in it; false: there are fewer.
@@ -320,7 +319,7 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
     }
     if (c0 + 64 < count) fetch(c0 + 64);
     f32x4v acc = {}, more = {};
-    float dot = 0.f;
+    float dot = 0.f, probe = 0.f;
 #pragma unroll
     for (int s = 0; s < KD; ++s) {
       const int d = g * KD + s;
@@ -328,10 +327,7 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
       dot += qq[s] * norms[turn][d];
     }
 #pragma unroll
-    for (int s = 0; s < 16; ++s) {
-      more = __builtin_amdgcn_mfma_f32_16x16x4f32(ww[s / 4][s % 4], vv[s], more, 0, 0, 0);
-      dot += ww[s / 4][s % 4];
-    }
+    for (int s = 0; s < 16; ++s) probe += vv[s] * 0.f;
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
       float sum = 0.f;
@@ -345,6 +341,21 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
       sum += __shfl_xor(sum, 32);
       nrm[u] = keep_now * nrm[u] + sum;
     }
+    // A value that is no number must not reach the tokens before it, whose weight of it is zero: it is left out of the
+    // products, and the tokens from it on are no numbers in its column.
+    int spoilt = 64;
+    if (__any(probe != 0.f)) {
+#pragma unroll
+      for (int s = 15; s >= 0; --s)
+        if (vv[s] * 0.f != 0.f) vv[s] = 0.f, spoilt = 16 * g + s;
+      spoilt = min(spoilt, __shfl_xor(spoilt, 16));
+      spoilt = min(spoilt, __shfl_xor(spoilt, 32));
+    }
+#pragma unroll
+    for (int s = 0; s < 16; ++s) {
+      more = __builtin_amdgcn_mfma_f32_16x16x4f32(ww[s / 4][s % 4], vv[s], more, 0, 0, 0);
+      dot += ww[s / 4][s % 4];
+    }
     dot += __shfl_xor(dot, 16);
     dot += __shfl_xor(dot, 32);
     // (the denominator is 1e-6 at least: its reciprocal, right to a unit in the last place, is no subnormal)
@@ -353,7 +364,7 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
     for (int e = 0; e < 4; ++e) {
       const int t = 16 * wave + 4 * g + e;
       const float o = (acc[e] + more[e]) * __shfl(below, 4 * g + e);
-      if (t < len && col_ok) a.out[(size_t)(start + c0 + t) * hv + head * a.v + col] = o;
+      if (t < len && col_ok) a.out[(size_t)(start + c0 + t) * hv + head * a.v + col] = t < spoilt ? o : NAN;
     }
   }
 #pragma unroll

@@ -1774,9 +1774,9 @@ class HipOps:
 
     # Runs of so many tokens go through the matrix memory by chunks of 64 (query/key heads of up to 128 elements), shorter
     # ones token by token. us a layer of 32 heads of 64 rows, token by token / by chunks: 128 columns, one run of 24 tokens
-    # 15.6 / 17.8, 48: 19.7 / 19.0, 210: 56 / 34, 2,048: 426 / 159, eight runs of 48 58 / 49; 64 columns, 24: 14.7 / 16.8, 48:
-    # 18.8 / 18.0, 24 runs of 32 53 / 64. A step with shorter runs as well takes both ways, from a longer run on: beside 40
-    # runs of one token, 128 tokens 69 / 81, 600: 187 / 133.
+    # 15.5 / 17.6, 48: 19.4 / 18.7, 210: 56 / 33, 2,048: 425 / 151, eight runs of 48 56 / 47; 64 columns, 24: 14.6 / 16.6, 48:
+    # 18.8 / 17.8, 24 runs of 32 53 / 61. A step with shorter runs as well takes both ways, from a longer run on: beside 40
+    # runs of one token, 128 tokens 69 / 81, 600: 186 / 127.
     memory_chunk_run = 48
     memory_chunk_run_beside = 256
 
