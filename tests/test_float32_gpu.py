@@ -99,3 +99,34 @@ def test_float32_attention_keeps_a_value_that_is_no_number_to_its_readers():
     assert bool(torch.isinf(got[21:, 1, 5]).all())
     got[21:, 1, 5] = clean[21:, 1, 5] = 0
     torch.testing.assert_close(got, clean, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("runs,cached", [([1], [0]), ([1, 1, 1], [63, 64, 200]), ([5, 1], [0, 30]), ([16], [120]), ([17], [7])])
+@pytest.mark.parametrize("heads,kv,hs,page,width", [(4, 4, 16, 16, 68), (6, 2, 48, 32, 1280), (16, 16, 64, 64, 1024), (3, 1, 80, 64, 2052),
+                                                    (64, 0, 64, 16, 516)])
+@pytest.mark.parametrize("turned", [False, True])
+def test_float32_projections_go_where_they_belong(runs, cached, heads, kv, hs, page, width, turned):
+    """From the few-rows product straight into queries, keys and values, against the product and the scatter apart: the same
+    operations on every number."""
+    from test_kernels_gpu import _make_step
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    pages = sum(-(-(r + c) // page) for r, c in zip(runs, cached)) + 2
+    ctx = _make_step(runs, cached, page, pages, seed=hs)
+    g = _gen(hs + width)
+    total = (heads + 2 * kv) * hs
+    h = torch.randn(ctx.num_tokens, width, device=DEV, generator=g)
+    w, bias = torch.randn(total, width, device=DEV, generator=g), torch.randn(total, device=DEV, generator=g)
+    turn = tuple(torch.randn(300, hs, device=DEV, generator=g) for _ in range(2)) if turned else None
+    made = []
+    for rows in (16, 0):
+        ops = HipOps(torch.float32, DEV)
+        ops.f32_scatter_rows = rows
+        for b in (bias, None):
+            kp = torch.full((pages, kv, page, hs), 7.0, device=DEV) if kv else None
+            vp = torch.full((pages, kv, hs, page), 7.0, device=DEV) if kv else None
+            q = ops.qkv_project(h, w, b, heads, kv, hs, 0.3, ctx, ctx.groups["full"], kp, vp, turn=turn)
+            made.append([q] + ([kp, vp] if kv else []))
+    for fused, apart in zip(made[:2], made[2:]):
+        for one, other in zip(fused, apart):
+            # (a multiplication and an addition may be one rounding here and two there)
+            assert torch.equal(one, other) or (turned and float((one - other).abs().max()) <= 2.0 ** -21 * float(other.abs().max()))

@@ -28,12 +28,13 @@ __device__ __forceinline__ void epilogue_store(float v, int m, int n, int N, con
 // tables [turn_rows, head_size] of float32. Element d of a query or key head of the token at position p
 // becomes a[p][d] x[d] + b[p][d] x[d ^ 1], bias added, before the query's scale: any map of each pair
 // (2i, 2i + 1) of a head that depends on the position alone (a rotation: a = cos, b = -sin and +sin).
-struct QkvScatter {
+template <typename T>
+struct QkvScatterOf {
   const int* token_page;
   const int* token_off;
-  bf16_t* q_out;
-  bf16_t* k_pages;
-  bf16_t* v_pages;
+  T* q_out;
+  T* k_pages;
+  T* v_pages;
   float scale;
   int nq, nk, head_size, num_kv, page_size, num_pages;
   int page_pad;          // elements between the end of one page and the start of the next
@@ -42,17 +43,20 @@ struct QkvScatter {
   const int* positions;
   int turn_rows;
 };
+typedef QkvScatterOf<bf16_t> QkvScatter;
+struct NoScatter {};
 
 // `v`: element n of token m's projections with its bias; `beside`: element n ^ 1 with its bias (read only
 // where the scatter turns pairs)
 // (`page`, `off`: what `token_page` and `token_off` say of token m)
-__device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, const QkvScatter& sc, int page, int off) {
+template <typename T>
+__device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, const QkvScatterOf<T>& sc, int page, int off) {
   if (sc.turn_a && n < sc.nq + sc.nk) {
     const size_t at = (size_t)min(max(sc.positions[m], 0), sc.turn_rows - 1) * sc.head_size + n % sc.head_size;
     v = sc.turn_a[at] * v + sc.turn_b[at] * beside;
   }
   if (n < sc.nq) {
-    sc.q_out[(size_t)m * sc.nq + n] = (bf16_t)(v * sc.scale);
+    sc.q_out[(size_t)m * sc.nq + n] = from_f32<T>(v * sc.scale);
     return;
   }
   if (page < 0 || page >= sc.num_pages) return;
@@ -63,9 +67,9 @@ __device__ __forceinline__ void qkv_store(float v, float beside, int m, int n, c
   const size_t head_elems = (size_t)sc.page_size * sc.head_size;
   const size_t head = (size_t)page * ((size_t)sc.num_kv * head_elems + sc.page_pad) + (size_t)h * head_elems;
   if (is_key)
-    sc.k_pages[head + (size_t)off * sc.head_size + d] = (bf16_t)v;
+    sc.k_pages[head + (size_t)off * sc.head_size + d] = from_f32<T>(v);
   else
-    sc.v_pages[head + (size_t)d * sc.page_size + off] = (bf16_t)v;
+    sc.v_pages[head + (size_t)d * sc.page_size + off] = from_f32<T>(v);
 }
 
 // ------------------------------------------------------------------------------------------ float32
@@ -132,11 +136,14 @@ gemm_f32_kernel(const float* __restrict__ x, const float* __restrict__ w, const 
 // are asked for together: what bounds a narrow matrix is how often a wave waits for memory, not the bytes. Measured at 3
 // rows, a wave for every 4 columns against four: 1,024 columns of K 4,096 13.8 us against 7.7, 4,096 of 1,024 9.8 against 8.3;
 // with bias and residual asked for first and the weight marked as read once 6.8 and 7.6.
-template <int MR, bool SPLIT, int UNROLL>
+// Scatter (`QkvScatterOf<float>`): queries, keys and values go where they belong from here, in place of a matrix that another
+// launch reads again. 3 rows of 3,072 by 1,024: 7.3 us, where the product took 6.5 and the other launch 3.2.
+template <int MR, bool SPLIT, int UNROLL, typename Scatter>
 __global__ void __launch_bounds__(256)
 gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                        const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
-                       int N, int K) {
+                       int N, int K, Scatter sc) {
+  constexpr bool SCATTER = !std::is_same<Scatter, NoScatter>::value;
   __shared__ float sums[SPLIT ? 4 : 1][4 * MR];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int n0 = (SPLIT ? blockIdx.x : blockIdx.x * 4 + wave) * 4;
@@ -153,6 +160,10 @@ gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
   float add = 0.f, onto = 0.f;
   if (puts && bias) add = bias[put_c];
   if (puts && residual) onto = residual[(size_t)put_m * N + put_c];
+  int page = -1, off = 0;
+  if constexpr (SCATTER) {
+    if (puts) page = sc.token_page[put_m], off = sc.token_off[put_m];
+  }
   float acc[4][MR];
 #pragma unroll
   for (int c = 0; c < 4; ++c)
@@ -201,7 +212,11 @@ gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
     __syncthreads();
     if (puts) mine = (sums[0][put] + sums[1][put]) + (sums[2][put] + sums[3][put]);
   }
-  if (puts) {
+  if constexpr (SCATTER) {
+    if (bias) mine += add;
+    const float beside = __shfl_xor(mine, MR);          // column c ^ 1 of the same row
+    if (puts) qkv_store(mine, beside, put_m, put_c, sc, page, off);
+  } else if (puts) {
     float v = mine;
     if (bias) v += add;
     v = apply_act(v, act);
@@ -210,22 +225,40 @@ gemm_f32_skinny_kernel(const float* __restrict__ x, const float* __restrict__ w,
   }
 }
 
-template <int MR>
+template <int MR, typename Scatter>
 static void launch_f32_skinny(const float* x, const float* w, const float* bias, const float* residual, void* out,
-                              int out_dtype, int act, int M, int N, int K, hipStream_t stream) {
+                              int out_dtype, int act, int M, int N, int K, const Scatter& sc, hipStream_t stream) {
   // Steps asked for together: as many as the rows leave registers for.
   constexpr int MOST = MR <= 4 ? 4 : MR <= 8 ? 2 : 1;
+#define SKINNY_F32(SPLIT, UNROLL, GRID)                                                                            \
+  gemm_f32_skinny_kernel<MR, SPLIT, UNROLL, Scatter><<<dim3(GRID), 256, 0, stream>>>(x, w, bias, residual, out,     \
+                                                                                     out_dtype, act, M, N, K, sc)
   // A wave for every 4 columns gives N / 16 blocks; below four blocks a compute unit the waves of a block share K instead.
   if ((N + 15) / 16 < 4 * tnx_compute_units()) {
-    const dim3 grid((N + 3) / 4);
     if (K > 1024 && MOST > 1)
-      gemm_f32_skinny_kernel<MR, true, MOST><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+      SKINNY_F32(true, MOST, (N + 3) / 4);
     else
-      gemm_f32_skinny_kernel<MR, true, 1><<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
+      SKINNY_F32(true, 1, (N + 3) / 4);
   } else {
-    gemm_f32_skinny_kernel<MR, false, (MOST > 2 ? 2 : MOST)><<<dim3((N + 15) / 16), 256, 0, stream>>>(x, w, bias, residual,
-                                                                                          out, out_dtype, act, M, N, K);
+    SKINNY_F32(false, (MOST > 2 ? 2 : MOST), (N + 15) / 16);
   }
+#undef SKINNY_F32
+}
+
+// By the number of rows, up to 16.
+template <typename Scatter>
+static void f32_skinny(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
+                       int act, int M, int N, int K, const Scatter& sc, hipStream_t stream) {
+  if (M <= 1)
+    launch_f32_skinny<1>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
+  else if (M <= 2)
+    launch_f32_skinny<2>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
+  else if (M <= 4)
+    launch_f32_skinny<4>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
+  else if (M <= 8)
+    launch_f32_skinny<8>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
+  else
+    launch_f32_skinny<16>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
 }
 
 // Many rows in float32, on the float32 matrix instructions (32x32x2: products and sums in float32, no operand is
@@ -403,16 +436,7 @@ extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, c
   TNX_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   if (M <= 16 && K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0) {
-    if (M <= 1)
-      launch_f32_skinny<1>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
-    else if (M <= 2)
-      launch_f32_skinny<2>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
-    else if (M <= 4)
-      launch_f32_skinny<4>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
-    else if (M <= 8)
-      launch_f32_skinny<8>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
-    else
-      launch_f32_skinny<16>(x, w, bias, residual, out, out_dtype, act, M, N, K, stream);
+    f32_skinny(x, w, bias, residual, out, out_dtype, act, M, N, K, NoScatter{}, stream);
     TNX_CHECK_LAUNCH("gemm_f32_skinny");
     return 0;
   }
@@ -1204,7 +1228,8 @@ extern "C" int tnx_gemm_bf16(const void* x, const void* w, const void* w_tiles, 
 // The fused projection of queries, keys and values: `x w^T + bias` with w = [Wq; Wk; Wv] stacked by rows,
 // queries scaled and written densely, keys and values written straight into their cache pages.
 // What both forms of the fused projection check and fill in of the pair-turning tables.
-static int qkv_turn(QkvScatter& sc, const float* turn_a, const float* turn_b, const int* positions, int turn_rows,
+template <typename T>
+static int qkv_turn(QkvScatterOf<T>& sc, const float* turn_a, const float* turn_b, const int* positions, int turn_rows,
                     int page_pad) {
   TNX_REQUIRE(page_pad >= 0 && page_pad % 8 == 0, "gemm_bf16_qkv: bad distance between pages");
   sc.page_pad = page_pad;
@@ -1242,6 +1267,24 @@ extern "C" int tnx_gemm_bf16_qkv(const void* x, const void* w, const void* w_til
   const int N = sc.nq + 2 * sc.nk;
   return gemm_bf16_dispatch(x, w, w_tiles, bias, nullptr, nullptr, TNX_BF16, TNX_ACT_NONE, M, N, K, force_tiled, &sc,
                             stream);
+}
+
+// The float32 engine's, for up to 16 rows and K of a multiple of 4.
+extern "C" int tnx_gemm_f32_qkv(const float* x, const float* w, const float* bias, int M, int K, const int* token_page,
+                                const int* token_off, float* q_out, float* k_pages, float* v_pages, float scale,
+                                int num_heads, int num_kv, int head_size, int page_size, int num_pages,
+                                const float* turn_a, const float* turn_b, const int* positions, int turn_rows, int page_pad,
+                                hipStream_t stream) {
+  TNX_REQUIRE(num_heads > 0 && num_kv >= 0 && head_size > 0 && head_size % 4 == 0 && page_size > 0, "gemm_f32_qkv: bad sizes");
+  TNX_REQUIRE(M >= 0 && M <= 16 && K > 0 && K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0,
+              "gemm_f32_qkv: up to 16 rows that begin at multiples of 16 bytes, got %d of %d", M, K);
+  QkvScatterOf<float> sc{token_page, token_off, q_out, k_pages, v_pages, scale, num_heads * head_size, num_kv * head_size,
+                         head_size, num_kv, page_size, num_pages};
+  if (int rc = qkv_turn(sc, turn_a, turn_b, positions, turn_rows, page_pad)) return rc;
+  if (M == 0) return 0;
+  f32_skinny(x, w, bias, nullptr, nullptr, TNX_F32, TNX_ACT_NONE, M, sc.nq + 2 * sc.nk, K, sc, stream);
+  TNX_CHECK_LAUNCH("gemm_f32_qkv");
+  return 0;
 }
 
 // The same two for the rows of a LayerNorm's input (float32), the norm folded into the product (see `NormFold`):
