@@ -222,15 +222,40 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
   const bool few = !greedy && k > 0 && k < vocab && k <= SAMPLE_GATHER;
   const float inv_temp = greedy ? 0.f : 1.f / temp;     // for the bins of the search only; weights divide by temp
 
+  // f(logit, token) for all of the row, in no order that counts. A block goes through a row several times and waits for memory
+  // each time: 16 logits a thread are asked for together. 3 rows of 50,272, top-k of 50: 33 us, one at a time 56.
+  const bool fours = vocab % 4 == 0 && (uintptr_t)row % 16 == 0;
+  auto over_row = [&](auto f) __attribute__((always_inline)) {
+    if (fours) {
+      const f32x4* row4 = (const f32x4*)row;
+      const int n4 = vocab / 4;
+      for (int i0 = tid; i0 < n4; i0 += 4 * SAMPLE_THREADS) {
+        f32x4 v[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) v[u] = row4[min(i0 + u * SAMPLE_THREADS, n4 - 1)];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int i = i0 + u * SAMPLE_THREADS;
+          if (i < n4) {
+#pragma unroll
+            for (int j = 0; j < 4; ++j) f(v[u][j], 4 * i + j);
+          }
+        }
+      }
+    } else {
+      for (int i = tid; i < vocab; i += SAMPLE_THREADS) f(row[i], i);
+    }
+  };
+
   // the largest key: argmax, and the maximum for the softmax (the gathered tokens bring their own)
   float xmax = 0.f;
   int arg = 0;
   if (!few) {
     uint64_t b = 0;
-    for (int i = tid; i < vocab; i += SAMPLE_THREADS) {
-      const uint64_t key = order_key(row[i], i);
+    over_row([&](float x, int i) {
+      const uint64_t key = order_key(x, i);
       b = key > b ? key : b;
-    }
+    });
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
       const uint64_t other = __shfl_xor((unsigned long long)b, o, 64);
@@ -265,10 +290,10 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
       const int shift = 56 - 8 * pass;
       for (int j = tid; j < 256 * 8; j += SAMPLE_THREADS) cnt8[j] = 0;
       __syncthreads();
-      for (int i = tid; i < vocab; i += SAMPLE_THREADS) {
-        const uint64_t key = order_key(row[i], i);
+      over_row([&](float x, int i) {
+        const uint64_t key = order_key(x, i);
         if ((key & mask) == prefix) atomicAdd(&cnt8[((unsigned int)(key >> shift) & 255u) * 8 + copy], 1u);
-      }
+      });
       __syncthreads();
       if (tid < 256) {
         unsigned int c = 0;
@@ -299,10 +324,10 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
         // ones beside it is the threshold (keys differ, so there is exactly one)
         if (tid == 0) sh_n = 0;
         __syncthreads();
-        for (int i = tid; i < vocab; i += SAMPLE_THREADS) {
-          const uint64_t key = order_key(row[i], i);
+        over_row([&](float x, int i) {
+          const uint64_t key = order_key(x, i);
           if ((key & mask) == prefix) tkey[atomicAdd(&sh_n, 1)] = key;
-        }
+        });
         __syncthreads();
         if (tid < (int)bin) {
           const uint64_t mine = tkey[tid];
@@ -335,16 +360,16 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
       sh_last = -1;
     }
     __syncthreads();
-    for (int i = tid; i < vocab; i += SAMPLE_THREADS) {
-      const uint64_t key = order_key(row[i], i);
+    over_row([&](float x, int i) {
+      const uint64_t key = order_key(x, i);
       if (key >= floor_key) {
         const int at = atomicAdd(&sh_n, 1);
         if (at < SAMPLE_GATHER) {
           tkey[at] = key;
-          tval[at] = row[i] != row[i] ? -INFINITY : row[i] / temp;
+          tval[at] = x != x ? -INFINITY : x / temp;
         }
       }
-    }
+    });
     __syncthreads();
     const int n = min(sh_n, SAMPLE_GATHER);
     const bool mine_too = wave * 64 < n;         // a wave with none of them has nothing to find out
