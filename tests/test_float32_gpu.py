@@ -101,6 +101,43 @@ def test_float32_attention_keeps_a_value_that_is_no_number_to_its_readers():
     torch.testing.assert_close(got, clean, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("runs,cached,first,last", [([160], [0], 32, 63), ([300], [0], 0, 31), ([33], [0], 32, 32), ([20], [90], 64, 95),
+                                                    ([1], [200], 64, 127), ([1], [128], 128, 128), ([1], [700], 0, 63), ([1, 1], [63, 448], 0, 511)])
+@pytest.mark.parametrize("window", [None, 37])
+@pytest.mark.parametrize("heads,kv,hs", [(4, 2, 64), (3, 3, 80)])
+def test_float32_attention_of_keys_that_are_no_numbers(runs, cached, first, last, window, heads, kv, hs):
+    """Keys `first` to `last`, the whole share of one wave or of several, are no numbers: nor is the result of a query that sees
+    one of them, and the others are as without. Keys infinitely far from a query weigh nothing."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g, page, n = HipOps(torch.float32, DEV), _gen(first + hs), 64, sum(runs)
+    ctx, pages = _step(runs, cached, page, seed=hs)
+    view = ctx.groups["full"]
+    clean = torch.randn(pages, kv, page, hs, device=DEV, generator=g)
+    vp = torch.randn(pages, kv, hs, page, device=DEV, generator=g)
+    q = torch.randn(n, heads * hs, device=DEV, generator=g) * hs ** -0.5
+    q.view(n, heads, hs)[..., 0] = 0.1
+    for spoil in (float("nan"), -float("inf")):
+        kp, want, sees = clean.clone(), [], []
+        for r, (count, c) in enumerate(zip(runs, cached)):
+            at = torch.arange(c + count, device=DEV)
+            table = view.block_table[r].long()[at // page]
+            own = (at >= first) & (at <= last)
+            kp[table[own], :, at[own] % page, 0] = spoil
+            keys, vals = (x.double().transpose(0, 1).repeat_interleave(heads // kv, 0)
+                          for x in (kp[table, :, at % page], vp[table, :, :, at % page]))
+            i = torch.arange(c, c + count, device=DEV)[:, None]
+            hidden = (at > i) | ((i - at >= window) if window else (at > i))
+            s = q[sum(runs[:r]):][:count].double().view(count, heads, hs).transpose(0, 1) @ keys.transpose(1, 2)
+            want.append((torch.softmax(s.masked_fill(hidden, float("-inf")), -1) @ vals).transpose(0, 1))
+            sees.append((own & ~hidden).any(1))
+        want, sees = torch.cat(want).reshape(n, -1), torch.cat(sees)
+        if spoil != spoil:
+            assert torch.equal(torch.isnan(want).any(1), sees) and torch.equal(torch.isnan(want).all(1), sees)
+        got = hip.attention(q, heads, kv, hs, ctx, view, kp, vp, window).double()
+        # (the bound of `test_float32_attention`: nothing here is longer)
+        torch.testing.assert_close(got, want, rtol=0, atol=5 * (8 * hs + 760) * 2.0 ** -24, equal_nan=True)
+
+
 @pytest.mark.parametrize("runs,cached", [([1], [0]), ([1, 1, 1], [63, 64, 200]), ([5, 1], [0, 30]), ([16], [120]), ([17], [7])])
 @pytest.mark.parametrize("heads,kv,hs,page,width", [(4, 4, 16, 16, 68), (6, 2, 48, 32, 1280), (16, 16, 64, 64, 1024), (3, 1, 80, 64, 2052),
                                                     (64, 0, 64, 16, 516)])

@@ -219,7 +219,8 @@ attention_prompt_f32_kernel(F32Attention a) {
 #pragma unroll
     for (int w = 0; w < 4; ++w) {
       const float mw = ms[w * 32 + r];
-      if (mw == -INFINITY) continue;               // a wave that saw no key of this query
+      // (a wave that saw no key of this query brings sums of zero; one whose scores are no numbers, which a maximum passes
+      // over, brings sums that are none either: no wave is left out)
       const float f = mw == top ? 1.f : expf(mw - top);
       sum += f * ls[w * 32 + r];
       v += f * merged[(size_t)(w * 32 + r) * ROW + d];
@@ -276,7 +277,7 @@ attention_decode_f32_kernel(F32Attention a) {
     const bool seen = key >= lo && key <= pos && held;
     const float s = seen ? (s4[0] + s4[1]) + (s4[2] + s4[3]) : -INFINITY;
     const float m_new = fmaxf(m, wave_max(s));
-    const float p = seen ? expf(s - m_new) : 0.f;
+    const float p = s == -INFINITY ? 0.f : expf(s - m_new);
     const float alpha = m == m_new ? 1.f : expf(m - m_new);
     l = l * alpha + wave_sum(p);
     m = m_new;
@@ -320,8 +321,7 @@ attention_decode_f32_kernel(F32Attention a) {
     float sum = 0.f, v = 0.f;
 #pragma unroll
     for (int w = 0; w < WAVES; ++w) {
-      if (ms[w] == -INFINITY) continue;
-      const float f = ms[w] == top ? 1.f : expf(ms[w] - top);
+      const float f = ms[w] == top ? 1.f : expf(ms[w] - top);       // (no wave is left out, as above)
       sum += f * ls[w];
       v += f * os[w][d];
     }
