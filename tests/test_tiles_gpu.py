@@ -64,6 +64,27 @@ def test_experts_by_tiles(counts, width, f, act, on, identity, rows):
         assert _apart(got - (r if r is not None else 0), want) < 2.0 ** -8
 
 
+@pytest.mark.parametrize("tokens,experts,top,width,f", [(16, 1, 1, 32768, 32768), (32768, 8, 8, 64, 8192), (65536, 1, 1, 32768, 64)])
+def test_experts_beyond_the_reach_of_tiles(tokens, experts, top, width, f):
+    """A matrix, the pairs' inner rows or the tokens' rows of 4 GB: more than the tiles can count, so the step goes the other way."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops, g = HipOps(torch.bfloat16, DEV), torch.Generator(device=DEV).manual_seed(width)
+    assert not ops._tiles_reach(tokens, experts, top, width, f, 128) and ops._tiles_reach(tokens // 2, experts, top, width, f // 2, 128)
+
+    def some(*shape, std=1.0):
+        return torch.empty(shape, device=DEV, dtype=torch.bfloat16).normal_(0.0, std, generator=g)
+
+    h, up, down = some(tokens, width), some(experts, f, width, std=width ** -0.5), some(experts, width, f, std=f ** -0.5)
+    chosen = torch.arange(top, device=DEV, dtype=torch.int32).expand(tokens, top).contiguous()
+    weights = torch.rand(tokens, top, device=DEV, generator=g) + 0.1
+    got = ops.expert_mixture(h, chosen, weights, up, down, "relu", "output", None)
+    rows = torch.arange(tokens, device=DEV) if tokens < 64 else torch.cat([torch.arange(32, device=DEV), torch.arange(tokens - 32, tokens, device=DEV)])
+    want = torch.zeros(len(rows), width, device=DEV)
+    for e in range(top):        # (in float32, whose error is none beside the inner values' rounding to bfloat16)
+        want += weights[rows, e, None] * (torch.relu(h[rows].float() @ up[e].float().T) @ down[e].float().T)
+    assert _apart(got[rows], want.double()) < 2.0 ** -8
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 64, 64), (33, 200, 64), (64, 72, 320), (65, 2048, 2048), (128, 136, 8192), (129, 128, 512),
                                    (333, 264, 2048), (700, 520, 2112)])
 @pytest.mark.parametrize("tile,shares", [(1, 1), (1, 3), (2, 1), (2, 5)])

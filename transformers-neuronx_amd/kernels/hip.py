@@ -2019,6 +2019,14 @@ class HipOps:
     expert_row_step = 128
     expert_plain_products = False      # tests set it: the kernel without the matrix unit in bfloat16 too
 
+    @staticmethod
+    def _tiles_reach(tokens, experts, top, width, f, rows) -> bool:
+        """Whether the experts' tiles reach all of their operands: a lane holds its place in one as 32 bits of bytes. Beyond
+        that (4 GB of rows or of one expert's matrix) the other ways, which count in 64 bits, take the step."""
+        pairs = tokens * top
+        return (pairs < 1 << 30 and tokens * width < 1 << 31 and pairs * f < 1 << 31 and width * f < 1 << 30
+                and (pairs // rows + experts) * (max(width, f) // 64 + 1) < 1 << 31)
+
     def expert_mixture(self, h, chosen, weights, w_gate_up, w_down, activation, weight_on, residual=None, may_wait=False,
                        limit=None, identity=0):
         """See `ReferenceOps.expert_mixture`. `may_wait`: the step is not being recorded, so the host may read
@@ -2040,10 +2048,11 @@ class HipOps:
         dev = h.device
         pairs = t * top
         out = torch.empty(t, width, dtype=torch.float32, device=dev)
+        rows = 128 if pairs >= self.expert_wide_tiles * experts else 64
         if (self.expert_grouped_rows > 0 and self.expert_library_rows > 0 and pairs >= self.expert_grouped_rows * experts
                 and not self.expert_plain_products and h.dtype == torch.bfloat16 and width % 64 == 0 and f % 64 == 0
+                and self._tiles_reach(t, experts, top, width, f, rows)
                 and (_ptr(h) | _ptr(w_gate_up) | _ptr(w_down)) % 16 == 0 and (residual is None or _ptr(residual) % 16 == 0)):
-            rows = 128 if pairs >= self.expert_wide_tiles * experts else 64
             ints = torch.empty(experts + 2 + 2 * pairs + 2 * (pairs // rows + experts), dtype=torch.int32, device=dev)
             inner = torch.empty(pairs, f, dtype=h.dtype, device=dev)
             y = torch.empty(pairs, width, dtype=torch.float32, device=dev)
