@@ -124,6 +124,15 @@ def test_products_that_the_tiles_take(m, n, k):
         torch.testing.assert_close(ops.linear(x, w, **kw).float(), lib.linear(x, w, **kw).float(), rtol=1e-2, atol=2e-2)
 
 
+@pytest.mark.parametrize("m,n,k", [(64, 12288, 4096), (40, 16384, 4096), (600, 4096, 16384), (640, 4096, 16384), (700, 3072, 12288),
+                                   (705, 2048, 8192), (768, 5120, 20480), (768, 2048, 2048)])
+def test_products_that_the_tiles_leave_alone(m, n, k):
+    """Products that bound a step by their own time, at sizes where the library was measured to be quicker."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops, x, w = HipOps(torch.bfloat16, DEV), torch.empty(m, k, device=DEV, dtype=torch.bfloat16), torch.empty(n, k, device=DEV, dtype=torch.bfloat16)
+    assert ops._tiles_room(m, n, k, x, w, None, False, False) == -1
+
+
 @pytest.mark.parametrize("tokens,top", [(1, 2), (3, 3), (8, 2), (9, 7), (32, 2), (33, 2), (16, 4)])
 @pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72)])
 @pytest.mark.parametrize("act,on", [("silu", "input"), ("relu2", "output")])

@@ -1617,18 +1617,30 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
   return 0;
 }
 
-// Which products these tiles take, and with which tile and how many shares of K (0: none, the vendor library is quicker).
-// Measured, us, library against tiles (which), bias and ReLU or residual included:
-//   long K, at least four times the columns, tiles of 128 x 128 and as many shares as give every unit a block: 100 rows 2,048
-//   (columns) x 8,192 (K) 20.4 / 18.4, 4,096 x 16,384 52.3 / 39.1; 333 rows 37.7 / 27.2 and 83.3 / 69.8; 640 rows 43.9 / 37.8
-//   and 120 / 109. Up to 768 rows: at 1,024 the library's larger tiles win (2,048 x 8,192 49 / 54).
-//   short K, up to 2,048, where tiles of 64 x 64 make at most one and a quarter a unit: 100 rows 6,144 x 2,048 14.3 / 13.3,
-//   8,192 x 2,048 16.7 / 15.2, 3,072 x 1,024 8.6 / 6.8; 333 rows 2,048 x 2,048 11.0 / 10.5, 3,072 x 1,024 10.4 / 8.5; or
-//   tiles of 128 x 128 at most one: 333 rows 6,144 x 2,048 25.2 / 20.7, 8,192 x 2,048 23.9 / 21.5; 640 rows 6,144 x 2,048
-//   24.8 / 23.7. Beyond (640 rows 8,192 x 2,048 27.3 / 32.3) the library.
-//   33 to 64 rows and K of 4,096, tiles of 64 x 64 with shares: 48 rows 4,096 x 4,096 16.2 / 13.2, 12,288 x 4,096 26.4 / 25.9.
+// Which products these tiles take, and with which tile and how many shares of K (0: none, the vendor library).
+// Two things count. A call of the library's takes the host some 13 us, a launch of ours 5, and a step that is not recorded is
+// bound by the host where its products take less: there the tiles win whole steps also where they take longer than the
+// library's kernel (prompts, us, with the library wherever that kernel is quicker / with the tiles: 1.3b 150 tokens 3,121 / 2,434,
+// 256 tokens 3,240 / 2,670, 2.7b 60 tokens 4,029 / 3,529, 350m 600 tokens 2,899 / 2,492). From some 30 us a product on the
+// device bounds the step, and there the quicker kernel is taken. Measured on weights that no cache holds, us, library / tiles
+// (with bias and ReLU, or the residual where a matrix is narrower than K), at 33 to 768 rows:
+//   K at least four times the columns: tiles of 128 x 128 with as many shares of K as give every unit a block. 144 rows 2,048
+//   (columns) x 8,192 (K) 24.6 / 19.8, 2,560 x 10,240 32.3 / 26.0, 4,096 x 16,384 73.8 / 48.2, 5,120 x 20,480 123 / 71; 333 rows
+//   38.3 / 26.3, 49.0 / 35.5, 83.0 / 78.8, 142 / 106; 640 rows 43.8 / 37.6, 67.0 / 60.4, -, 224 / 193. Above 128 rows K beyond
+//   4,096 has to give more than half of the units a block, and three quarters above 576 rows (4,096 x 16,384, 160 blocks: 560
+//   rows 124 / 119, 600 rows 119 / 131, 640 rows 119 / 141; 700 rows 3,072 x 12,288, 144 blocks, 88 / 98), and above 704 rows the
+//   library has a better tile: 700 and 768 rows 2,048 x 8,192 44.6 / 42.8 and 43.6 / 49.0, 5,120 x 20,480 237 / 170 and 179 / 200.
+//   A prompt of 6.7b's with 640 tokens: 11,401 us with tiles there, 10,590 without; 768 tokens 12,001 and 11,295.
+//   K up to 2,048: tiles of 64 x 64 where they make at most one and a quarter a unit, else of 128 x 128 at most one. 100 rows
+//   3,072 x 1,024 8.7 / 6.9, 6,144 x 2,048 14.1 / 13.4, 8,192 x 2,048 15.5 / 15.2; 333 rows 3,072 x 1,024 10.5 / 8.5, 6,144 x 2,048
+//   25.1 / 20.7, 8,192 x 2,048 24.0 / 21.7; 640 rows 6,144 x 2,048 24.9 / 23.5. The kernel alone is slower at 64 rows 6,144 x 2,048
+//   13.3 / 14.0 (a recorded step of 64 of 1.3b's 2,597 / 2,640), 160 to 300 rows 17.1 / 18.6 to 16.0 / 22.5 and 640 rows 2,048 x
+//   2,048 13.8 / 14.8: small enough for the host to bound the step. Above 640 rows tiles of 128 x 128 are to fill half the units:
+//   768 rows 2,048 x 2,048 (96) 14.1 / 19.1 (a prompt of 1.3b's with 768 tokens 4,037 with them, 3,624 without).
+//   33 to 64 rows and K up to 4,096: tiles of 64 x 64 with shares. 48 rows 3,072 x 4,096 13.4 / 12.6, 4,096 x 4,096 14.2 / 13.6, 7,680 x
+//   2,560 16.0 / 16.4, 10,240 x 2,560 21.6 / 20.8. Not from 2^25 elements on: 64 rows 12,288 x 4,096 27.9 / 31.6, 16,384 x 4,096 32.6 /
+//   36.0 (a step of 64 of 6.7b's 6,075 with tiles there, 5,897 without).
 // Up to 32 rows half a tile would be padding (32 rows 10,240 x 2,560: 17.7 / 20), and other kernels stand ready.
-// A call of the library's takes the host some 13 us, a launch of ours 5: a step of 333 tokens waits for that, too.
 // What bounds these sizes is the time a unit takes for a step of its one block (0.55 us for 128 x 128 x 64, of which the
 // matrix cores work 0.24), not memory: shares of K are the way to keep all units at it.
 enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2 };
@@ -1645,11 +1657,13 @@ static int choose_tiles(int M, int N, int K, int& shares) {
   if (M <= 32 || M > 768) return TILES_NONE;
   if (K >= 4ll * N && large <= units) {
     shares = share_out(large);
+    const long long blocks = large * shares;
+    if (K > 4096 && M > 128 && (M > 704 || 2 * blocks <= units || (M > 576 && 4 * blocks < 3 * units))) return TILES_NONE;
     return TILES_128;
   }
   if (K <= 2048 && 4 * small <= 5 * units) return TILES_64;
-  if (K <= 2048 && large <= units) return TILES_128;
-  if (M <= 64 && K <= 4096 && small <= units) {
+  if (K <= 2048 && large <= units && (M <= 640 || 2 * large > units)) return TILES_128;
+  if (M <= 64 && K <= 4096 && small <= units && (long long)N * K < 1ll << 25) {
     shares = share_out(small);
     return TILES_64;
   }

@@ -749,7 +749,7 @@ class HipOps:
                        work=lambda: self._product_work(m, n, k, out_item=out.element_size(), residual=residual is not None))
         return out
 
-    tile_products = True    # products of 17 to 768 rows by tiles of ours where those are quicker than the vendor library
+    tile_products = True    # products of 33 to 768 rows by tiles of ours where those are quicker than the vendor library
 
     def _tiles_room(self, m, n, k, x, w, residual, out_f32, force_tiled) -> int:
         """The floats of workspace that the product by tiles wants, -1 where it is not the way (the rule on sizes and what
