@@ -133,6 +133,15 @@ def test_products_that_the_tiles_leave_alone(m, n, k):
     assert ops._tiles_room(m, n, k, x, w, None, False, False) == -1
 
 
+@pytest.mark.parametrize("n,k,few", [(6144, 2048, True), (8192, 2048, True), (7680, 2560, False), (8320, 2048, False)])
+def test_few_rows_with_a_rounded_result(n, k, few):
+    """17 to 24 rows go to the few-rows kernel up to 2^24 elements of the matrix."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops, w = HipOps(torch.bfloat16, DEV), torch.empty(n, k, device=DEV, dtype=torch.bfloat16)
+    for m in (17, 24):
+        assert ops._library_product(m, n, k, w, False, plain=True) != few
+
+
 @pytest.mark.parametrize("tokens,top", [(1, 2), (3, 3), (8, 2), (9, 7), (32, 2), (33, 2), (16, 4)])
 @pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72)])
 @pytest.mark.parametrize("act,on", [("silu", "input"), ("relu2", "output")])

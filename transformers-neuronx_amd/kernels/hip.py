@@ -851,14 +851,19 @@ class HipOps:
             return False
         # small matrices at up to 32 rows: one launch of ours (5 to 10 us with its epilogue) beats the
         # library's product and the epilogue after it (11 to 15 us)
-        return not (m <= 32 and n * k <= (self.fused_matrix if scattered or (plain and m <= 24) else self.small_matrix))
+        few = self.fused_matrix if scattered else self.plain_matrix if plain and m <= 24 else self.small_matrix
+        return not (m <= 32 and n * k <= few)
 
     small_matrix = 1 << 23
-    # Queries, keys and values at 17 to 32 rows, us, few-rows kernel with everything in one launch against the library's
-    # product and `qkv_write`: 24 rows 6,144 x 2,048 11.5 / 18.9, 32 rows 12.3 / 16.4, 7,680 x 2,560 14.0 / 20.0 and
-    # 15.1 / 20.4; 12,288 x 4,096 33.7 / 33 and 38.2 / 33.6. The products of 17 to 24 rows with a bfloat16 result go the
-    # same way (24 rows 8,192 x 2,048 12.2 / 14.5 with the library), those of 32 have no clear winner.
+    # Queries, keys and values at 17 to 32 rows, us, the library's product and `qkv_write` / the few-rows kernel with everything
+    # in one launch, on weights that no cache holds: 24 rows 6,144 x 2,048 17.4 / 12.3, 4,608 x 3,072 17.3 / 14.3, 7,680 x 2,560
+    # 17.8 / 14.9, 4,608 x 4,096 (18.9 M elements) 18.9 / 17.0; 32 rows 15.0 / 13.1, 17.1 / 15.3, 18.3 / 16.2, 19.1 / 18.2;
+    # 12,288 x 4,096 33 / 33.7 and 33.6 / 38.2.
     fused_matrix = 20 << 20
+    # Products of 17 to 24 rows with a bfloat16 result likewise: 24 rows 6,144 x 2,048 13.0 / 11.4, 8,192 x 2,048 14.8 / 12.2;
+    # 7,680 x 2,560 13.0 / 13.8, and 8,320 x 2,048, whose blocks are more than one a unit, 15.1 / 19.0. Those of 25 to 32 rows
+    # have no clear winner.
+    plain_matrix = 1 << 24
 
     # ---------------------------------------------------------------- attention
 
