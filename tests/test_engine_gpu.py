@@ -300,7 +300,9 @@ def test_recorded_decode_steps_equal_open_ones(tiny_folders, tiny_folders_bf16, 
     if dtype.endswith("library"):
         dtype = "bfloat16"
         monkeypatch.setattr(HipOps, "library_rows", 2)
-        monkeypatch.setattr(HipOps, "small_matrix", 0)
+        for line in ("small_matrix", "fused_matrix", "plain_matrix"):
+            monkeypatch.setattr(HipOps, line, 0)
+        monkeypatch.setattr(HipOps, "tile_products", False)
     folder, cfg, weights = (tiny_folders if dtype == "float32" else tiny_folders_bf16)["B"]
     requests = _requests(cfg, [60, 3, 90], seed=17)
     expected = _expected(weights, cfg, requests)
@@ -395,11 +397,13 @@ def test_recorded_decoding_across_the_marks_of_256_keys(tmp_path, dtype, batch, 
     print(f"{dtype}, {batch} requests: worst error {worst:.2e} of the logit range")
 
 
-def test_schedules_with_library_products(tiny_folders_bf16, tmp_path, monkeypatch):
-    """The path long prompts take (vendor library for the plain products, our kernels around them), forced
-    on the tiny model by lowering the row count it starts at."""
+@pytest.mark.parametrize("tiles", [False, True])
+def test_schedules_with_library_products(tiny_folders_bf16, tmp_path, monkeypatch, tiles):
+    """The path long prompts take (vendor library for the plain products, or tiles of ours where those are taken, our
+    kernels around them), forced on the tiny model by lowering the row count it starts at."""
     from transformers_neuronx_amd.kernels.hip import HipOps
     monkeypatch.setattr(HipOps, "library_rows", 8)
+    monkeypatch.setattr(HipOps, "tile_products", tiles)
     folder, cfg, weights = tiny_folders_bf16["A"]
     requests = _requests(cfg, [17, 100, 128], seed=5)
     expected = _expected(weights, cfg, requests)

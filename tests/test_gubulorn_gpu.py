@@ -335,8 +335,8 @@ def test_attention_with_a_sink_finds_the_key_that_stands_out(name, dtype, tol, c
     (300, 60, 12, 6, 8, 3, 128, 24), (900, 6, 2, 4, 4, 2, 128, 64), (700, 1, 1, 1, 1, 1, 64, 32), (40, 100, 50, 5, 75, 3, 32, 8)])
 @pytest.mark.parametrize("forced", [None, "ours", "plain"])
 def test_experts_chosen_inside_groups_and_experts_without_tensors(name, dtype, tol, sizes, forced):
-    """`forced`: None, as the engine would (steps of many pairs an expert through the vendor library); "ours": the one
-    launch of ours at any size; "plain": without the matrix unit."""
+    """`forced`: None, as the engine would (steps of many pairs an expert by tiles where sizes are in 64s, else through the
+    vendor library); "ours": the launch with tiles of 16 pairs at any size; "plain": without the matrix unit."""
     from transformers_neuronx_amd.parts.feed_forward import ExpertMixture
     tokens, experts, identity, top, count, keep, width, inner = sizes
     if forced and (dtype == torch.float32 or (forced == "ours" and tokens < 100)):

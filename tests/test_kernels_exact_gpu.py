@@ -52,6 +52,7 @@ PRODUCT_CASES = [
     (32, 512, 2048, "few"), (24, 4096, 16384, "few"),
     (40, 4096, 4096, "some"), (64, 1024, 16384, "some"), (128, 256, 2048, "some"), (17, 4096, 4096, "some"),
     (64, 4096, 4096, "library"), (300, 1024, 2048, "library"), (2048, 512, 4096, "library"),
+    (64, 4096, 4096, "tiles"), (300, 1024, 2048, "tiles"), (150, 1280, 8192, "tiles"),
     (256, 1024, 4096, "wide"), (700, 520, 1024, "wide"), (2048, 4096, 1024, "wide"), (130, 264, 136, "wide"),
 ]
 
@@ -63,6 +64,7 @@ def test_products_of_small_integers_are_exact(m, n, k, way):
         hip.library_rows = 0            # our own kernels at every row count
     if way != "some":
         hip.some_rows = False
+    hip.tile_products = way == "tiles"
     g = torch.Generator(device=DEV).manual_seed(m + 3 * n + 7 * k)
     x, w = _ints(g, m, k).to(torch.bfloat16), _ints(g, n, k).to(torch.bfloat16)
     bias, residual = _ints(g, n, low=-64, high=64), _ints(g, m, n, low=-1000, high=1000)
@@ -70,8 +72,9 @@ def test_products_of_small_integers_are_exact(m, n, k, way):
     assert (pw.tiles is not None) == (n % 16 == 0 and k % 128 == 0)
     if way == "some":
         assert hip._some_rows_product(m, n, k, w, pw.tiles, residual, True, False)
-    if way == "library":
+    if way in ("library", "tiles"):
         assert hip._library_product(m, n, k, w, False)
+        assert (hip._tiles_room(m, n, k, x, w, residual, True, False) >= 0) == (way == "tiles")
     for weight in (pw, w):
         # what ends in the residual sum (float32), what a bfloat16 part reads next (with and without ReLU)
         got = hip.linear(x, weight, bias, residual=residual, out_f32=True)
@@ -130,6 +133,7 @@ def test_projection_that_turns_pairs_is_exact(m, own, normed):
     hip, ref = _ops(torch.bfloat16)
     if own:
         hip.library_rows = 0
+    hip.tile_products = False
     heads, kv, hs, ps, k = 3, 1, 32, 16, 256
     g = torch.Generator(device=DEV).manual_seed(m)
     cached = [int(c) for c in torch.randint(0, 90, (m,), generator=torch.Generator().manual_seed(m))]

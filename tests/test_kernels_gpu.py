@@ -621,10 +621,12 @@ def test_fused_projection_writes_what_the_two_kernels_write(dtype, heads, kv, hs
                                    (2048, 512, 1024)])
 def test_library_product_and_own_product_agree(m, n, k):
     """From `library_rows` rows on the plain product goes to the vendor library and our epilogue kernel
-    follows; below it, and always when told so, our own tiled kernel does all of it."""
+    follows, or to tiles of ours where those are taken; below it, and always when told so, our own tiled kernel does all of
+    it."""
     from transformers_neuronx_amd.kernels.hip import HipOps
     _, ref = _ops(torch.bfloat16)
-    lib, own = HipOps(torch.bfloat16, DEV), HipOps(torch.bfloat16, DEV)
+    lib, own, tiles = HipOps(torch.bfloat16, DEV), HipOps(torch.bfloat16, DEV), HipOps(torch.bfloat16, DEV)
+    lib.tile_products = False
     own.library_rows = 0
     g = torch.Generator(device=DEV).manual_seed(m + n)
     x = torch.randn(m, k, device=DEV, generator=g).to(torch.bfloat16)
@@ -636,7 +638,7 @@ def test_library_product_and_own_product_agree(m, n, k):
                    dict(act="relu", residual=res, out_f32=True), dict(act="gelu_new", residual=res, out_f32=True)):
         b = kwargs.pop("bias", bias)
         want = ref.linear(x, w, b, **kwargs).float()
-        for ops in (lib, own):
+        for ops in (lib, own, tiles):
             torch.testing.assert_close(ops.linear(x, w, b, **kwargs).float(), want, rtol=2e-2, atol=2e-2)
     # the head's float32 output never goes through a bfloat16 product
     torch.testing.assert_close(lib.linear(x, w, None, out_f32=True), ref.linear(x, w, None, out_f32=True),
@@ -647,7 +649,7 @@ def test_library_product_and_own_product_agree(m, n, k):
     torch.testing.assert_close(lib.linear(x, w, None, residual=res, out_f32=True), exact, rtol=1e-3, atol=1e-3)
     torch.testing.assert_close(lib.linear(x, w, bias, residual=res, out_f32=True), exact + bias, rtol=1e-3, atol=1e-3)
     rounded = HipOps(torch.bfloat16, DEV)
-    rounded.library_direct = False
+    rounded.library_direct = rounded.tile_products = False
     torch.testing.assert_close(rounded.linear(x, w, bias, residual=res, out_f32=True), exact + bias, rtol=2e-2, atol=2e-2)
 
 

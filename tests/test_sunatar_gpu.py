@@ -200,8 +200,8 @@ def test_router_and_experts(name, dtype, tol, sizes):
 @pytest.mark.parametrize("weight_on,score,renormalize", [("input", "sigmoid", False), ("output", "softmax", True)])
 @pytest.mark.parametrize("forced", [None, "ours", "plain"])
 def test_experts_of_a_step_of_many_tokens(weight_on, score, renormalize, forced):
-    """Many pairs an expert: the experts' products go to the vendor library over rows in expert order (the host
-    reads where each expert's rows begin); `forced`: the same step held on our own kernels, with and without the
+    """Many pairs an expert, an inner size that is not in 64s: the experts' products go to the vendor library over rows in
+    expert order (the host reads where each expert's rows begin); `forced`: the same step held on our own kernels, with and without the
     matrix unit. All against sums made token by token, with the router's own choice."""
     from transformers_neuronx_amd.parts.feed_forward import ExpertMixture
     tokens, experts, top, width, inner = 700, 4, 2, 128, 72

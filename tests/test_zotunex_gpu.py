@@ -283,11 +283,12 @@ def test_prompt_latent_attention_on_expanded_keys_with_a_sink_and_a_gate(case):
 @pytest.mark.parametrize("sizes", [
     # tokens, experts, a token's experts, width, inner size, shared inner size, limit
     (1, 4, 1, 64, 16, 0, 1.0), (37, 5, 2, 96, 40, 24, 0.7), (130, 10, 1, 192, 72, 88, 2.0), (9, 3, 3, 50, 30, 10, 0.5),
-    (300, 70, 4, 128, 24, 0, 7.0), (1300, 8, 4, 128, 64, 96, 1.0)])
+    (300, 70, 4, 128, 24, 0, 7.0), (1300, 8, 4, 128, 64, 96, 1.0),
+    (1300, 8, 4, 128, 72, 96, 1.0)])
 @pytest.mark.parametrize("forced", [None, "ours", "plain"])
 def test_corrected_choice_and_clamped_experts(name, dtype, tol, sizes, forced):
-    """`forced`: None, as the engine would (steps of many pairs an expert through the vendor library); "ours": the one
-    launch of ours at any size; "plain": without the matrix unit."""
+    """`forced`: None, as the engine would (steps of many pairs an expert by tiles where sizes are in 64s, else through the
+    vendor library); "ours": the launch with tiles of 16 pairs at any size; "plain": without the matrix unit."""
     from transformers_neuronx_amd.parts.feed_forward import ExpertMixture
     from types import SimpleNamespace
     tokens, experts, top, width, inner, shared, limit = sizes

@@ -351,8 +351,8 @@ def test_attention_mixers_alone(name, dtype, tol, kind):
     (900, 6, 4, 128, 64, 64), (700, 1, 1, 64, 32, 32), (40, 100, 5, 32, 8, 16), (8, 16, 2, 1024, 512, 256), (600, 3, 1, 64, 40, 0)])
 @pytest.mark.parametrize("forced", [None, "ours", "plain"])
 def test_experts_without_gates_beside_a_shared_one_with_a_number(name, dtype, tol, sizes, forced):
-    """`forced`: None, as the engine would (steps of many pairs an expert through the vendor library); "ours": the one
-    launch of ours at any size; "plain": without the matrix unit."""
+    """`forced`: None, as the engine would (steps of many pairs an expert by tiles where sizes are in 64s, else through the
+    vendor library); "ours": the launch with tiles of 16 pairs at any size; "plain": without the matrix unit."""
     from transformers_neuronx_amd.parts.feed_forward import ExpertMixture
     tokens, experts, top, width, inner, shared = sizes
     if forced and (dtype == torch.float32 or (forced == "ours" and tokens < 100)):
