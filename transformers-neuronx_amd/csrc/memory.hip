@@ -421,6 +421,8 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
       nrm[j] = d < a.n ? np_[d] : 0.f;
     }
   }
+  const size_t run_at = (size_t)head * a.tokens + start;
+  const float *my_keeps = keeps + run_at, *my_takes = takes + run_at, *my_floors = floors + run_at;
   f32x4 rq[QN], rk[QN], rv = {0.f, 0.f, 0.f, 0.f};
   float rt[QN], rkeep = 1.f, rfl = 0.f;
   auto fetch = [&](int t0) {
@@ -432,7 +434,7 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
       const float* row = a.proj + (size_t)(start + t0 + (in ? t : 0)) * a.ld + head * a.n + d;
       rq[u] = load4<ALIGNED>(row, in ? a.n - d : 0);
       rk[u] = load4<ALIGNED>(row + hn, in ? a.n - d : 0);
-      rt[u] = in ? takes[(size_t)head * a.tokens + start + t0 + t] : 0.f;
+      rt[u] = in ? my_takes[t0 + t] : 0.f;
     }
     if (threadIdx.x < CH * 4) {                            // a token's 16 values: four pieces
       const int t = threadIdx.x >> 2, c = 16 * cb + 4 * (threadIdx.x & 3);
@@ -441,8 +443,8 @@ __global__ void __launch_bounds__(256) memory_cell_kernel(CellArgs a, const floa
     }
     if (threadIdx.x < CH) {
       const bool in = threadIdx.x < len;
-      rkeep = in ? keeps[(size_t)head * a.tokens + start + t0 + threadIdx.x] : 1.f;
-      rfl = in ? floors[(size_t)head * a.tokens + start + t0 + threadIdx.x] : 1.f;
+      rkeep = in ? my_keeps[t0 + threadIdx.x] : 1.f;
+      rfl = in ? my_floors[t0 + threadIdx.x] : 1.f;
     }
   };
   auto stash = [&]() {
