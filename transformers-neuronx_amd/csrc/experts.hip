@@ -747,7 +747,10 @@ extern "C" int tnx_gated_activation(const float* gate_up, void* out, int dtype, 
   TNX_REQUIRE(dtype == TNX_F32 || dtype == TNX_BF16, "gated_activation: dtype %d", dtype);
   if (tokens == 0) return 0;
   const size_t total = (size_t)tokens * f;
-  const bool fours = f % 4 == 0 && (uintptr_t)gate_up % 16 == 0 && (uintptr_t)out % (dtype == TNX_F32 ? 16 : 8) == 0;
+  // (fewer elements than threads the units hold half of: one a thread. 33 rows of 4,096 2.64 us, four a thread 2.96; 33 of 8,192
+  // 3.00 and 3.00, 100 of 4,096 3.36 and 3.08.)
+  const bool fours = f % 4 == 0 && (uintptr_t)gate_up % 16 == 0 && (uintptr_t)out % (dtype == TNX_F32 ? 16 : 8) == 0 &&
+                     total > (size_t)1024 * tnx_compute_units();
 #define GATED_LAUNCH(T, V)                                                                                              \
   gated_activation_kernel<T, V><<<blocks_for(total / V), 256, 0, stream>>>(gate_up, (T*)out, f / V, act, total / V,      \
                                                                            row_weights, limit)
