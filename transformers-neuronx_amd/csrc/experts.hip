@@ -295,7 +295,7 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
   extern __shared__ __attribute__((aligned(16))) bf16_t staged[];     // [4 PARTS][ROWS * LD]
   __shared__ int pairs_of[64];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
-  const int part = wave >> 2, col0 = (blockIdx.x * 4 + (wave & 3)) * 16;
+  const int part = PARTS > 1 ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0, col0 = (blockIdx.x * 4 + (wave & 3)) * 16;
   int e = 0, pair;
   if (p.chosen) {
     // block y is tile y / experts of expert y % experts: its pairs are the lanes whose choice it is
@@ -350,7 +350,7 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
 #pragma unroll
     for (int i = 0; i < LOADS; ++i) got[i] = (src[i] != nullptr && k0 + lcol < p.k) ? load_once(src[i] + k0) : zero8;
   };
-  if (k_begin < k_end) ask(k_begin);
+  ask(k_begin);       // (a part beyond K asks for nothing; a branch around this made every load wait for the one before)
   for (int k0 = k_begin; k0 < k_end; k0 += KC) {
     bf16x8 x[STEPS];
 #pragma unroll
