@@ -143,7 +143,7 @@ def test_few_rows_with_a_rounded_result(n, k, few):
 
 
 @pytest.mark.parametrize("tokens,top", [(1, 2), (3, 3), (8, 2), (9, 7), (32, 2), (33, 2), (16, 4)])
-@pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72)])
+@pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72), (1, 1088, 40), (300, 72, 48)])
 @pytest.mark.parametrize("act,on", [("silu", "input"), ("relu2", "output")])
 def test_experts_of_few_pairs(tokens, top, experts, width, f, act, on):
     """Up to 64 pairs (the blocks find theirs) and beyond, one set of waves or two, experts with no pair and with all."""

@@ -283,31 +283,45 @@ __global__ void __launch_bounds__(256) expert_product_kernel(ProductArgs p) {
 // PARTS: the waves of a block come in so many sets of four, each with its part of K; the sets' sums meet in LDS. Where a step
 // is a few tokens an expert has one tile and a unit one block: with two sets there are twice as many loads under way, and half
 // as many chunks one after the other (measured at `launch_products`).
-template <int KIND, int PARTS>
+// FOUND: up to 64 pairs, whose choices a wave holds: a block finds its expert and pairs in them, and no launch orders them
+// first. Tiles are numbered without gaps, as the ordered ones are: blocks without one end at once, and where they stand between
+// the others some units get two blocks and some none (4,096 wide, 8 pairs of 8 experts: 97 us a layer with a tile an expert
+// whether it has pairs or not, 88.6 ordered).
+template <int KIND, int PARTS, bool FOUND>
 __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(ProductArgs p) {
   constexpr bool GATED = KIND == UP_GATED, UP = KIND != DOWN;
   constexpr int TM = 16;
   constexpr int ROWS = GATED ? 32 : 16;                   // rows of the matrix a wave holds
-  constexpr int KC = 256;                                 // elements of a row a chunk
+  constexpr int KC = 256;                                 // elements of K a chunk
   constexpr int LD = KC + 8;                              // a row in LDS: 16 bytes more, so that rows lie in different banks
   constexpr int LPR = KC / 8, RPI = 64 / LPR;             // lanes a row, rows an instruction
   constexpr int LOADS = ROWS / RPI;
   extern __shared__ __attribute__((aligned(16))) bf16_t staged[];     // [4 PARTS][ROWS * LD]
-  __shared__ int pairs_of[64];
+  __shared__ int pairs_of[FOUND ? TM : 1];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r = lane & 15, g = lane >> 4;
   const int part = PARTS > 1 ? __builtin_amdgcn_readfirstlane(wave >> 2) : 0, col0 = (blockIdx.x * 4 + (wave & 3)) * 16;
   int e = 0, pair;
-  if (p.chosen) {
-    // block y is tile y / experts of expert y % experts: its pairs are the lanes whose choice it is
-    e = blockIdx.y % p.experts;
-    const bool its = lane < p.pairs && p.chosen[min(lane, p.pairs - 1)] == e;
-    const unsigned long long all = __ballot(its);
-    const int begin = blockIdx.y / p.experts * TM;
-    if (__popcll(all) <= begin) return;
+  if constexpr (FOUND) {
+    const int mine = lane < p.pairs ? p.chosen[lane] : -1;
+    const bool counts = mine >= 0 && mine < p.experts;    // (beyond: an expert without tensors)
+    const unsigned long long below = (1ull << lane) - 1;
+    unsigned long long same = __ballot(counts);           // the lanes of the same expert, a bit of its number at a time
+    for (int b = 0; 1 << b < p.experts; ++b) {
+      const unsigned long long set = __ballot((mine >> b) & 1);
+      same &= (mine >> b) & 1 ? set : ~set;
+    }
+    const int place = __popcll(same & below);             // among the pairs of its expert; every 16th begins a tile
+    const bool begins = counts && place % TM == 0;
+    const unsigned long long all = __ballot(begins);
+    const unsigned long long its = __ballot(begins && __popcll(all & below) == (int)blockIdx.y);
+    if (its == 0) return;
+    const int from = __ffsll(its) - 1, begin = __shfl(place, from);
+    e = __builtin_amdgcn_readfirstlane(__shfl(mine, from));
+    const bool in = counts && mine == e && place >= begin && place < begin + TM;
     // (every wave writes the same numbers; a wave's LDS operations keep their order)
-    if (its) pairs_of[__popcll(all & ((1ull << lane) - 1))] = lane;
+    if (in) pairs_of[place - begin] = lane;
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    pair = begin + r < __popcll(all) ? pairs_of[begin + r] : -1;
+    pair = r < __popcll(__ballot(in)) ? pairs_of[r] : -1;
   } else {
     int tile = blockIdx.y, begin = 0, end = 0;
     for (; e < p.experts; ++e) {
@@ -321,7 +335,9 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
     begin += tile * TM;
     pair = begin + r < end ? p.order[begin + r] : -1;
   }
-  const float weight = pair >= 0 ? p.weights[pair] : 0.f;
+  if (PARTS == 1 && col0 >= p.n) return;
+  float weight = 0.f;                                     // (asked for first where the pair is known at once)
+  if (FOUND && pair >= 0) weight = p.weights[pair];
   const bf16_t* xrow = (const bf16_t*)p.a + (size_t)(pair < 0 ? 0 : (UP ? pair / p.top : pair)) * p.k;
   const bf16_t* W = (const bf16_t*)p.w + (size_t)e * (GATED ? 2 : 1) * p.n * p.k;
   bf16_t* mine = staged + wave * (ROWS * LD);
@@ -386,6 +402,7 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
     }
   }
   if (pair < 0) return;
+  if (!FOUND) weight = p.weights[pair];
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int col = col0 + 4 * g + i;        // the lane holds columns 4 g .. 4 g + 3 of pair r
@@ -405,17 +422,17 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
   }
 }
 
-template <int KIND, int PARTS>
+template <int KIND, int PARTS, bool FOUND>
 int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
   constexpr int bytes = 4 * PARTS * (KIND == UP_GATED ? 32 : 16) * (256 + 8) * 2;
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)expert_product_mfma_kernel<KIND, PARTS>,
+    hipError_t e = hipFuncSetAttribute((const void*)expert_product_mfma_kernel<KIND, PARTS, FOUND>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     TNX_REQUIRE(e == hipSuccess, "expert products: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
     configured = true;
   }
-  expert_product_mfma_kernel<KIND, PARTS><<<grid, 256 * PARTS, bytes, stream>>>(p);
+  expert_product_mfma_kernel<KIND, PARTS, FOUND><<<grid, 256 * PARTS, bytes, stream>>>(p);
   return 0;
 }
 
@@ -426,8 +443,9 @@ int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
 template <int KIND>
 int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
   const long long blocks = (long long)grid.x * min(p.experts, p.pairs);
-  return p.k >= 1024 && blocks <= tnx_compute_units() ? launch_products<KIND, 2>(p, grid, stream)
-                                                       : launch_products<KIND, 1>(p, grid, stream);
+  const bool two = p.k >= 1024 && blocks <= tnx_compute_units();
+  if (p.chosen) return two ? launch_products<KIND, 2, true>(p, grid, stream) : launch_products<KIND, 1, true>(p, grid, stream);
+  return two ? launch_products<KIND, 2, false>(p, grid, stream) : launch_products<KIND, 1, false>(p, grid, stream);
 }
 
 // ---------------------------------------------------------------- many pairs an expert
@@ -660,15 +678,15 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
   const int pairs = tokens * top;
   const bool mfma = dtype == TNX_BF16 && width % 8 == 0 && f % 8 == 0 && !plain;
   // Up to 64 pairs the products' blocks find their pairs themselves (a wave holds all choices), which saves the launch that
-  // orders them (3 to 4 us); a tile of 16 pairs an expert for every 16 pairs then, most of them empty.
-  const bool found = mfma && pairs <= 64 && (long long)experts * ((pairs + 15) / 16) <= 4096;
+  // orders them (3 to 4 us).
+  const bool found = mfma && pairs <= 64;
   if (!found) {
     order_kernel<<<1, 1024, 2 * experts * sizeof(int), stream>>>(chosen, pairs, experts, first, order, nullptr, nullptr, top,
                                                                  nullptr, nullptr, nullptr, 0, 0);
     TNX_CHECK_LAUNCH("expert order");
   }
-  // the most tiles of 16 pairs: every expert may end in a part of one
-  const int tiles = found ? experts * ((pairs + 15) / 16) : pairs / 16 + experts;
+  // the most tiles of 16 pairs: every expert that has pairs may end in a part of one
+  const int tiles = pairs / 16 + min(experts, pairs);
   const int* look = found ? chosen : nullptr;
   ProductArgs up{h, w_gate_up, first, order, weights, nullptr, inner, experts, top, f, width, act, weight_on_input, pairs,
                  limit, 0, look};
