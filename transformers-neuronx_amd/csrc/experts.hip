@@ -436,14 +436,15 @@ int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
   return 0;
 }
 
-// Two sets of waves where K has two chunks for each and the blocks that find pairs are at most one a unit. Measured at two
-// choices among 8 experts, us a layer with one set and with two: 2,048 wide, 1 token 45.6 / 34.8, 8 tokens 56.2 / 47.1 (256
-// blocks), 32 tokens 56.4 / 49.4; 4,096 wide, 1 token (128 blocks) 75.1 / 61.6, 2 tokens (256) 89.5 / 89.6, 8 tokens (512)
-// 150.7 / 166.0.
+// Two sets of waves where K has two chunks for each and the blocks with a tile are at most one a unit: an expert has one tile
+// where its pairs are few, ten on average at most; more, and some have two. Measured at two choices among 8 experts, us a layer
+// with one set and with two: 2,048 wide, 1 token 45.6 / 31.7, 8 tokens 56.1 / 45.8 (256 blocks), 32 tokens 56.4 / 46.6, 33 tokens,
+// 66 pairs, ordered first, 56.7 / 50.5, 48 tokens (96 pairs, 12 an expert) 67.5 / 73.9; 4,096 wide, 1 token (128 blocks) 73.9 / 59.5,
+// 2 tokens (256) 80.5 / 70.2, 8 tokens (512) 151 / 166.
 template <int KIND>
 int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
-  const long long blocks = (long long)grid.x * min(p.experts, p.pairs);
-  const bool two = p.k >= 1024 && blocks <= tnx_compute_units();
+  const long long tiles = min(p.experts, p.pairs) + (p.pairs > 10 * p.experts ? p.pairs / 16 : 0);
+  const bool two = p.k >= 1024 && grid.x * tiles <= tnx_compute_units();
   if (p.chosen) return two ? launch_products<KIND, 2, true>(p, grid, stream) : launch_products<KIND, 1, true>(p, grid, stream);
   return two ? launch_products<KIND, 2, false>(p, grid, stream) : launch_products<KIND, 1, false>(p, grid, stream);
 }
