@@ -1,6 +1,6 @@
 """Queries, keys and values of many tokens at once against the same tokens a few at a time (which `test_sunatar_gpu` holds
-against 64-bit arithmetic): values go into their pages by tiles of 64 tokens and 64 elements from 48 tiles on, and every
-number is made by the same operations either way."""
+against 64-bit arithmetic): values of long runs go into their pages by tiles of 64 tokens and 64 elements from 48 tiles on, and
+every number is made by the same operations either way."""
 import numpy as np
 import pytest
 import torch

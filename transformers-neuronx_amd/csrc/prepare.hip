@@ -233,13 +233,14 @@ __global__ void __launch_bounds__(256) qkv_prepare_kernel(PrepareArgs a) {
 
 }  // namespace
 
+// `longest`: the tokens of the step's longest run.
 extern "C" int tnx_qkv_prepare(const float* proj, int ld, const float* q_weight, const float* k_weight, float eps,
                                const float* freqs, int half, int interleaved, const int* positions, float scale,
                                const float* mix_weight, const float* first, long long first_ld, const int* token_page,
                                const int* token_offset, void* q_out, void* k_pages, void* v_pages, long long page_stride,
                                int num_pages, int page_size, int dtype, int tokens, int heads, int groups, int n, int v,
                                int d, int per_head, int values_at, const float* head_scale, float temp_coef, int temp_every,
-                               hipStream_t stream) {
+                               int longest, hipStream_t stream) {
   TNX_REQUIRE(tokens >= 0 && heads > 0 && groups > 0 && n > 0 && v > 0, "qkv_prepare: bad sizes");
   TNX_REQUIRE(d >= n && d >= v, "qkv_prepare: cached heads of %d elements do not hold %d and %d", d, n, v);
   if (values_at < 0) values_at = heads * n + groups * n;
@@ -262,10 +263,13 @@ extern "C" int tnx_qkv_prepare(const float* proj, int ld, const float* q_weight,
   int shares = 1;
   while (shares < 8 && 6ll * tokens * shares <= tnx_compute_units() && heads * d >= 1024 * shares) shares *= 2;
   const dim3 grid(tokens, 3, shares);
-  // Values by tiles from 48 tiles on, fewer leave most units without one. us, a token at a time / by tiles, 32 query heads:
-  // 8 heads of 64, 256 tokens (32 tiles) 5.9 / 6.7, 400 (56) 6.8 / 6.8, 2,048 19.4 / 15.1; 8 of 128, 64 tokens (16) 6.3 / 6.8,
-  // 256 (64) 8.1 / 7.1, 2,048 30.6 / 25.6; 32 of 128, 128 tokens (128) 10.4 / 7.0, 2,048 81.7 / 40.4.
-  const bool tiled = ((long long)tokens + 63) / 64 * (((long long)groups * d + 63) / 64) >= 48;
+  // Values by tiles where a tile's tokens lie side by side in their pages, from runs of 64 tokens on, and where there is a block
+  // for every tile: from 100 tokens on, and from 48 tiles, fewer leave most units without one. us, a token at a time / by
+  // tiles, 32 query heads, one run: 8 heads of 64, 256 tokens (32 tiles) 5.9 / 6.7, 400 (56) 6.8 / 6.8, 2,048 19.4 / 15.1; 8 of
+  // 128, 160 (48) 7.5 / 6.9, 256 (64) 8.2 / 7.2, 2,048 30.6 / 25.6; 32 of 128, 80 (128) 8.4 / 9.4, 100 9.9 / 10.0, 128 10.4 / 7.1,
+  // 2,048 81.7 / 40.4. Requests of one token each, whose places are a page apart: 1 (64 tiles, 8 blocks) 4.3 / 16.9, 64 10.1 /
+  // 12.5, 200 17.5 / 20.4, 400 31.1 / 32.6.
+  const bool tiled = longest >= 64 && tokens >= 100 && ((long long)tokens + 63) / 64 * (((long long)groups * d + 63) / 64) >= 48;
   if (dtype == TNX_F32) {
     if (tiled) qkv_prepare_kernel<float, true><<<grid, 256, 0, stream>>>(a);
     else qkv_prepare_kernel<float, false><<<grid, 256, 0, stream>>>(a);

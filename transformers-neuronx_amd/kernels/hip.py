@@ -142,7 +142,7 @@ _SIGNATURES = {
         "tnx_qkv_prepare": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_int, _c_int, _c_void_p,
                             _c_float, _c_void_p, _c_void_p, _c_ll, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                             _c_ll, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
-                            _c_int, _c_void_p, _c_float, _c_int, _c_void_p],
+                            _c_int, _c_void_p, _c_float, _c_int, _c_int, _c_void_p],
     },
     "memory": {
         "tnx_matrix_memory": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
@@ -1599,7 +1599,7 @@ class HipOps:
                    k_pages.stride(0), num_pages, view.page_size, _code(self.dtype), t, num_heads, num_kv, head_size,
                    value_size, cache_head, int(bool(per_head)), -1 if values_at is None else int(values_at),
                    _ptr(head_scale), float(temperature[0]) if temperature else 0.0, int(temperature[1]) if temperature else 0,
-                   _stream(),
+                   ctx.max_run, _stream(),
                    work=lambda: (f"{t}x{need}", t * (need * 4 + (num_heads + 2 * num_kv) * cache_head * q.element_size()), 0.0))
         return q
 
