@@ -21,7 +21,7 @@ struct F32Attention {
   const int* tile_start;
   const int* decode_runs;
   float* out;
-  int table_width, page_size, num_pages, num_heads, num_kv, window;
+  int table_width, page_size, num_pages, num_heads, num_kv, window, num_tiles;
   size_t page_stride;    // elements from one page to the next
 };
 
@@ -46,6 +46,9 @@ __device__ __forceinline__ float other_half(float x) {      // of lane ^ 32
 // lane, and need no LDS: a wave's 64 products of 64 cycles over a block of 32 keys (head size 64) are paid for with
 // 16 KB of reads, 4 bytes a cycle. What bounds it is the rate of the float32 matrix instructions.
 // Measured at runs of 300 and 101 tokens, 32 heads of 64: 27 us, against 362 with one wave a query and plain FMA.
+// The block's number counts heads first, then tiles, then the 32 queries within a tile: blocks go round the XCDs in their
+// order, and of a short run only the first 32 queries are there. With these first only every fourth block had work, all on
+// two XCDs of eight: 8 runs of 2 tokens, 32 heads of 80, 30.4 us, 10.7 so.
 template <int HD>
 __global__ void __launch_bounds__(256, HD <= 64 ? 2 : 1)
 attention_prompt_f32_kernel(F32Attention a) {
@@ -55,11 +58,12 @@ attention_prompt_f32_kernel(F32Attention a) {
   extern __shared__ float merged[];                // [4][32][ROW], then m and l [4][32] each
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int l32 = lane & 31, half = lane >> 5;
-  const int run = a.tile_run[blockIdx.x >> 2];
+  const int h = blockIdx.x % a.num_heads, kvh = h / (a.num_heads / a.num_kv);
+  const int of_all = blockIdx.x / a.num_heads, tile = of_all % a.num_tiles;
+  const int run = a.tile_run[tile];
   const int first = a.run_start[run], count = a.run_start[run + 1] - first;
-  const int q0 = a.tile_start[blockIdx.x >> 2] + 32 * (blockIdx.x & 3);
+  const int q0 = a.tile_start[tile] + 32 * (of_all / a.num_tiles);
   if (q0 >= count) return;                         // the whole block
-  const int h = blockIdx.y, kvh = h / (a.num_heads / a.num_kv);
   const int cached = a.cached_lens[run];
   const int* tab = a.table + (size_t)run * a.table_width;
   const size_t nq = (size_t)a.num_heads * HD;
@@ -340,7 +344,9 @@ int launch(const F32Attention& a, int num_tiles, int num_decode, hipStream_t str
       TNX_REQUIRE(e == hipSuccess, "attention_f32: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
       configured = true;
     }
-    attention_prompt_f32_kernel<HD><<<dim3(4 * num_tiles, a.num_heads), 256, bytes, stream>>>(a);
+    const long long blocks = 4ll * num_tiles * a.num_heads;
+    TNX_REQUIRE(blocks < (1ll << 31), "attention_f32: too many tiles");
+    attention_prompt_f32_kernel<HD><<<(unsigned)blocks, 256, bytes, stream>>>(a);
     TNX_CHECK_LAUNCH("attention_prompt_f32");
   }
   if (num_decode > 0) {
@@ -369,7 +375,7 @@ extern "C" int tnx_attention_f32(const float* q, const float* k_pages, const flo
   a.q = q; a.k_pages = k_pages; a.v_pages = v_pages; a.run_start = run_start; a.cached_lens = cached_lens;
   a.table = table; a.tile_run = tile_run; a.tile_start = tile_start; a.decode_runs = decode_runs; a.out = out;
   a.table_width = table_width; a.page_size = page_size; a.num_pages = num_pages; a.num_heads = num_heads;
-  a.num_kv = num_kv; a.window = window;
+  a.num_kv = num_kv; a.window = window; a.num_tiles = num_tiles;
   a.page_stride = (size_t)num_kv * page_size * head_size + page_pad;
   switch (head_size) {
     case 16: return launch<16>(a, num_tiles, num_decode, stream);
