@@ -101,6 +101,24 @@ def test_float32_attention_keeps_a_value_that_is_no_number_to_its_readers():
     torch.testing.assert_close(got, clean, rtol=1e-5, atol=1e-5)
 
 
+@pytest.mark.parametrize("runs,cached", [([2], [0]), ([16], [0]), ([17], [0]), ([24], [0]), ([25], [0]), ([5, 1, 3], [11, 15, 0]), ([16, 16], [0, 0])])
+@pytest.mark.parametrize("heads,kv,hs", [(4, 2, 64), (32, 8, 128), (40, 40, 16)])
+def test_float32_attention_of_short_steps(runs, cached, heads, kv, hs):
+    """Either side of the lengths up to which a wave takes a query alone, beside the kernel that always does."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, plain, g, page, n = HipOps(torch.float32, DEV), HipOps(torch.float32, DEV), _gen(hs), 32, sum(runs)
+    plain.force_plain_attention = True
+    ctx, pages = _step(runs, cached, page, seed=3)
+    few = max(r + c for r, c in zip(runs, cached)) <= (24 if hs > 96 else 16) and n * heads <= 1024
+    assert hip._few_scores(ctx, heads, hs) == few
+    kp = torch.randn(pages, kv, page, hs, device=DEV, generator=g)
+    vp = torch.randn(pages, kv, hs, page, device=DEV, generator=g)
+    q = torch.randn(n, heads * hs, device=DEV, generator=g) * hs ** -0.5
+    got, want = (x.attention(q, heads, kv, hs, ctx, ctx.groups["full"], kp, vp) for x in (hip, plain))
+    # (the bound of `test_float32_attention`)
+    torch.testing.assert_close(got, want, rtol=0, atol=5 * (8 * hs + 760) * 2.0 ** -24)
+
+
 @pytest.mark.parametrize("runs,cached,first,last", [([160], [0], 32, 63), ([300], [0], 0, 31), ([33], [0], 32, 32), ([20], [90], 64, 95),
                                                     ([1], [200], 64, 127), ([1], [128], 128, 128), ([1], [700], 0, 63), ([1, 1], [63, 448], 0, 511)])
 @pytest.mark.parametrize("window", [None, 37])

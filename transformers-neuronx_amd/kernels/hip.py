@@ -1052,7 +1052,8 @@ class HipOps:
                        "general attention kernel (one wave a query), several times slower than the matrix-unit "
                        "kernels that pages of 16, 32, 64, ... tokens get")
         if (self.dtype == torch.float32 and not self.force_plain_attention and head_size <= 128 and "tile_run" in ctx.plan
-                and _ptr(q) % 16 == 0):
+                and not self._few_scores(ctx, num_heads, head_size)
+                and (_ptr(q) | _ptr(k_pages) | _ptr(v_pages)) % 16 == 0):
             tiles, singles = ctx.plan["tile_run"], ctx.plan["decode_runs"]
             self._call("attention_f32", "tnx_attention_f32", _ptr(q), _ptr(k_pages), _ptr(v_pages), _ptr(ctx.run_start),
                        _ptr(ctx.cached_lens), _ptr(view.block_table), view.width, view.page_size, num_pages, _ptr(tiles),
@@ -1087,6 +1088,15 @@ class HipOps:
                        _ptr(ctx.plan["longest_decode"]), pad,
                        _stream(), work=lambda: self._attention_work(ctx, "decode", num_heads, num_kv_heads, head_size, window, 2))
         return out
+
+    @staticmethod
+    def _few_scores(ctx, num_heads, head_size) -> bool:
+        """float32 steps with a prompt so short that a wave a query is done before the tiles' waves have met: up to 16 tokens (24
+        with heads above 96), and at most one wave a SIMD. us, a wave a query / tiles, 32 heads: of 64, 2 tokens 5.2 / 7.7, 16
+        7.1 / 8.8, 32 10.2 / 10.3; of 80, 16 9.6 / 10.5, 24 12.8 / 11.5; of 128, 2 6.2 / 11.1, 24 14.9 / 15.4, 32 18.8 / 16.9; 8
+        runs of 16, 64 heads of 128, 54 / 29."""
+        return (ctx.plan["tile_run"].numel() > 0 and ctx.num_tokens * num_heads <= 1024
+                and ctx.max_total <= (24 if head_size > 96 else 16))
 
     # What the choice between one and two sets of waves a block rests on: the time of one 64-key step of a
     # block, in microseconds, measured on an MI355X at head size 128 (a block alone on its compute unit, two
