@@ -224,7 +224,9 @@ sample_kernel(const float* __restrict__ logits, const float* __restrict__ temper
 
   // f(logit, token) for all of the row, in no order that counts. A block goes through a row several times and waits for memory
   // each time: 16 logits a thread are asked for together. 3 rows of 50,272, top-k of 50: 33 us, one at a time 56.
-  const bool fours = vocab % 4 == 0 && (uintptr_t)row % 16 == 0;
+  // (Rows of fewer than 8 logits a thread go one at a time: four at once leave threads without any. 1,000 logits, top-k of 50:
+  // 10.1 us one at a time, 13.1 by sixteen; 2,048 10.3 and 11.6.)
+  const bool fours = vocab % 4 == 0 && vocab >= 8 * SAMPLE_THREADS && (uintptr_t)row % 16 == 0;
   auto over_row = [&](auto f) __attribute__((always_inline)) {
     if (fours) {
       const f32x4* row4 = (const f32x4*)row;
