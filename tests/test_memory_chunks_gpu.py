@@ -73,25 +73,32 @@ def test_memory_by_chunks(sizes, steps, gates, line):
 
 @pytest.mark.parametrize("column", ["query", "key", "value", "input gate", "forget gate"])
 @pytest.mark.parametrize("bad", [float("nan"), float("inf")])
-def test_a_token_that_is_no_number_leaves_the_ones_before_it(column, bad):
-    """One projection of token 70 of 130 is no number: the tokens before it are what they are without it, to the bit, and the
-    head's tokens from it on (of a query: the token alone) are no numbers. A gate's cap makes a number of an infinite one."""
+@pytest.mark.parametrize("at", [70, 129])
+def test_a_token_that_is_no_number_leaves_the_ones_before_it(column, bad, at):
+    """One projection of token 70 or of the last one of 130 is no number: the tokens before it are what they are without it, to
+    the bit, and the head's tokens from it on (of a query: the token alone) are no numbers. A gate's cap makes a number of an
+    infinite one. Token by token the same elements are no numbers, and the same of the state are none or infinite."""
     from transformers_neuronx_amd.kernels import make_ops
-    heads, n, v, at = 2, 64, 32, 70
+    heads, n, v = 2, 64, 32
     hn, hv = heads * n, heads * v
     ops = make_ops("hip", torch.float32, DEV)
-    ops.memory_chunk_run = 1
     g = torch.Generator().manual_seed(8)
     proj = torch.randn(130, 2 * hn + 2 * hv + 2 * heads, generator=g)
     weight = torch.rand(hv, generator=g) + 0.5
-    made = []
-    for spoil in (False, True):
+    made, states = [], []
+    for spoil, by_chunks in ((False, True), (True, True), (True, False)):
+        ops.memory_chunk_run = ops.memory_chunk_run_beside = 1 if by_chunks else 131
         x = proj.clone()
         if spoil:
             x[at, {"query": n, "key": hn + n, "value": 2 * hn + v, "input gate": -heads + -heads + 1, "forget gate": -1}[column]] = bad
         state = [torch.zeros(1, 2, heads, v, n, device=DEV), torch.zeros(1, 2, heads, n, device=DEV), torch.zeros(1, 2, heads, device=DEV)]
         made.append(ops.matrix_memory(x.to(DEV), heads, n, v, 9.0, 1e-5, weight.to(DEV), _ctx([130], [0], [0]), *state).cpu())
-    clean, spoilt = made
+        states.append([x[:, 1].cpu() for x in state])
+    clean, spoilt, walked = made
+    assert torch.equal(torch.isnan(spoilt), torch.isnan(walked))
+    for mine, theirs in zip(states[1], states[2]):
+        assert torch.equal(torch.isnan(mine), torch.isnan(theirs)) and torch.equal(torch.isposinf(mine), torch.isposinf(theirs))
+        assert torch.equal(torch.isneginf(mine), torch.isneginf(theirs))
     assert torch.isfinite(clean).all()
     assert torch.equal(clean[:at], spoilt[:at]) and torch.equal(clean[:, :v], spoilt[:, :v])      # (the head before: untouched)
     if not ("gate" in column and bad == float("inf")):

@@ -33,10 +33,12 @@ __device__ __forceinline__ float log_sigmoid(float z) {
   return fminf(z, 0.f) - log1pf(expf(-fabsf(z)));
 }
 
-// The recurrence is taken apart. The gates need nothing of S: one wave a (request, head) walks the run's tokens
-// (`memory_gates_kernel`), leaves every token's two factors exp(f + m - m'), exp(i - m') and the floor exp(-m') of
-// its denominator in memory, carries m on, and sets the normalizer the run begins with aside. The blocks that hold
-// S (`memory_cell_kernel`, 16 columns each) each carry the normalizer along as one more column, so that between
+// The recurrence is taken apart. The gates need nothing of S: one block a (request, head), of as many waves as the
+// longest run fills, takes a token a lane and joins their maxima (`memory_gates_kernel`), leaves every token's two factors
+// exp(f + m - m'), exp(i - m') and the floor exp(-m') of its denominator in memory, carries m on, and sets the normalizer
+// the run begins with aside. Long runs then go by chunks of 64 tokens (`memory_weights_kernel`, `memory_chunks_kernel`),
+// the others token by token. The blocks that hold
+// S (there `memory_cell_kernel`, 16 columns each) each carry the normalizer along as one more column, so that between
 // one token and the next there is nothing but multiply-adds and sums within 16 lanes, and no block reads state
 // that another writes: they read the normalizer from where the first kernel set it aside, and the block of a
 // head's first columns alone writes it back.
@@ -313,7 +315,8 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
     for (int s = 0; s < 4; ++s) ww[s] = w[s];
 #pragma unroll
     for (int s = 0; s < 16; ++s) {
-      vv[s] = v[s];
+      // (behind the run's end nothing, also of the last token's value: where that is infinite, zero times it is no number)
+      vv[s] = 16 * g + s < len ? v[s] : 0.f;
 #pragma unroll
       for (int u = 0; u < NU; ++u) kk[u][s] = 16 * g + s < len ? k[u][s] * ends[s] : 0.f;
     }
@@ -341,8 +344,10 @@ __global__ void __launch_bounds__(256, NT == 4 ? 2 : 1) memory_chunks_kernel(Cel
       sum += __shfl_xor(sum, 32);
       nrm[u] = keep_now * nrm[u] + sum;
     }
-    // A value that is no number must not reach the tokens before it, whose weight of it is zero: it is left out of the
-    // products, and the tokens from it on are no numbers in its column.
+    // A value that is infinite or no number must not reach the tokens before it, whose weight of it is zero: it is left out
+    // of the products, and the tokens from it on are no numbers in its column. (The walk adds up a row of S at a time: there
+    // an infinite value is an infinity of either sign a row, whose sum is no number either unless a token's products q_d k_d
+    // all have one sign, one token in 500 at 10 rows and none to speak of at 16.)
     int spoilt = 64;
     if (__any(probe != 0.f)) {
 #pragma unroll
