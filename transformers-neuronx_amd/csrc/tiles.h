@@ -1,5 +1,5 @@
-// The inner loop of bfloat16 products by tiles (those of the experts): out[row][column] = sum over k of x[row][k] w[column][k] for a tile of TM rows by TN columns, by the
-// waves of a block, with float32 sums.
+// The inner loop of bfloat16 products by tiles (plain ones in `gemm.hip`, those of the experts): out[row][column] = sum over k
+// of x[row][k] w[column][k] for a tile of TM rows by TN columns, by the waves of a block, with float32 sums.
 #pragma once
 #include "common.h"
 #include <type_traits>

@@ -2024,7 +2024,7 @@ class HipOps:
     # for 8 experts, two a token, us a layer, one launch of 16 pairs a tile or the library / tiles of 64 / of 128: 2,048 wide,
     # 12 pairs an expert 57 / 67 / 77, 16: 75 / 68 / 77, 50: 132 / 73 / 82, 99: 432 / 97 / 91, 512: 422 / 205 / 175; 4,096 wide,
     # 12: 199 / 218 / 209, 16: 218 / 216 / 208, 50: 469 / 224 / 209, 99: 449 / 283 / 220, 512: 795 / 688 / 543.
-    expert_grouped_rows = 16           # 0: never
+    expert_grouped_rows = 16           # 0: never (nor where `expert_library_rows` is 0: tiles of 16 pairs at any size then)
     expert_wide_tiles = 80
     # Other sizes, from this many pairs an expert on, in a step that is not being recorded: the host reads where each
     # expert's pairs begin (one small copy that waits for the device) and every expert's two products go to the vendor
