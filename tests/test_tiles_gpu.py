@@ -133,9 +133,11 @@ def test_products_that_the_tiles_leave_alone(m, n, k):
     assert ops._tiles_room(m, n, k, x, w, None, False, False) == -1
 
 
-@pytest.mark.parametrize("n,k,few", [(6144, 2048, True), (8192, 2048, True), (7680, 2560, False), (8320, 2048, False)])
+@pytest.mark.parametrize("n,k,few", [(6144, 2048, True), (8192, 2048, True), (7680, 2560, False), (8320, 2048, False), (4096, 4096, True),
+                                     (2048, 8192, False), (1024, 16384, False), (16384, 1024, True), (20480, 768, False), (2048, 4096, True),
+                                     (512, 16384, True)])
 def test_few_rows_with_a_rounded_result(n, k, few):
-    """17 to 24 rows go to the few-rows kernel up to 2^24 elements of the matrix."""
+    """17 to 24 rows go to the few-rows kernel up to 2^24 elements of the matrix, 2^23 where K is short or long."""
     from transformers_neuronx_amd.kernels.hip import HipOps
     ops, w = HipOps(torch.bfloat16, DEV), torch.empty(n, k, device=DEV, dtype=torch.bfloat16)
     for m in (17, 24):

@@ -851,7 +851,8 @@ class HipOps:
             return False
         # small matrices at up to 32 rows: one launch of ours (5 to 10 us with its epilogue) beats the
         # library's product and the epilogue after it (11 to 15 us)
-        few = self.fused_matrix if scattered else self.plain_matrix if plain and m <= 24 else self.small_matrix
+        few = (self.fused_matrix if scattered else self.plain_matrix if plain and m <= 24 and 1024 <= k <= 4096
+               else self.small_matrix)
         return not (m <= 32 and n * k <= few)
 
     small_matrix = 1 << 23
@@ -860,9 +861,11 @@ class HipOps:
     # 17.8 / 14.9, 4,608 x 4,096 (18.9 M elements) 18.9 / 17.0; 32 rows 15.0 / 13.1, 17.1 / 15.3, 18.3 / 16.2, 19.1 / 18.2;
     # 12,288 x 4,096 33 / 33.7 and 33.6 / 38.2.
     fused_matrix = 20 << 20
-    # Products of 17 to 24 rows with a bfloat16 result likewise: 24 rows 6,144 x 2,048 13.0 / 11.4, 8,192 x 2,048 14.8 / 12.2;
-    # 7,680 x 2,560 13.0 / 13.8, and 8,320 x 2,048, whose blocks are more than one a unit, 15.1 / 19.0. Those of 25 to 32 rows
-    # have no clear winner.
+    # Products of 17 to 24 rows with a bfloat16 result likewise, for K of 1,024 to 4,096: 24 rows 6,144 x 2,048 13.1 / 11.5, 8,192 x
+    # 2,048 14.7 / 12.1, 4,096 x 4,096 14.3 / 13.7, 3,072 x 3,072 11.0 / 10.5, 16,384 x 1,024 15.7 / 14.5; 17 rows 2,304 x 4,096
+    # 12.6 / 10.6. Not where a block's K is long (24 rows 2,048 x 5,120 11.4 / 13.8, 2,048 x 8,192 16.1 / 19.1, 1,024 x 16,384 19.1 /
+    # 33.8) or the blocks are more than one a unit (24 rows 8,320 x 2,048 15.1 / 19.0, 11,264 x 768 10.4 / 11.7, 20,480 x 768 14.1 /
+    # 17.8; also 7,680 x 2,560 13.0 / 13.8). Those of 25 to 32 rows have no clear winner.
     plain_matrix = 1 << 24
 
     # ---------------------------------------------------------------- attention
