@@ -144,6 +144,14 @@ def test_few_rows_with_a_rounded_result(n, k, few):
         assert ops._library_product(m, n, k, w, False, plain=True) != few
 
 
+@pytest.mark.parametrize("m,n,k,few", [(17, 6144, 2048, True), (32, 4608, 4096, True), (24, 2688, 7168, True), (17, 1536, 8192, False),
+                                       (32, 1024, 8192, True), (24, 18432, 1024, True), (25, 18432, 1024, False), (24, 12288, 4096, False)])
+def test_few_rows_of_queries_keys_and_values(m, n, k, few):
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops, w = HipOps(torch.bfloat16, DEV), torch.empty(n, k, device=DEV, dtype=torch.bfloat16)
+    assert ops._library_product(m, n, k, w, False, True) != few
+
+
 @pytest.mark.parametrize("tokens,top", [(1, 2), (3, 3), (8, 2), (9, 7), (32, 2), (33, 2), (16, 4)])
 @pytest.mark.parametrize("experts,width,f", [(4, 1024, 1040), (8, 200, 1288), (40, 1032, 72), (1, 1088, 40), (300, 72, 48)])
 @pytest.mark.parametrize("act,on", [("silu", "input"), ("relu2", "output")])

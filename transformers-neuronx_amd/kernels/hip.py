@@ -851,15 +851,19 @@ class HipOps:
             return False
         # small matrices at up to 32 rows: one launch of ours (5 to 10 us with its epilogue) beats the
         # library's product and the epilogue after it (11 to 15 us)
-        few = (self.fused_matrix if scattered else self.plain_matrix if plain and m <= 24 and 1024 <= k <= 4096
-               else self.small_matrix)
+        if scattered:
+            few = self.fused_matrix if k <= 4 * n and (n <= 1 << 14 or m <= 24) else self.small_matrix
+        else:
+            few = self.plain_matrix if plain and m <= 24 and 1024 <= k <= 4096 else self.small_matrix
         return not (m <= 32 and n * k <= few)
 
     small_matrix = 1 << 23
     # Queries, keys and values at 17 to 32 rows, us, the library's product and `qkv_write` / the few-rows kernel with everything
     # in one launch, on weights that no cache holds: 24 rows 6,144 x 2,048 17.4 / 12.3, 4,608 x 3,072 17.3 / 14.3, 7,680 x 2,560
     # 17.8 / 14.9, 4,608 x 4,096 (18.9 M elements) 18.9 / 17.0; 32 rows 15.0 / 13.1, 17.1 / 15.3, 18.3 / 16.2, 19.1 / 18.2;
-    # 12,288 x 4,096 33 / 33.7 and 33.6 / 38.2.
+    # 12,288 x 4,096 33 / 33.7 and 33.6 / 38.2. Long K of few columns goes to the library (24 rows 1,536 x 8,192 16.5 / 18.9, 1,536 x
+    # 7,168 16.3 / 17.4; 2,688 x 7,168 21.3 / 18.2), and more than 24 rows of so many columns that the blocks are more than one a
+    # unit (18,432 x 1,024: 24 rows 22.7 / 22.0, 32 rows 22.4 / 26.2; 24,576 x 768, 32 rows 21.0 / 22.3).
     fused_matrix = 20 << 20
     # Products of 17 to 24 rows with a bfloat16 result likewise, for K of 1,024 to 4,096: 24 rows 6,144 x 2,048 13.1 / 11.5, 8,192 x
     # 2,048 14.7 / 12.1, 4,096 x 4,096 14.3 / 13.7, 3,072 x 3,072 11.0 / 10.5, 16,384 x 1,024 15.7 / 14.5; 17 rows 2,304 x 4,096
