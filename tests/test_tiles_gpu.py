@@ -110,7 +110,7 @@ def test_product_by_tiles(m, n, k, tile, shares):
         assert bool(((out.double() - want).abs() <= bound).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(40, 2048, 2048), (100, 6144, 2048), (333, 2048, 8192)])
+@pytest.mark.parametrize("m,n,k", [(40, 2048, 2048), (100, 6144, 2048), (333, 2048, 8192), (512, 2048, 2048), (640, 6144, 2048), (640, 3072, 1024)])
 def test_products_that_the_tiles_take(m, n, k):
     """`linear` takes the tiles there, with what the library's way gives up to the rounding of the result."""
     from transformers_neuronx_amd.kernels.hip import HipOps
@@ -125,7 +125,8 @@ def test_products_that_the_tiles_take(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(64, 12288, 4096), (40, 16384, 4096), (600, 4096, 16384), (640, 4096, 16384), (700, 3072, 12288),
-                                   (705, 2048, 8192), (768, 5120, 20480), (768, 2048, 2048)])
+                                   (705, 2048, 8192), (768, 5120, 20480), (768, 2048, 2048), (513, 2048, 2048), (640, 3072, 2048),
+                                   (700, 1536, 2048)])
 def test_products_that_the_tiles_leave_alone(m, n, k):
     """Products that bound a step by their own time, at sizes where the library was measured to be quicker."""
     from transformers_neuronx_amd.kernels.hip import HipOps

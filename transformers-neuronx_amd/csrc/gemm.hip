@@ -1634,9 +1634,12 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 //   K up to 2,048: tiles of 64 x 64 where they make at most one and a quarter a unit, else of 128 x 128 at most one. 100 rows
 //   3,072 x 1,024 8.7 / 6.9, 6,144 x 2,048 14.1 / 13.4, 8,192 x 2,048 15.5 / 15.2; 333 rows 3,072 x 1,024 10.5 / 8.5, 6,144 x 2,048
 //   25.1 / 20.7, 8,192 x 2,048 24.0 / 21.7; 640 rows 6,144 x 2,048 24.9 / 23.5. The kernel alone is slower at 64 rows 6,144 x 2,048
-//   13.3 / 14.0 (a recorded step of 64 of 1.3b's 2,597 / 2,640), 160 to 300 rows 17.1 / 18.6 to 16.0 / 22.5 and 640 rows 2,048 x
-//   2,048 13.8 / 14.8: small enough for the host to bound the step. Above 640 rows tiles of 128 x 128 are to fill half the units:
-//   768 rows 2,048 x 2,048 (96) 14.1 / 19.1 (a prompt of 1.3b's with 768 tokens 4,037 with them, 3,624 without).
+//   13.3 / 14.0 (a recorded step of 64 of 1.3b's 2,597 / 2,640) and 160 to 300 rows 17.1 / 18.6 to 16.0 / 22.5: small enough for
+//   the host to bound the step. From 2^20 elements of x on (512 rows of K 2,048: there a step of 1.3b's is 3.6 ms of kernels, what
+//   the host takes with the library) tiles of 64 x 64 are to be at most one a unit, and from there on and above 640 rows those of
+//   128 x 128 are to fill half the units: 640 rows 2,048 x 2,048 (320 and 80) 15.2 / 16.9, 3,072 x 2,048 (120 of 128 x 128) 17.7 /
+//   24.4, 700 rows 1,536 x 2,048 13.6 / 15.2, 768 rows 2,048 x 2,048 (96) 14.1 / 19.1 (a prompt of 1.3b's with 768 tokens 4,037 with
+//   them, 3,624 without); up to it one and a quarter a unit lose less than the host's 8 us (333 rows 3,072 x 2,048 16.0 / 16.4).
 //   33 to 64 rows and K up to 4,096: tiles of 64 x 64 with shares. 48 rows 3,072 x 4,096 13.4 / 12.6, 4,096 x 4,096 14.2 / 13.6, 7,680 x
 //   2,560 16.0 / 16.4, 10,240 x 2,560 21.6 / 20.8. Not from 2^25 elements on: 64 rows 12,288 x 4,096 27.9 / 31.6, 16,384 x 4,096 32.6 /
 //   36.0 (a step of 64 of 6.7b's 6,075 with tiles there, 5,897 without).
@@ -1661,8 +1664,9 @@ static int choose_tiles(int M, int N, int K, int& shares) {
     if (K > 4096 && M > 128 && (M > 704 || 2 * blocks <= units || (M > 576 && 4 * blocks < 3 * units))) return TILES_NONE;
     return TILES_128;
   }
-  if (K <= 2048 && 4 * small <= 5 * units) return TILES_64;
-  if (K <= 2048 && large <= units && (M <= 640 || 2 * large > units)) return TILES_128;
+  const bool many = (long long)M * K > 1ll << 20;
+  if (K <= 2048 && 4 * small <= (many ? 4 : 5) * units) return TILES_64;
+  if (K <= 2048 && large <= units && ((M <= 640 && !many) || 2 * large > units)) return TILES_128;
   if (M <= 64 && K <= 4096 && small <= units && (long long)N * K < 1ll << 25) {
     shares = share_out(small);
     return TILES_64;
