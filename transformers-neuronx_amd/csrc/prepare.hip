@@ -233,7 +233,7 @@ __global__ void __launch_bounds__(256) qkv_prepare_kernel(PrepareArgs a) {
 
 }  // namespace
 
-// `longest`: the tokens of the step's longest run.
+// `longest`: the tokens of the step's longest run, or fewer where 64 of them or `tokens` below 100 say enough.
 extern "C" int tnx_qkv_prepare(const float* proj, int ld, const float* q_weight, const float* k_weight, float eps,
                                const float* freqs, int half, int interleaved, const int* positions, float scale,
                                const float* mix_weight, const float* first, long long first_ld, const int* token_page,
