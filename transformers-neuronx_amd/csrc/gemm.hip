@@ -1626,7 +1626,9 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 // (with bias and ReLU, or the residual where a matrix is narrower than K), at 33 to 768 rows:
 //   K at least four times the columns: tiles of 128 x 128 with as many shares of K as give every unit a block. 144 rows 2,048
 //   (columns) x 8,192 (K) 24.6 / 19.8, 2,560 x 10,240 32.3 / 26.0, 4,096 x 16,384 73.8 / 48.2, 5,120 x 20,480 123 / 71; 333 rows
-//   38.3 / 26.3, 49.0 / 35.5, 83.0 / 78.8, 142 / 106; 640 rows 43.8 / 37.6, 67.0 / 60.4, -, 224 / 193. Above 128 rows K beyond
+//   38.3 / 26.3, 49.0 / 35.5, 83.0 / 78.8, 142 / 106; 640 rows 43.8 / 37.6, 67.0 / 60.4, -, 224 / 193. Fewer rows come here only
+//   where `gemm_bf16_mid` has no copy of the weight: 33 rows 1,024 x 4,096 11.4 / 11.2, 2,048 x 8,192 14.4 / 16.9, 2,560 x 10,240
+//   23.1 / 20.6, 4,096 x 16,384 36.6 / 39.4, 64 rows 11.4 / 11.9, 16.8 / 17.0, 27.8 / 21.5, 43.9 / 39.5. Above 128 rows K beyond
 //   4,096 has to give more than half of the units a block, and three quarters above 576 rows (4,096 x 16,384, 160 blocks: 560
 //   rows 124 / 119, 600 rows 119 / 131, 640 rows 119 / 141; 700 rows 3,072 x 12,288, 144 blocks, 88 / 98), and above 704 rows the
 //   library has a better tile: 700 and 768 rows 2,048 x 8,192 44.6 / 42.8 and 43.6 / 49.0, 5,120 x 20,480 237 / 170 and 179 / 200.
