@@ -38,6 +38,36 @@ def test_float32_product(m, n, k):
     assert bool(torch.isfinite(got[rest]).all())
 
 
+@pytest.mark.parametrize("m,n,k", [(17, 64, 32), (64, 132, 96), (65, 2048, 224), (128, 129, 1024), (180, 3072, 1024), (401, 512, 2048)])
+def test_float32_product_by_parts(m, n, k):
+    """Products of more than 16 rows are made of the operands' bfloat16 parts: operands over twenty powers of two, whose lower
+    parts count, and numbers that have no parts. An element's error is at most one rounding of a running sum for each 16 of K
+    (h h; 16 exact products join it), one for the five other products' sums (2^-8 of the magnitudes, 5 roundings for each 16 of K),
+    what is left out (2^-26) and the shares' sum: together less than (k / 16 + 8) 2^-23 of the sum of magnitudes."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g = HipOps(torch.float32, DEV), _gen(m + n + k)
+
+    def some(*shape):
+        x = torch.randn(*shape, device=DEV, generator=g)
+        return x * torch.exp2(torch.randint(-10, 10, shape, device=DEV, generator=g).float())
+
+    x, w = some(m, k), some(n, k)
+    want, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    got = hip.linear(x, w, out_f32=True).double()
+    assert bool(((got - want).abs() <= (k / 16 + 8) * 2.0 ** -23 * size).all())
+    # infinities meet weights that one part holds whole (the others are 0), and numbers that round to an infinity
+    w[0], w[1] = 1.0, -0.5
+    x[0, 3], x[1, k - 1], x[2, 5], x[2, 6] = float("inf"), float("-inf"), float("inf"), float("-inf")
+    x[3], x[4], x[4, 7] = 0.0, 0.0, float("nan")
+    x[3, 1], w[2] = 3.4e38, 0.25
+    got = hip.linear(x, w, out_f32=True)
+    assert got[0, 0].item() == float("inf") and got[0, 1].item() == float("-inf")
+    assert got[1, 0].item() == float("-inf") and got[1, 1].item() == float("inf")
+    assert bool(got[2, :2].isnan().all()) and bool(got[4].isnan().all())
+    assert got[3, 2].item() == x[3, 1].item() * 0.25 and got[3, 1].item() == x[3, 1].item() * -0.5
+    assert bool(torch.isfinite(got[5:]).all())
+
+
 def _step(runs, cached, page, seed):
     from transformers_neuronx_amd.engine.batch import StepEntry, build_context
     from transformers_neuronx_amd.kernels.attention_plan import attention_plan

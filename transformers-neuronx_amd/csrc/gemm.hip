@@ -1,6 +1,6 @@
 // Matrix products `out[M, N] = act(x[M, K] w[N, K]^T + bias[N]) + residual[M, N]` with float32 accumulation.
-//   gemm_f32        float32 operands, on the float32 matrix instructions (nothing is rounded to fewer bits), on plain
-//                   FMA for few rows and for sizes that are no multiples of 32 in K
+//   gemm_f32        float32 operands, as three bfloat16 parts each on the matrix instructions (nothing of an operand is lost), on
+//                   plain FMA for few rows and for sizes that are no multiples of 32 in K
 //   gemm_bf16       bfloat16 operands on MFMA, many rows (prompts): 256x256x64 tiles, operands straight from
 //                   global memory into two LDS stages, four waves of 128x128 (sizes in whole 64-steps of K);
 //                   128x128 tiles staged through registers for every other size
@@ -261,136 +261,232 @@ static void f32_skinny(const float* x, const float* w, const float* bias, const 
     launch_f32_skinny<16>(x, w, bias, residual, out, out_dtype, act, M, N, K, sc, stream);
 }
 
-// Many rows in float32, on the float32 matrix instructions (32x32x2: products and sums in float32, no operand is
-// rounded): tiles of 64 MI rows of `x` by 64 NI of `w`, four waves (2 x 2) of 32 MI x 32 NI each. What bounds the product is
-// these instructions' rate (256 flops a cycle and unit: 157 TFLOP/s), 16 times below bfloat16's, so a plain pipeline feeds
-// them: tiles of 32 floats of K go straight into LDS, NSTAGE deep, 16-byte chunks swizzled by row; a lane reads four floats
-// of K of its row at once, which serve four instructions (which two places of K an instruction joins is free, as long as
-// both operands agree: here k and k + 4). The share of K that a block takes (gridDim.y of them) keeps the units busy where
-// the result has few tiles; its sums then go to `partial` and are added by `gemm_mid_sum_kernel`.
-// Measured at 401 rows, us (TFLOP/s), with these tiles and with the tiles of 64 x 64 on plain FMA that served such sizes
-// before: 8,192 columns of K 2,048: 159 (85) against 446; 6,144 of 2,048: 142 (71) against 372; 2,048 of 2,048 and of 8,192:
-// 52 (65) and 144 (93, with the sum of four shares) against 561 on average. Its error against 64 bits is the smaller one.
-template <int MI, int NI, int NSTAGE>
-__global__ void __launch_bounds__(256)
-gemm_f32_tiles_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
+// Many rows in float32, on the bfloat16 matrix instructions: every operand is the sum of three bfloat16 parts, x = h + m + l
+// with h = x rounded, m = (x - h) rounded and l the rest, which eight bits hold: nothing of x is lost. Of the nine products of
+// parts six are made, each exact, with float32 sums; l l, l m and m l, at most 2^-26 of |x w| between them, are left out. (Below
+// 2^-110 a lower part may be too small for a number: an operand is then off by 2^-133.)
+// The float32 instructions give 256 flops a cycle and unit, the bfloat16 ones 4,096, of which a sixth is 683.
+// h h has sums of its own, the other five share theirs: six times fewer roundings at the size of the result, which is why the
+// error against 64 bits is 0.34 to 0.7 of what the float32 instructions left (K 2,048: 2.7e-7 for 8.1e-7, 1,024: 1.9e-7 for 5.7e-7;
+// with one set of sums for all six 7.0e-7).
+// Tiles of 32 MI WM rows of `x` by 32 NI WN of `w`, 32 of K a step. A thread loads rows three steps ahead into registers, splits
+// them beside the products of the two steps before their own and leaves the parts in LDS, two stages of them (a split wave by
+// wave, from float32 in LDS, would be made again by every wave that shares the rows). Of a step of 128 x 128 the matrix cores
+// need 0.64 us; it takes 0.89 with a block on every fourth unit and 1.3 with one on each: the products alone, without loads,
+// splits and meetings, 0.56 and 0.8. Split between the products of both halves of a step; all in the first half, 1.06 and 1.4.
+// The share of K that a block takes (gridDim.y of them) keeps the units busy where the result has few tiles; its sums then go
+// to `partial` and are added by `gemm_mid_sum_kernel`.
+// Measured at 401 rows on weights that no cache holds, us, by the float32 instructions (32x32x2, which this took the place of) and
+// so: 8,192 columns of K 2,048 151 / 90, 6,144 of 2,048 134 / 75, 2,048 of 8,192 142 / 93, 2,048 of 2,048 46 / 33, 3,072 of 1,024
+// 44 / 26, 1,024 of 1,024 17.8 / 17.0.
+template <int MI, int NI, int WM, int WN>
+__global__ void __launch_bounds__(64 * WM * WN)
+gemm_f32_parts_kernel(const float* __restrict__ x, const float* __restrict__ w, const float* __restrict__ bias,
                       const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act,
-                      float* __restrict__ partial, int M, int N, int K, int tiles_m, int steps_per_share) {
+                      float* __restrict__ partial, int whole, int M, int N, int K, int tiles_m, int steps_per_share) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  constexpr int TM = 64 * MI, TN = 64 * NI, STAGE = (TM + TN) * 128;
-  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  constexpr int T = 64 * WM * WN, TM = 32 * MI * WM, TN = 32 * NI * WN, ROWS = TM + TN;
+  constexpr int PLANE = ROWS * 64, STAGE = 3 * PLANE;     // bytes: a part of a step's rows (32 of K), all three parts
+  constexpr int L = ROWS * 8 / T;                         // loads of a thread a step, of T / 8 rows each
+  static_assert(TM % (T / 8) == 0 && TN % (T / 8) == 0, "a load is of rows of x or of w");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int l32 = lane & 31, half = lane >> 5;
-  const int wm = (wave & 1) * 32 * MI, wn = (wave >> 1) * 32 * NI;
-  // blocks of one XCD (every eighth) take neighbouring tiles, those of the same columns of `w` first
-  const int nb = gridDim.x, xcd = blockIdx.x & 7, each = nb >> 3, more_of = nb & 7;
-  const int bid = xcd * each + min(xcd, more_of) + (blockIdx.x >> 3);
-  const int m0 = bid % tiles_m * TM, n0 = bid / tiles_m * TN;
+  const int wm = (wave % WM) * 32 * MI, wn = (wave / WM) * 32 * NI;
+  const int at = by_xcd(blockIdx.x, gridDim.x);
+  const int m0 = at % tiles_m * TM, n0 = at / tiles_m * TN;
   const int first = blockIdx.y * steps_per_share, steps = min(K / 32 - first, steps_per_share);
-
-  const int lrow = lane >> 3, lpos = lane & 7;
-  const float* xsrc[2 * MI];
-  const float* wsrc[2 * NI];
+  // 8 threads take the 128 bytes of a row; what a thread loads at step 0, in bytes from the tile's first row
+  const int lrow = tid >> 3, lchunk = tid & 7;
+  const auto xtile = __builtin_amdgcn_make_buffer_rsrc((void*)(x + (size_t)m0 * K + 32 * first), 0, -1, 0x00020000);
+  const auto wtile = __builtin_amdgcn_make_buffer_rsrc((void*)(w + (size_t)n0 * K + 32 * first), 0, -1, 0x00020000);
+  int from[L];
 #pragma unroll
-  for (int j = 0; j < 2 * MI; ++j) {
-    const int row = (2 * MI * wave + j) * 8 + lrow;
-    xsrc[j] = x + (size_t)min(m0 + row, M - 1) * K + 32 * first + 4 * (lpos ^ ((row >> 1) & 7));
+  for (int j = 0; j < L; ++j) {
+    const int row = j * (T / 8) + lrow;
+    from[j] = 4 * ((j * (T / 8) < TM ? min(row, M - 1 - m0) : min(row - TM, N - 1 - n0)) * K + 4 * lchunk);
   }
+  // 16-byte chunks (8 of K) of a row of 64 bytes, swizzled so that 16 rows' reads of one chunk meet no bank twice
+  char* dst = smem + lrow * 64 + (((lchunk >> 1) ^ ((lrow >> 2) & 3)) * 16) + (lchunk & 1) * 8;
+  f32x4 raw[3][L];
+  auto load = [&](int set, int t) {
+    const int k = 128 * min(t, steps - 1);
 #pragma unroll
-  for (int j = 0; j < 2 * NI; ++j) {
-    const int row = (2 * NI * wave + j) * 8 + lrow;
-    wsrc[j] = w + (size_t)min(n0 + row, N - 1) * K + 32 * first + 4 * (lpos ^ ((row >> 1) & 7));
-  }
-  auto issue = [&](int t) {
-    char* a_dst = smem + (t % NSTAGE) * STAGE + 2 * MI * wave * 1024;
-    char* b_dst = smem + (t % NSTAGE) * STAGE + TM * 128 + 2 * NI * wave * 1024;
-#pragma unroll
-    for (int j = 0; j < 2 * MI; ++j) load_to_lds(xsrc[j] + 32 * t, lds_offset(a_dst + j * 1024));
-#pragma unroll
-    for (int j = 0; j < 2 * NI; ++j) load_to_lds(wsrc[j] + 32 * t, lds_offset(b_dst + j * 1024));
+    for (int j = 0; j < L; ++j)
+      raw[set][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(j * (T / 8) < TM ? xtile : wtile, from[j], k, 0));
   };
-  f32x16 acc[MI][NI];
+  uint2 part[L][3];
+  auto split = [&](int set, int j) {
+    const f32x4 v = raw[set][j];
+    float r[4] = {v[0], v[1], v[2], v[3]};
+#pragma unroll
+    for (int p = 0; p < 3; ++p) {
+      typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
+      unsigned two[2];
+#pragma unroll
+      for (int e = 0; e < 2; ++e) {
+        const bf16x2 b = {(bf16_t)r[2 * e], (bf16_t)r[2 * e + 1]};
+        two[e] = __builtin_bit_cast(unsigned, b);
+        if (p < 2) {
+          r[2 * e] -= __uint_as_float(two[e] << 16);
+          r[2 * e + 1] -= __uint_as_float(two[e] & 0xffff0000u);
+        }
+      }
+      part[j][p] = make_uint2(two[0], two[1]);
+    }
+  };
+  auto write = [&](int stage, int j) {
+#pragma unroll
+    for (int p = 0; p < 3; ++p) *(uint2*)(dst + stage * STAGE + j * (T / 8) * 64 + p * PLANE) = part[j][p];
+  };
+  f32x16 acc[MI][NI], low[MI][NI];
 #pragma unroll
   for (int i = 0; i < MI; ++i)
 #pragma unroll
     for (int j = 0; j < NI; ++j)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+      for (int e = 0; e < 16; ++e) acc[i][j][e] = low[i][j][e] = 0.f;
+  const int swizzle = (l32 >> 2) & 3;
+  bf16x8 a[2][MI][3], b[2][NI][3];
+  auto frags = [&](int stage, int s) {
+    const char* base = smem + stage * STAGE + l32 * 64 + (((2 * s + half) ^ swizzle) * 16);
 #pragma unroll
-  for (int p = 0; p < NSTAGE - 1; ++p)
-    if (p < steps) issue(p);
-  const int swizzle = (l32 >> 1) & 7;
-  for (int t = 0; t < steps; ++t) {
-    // tile t has landed when at most the loads of the NSTAGE - 2 tiles behind it are still in flight
-    constexpr int L = 2 * MI + 2 * NI;
-    const int ahead = min(NSTAGE - 2, steps - 1 - t);
-    if (NSTAGE > 3 && ahead == 2) __builtin_amdgcn_s_waitcnt(0x0F70 | ((2 * L) & 15) | (((2 * L) >> 4) << 14));
-    else if (NSTAGE > 2 && ahead == 1) __builtin_amdgcn_s_waitcnt(0x0F70 | (L & 15) | ((L >> 4) << 14));
-    else __builtin_amdgcn_s_waitcnt(0x0F70);
-    __syncthreads();
-    if (t + NSTAGE - 1 < steps) issue(t + NSTAGE - 1);
-    const char* base = smem + (t % NSTAGE) * STAGE;
+    for (int p = 2; p >= 0; --p) {
 #pragma unroll
-    for (int s = 0; s < 4; ++s) {
-      const int chunk = ((2 * s + half) ^ swizzle) * 16;
-      f32x4 a[MI], b[NI];
+      for (int i = 0; i < MI; ++i) a[s][i][2 - p] = *(const bf16x8*)(base + (2 - p) * PLANE + (wm + 32 * i) * 64);
 #pragma unroll
-      for (int i = 0; i < MI; ++i) a[i] = *(const f32x4*)(base + (wm + 32 * i + l32) * 128 + chunk);
-#pragma unroll
-      for (int j = 0; j < NI; ++j) b[j] = *(const f32x4*)(base + TM * 128 + (wn + 32 * j + l32) * 128 + chunk);
-#pragma unroll
-      for (int c = 0; c < 4; ++c)
-#pragma unroll
-        for (int i = 0; i < MI; ++i)
-#pragma unroll
-          for (int j = 0; j < NI; ++j)
-            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j][c], a[i][c], acc[i][j], 0, 0, 0);
+      for (int j = 0; j < NI; ++j) b[s][j][p] = *(const bf16x8*)(base + p * PLANE + (TM + wn + 32 * j) * 64);
     }
-  }
-  // element e of a lane: row lane % 32, column 8 (e / 4) + 4 (lane / 32) + e % 4 of the 32 x 32
+  };
+  auto products = [&](int s) {
+    constexpr int pa[6] = {0, 0, 1, 1, 2, 0}, pb[6] = {2, 1, 1, 0, 0, 0};
 #pragma unroll
-  for (int i = 0; i < MI; ++i) {
-    const int m = m0 + wm + 32 * i + l32;
-    if (m >= M) continue;
+    for (int p = 0; p < 6; ++p)
 #pragma unroll
-    for (int j = 0; j < NI; ++j)
+      for (int i = 0; i < MI; ++i)
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int n = n0 + wn + 32 * j + 8 * g + 4 * half;
-        if (partial) {
-          // (N is a multiple of 4 here: four columns are inside or outside together)
-          if (n < N)
-            *(f32x4*)(partial + ((size_t)blockIdx.y * M + m) * N + n) =
-                (f32x4){acc[i][j][4 * g], acc[i][j][4 * g + 1], acc[i][j][4 * g + 2], acc[i][j][4 * g + 3]};
-        } else {
-#pragma unroll
-          for (int e = 0; e < 4; ++e)
-            if (n + e < N) epilogue_store(acc[i][j][4 * g + e], m, n + e, N, bias, residual, out, out_dtype, act);
+        for (int j = 0; j < NI; ++j) {
+          if (p < 5) low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[s][j][pb[p]], a[s][i][pa[p]], low[i][j], 0, 0, 0);
+          else acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(b[s][j][pb[p]], a[s][i][pa[p]], acc[i][j], 0, 0, 0);
         }
-      }
+  };
+  load(0, 0);
+  load(1, 1);
+  load(2, 2);
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int j = 0; j < L; ++j) split(0, j), write(0, j);
+#pragma unroll
+  for (int j = L / 2; j < L; ++j) split(1, j);
+  __syncthreads();
+  frags(0, 0);
+  // Step t (its rows in stage t % 2, the first half of its fragments in registers): the meeting is in the middle, and the next
+  // step's first fragments come during the second half; the next step's rows are split beside the products of both halves.
+  // (a product, and a share of the 11 instructions that two elements take to split, in turn)
+  auto in_turn = [&] {
+    constexpr int P = 6 * MI * NI, V = (11 * L + P - 1) / P;
+#pragma unroll
+    for (int i = 0; i < P; ++i) {
+      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+      __builtin_amdgcn_sched_group_barrier(0x2, V, 0);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  auto step = [&](auto place, int t) {
+    constexpr int u = decltype(place)::value, stage = u & 1;
+    frags(stage, 1);
+    load(u % 3, t + 3);
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int j = L / 2; j < L; ++j) write(stage ^ 1, j);
+    products(0);
+#pragma unroll
+    for (int j = 0; j < L / 2; ++j) split((u + 1) % 3, j), write(stage ^ 1, j);
+    in_turn();
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    frags(stage ^ 1, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    products(1);
+#pragma unroll
+    for (int j = L / 2; j < L; ++j) split((u + 2) % 3, j);
+    in_turn();
+  };
+  int t = 0;
+  for (; t + 6 <= steps; t += 6) {
+    step(std::integral_constant<int, 0>{}, t);
+    step(std::integral_constant<int, 1>{}, t + 1);
+    step(std::integral_constant<int, 2>{}, t + 2);
+    step(std::integral_constant<int, 3>{}, t + 3);
+    step(std::integral_constant<int, 4>{}, t + 4);
+    step(std::integral_constant<int, 5>{}, t + 5);
   }
+  if (t < steps) step(std::integral_constant<int, 0>{}, t);
+  if (t + 1 < steps) step(std::integral_constant<int, 1>{}, t + 1);
+  if (t + 2 < steps) step(std::integral_constant<int, 2>{}, t + 2);
+  if (t + 3 < steps) step(std::integral_constant<int, 3>{}, t + 3);
+  if (t + 4 < steps) step(std::integral_constant<int, 4>{}, t + 4);
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j) acc[i][j] += low[i][j];
+  // An element that is no finite number: an operand was none, or was rounded to one (from 3.395e38 on), and its parts are no
+  // sum of it. It is made again from the operands themselves.
+  auto checked = [&](float v, int m, int n) {
+    if (__builtin_expect(fabsf(v) <= 3.4028235e38f, 1)) return v;
+    const float *xr = x + (size_t)m * K + 32 * first, *wr = w + (size_t)n * K + 32 * first;
+    float sum = 0.f;
+    for (int k = 0; k < 32 * steps; ++k) sum = fmaf(xr[k], wr[k], sum);
+    return sum;
+  };
+  __syncthreads();      // the stages are free: the result goes through them
+  const int mw = m0 + wm, nw = n0 + wn;
+  float added[NI][16];
+#pragma unroll
+  for (int j = 0; j < NI; ++j)
+#pragma unroll
+    for (int e = 0; e < 16; ++e) added[j][e] = bias && !partial ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3), N - 1)] : 0.f;
+  auto value = [&](int i, int j, int e, int row, int column) {
+    const float v = mw + row < M && nw + column < N ? checked(acc[i][j][e], mw + row, nw + column) : 0.f;
+    return partial ? v : apply_act(v + added[j][e], act);
+  };
+  float* dest = partial ? partial + (size_t)blockIdx.y * M * N : (float*)out;
+  const float* onto = partial ? nullptr : residual;
+  Tile<MI, NI, 2, WM, WN>::template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
+    if (mw + r >= M || nw + c >= N) return;
+    const size_t o = (size_t)(mw + r) * N + nw + c;
+    if (whole) {
+      if (onto) chunk += *(const f32x4*)(onto + o);
+      *(f32x4*)(dest + o) = chunk;
+    } else {
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if (nw + c + e < N) store_any(out, out_dtype, o + e, chunk[e] + (onto ? onto[o + e] : 0.f));
+    }
+  });
 }
 
 __global__ void gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__ bias,
                                     const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
                                     int N, int shares);
 
-template <int MI, int NI, int NSTAGE>
-static int launch_f32_tiles(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
+template <int MI, int NI, int WM, int WN>
+static int launch_f32_parts(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
                             int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
-  constexpr int bytes = NSTAGE * (64 * MI + 64 * NI) * 128;
+  constexpr int bytes = 2 * 3 * (32 * MI * WM + 32 * NI * WN) * 64;
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_tiles_kernel<MI, NI, NSTAGE>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_f32_parts_kernel<MI, NI, WM, WN>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     TNX_REQUIRE(e == hipSuccess, "gemm_f32: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
     configured = true;
   }
-  const int tiles_m = (M + 64 * MI - 1) / (64 * MI), tiles_n = (N + 64 * NI - 1) / (64 * NI);
+  const int tiles_m = (M + 32 * MI * WM - 1) / (32 * MI * WM), tiles_n = (N + 32 * NI * WN - 1) / (32 * NI * WN);
   const int per = (K / 32 + shares - 1) / shares;
   shares = (K / 32 + per - 1) / per;
-  gemm_f32_tiles_kernel<MI, NI, NSTAGE><<<dim3(tiles_m * tiles_n, shares), 256, bytes, stream>>>(
-      x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, M, N, K, tiles_m, per);
-  TNX_CHECK_LAUNCH("gemm_f32_tiles");
+  // whole chunks of 16 bytes in every row of the result (of the shares' sums always: the caller sees to it)
+  const int whole = shares > 1 || (N % 4 == 0 && out_dtype == TNX_F32 && ((uintptr_t)out | (uintptr_t)residual) % 16 == 0);
+  gemm_f32_parts_kernel<MI, NI, WM, WN><<<dim3(tiles_m * tiles_n, shares), 64 * WM * WN, bytes, stream>>>(
+      x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, whole, M, N, K, tiles_m, per);
+  TNX_CHECK_LAUNCH("gemm_f32_parts");
   if (shares > 1) {
     gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
                                                                                         act, M, N, shares);
@@ -402,20 +498,21 @@ static int launch_f32_tiles(const float* x, const float* w, const float* bias, c
 // The most floats that the shares' sums of one product may take (32 MB).
 constexpr long long F32_SHARES_MOST = 8 << 20;
 
-// The tile and the shares of K: what the fullest compute unit has to do, in steps of 32 of K of a 64 x 64 tile (0.43 us at
-// the instructions' rate), a step in which a block fills and empties its pipeline, and the sum of the shares.
+// The tile (128 x 128, 64 x 128, 64 x 64) and the shares of K, by what the fullest compute unit takes in us: a step of 32 of K of
+// the blocks it has (measured: one of 128 x 128 1.28, and no second fits its LDS; 64 x 128 0.70 and 1.35 for one and two at once;
+// 64 x 64 0.50, 0.88, 1.26), a beginning and an end, and the sum of the shares.
 static void choose_f32_tiles(int M, int N, int K, int& tile, int& shares) {
   const int units = tnx_compute_units(), steps = K / 32;
-  const int sizes[3][2] = {{1, 1}, {2, 1}, {2, 2}};
-  const double cost_of_step[3] = {1.0, 1.9, 3.6};
+  const int sizes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
+  const double block_step[3] = {1.28, 0.65, 0.38}, step_more[3] = {0.0, 0.05, 0.12};
   double best = 1e30;
   for (int i = 0; i < 3; ++i) {
-    const long long tiles = (long long)((M + 64 * sizes[i][0] - 1) / (64 * sizes[i][0])) * ((N + 64 * sizes[i][1] - 1) / (64 * sizes[i][1]));
+    const long long tiles = (long long)((M + sizes[i][0] - 1) / sizes[i][0]) * ((N + sizes[i][1] - 1) / sizes[i][1]);
     for (int s = 1; s <= 8 && (s == 1 || (N % 4 == 0 && steps / s >= 4 && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
       const int per = (steps + s - 1) / s;
-      const long long rounds = (tiles * s + units - 1) / units;
-      double cost = (double)rounds * (per * cost_of_step[i] + 3.0);
-      if (s > 1) cost += 8.0 + (double)M * N * (s + 1) * 4e-6 / 4.0 / 0.43;
+      const long long blocks = (tiles * s + units - 1) / units;
+      double cost = per * ((double)blocks * block_step[i] + step_more[i]) + (i == 0 ? 8.0 * blocks : 8.0);
+      if (s > 1) cost += 5.0 + (double)M * N * (s + 1) * 1e-6;
       if (cost < best) best = cost, tile = i, shares = s;
     }
   }
@@ -440,12 +537,13 @@ extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, c
     TNX_CHECK_LAUNCH("gemm_f32_skinny");
     return 0;
   }
-  if (K % 32 == 0 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) % 16 == 0) {
+  if (K % 32 == 0 && K < 1 << 22 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) % 16 == 0) {
     int tile = 0, shares = 1;
     choose_f32_tiles(M, N, K, tile, shares);
     if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
-#define F32_TILES(MI, NI, ST) launch_f32_tiles<MI, NI, ST>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
-    return tile == 0 ? F32_TILES(1, 1, 4) : tile == 1 ? F32_TILES(2, 1, 3) : F32_TILES(2, 2, 2);
+#define F32_TILES(MI, NI, WM, WN) \
+  launch_f32_parts<MI, NI, WM, WN>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
+    return tile == 0 ? F32_TILES(1, 2, 4, 2) : tile == 1 ? F32_TILES(1, 1, 2, 4) : F32_TILES(1, 1, 2, 2);
 #undef F32_TILES
   }
   dim3 grid((N + F32_TILE - 1) / F32_TILE, (M + F32_TILE - 1) / F32_TILE);

@@ -120,7 +120,7 @@ struct Tile {
   // j and e of the accumulator); COLS columns of a wave go out (all 32 NI, or the first 32 j = 0 where `value` joins
   // several). `put(row, column, chunk)`: 16 bytes of the result, of type T, at a row and column of the wave's tile.
   template <typename T, int COLS, typename Value, typename Put>
-  __device__ __forceinline__ void hand_out(char* smem, Value value, Put put) {
+  static __device__ __forceinline__ void hand_out(char* smem, Value value, Put put) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
     constexpr int ROW = COLS * (int)sizeof(T) + 16;
     char* mine = smem + wave() * OUT;
