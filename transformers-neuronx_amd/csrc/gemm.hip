@@ -902,6 +902,87 @@ static int launch_wide(const bf16_t* x, const bf16_t* w, const float* bias, cons
 
 // ------------------------------------------------------------------------------------------ bfloat16, few rows
 
+// Products of few rows next to a norm: a block asks for the rows and then for its first weights, and norms the rows while the
+// weights come: all of them into LDS as the operand (NORM_OPERAND), or their means and deviations alone, with which a thread
+// norms the element of the residual that it adds (NORM_RESIDUAL: behind a sum, what a norm gives is the stream itself, operand of
+// the next product and residual of the one after that). The rows come first because loads are waited for in the order they were
+// made: asked for after the weights they made every product 2 us longer. Statistics in float32 in two passes over registers, as
+// the norm's own kernel takes them; the operand is read from LDS, which is nearer than rows that other units left in memory.
+// Measured, us, at 1 and 8 rows: the norm's kernel and the product / the norm folded into the product (`NormFold`) / so:
+// 4,096 columns of K 1,024 6.4, 7.0 / 5.2, 6.4 / 4.2, 4.5; 8,192 of 2,048 11.6, 12.3 / 9.9, 11.8 / 9.2, 10.1; 10,240 of 2,560 15.4, 16.3 /
+// 14.3, 16.0 / 13.5, 15.3; but 16,384 of 4,096 28.5, 29.6 / 27.3, 30.5 / 28.8, 32.3: wider rows take the registers and the time
+// of too many blocks. As a residual of 1,024, with the product of K 1,024 and of 4,096: 3.4, 4.0 and 6.1, 7.3 with the normed
+// residual there, 3.8, 4.4 and 6.4, 7.9 so.
+struct RowNorm {
+  const float* x;        // [M][width] float32
+  const float* weight;   // [width], with `bias` or both null
+  const float* bias;
+  float eps;
+  int center;            // 0: a norm that only scales
+};
+enum NormKind { NORM_NONE = 0, NORM_OPERAND = 1, NORM_RESIDUAL = 2 };
+struct NoNorm {};
+template <int KIND>
+using NormArg = std::conditional_t<KIND == NORM_NONE, NoNorm, RowNorm>;
+constexpr int NORM_WIDTH = 3072;
+
+// Rows wave, wave + 4 (below M) of the norm's by this wave of four. `ask` comes before the block asks for its weights: loads are
+// waited for in the order they were made.
+template <int ROWS, int PER, bool OPERAND>
+struct NormedRows {
+  f32x4 v[ROWS][PER], gw[OPERAND ? PER : 1], gb[OPERAND ? PER : 1];
+  __device__ __forceinline__ void ask(const RowNorm& n, int M, int width) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r)
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (256 * j < width) v[r][j] = *(const f32x4*)(n.x + (size_t)min(wave + 4 * r, M - 1) * width + min(256 * j + 4 * lane, width - 4));
+    if constexpr (OPERAND) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) {
+        const int i = min(256 * j + 4 * lane, width - 4);
+        gw[j] = n.weight ? *(const f32x4*)(n.weight + i) : (f32x4){1.f, 1.f, 1.f, 1.f};
+        gb[j] = n.bias ? *(const f32x4*)(n.bias + i) : (f32x4){0.f, 0.f, 0.f, 0.f};
+      }
+    }
+  }
+  // Mean and 1 / deviation into `stat`; as the operand, the normed rows into `rows` (LDS, `pitch` elements a row).
+  __device__ __forceinline__ void finish(const RowNorm& n, int M, int width, bf16_t* rows, int pitch, float (*stat)[2]) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+#pragma unroll
+    for (int r = 0; r < ROWS; ++r) {
+      const int m = wave + 4 * r;
+      if (m >= M) continue;
+      float s = 0.f, q = 0.f;
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (256 * j + 4 * lane < width) s += (v[r][j].x + v[r][j].y) + (v[r][j].z + v[r][j].w);
+      const float mean = n.center ? wave_sum(s) / (float)width : 0.f;
+#pragma unroll
+      for (int j = 0; j < PER; ++j)
+        if (256 * j + 4 * lane < width) {
+          const f32x4 d = v[r][j] - mean;
+          q += (d.x * d.x + d.y * d.y) + (d.z * d.z + d.w * d.w);
+        }
+      const float rstd = rsqrtf(wave_sum(q) / (float)width + n.eps);
+      if (lane == 0) stat[m][0] = mean, stat[m][1] = rstd;
+      if constexpr (OPERAND) {
+#pragma unroll
+        for (int j = 0; j < PER; ++j) {
+          const int i = 256 * j + 4 * lane;
+          if (i >= width) continue;
+          const f32x4 y = (v[r][j] - mean) * rstd * gw[j] + gb[j];
+          bf16x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (bf16_t)y[e];
+          *(bf16x4*)(rows + m * pitch + i) = o;
+        }
+      }
+    }
+  }
+};
+
 // One block of WAVES waves makes 16 * RT columns of the output (RT tiles of 16 rows of `w`) for all
 // M <= 16 * MT rows of `x`; with RT = 2 every fragment of `x` serves two products, which pays for wide
 // matrices (N >= 16,384: 29.2 -> 27.2 us at 8 rows, 34.1 -> 29.6 at 16) and costs blocks for narrow ones.
@@ -931,11 +1012,15 @@ struct NormFold {
   int center;          // 0: a norm that only scales (the mean is taken as 0, and nothing is shifted before rounding)
 };
 
-template <int MT, int WAVES, bool QKV, bool SHUF, int RT, bool NORMED = false>
+template <int MT, int WAVES, bool QKV, bool SHUF, int RT, bool NORMED = false, int NORM = NORM_NONE, int ROWS = 1, int PER = 1>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                         const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
-                        int N, int K, QkvScatter sc, NormFold nf) {
+                        int N, int K, QkvScatter sc, NormFold nf, NormArg<NORM> norm) {
+  static_assert(NORM == NORM_NONE || (MT == 1 && WAVES == 4 && !NORMED), "two rows a wave of four");
+  __shared__ float norm_stat[NORM ? 16 : 1][2];
+  extern __shared__ __attribute__((aligned(16))) char normed_rows[];
+  const int norm_pitch = K + 8;       // (16 bytes more than a row: rows would share their banks)
   __shared__ float red[WAVES][MT][RT][4][64];
   __shared__ float stat[WAVES][MT][2][16];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -949,6 +1034,11 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     wrow[j] = SHUF ? w + (size_t)min((int)blockIdx.x * RT + j, N / 16 - 1) * 16 * K + (r * 4 + g) * 8
                    : w + (size_t)min(n0 + 16 * j + r, N - 1) * K + 8 * g;
   const bf16x8 zero = {0, 0, 0, 0, 0, 0, 0, 0};
+  NormedRows<ROWS, PER, NORM == NORM_OPERAND> normed;
+  if constexpr (NORM != NORM_NONE) {
+    normed.ask(norm, M, NORM == NORM_OPERAND ? K : N);
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // What the end of the kernel adds (bias, residual, the folded norm's vectors) is asked for first: there it would be one
   // more time to reach memory after the last product. A thread's element q is (row, column) of `place(q)`.
   constexpr int OUTS = MT * RT * 4 / WAVES;      // elements a thread makes: MT RT tiles of 256 by 64 WAVES threads
@@ -959,7 +1049,9 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
   };
   constexpr bool EARLY = OUTS >= 1 && OUTS <= 4 && MT * RT * 4 % WAVES == 0;
   float add[EARLY ? OUTS : 1], onto[EARLY ? OUTS : 1], fold_c[EARLY ? OUTS : 1], fold_d[EARLY ? OUTS : 1];
+  float onto_w[EARLY ? OUTS : 1], onto_b[EARLY ? OUTS : 1];
   int page[EARLY ? OUTS : 1], off[EARLY ? OUTS : 1];
+  static_assert(NORM == NORM_NONE || EARLY, "the residual is normed where it was asked for");
   if constexpr (EARLY) {
 #pragma unroll
     for (int q = 0; q < OUTS; ++q) {
@@ -969,6 +1061,11 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
       add[q] = bias ? bias[n] : 0.f;
       if (NORMED) fold_c[q] = nf.c[n], fold_d[q] = nf.d[n];
       onto[q] = !QKV && residual ? residual[(size_t)m * N + n] : 0.f;
+      if constexpr (NORM == NORM_RESIDUAL) {
+        onto[q] = norm.x[(size_t)m * N + n];
+        onto_w[q] = norm.weight ? norm.weight[n] : 1.f;
+        onto_b[q] = norm.bias ? norm.bias[n] : 0.f;
+      }
       if (QKV) page[q] = sc.token_page[m], off[q] = sc.token_off[m];
     }
   }
@@ -983,7 +1080,7 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
 #pragma unroll
   for (int t = 0; t < MT; ++t) {
     const size_t row = (size_t)min(t * 16 + r, M - 1) * K;
-    xrow[t] = NORMED ? nullptr : x + row + 8 * g;
+    xrow[t] = NORMED || NORM == NORM_OPERAND ? nullptr : x + row + 8 * g;
     xfrow[t] = NORMED ? nf.x + row + 8 * g : nullptr;
     if (NORMED && nf.center) {
       // the shift: the median of the medians of three times three elements spread over the row, which a few
@@ -1022,6 +1119,12 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
     f32x4 xr[NORMED ? 2 : 1][MT][4][2];
     auto fetch_x = [&](int slot, int kc) {
       const int k = min(kc, k_last);
+      if constexpr (NORM == NORM_OPERAND) {
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+          xf[slot][0][s] = *(const bf16x8*)((const bf16_t*)normed_rows + min(r, M - 1) * norm_pitch + 8 * g + k + 32 * s);
+        return;
+      }
       if (NORMED) {
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
@@ -1067,9 +1170,18 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
           for (int j = 0; j < RT; ++j)
             acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[wslot][j][s], xf[xslot][t][s], acc[t][j], 0, 0, 0);
     };
-    fetch_x(0, kb0);
+    if constexpr (NORM != NORM_OPERAND) fetch_x(0, kb0);
     fetch_w(0, kb0);
     fetch_w(1, kb0 + STRIDE);
+    if constexpr (NORM != NORM_NONE) {
+      __builtin_amdgcn_sched_barrier(0);
+      normed.finish(norm, M, NORM == NORM_OPERAND ? K : N, (bf16_t*)normed_rows, norm_pitch, norm_stat);
+      if constexpr (NORM == NORM_OPERAND) {
+        __syncthreads();
+        fetch_x(0, kb0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
     // six steps a round, so that every buffer index is a constant (3 weight buffers, 2 x buffers)
     for (int kb = kb0; kb < k_full; kb += 6 * STRIDE) {
 #pragma unroll
@@ -1157,7 +1269,8 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
       } else if (EARLY) {
         if (bias) v += add[q];
         v = apply_act(v, act);
-        if (residual) v += onto[q];
+        if (NORM == NORM_RESIDUAL) v += (onto[q] - norm_stat[m][0]) * norm_stat[m][1] * onto_w[q] + onto_b[q];
+        else if (residual) v += onto[q];
         store_any(out, out_dtype, (size_t)m * N + n, v);
       } else {
         epilogue_store(v, m, n, N, bias, residual, out, out_dtype, act);
@@ -1183,25 +1296,70 @@ static void launch_skinny(const bf16_t* xp, const bf16_t* wp, const bf16_t* ws, 
     if constexpr (MT <= 2) {
       if (sc)
         gemm_bf16_skinny_kernel<MT, WAVES, true, true, RT, true><<<grid, block, 0, stream>>>(
-            nullptr, ws, bias, residual, out, out_dtype, act, M, N, K, *sc, *nf);
+            nullptr, ws, bias, residual, out, out_dtype, act, M, N, K, *sc, *nf, NoNorm{});
       else
         gemm_bf16_skinny_kernel<MT, WAVES, false, true, RT, true><<<grid, block, 0, stream>>>(
-            nullptr, ws, bias, residual, out, out_dtype, act, M, N, K, none, *nf);
+            nullptr, ws, bias, residual, out, out_dtype, act, M, N, K, none, *nf, NoNorm{});
     }
     return;
   }
   if (ws && sc)
     gemm_bf16_skinny_kernel<MT, WAVES, true, true, RT><<<grid, block, 0, stream>>>(xp, ws, bias, residual, out,
-                                                                                out_dtype, act, M, N, K, *sc, plain);
+                                                                                out_dtype, act, M, N, K, *sc, plain, NoNorm{});
   else if (ws)
     gemm_bf16_skinny_kernel<MT, WAVES, false, true, RT><<<grid, block, 0, stream>>>(xp, ws, bias, residual, out,
-                                                                                 out_dtype, act, M, N, K, none, plain);
+                                                                                 out_dtype, act, M, N, K, none, plain, NoNorm{});
   else if (sc)
     gemm_bf16_skinny_kernel<MT, WAVES, true, false, RT><<<grid, block, 0, stream>>>(xp, wp, bias, residual, out,
-                                                                                 out_dtype, act, M, N, K, *sc, plain);
+                                                                                 out_dtype, act, M, N, K, *sc, plain, NoNorm{});
   else
     gemm_bf16_skinny_kernel<MT, WAVES, false, false, RT><<<grid, block, 0, stream>>>(xp, wp, bias, residual, out,
-                                                                                  out_dtype, act, M, N, K, none, plain);
+                                                                                  out_dtype, act, M, N, K, none, plain, NoNorm{});
+}
+
+// The same next to a norm (see `RowNorm`), up to 8 rows, from the tile-ordered weight.
+template <int RT, int NORM, int ROWS, int PER>
+static int launch_skinny_norm(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
+                              int K, const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
+  const dim3 grid((N + 16 * RT - 1) / (16 * RT));
+  const unsigned lds = NORM == NORM_OPERAND ? M * (K + 8) * 2 : 0;
+  auto launch = [&](auto* kernel, const QkvScatter& places) {
+    if (lds > 32 * 1024) {
+      static bool configured = false;
+      if (!configured) {
+        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * (NORM_WIDTH + 8) * 2);
+        TNX_REQUIRE(e == hipSuccess, "product next to a norm: cannot reserve LDS: %s", hipGetErrorString(e));
+        configured = true;
+      }
+    }
+    kernel<<<grid, 256, lds, stream>>>(xp, ws, bias, nullptr, out, out_dtype, act, M, N, K, places, NormFold{}, norm);
+    return 0;
+  };
+  if constexpr (NORM == NORM_OPERAND) {
+    if (sc) {
+      const auto with = [&](const QkvScatter& places) { return launch(gemm_bf16_skinny_kernel<1, 4, true, true, RT, false, NORM, ROWS, PER>, places); };
+      return with(*sc);
+    }
+  }
+  return launch(gemm_bf16_skinny_kernel<1, 4, false, true, RT, false, NORM, ROWS, PER>, QkvScatter{});
+}
+template <int RT, int NORM>
+static int skinny_norm_rows(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
+                            const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
+  const int width = NORM == NORM_OPERAND ? K : N;       // (registers for the rows as they are)
+#define SKINNY_NORM(PER)                                                                                                            \
+  return M <= 4 ? launch_skinny_norm<RT, NORM, 1, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)              \
+                : launch_skinny_norm<RT, NORM, 2, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
+  if (width <= 1024) SKINNY_NORM(4);
+  if (width <= 2048) SKINNY_NORM(8);
+  SKINNY_NORM(12);
+#undef SKINNY_NORM
+}
+template <int RT>
+static int skinny_norm(int kind, const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
+                       int K, const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
+  return kind == NORM_OPERAND ? skinny_norm_rows<RT, NORM_OPERAND>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
+                              : skinny_norm_rows<RT, NORM_RESIDUAL>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);
 }
 
 // How many tiles of 16 weight rows a block of the few-rows kernel takes (1, 2 or 3). Every block reads all of
@@ -1382,6 +1540,50 @@ extern "C" int tnx_gemm_f32_qkv(const float* x, const float* w, const float* bia
   if (M == 0) return 0;
   f32_skinny(x, w, bias, nullptr, nullptr, TNX_F32, TNX_ACT_NONE, M, sc.nq + 2 * sc.nk, K, sc, stream);
   TNX_CHECK_LAUNCH("gemm_f32_qkv");
+  return 0;
+}
+
+// Products of up to 8 rows next to a norm (see `RowNorm`), `w` in tile order. `kind` NORM_OPERAND: x is what `norm` gives (its
+// width is K); NORM_RESIDUAL: what it gives is added to the result (its width is N).
+static int norm_fits(int kind, const RowNorm* norm, const void* w, int M, int N, int K) {
+  TNX_REQUIRE(norm && norm->x && (kind == NORM_OPERAND || kind == NORM_RESIDUAL), "product next to a norm: no norm");
+  const int width = kind == NORM_OPERAND ? K : N;
+  TNX_REQUIRE(width <= NORM_WIDTH && norm->eps > 0.f &&
+              ((uintptr_t)norm->x | (uintptr_t)norm->weight | (uintptr_t)norm->bias | (uintptr_t)w) % 16 == 0,
+              "product next to a norm: rows of up to %d that begin at multiples of 16 bytes, got %d", NORM_WIDTH, width);
+  TNX_REQUIRE(M > 0 && M <= 8 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0, "product next to a norm: bad sizes M=%d N=%d K=%d", M, N, K);
+  return 0;
+}
+
+extern "C" int tnx_gemm_bf16_by_norm(int kind, const RowNorm* norm, const void* x, const void* w, const float* bias, void* out,
+                                     int out_dtype, int act, int M, int N, int K, hipStream_t stream) {
+  if (int rc = norm_fits(kind, norm, w, M, N, K)) return rc;
+  TNX_REQUIRE(kind == NORM_OPERAND || (x && (uintptr_t)x % 16 == 0), "product next to a norm: its rows begin at multiples of 16 bytes");
+  const bf16_t *xp = (const bf16_t*)x, *ws = (const bf16_t*)w;
+  const int tiles = skinny_tiles_per_block(M, N);
+#define BY_NORM(RT) skinny_norm<RT>(kind, xp, ws, bias, out, out_dtype, act, M, N, K, nullptr, *norm, stream)
+  if (int rc = tiles == 3 ? BY_NORM(3) : tiles == 2 ? BY_NORM(2) : BY_NORM(1)) return rc;
+#undef BY_NORM
+  TNX_CHECK_LAUNCH("gemm_bf16_by_norm");
+  return 0;
+}
+
+// Queries, keys and values of what a norm gives, straight to their places.
+extern "C" int tnx_gemm_bf16_by_norm_qkv(const RowNorm* norm, const void* w, const float* bias, int M, int K, const int* token_page,
+                                         const int* token_off, void* q_out, void* k_pages, void* v_pages, float scale, int num_heads,
+                                         int num_kv, int head_size, int page_size, int num_pages, const float* turn_a,
+                                         const float* turn_b, const int* positions, int turn_rows, int page_pad, hipStream_t stream) {
+  TNX_REQUIRE(num_heads > 0 && num_kv >= 0 && head_size > 0 && page_size > 0, "gemm_bf16_by_norm_qkv: bad sizes");
+  const int nq = num_heads * head_size, nk = num_kv * head_size, N = nq + 2 * nk;
+  if (int rc = norm_fits(NORM_OPERAND, norm, w, M, N, K)) return rc;
+  QkvScatter sc{token_page, token_off, (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages, scale, nq, nk, head_size, num_kv, page_size, num_pages};
+  if (int rc = qkv_turn(sc, turn_a, turn_b, positions, turn_rows, page_pad)) return rc;
+  const bf16_t* ws = (const bf16_t*)w;
+  const int tiles = skinny_tiles_per_block(M, N);
+#define BY_NORM(RT) skinny_norm<RT>(NORM_OPERAND, nullptr, ws, bias, nullptr, TNX_BF16, TNX_ACT_NONE, M, N, K, &sc, *norm, stream)
+  if (int rc = tiles == 3 ? BY_NORM(3) : tiles == 2 ? BY_NORM(2) : BY_NORM(1)) return rc;
+#undef BY_NORM
+  TNX_CHECK_LAUNCH("gemm_bf16_by_norm_qkv");
   return 0;
 }
 

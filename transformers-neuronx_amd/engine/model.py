@@ -173,16 +173,28 @@ class DecoderModel:
         ctx.input_state = caches[self.input_state_id] if self.input_state_id is not None else None
         stream: Stream = self.embedding.forward(ctx, want_compute)
         debug.tap("embedding", stream.x)
+        between = False             # what the last block left may be a norm that the next products do (`norms_between`)
         for call, (layer, cid, writes) in enumerate(self.schedule):
             cache = caches[cid] if writes else caches[cid].reader()
             state_id = self.call_state_ids[call]
             ctx.call_state = caches[state_id] if state_id is not None else None
-            stream = self.layers[layer].block.forward(stream, ctx, cache)
+            block = self.layers[layer].block
+            if between and not getattr(block, "norms_between", False):
+                stream = self._settled(stream)
+            stream = block.forward(stream, ctx, cache)
+            between = getattr(block, "norms_between", False)
             debug.tap(f"call{call}.layer{layer}", stream.x)
+        if between:
+            stream = self._settled(stream)
         if stream.copies is not None and (stream.x is None or stream.pending is not None):
             # an arrangement that keeps several copies of the stream: their sum is what the head reads
             stream = Stream(self.ops.hyper_sum(stream.copies, stream.pending))
         return debug.tap("logits", self.head.forward(stream, ctx))
+
+
+    def _settled(self, stream: Stream) -> Stream:
+        x = self.ops.settled(stream.x)
+        return stream if x is stream.x else Stream(x, None)
 
 
 def model_param_decls(spec: ModelSpec) -> List[ParamDecl]:

@@ -48,6 +48,11 @@ _SIGNATURES = {
         "tnx_gemm_f32_qkv": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                              _c_void_p, _c_float, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p,
                              _c_int, _c_int, _c_void_p],
+        "tnx_gemm_bf16_by_norm": [_c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
+                                  _c_void_p],
+        "tnx_gemm_bf16_by_norm_qkv": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                      _c_void_p, _c_float, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p,
+                                      _c_int, _c_int, _c_void_p],
         "tnx_gemm_skinny_tiles_per_block": [_c_int, _c_int],
         "tnx_gemm_bf16_mid": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                               _c_int, _c_void_p, ctypes.c_size_t, _c_int, _c_int, _c_void_p],
@@ -265,6 +270,12 @@ class FoldedNorm:
         return self._with_bias[k]
 
 
+class _RowNorm(ctypes.Structure):
+    """The norm of rows as the products next to it take it."""
+    _fields_ = [("x", ctypes.c_void_p), ("weight", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("eps", ctypes.c_float),
+                ("center", ctypes.c_int)]
+
+
 class DeferredNorm:
     """The input of a LayerNorm whose output only a matrix product reads: the product of few rows applies the
     norm itself (`HipOps.linear`, `HipOps.qkv_project`); whoever else gets one calls `materialize()`."""
@@ -290,6 +301,35 @@ class DeferredNorm:
     def normalised(self):
         """`(x - mean) rstd` alone, for a product with a folded copy."""
         return self.ops.layernorm(self.x, None, None, self.eps, self.dtype, False, True, self.center)[1]
+
+    def as_argument(self, alone=False):
+        """For the products next to a norm; `alone`: without weight and bias, as `normalised`."""
+        return _RowNorm(_ptr(self.x), None if alone else _ptr(self.weight), None if alone else _ptr(self.bias), self.eps,
+                        int(bool(self.center)))
+
+
+class NormBetween(DeferredNorm):
+    """The input of a norm that stands behind a sum, in steps of few rows, in the place of what the norm gives: a product
+    that reads it norms its rows itself, and one whose result it joins as the residual the elements it adds. Whoever else
+    gets one calls `settled()`; the norm's kernel then runs, once."""
+
+    __slots__ = ("done",)
+
+    def __init__(self, *args):
+        super().__init__(*args)
+        self.done = None
+
+    def settled(self):
+        """(float32, compute dtype) of the norm's result."""
+        if self.done is None:
+            self.done = self.ops.layernorm(self.x, self.weight, self.bias, self.eps, self.dtype, True, True, self.center)
+        return self.done
+
+    def materialize(self):
+        return self.settled()[1]
+
+    def normalised(self):
+        raise TypeError("a norm behind a sum is folded into no product")
 
 
 def tile_order(w: torch.Tensor) -> torch.Tensor:
@@ -583,6 +623,52 @@ class HipOps:
         w.tiles = None          # the few-rows steps read the folded copy; the memory stays what it was
         return True
 
+    # A norm next to bfloat16 products of few rows is done by those products up to so many rows of so many elements, as their
+    # operand and as the residual of the next (what was measured stands with `RowNorm` beside the kernels: every block reads all
+    # rows, and from there on the norm folded into the product, or the norm's own kernel, is the quicker).
+    norm_beside = True
+    norm_beside_rows = 8
+    norm_operand_width = 3072
+    norm_between_width = 2048
+
+    def _norm_beside(self, rows, width, most) -> bool:
+        return (self.norm_beside and self.dtype == torch.bfloat16 and 0 < rows <= self.norm_beside_rows and width % 128 == 0
+                and width <= most and not debug.tapping())
+
+    def norm_between(self, x, weight, bias, eps, dtype, center=True):
+        """(float32, compute dtype) of a norm whose result is the stream itself; both a `NormBetween` in steps of few rows."""
+        if dtype == torch.bfloat16 and self._norm_beside(x.shape[0], x.shape[1], self.norm_between_width):
+            _want(x, "x", torch.float32)
+            for v, name in ((weight, "norm weight"), (bias, "norm bias")):
+                if v is not None:
+                    _want(v, name, torch.float32, (x.shape[1],))
+            d = NormBetween(self, x, weight, bias, eps, dtype, center)
+            return d, d
+        return self.layernorm(x, weight, bias, eps, dtype, True, True, center)
+
+    @staticmethod
+    def settled(stream_x):
+        """What a stream holds as a tensor."""
+        return stream_x.settled()[0] if isinstance(stream_x, NormBetween) else stream_x
+
+    def _beside_weight(self, w, m, norm):
+        """The tile-ordered matrix that the products next to a norm read, or None where they do not take the sizes."""
+        if norm.done is not None or not self._norm_beside(m, norm.x.shape[1], self.norm_between_width) or not isinstance(w, PreparedWeight) or w.tiles is None:
+            return None
+        return None if any((_ptr(a) or 0) % 16 for a in (w.tiles, norm.x, norm.weight, norm.bias)) else w.tiles
+
+    def _folded_beside(self, h, folded) -> bool:
+        """A folded copy's product norms the rows itself, from LDS."""
+        return self._norm_beside(h.x.shape[0], h.x.shape[1], self.norm_operand_width) and (_ptr(h.x) | _ptr(folded.tiles)) % 16 == 0
+
+    def _linear_beside_norm(self, kind, norm, x, t, bias, act, out_dtype, m, n, k, alone=False):
+        out = torch.empty(m, n, dtype=out_dtype, device=norm.x.device)
+        how = norm.as_argument(alone)
+        self._call("gemm", "tnx_gemm_bf16_by_norm", kind, ctypes.addressof(how), _ptr(x), _ptr(t), _ptr(bias), _ptr(out), _code(out_dtype),
+                   _ACT[act], m, n, k, _stream(),
+                   work=lambda: self._product_work(m, n, k, x_item=4 if kind == 1 else 2, out_item=out.element_size(), residual=kind == 2))
+        return out
+
     def layernorm_deferred(self, x, weight, bias, eps, dtype, center=True):
         """The compute-dtype output of the norm, or, in steps of few rows, a `DeferredNorm`."""
         if self.fuse_norm and dtype == torch.bfloat16 and self.dtype == torch.bfloat16 \
@@ -637,6 +723,20 @@ class HipOps:
         """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
         left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
         of a larger tensor), instead of a tensor of its own."""
+        if isinstance(residual, NormBetween) or isinstance(x, NormBetween):
+            n, k = w.shape
+            norm, kind = (x, 1) if isinstance(x, NormBetween) else (residual, 2)
+            plain = x is not residual and not force_tiled and into is None and act in _ACT and (kind == 2) == (residual is not None)
+            t = self._beside_weight(w, x.shape[0], norm) if plain and (kind == 1 or out_f32) else None
+            if t is not None and kind == 2:
+                t = t if _want(x, "x", self.dtype, (norm.x.shape[0], k)) is x and norm.x.shape[1] == n and _ptr(x) % 16 == 0 else None
+            if t is not None and (kind == 2 or norm.x.shape[1] == k):
+                if bias is not None:
+                    _want(bias, "bias", torch.float32, (n,))
+                return self._linear_beside_norm(kind, norm, x if kind == 2 else None, t, bias, act,
+                                                torch.float32 if out_f32 else self.dtype, x.shape[0], n, k)
+            residual = self.settled(residual)
+            x = x.settled()[1] if isinstance(x, NormBetween) else x
         if isinstance(x, DeferredNorm):
             folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
             if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
@@ -644,6 +744,9 @@ class HipOps:
                 folded = None
             if folded is None:
                 x = x.materialize()
+            elif not force_tiled and act in _ACT and self._folded_beside(x, folded):
+                return self._linear_beside_norm(1, x, None, folded.tiles, folded.d_with(bias), act, self.dtype, x.shape[0],
+                                                w.tensor.shape[0], w.tensor.shape[1], alone=True)
             elif not self._norm_in_the_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
                 # the norm's kernel without weight and bias, then the plain product of the folded copy
                 m, k = x.shape
@@ -916,6 +1019,12 @@ class HipOps:
         `turn` = (a, b), float32 `[positions, head_size]`: element d of every query and key head of a token at
         position p becomes a[p, d] x[d] + b[p, d] x[d ^ 1] (bias added, before the scale), in the same launch."""
         turn_a, turn_b, turn_pos, turn_rows = self._turn_args(turn, head_size, ctx)
+        if isinstance(h, NormBetween):
+            tiles = None if force_tiled else self._beside_weight(w, h.x.shape[0], h)
+            if tiles is not None:
+                return self._qkv_beside_norm(h, tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
+                                             k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
+            h = h.settled()[1]
         if isinstance(h, DeferredNorm):
             folded = self._folded_for(h, w) if force_tiled != 1 else None
             if folded is not None and (ctx.num_tokens >= 128 or self._library_product(
@@ -923,6 +1032,9 @@ class HipOps:
                 folded = None
             if folded is None:
                 h = h.materialize()
+            elif not force_tiled and self._folded_beside(h, folded):
+                return self._qkv_beside_norm(h, folded.tiles, folded.d_with(bias), tuple(w.tensor.shape), num_heads, num_kv_write, head_size,
+                                             scale, ctx, view, k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows, alone=True)
             elif not self._norm_in_the_product(h.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
                 # the norm's kernel without weight and bias, then the fused projection of the folded copy
                 h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
@@ -988,6 +1100,29 @@ class HipOps:
                    _ptr(turn_b), _ptr(turn_pos), turn_rows,
                    self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size, view.page_size), _stream(),
                    work=lambda: self._product_work(t, total, h.shape[1]))
+        return q
+
+    def _qkv_beside_norm(self, h, tensor, bias, shape, num_heads, num_kv_write, head_size, scale, ctx, view, k_pages, v_pages, turn_a,
+                         turn_b, turn_pos, turn_rows, alone=False):
+        """Queries, keys and values of what the norm `h` gives; `tensor` the tile-ordered matrix of `shape`."""
+        t, k = ctx.num_tokens, h.x.shape[1]
+        total = (num_heads + 2 * num_kv_write) * head_size
+        _want(h.x, "x", torch.float32, (t, k))
+        if shape != (total, k):
+            raise ValueError(f"w is {shape}, the projections need {(total, k)}")
+        if bias is not None:
+            _want(bias, "qkv bias", torch.float32, (total,))
+        num_pages = self._check_pages(k_pages, v_pages, num_kv_write, head_size, view.page_size) if num_kv_write else 0
+        _want(view.token_page, "token pages", torch.int32, (t,))
+        _want(view.token_offset, "token offsets", torch.int32, (t,))
+        q = torch.empty(t, num_heads * head_size, dtype=self.dtype, device=h.x.device)
+        how = h.as_argument(alone)
+        self._call("gemm", "tnx_gemm_bf16_by_norm_qkv", ctypes.addressof(how), _ptr(tensor), _ptr(bias), t, k,
+                   _ptr(view.token_page), _ptr(view.token_offset), _ptr(q), _ptr(k_pages) if num_kv_write else None,
+                   _ptr(v_pages) if num_kv_write else None, float(scale), num_heads, num_kv_write, head_size, view.page_size, num_pages,
+                   _ptr(turn_a), _ptr(turn_b), _ptr(turn_pos), turn_rows,
+                   self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size, view.page_size), _stream(),
+                   work=lambda: self._product_work(t, total, k, x_item=4))
         return q
 
     # Float32 queries, keys and values of so many rows leave the few-rows product for their places, without `qkv_write`: 3

@@ -113,6 +113,15 @@ class ReferenceOps:
     def fold_norm(self, w, weight, bias, center=True) -> bool:
         return False
 
+    def norm_between(self, x, weight, bias, eps, dtype, center=True):
+        """A norm whose result is the stream itself: (float32, compute dtype); a backend may hand back twice something that
+        the products next to it resolve (`HipOps.norm_between`), and `settled` makes a tensor of."""
+        return self.layernorm(x, weight, bias, eps, dtype, True, True, center)
+
+    @staticmethod
+    def settled(stream_x):
+        return stream_x
+
     def prepare_weight(self, w):
         """Matrices are used as they are here."""
         return w

@@ -44,6 +44,20 @@ class PostNormBlock(Block):
 
     reads_compute_copy = True      # the mixer reads the stream itself, in the compute dtype
 
+    # Both parts do with the stream nothing but a product of its rows and adding it to their last product's sums, and the norms
+    # are of a form that the backend's products know: in steps of few rows they norm it themselves.
+    norms_between = False
+
+    def after_load(self) -> None:
+        norms = (self.mixer_norm, self.feed_forward_norm)
+        self.norms_between = (self.alpha is None and self.has_ff and self.mixer.first_weight() is not None
+                              and self.feed_forward.first_weight() is not None and all(hasattr(n, "fused_form") for n in norms)
+                              and hasattr(self.mixer_norm.ops, "norm_between"))
+
+    def _between(self, norm, x):
+        weight, bias, center, eps = norm.fused_form()
+        return norm.ops.norm_between(x, weight, bias, eps, norm.dtype, center)
+
     def __init__(self, mixer, feed_forward, mixer_norm, feed_forward_norm, *, alpha=None):
         super().__init__(mixer, feed_forward, mixer_norm, feed_forward_norm)
         self.alpha = None if alpha is None else float(alpha)
@@ -66,6 +80,13 @@ class PostNormBlock(Block):
             if self.has_ff:
                 x, h = self._join(self.feed_forward_norm, x, [(self.feed_forward.forward(h, ctx, None), None, None, 1.0)])
             return Stream(x, h)
+        if self.norms_between:
+            x, h = stream.x, stream.compute
+            if h is None:
+                h = self.mixer_norm.ops.cast(x, self.mixer_norm.dtype)
+            x, h = self._between(self.mixer_norm, self.mixer.forward(h, ctx, cache, x))
+            debug.tap("after_mixer", x)
+            return Stream(*self._between(self.feed_forward_norm, self.feed_forward.forward(h, ctx, x)))
         h = stream.compute if stream.compute is not None else self.mixer_norm.ops.cast(stream.x, self.mixer_norm.dtype)
         t = self.mixer.forward(h, ctx, cache, stream.x)
         x, h = self.mixer_norm.forward(t, True, True)
