@@ -110,3 +110,21 @@ def test_folded_copies(m, k, n):
     # the folded weight, the operand (or its shifted row, as large) and the result are each rounded once
     sizes = (bare.abs() + 2) @ (w.double() * gamma).abs().T + (w.double() @ beta.double()).abs() + bias.abs()
     assert bool(((got.double() - exact.relu()).abs() <= 3 * 2.0 ** -8 * sizes).all())
+
+
+@pytest.mark.parametrize("m,k,n", [(1, 256, 48), (8, 2048, 6144), (5, 3072, 1040), (9, 2048, 6144), (3, 3200, 96)])
+@pytest.mark.parametrize("center", [True, False])
+def test_deferred_norms_of_plain_copies(m, k, n, center):
+    """A layer's norm before its matrix: rows of up to 3,072 leave the matrix as it is."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g = HipOps(torch.bfloat16, DEV), _gen(m + k + n)
+    t = torch.randn(m, k, device=DEV, generator=g) * 3 + 1
+    gamma, beta = 1 + 0.1 * torch.randn(k, device=DEV, generator=g), torch.randn(k, device=DEV, generator=g)
+    w = torch.randn(n, k, device=DEV, generator=g).to(torch.bfloat16)
+    pw, bias = hip.prepare_weight(w), torch.randn(n, device=DEV, generator=g)
+    assert hip.defer_norm(pw, gamma, beta, center) and (pw.folded is None) == (k <= 3072)
+    got = hip.linear(hip.layernorm_deferred(t, gamma, beta, 1e-5, torch.bfloat16, center), pw, bias)
+    y = _normed(t, gamma, beta, 1e-5, center)
+    want = y @ w.double().T + bias
+    # independent roundings to bfloat16: the operand's and the result's, and a folded weight's
+    assert (got.double() - want).norm() <= 2.5 * 2.0 ** -9 * want.norm()

@@ -1639,16 +1639,18 @@ extern "C" int tnx_gemm_bf16_qkv_normed(const float* x, const void* w_folded, co
 // the chip also where N is small) leave their float32 partial sums in a workspace [shares][M][N] that a
 // second kernel adds up in a fixed order, with bias, activation and residual; one share alone writes the
 // result itself.
-template <int MT, int AHEAD>
-__global__ void __launch_bounds__(256)
+template <int MT, int AHEAD, int NW, typename Scatter>
+__global__ void __launch_bounds__(64 * NW)
 gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_tiles, const float* __restrict__ bias,
                      const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act,
-                     float* __restrict__ partial, int M, int N, int K, int steps_per_share) {
+                     float* __restrict__ partial, int M, int N, int K, int steps_per_share, Scatter sc) {
+  constexpr bool SCATTER = !std::is_same<Scatter, NoScatter>::value;
   extern __shared__ __attribute__((aligned(16))) char mid_smem[];
   constexpr int NST = AHEAD + 1;                    // stages: the step that is multiplied and those in flight
   constexpr int XSTAGE = 16 * MT * 256;             // bytes of a step's rows of x
   constexpr int WSTAGE = 4 * 1024;                  // bytes of a step's weights of one wave
-  constexpr int LOADS = MT + 4;                     // loads of a wave a step
+  constexpr int XLOADS = (4 * MT + NW - 1) / NW;    // loads of x of a wave a step (where they do not come out even, some twice)
+  constexpr int LOADS = XLOADS + 4;                 // loads of a wave a step
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int share = blockIdx.y;
@@ -1656,14 +1658,14 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_
   const int step0 = share * steps_per_share;
   const int steps = min(steps_per_share, steps_all - step0);      // at least one: the host cuts no empty share
   const int last = step0 + steps - 1;
-  const int tile = blockIdx.x * 4 + wave;           // this wave's tile of 16 weight rows
+  const int tile = blockIdx.x * NW + wave;          // this wave's tile of 16 weight rows
   const char* wtile = (const char*)(w_tiles + (size_t)min(tile, N / 16 - 1) * 16 * K);
-  // the loads of x: wave-load u of this wave brings rows 4 q .. 4 q + 3 (q = wave + 4 u), 16 lanes a row; the
+  // the loads of x: wave-load u of this wave brings rows 4 q .. 4 q + 3 (q = wave + NW u), 16 lanes a row; the
   // lane at place p of row m brings chunk p ^ (m % 16), so that fragment reads meet no bank twice
-  unsigned xoff[MT];
+  unsigned xoff[XLOADS];
 #pragma unroll
-  for (int u = 0; u < MT; ++u) {
-    const int row = 4 * (wave + 4 * u) + (lane >> 4);
+  for (int u = 0; u < XLOADS; ++u) {
+    const int row = 4 * min(wave + NW * u, 4 * MT - 1) + (lane >> 4);
     xoff[u] = (unsigned)(((size_t)min(row, M - 1) * K + (((lane & 15) ^ (row & 15)) * 8)) * 2);
   }
   const unsigned x_lds = lds_offset(mid_smem);
@@ -1673,7 +1675,8 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_
     const int st = min(step, last);                 // beyond the share: the last step again, into a stage nobody reads
     const char* xbase = (const char*)(x + (size_t)st * 128);
 #pragma unroll
-    for (int u = 0; u < MT; ++u) load_to_lds(xbase, xoff[u], x_lds + stage * XSTAGE + (wave + 4 * u) * 1024);
+    for (int u = 0; u < XLOADS; ++u)
+      load_to_lds(xbase, xoff[u], x_lds + stage * XSTAGE + min(wave + NW * u, 4 * MT - 1) * 1024);
     const char* wbase = wtile + (size_t)st * (128 * 16 * 2);
 #pragma unroll
     for (int s = 0; s < 4; ++s) load_to_lds_once(wbase + 1024 * s, (unsigned)((r * 4 + g) * 16), w_lds + stage * WSTAGE + 1024 * s);
@@ -1717,7 +1720,13 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_
     for (int t = 0; t < MT; ++t) {
       const int m = 16 * t + r;
       if (m >= M) continue;
-      if (shares == 1) {
+      if constexpr (SCATTER) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = acc[t][e] + (bias ? bias[n + e] : 0.f);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qkv_store(v[e], v[e ^ 1], m, n + e, sc, sc.token_page[m], sc.token_off[m]);
+      } else if (shares == 1) {
 #pragma unroll
         for (int e = 0; e < 4; ++e) epilogue_store(acc[t][e], m, n + e, N, bias, residual, out, out_dtype, act);
       } else {
@@ -1757,14 +1766,15 @@ gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__
   for (int e = 0; e < 4; ++e) epilogue_store(v[e], m, n + e, N, bias, residual, out, out_dtype, act);
 }
 
-template <int MT, int AHEAD>
+template <int MT, int AHEAD, int NW = 4, typename Scatter = NoScatter>
 static int launch_mid(const bf16_t* x, const bf16_t* w_tiles, const float* bias, const float* residual, void* out,
-                      int out_dtype, int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
-  constexpr int bytes = (AHEAD + 1) * (16 * MT * 256 + 4 * 4 * 1024);
+                      int out_dtype, int act, float* partial, int M, int N, int K, int shares, hipStream_t stream,
+                      const Scatter& sc = Scatter{}) {
+  constexpr int bytes = (AHEAD + 1) * (16 * MT * 256 + NW * 4 * 1024);
   static_assert(bytes <= 160 * 1024, "the stages do not fit the LDS of a compute unit");
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_mid_kernel<MT, AHEAD>,
+    hipError_t e = hipFuncSetAttribute((const void*)gemm_bf16_mid_kernel<MT, AHEAD, NW, Scatter>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     if (e != hipSuccess) {
       tnx_set_error("gemm_bf16_mid: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
@@ -1773,9 +1783,9 @@ static int launch_mid(const bf16_t* x, const bf16_t* w_tiles, const float* bias,
     configured = true;
   }
   const int steps_all = K / 128, per = (steps_all + shares - 1) / shares;
-  const dim3 grid((N / 16 + 3) / 4, (steps_all + per - 1) / per);
-  gemm_bf16_mid_kernel<MT, AHEAD><<<grid, 256, bytes, stream>>>(x, w_tiles, bias, residual, out, out_dtype, act,
-                                                                 partial, M, N, K, per);
+  const dim3 grid((N / 16 + NW - 1) / NW, (steps_all + per - 1) / per);
+  gemm_bf16_mid_kernel<MT, AHEAD, NW, Scatter><<<grid, 64 * NW, bytes, stream>>>(x, w_tiles, bias, residual, out, out_dtype,
+                                                                                 act, partial, M, N, K, per, sc);
   TNX_CHECK_LAUNCH("gemm_bf16_mid");
   if (grid.y > 1) {
     gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out,
@@ -1830,6 +1840,65 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 #undef MID_HIGH
 #undef MID_LOW
 #undef MID
+}
+
+// The same for 9 to 48 rows with a rounded result, or with queries, keys and values put in their places, and K whole: no sum
+// follows, and what fills the chip is the number of waves a block has, one to four of 16 columns each: as many as leave every
+// compute unit one block (`whole_waves`). A unit brings some 30 bytes a nanosecond from memory however many ask on it, so what
+// counts is that all of them do: 10,240 columns of K 2,560 at 24 rows by blocks of one wave (640 blocks) to four (160) 17.2, 18.2,
+// 14.6 and 17.0 us. Measured on weights that no cache holds, us, with what took them before (the few-rows kernel up to 24 rows
+// or where the matrix is small, the vendor library beyond) / so, at 16, 24, 32 and 48 rows: 6,144 x 2,048 9.3 / 8.6, 11.1 / 9.8, 11.8 / 10.2,
+// 13.5 / 11.9; 8,192 x 2,048 10.3 / 9.2, 12.0 / 10.3, 14.4 / 10.6, 15.1 / 12.6; 10,240 x 2,560 14.6 / 13.0, 20.8 / 14.6, 21.3 / 15.4, 20.7 / 19.8;
+// 12,288 x 4,096 21.6 / 20.4, 28.4 / 21.5, 33.0 / 22.1, 28.2 / 25.2; 16,384 x 4,096 28.3 / 28.6, 32.0 / 29.8, 33.5 / 29.9, 35.6 / 32.6. Not for
+// small matrices (24 rows 3,072 x 1,024 6.1 / 6.4: a chain of steps, where the few-rows kernel's waves share K) nor at 64 rows
+// (12,288 x 4,096 27.5 / 29.4: the rows weigh as much as the weights).
+template <typename Scatter>
+static int launch_whole(const bf16_t* x, const bf16_t* w_tiles, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
+                        int waves, const Scatter& sc, hipStream_t stream) {
+#define WHOLE(MT, NW) launch_mid<MT, 3, NW, Scatter>(x, w_tiles, bias, nullptr, out, out_dtype, act, nullptr, M, N, K, 1, stream, sc)
+#define WHOLE_MT(MT) return waves == 1 ? WHOLE(MT, 1) : waves == 2 ? WHOLE(MT, 2) : waves == 3 ? WHOLE(MT, 3) : WHOLE(MT, 4)
+  switch ((M + 15) / 16) {
+    case 1:
+    case 2: WHOLE_MT(2);
+    case 3: WHOLE_MT(3);
+    default: WHOLE_MT(4);
+  }
+#undef WHOLE_MT
+#undef WHOLE
+}
+
+static int whole_waves(int N) {
+  const int units = tnx_compute_units(), tiles = N / 16;
+  return max(1, min(4, (tiles + units - 1) / units));
+}
+
+static int whole_fits(const void* x, const void* w_tiles, int M, int N, int K, int waves) {
+  TNX_REQUIRE(M > 0 && M <= 64 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && waves >= 0 && waves <= 4,
+              "gemm_bf16_whole: up to 64 rows, N a multiple of 16, K of 128; got M=%d N=%d K=%d", M, N, K);
+  TNX_REQUIRE(x && w_tiles && ((uintptr_t)x | (uintptr_t)w_tiles) % 16 == 0, "gemm_bf16_whole: operands must be there and 16-byte aligned");
+  return 0;
+}
+
+// `waves` 0: chosen here.
+extern "C" int tnx_gemm_bf16_whole(const void* x, const void* w_tiles, const float* bias, void* out, int out_dtype, int act, int M, int N,
+                                   int K, int waves, hipStream_t stream) {
+  if (int rc = whole_fits(x, w_tiles, M, N, K, waves)) return rc;
+  TNX_REQUIRE(out && (out_dtype == TNX_F32 || out_dtype == TNX_BF16), "gemm_bf16_whole: the result is float32 or bfloat16");
+  return launch_whole((const bf16_t*)x, (const bf16_t*)w_tiles, bias, out, out_dtype, act, M, N, K, waves ? waves : whole_waves(N),
+                      NoScatter{}, stream);
+}
+
+extern "C" int tnx_gemm_bf16_whole_qkv(const void* x, const void* w_tiles, const float* bias, int M, int K, const int* token_page,
+                                       const int* token_off, void* q_out, void* k_pages, void* v_pages, float scale, int num_heads,
+                                       int num_kv, int head_size, int page_size, int num_pages, int waves, const float* turn_a,
+                                       const float* turn_b, const int* positions, int turn_rows, int page_pad, hipStream_t stream) {
+  TNX_REQUIRE(num_heads > 0 && num_kv >= 0 && head_size > 0 && page_size > 0, "gemm_bf16_whole_qkv: bad sizes");
+  const int nq = num_heads * head_size, nk = num_kv * head_size, N = nq + 2 * nk;
+  if (int rc = whole_fits(x, w_tiles, M, N, K, waves)) return rc;
+  QkvScatter sc{token_page, token_off, (bf16_t*)q_out, (bf16_t*)k_pages, (bf16_t*)v_pages, scale, nq, nk, head_size, num_kv, page_size, num_pages};
+  if (int rc = qkv_turn(sc, turn_a, turn_b, positions, turn_rows, page_pad)) return rc;
+  return launch_whole((const bf16_t*)x, (const bf16_t*)w_tiles, bias, nullptr, TNX_BF16, TNX_ACT_NONE, M, N, K,
+                      waves ? waves : whole_waves(N), sc, stream);
 }
 
 // ------------------------------------------------------------------------------------- bfloat16, tiles

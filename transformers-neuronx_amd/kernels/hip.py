@@ -54,6 +54,10 @@ _SIGNATURES = {
                                       _c_void_p, _c_float, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p,
                                       _c_int, _c_int, _c_void_p],
         "tnx_gemm_skinny_tiles_per_block": [_c_int, _c_int],
+        "tnx_gemm_bf16_whole": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p],
+        "tnx_gemm_bf16_whole_qkv": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
+                                    _c_void_p, _c_float, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
+                                    _c_void_p, _c_int, _c_int, _c_void_p],
         "tnx_gemm_bf16_mid": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                               _c_int, _c_void_p, ctypes.c_size_t, _c_int, _c_int, _c_void_p],
         "tnx_gemm_bf16_tiles": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -229,11 +233,13 @@ class PreparedWeight:
     `[out/16][in/128][4][16][4][8]`: each block then reads one contiguous run of memory. The copy doubles
     the memory of the matrices; it is what decoding reads, the plain tensor is what prompts read."""
 
-    __slots__ = ("tensor", "tiles", "folded", "inner")
+    __slots__ = ("tensor", "tiles", "folded", "inner", "norm_before")
 
     def __init__(self, tensor: torch.Tensor, tiles: Optional[torch.Tensor], inner: Optional[int] = None):
         self.tensor, self.tiles = tensor, tiles
         self.folded: Optional["FoldedNorm"] = None
+        # the norm (`DeferredNorm.key`) whose result this matrix alone reads and its products of few rows make themselves
+        self.norm_before: Optional[tuple] = None
         # the matrix's own inner size where `tensor` carries columns of zeros after it (bfloat16 rows are
         # read 16 bytes at a time: an inner size that is no multiple of 8 is filled up once, here, and the
         # rows that meet it are filled up as they come)
@@ -270,6 +276,11 @@ class FoldedNorm:
         return self._with_bias[k]
 
 
+def _norm_key(weight, bias, center):
+    """Names a norm by its tensors (which the layer that has it keeps)."""
+    return (weight.data_ptr() if weight is not None else 0, bias.data_ptr() if bias is not None else 0, bool(center))
+
+
 class _RowNorm(ctypes.Structure):
     """The norm of rows as the products next to it take it."""
     _fields_ = [("x", ctypes.c_void_p), ("weight", ctypes.c_void_p), ("bias", ctypes.c_void_p), ("eps", ctypes.c_float),
@@ -292,8 +303,7 @@ class DeferredNorm:
 
     @property
     def key(self):
-        return (self.weight.data_ptr() if self.weight is not None else 0,
-                self.bias.data_ptr() if self.bias is not None else 0, bool(self.center))
+        return _norm_key(self.weight, self.bias, self.center)
 
     def materialize(self):
         return self.ops.layernorm(self.x, self.weight, self.bias, self.eps, self.dtype, False, True, self.center)[1]
@@ -618,8 +628,7 @@ class HipOps:
         scaled = (full * weight.float()[None, :] if weight is not None else full).to(torch.bfloat16)
         c = scaled.float().sum(dim=1).contiguous()
         d = (full @ bias.float() if bias is not None else torch.zeros_like(c)).contiguous()
-        key = (weight.data_ptr() if weight is not None else 0, bias.data_ptr() if bias is not None else 0, bool(center))
-        w.folded = FoldedNorm(tile_order(scaled), c, d, key)
+        w.folded = FoldedNorm(tile_order(scaled), c, d, _norm_key(weight, bias, center))
         w.tiles = None          # the few-rows steps read the folded copy; the memory stays what it was
         return True
 
@@ -656,6 +665,23 @@ class HipOps:
         if norm.done is not None or not self._norm_beside(m, norm.x.shape[1], self.norm_between_width) or not isinstance(w, PreparedWeight) or w.tiles is None:
             return None
         return None if any((_ptr(a) or 0) % 16 for a in (w.tiles, norm.x, norm.weight, norm.bias)) else w.tiles
+
+    def defer_norm(self, w, weight, bias, center=True) -> bool:
+        """Called once when a layer has its tensors, for a matrix `w` that reads a norm's output and nothing else does: whether
+        products of few rows norm their rows themselves (`layernorm_deferred`). Rows of up to `norm_operand_width` elements they
+        take as they are, with the norm's weight and bias; for wider ones the norm is folded into a copy (`fold_norm`)."""
+        if (self.norm_beside and self.fuse_norm and self.dtype == torch.bfloat16 and isinstance(w, PreparedWeight)
+                and w.tiles is not None and w.tensor.shape[1] <= self.norm_operand_width):
+            w.norm_before = _norm_key(weight, bias, center)
+            return True
+        return self.fold_norm(w, weight, bias, center)
+
+    def _plain_beside(self, h, w) -> bool:
+        """The norm `h` is the one before `w`, and the product of `w`'s own tile-ordered copy makes it."""
+        return (isinstance(w, PreparedWeight) and w.tiles is not None and w.norm_before is not None and w.norm_before == h.key
+                and w.tensor.shape[1] == h.x.shape[1]
+                and self._norm_beside(*h.x.shape, self.norm_operand_width)
+                and all((_ptr(a) or 0) % 16 == 0 for a in (w.tiles, h.x, h.weight, h.bias)))
 
     def _folded_beside(self, h, folded) -> bool:
         """A folded copy's product norms the rows itself, from LDS."""
@@ -742,6 +768,12 @@ class HipOps:
             if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
                                                               w.tensor, force_tiled, plain=True):
                 folded = None
+            if residual is None and not out_f32 and not force_tiled and act in _ACT and self._plain_beside(x, w):
+                if bias is not None:
+                    _want(bias, "bias", torch.float32, (w.tensor.shape[0],))
+                return self._linear_beside_norm(1, x, None, w.tiles, bias, act, self.dtype, x.shape[0], *w.tensor.shape)
+            if folded is not None and not force_tiled and self._whole_product(x.shape[0], *w.tensor.shape):
+                return self._linear_whole(x.normalised(), folded.tiles, folded.d_with(bias), act, *w.tensor.shape)
             if folded is None:
                 x = x.materialize()
             elif not force_tiled and act in _ACT and self._folded_beside(x, folded):
@@ -787,6 +819,9 @@ class HipOps:
         if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
         out_dtype = torch.float32 if out_f32 else self.dtype
+        if (tiles is not None and residual is None and not out_f32 and not force_tiled and into is None and w.dtype == torch.bfloat16
+                and _ptr(x) % 16 == 0 and self._whole_product(m, n, k)):
+            return self._linear_whole(self.cast(x, torch.bfloat16), tiles, bias, act, n, k)
         if self._some_rows_product(m, n, k, w, tiles, residual, out_f32, force_tiled):
             # decode batches of 33 to 128 requests, a float32 result: our kernel for some rows
             out = torch.empty(m, n, dtype=out_dtype, device=x.device)
@@ -946,6 +981,28 @@ class HipOps:
         shares = max(1, min(self.compute_units // column_blocks, k // 512))     # as the kernel shares K out
         return small or 4 * column_blocks * shares >= 3 * self.compute_units
 
+    # Products of so many rows with a rounded result from a tile-ordered copy, where a block of one to four waves a compute unit
+    # fills seven tenths of them (`gemm_bf16_mid`'s form with K whole; what it measured stands there).
+    whole_rows_from, whole_rows = 9, 48
+
+    def _whole_product(self, m, n, k) -> bool:
+        if not (self.whole_rows_from <= m <= self.whole_rows and self.dtype == torch.bfloat16 and n * k > self.small_matrix):
+            return False
+        waves = -(-n // (16 * self.compute_units))
+        return waves <= 4 and 10 * n >= 7 * 16 * waves * self.compute_units
+
+    def _linear_whole(self, x, tiles, bias, act, n, k):
+        if act not in _ACT:
+            raise ValueError(f"unknown activation {act!r}")
+        m = x.shape[0]
+        _want(x, "x", torch.bfloat16, (m, k))
+        if bias is not None:
+            _want(bias, "bias", torch.float32, (n,))
+        out = torch.empty(m, n, dtype=self.dtype, device=x.device)
+        self._call("gemm", "tnx_gemm_bf16_whole", _ptr(x), _ptr(tiles), _ptr(bias), _ptr(out), _code(self.dtype), _ACT[act], m, n, k, 0,
+                   _stream(), work=lambda: self._product_work(m, n, k))
+        return out
+
     def _library_product(self, m, n, k, w, force_tiled, scattered=False, plain=False) -> bool:
         """`scattered`: the fused projection of queries, keys and values, whose result the few-rows kernel puts in its
         places itself (after the library's product a kernel of 6 to 7 us does that). `plain`: a bfloat16 result."""
@@ -1027,10 +1084,15 @@ class HipOps:
             h = h.settled()[1]
         if isinstance(h, DeferredNorm):
             folded = self._folded_for(h, w) if force_tiled != 1 else None
-            if folded is not None and (ctx.num_tokens >= 128 or self._library_product(
-                    ctx.num_tokens, w.tensor.shape[0], w.tensor.shape[1], w.tensor, force_tiled, True)):
-                folded = None
-            if folded is None:
+            rows = h.shape[0]
+            few = (folded is not None and rows <= self.few_rows and ctx.num_tokens < 128
+                   and not self._library_product(ctx.num_tokens, *w.tensor.shape, w.tensor, force_tiled, True))
+            if not force_tiled and self._plain_beside(h, w):
+                return self._qkv_beside_norm(h, w.tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
+                                             k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
+            if few and not force_tiled and self._whole_product(rows, *w.tensor.shape):
+                h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
+            elif not few:
                 h = h.materialize()
             elif not force_tiled and self._folded_beside(h, folded):
                 return self._qkv_beside_norm(h, folded.tiles, folded.d_with(bias), tuple(w.tensor.shape), num_heads, num_kv_write, head_size,
@@ -1064,8 +1126,10 @@ class HipOps:
         tiles = None
         if isinstance(w, PreparedWeight):
             w, tiles = w.tensor, w.tiles
-        many = ctx.num_tokens >= 128 and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and not force_tiled
-        if self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (many or self._library_product(
+        whole = (tiles is not None and not force_tiled and w.dtype == h.dtype == torch.bfloat16 and _ptr(h) % 16 == 0
+                 and self._whole_product(ctx.num_tokens, *w.shape))
+        many = not whole and ctx.num_tokens >= 128 and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and not force_tiled
+        if not whole and self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (many or self._library_product(
                 ctx.num_tokens, w.shape[0], w.shape[1], w, force_tiled, tiles is not None)):
             # many rows (the vendor library, or our wide-tile kernel where sizes allow): the bias joins the
             # product's float32 sums before they are rounded, once, as in the fused kernel below, so that keys
@@ -1093,6 +1157,14 @@ class HipOps:
         _want(view.token_page, "token pages", torch.int32, (t,))
         _want(view.token_offset, "token offsets", torch.int32, (t,))
         q = torch.empty(t, num_heads * head_size, dtype=self.dtype, device=h.device)
+        if whole:
+            self._call("gemm", "tnx_gemm_bf16_whole_qkv", _ptr(h), _ptr(tiles), _ptr(bias), t, h.shape[1], _ptr(view.token_page),
+                       _ptr(view.token_offset), _ptr(q), _ptr(k_pages) if num_kv_write else None,
+                       _ptr(v_pages) if num_kv_write else None, float(scale), num_heads, num_kv_write, head_size, view.page_size,
+                       num_pages, 0, _ptr(turn_a), _ptr(turn_b), _ptr(turn_pos), turn_rows,
+                       self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size, view.page_size), _stream(),
+                       work=lambda: self._product_work(t, total, h.shape[1]))
+            return q
         self._call("gemm", "tnx_gemm_bf16_qkv", _ptr(h), _ptr(w), _ptr(tiles), _ptr(bias), t, h.shape[1],
                    _ptr(view.token_page), _ptr(view.token_offset), _ptr(q),
                    _ptr(k_pages) if num_kv_write else None, _ptr(v_pages) if num_kv_write else None, float(scale),

@@ -113,6 +113,9 @@ class ReferenceOps:
     def fold_norm(self, w, weight, bias, center=True) -> bool:
         return False
 
+    def defer_norm(self, w, weight, bias, center=True) -> bool:
+        return False
+
     def norm_between(self, x, weight, bias, eps, dtype, center=True):
         """A norm whose result is the stream itself: (float32, compute dtype); a backend may hand back twice something that
         the products next to it resolve (`HipOps.norm_between`), and `settled` makes a tensor of."""

@@ -48,7 +48,7 @@ class LayerNorm(Norm):
         return self.weight, self.bias, True, self.eps
 
     def fold_into(self, w) -> bool:
-        return self.ops.fold_norm(w, self.weight, self.bias)
+        return self.ops.defer_norm(w, self.weight, self.bias)
 
     def deferred(self, x):
         return self.ops.layernorm_deferred(x, self.weight, self.bias, self.eps, self.dtype)
@@ -92,7 +92,7 @@ class RMSNorm(Norm):
         return self.weight, None, False, self.eps
 
     def fold_into(self, w) -> bool:
-        return self.ops.fold_norm(w, self.weight, None, center=False)
+        return self.ops.defer_norm(w, self.weight, None, center=False)
 
     def deferred(self, x):
         return self.ops.layernorm_deferred(x, self.weight, None, self.eps, self.dtype, center=False)
