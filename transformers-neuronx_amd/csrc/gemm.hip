@@ -1319,47 +1319,36 @@ static void launch_skinny(const bf16_t* xp, const bf16_t* wp, const bf16_t* ws, 
 
 // The same next to a norm (see `RowNorm`), up to 8 rows, from the tile-ordered weight.
 template <int RT, int NORM, int ROWS, int PER>
-static int launch_skinny_norm(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
-                              int K, const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
+static void launch_skinny_norm(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
+                               int K, const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
   const dim3 grid((N + 16 * RT - 1) / (16 * RT));
   const unsigned lds = NORM == NORM_OPERAND ? M * (K + 8) * 2 : 0;
-  auto launch = [&](auto* kernel, const QkvScatter& places) {
-    if (lds > 32 * 1024) {
-      static bool configured = false;
-      if (!configured) {
-        const hipError_t e = hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 8 * (NORM_WIDTH + 8) * 2);
-        TNX_REQUIRE(e == hipSuccess, "product next to a norm: cannot reserve LDS: %s", hipGetErrorString(e));
-        configured = true;
-      }
-    }
-    kernel<<<grid, 256, lds, stream>>>(xp, ws, bias, nullptr, out, out_dtype, act, M, N, K, places, NormFold{}, norm);
-    return 0;
-  };
+  // (8 rows of 3,072 and what the kernel has beside them are 62 KB: no more than any launch may ask for)
   if constexpr (NORM == NORM_OPERAND) {
     if (sc) {
-      const auto with = [&](const QkvScatter& places) { return launch(gemm_bf16_skinny_kernel<1, 4, true, true, RT, false, NORM, ROWS, PER>, places); };
-      return with(*sc);
+      gemm_bf16_skinny_kernel<1, 4, true, true, RT, false, NORM, ROWS, PER><<<grid, 256, lds, stream>>>(
+          nullptr, ws, bias, nullptr, out, out_dtype, act, M, N, K, *sc, NormFold{}, norm);
+      return;
     }
   }
-  return launch(gemm_bf16_skinny_kernel<1, 4, false, true, RT, false, NORM, ROWS, PER>, QkvScatter{});
+  gemm_bf16_skinny_kernel<1, 4, false, true, RT, false, NORM, ROWS, PER><<<grid, 256, lds, stream>>>(
+      xp, ws, bias, nullptr, out, out_dtype, act, M, N, K, QkvScatter{}, NormFold{}, norm);
 }
 template <int RT, int NORM>
-static int skinny_norm_rows(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
+static void skinny_norm_rows(const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
                             const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
   const int width = NORM == NORM_OPERAND ? K : N;       // (registers for the rows as they are)
-#define SKINNY_NORM(PER)                                                                                                            \
-  return M <= 4 ? launch_skinny_norm<RT, NORM, 1, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)              \
-                : launch_skinny_norm<RT, NORM, 2, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
-  if (width <= 1024) SKINNY_NORM(4);
-  if (width <= 2048) SKINNY_NORM(8);
-  SKINNY_NORM(12);
+#define SKINNY_NORM(PER)                                                                                                             \
+  if (M <= 4) launch_skinny_norm<RT, NORM, 1, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);                  \
+  else launch_skinny_norm<RT, NORM, 2, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
+  if (width <= 1024) { SKINNY_NORM(4); } else if (width <= 2048) { SKINNY_NORM(8); } else { SKINNY_NORM(12); }
 #undef SKINNY_NORM
 }
 template <int RT>
-static int skinny_norm(int kind, const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
+static void skinny_norm(int kind, const bf16_t* xp, const bf16_t* ws, const float* bias, void* out, int out_dtype, int act, int M, int N,
                        int K, const QkvScatter* sc, const RowNorm& norm, hipStream_t stream) {
-  return kind == NORM_OPERAND ? skinny_norm_rows<RT, NORM_OPERAND>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
-                              : skinny_norm_rows<RT, NORM_RESIDUAL>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);
+  if (kind == NORM_OPERAND) skinny_norm_rows<RT, NORM_OPERAND>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);
+  else skinny_norm_rows<RT, NORM_RESIDUAL>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);
 }
 
 // How many tiles of 16 weight rows a block of the few-rows kernel takes (1, 2 or 3). Every block reads all of
@@ -1562,7 +1551,7 @@ extern "C" int tnx_gemm_bf16_by_norm(int kind, const RowNorm* norm, const void* 
   const bf16_t *xp = (const bf16_t*)x, *ws = (const bf16_t*)w;
   const int tiles = skinny_tiles_per_block(M, N);
 #define BY_NORM(RT) skinny_norm<RT>(kind, xp, ws, bias, out, out_dtype, act, M, N, K, nullptr, *norm, stream)
-  if (int rc = tiles == 3 ? BY_NORM(3) : tiles == 2 ? BY_NORM(2) : BY_NORM(1)) return rc;
+  if (tiles == 3) BY_NORM(3); else if (tiles == 2) BY_NORM(2); else BY_NORM(1);
 #undef BY_NORM
   TNX_CHECK_LAUNCH("gemm_bf16_by_norm");
   return 0;
@@ -1581,7 +1570,7 @@ extern "C" int tnx_gemm_bf16_by_norm_qkv(const RowNorm* norm, const void* w, con
   const bf16_t* ws = (const bf16_t*)w;
   const int tiles = skinny_tiles_per_block(M, N);
 #define BY_NORM(RT) skinny_norm<RT>(NORM_OPERAND, nullptr, ws, bias, nullptr, TNX_BF16, TNX_ACT_NONE, M, N, K, &sc, *norm, stream)
-  if (int rc = tiles == 3 ? BY_NORM(3) : tiles == 2 ? BY_NORM(2) : BY_NORM(1)) return rc;
+  if (tiles == 3) BY_NORM(3); else if (tiles == 2) BY_NORM(2); else BY_NORM(1);
 #undef BY_NORM
   TNX_CHECK_LAUNCH("gemm_bf16_by_norm_qkv");
   return 0;

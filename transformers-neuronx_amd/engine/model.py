@@ -173,7 +173,8 @@ class DecoderModel:
         ctx.input_state = caches[self.input_state_id] if self.input_state_id is not None else None
         stream: Stream = self.embedding.forward(ctx, want_compute)
         debug.tap("embedding", stream.x)
-        between = False             # what the last block left may be a norm that the next products do (`norms_between`)
+        # in steps of few rows, what the last block left may be a norm that the next products do (`norms_between`)
+        few, between = ctx.num_tokens <= getattr(self.ops, "norm_beside_rows", 0), False
         for call, (layer, cid, writes) in enumerate(self.schedule):
             cache = caches[cid] if writes else caches[cid].reader()
             state_id = self.call_state_ids[call]
@@ -182,7 +183,7 @@ class DecoderModel:
             if between and not getattr(block, "norms_between", False):
                 stream = self._settled(stream)
             stream = block.forward(stream, ctx, cache)
-            between = getattr(block, "norms_between", False)
+            between = few and getattr(block, "norms_between", False)
             debug.tap(f"call{call}.layer{layer}", stream.x)
         if between:
             stream = self._settled(stream)

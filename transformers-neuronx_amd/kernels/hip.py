@@ -676,6 +676,11 @@ class HipOps:
             return True
         return self.fold_norm(w, weight, bias, center)
 
+    def defer_rows(self, width) -> int:
+        """Steps of more rows have the norm's own kernel (and the host asks no further: what an unrecorded step of a short prompt
+        takes is host work)."""
+        return self.norm_beside_rows if width <= self.norm_operand_width else self.few_rows
+
     def _plain_beside(self, h, w) -> bool:
         """The norm `h` is the one before `w`, and the product of `w`'s own tile-ordered copy makes it."""
         return (isinstance(w, PreparedWeight) and w.tiles is not None and w.norm_before is not None and w.norm_before == h.key
@@ -749,7 +754,8 @@ class HipOps:
         """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
         left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
         of a larger tensor), instead of a tensor of its own."""
-        if isinstance(residual, NormBetween) or isinstance(x, NormBetween):
+        deferred = type(x) is not torch.Tensor and isinstance(x, DeferredNorm)
+        if (deferred and type(x) is NormBetween) or type(residual) is NormBetween:
             n, k = w.shape
             norm, kind = (x, 1) if isinstance(x, NormBetween) else (residual, 2)
             plain = x is not residual and not force_tiled and into is None and act in _ACT and (kind == 2) == (residual is not None)
@@ -762,8 +768,8 @@ class HipOps:
                 return self._linear_beside_norm(kind, norm, x if kind == 2 else None, t, bias, act,
                                                 torch.float32 if out_f32 else self.dtype, x.shape[0], n, k)
             residual = self.settled(residual)
-            x = x.settled()[1] if isinstance(x, NormBetween) else x
-        if isinstance(x, DeferredNorm):
+            x, deferred = (x.settled()[1], False) if type(x) is NormBetween else (x, deferred)
+        if deferred:
             folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
             if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
                                                               w.tensor, force_tiled, plain=True):
@@ -819,8 +825,8 @@ class HipOps:
         if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
         out_dtype = torch.float32 if out_f32 else self.dtype
-        if (tiles is not None and residual is None and not out_f32 and not force_tiled and into is None and w.dtype == torch.bfloat16
-                and _ptr(x) % 16 == 0 and self._whole_product(m, n, k)):
+        if (m <= self.whole_rows and tiles is not None and residual is None and not out_f32 and not force_tiled and into is None
+                and self._whole_product(m, n, k) and w.dtype == torch.bfloat16 and _ptr(x) % 16 == 0):
             return self._linear_whole(self.cast(x, torch.bfloat16), tiles, bias, act, n, k)
         if self._some_rows_product(m, n, k, w, tiles, residual, out_f32, force_tiled):
             # decode batches of 33 to 128 requests, a float32 result: our kernel for some rows
@@ -1126,8 +1132,8 @@ class HipOps:
         tiles = None
         if isinstance(w, PreparedWeight):
             w, tiles = w.tensor, w.tiles
-        whole = (tiles is not None and not force_tiled and w.dtype == h.dtype == torch.bfloat16 and _ptr(h) % 16 == 0
-                 and self._whole_product(ctx.num_tokens, *w.shape))
+        whole = (ctx.num_tokens <= self.whole_rows and tiles is not None and not force_tiled and self._whole_product(ctx.num_tokens, *w.shape)
+                 and w.dtype == h.dtype == torch.bfloat16 and _ptr(h) % 16 == 0)
         many = not whole and ctx.num_tokens >= 128 and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and not force_tiled
         if not whole and self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (many or self._library_product(
                 ctx.num_tokens, w.shape[0], w.shape[1], w, force_tiled, tiles is not None)):

@@ -116,6 +116,12 @@ class ReferenceOps:
     def defer_norm(self, w, weight, bias, center=True) -> bool:
         return False
 
+    norm_beside_rows = 0
+
+    def defer_rows(self, width) -> int:
+        """Up to how many rows `layernorm_deferred` may hand back something else than the norm's output."""
+        return 0
+
     def norm_between(self, x, weight, bias, eps, dtype, center=True):
         """A norm whose result is the stream itself: (float32, compute dtype); a backend may hand back twice something that
         the products next to it resolve (`HipOps.norm_between`), and `settled` makes a tensor of."""

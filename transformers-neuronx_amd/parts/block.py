@@ -80,7 +80,7 @@ class PostNormBlock(Block):
             if self.has_ff:
                 x, h = self._join(self.feed_forward_norm, x, [(self.feed_forward.forward(h, ctx, None), None, None, 1.0)])
             return Stream(x, h)
-        if self.norms_between:
+        if self.norms_between and ctx.num_tokens <= self.mixer_norm.ops.norm_beside_rows:
             x, h = stream.x, stream.compute
             if h is None:
                 h = self.mixer_norm.ops.cast(x, self.mixer_norm.dtype)

@@ -48,9 +48,12 @@ class LayerNorm(Norm):
         return self.weight, self.bias, True, self.eps
 
     def fold_into(self, w) -> bool:
+        self.defer_rows = self.ops.defer_rows(self.width)
         return self.ops.defer_norm(w, self.weight, self.bias)
 
     def deferred(self, x):
+        if x.shape[0] > self.defer_rows:
+            return self.forward(x, False, True)[1]
         return self.ops.layernorm_deferred(x, self.weight, self.bias, self.eps, self.dtype)
 
 
@@ -92,7 +95,10 @@ class RMSNorm(Norm):
         return self.weight, None, False, self.eps
 
     def fold_into(self, w) -> bool:
+        self.defer_rows = self.ops.defer_rows(self.width)
         return self.ops.defer_norm(w, self.weight, None, center=False)
 
     def deferred(self, x):
+        if x.shape[0] > self.defer_rows:
+            return self.forward(x, False, True)[1]
         return self.ops.layernorm_deferred(x, self.weight, None, self.eps, self.dtype, center=False)
