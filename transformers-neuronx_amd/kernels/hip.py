@@ -754,22 +754,15 @@ class HipOps:
         """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
         left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
         of a larger tensor), instead of a tensor of its own."""
-        deferred = type(x) is not torch.Tensor and isinstance(x, DeferredNorm)
-        if (deferred and type(x) is NormBetween) or type(residual) is NormBetween:
-            n, k = w.shape
-            norm, kind = (x, 1) if isinstance(x, NormBetween) else (residual, 2)
-            plain = x is not residual and not force_tiled and into is None and act in _ACT and (kind == 2) == (residual is not None)
-            t = self._beside_weight(w, x.shape[0], norm) if plain and (kind == 1 or out_f32) else None
-            if t is not None and kind == 2:
-                t = t if _want(x, "x", self.dtype, (norm.x.shape[0], k)) is x and norm.x.shape[1] == n and _ptr(x) % 16 == 0 else None
-            if t is not None and (kind == 2 or norm.x.shape[1] == k):
+        if type(x) is NormBetween:
+            tiles = self._beside_weight(w, x.x.shape[0], x) if residual is None and not force_tiled and into is None and act in _ACT else None
+            if tiles is not None and w.tensor.shape[1] == x.x.shape[1]:
                 if bias is not None:
-                    _want(bias, "bias", torch.float32, (n,))
-                return self._linear_beside_norm(kind, norm, x if kind == 2 else None, t, bias, act,
-                                                torch.float32 if out_f32 else self.dtype, x.shape[0], n, k)
-            residual = self.settled(residual)
-            x, deferred = (x.settled()[1], False) if type(x) is NormBetween else (x, deferred)
-        if deferred:
+                    _want(bias, "bias", torch.float32, (w.tensor.shape[0],))
+                return self._linear_beside_norm(1, x, None, tiles, bias, act, torch.float32 if out_f32 else self.dtype, x.x.shape[0],
+                                                *w.tensor.shape)
+            x = x.settled()[1]
+        if isinstance(x, DeferredNorm):
             folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
             if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
                                                               w.tensor, force_tiled, plain=True):
@@ -823,6 +816,13 @@ class HipOps:
         if bias is not None:
             _want(bias, "bias", torch.float32, (n,))
         if residual is not None:
+            if type(residual) is NormBetween:
+                norm, residual = residual, None
+                if (tiles is not None and out_f32 and not force_tiled and into is None and x.dtype == torch.bfloat16 and _ptr(x) % 16 == 0
+                        and tuple(norm.x.shape) == (m, n) and norm.done is None and self._norm_beside(m, n, self.norm_between_width)
+                        and all((_ptr(a) or 0) % 16 == 0 for a in (tiles, norm.x, norm.weight, norm.bias))):
+                    return self._linear_beside_norm(2, norm, x, tiles, bias, act, torch.float32, m, n, k)
+                residual = norm.settled()[0]
             _want(residual, "residual", torch.float32, (m, n))
         out_dtype = torch.float32 if out_f32 else self.dtype
         if (m <= self.whole_rows and tiles is not None and residual is None and not out_f32 and not force_tiled and into is None
@@ -1082,7 +1082,7 @@ class HipOps:
         `turn` = (a, b), float32 `[positions, head_size]`: element d of every query and key head of a token at
         position p becomes a[p, d] x[d] + b[p, d] x[d ^ 1] (bias added, before the scale), in the same launch."""
         turn_a, turn_b, turn_pos, turn_rows = self._turn_args(turn, head_size, ctx)
-        if isinstance(h, NormBetween):
+        if type(h) is NormBetween:
             tiles = None if force_tiled else self._beside_weight(w, h.x.shape[0], h)
             if tiles is not None:
                 return self._qkv_beside_norm(h, tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
