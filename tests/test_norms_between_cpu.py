@@ -1,0 +1,125 @@
+"""What a post-norm block hands to its parts in steps of few rows, with a backend that leaves a norm behind a sum to the products
+next to it: parts that say they take that get it, every other part, norm and arrangement gets tensors as in longer steps."""
+import pytest
+import torch
+
+from transformers_neuronx_amd.kernels.reference import ReferenceOps
+from transformers_neuronx_amd.parts import FeedForward, Mixer, Stream
+from transformers_neuronx_amd.parts.block import PostNormBlock
+from transformers_neuronx_amd.parts.feed_forward import DenseFeedForward
+from transformers_neuronx_amd.parts.base import residual_to_product
+from transformers_neuronx_amd.parts.norm import LayerNorm
+
+WIDTH, ROWS = 32, 5
+
+
+class Unmade:
+    """Stands for (float32, compute dtype) of a norm: nothing that a tensor can do."""
+
+    def __init__(self, made):
+        self.made = made
+
+
+class LateOps(ReferenceOps):
+    """Leaves the norms of up to eight rows to `linear`, as the HIP backend does."""
+
+    norm_beside_rows = 8
+
+    def __init__(self):
+        super().__init__(torch.float32, "cpu")
+        self.left = 0
+
+    def norm_between(self, x, weight, bias, eps, dtype, center=True):
+        made = self.layernorm(x, weight, bias, eps, dtype, True, True, center)
+        if x.shape[0] > self.norm_beside_rows:
+            return made
+        self.left += 1
+        return (Unmade(made),) * 2
+
+    def linear(self, x, w, bias=None, act=None, residual=None, **more):
+        x = x.made[1] if isinstance(x, Unmade) else x
+        residual = residual.made[0] if isinstance(residual, Unmade) else residual
+        return super().linear(x, w, bias, act=act, residual=residual, **more)
+
+    @staticmethod
+    def settled(x):
+        return x.made[0] if isinstance(x, Unmade) else x
+
+
+class Multiplies(Mixer):
+    def __init__(self, seed):
+        self.w = torch.randn(WIDTH, WIDTH, generator=torch.Generator().manual_seed(seed)) / WIDTH ** 0.5
+
+    def first_weight(self):
+        return self.w
+
+    @residual_to_product
+    def forward(self, h, ctx, cache, residual):
+        return self.ops.linear(self.ops.linear(h, self.w), self.w, None, residual=residual, out_f32=True)
+
+
+class AddsItself(Multiplies):
+    """Has a `first_weight` and adds the stream by itself."""
+
+    def forward(self, h, ctx, cache, residual):
+        return residual + self.ops.linear(self.ops.linear(h, self.w), self.w, None, out_f32=True)
+
+
+class DenseThatAdds(DenseFeedForward):
+    def forward(self, h, ctx, residual):
+        return residual * 1.0 + super().forward(h, ctx, None)
+
+
+class Counting(PostNormBlock):
+    """An arrangement of its own that looks at the stream."""
+
+    def forward(self, stream, ctx, cache):
+        self.seen = float(stream.x.sum())
+        return super().forward(stream, ctx, cache)
+
+
+class _Ctx:
+    num_tokens = ROWS
+
+
+def _dense(cls):
+    ff = cls(WIDTH, 48, "relu", "up", "down")
+    g = torch.Generator().manual_seed(3)
+    return ff, {"up.weight": torch.randn(48, WIDTH, generator=g) / 6, "up.bias": torch.randn(48, generator=g),
+                "down.weight": torch.randn(WIDTH, 48, generator=g) / 7, "down.bias": torch.randn(WIDTH, generator=g)}
+
+
+def _run(ops, mixer, ff, norm=LayerNorm, arrangement=PostNormBlock, layers=2):
+    g = torch.Generator().manual_seed(5)
+    stream, blocks = Stream(torch.randn(ROWS, WIDTH, generator=g)), []
+    for layer in range(layers):
+        m, (f, tensors), norms = mixer(layer), _dense(ff), [norm(WIDTH, 1e-5) for _ in "ab"]
+        for part, t in [(m, {}), (f, tensors)] + [(n, {".weight": 1 + torch.randn(WIDTH, generator=g) / 9,
+                                                      ".bias": torch.randn(WIDTH, generator=g)}) for n in norms]:
+            part.load(t, "", ops, torch.float32)
+        block = arrangement(m, f, *norms)
+        block.load({}, "", ops, torch.float32) if hasattr(block, "load") else None
+        block.after_load()
+        blocks.append(block)
+        if not block.norms_between:
+            stream = Stream(ops.settled(stream.x), None)
+        stream = block.forward(stream, _Ctx(), None)
+    return ops.settled(stream.x), blocks
+
+
+@pytest.mark.parametrize("mixer,ff,arrangement,left", [
+    (Multiplies, DenseFeedForward, PostNormBlock, True), (AddsItself, DenseFeedForward, PostNormBlock, False),
+    (Multiplies, DenseThatAdds, PostNormBlock, False), (Multiplies, DenseFeedForward, Counting, False)])
+def test_parts_that_take_a_norm_left_to_them(mixer, ff, arrangement, left):
+    want, _ = _run(ReferenceOps(torch.float32, "cpu"), mixer, ff, arrangement=arrangement)
+    ops = LateOps()
+    got, blocks = _run(ops, mixer, ff, arrangement=arrangement)
+    assert [b.norms_between for b in blocks] == [left] * 2 and (ops.left > 0) == left
+    assert torch.equal(got, want)
+
+
+def test_built_in_parts_say_so():
+    from transformers_neuronx_amd.parts.mixer import Attention
+    for part in (Attention, DenseFeedForward):
+        assert part.forward.residual_to_product
+    assert not getattr(FeedForward.forward, "residual_to_product", False) and not getattr(Mixer.forward, "residual_to_product", False)

@@ -1,5 +1,5 @@
 from .base import (BLOCKS, EMBEDDINGS, FEED_FORWARDS, HEADS, MIXERS, NORMS, POSITIONS, Block, CacheNeed,
-                   FeedForward, Mixer, Norm, Part, PositionEncoding, Stream, register_block,
+                   FeedForward, Mixer, Norm, Part, PositionEncoding, Stream, register_block, residual_to_product,
                    register_embedding, register_feed_forward, register_head, register_mixer,
                    register_norm, register_position)
 from .spec import LayerCall, LayerSpec, ModelSpec, ParamDecl, PartSpec

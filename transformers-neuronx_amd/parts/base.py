@@ -141,6 +141,15 @@ def joined_rows(parts):
     return w.contiguous(), bias, places
 
 
+def residual_to_product(forward):
+    """Marks the `forward` of a mixer or feed-forward that has a `first_weight` and does with `residual` nothing but hand it to
+    `ops.linear` as the residual of its last product. A block behind whose sums a norm
+    stands may then hand over `h` and `residual` as what `ops.norm_between` returns. The mark is the function's: a subclass with
+    a `forward` of its own has tensors again unless that is marked too."""
+    forward.residual_to_product = True
+    return forward
+
+
 class Mixer(Part):
     """Mixes information between the tokens of a request.
 

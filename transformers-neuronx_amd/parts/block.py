@@ -45,14 +45,16 @@ class PostNormBlock(Block):
     reads_compute_copy = True      # the mixer reads the stream itself, in the compute dtype
 
     # Both parts do with the stream nothing but a product of its rows and adding it to their last product's sums, and the norms
-    # are of a form that the backend's products know: in steps of few rows they norm it themselves.
+    # are of a form that the backend's products know: in steps of few rows they norm it themselves. Parts say so
+    # (`residual_to_product`), and an arrangement of its own around the same sums gets tensors.
     norms_between = False
 
     def after_load(self) -> None:
-        norms = (self.mixer_norm, self.feed_forward_norm)
-        self.norms_between = (self.alpha is None and self.has_ff and self.mixer.first_weight() is not None
-                              and self.feed_forward.first_weight() is not None and all(hasattr(n, "fused_form") for n in norms)
-                              and hasattr(self.mixer_norm.ops, "norm_between"))
+        norms, parts = (self.mixer_norm, self.feed_forward_norm), (self.mixer, self.feed_forward)
+        self.norms_between = (self.alpha is None and self.has_ff and hasattr(self.mixer_norm.ops, "norm_between")
+                              and type(self).forward is PostNormBlock.forward
+                              and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
+                              and all(hasattr(n, "fused_form") for n in norms))
 
     def _between(self, norm, x):
         weight, bias, center, eps = norm.fused_form()

@@ -1,7 +1,7 @@
 """Feed-forward parts."""
 from typing import Dict, List
 
-from .base import FeedForward, OffersRows, register_feed_forward
+from .base import FeedForward, OffersRows, register_feed_forward, residual_to_product
 from .spec import ParamDecl
 
 
@@ -48,6 +48,7 @@ class DenseFeedForward(FeedForward):
     def first_weight(self):
         return self.w1
 
+    @residual_to_product
     def forward(self, h, ctx, residual):
         """`residual` None: f(h) alone, in float32 (for an arrangement that norms it before the sum)."""
         if self.activation == "poly_norm":

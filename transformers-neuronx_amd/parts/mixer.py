@@ -4,7 +4,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-from .base import POSITIONS, CacheNeed, Mixer, OffersRows, register_mixer
+from .base import POSITIONS, CacheNeed, Mixer, OffersRows, register_mixer, residual_to_product
 from .spec import ParamDecl
 
 
@@ -326,6 +326,7 @@ class Attention(OffersRows, Mixer):
                                     distance_bias=self.bias_by_distance, gate=gate, value_size=self.value_size,
                                     out=out, out_scale=out_scale, **more)
 
+    @residual_to_product
     def forward(self, h, ctx, cache, residual, rows=None):
         if cache.writes != self.own_kv:
             raise ValueError("an attention mixer with own_kv writes its cache; one without reads another's")
