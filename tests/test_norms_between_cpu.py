@@ -8,7 +8,7 @@ from transformers_neuronx_amd.parts import FeedForward, Mixer, Stream
 from transformers_neuronx_amd.parts.block import PostNormBlock
 from transformers_neuronx_amd.parts.feed_forward import DenseFeedForward
 from transformers_neuronx_amd.parts.base import residual_to_product
-from transformers_neuronx_amd.parts.norm import LayerNorm
+from transformers_neuronx_amd.parts.norm import LayerNorm, RMSNorm
 
 WIDTH, ROWS = 32, 5
 
@@ -116,6 +116,23 @@ def test_parts_that_take_a_norm_left_to_them(mixer, ff, arrangement, left):
     got, blocks = _run(ops, mixer, ff, arrangement=arrangement)
     assert [b.norms_between for b in blocks] == [left] * 2 and (ops.left > 0) == left
     assert torch.equal(got, want)
+
+
+class Doubled(LayerNorm):
+    def forward(self, x, want_f32, want_compute):
+        return tuple(None if y is None else 2 * y for y in super().forward(x, want_f32, want_compute))
+
+
+class Renamed(RMSNorm):
+    pass
+
+
+@pytest.mark.parametrize("norm,left", [(LayerNorm, True), (RMSNorm, True), (Renamed, True), (Doubled, False)])
+def test_norms_with_a_forward_of_their_own_are_run(norm, left):
+    want, _ = _run(ReferenceOps(torch.float32, "cpu"), Multiplies, DenseFeedForward, norm=norm)
+    ops = LateOps()
+    got, _ = _run(ops, Multiplies, DenseFeedForward, norm=norm)
+    assert (ops.left > 0) == left and torch.equal(got, want)
 
 
 def test_built_in_parts_say_so():

@@ -32,6 +32,14 @@ class PreNormBlock(Block):
         return Stream(x, None)
 
 
+def _is_its_fused_form(norm) -> bool:
+    """Whether a norm's `forward` is what its `fused_form` says: one class has both (a subclass that changes one of them alone
+    is run, not formed again)."""
+    def owner(name):
+        return next((c for c in type(norm).__mro__ if name in vars(c)), None)
+    return owner("fused_form") is not None and owner("forward") is owner("fused_form")
+
+
 @register_block("post_norm")
 class PostNormBlock(Block):
     """`x = norm(alpha x + mixer(x))`, `x = norm(alpha x + feed_forward(x))`: the norm follows
@@ -54,7 +62,7 @@ class PostNormBlock(Block):
         self.norms_between = (self.alpha is None and self.has_ff and hasattr(self.mixer_norm.ops, "norm_between")
                               and type(self).forward is PostNormBlock.forward
                               and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
-                              and all(hasattr(n, "fused_form") for n in norms))
+                              and all(_is_its_fused_form(n) for n in norms))
 
     def _between(self, norm, x):
         weight, bias, center, eps = norm.fused_form()
