@@ -135,6 +135,25 @@ def test_norms_with_a_forward_of_their_own_are_run(norm, left):
     assert (ops.left > 0) == left and torch.equal(got, want)
 
 
+@pytest.mark.parametrize("norm", [LayerNorm, RMSNorm])
+def test_deferred_without_the_classes_own_fold_into(norm):
+    """A subclass that folds in a way of its own and inherits `deferred`."""
+    class Folding(norm):
+        def fold_into(self, w):
+            return self.ops.fold_norm(w, self.weight, None)
+
+    class FoldingOps(ReferenceOps):
+        def fold_norm(self, w, weight, bias, center=True):
+            return True
+
+        def layernorm_deferred(self, x, *more, **named):
+            return "left to the product"
+
+    n = Folding(WIDTH, 1e-5)
+    n.load({".weight": torch.ones(WIDTH), ".bias": torch.zeros(WIDTH)}, "", FoldingOps(torch.float32, "cpu"), torch.float32)
+    assert n.fold_into(None) and n.deferred(torch.zeros(3, WIDTH)) == "left to the product"
+
+
 def test_built_in_parts_say_so():
     from transformers_neuronx_amd.parts.mixer import Attention
     for part in (Attention, DenseFeedForward):

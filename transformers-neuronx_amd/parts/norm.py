@@ -1,4 +1,5 @@
 """Norm parts."""
+import math
 from typing import Dict, List
 
 from .base import Norm, register_norm
@@ -12,6 +13,8 @@ class LayerNorm(Norm):
     (reference: hlo.py:84-105, eps of hlo.py:51 passed in as a parameter)."""
 
     recordable = True
+
+    defer_rows = math.inf       # `deferred` asks the backend for steps of up to so many rows
 
     def __init__(self, width: int, eps: float, affine: bool = True, weight_suffix: str = ".weight",
                  bias_suffix: str = ".bias", bias: bool = True):
@@ -64,6 +67,8 @@ class RMSNorm(Norm):
     in float32)."""
 
     recordable = True
+
+    defer_rows = math.inf
 
     def __init__(self, width: int, eps: float, weight_suffix: str = ".weight", unit_offset: bool = False,
                  scalar: bool = False):
