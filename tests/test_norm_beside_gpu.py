@@ -128,3 +128,21 @@ def test_deferred_norms_of_plain_copies(m, k, n, center):
     want = y @ w.double().T + bias
     # independent roundings to bfloat16: the operand's and the result's, and a folded weight's
     assert (got.double() - want).norm() <= 2.5 * 2.0 ** -9 * want.norm()
+
+
+@pytest.mark.parametrize("m,k", [(4, 256), (8, 2048), (12, 1024)])
+def test_rows_and_vectors_that_no_norm_takes(m, k):
+    """Refused as the norm's own kernel refuses them, before a product is handed their addresses."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    dt = torch.bfloat16
+    hip = HipOps(dt, DEV)
+    x, weight = torch.randn(m, k, device=DEV), torch.ones(k, device=DEV)
+    w = hip.prepare_weight(torch.randn(64, k, device=DEV).to(dt))
+    assert hip.defer_norm(w, weight, None)
+    wide = torch.randn(m, 2 * k, device=DEV)
+    for rows, vector, error in ((wide[:, :k], weight, ValueError), (x[:1].expand(m, k), weight, ValueError),
+                                (torch.randn(k, m, device=DEV).t(), weight, ValueError), (x.to(dt), weight, TypeError),
+                                (x, weight[:k // 2], ValueError), (x, weight.to(dt), TypeError)):
+        for make in (lambda: hip.layernorm_deferred(rows, vector, None, 1e-5, dt), lambda: hip.norm_between(rows, vector, None, 1e-5, dt)[1]):
+            with pytest.raises(error):
+                hip.linear(make(), w)

@@ -644,13 +644,18 @@ class HipOps:
         return (self.norm_beside and self.dtype == torch.bfloat16 and 0 < rows <= self.norm_beside_rows and width % 128 == 0
                 and width <= most and not debug.tapping())
 
+    @staticmethod
+    def _want_norm(x, weight, bias):
+        """As `layernorm` wants them: a product that makes the norm is handed their addresses."""
+        _want(x, "x", torch.float32)
+        for v, name in ((weight, "norm weight"), (bias, "norm bias")):
+            if v is not None:
+                _want(v, name, torch.float32, (x.shape[1],))
+
     def norm_between(self, x, weight, bias, eps, dtype, center=True):
         """(float32, compute dtype) of a norm whose result is the stream itself; both a `NormBetween` in steps of few rows."""
         if dtype == torch.bfloat16 and self._norm_beside(x.shape[0], x.shape[1], self.norm_between_width):
-            _want(x, "x", torch.float32)
-            for v, name in ((weight, "norm weight"), (bias, "norm bias")):
-                if v is not None:
-                    _want(v, name, torch.float32, (x.shape[1],))
+            self._want_norm(x, weight, bias)
             d = NormBetween(self, x, weight, bias, eps, dtype, center)
             return d, d
         return self.layernorm(x, weight, bias, eps, dtype, True, True, center)
@@ -704,6 +709,7 @@ class HipOps:
         """The compute-dtype output of the norm, or, in steps of few rows, a `DeferredNorm`."""
         if self.fuse_norm and dtype == torch.bfloat16 and self.dtype == torch.bfloat16 \
                 and x.shape[0] <= self.few_rows and x.shape[1] % 128 == 0 and not debug.tapping():
+            self._want_norm(x, weight, bias)
             return DeferredNorm(self, x, weight, bias, eps, dtype, center)
         return self.layernorm(x, weight, bias, eps, dtype, False, True, center)[1]
 
