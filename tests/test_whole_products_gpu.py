@@ -53,6 +53,24 @@ def test_folded_and_plain_copies_of_their_sizes(m):
         assert (got.double() - want).norm() <= 3 * 2.0 ** -9 * want.norm()
 
 
+@pytest.mark.parametrize("m,n,k,linear,placed", [
+    (16, 3072, 16384, False, False), (24, 4096, 4096, False, False), (48, 4096, 16384, False, False), (9, 6144, 4096, False, False),
+    (16, 8192, 8192, False, False), (16, 16384, 4096, False, False), (17, 16384, 4096, True, True), (16, 12288, 4096, True, True),
+    (16, 15360, 5120, True, True), (16, 8192, 2048, True, True), (24, 6144, 4096, True, True), (32, 6144, 4096, False, True),
+    (33, 6144, 4096, True, True), (48, 16384, 1024, False, True), (48, 12288, 2048, True, True), (32, 16384, 1024, True, True),
+    (40, 5632, 4096, False, False), (40, 16400, 4096, False, False), (40, 8192, 1024, False, False)])
+def test_the_rule_on_sizes(m, n, k, linear, placed):
+    """The lines of the rule at 256 units, by what lies on either side of each, and that a step goes where the rule says."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip = HipOps(torch.bfloat16, DEV)
+    hip.compute_units = 256
+    assert (hip._whole_product(m, n, k), hip._whole_product(m, n, k, placed=True)) == (linear, placed)
+    called = []
+    hip._linear_whole = lambda *a: called.append(a)
+    hip.linear(torch.zeros(m, k, device=DEV, dtype=torch.bfloat16), hip.prepare_weight(torch.zeros(n, k, device=DEV, dtype=torch.bfloat16)))
+    assert bool(called) == (linear and n % 16 == 0)
+
+
 @pytest.mark.parametrize("m,heads,kv,hs,k,turned", [(9, 32, 32, 64, 2048, False), (40, 32, 32, 64, 2048, True), (24, 32, 32, 80, 2560, False)])
 def test_queries_keys_and_values(m, heads, kv, hs, k, turned):
     """The same places hold what the few-rows kernel, or the product and the launch behind it, leave there."""

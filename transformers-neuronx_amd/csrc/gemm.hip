@@ -1832,7 +1832,7 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 }
 
 // The same for 9 to 48 rows with a rounded result, or with queries, keys and values put in their places, and K whole: no sum
-// follows, and what fills the chip is the number of waves a block has, one to four of 16 columns each: as many as leave every
+// follows, and what fills the chip is the number of waves a block has, two to four of 16 columns each: as many as leave every
 // compute unit one block (`whole_waves`). A unit brings some 30 bytes a nanosecond from memory however many ask on it, so what
 // counts is that all of them do: 10,240 columns of K 2,560 at 24 rows by blocks of one wave (640 blocks) to four (160) 17.2, 18.2,
 // 14.6 and 17.0 us. Measured on weights that no cache holds, us, with what took them before (the few-rows kernel up to 24 rows
@@ -1840,7 +1840,8 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 // 13.5 / 11.9; 8,192 x 2,048 10.3 / 9.2, 12.0 / 10.3, 14.4 / 10.6, 15.1 / 12.6; 10,240 x 2,560 14.6 / 13.0, 20.8 / 14.6, 21.3 / 15.4, 20.7 / 19.8;
 // 12,288 x 4,096 21.6 / 20.4, 28.4 / 21.5, 33.0 / 22.1, 28.2 / 25.2; 16,384 x 4,096 28.3 / 28.6, 32.0 / 29.8, 33.5 / 29.9, 35.6 / 32.6. Not for
 // small matrices (24 rows 3,072 x 1,024 6.1 / 6.4: a chain of steps, where the few-rows kernel's waves share K) nor at 64 rows
-// (12,288 x 4,096 27.5 / 29.4: the rows weigh as much as the weights).
+// (12,288 x 4,096 27.5 / 29.4: the rows weigh as much as the weights), nor where one wave a block covers the columns (16 rows
+// 4,096 x 4,096 10.4 / 12.8: the same chain); further lines stand with the rule (`HipOps._whole_product`).
 template <typename Scatter>
 static int launch_whole(const bf16_t* x, const bf16_t* w_tiles, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
                         int waves, const Scatter& sc, hipStream_t stream) {

@@ -993,15 +993,31 @@ class HipOps:
         shares = max(1, min(self.compute_units // column_blocks, k // 512))     # as the kernel shares K out
         return small or 4 * column_blocks * shares >= 3 * self.compute_units
 
-    # Products of so many rows with a rounded result from a tile-ordered copy, where a block of one to four waves a compute unit
+    # Products of so many rows with a rounded result from a tile-ordered copy, where a block of two to four waves a compute unit
     # fills seven tenths of them (`gemm_bf16_mid`'s form with K whole; what it measured stands there).
     whole_rows_from, whole_rows = 9, 48
 
-    def _whole_product(self, m, n, k) -> bool:
+    def _whole_product(self, m, n, k, placed=False) -> bool:
+        """`placed`: queries, keys and values, which the other ways of more than 24 rows put in their places by a launch of its
+        own. The lines by old / new us on weights that no cache holds, 256 units:
+        - two waves or more: columns that one wave a block covers leave each unit one chain of K, where the other kernels share
+          K out (16 rows 3,072 x 4,096 9.3 / 11.3, 4,096 x 16,384 29.7 / 38.7; 48 rows 30.8 / 47.1 and 40.5 / 47.8);
+        - up to 16 rows and K of 4,096 or more, three waves, or four that not every unit has: 9 rows 6,144 x 4,096 13.1 / 14.1, 8,192 x
+          8,192 25.4 / 26.2, 16,384 x 4,096 26.8 / 28.1, but 12,288 x 4,096 21.2 / 20.2, 9,216 x 9,216 and 15,360 x 5,120 3 and 8 % less;
+        - 25 to 32 rows, not placed: not two waves that fewer than eight units in ten have (32 rows 5,760 x 4,096 16.0 / 17.1);
+        - more than 32 rows, not placed: K of 2,048 or more, or two waves: the tiles, which read the rows once for more columns, take
+          many columns of short K (48 rows 16,384 x 1,024 10.3 / 13.1, x 2,048 16.8 / 16.6; placed, 12,288 x 768 14.9 / 11.3)."""
         if not (self.whole_rows_from <= m <= self.whole_rows and self.dtype == torch.bfloat16 and n * k > self.small_matrix):
             return False
-        waves = -(-n // (16 * self.compute_units))
-        return waves <= 4 and 10 * n >= 7 * 16 * waves * self.compute_units
+        wave = 16 * self.compute_units         # columns of a wave on every unit
+        waves = -(-n // wave)
+        if not (2 <= waves <= 4 and 10 * n >= 7 * waves * wave):
+            return False
+        if m <= 16 and k >= 4096:
+            return 2 * wave < n < 4 * wave
+        if placed or m <= 24:
+            return True
+        return 10 * n >= 16 * wave if m <= 32 else waves == 2 or k >= 2048
 
     def _linear_whole(self, x, tiles, bias, act, n, k):
         if act not in _ACT:
@@ -1102,7 +1118,7 @@ class HipOps:
             if not force_tiled and self._plain_beside(h, w):
                 return self._qkv_beside_norm(h, w.tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
                                              k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
-            if few and not force_tiled and self._whole_product(rows, *w.tensor.shape):
+            if few and not force_tiled and self._whole_product(rows, *w.tensor.shape, placed=True):
                 h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
             elif not few:
                 h = h.materialize()
@@ -1138,7 +1154,7 @@ class HipOps:
         tiles = None
         if isinstance(w, PreparedWeight):
             w, tiles = w.tensor, w.tiles
-        whole = (ctx.num_tokens <= self.whole_rows and tiles is not None and not force_tiled and self._whole_product(ctx.num_tokens, *w.shape)
+        whole = (ctx.num_tokens <= self.whole_rows and tiles is not None and not force_tiled and self._whole_product(ctx.num_tokens, *w.shape, placed=True)
                  and w.dtype == h.dtype == torch.bfloat16 and _ptr(h) % 16 == 0)
         many = not whole and ctx.num_tokens >= 128 and w.shape[1] % 64 == 0 and w.shape[0] % 8 == 0 and not force_tiled
         if not whole and self.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and (many or self._library_product(
