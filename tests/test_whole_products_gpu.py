@@ -57,7 +57,7 @@ def test_folded_and_plain_copies_of_their_sizes(m):
     (16, 3072, 16384, False, False), (24, 4096, 4096, False, False), (48, 4096, 16384, False, False), (9, 6144, 4096, False, False),
     (16, 8192, 8192, False, False), (16, 16384, 4096, False, False), (17, 16384, 4096, True, True), (16, 12288, 4096, True, True),
     (16, 15360, 5120, True, True), (16, 8192, 2048, True, True), (24, 6144, 4096, True, True), (32, 6144, 4096, False, True),
-    (33, 6144, 4096, True, True), (48, 16384, 1024, False, True), (48, 12288, 2048, True, True), (32, 16384, 1024, True, True),
+    (33, 6144, 4096, True, True), (48, 15360, 5120, False, True), (48, 16384, 4096, True, True), (48, 16384, 1024, False, True), (48, 12288, 2048, True, True), (32, 16384, 1024, True, True),
     (40, 5632, 4096, False, False), (40, 16400, 4096, False, False), (40, 8192, 1024, False, False)])
 def test_the_rule_on_sizes(m, n, k, linear, placed):
     """The lines of the rule at 256 units, by what lies on either side of each, and that a step goes where the rule says."""

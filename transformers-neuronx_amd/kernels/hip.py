@@ -1006,7 +1006,8 @@ class HipOps:
           8,192 25.4 / 26.2, 16,384 x 4,096 26.8 / 28.1, but 12,288 x 4,096 21.2 / 20.2, 9,216 x 9,216 and 15,360 x 5,120 3 and 8 % less;
         - 25 to 32 rows, not placed: not two waves that fewer than eight units in ten have (32 rows 5,760 x 4,096 16.0 / 17.1);
         - more than 32 rows, not placed: K of 2,048 or more, or two waves: the tiles, which read the rows once for more columns, take
-          many columns of short K (48 rows 16,384 x 1,024 10.3 / 13.1, x 2,048 16.8 / 16.6; placed, 12,288 x 768 14.9 / 11.3)."""
+          many columns of short K (48 rows 16,384 x 1,024 10.3 / 13.1, x 2,048 16.8 / 16.6; placed, 12,288 x 768 14.9 / 11.3); and
+          not four waves that some units lack (48 rows 15,360 x 5,120 35.3 / 37.8, 13,056 x 2,048 17.0 / 18.0)."""
         if not (self.whole_rows_from <= m <= self.whole_rows and self.dtype == torch.bfloat16 and n * k > self.small_matrix):
             return False
         wave = 16 * self.compute_units         # columns of a wave on every unit
@@ -1017,7 +1018,9 @@ class HipOps:
             return 2 * wave < n < 4 * wave
         if placed or m <= 24:
             return True
-        return 10 * n >= 16 * wave if m <= 32 else waves == 2 or k >= 2048
+        if m <= 32:
+            return 10 * n >= 16 * wave
+        return waves == 2 or (k >= 2048 and (waves == 3 or n == 4 * wave))
 
     def _linear_whole(self, x, tiles, bias, act, n, k):
         if act not in _ACT:
