@@ -68,6 +68,29 @@ def test_float32_product_by_parts(m, n, k):
     assert bool(torch.isfinite(got[5:]).all())
 
 
+@pytest.mark.parametrize("m,n,k,shares", [(17, 1024, 1024, 16), (64, 1024, 1024, 11), (31, 132, 4096, 16), (33, 2304, 768, 6), (128, 512, 4096, 16),
+                                          (129, 512, 4096, 8)])
+def test_shares_of_few_rows(m, n, k, shares):
+    """K shared out over up to sixteen blocks at 128 rows, eight beyond; every share's sums go out by themselves, and what is not
+    finite in one is made again in it. Bound: as `test_float32_product_by_parts`, and the shares' sum."""
+    from transformers_neuronx_amd.kernels.hip import HipOps, library
+    hip, g = HipOps(torch.float32, DEV), _gen(m + n + k)
+    if hip.compute_units == 256:
+        assert library("gemm").tnx_gemm_f32_workspace(m, n, k) == shares * m * n
+    x, w = torch.randn(m, k, device=DEV, generator=g), torch.randn(n, k, device=DEV, generator=g)
+    bias, residual = torch.randn(n, device=DEV, generator=g), torch.randn(m, n, device=DEV, generator=g)
+    want = (x.double() @ w.double().T + bias).relu() + residual
+    size = x.double().abs() @ w.double().abs().T + bias.abs() + residual.abs()
+    got = hip.linear(x, w, bias, act="relu", residual=residual, out_f32=True)
+    assert bool(((got.double() - want).abs() <= (k / 16 + 8 + 16) * 2.0 ** -23 * size).all())
+    w[3] = w[3].abs()
+    x[0, 5], x[1, k - 1], x[m - 1, k // 2] = float("inf"), float("nan"), 3.4e38
+    w[:, k // 2] = 0.25
+    got = hip.linear(x, w, None, out_f32=True)
+    assert got[0, 3].item() == float("inf") and bool(got[1].isnan().all())
+    assert bool((got[m - 1] == x[m - 1, k // 2] * 0.25).all()) and bool(torch.isfinite(got[2:]).all())
+
+
 def _step(runs, cached, page, seed):
     from transformers_neuronx_amd.engine.batch import StepEntry, build_context
     from transformers_neuronx_amd.kernels.attention_plan import attention_plan

@@ -437,29 +437,53 @@ gemm_f32_parts_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     for (int k = 0; k < 32 * steps; ++k) sum = fmaf(xr[k], wr[k], sum);
     return sum;
   };
-  __syncthreads();      // the stages are free: the result goes through them
   const int mw = m0 + wm, nw = n0 + wn;
+  if (partial) {
+    // A share's sums go out from the registers as they lie, four columns of a lane together (N is a multiple of 4): through LDS,
+    // as the result below, the whole kernel took 1.1 us longer.
+#pragma unroll
+    for (int i = 0; i < MI; ++i) {
+      const int m = mw + 32 * i + l32;
+      if (m >= M) continue;
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const int n = nw + 32 * j + 8 * g + 4 * half;
+          if (n >= N) continue;
+          f32x4 v;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][4 * g + e];
+          const float none = (v[0] * 0.f + v[1] * 0.f) + (v[2] * 0.f + v[3] * 0.f);     // 0, or no number where one of them is not finite
+          if (__builtin_expect(none != none, 0)) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = checked(v[e], m, n + e);
+          }
+          *(f32x4*)(partial + ((size_t)blockIdx.y * M + m) * N + n) = v;
+        }
+    }
+    return;
+  }
+  __syncthreads();      // the stages are free: the result goes through them
   float added[NI][16];
 #pragma unroll
   for (int j = 0; j < NI; ++j)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) added[j][e] = bias && !partial ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3), N - 1)] : 0.f;
+    for (int e = 0; e < 16; ++e) added[j][e] = bias ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3), N - 1)] : 0.f;
   auto value = [&](int i, int j, int e, int row, int column) {
     const float v = mw + row < M && nw + column < N ? checked(acc[i][j][e], mw + row, nw + column) : 0.f;
-    return partial ? v : apply_act(v + added[j][e], act);
+    return apply_act(v + added[j][e], act);
   };
-  float* dest = partial ? partial + (size_t)blockIdx.y * M * N : (float*)out;
-  const float* onto = partial ? nullptr : residual;
   Tile<MI, NI, 2, WM, WN>::template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
     if (mw + r >= M || nw + c >= N) return;
     const size_t o = (size_t)(mw + r) * N + nw + c;
     if (whole) {
-      if (onto) chunk += *(const f32x4*)(onto + o);
-      *(f32x4*)(dest + o) = chunk;
+      if (residual) chunk += *(const f32x4*)(residual + o);
+      *(f32x4*)((float*)out + o) = chunk;
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e)
-        if (nw + c + e < N) store_any(out, out_dtype, o + e, chunk[e] + (onto ? onto[o + e] : 0.f));
+        if (nw + c + e < N) store_any(out, out_dtype, o + e, chunk[e] + (residual ? residual[o + e] : 0.f));
     }
   });
 }
@@ -482,8 +506,8 @@ static int launch_f32_parts(const float* x, const float* w, const float* bias, c
   const int tiles_m = (M + 32 * MI * WM - 1) / (32 * MI * WM), tiles_n = (N + 32 * NI * WN - 1) / (32 * NI * WN);
   const int per = (K / 32 + shares - 1) / shares;
   shares = (K / 32 + per - 1) / per;
-  // whole chunks of 16 bytes in every row of the result (of the shares' sums always: the caller sees to it)
-  const int whole = shares > 1 || (N % 4 == 0 && out_dtype == TNX_F32 && ((uintptr_t)out | (uintptr_t)residual) % 16 == 0);
+  // whole chunks of 16 bytes in every row of the result
+  const int whole = N % 4 == 0 && out_dtype == TNX_F32 && ((uintptr_t)out | (uintptr_t)residual) % 16 == 0;
   gemm_f32_parts_kernel<MI, NI, WM, WN><<<dim3(tiles_m * tiles_n, shares), 64 * WM * WN, bytes, stream>>>(
       x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, whole, M, N, K, tiles_m, per);
   TNX_CHECK_LAUNCH("gemm_f32_parts");
@@ -498,21 +522,30 @@ static int launch_f32_parts(const float* x, const float* w, const float* bias, c
 // The most floats that the shares' sums of one product may take (32 MB).
 constexpr long long F32_SHARES_MOST = 8 << 20;
 
-// The tile (128 x 128, 64 x 128, 64 x 64) and the shares of K, by what the fullest compute unit takes in us: a step of 32 of K of
-// the blocks it has (measured: one of 128 x 128 1.28, and no second fits its LDS; 64 x 128 0.70 and 1.35 for one and two at once;
-// 64 x 64 0.50, 0.88, 1.26), a beginning and an end, and the sum of the shares.
+// The tile (128 x 128, 64 x 128, 64 x 64) and the shares of K, by what a launch takes in us: a step of 32 of K of the blocks that
+// the fullest compute unit has (measured: one of 128 x 128 1.28, and no second fits its LDS; 64 x 128 0.70 and 1.35 for one and two
+// at once; 64 x 64 0.50, 0.88, 1.26), a beginning and an end, and the sum of the shares.
+// Up to 128 rows the launch is a chain of few steps, and its parts are a fit to 2,253 launches: 17 matrices from 64 x 64 to 12,288 x
+// 4,096, 17 to 128 rows, all tiles, up to 16 shares of two steps or more, on weights that no cache holds; what it picks takes 1.01 of
+// the quickest on average, 1.14 at most. Beyond, up to eight shares of four steps: fewer of them would be up to 15 % quicker at 180
+// to 400 rows of many columns, at sums of twice the length and error.
+// us by the float32 instructions (32x32x2) before / so: 1,024 x 1,024 at 17, 64 and 256 rows 8.7 / 8.7, 9.4 / 9.4, 13.3 / 14.5; 3,072 x 1,024
+// at 17 and 64 10.6 / 10.7, 12.3 / 12.8; 1,024 x 4,096 15.9 / 12.3 and 16.7 / 14.0; 2,048 x 2,048 at 64 13.5 / 14.0; the worst 2,304 x 768 at
+// 17 and 64, 8.8 / 9.4 and 10.4 / 11.0, and single tiles (64 x 64 of K 64 5.6 / 6.0): the split of an operand is a longer beginning.
 static void choose_f32_tiles(int M, int N, int K, int& tile, int& shares) {
-  const int units = tnx_compute_units(), steps = K / 32;
+  const int units = tnx_compute_units(), steps = K / 32, few = M <= 128;
   const int sizes[3][2] = {{128, 128}, {64, 128}, {64, 64}};
-  const double block_step[3] = {1.28, 0.65, 0.38}, step_more[3] = {0.0, 0.05, 0.12};
+  const double block_step[2][3] = {{1.28, 0.65, 0.38}, {1.0, 0.655, 0.346}}, step_more[2][3] = {{0.0, 0.05, 0.12}, {0.0, 0.0, 0.19}};
+  const double ends[2][3] = {{0.0, 8.0, 8.0}, {6.1, 5.1, 5.5}}, block_ends[2][3] = {{8.0, 0.0, 0.0}, {0.45, 0.66, 0.0}};
+  const double sum[2] = {5.0, 1.0}, sum_element[2] = {1e-6, 2e-6};
   double best = 1e30;
   for (int i = 0; i < 3; ++i) {
     const long long tiles = (long long)((M + sizes[i][0] - 1) / sizes[i][0]) * ((N + sizes[i][1] - 1) / sizes[i][1]);
-    for (int s = 1; s <= 8 && (s == 1 || (N % 4 == 0 && steps / s >= 4 && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
+    for (int s = 1; s <= (few ? 16 : 8) && (s == 1 || (N % 4 == 0 && steps / s >= (few ? 2 : 4) && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
       const int per = (steps + s - 1) / s;
-      const long long blocks = (tiles * s + units - 1) / units;
-      double cost = per * ((double)blocks * block_step[i] + step_more[i]) + (i == 0 ? 8.0 * blocks : 8.0);
-      if (s > 1) cost += 5.0 + (double)M * N * (s + 1) * 1e-6;
+      const long long blocks = (tiles * (few ? (steps + per - 1) / per : s) + units - 1) / units;
+      double cost = per * ((double)blocks * block_step[few][i] + step_more[few][i]) + ends[few][i] + blocks * block_ends[few][i];
+      if (s > 1) cost += sum[few] + (double)M * N * (s + 1) * sum_element[few];
       if (cost < best) best = cost, tile = i, shares = s;
     }
   }
@@ -1736,15 +1769,24 @@ gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__
   const size_t i = ((size_t)blockIdx.x * 256 + threadIdx.x) * 4;
   if (i >= (size_t)M * N) return;
   f32x4 v;
+  // every share is asked for before the first is added, so that the kernel waits for memory once; the order of the sum stays
+  // (up to eight, shares beyond the last read the last one again and are left out)
   if (shares <= 8) {
-    // every share is asked for before the first is added (shares beyond the last read the last one again and
-    // are left out), so that the kernel waits for memory once; the order of the sum stays
     f32x4 p[8];
 #pragma unroll
     for (int s = 0; s < 8; ++s) p[s] = *(const f32x4*)(partial + (size_t)min(s, shares - 1) * M * N + i);
     v = p[0];
 #pragma unroll
     for (int s = 1; s < 8; ++s)
+      if (s < shares) v += p[s];
+  } else if (shares <= 16) {
+    f32x4 p[16];
+#pragma unroll
+    for (int s = 0; s < 16; ++s)
+      if (s < shares) p[s] = *(const f32x4*)(partial + (size_t)s * M * N + i);
+    v = p[0];
+#pragma unroll
+    for (int s = 1; s < 16; ++s)
       if (s < shares) v += p[s];
   } else {
     v = *(const f32x4*)(partial + i);
