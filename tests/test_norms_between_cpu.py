@@ -5,7 +5,7 @@ import torch
 
 from transformers_neuronx_amd.kernels.reference import ReferenceOps
 from transformers_neuronx_amd.parts import FeedForward, Mixer, Stream
-from transformers_neuronx_amd.parts.block import PostNormBlock
+from transformers_neuronx_amd.parts.block import PostNormBlock, PreNormBlock
 from transformers_neuronx_amd.parts.feed_forward import DenseFeedForward
 from transformers_neuronx_amd.parts.base import residual_to_product
 from transformers_neuronx_amd.parts.norm import LayerNorm, RMSNorm
@@ -152,6 +152,33 @@ def test_deferred_without_the_classes_own_fold_into(norm):
     n = Folding(WIDTH, 1e-5)
     n.load({".weight": torch.ones(WIDTH), ".bias": torch.zeros(WIDTH)}, "", FoldingOps(torch.float32, "cpu"), torch.float32)
     assert n.fold_into(None) and n.deferred(torch.zeros(3, WIDTH)) == "left to the product"
+
+
+@pytest.mark.parametrize("tokens,asked", [(4, True), (5, False)])
+def test_longer_steps_ask_nothing_of_a_norm_left_to_a_product(tokens, asked):
+    """The pre-norm block compares the step's tokens with what the norm said at load, once a norm."""
+    class Few(LayerNorm):
+        calls = 0
+
+        def fold_into(self, w):
+            self.defer_rows = 4
+            return True
+
+        def deferred(self, x):
+            self.calls += 1
+            return self.forward(x, False, True)[1]
+
+    class Step(_Ctx):
+        num_tokens = tokens
+
+    ops, norms = ReferenceOps(torch.float32, "cpu"), [Few(WIDTH, 1e-5, affine=False) for _ in "ab"]
+    mixer, (ff, tensors) = Multiplies(1), _dense(DenseFeedForward)
+    for part, t in [(mixer, {}), (ff, tensors)] + [(n, {}) for n in norms]:
+        part.load(t, "", ops, torch.float32)
+    block = PreNormBlock(mixer, ff, *norms)
+    block.after_load()
+    block.forward(Stream(torch.randn(tokens, WIDTH)), Step(), None)
+    assert [n.calls for n in norms] == [int(asked)] * 2
 
 
 def test_built_in_parts_say_so():

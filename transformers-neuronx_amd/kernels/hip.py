@@ -755,56 +755,63 @@ class HipOps:
                 taken += size
         return taken
 
-    def linear(self, x, w, bias=None, act=None, residual=None, out_f32=False, force_tiled=False, f32_by_library=False,
-               into=None):
-        """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
-        left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
-        of a larger tensor), instead of a tensor of its own."""
+    def _linear_of_norm(self, x, w, bias, act, residual, out_f32, force_tiled, into):
+        """A product that reads a norm left to it: (the result, None), or (None, the norm's output) where the product is one
+        that takes tensors."""
         if type(x) is NormBetween:
             tiles = self._beside_weight(w, x.x.shape[0], x) if residual is None and not force_tiled and into is None and act in _ACT else None
             if tiles is not None and w.tensor.shape[1] == x.x.shape[1]:
                 if bias is not None:
                     _want(bias, "bias", torch.float32, (w.tensor.shape[0],))
                 return self._linear_beside_norm(1, x, None, tiles, bias, act, torch.float32 if out_f32 else self.dtype, x.x.shape[0],
-                                                *w.tensor.shape)
-            x = x.settled()[1]
+                                                *w.tensor.shape), None
+            return None, x.settled()[1]
+        folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
+        if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
+                                                          w.tensor, force_tiled, plain=True):
+            folded = None
+        if residual is None and not out_f32 and not force_tiled and act in _ACT and self._plain_beside(x, w):
+            if bias is not None:
+                _want(bias, "bias", torch.float32, (w.tensor.shape[0],))
+            return self._linear_beside_norm(1, x, None, w.tiles, bias, act, self.dtype, x.shape[0], *w.tensor.shape), None
+        if folded is not None and not force_tiled and self._whole_product(x.shape[0], *w.tensor.shape):
+            return self._linear_whole(x.normalised(), folded.tiles, folded.d_with(bias), act, *w.tensor.shape), None
+        if folded is None:
+            return None, x.materialize()
+        elif not force_tiled and act in _ACT and self._folded_beside(x, folded):
+            return self._linear_beside_norm(1, x, None, folded.tiles, folded.d_with(bias), act, self.dtype, x.shape[0],
+                                            w.tensor.shape[0], w.tensor.shape[1], alone=True), None
+        elif not self._norm_in_the_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
+            # the norm's kernel without weight and bias, then the plain product of the folded copy
+            m, k = x.shape
+            n = w.tensor.shape[0]
+            out = torch.empty(m, n, dtype=self.dtype, device=x.x.device)
+            rows, shift = x.normalised(), folded.d_with(bias)     # held until the launch is made
+            self._call("gemm", "tnx_gemm_bf16", _ptr(rows), _ptr(w.tensor), _ptr(folded.tiles), _ptr(shift), None,
+                       _ptr(out), _code(self.dtype), _ACT[act], m, n, k, int(force_tiled), _stream(),
+                       work=lambda: self._product_work(m, n, k))
+            return out, None
+        else:
+            if act not in _ACT:
+                raise ValueError(f"unknown activation {act!r}")
+            m, k = x.shape
+            n = w.tensor.shape[0]
+            if bias is not None:
+                _want(bias, "bias", torch.float32, (n,))
+            out = torch.empty(m, n, dtype=self.dtype, device=x.x.device)
+            self._call("gemm", "tnx_gemm_bf16_normed", _ptr(x.x), _ptr(folded.tiles), _ptr(folded.c),
+                       _ptr(folded.d), float(x.eps), _ptr(bias), _ptr(out), _code(self.dtype), _ACT[act], m, n, k,
+                       int(force_tiled), int(bool(x.center)), _stream(), work=lambda: self._product_work(m, n, k, x_item=4))
+            return out, None
+
+    def linear(self, x, w, bias=None, act=None, residual=None, out_f32=False, force_tiled=False, f32_by_library=False,
+               into=None):
+        """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
+        left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
+        of a larger tensor), instead of a tensor of its own."""
         if isinstance(x, DeferredNorm):
-            folded = self._folded_for(x, w) if (residual is None and not out_f32 and force_tiled != 1) else None
-            if folded is not None and self._library_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1],
-                                                              w.tensor, force_tiled, plain=True):
-                folded = None
-            if residual is None and not out_f32 and not force_tiled and act in _ACT and self._plain_beside(x, w):
-                if bias is not None:
-                    _want(bias, "bias", torch.float32, (w.tensor.shape[0],))
-                return self._linear_beside_norm(1, x, None, w.tiles, bias, act, self.dtype, x.shape[0], *w.tensor.shape)
-            if folded is not None and not force_tiled and self._whole_product(x.shape[0], *w.tensor.shape):
-                return self._linear_whole(x.normalised(), folded.tiles, folded.d_with(bias), act, *w.tensor.shape)
-            if folded is None:
-                x = x.materialize()
-            elif not force_tiled and act in _ACT and self._folded_beside(x, folded):
-                return self._linear_beside_norm(1, x, None, folded.tiles, folded.d_with(bias), act, self.dtype, x.shape[0],
-                                                w.tensor.shape[0], w.tensor.shape[1], alone=True)
-            elif not self._norm_in_the_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
-                # the norm's kernel without weight and bias, then the plain product of the folded copy
-                m, k = x.shape
-                n = w.tensor.shape[0]
-                out = torch.empty(m, n, dtype=self.dtype, device=x.x.device)
-                rows, shift = x.normalised(), folded.d_with(bias)     # held until the launch is made
-                self._call("gemm", "tnx_gemm_bf16", _ptr(rows), _ptr(w.tensor), _ptr(folded.tiles), _ptr(shift), None,
-                           _ptr(out), _code(self.dtype), _ACT[act], m, n, k, int(force_tiled), _stream(),
-                           work=lambda: self._product_work(m, n, k))
-                return out
-            else:
-                if act not in _ACT:
-                    raise ValueError(f"unknown activation {act!r}")
-                m, k = x.shape
-                n = w.tensor.shape[0]
-                if bias is not None:
-                    _want(bias, "bias", torch.float32, (n,))
-                out = torch.empty(m, n, dtype=self.dtype, device=x.x.device)
-                self._call("gemm", "tnx_gemm_bf16_normed", _ptr(x.x), _ptr(folded.tiles), _ptr(folded.c),
-                           _ptr(folded.d), float(x.eps), _ptr(bias), _ptr(out), _code(self.dtype), _ACT[act], m, n, k,
-                           int(force_tiled), int(bool(x.center)), _stream(), work=lambda: self._product_work(m, n, k, x_item=4))
+            out, x = self._linear_of_norm(x, w, bias, act, residual, out_f32, force_tiled, into)
+            if out is not None:
                 return out
         tiles = None
         if isinstance(w, PreparedWeight):
@@ -821,7 +828,8 @@ class HipOps:
             raise ValueError(f"x is {k} wide, w takes {kw}")
         if bias is not None:
             _want(bias, "bias", torch.float32, (n,))
-        if residual is not None:
+        out_dtype = torch.float32 if out_f32 else self.dtype
+        if m <= self.few_most:
             if type(residual) is NormBetween:
                 norm, residual = residual, None
                 if (tiles is not None and out_f32 and not force_tiled and into is None and x.dtype == torch.bfloat16 and _ptr(x) % 16 == 0
@@ -829,11 +837,11 @@ class HipOps:
                         and all((_ptr(a) or 0) % 16 == 0 for a in (tiles, norm.x, norm.weight, norm.bias))):
                     return self._linear_beside_norm(2, norm, x, tiles, bias, act, torch.float32, m, n, k)
                 residual = norm.settled()[0]
+            if (tiles is not None and residual is None and not out_f32 and not force_tiled and into is None
+                    and self._whole_product(m, n, k) and w.dtype == torch.bfloat16 and _ptr(x) % 16 == 0):
+                return self._linear_whole(self.cast(x, torch.bfloat16), tiles, bias, act, n, k)
+        if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
-        out_dtype = torch.float32 if out_f32 else self.dtype
-        if (m <= self.whole_rows and tiles is not None and residual is None and not out_f32 and not force_tiled and into is None
-                and self._whole_product(m, n, k) and w.dtype == torch.bfloat16 and _ptr(x) % 16 == 0):
-            return self._linear_whole(self.cast(x, torch.bfloat16), tiles, bias, act, n, k)
         if self._some_rows_product(m, n, k, w, tiles, residual, out_f32, force_tiled):
             # decode batches of 33 to 128 requests, a float32 result: our kernel for some rows
             out = torch.empty(m, n, dtype=out_dtype, device=x.device)
@@ -996,6 +1004,7 @@ class HipOps:
     # Products of so many rows with a rounded result from a tile-ordered copy, where a block of two to four waves a compute unit
     # fills seven tenths of them (`gemm_bf16_mid`'s form with K whole; what it measured stands there).
     whole_rows_from, whole_rows = 9, 48
+    few_most = 48           # products of more rows are asked none of this: their host time is part of a short prompt's
 
     def _whole_product(self, m, n, k, placed=False) -> bool:
         """`placed`: queries, keys and values, which the other ways of more than 24 rows put in their places by a launch of its
@@ -1107,53 +1116,54 @@ class HipOps:
         `turn` = (a, b), float32 `[positions, head_size]`: element d of every query and key head of a token at
         position p becomes a[p, d] x[d] + b[p, d] x[d ^ 1] (bias added, before the scale), in the same launch."""
         turn_a, turn_b, turn_pos, turn_rows = self._turn_args(turn, head_size, ctx)
-        if type(h) is NormBetween:
-            tiles = None if force_tiled else self._beside_weight(w, h.x.shape[0], h)
-            if tiles is not None:
-                return self._qkv_beside_norm(h, tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
-                                             k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
-            h = h.settled()[1]
         if isinstance(h, DeferredNorm):
-            folded = self._folded_for(h, w) if force_tiled != 1 else None
-            rows = h.shape[0]
-            few = (folded is not None and rows <= self.few_rows and ctx.num_tokens < 128
-                   and not self._library_product(ctx.num_tokens, *w.tensor.shape, w.tensor, force_tiled, True))
-            if not force_tiled and self._plain_beside(h, w):
-                return self._qkv_beside_norm(h, w.tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
-                                             k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
-            if few and not force_tiled and self._whole_product(rows, *w.tensor.shape, placed=True):
-                h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
-            elif not few:
-                h = h.materialize()
-            elif not force_tiled and self._folded_beside(h, folded):
-                return self._qkv_beside_norm(h, folded.tiles, folded.d_with(bias), tuple(w.tensor.shape), num_heads, num_kv_write, head_size,
-                                             scale, ctx, view, k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows, alone=True)
-            elif not self._norm_in_the_product(h.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
-                # the norm's kernel without weight and bias, then the fused projection of the folded copy
-                h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
+            if type(h) is NormBetween:
+                tiles = None if force_tiled else self._beside_weight(w, h.x.shape[0], h)
+                if tiles is not None:
+                    return self._qkv_beside_norm(h, tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
+                                                 k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
+                h = h.settled()[1]
             else:
-                t = ctx.num_tokens
-                total = (num_heads + 2 * num_kv_write) * head_size
-                _want(h.x, "x", torch.float32, (t, w.tensor.shape[1]))
-                if tuple(w.tensor.shape) != (total, h.x.shape[1]):
-                    raise ValueError(f"w is {tuple(w.tensor.shape)}, the projections need {(total, h.x.shape[1])}")
-                if bias is not None:
-                    _want(bias, "qkv bias", torch.float32, (total,))
-                num_pages = 0
-                if num_kv_write:
-                    num_pages = self._check_pages(k_pages, v_pages, num_kv_write, head_size, view.page_size)
-                _want(view.token_page, "token pages", torch.int32, (t,))
-                _want(view.token_offset, "token offsets", torch.int32, (t,))
-                q = torch.empty(t, num_heads * head_size, dtype=self.dtype, device=h.x.device)
-                self._call("gemm", "tnx_gemm_bf16_qkv_normed", _ptr(h.x), _ptr(folded.tiles), _ptr(folded.c),
-                           _ptr(folded.d), float(h.eps), _ptr(bias), t, h.x.shape[1], _ptr(view.token_page),
-                           _ptr(view.token_offset), _ptr(q), _ptr(k_pages) if num_kv_write else None,
-                           _ptr(v_pages) if num_kv_write else None, float(scale), num_heads, num_kv_write, head_size,
-                           view.page_size, num_pages, int(force_tiled), _ptr(turn_a), _ptr(turn_b), _ptr(turn_pos),
-                           turn_rows, self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size,
-                                                     view.page_size), int(bool(h.center)), _stream(),
-                           work=lambda: self._product_work(t, total, h.x.shape[1], x_item=4))
-                return q
+                folded = self._folded_for(h, w) if force_tiled != 1 else None
+                rows = h.shape[0]
+                few = (folded is not None and rows <= self.few_rows and ctx.num_tokens < 128
+                       and not self._library_product(ctx.num_tokens, *w.tensor.shape, w.tensor, force_tiled, True))
+                if not force_tiled and self._plain_beside(h, w):
+                    return self._qkv_beside_norm(h, w.tiles, bias, tuple(w.tensor.shape), num_heads, num_kv_write, head_size, scale, ctx, view,
+                                                 k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows)
+                if few and not force_tiled and self._whole_product(rows, *w.tensor.shape, placed=True):
+                    h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
+                elif not few:
+                    h = h.materialize()
+                elif not force_tiled and self._folded_beside(h, folded):
+                    return self._qkv_beside_norm(h, folded.tiles, folded.d_with(bias), tuple(w.tensor.shape), num_heads, num_kv_write, head_size,
+                                                 scale, ctx, view, k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows, alone=True)
+                elif not self._norm_in_the_product(h.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
+                    # the norm's kernel without weight and bias, then the fused projection of the folded copy
+                    h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
+                else:
+                    t = ctx.num_tokens
+                    total = (num_heads + 2 * num_kv_write) * head_size
+                    _want(h.x, "x", torch.float32, (t, w.tensor.shape[1]))
+                    if tuple(w.tensor.shape) != (total, h.x.shape[1]):
+                        raise ValueError(f"w is {tuple(w.tensor.shape)}, the projections need {(total, h.x.shape[1])}")
+                    if bias is not None:
+                        _want(bias, "qkv bias", torch.float32, (total,))
+                    num_pages = 0
+                    if num_kv_write:
+                        num_pages = self._check_pages(k_pages, v_pages, num_kv_write, head_size, view.page_size)
+                    _want(view.token_page, "token pages", torch.int32, (t,))
+                    _want(view.token_offset, "token offsets", torch.int32, (t,))
+                    q = torch.empty(t, num_heads * head_size, dtype=self.dtype, device=h.x.device)
+                    self._call("gemm", "tnx_gemm_bf16_qkv_normed", _ptr(h.x), _ptr(folded.tiles), _ptr(folded.c),
+                               _ptr(folded.d), float(h.eps), _ptr(bias), t, h.x.shape[1], _ptr(view.token_page),
+                               _ptr(view.token_offset), _ptr(q), _ptr(k_pages) if num_kv_write else None,
+                               _ptr(v_pages) if num_kv_write else None, float(scale), num_heads, num_kv_write, head_size,
+                               view.page_size, num_pages, int(force_tiled), _ptr(turn_a), _ptr(turn_b), _ptr(turn_pos),
+                               turn_rows, self._page_pad(k_pages if num_kv_write else None, num_kv_write, head_size,
+                                                         view.page_size), int(bool(h.center)), _stream(),
+                               work=lambda: self._product_work(t, total, h.x.shape[1], x_item=4))
+                    return q
         tiles = None
         if isinstance(w, PreparedWeight):
             w, tiles = w.tensor, w.tiles

@@ -6,6 +6,7 @@ step's context. Mixers also declare what they keep between steps
 (`cache_need`). Registering a class under a new kind is all it takes to use it
 from a `ModelSpec`.
 """
+import math
 from dataclasses import dataclass
 from typing import Callable, Dict, Hashable, List, Optional, Tuple
 
@@ -201,6 +202,8 @@ class Norm(Part):
         """Asked once, after loading, by a block whose next part only multiplies this norm's output by `w`:
         True if the backend has folded the norm into `w`, so that `deferred` may be used for that part."""
         return False
+
+    defer_rows = math.inf       # a block asks for `deferred` in steps of up to so many tokens (known once `fold_into` was asked)
 
     def deferred(self, x):
         """The compute-dtype output for a part whose `first_weight` this norm was folded into: the output

@@ -12,6 +12,7 @@ class PreNormBlock(Block):
     recordable = True
 
     fold_mixer_norm = fold_feed_forward_norm = False
+    mixer_norm_rows = feed_forward_norm_rows = -1     # up to how many tokens: what a step asks, once a norm
 
     def after_load(self) -> None:
         # Each norm's output goes to one part only; where that part does nothing with it but one matrix
@@ -21,12 +22,14 @@ class PreNormBlock(Block):
         self.fold_mixer_norm = w is not None and self.mixer_norm.fold_into(w)
         w = self.feed_forward.first_weight()
         self.fold_feed_forward_norm = w is not None and self.feed_forward_norm.fold_into(w)
+        self.mixer_norm_rows = self.mixer_norm.defer_rows if self.fold_mixer_norm else -1
+        self.feed_forward_norm_rows = self.feed_forward_norm.defer_rows if self.fold_feed_forward_norm else -1
 
     def forward(self, stream: Stream, ctx, cache) -> Stream:
-        h = (self.mixer_norm.deferred(stream.x) if self.fold_mixer_norm
+        h = (self.mixer_norm.deferred(stream.x) if ctx.num_tokens <= self.mixer_norm_rows
              else self.mixer_norm.forward(stream.x, False, True)[1])
         x = debug.tap("after_mixer", self.mixer.forward(h, ctx, cache, stream.x))
-        h = (self.feed_forward_norm.deferred(x) if self.fold_feed_forward_norm
+        h = (self.feed_forward_norm.deferred(x) if ctx.num_tokens <= self.feed_forward_norm_rows
              else self.feed_forward_norm.forward(x, False, True)[1])
         x = self.feed_forward.forward(h, ctx, x)
         return Stream(x, None)
@@ -56,6 +59,7 @@ class PostNormBlock(Block):
     # are of a form that the backend's products know: in steps of few rows they norm it themselves. Parts say so
     # (`residual_to_product`), and an arrangement of its own around the same sums gets tensors.
     norms_between = False
+    between_rows = -1              # and few are so many
 
     def after_load(self) -> None:
         norms, parts = (self.mixer_norm, self.feed_forward_norm), (self.mixer, self.feed_forward)
@@ -63,6 +67,7 @@ class PostNormBlock(Block):
                               and type(self).forward is PostNormBlock.forward
                               and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
                               and all(_is_its_fused_form(n) for n in norms))
+        self.between_rows = self.mixer_norm.ops.norm_beside_rows if self.norms_between else -1
 
     def _between(self, norm, x):
         weight, bias, center, eps = norm.fused_form()
@@ -90,7 +95,7 @@ class PostNormBlock(Block):
             if self.has_ff:
                 x, h = self._join(self.feed_forward_norm, x, [(self.feed_forward.forward(h, ctx, None), None, None, 1.0)])
             return Stream(x, h)
-        if self.norms_between and ctx.num_tokens <= self.mixer_norm.ops.norm_beside_rows:
+        if ctx.num_tokens <= self.between_rows:
             x, h = stream.x, stream.compute
             if h is None:
                 h = self.mixer_norm.ops.cast(x, self.mixer_norm.dtype)

@@ -1,5 +1,4 @@
 """Norm parts."""
-import math
 from typing import Dict, List
 
 from .base import Norm, register_norm
@@ -13,8 +12,6 @@ class LayerNorm(Norm):
     (reference: hlo.py:84-105, eps of hlo.py:51 passed in as a parameter)."""
 
     recordable = True
-
-    defer_rows = math.inf       # `deferred` asks the backend for steps of up to so many rows
 
     def __init__(self, width: int, eps: float, affine: bool = True, weight_suffix: str = ".weight",
                  bias_suffix: str = ".bias", bias: bool = True):
@@ -55,8 +52,6 @@ class LayerNorm(Norm):
         return self.ops.defer_norm(w, self.weight, self.bias)
 
     def deferred(self, x):
-        if x.shape[0] > self.defer_rows:
-            return self.forward(x, False, True)[1]
         return self.ops.layernorm_deferred(x, self.weight, self.bias, self.eps, self.dtype)
 
 
@@ -67,8 +62,6 @@ class RMSNorm(Norm):
     in float32)."""
 
     recordable = True
-
-    defer_rows = math.inf
 
     def __init__(self, width: int, eps: float, weight_suffix: str = ".weight", unit_offset: bool = False,
                  scalar: bool = False):
@@ -104,6 +97,4 @@ class RMSNorm(Norm):
         return self.ops.defer_norm(w, self.weight, None, center=False)
 
     def deferred(self, x):
-        if x.shape[0] > self.defer_rows:
-            return self.forward(x, False, True)[1]
         return self.ops.layernorm_deferred(x, self.weight, None, self.eps, self.dtype, center=False)
