@@ -96,7 +96,7 @@ def test_queries_keys_and_values(m, heads, kv, hs, k):
 
 @pytest.mark.parametrize("m,k,n", [(1, 256, 48), (8, 1024, 4096), (5, 2176, 6144), (8, 3072, 1040), (4, 2560, 10240), (8, 4096, 4096), (8, 3200, 4096)])
 def test_folded_copies(m, k, n):
-    """A folded copy's product from rows that it norms in LDS (up to 3,072 wide) and from shifted rows (wider)."""
+    """A folded copy's product, of the widths that layers fold (beyond 3,072) and of others, from shifted rows and behind the norm's kernel."""
     from transformers_neuronx_amd.kernels.hip import HipOps
     hip, g = HipOps(torch.bfloat16, DEV), _gen(m + k + n)
     t = torch.randn(m, k, device=DEV, generator=g) * 3 + torch.randn(m, 1, device=DEV, generator=g) * 5

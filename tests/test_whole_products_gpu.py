@@ -1,4 +1,4 @@
-"""Products of 9 to 48 rows by blocks of one to four waves with K whole, at the edges of their rows, columns and steps of K, against
+"""Products of 9 to 48 rows by blocks of two to four waves with K whole, at the edges of their rows, columns and steps of K, against
 64 bits. Bound: n 2^-24 of the sum of magnitudes for float32 sums of n exact products (first order; 2 covers the rest), and the
 result's rounding to bfloat16."""
 import pytest
@@ -13,9 +13,9 @@ def _gen(seed):
     return torch.Generator(device=DEV).manual_seed(seed)
 
 
-@pytest.mark.parametrize("waves", [1, 2, 3, 4])
+@pytest.mark.parametrize("waves", [0, 2, 3, 4])
 @pytest.mark.parametrize("m,n,k", [(1, 16, 128), (9, 48, 256), (16, 80, 384), (17, 208, 512), (32, 1040, 640), (33, 64, 1152), (48, 112, 2048),
-                                   (64, 96, 128)])
+                                   (48, 96, 128)])
 def test_sizes(m, n, k, waves):
     from transformers_neuronx_amd.kernels.hip import HipOps, tile_order
     hip, g = HipOps(torch.bfloat16, DEV), _gen(m + n + k + waves)

@@ -945,7 +945,8 @@ static int launch_wide(const bf16_t* x, const bf16_t* w, const float* bias, cons
 // 4,096 columns of K 1,024 6.4, 7.0 / 5.2, 6.4 / 4.2, 4.5; 8,192 of 2,048 11.6, 12.3 / 9.9, 11.8 / 9.2, 10.1; 10,240 of 2,560 15.4, 16.3 /
 // 14.3, 16.0 / 13.5, 15.3; but 16,384 of 4,096 28.5, 29.6 / 27.3, 30.5 / 28.8, 32.3: wider rows take the registers and the time
 // of too many blocks. As a residual of 1,024, with the product of K 1,024 and of 4,096: 3.4, 4.0 and 6.1, 7.3 with the normed
-// residual there, 3.8, 4.4 and 6.4, 7.9 so.
+// residual there, 3.8, 4.4 and 6.4, 7.9 so. Norm, first product and second with the residual of a feed-forward of four times the
+// width, at 1 and 8 rows: 1,024 12.1, 13.8 / 10.7, 12.4; 1,536 17.8, 19.6 / 16.3, 19.2; 2,048 22.5, 25.6 / 21.1, 24.9, where it ends.
 struct RowNorm {
   const float* x;        // [M][width] float32
   const float* weight;   // [width], with `bias` or both null
@@ -957,7 +958,7 @@ enum NormKind { NORM_NONE = 0, NORM_OPERAND = 1, NORM_RESIDUAL = 2 };
 struct NoNorm {};
 template <int KIND>
 using NormArg = std::conditional_t<KIND == NORM_NONE, NoNorm, RowNorm>;
-constexpr int NORM_WIDTH = 3072;
+constexpr int NORM_OPERAND_WIDTH = 3072, NORM_RESIDUAL_WIDTH = 2048;
 
 // Rows wave, wave + 4 (below M) of the norm's by this wave of four. `ask` comes before the block asks for its weights: loads are
 // waited for in the order they were made.
@@ -1374,7 +1375,10 @@ static void skinny_norm_rows(const bf16_t* xp, const bf16_t* ws, const float* bi
 #define SKINNY_NORM(PER)                                                                                                             \
   if (M <= 4) launch_skinny_norm<RT, NORM, 1, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream);                  \
   else launch_skinny_norm<RT, NORM, 2, PER>(xp, ws, bias, out, out_dtype, act, M, N, K, sc, norm, stream)
-  if (width <= 1024) { SKINNY_NORM(4); } else if (width <= 2048) { SKINNY_NORM(8); } else { SKINNY_NORM(12); }
+  if (width <= 1024) { SKINNY_NORM(4); return; }
+  if constexpr (NORM == NORM_OPERAND)
+    if (width > 2048) { SKINNY_NORM(12); return; }
+  SKINNY_NORM(8);
 #undef SKINNY_NORM
 }
 template <int RT>
@@ -1569,10 +1573,10 @@ extern "C" int tnx_gemm_f32_qkv(const float* x, const float* w, const float* bia
 // width is K); NORM_RESIDUAL: what it gives is added to the result (its width is N).
 static int norm_fits(int kind, const RowNorm* norm, const void* w, int M, int N, int K) {
   TNX_REQUIRE(norm && norm->x && (kind == NORM_OPERAND || kind == NORM_RESIDUAL), "product next to a norm: no norm");
-  const int width = kind == NORM_OPERAND ? K : N;
-  TNX_REQUIRE(width <= NORM_WIDTH && norm->eps > 0.f &&
+  const int width = kind == NORM_OPERAND ? K : N, most = kind == NORM_OPERAND ? NORM_OPERAND_WIDTH : NORM_RESIDUAL_WIDTH;
+  TNX_REQUIRE(width <= most && norm->eps > 0.f &&
               ((uintptr_t)norm->x | (uintptr_t)norm->weight | (uintptr_t)norm->bias | (uintptr_t)w) % 16 == 0,
-              "product next to a norm: rows of up to %d that begin at multiples of 16 bytes, got %d", NORM_WIDTH, width);
+              "product next to a norm: rows of up to %d that begin at multiples of 16 bytes, got %d", most, width);
   TNX_REQUIRE(M > 0 && M <= 8 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0, "product next to a norm: bad sizes M=%d N=%d K=%d", M, N, K);
   return 0;
 }
@@ -1888,25 +1892,21 @@ template <typename Scatter>
 static int launch_whole(const bf16_t* x, const bf16_t* w_tiles, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
                         int waves, const Scatter& sc, hipStream_t stream) {
 #define WHOLE(MT, NW) launch_mid<MT, 3, NW, Scatter>(x, w_tiles, bias, nullptr, out, out_dtype, act, nullptr, M, N, K, 1, stream, sc)
-#define WHOLE_MT(MT) return waves == 1 ? WHOLE(MT, 1) : waves == 2 ? WHOLE(MT, 2) : waves == 3 ? WHOLE(MT, 3) : WHOLE(MT, 4)
-  switch ((M + 15) / 16) {
-    case 1:
-    case 2: WHOLE_MT(2);
-    case 3: WHOLE_MT(3);
-    default: WHOLE_MT(4);
-  }
+#define WHOLE_MT(MT) return waves == 2 ? WHOLE(MT, 2) : waves == 3 ? WHOLE(MT, 3) : WHOLE(MT, 4)
+  if (M <= 32) WHOLE_MT(2);
+  WHOLE_MT(3);
 #undef WHOLE_MT
 #undef WHOLE
 }
 
 static int whole_waves(int N) {
   const int units = tnx_compute_units(), tiles = N / 16;
-  return max(1, min(4, (tiles + units - 1) / units));
+  return max(2, min(4, (tiles + units - 1) / units));
 }
 
 static int whole_fits(const void* x, const void* w_tiles, int M, int N, int K, int waves) {
-  TNX_REQUIRE(M > 0 && M <= 64 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && waves >= 0 && waves <= 4,
-              "gemm_bf16_whole: up to 64 rows, N a multiple of 16, K of 128; got M=%d N=%d K=%d", M, N, K);
+  TNX_REQUIRE(M > 0 && M <= 48 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && (waves == 0 || (waves >= 2 && waves <= 4)),
+              "gemm_bf16_whole: up to 48 rows, N a multiple of 16, K of 128, two to four waves; got M=%d N=%d K=%d waves=%d", M, N, K, waves);
   TNX_REQUIRE(x && w_tiles && ((uintptr_t)x | (uintptr_t)w_tiles) % 16 == 0, "gemm_bf16_whole: operands must be there and 16-byte aligned");
   return 0;
 }

@@ -312,10 +312,9 @@ class DeferredNorm:
         """`(x - mean) rstd` alone, for a product with a folded copy."""
         return self.ops.layernorm(self.x, None, None, self.eps, self.dtype, False, True, self.center)[1]
 
-    def as_argument(self, alone=False):
-        """For the products next to a norm; `alone`: without weight and bias, as `normalised`."""
-        return _RowNorm(_ptr(self.x), None if alone else _ptr(self.weight), None if alone else _ptr(self.bias), self.eps,
-                        int(bool(self.center)))
+    def as_argument(self):
+        """For the products next to a norm."""
+        return _RowNorm(_ptr(self.x), _ptr(self.weight), _ptr(self.bias), self.eps, int(bool(self.center)))
 
 
 class NormBetween(DeferredNorm):
@@ -693,13 +692,9 @@ class HipOps:
                 and self._norm_beside(*h.x.shape, self.norm_operand_width)
                 and all((_ptr(a) or 0) % 16 == 0 for a in (w.tiles, h.x, h.weight, h.bias)))
 
-    def _folded_beside(self, h, folded) -> bool:
-        """A folded copy's product norms the rows itself, from LDS."""
-        return self._norm_beside(h.x.shape[0], h.x.shape[1], self.norm_operand_width) and (_ptr(h.x) | _ptr(folded.tiles)) % 16 == 0
-
-    def _linear_beside_norm(self, kind, norm, x, t, bias, act, out_dtype, m, n, k, alone=False):
+    def _linear_beside_norm(self, kind, norm, x, t, bias, act, out_dtype, m, n, k):
         out = torch.empty(m, n, dtype=out_dtype, device=norm.x.device)
-        how = norm.as_argument(alone)
+        how = norm.as_argument()
         self._call("gemm", "tnx_gemm_bf16_by_norm", kind, ctypes.addressof(how), _ptr(x), _ptr(t), _ptr(bias), _ptr(out), _code(out_dtype),
                    _ACT[act], m, n, k, _stream(),
                    work=lambda: self._product_work(m, n, k, x_item=4 if kind == 1 else 2, out_item=out.element_size(), residual=kind == 2))
@@ -778,9 +773,6 @@ class HipOps:
             return self._linear_whole(x.normalised(), folded.tiles, folded.d_with(bias), act, *w.tensor.shape), None
         if folded is None:
             return None, x.materialize()
-        elif not force_tiled and act in _ACT and self._folded_beside(x, folded):
-            return self._linear_beside_norm(1, x, None, folded.tiles, folded.d_with(bias), act, self.dtype, x.shape[0],
-                                            w.tensor.shape[0], w.tensor.shape[1], alone=True), None
         elif not self._norm_in_the_product(x.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
             # the norm's kernel without weight and bias, then the plain product of the folded copy
             m, k = x.shape
@@ -1135,9 +1127,6 @@ class HipOps:
                     h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
                 elif not few:
                     h = h.materialize()
-                elif not force_tiled and self._folded_beside(h, folded):
-                    return self._qkv_beside_norm(h, folded.tiles, folded.d_with(bias), tuple(w.tensor.shape), num_heads, num_kv_write, head_size,
-                                                 scale, ctx, view, k_pages, v_pages, turn_a, turn_b, turn_pos, turn_rows, alone=True)
                 elif not self._norm_in_the_product(h.shape[0], w.tensor.shape[0], w.tensor.shape[1]):
                     # the norm's kernel without weight and bias, then the fused projection of the folded copy
                     h, w, bias = h.normalised(), PreparedWeight(w.tensor, folded.tiles), folded.d_with(bias)
@@ -1216,7 +1205,7 @@ class HipOps:
         return q
 
     def _qkv_beside_norm(self, h, tensor, bias, shape, num_heads, num_kv_write, head_size, scale, ctx, view, k_pages, v_pages, turn_a,
-                         turn_b, turn_pos, turn_rows, alone=False):
+                         turn_b, turn_pos, turn_rows):
         """Queries, keys and values of what the norm `h` gives; `tensor` the tile-ordered matrix of `shape`."""
         t, k = ctx.num_tokens, h.x.shape[1]
         total = (num_heads + 2 * num_kv_write) * head_size
@@ -1229,7 +1218,7 @@ class HipOps:
         _want(view.token_page, "token pages", torch.int32, (t,))
         _want(view.token_offset, "token offsets", torch.int32, (t,))
         q = torch.empty(t, num_heads * head_size, dtype=self.dtype, device=h.x.device)
-        how = h.as_argument(alone)
+        how = h.as_argument()
         self._call("gemm", "tnx_gemm_bf16_by_norm_qkv", ctypes.addressof(how), _ptr(tensor), _ptr(bias), t, k,
                    _ptr(view.token_page), _ptr(view.token_offset), _ptr(q), _ptr(k_pages) if num_kv_write else None,
                    _ptr(v_pages) if num_kv_write else None, float(scale), num_heads, num_kv_write, head_size, view.page_size, num_pages,
