@@ -38,12 +38,14 @@ def test_float32_product(m, n, k):
     assert bool(torch.isfinite(got[rest]).all())
 
 
-@pytest.mark.parametrize("m,n,k", [(17, 64, 32), (64, 132, 96), (65, 2048, 224), (128, 129, 1024), (180, 3072, 1024), (401, 512, 2048)])
+@pytest.mark.parametrize("m,n,k", [(17, 64, 32), (64, 132, 96), (65, 2048, 224), (128, 129, 1024), (180, 3072, 1024), (401, 512, 2048),
+                                   (401, 2048, 2048), (401, 8192, 2048), (401, 8190, 2048)])
 def test_float32_product_by_parts(m, n, k):
     """Products of more than 16 rows are made of the operands' bfloat16 parts: operands over twenty powers of two, whose lower
     parts count, and numbers that have no parts. An element's error is at most one rounding of a running sum for each 16 of K
     (h h; 16 exact products join it), one for the five other products' sums (2^-8 of the magnitudes, 5 roundings for each 16 of K),
-    what is left out (2^-26) and the shares' sum: together less than (k / 16 + 8) 2^-23 of the sum of magnitudes."""
+    what is left out (2^-24) and the shares' sum: together less than (k / 16 + 8) 2^-23 of the sum of magnitudes. (A lost part of a
+    long sum hides in that: `test_every_part_reaches_the_result` has results of one product each.)"""
     from transformers_neuronx_amd.kernels.hip import HipOps
     hip, g = HipOps(torch.float32, DEV), _gen(m + n + k)
 
@@ -66,6 +68,61 @@ def test_float32_product_by_parts(m, n, k):
     assert bool(got[2, :2].isnan().all()) and bool(got[4].isnan().all())
     assert got[3, 2].item() == x[3, 1].item() * 0.25 and got[3, 1].item() == x[3, 1].item() * -0.5
     assert bool(torch.isfinite(got[5:]).all())
+
+
+def _full(shape, g, least, most):
+    """Numbers with all 24 bits of a mantissa, from 2^least to 2^(most + 1), of either sign."""
+    bits = torch.randint(0, 1 << 23, shape, device=DEV, generator=g).double() / (1 << 23)
+    power = torch.randint(least, most + 1, shape, device=DEV, generator=g).double()
+    sign = torch.randint(0, 2, shape, device=DEV, generator=g).double() * 2 - 1
+    return (sign * (1 + bits) * torch.exp2(power)).float()
+
+
+def _by_parts(x, w, tile, shares):
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, (m, k), n = HipOps(torch.float32, DEV), x.shape, w.shape[0]
+    out, space = torch.full((m + 1, n), 7.0, device=DEV), torch.empty(shares * m * n, device=DEV)
+    hip.call("gemm", "tnx_gemm_f32_parts", x.data_ptr(), w.data_ptr(), None, None, out.data_ptr(), 0, 0, m, n, k, tile, shares,
+             space.data_ptr(), space.numel(), hip.stream())
+    assert bool((out[m] == 7).all())              # (a row behind the last stays)
+    return out[:m].double()
+
+
+def _one_a_row(m, k):
+    """A place of K for every row, over all steps of 32 and the places in them."""
+    row, steps = torch.arange(m, device=DEV), k // 32
+    return row, 32 * (row % steps) + (11 * row + row // steps) % 32
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("m,n,k,shares", [(130, 129, 32 * steps, 1) for steps in range(1, 9)] +
+                         [(17, 66, 416, 1), (65, 64, 512, 16), (257, 132, 1184, 4), (401, 260, 2048, 8), (128, 128, 2048, 1)])
+def test_every_part_reaches_the_result(m, n, k, shares, tile):
+    """One number in a row of x, so that a result is one product of two numbers of 24 bits. What is left out is 2^-24 of it
+    (l m and m l, 2^-17 and 2^-8 of the operands at most) and 2^-34 (l l), the sum of the other five parts rounds below 2^-30, and
+    that joins the h h with one rounding, 2^-24: together under 2.05 of those, on every
+    tile, at every number of steps, in every share. The smallest part made, a product of an h with an l, is up to 2^-17."""
+    g = _gen(m + n + k + tile)
+    row, place = _one_a_row(m, k)
+    x, w = torch.zeros(m, k, device=DEV), _full((n, k), g, -9, 9)
+    x[row, place] = _full((m,), g, -9, 9)
+    want = x[row, place].double()[:, None] * w[:, place].double().T
+    assert bool(((_by_parts(x, w, tile, shares) - want).abs() <= 2.05 * 2.0 ** -24 * want.abs()).all())
+
+
+@pytest.mark.parametrize("tile", [0, 1, 2])
+@pytest.mark.parametrize("least,most", [(-113, -105), (-126, -114), (-136, -127)])
+def test_operands_whose_parts_are_too_small_for_numbers(least, most, tile):
+    """Lower parts end at 2^-133, the smallest bfloat16 number: an operand under 2^-110 is off by up to half of that, no more."""
+    m, n, k = 130, 128, 256
+    g = _gen(least + tile)
+    row, place = _one_a_row(m, k)
+    x, w = torch.zeros(m, k, device=DEV), _full((n, k), g, 95, 100)
+    x[row, place] = _full((m,), g, least, most)
+    assert bool((x[row, place] != 0).all())
+    want = x[row, place].double()[:, None] * w[:, place].double().T
+    off = 2.05 * 2.0 ** -24 * want.abs() + 2.0 ** -134 * w[:, place].double().abs().T
+    assert bool(((_by_parts(x, w, tile, 1) - want).abs() <= off).all())
 
 
 @pytest.mark.parametrize("m,n,k,shares", [(17, 1024, 1024, 16), (64, 1024, 1024, 11), (31, 132, 4096, 16), (33, 2304, 768, 6), (128, 512, 4096, 16),

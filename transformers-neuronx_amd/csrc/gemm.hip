@@ -263,8 +263,11 @@ static void f32_skinny(const float* x, const float* w, const float* bias, const 
 
 // Many rows in float32, on the bfloat16 matrix instructions: every operand is the sum of three bfloat16 parts, x = h + m + l
 // with h = x rounded, m = (x - h) rounded and l the rest, which eight bits hold: nothing of x is lost. Of the nine products of
-// parts six are made, each exact, with float32 sums; l l, l m and m l, at most 2^-26 of |x w| between them, are left out. (Below
-// 2^-110 a lower part may be too small for a number: an operand is then off by 2^-133.)
+// parts six are made, each exact, with float32 sums (the scheme of Henry, Tang and Heinecke, "Leveraging the bfloat16 artificial
+// intelligence datatype for higher-precision computations", 2019); l l, l m and m l are left out: |m| is at most 2^-8 and |l| 2^-17
+// of |x|, which makes them 2^-24 of |x w| between them, as much again as a rounding of the product. A result of one product is thus
+// off by up to twice that rounding, where the float32 instructions made one; on average it is as near, and a sum of many is nearer
+// (below). Operands under 2^-110 lose more, what of a lower part is under the smallest bfloat16 number: up to 2^-134 of themselves.
 // The float32 instructions give 256 flops a cycle and unit, the bfloat16 ones 4,096, of which a sixth is 683.
 // h h has sums of its own, the other five share theirs: six times fewer roundings at the size of the result, which is why the
 // error against 64 bits is 0.34 to 0.7 of what the float32 instructions left (K 2,048: 2.7e-7 for 8.1e-7, 1,024: 1.9e-7 for 5.7e-7;
@@ -559,6 +562,27 @@ extern "C" int tnx_gemm_f32_workspace(int M, int N, int K) {
   return shares > 1 ? shares * M * N : 0;
 }
 
+// `tile` as in `choose_f32_tiles`.
+static int f32_parts(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype, int act, int M,
+                     int N, int K, int tile, int shares, float* workspace, hipStream_t stream) {
+#define F32_TILES(MI, NI, WM, WN) \
+  launch_f32_parts<MI, NI, WM, WN>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
+  return tile == 0 ? F32_TILES(1, 2, 4, 2) : tile == 1 ? F32_TILES(1, 1, 2, 4) : F32_TILES(1, 1, 2, 2);
+#undef F32_TILES
+}
+
+// The product by parts with a tile and shares of the caller's (`tnx_gemm_f32` chooses them).
+extern "C" int tnx_gemm_f32_parts(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
+                                  int act, int M, int N, int K, int tile, int shares, float* workspace, size_t workspace_floats,
+                                  hipStream_t stream) {
+  TNX_REQUIRE(M > 0 && N > 0 && K > 0 && K % 32 == 0 && K < 1 << 22 && ((uintptr_t)x | (uintptr_t)w | (uintptr_t)workspace) % 16 == 0,
+              "gemm_f32_parts: K in 32s below 2^22 and operands 16-byte aligned, got M=%d N=%d K=%d", M, N, K);
+  TNX_REQUIRE(tile >= 0 && tile <= 2 && shares >= 1 && shares <= 16 && shares <= K / 32, "gemm_f32_parts: tile 0 to 2, up to 16 shares");
+  TNX_REQUIRE(shares == 1 || (N % 4 == 0 && workspace && workspace_floats >= (size_t)shares * M * N),
+              "gemm_f32_parts: shares want N a multiple of 4 and a workspace of shares x M x N floats");
+  return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, stream);
+}
+
 // `workspace`: as many floats as `tnx_gemm_f32_workspace` names for the sizes; with less, K is not shared out.
 extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, const float* residual, void* out,
                             int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
@@ -574,10 +598,7 @@ extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, c
     int tile = 0, shares = 1;
     choose_f32_tiles(M, N, K, tile, shares);
     if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
-#define F32_TILES(MI, NI, WM, WN) \
-  launch_f32_parts<MI, NI, WM, WN>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
-    return tile == 0 ? F32_TILES(1, 2, 4, 2) : tile == 1 ? F32_TILES(1, 1, 2, 4) : F32_TILES(1, 1, 2, 2);
-#undef F32_TILES
+    return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, stream);
   }
   dim3 grid((N + F32_TILE - 1) / F32_TILE, (M + F32_TILE - 1) / F32_TILE);
   TNX_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d is too large", M);

@@ -39,6 +39,8 @@ _SIGNATURES = {
     "gemm": {
         "tnx_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                          _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
+        "tnx_gemm_f32_parts": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
+                               _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
         "tnx_gemm_f32_workspace": [_c_int, _c_int, _c_int],
         "tnx_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_void_p],
