@@ -146,3 +146,24 @@ def test_rows_and_vectors_that_no_norm_takes(m, k):
         for make in (lambda: hip.layernorm_deferred(rows, vector, None, 1e-5, dt), lambda: hip.norm_between(rows, vector, None, 1e-5, dt)[1]):
             with pytest.raises(error):
                 hip.linear(make(), w)
+
+
+@pytest.mark.parametrize("m,k,n,beside", [(8, 3072, 12288, True), (1, 3072, 12304, False), (4, 2048, 40960, True), (5, 2048, 16384, True),
+                                          (5, 2048, 16400, False), (8, 1024, 40960, True)])
+def test_very_many_columns_read_the_norms_kernel(m, k, n, beside):
+    """The line at 256 units, for norms before a matrix and behind a sum; the results are of one norm either way."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g, dt = HipOps(torch.bfloat16, DEV), _gen(m + k + n), torch.bfloat16
+    hip.compute_units = 256
+    t, gamma = torch.randn(m, k, device=DEV, generator=g) * 3 + 1, 1 + 0.1 * torch.randn(k, device=DEV, generator=g)
+    w = hip.prepare_weight((torch.randn(n, k, device=DEV, generator=g) * 0.05).to(dt))
+    assert hip.defer_norm(w, gamma, None)
+    want = _normed(t, gamma, None, 1e-5, True) @ w.tensor.double().T
+    way, made = [], hip._linear_beside_norm
+    hip._linear_beside_norm = lambda *a: way.append(a) or made(*a)
+    d = hip.layernorm_deferred(t, gamma, None, 1e-5, dt)
+    # (independent roundings to bfloat16: the operand's and the result's)
+    assert (hip.linear(d, w).double() - want).norm() <= 2.0 * 2.0 ** -9 * want.norm() and bool(way) == beside
+    if k <= hip.norm_between_width:
+        d = hip.norm_between(t, gamma, None, 1e-5, dt)[0]
+        assert (hip.linear(d, w, out_f32=True).double() - want).norm() <= 2.0 ** -9 * 1.5 * want.norm() and (d.done is None) == beside

@@ -98,7 +98,7 @@ def _run(ops, mixer, ff, norm=LayerNorm, arrangement=PostNormBlock, layers=2):
                                                       ".bias": torch.randn(WIDTH, generator=g)}) for n in norms]:
             part.load(t, "", ops, torch.float32)
         block = arrangement(m, f, *norms)
-        block.load({}, "", ops, torch.float32) if hasattr(block, "load") else None
+        block.load({}, "", ops, torch.float32)
         block.after_load()
         blocks.append(block)
         if not block.norms_between:

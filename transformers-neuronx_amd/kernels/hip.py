@@ -645,6 +645,13 @@ class HipOps:
         return (self.norm_beside and self.dtype == torch.bfloat16 and 0 < rows <= self.norm_beside_rows and width % 128 == 0
                 and width <= most and not debug.tapping())
 
+    def _beside_columns(self, rows, width, n) -> bool:
+        """Every block makes the norm again, and the blocks of very many columns come several to a unit, one after another. Norm's
+        kernel and product / so, us, 256 units, 8 rows: width 3,072 and 12,288 columns 19.9 / 19.2, 16,384 24.9 / 26.7, 40,960 51.0 / 59.2;
+        2,048 and 16,384 19.2 / 17.8, 20,480 24.5 / 24.7 (5 rows 22.9 / 24.3, 4 rows 22.7 / 21.8); 1,024 and 40,960 25.8 / 23.4."""
+        tile = 16 * self.compute_units
+        return n <= 3 * tile or width <= 1024 or (width <= 2048 and (rows <= 4 or n <= 4 * tile))
+
     @staticmethod
     def _want_norm(x, weight, bias):
         """As `layernorm` wants them: a product that makes the norm is handed their addresses."""
@@ -668,7 +675,8 @@ class HipOps:
 
     def _beside_weight(self, w, m, norm):
         """The tile-ordered matrix that the products next to a norm read, or None where they do not take the sizes."""
-        if norm.done is not None or not self._norm_beside(m, norm.x.shape[1], self.norm_between_width) or not isinstance(w, PreparedWeight) or w.tiles is None:
+        if (norm.done is not None or not self._norm_beside(m, norm.x.shape[1], self.norm_between_width) or not isinstance(w, PreparedWeight)
+                or w.tiles is None or not self._beside_columns(m, norm.x.shape[1], w.tensor.shape[0])):
             return None
         return None if any((_ptr(a) or 0) % 16 for a in (w.tiles, norm.x, norm.weight, norm.bias)) else w.tiles
 
@@ -691,7 +699,7 @@ class HipOps:
         """The norm `h` is the one before `w`, and the product of `w`'s own tile-ordered copy makes it."""
         return (isinstance(w, PreparedWeight) and w.tiles is not None and w.norm_before is not None and w.norm_before == h.key
                 and w.tensor.shape[1] == h.x.shape[1]
-                and self._norm_beside(*h.x.shape, self.norm_operand_width)
+                and self._norm_beside(*h.x.shape, self.norm_operand_width) and self._beside_columns(*h.x.shape, w.tensor.shape[0])
                 and all((_ptr(a) or 0) % 16 == 0 for a in (w.tiles, h.x, h.weight, h.bias)))
 
     def _linear_beside_norm(self, kind, norm, x, t, bias, act, out_dtype, m, n, k):
