@@ -77,6 +77,7 @@ class DecoderModel:
                 self.part_state_needs[nxt] = need
                 nxt += 1
         self.loaded = False
+        self.layers_in_one: Dict[int, int] = {}       # runs of calls that are one launch in decode steps of few rows
         parts = [self.embedding, self.embedding.position, self.head] + ([self.head.norm] if self.head.norm else [])
         for l in self.layers:
             parts += [l.block, l.mixer, l.feed_forward, l.mixer_norm, l.feed_forward_norm]
@@ -157,11 +158,14 @@ class DecoderModel:
         self.ops, self.dtype, self.device = ops, dtype, device
         self.weight_bytes = sum(t.numel() * t.element_size() for t in {id(t): t for t in tensors.values()}.values())
         self.loaded = True
+        if finish:
+            self.layers_in_one = self._layers_in_one() if hasattr(ops, "layers_most") else {}
         return self
 
     def finish_load(self) -> None:
         for layer in self.layers:
             layer.block.after_load()
+        self.layers_in_one = self._layers_in_one() if hasattr(self.ops, "layers_most") else {}
 
     # ---------------------------------------------------------------- one step
 
@@ -175,7 +179,17 @@ class DecoderModel:
         debug.tap("embedding", stream.x)
         # in steps of few rows, what the last block left may be a norm that the next products do (`norms_between`)
         few, between = ctx.num_tokens <= getattr(self.ops, "norm_beside_rows", 0), False
+        in_one = self.layers_in_one if ctx.num_tokens <= getattr(self.ops, "layer_rows", 0) and self.ops.layers_fit(ctx) else {}
+        done = 0
         for call, (layer, cid, writes) in enumerate(self.schedule):
+            if call < done:
+                continue
+            if call in in_one:
+                behind = self._run_in_one(stream, call, in_one[call], ctx, caches)
+                if behind is not None:
+                    stream, done = behind, in_one[call]
+                    between = few and getattr(self.layers[self.schedule[done - 1][0]].block, "norms_between", False)
+                    continue
             cache = caches[cid] if writes else caches[cid].reader()
             state_id = self.call_state_ids[call]
             ctx.call_state = caches[state_id] if state_id is not None else None
@@ -192,6 +206,34 @@ class DecoderModel:
             stream = Stream(self.ops.hyper_sum(stream.copies, stream.pending))
         return debug.tap("logits", self.head.forward(stream, ctx))
 
+
+    def _layers_in_one(self) -> Dict[int, int]:
+        """{first call: the call behind the last} of the runs of calls whose blocks can be one launch (`Block.in_one`)."""
+        out, call, n = {}, 0, len(self.schedule)
+        layers = [self.layers[layer] for layer, _, _ in self.schedule]
+
+        def joins(call, end):
+            first, before, this = layers[call], layers[end - 1], layers[end]
+            return (type(this.block) is type(first.block) and this.mixer.cache_need().group_key() == first.mixer.cache_need().group_key()
+                    and self.ops.layers_alike(first.block, this.block, before.block))
+        while call < n:
+            end = call
+            while (end < n and end - call < self.ops.layers_most and layers[end].block.in_one is not None and self.schedule[end][2]
+                   and (end == call or joins(call, end))):
+                end += 1
+            if end > call:
+                out[call] = end
+            call = max(end, call + 1)
+        return out
+
+    def _run_in_one(self, stream: Stream, begin: int, end: int, ctx, caches):
+        """The stream behind the calls from `begin` to `end`, run as one launch; None where the backend does not take the step."""
+        blocks = [self.layers[layer].block for layer, _, _ in self.schedule[begin:end]]
+        of_calls = [caches[cid] for _, cid, _ in self.schedule[begin:end]]
+        x, first, residual_normed = blocks[0].into_one(stream)
+        norms = [(first, blocks[0].norms_in_one(blocks[0])[1])] + [b.norms_in_one(before) for before, b in zip(blocks, blocks[1:])]
+        y = self.ops.decode_layers([b.in_one for b in blocks], x, norms, residual_normed, ctx, ctx.groups[of_calls[0].group], of_calls)
+        return None if y is None else blocks[-1].out_of_one(y)
 
     def _settled(self, stream: Stream) -> Stream:
         x = self.ops.settled(stream.x)

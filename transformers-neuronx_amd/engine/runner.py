@@ -106,6 +106,7 @@ class ModelRunner:
         self.kept_tokens = torch.zeros(cache.max_seqs, dtype=torch.int32, device=model.device)
         self._last_ctx: Optional[StepContext] = None
         self._staging = _Staging(ops) if hasattr(ops, "pinned_ints") else None
+        self._raise_if_lost = getattr(ops, "raise_if_lost", None)
         # steps written to a folder for running them again alone (`engine/snapshot.py`); None: none are
         self.snapshots = snapshots_from_environment()
 
@@ -175,6 +176,8 @@ class ModelRunner:
         their `want`; None when nothing is wanted (the step still runs)."""
         if not entries:
             return None
+        if self._raise_if_lost is not None:
+            self._raise_if_lost()
         taking = self.snapshots is not None and self.snapshots.wanted()
         recordable = (self.use_graphs and not debug.active() and not taking
                       and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries))

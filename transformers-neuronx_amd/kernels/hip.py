@@ -216,6 +216,10 @@ _SIGNATURES = {
         "tnx_gated_norm": [_c_void_p, _c_void_p, _c_ll, _c_void_p, _c_float, _c_int, _c_int, _c_void_p, _c_int, _c_void_p,
                            _c_ll, _c_void_p, _c_ll, _c_float, _c_int, _c_int, _c_int, _c_void_p],
     },
+    "layer": {
+        "tnx_decode_layer_words": [_c_int, _c_int, _c_int, _c_int],
+        "tnx_decode_layers": [_c_void_p, _c_int, _c_void_p],
+    },
     "probe": {
         "tnx_probe_stream_read": [_c_void_p, ctypes.c_size_t, _c_void_p, _c_int, _c_void_p],
         "tnx_probe_mfma_loop": [_c_int, _c_int, _c_void_p, _c_void_p],
@@ -343,6 +347,35 @@ class NormBetween(DeferredNorm):
         raise TypeError("a norm behind a sum is folded into no product")
 
 
+class _LayerOf(ctypes.Structure):
+    """What a layer has of its own for `tnx_decode_layers` (`LayerOf` in layer.hip)."""
+    _fields_ = [(n, _c_void_p) for n in ("w_qkv", "w_out", "w_up", "w_down", "b_qkv", "b_out", "b_up", "b_down", "first_weight", "first_bias",
+                                         "second_weight", "second_bias", "k_pages", "v_pages")]
+
+
+LAYERS_MOST = 30        # of one launch: its arguments are 4 KB at most
+
+
+class _Layers(ctypes.Structure):
+    """The arguments of `tnx_decode_layers` (`Layers` in layer.hip)."""
+    _fields_ = ([(n, _c_void_p) for n in ("x", "out", "token_page", "token_off", "cached_lens", "table", "words", "failed")]
+                + [("at", _c_int * 7), ("scale", _c_float), ("eps", _c_float)]
+                + [(n, _c_int) for n in ("rows", "width", "inner_width", "act", "center", "residual_normed", "first_normed", "table_width",
+                                         "page_shift", "num_pages", "page_pad", "splits", "chunk", "layers", "blocks")]
+                + [("of", _LayerOf * LAYERS_MOST)])
+
+
+class LayerParts:
+    """A layer as `HipOps.decode_layers` runs it, from what its parts say of themselves: softmax attention with a head for every
+    query and as many for keys and values, a feed-forward of two products, a norm before each or behind each sum."""
+
+    __slots__ = ("w_qkv", "b_qkv", "w_out", "b_out", "heads", "scale", "w_up", "b_up", "act", "w_down", "b_down")
+
+    def __init__(self, attention, feed_forward):
+        self.w_qkv, self.b_qkv, self.w_out, self.b_out, self.heads, self.scale = attention
+        self.w_up, self.b_up, self.act, self.w_down, self.b_down = feed_forward
+
+
 def tile_order(w: torch.Tensor) -> torch.Tensor:
     """`w[n, k]` -> `[n/16][k/128][s][r][g][e]` with n = 16*nt + r and k = 128*kt + 32*s + 8*g + e."""
     n, k = w.shape
@@ -413,6 +446,7 @@ class HipOps:
         self._tiles_per_block = {}
         self._tiles_rooms = {}
         self._landing, self._landing_turn = [None, None], 0
+        self._lost = self._ones_zeros = None
         self._ints, self._ints_done, self._ints_turn = [None, None], [None, None], 0
 
     def _call(self, module: str, fn: str, *args, work=None):
@@ -1452,6 +1486,116 @@ class HipOps:
         blocks = self._decode_blocks(num_heads, num_kv_heads or num_heads, head_size)
         return ("decode", blocks, head_size) + self._splits_for(step.length_bound, fills, alike, n_dec * blocks,
                                                                 int(window or 0), head_size)
+
+    # ---------------------------------------------------------------- layers in one launch
+
+    # Decode steps of so few rows run layers of so many columns as one launch, as many as its arguments hold (`layer.hip`). us a layer,
+    # launches apart / in one: bfloat16, 1 request of 100 tokens, 1,024 columns 23.1 / 17.0, 512 18.9 / 16.0; 8 of 2,000 41.9 / 36.6; float32, 3
+    # of 70, 1,024 34.4 / 26.8, 768 32.7 / 27.9, 512 24.6 / 22.2, but 256 19.4 / 21.0: what is handed on between blocks takes as long as
+    # launches there. 2,048 columns 37.4 / 43.6: half of the units do not bring 100 MB of weights as quickly as all of them.
+    layer_in_one = True
+    layer_rows = 8
+    layer_widths, layer_inner = (512, 1024), 4096
+    layers_most = LAYERS_MOST
+
+    def layer_parts(self, attention, feed_forward):
+        """Asked once when a layer has its tensors: what `decode_layers` takes for it, or None where the layer is none of its
+        kind. `attention` = (w_qkv, b_qkv, w_out, b_out, heads, scale), `feed_forward` = (w_up, b_up, act, w_down, b_down)."""
+        p = LayerParts(attention, feed_forward)
+        weights = (p.w_qkv, p.w_out, p.w_up, p.w_down)
+        if not all(isinstance(w, PreparedWeight) and w.tensor.dtype == self.dtype and w.inner == w.tensor.shape[1] for w in weights):
+            return None
+        width, inner = p.w_qkv.shape[1], p.w_up.shape[0]
+        fits = (p.act in _ACT and width == 64 * p.heads and width % 128 == 0 and self.layer_widths[0] <= width <= self.layer_widths[1] and inner % 128 == 0 and inner <= self.layer_inner
+                and tuple(p.w_qkv.shape) == (3 * width, width) and tuple(p.w_out.shape) == (width, width)
+                and tuple(p.w_up.shape) == (inner, width) and tuple(p.w_down.shape) == (width, inner))
+        return p if fits else None
+
+    def layers_fit(self, ctx) -> bool:
+        """Whether a step is one that `decode_layers` runs: few rows, one token a request."""
+        return self.layer_in_one and ctx.num_tokens <= self.layer_rows and ctx.num_tokens == ctx.num_requests and not debug.tapping()
+
+    @staticmethod
+    def layers_alike(first, block, before) -> bool:
+        """Whether `block`, behind `before`, goes into one launch with `first`: sizes, activation, scale and norms of one kind."""
+        a, b = first.in_one, block.in_one
+        norms = [n for n in first.norms_in_one(first) + block.norms_in_one(before)]
+        return (a.w_qkv.shape == b.w_qkv.shape and a.w_up.shape == b.w_up.shape and (a.act, a.scale) == (b.act, b.scale)
+                and all(n[2:] == norms[0][2:] for n in norms))
+
+    def _layer_weights(self, p):
+        """The four matrices as the launch reads them, or None where one has no such copy."""
+        of = [(w.tiles if self.dtype == torch.bfloat16 else w.tensor) for w in (p.w_qkv, p.w_out, p.w_up, p.w_down)]
+        return None if any(t is None or _ptr(t) % 16 for t in of) else of
+
+    def decode_layers(self, layers, x, norms, residual_normed, ctx, view, caches):
+        """Consecutive layers (`layer_parts`, alike) over a step that `layers_fit`, in one launch; None where something about it is
+        not as the launch wants it. `x` float32; `norms`: for every layer (weight, bias, center, eps) of what its two halves read,
+        the first layer's first None where that is `x` itself; `residual_normed`: the sums are made with the normed rows; `caches`:
+        the layers' `LayerCache`s, of one group. Returns the float32 sum behind the last feed-forward."""
+        t, p = ctx.num_tokens, layers[0]
+        if not (self.layers_fit(ctx) and view.page_size >= 64 and view.page_size & (view.page_size - 1) == 0):
+            return None
+        width, inner = p.w_qkv.shape[1], p.w_up.shape[0]
+        if any(n is not None and n[2:] != norms[0][1][2:] for pair in norms for n in pair):
+            return None
+        _want(x, "x", torch.float32, (t, width))
+        args = _Layers()
+        if self._ones_zeros is None:
+            self._ones_zeros = torch.ones(4096, dtype=torch.float32, device=self.device), torch.zeros(4096, dtype=torch.float32, device=self.device)
+        ones, zeros = self._ones_zeros
+        num_pages, pad = 0, self._page_pad(caches[0].k_pages, p.heads, 64, view.page_size)
+        for at, (of, p, (first, second), cache) in enumerate(zip(args.of, layers, norms, caches)):
+            weights = self._layer_weights(p)
+            vectors = [*(first[:2] if first is not None else (None, None)), *second[:2]]
+            if weights is None or any((_ptr(a) or 0) % 16 for a in (x, cache.k_pages, cache.v_pages, p.b_qkv, p.b_out, p.b_up, p.b_down, *vectors)):
+                return None
+            for v, name, n in ((p.b_qkv, "qkv bias", 3 * width), (p.b_out, "bias", width), (p.b_up, "bias", inner), (p.b_down, "bias", width),
+                               *((v, "norm vector", width) for v in vectors)):
+                if v is not None:
+                    _want(v, name, torch.float32, (n,))
+            pages = self._check_pages(cache.k_pages, cache.v_pages, p.heads, 64, view.page_size)
+            if (at and pages != num_pages) or self._page_pad(cache.k_pages, p.heads, 64, view.page_size) != pad:
+                return None
+            num_pages = pages
+            (of.w_qkv, of.w_out, of.w_up, of.w_down, of.b_qkv, of.b_out, of.b_up, of.b_down, of.first_weight, of.first_bias, of.second_weight,
+             of.second_bias, of.k_pages, of.v_pages) = (_ptr(a) for a in (
+                 *weights, *(zeros if v is None else v for v in (p.b_qkv, p.b_out, p.b_up, p.b_down)),
+                 *(plain if v is None else v for v, plain in zip(vectors, (ones, zeros, ones, zeros))), cache.k_pages, cache.v_pages))
+        _want(view.block_table, "block table", torch.int32, (ctx.num_requests, view.width))
+        _want(view.token_page, "token pages", torch.int32, (t,))
+        _want(view.token_offset, "token offsets", torch.int32, (t,))
+        if ctx.max_total > view.width * view.page_size:
+            raise ValueError("a request is longer than its block table")
+        out = torch.empty_like(x)
+        # the places of the handoffs, marked as empty (by a launch of its own: whatever came before, they are)
+        words = torch.full((len(layers) * library("layer").tnx_decode_layer_words(_code(self.dtype), t, width, inner),), -1, dtype=torch.int32,
+                           device=x.device)
+        if self._lost is None:
+            self._lost = self.pinned_ints(1)
+            self._lost[0].zero_()
+        args.x, args.out, args.words, args.failed = _ptr(x), _ptr(out), _ptr(words), self._lost[1].value
+        args.token_page, args.token_off, args.cached_lens, args.table = (_ptr(a) for a in (view.token_page, view.token_offset, ctx.cached_lens,
+                                                                                          view.block_table))
+        args.scale, args.eps, args.center = float(p.scale), float(norms[0][1][3]), int(bool(norms[0][1][2]))
+        args.rows, args.width, args.inner_width, args.act, args.layers = t, width, inner, _ACT[p.act], len(layers)
+        args.residual_normed, args.first_normed = int(bool(residual_normed)), int(norms[0][0] is not None)
+        args.table_width, args.page_shift, args.num_pages, args.page_pad = view.width, view.page_size.bit_length() - 1, num_pages, pad
+
+        def work():
+            item = 2 if self.dtype == torch.bfloat16 else 4
+            n = width * (4 * width + 2 * inner)
+            keys = float(ctx.cached_lens_host.sum())
+            return (f"{len(layers)} layers {t}x{width}x{inner}", len(layers) * (n * item + keys * 2 * width * item) + 8 * t * width,
+                    len(layers) * (2.0 * t * n + 4.0 * keys * width))
+        self._call("layer", "tnx_decode_layers", ctypes.addressof(args), _code(self.dtype), _stream(), work=work)
+        return out
+
+    def raise_if_lost(self) -> None:
+        """A wait inside a launch that went on without an answer has left results that are no numbers: said here, by the host's
+        next step."""
+        if self._lost is not None and int(self._lost[0][0]):
+            raise RuntimeError("a layer's launch waited in vain for blocks of its own that were not run beside it; its step's results are void")
 
     # ---------------------------------------------------------------- parts of other designs
 

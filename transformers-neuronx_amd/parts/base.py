@@ -179,6 +179,12 @@ class Mixer(Part):
         what `Norm.deferred` returns and let the product apply the norm."""
         return None
 
+    def layer_form(self):
+        """What a backend that runs a whole layer in one launch takes of this part, where its `forward` is that and nothing else:
+        for a mixer (w_qkv, b_qkv, w_out, b_out, heads, scale) of softmax attention over all keys of a request, heads of 64 with
+        keys and values of their own; for a feed-forward (w_up, b_up, activation, w_down, b_down). None otherwise."""
+        return None
+
 
 class FeedForward(Part):
     """forward(h, ctx, residual) -> float32 `[T, hidden]`: residual + f(h), token by token."""
@@ -188,6 +194,10 @@ class FeedForward(Part):
 
     def first_weight(self):
         """As `Mixer.first_weight`."""
+        return None
+
+    def layer_form(self):
+        """As `Mixer.layer_form`."""
         return None
 
 
@@ -252,6 +262,23 @@ class Block(Part):
         """Tensors of the arrangement itself (norms after a part, a convolution before it, ...), named from the
         layer's prefix. The four parts declare their own."""
         return []
+
+    # Where the backend can run this layer and its neighbours of the same kind as one launch in decode steps of few rows: what it
+    # takes for it (`ops.layer_parts`), known once the parts have their tensors. The arrangement then says what goes in and out.
+    in_one = None
+
+    def norms_in_one(self, before):
+        """`Norm.fused_form` of what the layer's two halves read, where `before` is the block of the layer before in that launch."""
+        raise NotImplementedError
+
+    def into_one(self, stream):
+        """For the first layer of a launch: (float32 rows, the norm of what its first half reads or None where that is the rows
+        themselves, whether the sums are made with the normed rows)."""
+        raise NotImplementedError
+
+    def out_of_one(self, y):
+        """The stream behind the last one, from its float32 sum."""
+        return Stream(y, None)
 
     def after_load(self) -> None:
         """Called when the four parts have their tensors."""

@@ -3,6 +3,25 @@ from .. import debug
 from .base import Block, Stream, joined_rows, register_block
 
 
+def _is_its_fused_form(norm) -> bool:
+    """Whether a norm's `forward` is what its `fused_form` says: one class has both (a subclass that changes one of them alone
+    is run, not formed again)."""
+    def owner(name):
+        return next((c for c in type(norm).__mro__ if name in vars(c)), None)
+    return owner("fused_form") is not None and owner("forward") is owner("fused_form")
+
+
+def _layer_parts(block, kind):
+    """What the backend takes to run the layer as part of a launch of several (`Block.in_one`), or None: an arrangement of its own
+    (a subclass with another `forward`), and parts and norms that say nothing of themselves, are run part by part."""
+    ops = block.mixer_norm.ops
+    if (type(block).forward is not kind.forward or not hasattr(ops, "layer_parts")
+            or not all(_is_its_fused_form(n) for n in (block.mixer_norm, block.feed_forward_norm))):
+        return None
+    attention, feed_forward = block.mixer.layer_form(), block.feed_forward.layer_form()
+    return ops.layer_parts(attention, feed_forward) if attention is not None and feed_forward is not None else None
+
+
 @register_block("pre_norm")
 class PreNormBlock(Block):
     """`x = x + mixer(norm(x))`, `x = x + feed_forward(norm(x))`
@@ -24,6 +43,13 @@ class PreNormBlock(Block):
         self.fold_feed_forward_norm = w is not None and self.feed_forward_norm.fold_into(w)
         self.mixer_norm_rows = self.mixer_norm.defer_rows if self.fold_mixer_norm else -1
         self.feed_forward_norm_rows = self.feed_forward_norm.defer_rows if self.fold_feed_forward_norm else -1
+        self.in_one = _layer_parts(self, PreNormBlock)
+
+    def norms_in_one(self, before):
+        return self.mixer_norm.fused_form(), self.feed_forward_norm.fused_form()
+
+    def into_one(self, stream):
+        return stream.x, self.mixer_norm.fused_form(), False
 
     def forward(self, stream: Stream, ctx, cache) -> Stream:
         h = (self.mixer_norm.deferred(stream.x) if ctx.num_tokens <= self.mixer_norm_rows
@@ -33,14 +59,6 @@ class PreNormBlock(Block):
              else self.feed_forward_norm.forward(x, False, True)[1])
         x = self.feed_forward.forward(h, ctx, x)
         return Stream(x, None)
-
-
-def _is_its_fused_form(norm) -> bool:
-    """Whether a norm's `forward` is what its `fused_form` says: one class has both (a subclass that changes one of them alone
-    is run, not formed again)."""
-    def owner(name):
-        return next((c for c in type(norm).__mro__ if name in vars(c)), None)
-    return owner("fused_form") is not None and owner("forward") is owner("fused_form")
 
 
 @register_block("post_norm")
@@ -68,6 +86,19 @@ class PostNormBlock(Block):
                               and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
                               and all(_is_its_fused_form(n) for n in norms))
         self.between_rows = self.mixer_norm.ops.norm_beside_rows if self.norms_between else -1
+        self.in_one = _layer_parts(self, PostNormBlock) if self.norms_between else None
+
+    def norms_in_one(self, before):
+        return before.feed_forward_norm.fused_form(), self.mixer_norm.fused_form()
+
+    def into_one(self, stream):
+        x = stream.x
+        if hasattr(x, "settled") and x.done is None:         # the norm behind the sum before, which has not been made
+            return x.x, (x.weight, x.bias, x.center, x.eps), True
+        return self.mixer_norm.ops.settled(x), None, True
+
+    def out_of_one(self, y):
+        return Stream(*self._between(self.feed_forward_norm, y))
 
     def _between(self, norm, x):
         weight, bias, center, eps = norm.fused_form()

@@ -48,6 +48,11 @@ class DenseFeedForward(FeedForward):
     def first_weight(self):
         return self.w1
 
+    def layer_form(self):
+        if type(self).forward is not DenseFeedForward.forward or self.activation == "poly_norm":
+            return None
+        return self.w1, self.b1, self.activation, self.w2, self.b2
+
     @residual_to_product
     def forward(self, h, ctx, residual):
         """`residual` None: f(h) alone, in float32 (for an arrangement that norms it before the sum)."""

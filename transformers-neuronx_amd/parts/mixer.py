@@ -238,6 +238,12 @@ class Attention(OffersRows, Mixer):
     def first_weight(self):
         return None if self.prepared else self.w_in
 
+    def layer_form(self):
+        if (type(self).forward is not Attention.forward or self.prepared or not self.own_kv or self.rotation is not None
+                or self.window is not None or self.defer_out or self.defer_in or self.num_kv_heads != self.num_heads or self.head_size != 64):
+            return None
+        return self.w_in, self.b_in, self.w_out, self.b_out, self.num_heads, self.scale
+
     @property
     def w_qkv(self):
         return self.w_in
