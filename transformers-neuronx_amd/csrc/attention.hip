@@ -40,60 +40,70 @@ __device__ __forceinline__ void store8<bf16_t>(bf16_t* p, const float* v) {
 }
 
 template <typename T>
-__global__ void __launch_bounds__(256)
-qkv_write_kernel(const T* __restrict__ qkv, const float* __restrict__ bias, float scale,
-                 const int* __restrict__ positions, const int* __restrict__ token_request,
-                 const int* __restrict__ table, int table_width, int page_size, int num_pages, T* __restrict__ q_out,
-                 T* __restrict__ k_pages, T* __restrict__ v_pages, int num_heads, int num_kv, int head_size,
-                 const int* __restrict__ run_start, int values_of_single_tokens_only,
-                 const float* __restrict__ turn_a, const float* __restrict__ turn_b, int turn_rows, int page_pad) {
-  const size_t page_stride = (size_t)num_kv * page_size * head_size + page_pad;     // elements from page to page
-  const int t = blockIdx.x;
+struct QkvPlaces {
+  const T* qkv;
+  const float* bias;
+  float scale;
+  const int *positions, *token_request, *table;
+  int table_width, page_size, num_pages;
+  T *q_out, *k_pages, *v_pages;
+  int num_heads, num_kv, head_size;
+  const int *run_start, *cached_lens;
+  const float *turn_a, *turn_b;
+  int turn_rows, page_pad;
+  const int *tile_run, *tile_q0;
+};
+
+// Eight elements of token `t`, part `part` of its row.
+template <typename T, bool VALUES_OF_SINGLE_TOKENS_ONLY>
+__device__ __forceinline__ void write_token(const QkvPlaces<T>& a, int t, int part) {
+  const int num_heads = a.num_heads, num_kv = a.num_kv, head_size = a.head_size, page_size = a.page_size;
+  const size_t page_stride = (size_t)num_kv * page_size * head_size + a.page_pad;     // elements from page to page
   const int nq = num_heads * head_size, nk = num_kv * head_size;
   const int total = nq + 2 * nk;
-  const int i0 = (blockIdx.y * 256 + threadIdx.x) * 8;
+  const int i0 = (part * 256 + threadIdx.x) * 8;
   if (i0 >= total) return;
-  if (values_of_single_tokens_only && i0 >= nq + nk) {   // the values of longer runs are written by tiles
-    const int r = token_request[t];
-    if (run_start[r + 1] - run_start[r] > 1) return;
+  if (VALUES_OF_SINGLE_TOKENS_ONLY && i0 >= nq + nk) {   // the values of longer runs are written by tiles
+    const int r = a.token_request[t];
+    if (a.run_start[r + 1] - a.run_start[r] > 1) return;
   }
   float v[8];
-  load8<T>(qkv + (size_t)t * total + i0, v);
-  if (bias) {
-    const f32x4 b0 = *(const f32x4*)(bias + i0), b1 = *(const f32x4*)(bias + i0 + 4);
+  load8<T>(a.qkv + (size_t)t * total + i0, v);
+  if (a.bias) {
+    const f32x4 b0 = *(const f32x4*)(a.bias + i0), b1 = *(const f32x4*)(a.bias + i0 + 4);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
       v[j] += b0[j];
       v[4 + j] += b1[j];
     }
   }
-  if (turn_a && i0 < nq + nk) {
+  if (a.turn_a && i0 < nq + nk) {
     // a position encoding that turns queries and keys pair by pair: x[d] becomes a[p][d] x[d] + b[p][d] x[d ^ 1]
     // (the eight elements of a thread lie in one head: head sizes are multiples of 8)
-    const size_t at = (size_t)min(max(positions[t], 0), turn_rows - 1) * head_size + i0 % head_size;
+    const size_t at = (size_t)min(max(a.positions[t], 0), a.turn_rows - 1) * head_size + i0 % head_size;
     float w[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) w[j] = turn_a[at + j] * v[j] + turn_b[at + j] * v[j ^ 1];
+    for (int j = 0; j < 8; ++j) w[j] = a.turn_a[at + j] * v[j] + a.turn_b[at + j] * v[j ^ 1];
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[j] = w[j];
   }
   if (i0 < nq) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) v[j] *= scale;
-    store8<T>(q_out + (size_t)t * nq + i0, v);
+    for (int j = 0; j < 8; ++j) v[j] *= a.scale;
+    store8<T>(a.q_out + (size_t)t * nq + i0, v);
     return;
   }
-  const int pos = positions[t];
+  const int pos = a.positions[t];
   const int blk = pos / page_size, off = pos % page_size;
   int page = -1;
-  if (blk < table_width) page = table[token_request[t] * table_width + blk];
-  if (page < 0 || page >= num_pages) return;
+  if (blk < a.table_width) page = a.table[a.token_request[t] * a.table_width + blk];
+  if (page < 0 || page >= a.num_pages) return;
   if (i0 < nq + nk) {
     const int j0 = i0 - nq, h = j0 / head_size, d = j0 % head_size;
-    store8<T>(k_pages + (size_t)page * page_stride + ((size_t)h * page_size + off) * head_size + d, v);
+    store8<T>(a.k_pages + (size_t)page * page_stride + ((size_t)h * page_size + off) * head_size + d, v);
   } else {
     const int j0 = i0 - nq - nk, h = j0 / head_size, d = j0 % head_size;
-    T* dst = v_pages + (size_t)page * page_stride + ((size_t)h * head_size + d) * page_size + off;
+    T* dst = a.v_pages + (size_t)page * page_stride + ((size_t)h * head_size + d) * page_size + off;
 #pragma unroll
     for (int j = 0; j < 8; ++j) dst[(size_t)j * page_size] = from_f32<T>(v[j]);
   }
@@ -107,20 +117,16 @@ qkv_write_kernel(const T* __restrict__ qkv, const float* __restrict__ bias, floa
 // to the tile; a group that the tile covers in part is written element by element.
 constexpr int VT_TOKENS = 128;
 
-__global__ void __launch_bounds__(256)
-value_tiles_kernel(const bf16_t* __restrict__ qkv, const float* __restrict__ bias, const int* __restrict__ run_start,
-                   const int* __restrict__ cached_lens, const int* __restrict__ table, int table_width,
-                   int page_size, int num_pages, const int* __restrict__ tile_run,
-                   const int* __restrict__ tile_q0, bf16_t* __restrict__ v_pages, int num_heads, int num_kv,
-                   int head_size, int page_pad) {
-  const size_t page_stride = (size_t)num_kv * page_size * head_size + page_pad;
-  const int run = tile_run[blockIdx.x], q0 = tile_q0[blockIdx.x], kvh = blockIdx.y;
-  const int t0 = run_start[run] + q0;
-  const int n = min(VT_TOKENS, run_start[run + 1] - t0);
-  const int p0 = cached_lens[run] + q0;   // position of the tile's first token
+__device__ __forceinline__ void write_value_tile(const QkvPlaces<bf16_t>& a, int tile, int kvh) {
+  const int num_heads = a.num_heads, num_kv = a.num_kv, head_size = a.head_size, page_size = a.page_size;
+  const size_t page_stride = (size_t)num_kv * page_size * head_size + a.page_pad;
+  const int run = a.tile_run[tile], q0 = a.tile_q0[tile];
+  const int t0 = a.run_start[run] + q0;
+  const int n = min(VT_TOKENS, a.run_start[run + 1] - t0);
+  const int p0 = a.cached_lens[run] + q0;   // position of the tile's first token
   const int total = (num_heads + 2 * num_kv) * head_size;
   const int col0 = (num_heads + num_kv) * head_size + kvh * head_size;
-  const int* tab = table + (size_t)run * table_width;
+  const int* tab = a.table + (size_t)run * a.table_width;
   const int groups = (p0 + n - 1) / 8 - p0 / 8 + 1;
   const int chunks = head_size / 8;
   // item = (chunk / 8, group / 8, chunk % 8, group % 8): the groups run fastest within a wave's 64 lanes
@@ -131,23 +137,23 @@ value_tiles_kernel(const bf16_t* __restrict__ qkv, const float* __restrict__ bia
     if (g >= groups || c >= chunks) continue;
     const int pos = (p0 / 8 + g) * 8;                 // first position of the group
     const int blk = pos / page_size;
-    const int page = blk < table_width ? tab[blk] : -1;
-    if (page < 0 || page >= num_pages) continue;
+    const int page = blk < a.table_width ? tab[blk] : -1;
+    if (page < 0 || page >= a.num_pages) continue;
     const int i0 = pos - p0;                           // the group's first token within the tile; may be < 0
     bf16x8 rows[8];
 #pragma unroll
     for (int j = 0; j < 8; ++j) {
       const int i = min(max(i0 + j, 0), n - 1);        // (tokens outside the tile are read somewhere and not written)
-      rows[j] = *(const bf16x8*)(qkv + (size_t)(t0 + i) * total + col0 + c * 8);
+      rows[j] = *(const bf16x8*)(a.qkv + (size_t)(t0 + i) * total + col0 + c * 8);
     }
-    if (bias) {
-      const f32x4 b0 = *(const f32x4*)(bias + col0 + c * 8), b1 = *(const f32x4*)(bias + col0 + c * 8 + 4);
+    if (a.bias) {
+      const f32x4 b0 = *(const f32x4*)(a.bias + col0 + c * 8), b1 = *(const f32x4*)(a.bias + col0 + c * 8 + 4);
 #pragma unroll
       for (int j = 0; j < 8; ++j)
 #pragma unroll
         for (int e = 0; e < 8; ++e) rows[j][e] = (bf16_t)((float)rows[j][e] + (e < 4 ? b0[e] : b1[e - 4]));
     }
-    bf16_t* dst = v_pages + (size_t)page * page_stride + ((size_t)kvh * head_size + c * 8) * page_size + pos % page_size;
+    bf16_t* dst = a.v_pages + (size_t)page * page_stride + ((size_t)kvh * head_size + c * 8) * page_size + pos % page_size;
     const bool whole = i0 >= 0 && i0 + 8 <= n;
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
@@ -165,8 +171,23 @@ value_tiles_kernel(const bf16_t* __restrict__ qkv, const float* __restrict__ bia
   }
 }
 
+// Queries and keys, and values token by token.
+template <typename T>
+__global__ void __launch_bounds__(256) qkv_write_kernel(QkvPlaces<T> a) {
+  write_token<T, false>(a, blockIdx.x, blockIdx.y);
+}
+
+// The same, but the values of longer runs by tiles, by the first blocks (`num_tiles` of them a head), `parts` blocks a token behind
+// them. One launch: as two, one behind the other, they took 9.4 us for 333 tokens of 2,048 columns (a prompt of 24 layers 2,821 us, so
+// 2,771), 12.5 for 640 (a step of 40 requests beside a prompt 4,300 us, so 4,190).
+__global__ void __launch_bounds__(256) qkv_tiles_kernel(QkvPlaces<bf16_t> a, int num_tiles, int parts) {
+  const int tiles = num_tiles * a.num_kv, at = (int)blockIdx.x - tiles;
+  if (at < 0) write_value_tile(a, (int)blockIdx.x % num_tiles, (int)blockIdx.x / num_tiles);
+  else write_token<bf16_t, true>(a, at / parts, at % parts);
+}
+
 // With `num_tiles > 0` (bfloat16 only) the values of the runs that `tile_run` / `tile_q0` cut into tiles of
-// `tile_tokens` tokens are written by tiles, and the token-wise kernel leaves them out.
+// `tile_tokens` tokens are written by tiles, and not token by token.
 extern "C" int tnx_qkv_write(const void* qkv, int dtype, const float* bias, float scale, const int* positions,
                              const int* token_request, const int* table, int table_width, int page_size,
                              int num_pages, void* q_out, void* k_pages, void* v_pages, int tokens, int num_heads,
@@ -193,25 +214,20 @@ extern "C" int tnx_qkv_write(const void* qkv, int dtype, const float* bias, floa
     TNX_REQUIRE(run_start && cached_lens && tile_run && tile_q0, "qkv_write: tiles without their tables");
     TNX_REQUIRE(num_kv <= 65535, "qkv_write: too many heads");
   }
-  const dim3 grid(tokens, ((num_heads + 2 * num_kv) * head_size / 8 + 255) / 256);
-  if (dtype == TNX_F32)
-    qkv_write_kernel<float><<<grid, 256, 0, stream>>>((const float*)qkv, bias, scale, positions, token_request,
-                                                        table, table_width, page_size, num_pages, (float*)q_out,
-                                                        (float*)k_pages, (float*)v_pages, num_heads, num_kv, head_size,
-                                                        run_start, 0, turn_a, turn_b, turn_rows, page_pad);
-  else
-    qkv_write_kernel<bf16_t><<<grid, 256, 0, stream>>>((const bf16_t*)qkv, bias, scale, positions, token_request,
-                                                         table, table_width, page_size, num_pages, (bf16_t*)q_out,
-                                                         (bf16_t*)k_pages, (bf16_t*)v_pages, num_heads, num_kv,
-                                                         head_size, run_start, by_tiles ? 1 : 0, turn_a, turn_b,
-                                                         turn_rows, page_pad);
-  TNX_CHECK_LAUNCH("qkv_write");
-  if (by_tiles) {
-    value_tiles_kernel<<<dim3(num_tiles, num_kv), 256, 0, stream>>>(
-        (const bf16_t*)qkv, bias, run_start, cached_lens, table, table_width, page_size, num_pages, tile_run, tile_q0,
-        (bf16_t*)v_pages, num_heads, num_kv, head_size, page_pad);
-    TNX_CHECK_LAUNCH("value_tiles");
+  const int parts = ((num_heads + 2 * num_kv) * head_size / 8 + 255) / 256;
+#define PLACES(T)                                                                                                                     \
+  QkvPlaces<T>{(const T*)qkv, bias, scale, positions, token_request, table, table_width, page_size, num_pages, (T*)q_out, (T*)k_pages, \
+               (T*)v_pages, num_heads, num_kv, head_size, run_start, cached_lens, turn_a, turn_b, turn_rows, page_pad, tile_run, tile_q0}
+  if (dtype == TNX_F32) {
+    qkv_write_kernel<float><<<dim3(tokens, parts), 256, 0, stream>>>(PLACES(float));
+  } else if (!by_tiles) {
+    qkv_write_kernel<bf16_t><<<dim3(tokens, parts), 256, 0, stream>>>(PLACES(bf16_t));
+  } else {
+    TNX_REQUIRE((long long)num_tiles * num_kv + (long long)tokens * parts < (1ll << 31), "qkv_write: too many tokens");
+    qkv_tiles_kernel<<<(unsigned)(num_tiles * num_kv + tokens * parts), 256, 0, stream>>>(PLACES(bf16_t), num_tiles, parts);
   }
+#undef PLACES
+  TNX_CHECK_LAUNCH("qkv_write");
   return 0;
 }
 
