@@ -500,28 +500,30 @@ __global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
     const unsigned from = (GATED && (row & 32) ? p.n : 0) + min(col, p.n - 1);
     t.woff[j] = 2u * (from * (unsigned)p.k + Products::k_of(row));
   }
-  t.run(smem, p.a, w, p.k / 64);
   const int r0 = Products::row0(), c0 = n0 + (GATED ? Products::col0() / 2 : Products::col0());
+  float weight[GATED ? MI : 1];      // (looked up before the products: at their end it would be two more times to reach memory)
   if constexpr (GATED) {
-    float weight[MI];
 #pragma unroll
     for (int i = 0; i < MI; ++i)
       weight[i] = p.weights ? p.weights[p.order[begin + min(r0 + 32 * i + (int)(threadIdx.x & 31), count - 1)]] : 1.f;
+  }
+  t.run(smem, p.a, w, p.k / 64);
+  if constexpr (GATED) {
     t.template hand_out<bf16_t, 32>(
         smem, [&](int i, int, int e, int, int) { return gated(t.acc[i][0][e] * weight[i], t.acc[i][1][e] * weight[i], p.act, p.limit); },
-        [&](int r, int c, f32x4 chunk) {
+        [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((bf16_t*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
   } else if constexpr (UP) {
     t.template hand_out<bf16_t, 64>(
         smem, [&](int i, int j, int e, int, int) { return apply_act(t.acc[i][j][e], p.act); },
-        [&](int r, int c, f32x4 chunk) {
+        [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((bf16_t*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
   } else {
     t.template hand_out<float, 64>(
         smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
-        [&](int r, int c, f32x4 chunk) {
+        [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((float*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
   }

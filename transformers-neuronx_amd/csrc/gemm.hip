@@ -477,7 +477,7 @@ gemm_f32_parts_kernel(const float* __restrict__ x, const float* __restrict__ w, 
     const float v = mw + row < M && nw + column < N ? checked(acc[i][j][e], mw + row, nw + column) : 0.f;
     return apply_act(v + added[j][e], act);
   };
-  Tile<MI, NI, 2, WM, WN>::template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
+  Tile<MI, NI, 2, WM, WN>::template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk, int) {
     if (mw + r >= M || nw + c >= N) return;
     const size_t o = (size_t)(mw + r) * N + nw + c;
     if (whole) {
@@ -1981,34 +1981,44 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_tiles_kernel(const bf1
     const int row = Products::w_row(j);
     t.woff[j] = 2u * ((unsigned)min(n0 + row, N - 1) * (unsigned)K + Products::k_of(row));
   }
-  t.run(smem, x + 64 * first, w + 64 * first, steps);
   const int mw = m0 + Products::row0(), nw = n0 + Products::col0();
+  // What the end adds is asked for before the products: there it would be one more time to reach memory, or two.
+  float added[NI][16];
+  f32x4 onto[Products::template out_count<float, 32 * NI>()];
+  if (!partial) {
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int n = nw + 32 * j + 8 * g + 4 * (int)((threadIdx.x >> 5) & 1);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) added[j][4 * g + e] = bias ? bias[min(n + e, N - 1)] : 0.f;
+      }
+    if (residual) {
+#pragma unroll
+      for (int k = 0; k < Products::template out_count<float, 32 * NI>(); ++k)
+        onto[k] = *(const f32x4*)(residual + (size_t)min(mw + Products::template out_row<float, 32 * NI>(k), M - 1) * N +
+                                  min(nw + Products::template out_column<float, 32 * NI>(), N - 4));
+    }
+  }
+  t.run(smem, x + 64 * first, w + 64 * first, steps);
   if (partial) {
     float* mine = partial + (size_t)blockIdx.y * M * N;
     t.template hand_out<float, 32 * NI>(
         smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
-        [&](int r, int c, f32x4 chunk) {
+        [&](int r, int c, f32x4 chunk, int) {
           if (mw + r < M && nw + c < N) *(f32x4*)(mine + (size_t)(mw + r) * N + nw + c) = chunk;
         });
     return;
   }
-  float added[NI][16];
-#pragma unroll
-  for (int j = 0; j < NI; ++j)
-#pragma unroll
-    for (int e = 0; e < 16; ++e)
-      added[j][e] = bias ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * (int)((threadIdx.x >> 5) & 1) + (e & 3), N - 1)] : 0.f;
   auto value = [&](int i, int j, int e, int, int) { return apply_act(t.acc[i][j][e] + added[j][e], act); };
   if (out_dtype == TNX_F32) {
-    t.template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
-      if (mw + r < M && nw + c < N) {
-        const size_t o = (size_t)(mw + r) * N + nw + c;
-        if (residual) chunk += *(const f32x4*)(residual + o);
-        *(f32x4*)((float*)out + o) = chunk;
-      }
+    t.template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk, int k) {
+      if (residual) chunk += onto[k];
+      if (mw + r < M && nw + c < N) *(f32x4*)((float*)out + (size_t)(mw + r) * N + nw + c) = chunk;
     });
   } else {
-    t.template hand_out<bf16_t, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk) {
+    t.template hand_out<bf16_t, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk, int) {
       if (mw + r < M && nw + c < N) *(f32x4*)((bf16_t*)out + (size_t)(mw + r) * N + nw + c) = chunk;
     });
   }

@@ -118,7 +118,20 @@ struct Tile {
 
   // Hands the result over by rows. `value(i, j, e, row, column)`: the element as it goes out (row and column of the tile,
   // j and e of the accumulator); COLS columns of a wave go out (all 32 NI, or the first 32 j = 0 where `value` joins
-  // several). `put(row, column, chunk)`: 16 bytes of the result, of type T, at a row and column of the wave's tile.
+  // several). `put(row, column, chunk, k)`: 16 bytes of the result, of type T, at a row and column of the wave's tile, the lane's
+  // k-th (`out_row`, `out_column`: where that is).
+  template <typename T, int COLS>
+  static constexpr int out_count() { return MI * 32 * COLS * (int)sizeof(T) / 16 / 64; }
+  template <typename T, int COLS>
+  static __device__ __forceinline__ int out_row(int k) {
+    constexpr int CHUNKS = COLS * (int)sizeof(T) / 16;
+    return k * (64 / CHUNKS) + (int)(threadIdx.x & 63) / CHUNKS;
+  }
+  template <typename T, int COLS>
+  static __device__ __forceinline__ int out_column() {
+    constexpr int CHUNKS = COLS * (int)sizeof(T) / 16;
+    return (int)(threadIdx.x & 63) % CHUNKS * (16 / (int)sizeof(T));
+  }
   template <typename T, int COLS, typename Value, typename Put>
   static __device__ __forceinline__ void hand_out(char* smem, Value value, Put put) {
     const int lane = threadIdx.x & 63, l32 = lane & 31, half = lane >> 5;
@@ -144,7 +157,7 @@ struct Tile {
 #pragma unroll
       for (int r0 = 0; r0 < 32; r0 += PASS) {
         const int r = r0 + lane / CHUNKS, c = lane % CHUNKS;
-        put(32 * i + r, c * (16 / (int)sizeof(T)), *(const f32x4*)(mine + r * ROW + c * 16));
+        put(32 * i + r, c * (16 / (int)sizeof(T)), *(const f32x4*)(mine + r * ROW + c * 16), (32 * i + r0) / PASS);
       }
       __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
       __builtin_amdgcn_wave_barrier();
