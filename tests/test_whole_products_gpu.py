@@ -71,7 +71,8 @@ def test_the_rule_on_sizes(m, n, k, linear, placed):
     assert bool(called) == (linear and n % 16 == 0)
 
 
-@pytest.mark.parametrize("m,heads,kv,hs,k,turned", [(9, 32, 32, 64, 2048, False), (40, 32, 32, 64, 2048, True), (24, 32, 32, 80, 2560, False)])
+@pytest.mark.parametrize("m,heads,kv,hs,k,turned", [(9, 32, 32, 64, 2048, False), (40, 32, 32, 64, 2048, True), (24, 32, 32, 80, 2560, False),
+                                                       (9, 320, 40, 18, 1024, True)])       # heads that do not come in fours
 def test_queries_keys_and_values(m, heads, kv, hs, k, turned):
     """The same places hold what the few-rows kernel, or the product and the launch behind it, leave there."""
     from test_float32_gpu import _step
