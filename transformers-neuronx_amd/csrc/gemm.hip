@@ -547,9 +547,30 @@ __global__ void gemm_mid_sum_kernel(const float* __restrict__ partial, const flo
                                     const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
                                     int N, int shares);
 
+// What follows a product whose K was shared out: the sum of the shares, or, with `left`, nothing but their number (1: the result
+// is made); whoever asked for it adds them (`tnx_shares_norm` or `tnx_gemm_shares_sum`).
+static int sum_shares(const float* partial, const float* bias, const float* residual, void* out, int out_dtype, int act, int M, int N,
+                      int shares, int* left, hipStream_t stream) {
+  if (left) *left = shares;
+  if (shares > 1 && !left) {
+    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
+                                                                                        act, M, N, shares);
+    TNX_CHECK_LAUNCH("gemm_mid_sum");
+  }
+  return 0;
+}
+
+// The sum alone, of a product that left its shares.
+extern "C" int tnx_gemm_shares_sum(const float* partial, const float* bias, const float* residual, float* out, int M, int N, int shares,
+                                   hipStream_t stream) {
+  TNX_REQUIRE(M > 0 && N > 0 && N % 4 == 0 && shares > 1 && partial && out && ((uintptr_t)partial & 15) == 0, "gemm_shares_sum: bad sizes");
+  return sum_shares(partial, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, shares, nullptr, stream);
+}
+
+
 template <int MI, int NI, int WM, int WN>
 static int launch_f32_parts(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype,
-                            int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
+                            int act, float* partial, int M, int N, int K, int shares, int* left, hipStream_t stream) {
   constexpr int bytes = 2 * 3 * (32 * MI * WM + 32 * NI * WN) * 64;
   static bool configured = false;
   if (!configured) {
@@ -566,12 +587,7 @@ static int launch_f32_parts(const float* x, const float* w, const float* bias, c
   gemm_f32_parts_kernel<MI, NI, WM, WN><<<dim3(tiles_m * tiles_n, shares), 64 * WM * WN, bytes, stream>>>(
       x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, whole, M, N, K, tiles_m, per);
   TNX_CHECK_LAUNCH("gemm_f32_parts");
-  if (shares > 1) {
-    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
-                                                                                        act, M, N, shares);
-    TNX_CHECK_LAUNCH("gemm_mid_sum");
-  }
-  return 0;
+  return sum_shares(partial, bias, residual, out, out_dtype, act, M, N, shares, left, stream);
 }
 
 // The most floats that the shares' sums of one product may take (32 MB).
@@ -616,9 +632,9 @@ extern "C" int tnx_gemm_f32_workspace(int M, int N, int K) {
 
 // `tile` as in `choose_f32_tiles`.
 static int f32_parts(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype, int act, int M,
-                     int N, int K, int tile, int shares, float* workspace, hipStream_t stream) {
+                     int N, int K, int tile, int shares, float* workspace, int* left, hipStream_t stream) {
 #define F32_TILES(MI, NI, WM, WN) \
-  launch_f32_parts<MI, NI, WM, WN>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
+  launch_f32_parts<MI, NI, WM, WN>(x, w, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream)
   return tile == 0 ? F32_TILES(1, 2, 4, 2) : tile == 1 ? F32_TILES(1, 1, 2, 4) : F32_TILES(1, 1, 2, 2);
 #undef F32_TILES
 }
@@ -632,13 +648,13 @@ extern "C" int tnx_gemm_f32_parts(const float* x, const float* w, const float* b
   TNX_REQUIRE(tile >= 0 && tile <= 2 && shares >= 1 && shares <= 16 && shares <= K / 32, "gemm_f32_parts: tile 0 to 2, up to 16 shares");
   TNX_REQUIRE(shares == 1 || (N % 4 == 0 && workspace && workspace_floats >= (size_t)shares * M * N),
               "gemm_f32_parts: shares want N a multiple of 4 and a workspace of shares x M x N floats");
-  return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, stream);
+  return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, nullptr, stream);
 }
 
 // `workspace`: as many floats as `tnx_gemm_f32_workspace` names for the sizes; with less, K is not shared out.
-extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, const float* residual, void* out,
-                            int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
-                            hipStream_t stream) {
+static int gemm_f32(const float* x, const float* w, const float* bias, const float* residual, void* out, int out_dtype, int act,
+                    int M, int N, int K, float* workspace, size_t workspace_floats, int* left, hipStream_t stream) {
+  if (left) *left = 1;
   TNX_REQUIRE(M >= 0 && N > 0 && K > 0, "gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
   if (M == 0) return 0;
   if (M <= 16 && K % 4 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0) {
@@ -650,13 +666,19 @@ extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, c
     int tile = 0, shares = 1;
     choose_f32_tiles(M, N, K, tile, shares);
     if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
-    return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, stream);
+    return f32_parts(x, w, bias, residual, out, out_dtype, act, M, N, K, tile, shares, workspace, left, stream);
   }
   dim3 grid((N + F32_TILE - 1) / F32_TILE, (M + F32_TILE - 1) / F32_TILE);
   TNX_REQUIRE(grid.y <= 65535, "gemm_f32: M=%d is too large", M);
   gemm_f32_kernel<<<grid, 256, 0, stream>>>(x, w, bias, residual, out, out_dtype, act, M, N, K);
   TNX_CHECK_LAUNCH("gemm_f32");
   return 0;
+}
+
+extern "C" int tnx_gemm_f32(const float* x, const float* w, const float* bias, const float* residual, void* out,
+                            int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
+                            hipStream_t stream) {
+  return gemm_f32(x, w, bias, residual, out, out_dtype, act, M, N, K, workspace, workspace_floats, nullptr, stream);
 }
 
 // ------------------------------------------------------------------------------------------ bfloat16, tiled
@@ -1914,7 +1936,7 @@ gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__
 
 template <int MT, int AHEAD, int NW = 4, typename Scatter = NoScatter>
 static int launch_mid(const bf16_t* x, const bf16_t* w_tiles, const float* bias, const float* residual, void* out,
-                      int out_dtype, int act, float* partial, int M, int N, int K, int shares, hipStream_t stream,
+                      int out_dtype, int act, float* partial, int M, int N, int K, int shares, int* left, hipStream_t stream,
                       const Scatter& sc = Scatter{}) {
   constexpr int bytes = (AHEAD + 1) * (16 * MT * 256 + NW * 4 * 1024);
   static_assert(bytes <= 160 * 1024, "the stages do not fit the LDS of a compute unit");
@@ -1933,19 +1955,14 @@ static int launch_mid(const bf16_t* x, const bf16_t* w_tiles, const float* bias,
   gemm_bf16_mid_kernel<MT, AHEAD, NW, Scatter><<<grid, 64 * NW, bytes, stream>>>(x, w_tiles, bias, residual, out, out_dtype,
                                                                                  act, partial, M, N, K, per, sc);
   TNX_CHECK_LAUNCH("gemm_bf16_mid");
-  if (grid.y > 1) {
-    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out,
-                                                                                        out_dtype, act, M, N, grid.y);
-    TNX_CHECK_LAUNCH("gemm_mid_sum");
-  }
-  return 0;
+  return sum_shares(partial, bias, residual, out, out_dtype, act, M, N, (int)grid.y, left, stream);
 }
 
 // `shares` 0: chosen here (as many as give every compute unit a block at most, each with four steps of K or more,
 // within the workspace); `ahead` 0: three steps in flight up to 64 rows, two beyond (what LDS holds).
-extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float* bias, const float* residual,
-                                 void* out, int out_dtype, int act, int M, int N, int K, float* workspace,
-                                 size_t workspace_floats, int shares, int ahead, hipStream_t stream) {
+static int gemm_bf16_mid(const void* x, const void* w_tiles, const float* bias, const float* residual, void* out, int out_dtype,
+                         int act, int M, int N, int K, float* workspace, size_t workspace_floats, int shares, int ahead, int* left,
+                         hipStream_t stream) {
   TNX_REQUIRE(M > 0 && M <= 128 && N > 0 && K > 0, "gemm_bf16_mid: takes 1 to 128 rows, got M=%d N=%d K=%d", M, N, K);
   TNX_REQUIRE(N % 16 == 0 && K % 128 == 0, "gemm_bf16_mid: the tile-ordered weight needs N a multiple of 16 and K "
               "of 128, got N=%d K=%d", N, K);
@@ -1970,7 +1987,7 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
   const int mt = (M + 15) / 16;
   if (ahead == 0) ahead = mt <= 4 ? 3 : 2;
   if (mt > 4 && ahead > 2) ahead = 2;               // what LDS holds
-#define MID(MT, A) launch_mid<MT, A>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream)
+#define MID(MT, A) launch_mid<MT, A>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream)
 #define MID_LOW(MT) return ahead == 2 ? MID(MT, 2) : MID(MT, 3)
 #define MID_HIGH(MT) return MID(MT, 2)
   switch (mt) {
@@ -1988,6 +2005,13 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 #undef MID
 }
 
+extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float* bias, const float* residual,
+                                 void* out, int out_dtype, int act, int M, int N, int K, float* workspace,
+                                 size_t workspace_floats, int shares, int ahead, hipStream_t stream) {
+  return gemm_bf16_mid(x, w_tiles, bias, residual, out, out_dtype, act, M, N, K, workspace, workspace_floats, shares, ahead, nullptr,
+                       stream);
+}
+
 // The same for 9 to 48 rows with a rounded result, or with queries, keys and values put in their places, and K whole: no sum
 // follows, and what fills the chip is the number of waves a block has, two to four of 16 columns each: as many as leave every
 // compute unit one block (`whole_waves`). A unit brings some 30 bytes a nanosecond from memory however many ask on it, so what
@@ -2002,7 +2026,7 @@ extern "C" int tnx_gemm_bf16_mid(const void* x, const void* w_tiles, const float
 template <typename Scatter>
 static int launch_whole(const bf16_t* x, const bf16_t* w_tiles, const float* bias, void* out, int out_dtype, int act, int M, int N, int K,
                         int waves, const Scatter& sc, hipStream_t stream) {
-#define WHOLE(MT, NW) launch_mid<MT, 3, NW, Scatter>(x, w_tiles, bias, nullptr, out, out_dtype, act, nullptr, M, N, K, 1, stream, sc)
+#define WHOLE(MT, NW) launch_mid<MT, 3, NW, Scatter>(x, w_tiles, bias, nullptr, out, out_dtype, act, nullptr, M, N, K, 1, nullptr, stream, sc)
 #define WHOLE_MT(MT) return waves == 2 ? WHOLE(MT, 2) : waves == 3 ? WHOLE(MT, 3) : WHOLE(MT, 4)
   if (M <= 32) WHOLE_MT(2);
   WHOLE_MT(3);
@@ -2116,7 +2140,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_tiles_kernel(const bf1
 
 template <int MI, int NI, int ST, int WM, int WN>
 static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, const float* residual, void* out, int out_dtype,
-                        int act, float* partial, int M, int N, int K, int shares, hipStream_t stream) {
+                        int act, float* partial, int M, int N, int K, int shares, int* left, hipStream_t stream) {
   constexpr int bytes = Tile<MI, NI, ST, WM, WN>::BYTES;
   static bool configured = false;
   if (!configured) {
@@ -2131,12 +2155,7 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
   gemm_bf16_tiles_kernel<MI, NI, ST, WM, WN><<<dim3(tiles_m * tiles_n, shares), 64 * WM * WN, bytes, stream>>>(
       x, w, bias, residual, out, out_dtype, act, shares > 1 ? partial : nullptr, M, N, K, tiles_m, per);
   TNX_CHECK_LAUNCH("gemm_bf16_tiles");
-  if (shares > 1) {
-    gemm_mid_sum_kernel<<<(unsigned)(((size_t)M * N / 4 + 255) / 256), 256, 0, stream>>>(partial, bias, residual, out, out_dtype,
-                                                                                        act, M, N, shares);
-    TNX_CHECK_LAUNCH("gemm_mid_sum");
-  }
-  return 0;
+  return sum_shares(partial, bias, residual, out, out_dtype, act, M, N, shares, left, stream);
 }
 
 // Which products these tiles take, and with which tile and how many shares of K (0: none, the vendor library).
@@ -2208,9 +2227,9 @@ extern "C" int tnx_gemm_bf16_tiles_workspace(int M, int N, int K) {
 }
 
 // `workspace`: as many floats as `tnx_gemm_bf16_tiles_workspace` names for the sizes. `tile`, `shares` 0: chosen here.
-extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bias, const float* residual, void* out,
-                                   int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
-                                   int tile, int shares, hipStream_t stream) {
+static int gemm_bf16_tiles(const void* x, const void* w, const float* bias, const float* residual, void* out, int out_dtype, int act,
+                           int M, int N, int K, float* workspace, size_t workspace_floats, int tile, int shares, int* left,
+                           hipStream_t stream) {
   TNX_REQUIRE(M > 0 && N > 0 && N % 8 == 0 && K > 0 && K % 64 == 0, "gemm_bf16_tiles: N in 8s and K in 64s, got M=%d N=%d K=%d", M, N, K);
   TNX_REQUIRE((long long)M * K < (1ll << 31) && (long long)N * K < (1ll << 31), "gemm_bf16_tiles: operands of 4 GB or more");
   TNX_REQUIRE(out_dtype == TNX_F32 || (out_dtype == TNX_BF16 && residual == nullptr), "gemm_bf16_tiles: a residual beside a float32 result");
@@ -2224,8 +2243,28 @@ extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bi
   if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
   const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
   if (tile == TILES_128)
-    return launch_tiles<2, 1, 4, 2, 4>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream);
-  return launch_tiles<1, 1, 4, 2, 2>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, stream);
+    return launch_tiles<2, 1, 4, 2, 4>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream);
+  return launch_tiles<1, 1, 4, 2, 2>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream);
+}
+
+extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bias, const float* residual, void* out,
+                                   int out_dtype, int act, int M, int N, int K, float* workspace, size_t workspace_floats,
+                                   int tile, int shares, hipStream_t stream) {
+  return gemm_bf16_tiles(x, w, bias, residual, out, out_dtype, act, M, N, K, workspace, workspace_floats, tile, shares, nullptr, stream);
+}
+
+// A product of a float32 result onto a residual, by rows of some number (`way` 0), by tiles (1) or in float32 (2), whose shares of K
+// stay apart where K is shared out: `left` says how many lie in `workspace`, one behind the other, for `tnx_shares_norm` or
+// `tnx_gemm_shares_sum`; 1: `out` is the result.
+extern "C" int tnx_gemm_left(int way, const void* x, const void* w, const float* bias, const float* residual, float* out, int M, int N,
+                             int K, float* workspace, size_t workspace_floats, int* left, hipStream_t stream) {
+  TNX_REQUIRE(way >= 0 && way <= 2 && left, "gemm_left: ways are 0 to 2");
+  if (way == 0)
+    return gemm_bf16_mid(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, 0, 0, left, stream);
+  if (way == 1)
+    return gemm_bf16_tiles(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, 0, 0, left, stream);
+  return gemm_f32((const float*)x, (const float*)w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, left,
+                  stream);
 }
 
 // ------------------------------------------------------------------------------------- the vendor library

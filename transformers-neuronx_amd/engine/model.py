@@ -179,11 +179,14 @@ class DecoderModel:
         debug.tap("embedding", stream.x)
         # in steps of few rows, what the last block left may be a norm that the next products do (`norms_between`)
         few, between = ctx.num_tokens <= getattr(self.ops, "norm_beside_rows", 0), False
+        left = False                    # and in steps of more, shares of a sum that the next norm adds (`leaves_shares`)
         in_one = self.layers_in_one if ctx.num_tokens <= getattr(self.ops, "layer_rows", 0) and self.ops.layers_fit(ctx) else {}
         done = 0
         for call, (layer, cid, writes) in enumerate(self.schedule):
             if call < done:
                 continue
+            if left and (call in in_one or not getattr(self.layers[layer].block, "leaves_shares", False)):
+                stream, left = self._settled(stream), False
             if call in in_one:
                 behind = self._run_in_one(stream, call, in_one[call], ctx, caches)
                 if behind is not None:
@@ -198,8 +201,9 @@ class DecoderModel:
                 stream = self._settled(stream)
             stream = block.forward(stream, ctx, cache)
             between = few and getattr(block, "norms_between", False)
+            left = getattr(block, "leaves_shares", False)
             debug.tap(f"call{call}.layer{layer}", stream.x)
-        if between:
+        if between or left:
             stream = self._settled(stream)
         if stream.copies is not None and (stream.x is None or stream.pending is not None):
             # an arrangement that keeps several copies of the stream: their sum is what the head reads

@@ -35,8 +35,13 @@ _SIGNATURES = {
         "tnx_scale_and_cap": [_c_void_p, _c_float, _c_float, _c_ll, _c_void_p],
         "tnx_layernorm": [_c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                           _c_int, _c_void_p],
+        "tnx_shares_norm": [_c_void_p, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_float, _c_void_p, _c_void_p,
+                            _c_int, _c_int, _c_int, _c_void_p],
     },
     "gemm": {
+        "tnx_gemm_left": [_c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p,
+                          ctypes.c_size_t, _c_void_p, _c_void_p],
+        "tnx_gemm_shares_sum": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                          _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
         "tnx_gemm_f32_parts": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
@@ -345,6 +350,54 @@ class NormBetween(DeferredNorm):
 
     def normalised(self):
         raise TypeError("a norm behind a sum is folded into no product")
+
+
+class Onto:
+    """A residual handed to `HipOps.linear` by someone who norms the sum next and does nothing else with it before: where the
+    product shares K out, what it gives back is a `SharesLeft`."""
+
+    __slots__ = ("x",)
+
+    def __init__(self, x):
+        self.x = x
+
+
+class SharesLeft:
+    """A product's float32 result of which the shares of K have not been added yet. `normed` adds them in the launch of the norm
+    that follows, `settled` by a launch of their own; either once."""
+
+    __slots__ = ("ops", "shares", "count", "bias", "residual", "out", "added")
+
+    def __init__(self, ops, shares, count, bias, residual, out):
+        self.ops, self.shares, self.count, self.bias, self.residual, self.out = ops, shares, count, bias, residual, out
+        self.added = False
+
+    def settled(self):
+        if not self.added:
+            m, n = self.out.shape
+            self.ops._call("gemm", "tnx_gemm_shares_sum", _ptr(self.shares), _ptr(self.bias), _ptr(self.residual), _ptr(self.out), m, n,
+                           self.count, _stream())
+            self._done()
+        return self.out
+
+    def normed(self, weight, bias, eps, dtype, center):
+        """(the sum, its norm in `dtype`)."""
+        out, f32 = self.out, dtype == torch.float32
+        m, n = out.shape
+        if (self.added or n > self.ops.shares_norm_width or n % 4 or (not f32 and dtype != torch.bfloat16)
+                or any((_ptr(a) or 0) % 16 for a in (self.bias, self.residual, weight, bias))):
+            return self.settled(), self.ops.layernorm(out, weight, bias, eps, dtype, False, True, center)[1]
+        self.ops._want_norm(out, weight, bias)
+        h = torch.empty(m, n, dtype=dtype, device=out.device)
+        self.ops._call("elementwise", "tnx_shares_norm", _ptr(self.shares), self.count, _ptr(self.bias), _ptr(self.residual), _ptr(out),
+                       _ptr(weight), _ptr(bias), float(eps), _ptr(h) if f32 else None, None if f32 else _ptr(h), m, n,
+                       int(bool(center)), _stream(),
+                       work=lambda: (f"{m}x{n}", m * n * (4 * self.count + 8 + h.element_size()), 0.0))
+        self._done()
+        return out, h
+
+    def _done(self):
+        self.added, self.shares, self.residual = True, None, None
 
 
 class _LayerOf(ctypes.Structure):
@@ -705,7 +758,26 @@ class HipOps:
     @staticmethod
     def settled(stream_x):
         """What a stream holds as a tensor."""
+        if type(stream_x) is SharesLeft:
+            return stream_x.settled()
         return stream_x.settled()[0] if isinstance(stream_x, NormBetween) else stream_x
+
+    # Rows that the norm's launch adds a product's shares for: what its registers hold.
+    shares_norm_width = 4096
+
+    @staticmethod
+    def onto(x):
+        """The residual of a product whose result goes to a norm, and to a sum behind that norm, and nowhere else."""
+        return x if debug.tapping() else Onto(x)
+
+    def _left(self, way, x, w, bias, residual, m, n, k, room):
+        """The product with its shares of K left apart."""
+        out = torch.empty(m, n, dtype=torch.float32, device=x.device)
+        space, left = torch.empty(room, dtype=torch.float32, device=x.device), _c_int()
+        self._call("gemm", "tnx_gemm_left", way, _ptr(x), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out), m, n, k, _ptr(space), room,
+                   ctypes.addressof(left), _stream(),
+                   work=lambda: self._product_work(m, n, k, x.element_size(), w.element_size(), 4, True))
+        return out if left.value == 1 else SharesLeft(self, space, left.value, bias, residual, out)
 
     def _beside_weight(self, w, m, norm):
         """The tile-ordered matrix that the products next to a norm read, or None where they do not take the sizes."""
@@ -846,10 +918,12 @@ class HipOps:
         left False such a product (the head's) stays on our kernel. `into`: where such a float32 result goes (rows
         of a larger tensor), instead of a tensor of its own."""
         if isinstance(x, DeferredNorm):
-            out, x = self._linear_of_norm(x, w, bias, act, residual, out_f32, force_tiled, into)
+            out, x = self._linear_of_norm(x, w, bias, act, residual.x if type(residual) is Onto else residual, out_f32, force_tiled, into)
             if out is not None:
                 return out
-        tiles = None
+        tiles, leaves = None, type(residual) is Onto
+        if leaves:
+            residual, leaves = residual.x, act in (None, "none") and out_f32 and into is None
         if isinstance(w, PreparedWeight):
             if w.inner != w.tensor.shape[1] and x.shape[1] == w.inner:
                 x = torch.nn.functional.pad(x, (0, w.tensor.shape[1] - w.inner))
@@ -880,6 +954,9 @@ class HipOps:
             _want(residual, "residual", torch.float32, (m, n))
         if self._some_rows_product(m, n, k, w, tiles, residual, out_f32, force_tiled):
             # decode batches of 33 to 128 requests, a float32 result: our kernel for some rows
+            shares = max(1, min(self.compute_units // -(-n // 64), k // 512))       # as the kernel shares K out
+            if leaves and shares > 1:
+                return self._left(0, self.cast(x, torch.bfloat16), tiles, bias, residual, m, n, k, shares * m * n)
             out = torch.empty(m, n, dtype=out_dtype, device=x.device)
             space = self._library_workspace(x.device)
             self._call("gemm", "tnx_gemm_bf16_mid", _ptr(self.cast(x, torch.bfloat16)), _ptr(tiles), _ptr(bias),
@@ -887,6 +964,8 @@ class HipOps:
                        0, 0, _stream(), work=lambda: self._product_work(m, n, k, out_item=4, residual=residual is not None))
             return out
         room = self._tiles_room(m, n, k, x, w, residual, out_f32, force_tiled) if f32_by_library or residual is not None or not out_f32 else -1
+        if room > 0 and leaves:
+            return self._left(1, self.cast(x, torch.bfloat16), w, bias, residual, m, n, k, room)
         if room >= 0:
             out = torch.empty(m, n, dtype=out_dtype, device=x.device) if into is None else _want(into, "into", out_dtype, (m, n))
             if _ptr(out) % 16 == 0:
@@ -932,6 +1011,8 @@ class HipOps:
         if w.dtype == torch.float32:
             xa = self.cast(x, torch.float32)
             room = library("gemm").tnx_gemm_f32_workspace(m, n, k)
+            if room and leaves and (_ptr(xa) | _ptr(w)) % 16 == 0:
+                return self._left(2, xa, w, bias, residual, m, n, k, room)
             space = torch.empty(room, dtype=torch.float32, device=x.device) if room else None
             self._call("gemm", "tnx_gemm_f32", _ptr(xa), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out),
                        _code(out_dtype), _ACT[act], m, n, k, _ptr(space), room, _stream(),

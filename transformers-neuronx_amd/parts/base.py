@@ -145,7 +145,8 @@ def joined_rows(parts):
 def residual_to_product(forward):
     """Marks the `forward` of a mixer or feed-forward that has a `first_weight` and does with `residual` nothing but hand it to
     `ops.linear` as the residual of its last product. A block behind whose sums a norm
-    stands may then hand over `h` and `residual` as what `ops.norm_between` returns. The mark is the function's: a subclass with
+    stands may then hand over `h` and `residual` as what `ops.norm_between` returns, and one before whose next norm nothing else reads
+    the sum `residual` as `ops.onto` makes it and take a result that is no tensor yet. The mark is the function's: a subclass with
     a `forward` of its own has tensors again unless that is marked too."""
     forward.residual_to_product = True
     return forward

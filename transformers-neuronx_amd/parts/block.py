@@ -33,6 +33,11 @@ class PreNormBlock(Block):
     fold_mixer_norm = fold_feed_forward_norm = False
     mixer_norm_rows = feed_forward_norm_rows = -1     # up to how many tokens: what a step asks, once a norm
 
+    # Each part's last product adds the stream, and behind it stands a norm, of this block or the next: the backend may leave the
+    # product's shares of K to the norm's launch (`HipOps.onto`). The block then takes a stream whose sum has not been made, and
+    # leaves one.
+    leaves_shares = False
+
     def after_load(self) -> None:
         # Each norm's output goes to one part only; where that part does nothing with it but one matrix
         # product, the backend may do the norm inside the product (the few-rows products of decode steps:
@@ -44,6 +49,10 @@ class PreNormBlock(Block):
         self.mixer_norm_rows = self.mixer_norm.defer_rows if self.fold_mixer_norm else -1
         self.feed_forward_norm_rows = self.feed_forward_norm.defer_rows if self.fold_feed_forward_norm else -1
         self.in_one = _layer_parts(self, PreNormBlock)
+        self.leaves_shares = (hasattr(self.mixer_norm.ops, "onto") and type(self).forward is PreNormBlock.forward
+                              and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None
+                                      for p in (self.mixer, self.feed_forward))
+                              and all(_is_its_fused_form(n) for n in (self.mixer_norm, self.feed_forward_norm)))
 
     def norms_in_one(self, before):
         return self.mixer_norm.fused_form(), self.feed_forward_norm.fused_form()
@@ -51,14 +60,21 @@ class PreNormBlock(Block):
     def into_one(self, stream):
         return stream.x, self.mixer_norm.fused_form(), False
 
+    def _normed(self, norm, x, deferred):
+        """(x, its norm): `x` as a tensor, whatever the product before left of it."""
+        if self.leaves_shares and hasattr(type(x), "normed"):
+            if not deferred:
+                weight, bias, center, eps = norm.fused_form()
+                return x.normed(weight, bias, eps, norm.dtype, center)
+            x = x.settled()
+        return x, norm.deferred(x) if deferred else norm.forward(x, False, True)[1]
+
     def forward(self, stream: Stream, ctx, cache) -> Stream:
-        h = (self.mixer_norm.deferred(stream.x) if ctx.num_tokens <= self.mixer_norm_rows
-             else self.mixer_norm.forward(stream.x, False, True)[1])
-        x = debug.tap("after_mixer", self.mixer.forward(h, ctx, cache, stream.x))
-        h = (self.feed_forward_norm.deferred(x) if ctx.num_tokens <= self.feed_forward_norm_rows
-             else self.feed_forward_norm.forward(x, False, True)[1])
-        x = self.feed_forward.forward(h, ctx, x)
-        return Stream(x, None)
+        onto = self.mixer_norm.ops.onto if self.leaves_shares else None
+        x, h = self._normed(self.mixer_norm, stream.x, ctx.num_tokens <= self.mixer_norm_rows)
+        x = debug.tap("after_mixer", self.mixer.forward(h, ctx, cache, onto(x) if onto else x))
+        x, h = self._normed(self.feed_forward_norm, x, ctx.num_tokens <= self.feed_forward_norm_rows)
+        return Stream(self.feed_forward.forward(h, ctx, onto(x) if onto else x), None)
 
 
 @register_block("post_norm")
