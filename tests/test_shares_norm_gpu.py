@@ -48,6 +48,7 @@ def test_products(dtype, m, n, k):
     """Every way a product shares K out, and results that are whole."""
     from transformers_neuronx_amd.kernels.hip import HipOps, SharesLeft
     hip, g = HipOps(dtype, DEV), _gen(m + n)
+    hip._choose_left = lambda *a: None              # the same way with a sum of its own and without
     x = torch.randn(m, k, device=DEV, generator=g).to(dtype)
     w = hip.prepare_weight((torch.randn(n, k, device=DEV, generator=g) * 0.02).to(dtype))
     residual, bias, weight = torch.randn(m, n, device=DEV, generator=g), torch.randn(n, device=DEV, generator=g), torch.randn(n, device=DEV, generator=g)
@@ -66,6 +67,34 @@ def test_products(dtype, m, n, k):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("m,n,k,way", [(9, 1024, 4096, (0, 0, 8)), (16, 1024, 1024, None), (17, 1024, 1024, (0, 0, 4)), (32, 768, 768, (0, 0, 3)),
+                                       (32, 512, 512, None), (48, 2560, 2560, (0, 0, 5)), (48, 2688, 2688, (0, 0, 5)), (48, 2752, 2688, None),
+                                       (48, 3072, 3072, None), (49, 3072, 3072, (1, 1, 5)), (33, 4096, 4096, (1, 1, 4)), (64, 4096, 16384, None),
+                                       (65, 1032, 1088, (1, 1, 4)), (256, 2048, 2048, (1, 1, 2)), (257, 2048, 2048, None), (768, 640, 512, (1, 1, 2)),
+                                       (769, 640, 512, None), (8, 2048, 8192, None), (100, 4104, 4096, None)])
+def test_ways(m, n, k, way):
+    """The rule's lines at 256 units, and that the product is right wherever it sends one, for rows that fill no tile as well."""
+    from transformers_neuronx_amd.kernels.hip import HipOps, SharesLeft
+    hip, g = HipOps(BF16, DEV), _gen(m + n + k)
+    x = torch.randn(m, k, device=DEV, generator=g).to(BF16)
+    raw = (torch.randn(n, k, device=DEV, generator=g) * 0.02).to(BF16)
+    w = hip.prepare_weight(raw)
+    hip.compute_units = 256
+    if n % 16 == 0 and k % 128 == 0:
+        assert hip._choose_left(m, n, k, True) == way
+    elif way is not None:
+        assert w.tiles is None and hip._choose_left(m, n, k, False) == way
+    residual, bias = torch.randn(m, n, device=DEV, generator=g), torch.randn(n, device=DEV, generator=g)
+    out = hip.linear(x, w, bias, residual=hip.onto(residual), out_f32=True)
+    assert way is None or type(out) is SharesLeft and out.count in (way[2], way[2] - 1)      # (whole steps a share: the last may be none)
+    out = hip.settled(out).double()
+    want = x.double() @ raw.double().t() + bias.double() + residual.double()
+    bound = x.double().abs() @ raw.double().abs().t() + bias.double().abs() + residual.double().abs()
+    # k + 2 float32 sums, each off by 2^-24 of at most the sum of the magnitudes
+    assert bool(((out - want).abs() <= (k + 2) * 2.0 ** -24 * bound).all())
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
 def test_through_the_model(tmp_path, dtype):
     """Prompts, a step of both kinds and recorded decode steps: the same logits, bit for bit, and sums that are looked at are made."""
@@ -79,9 +108,11 @@ def test_through_the_model(tmp_path, dtype):
                enable_bias=True, layer_norm_elementwise_affine=True, init_std=0.04)
     write_random_model(OPTConfig.from_dict(raw), str(tmp_path), 3, dtype=dtype)
     logits, made = {}, []
-    for fused in (True, False):
+    for fused in (True, False, "by the rule"):
         runner = runner_from_folder(str(tmp_path), EngineConfig(dtype=dtype, page_size=64, max_tokens=8192, max_num_seqs=48, device=DEV))
         runner.use_graphs = True
+        if fused != "by the rule":
+            runner.ops._choose_left = lambda *a: None
         if fused:
             call = runner.ops._call
             runner.ops._call = lambda lib, name, *a, **k: (made.append(name), call(lib, name, *a, **k))[1]
@@ -96,6 +127,8 @@ def test_through_the_model(tmp_path, dtype):
         steps += [[StepEntry(n, [5 + i for i in range(60)], [59])] + [StepEntry(r, [r], [0]) for r in range(n)]]
         logits[fused] = torch.cat([runner.step(step).float().cpu() for step in steps])
     assert torch.equal(logits[True], logits[False])
+    # (sums in another order, rounded to bfloat16 between the products)
+    assert float((logits["by the rule"] - logits[False]).norm() / logits[False].norm()) < (0.02 if dtype == "bfloat16" else 1e-6)
     assert "tnx_shares_norm" in made and "tnx_gemm_shares_sum" in made      # (the last sum is the head's, a norm of its own)
     del made[:]
     with debug.debug_context() as kept:

@@ -2257,12 +2257,12 @@ extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bi
 // stay apart where K is shared out: `left` says how many lie in `workspace`, one behind the other, for `tnx_shares_norm` or
 // `tnx_gemm_shares_sum`; 1: `out` is the result.
 extern "C" int tnx_gemm_left(int way, const void* x, const void* w, const float* bias, const float* residual, float* out, int M, int N,
-                             int K, float* workspace, size_t workspace_floats, int* left, hipStream_t stream) {
+                             int K, float* workspace, size_t workspace_floats, int tile, int shares, int* left, hipStream_t stream) {
   TNX_REQUIRE(way >= 0 && way <= 2 && left, "gemm_left: ways are 0 to 2");
   if (way == 0)
-    return gemm_bf16_mid(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, 0, 0, left, stream);
+    return gemm_bf16_mid(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, shares, 0, left, stream);
   if (way == 1)
-    return gemm_bf16_tiles(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, 0, 0, left, stream);
+    return gemm_bf16_tiles(x, w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, tile, shares, left, stream);
   return gemm_f32((const float*)x, (const float*)w, bias, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, workspace, workspace_floats, left,
                   stream);
 }

@@ -40,7 +40,7 @@ _SIGNATURES = {
     },
     "gemm": {
         "tnx_gemm_left": [_c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p,
-                          ctypes.c_size_t, _c_void_p, _c_void_p],
+                          ctypes.c_size_t, _c_int, _c_int, _c_void_p, _c_void_p],
         "tnx_gemm_shares_sum": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gemm_f32": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int,
                          _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
@@ -498,6 +498,7 @@ class HipOps:
         self._later = []
         self._tiles_per_block = {}
         self._tiles_rooms = {}
+        self._left_ways = {}
         self._landing, self._landing_turn = [None, None], 0
         self._lost = self._ones_zeros = None
         self._ints, self._ints_done, self._ints_turn = [None, None], [None, None], 0
@@ -770,11 +771,45 @@ class HipOps:
         """The residual of a product whose result goes to a norm, and to a sum behind that norm, and nowhere else."""
         return x if debug.tapping() else Onto(x)
 
-    def _left(self, way, x, w, bias, residual, m, n, k, room):
-        """The product with its shares of K left apart."""
+    def _way_to_leave(self, m, n, k, copy):
+        """(way, tile, shares) for `tnx_gemm_left` where the norm's launch, which comes anyway, makes shares worth more than they are
+        with a sum of their own; None: as without a norm behind. Product and norm on weights that no cache holds, us, without /
+        with the rule; over 346 sizes of 256 to 4,096 columns and 9 to 768 rows, most of them drawn, 1.17 times as quick, and 1.2 %
+        slower at the worst (48 rows 2,048 x 2,048):
+        - 9 to 48 rows, where the rows-of-some-number kernel has columns few enough for six shares or more (2,560 at 256 units): as
+          many as fill the units, of K 512, or four of 256. 32 rows 1,024 x 1,024 (columns x K) 8.5 / 6.8, 2,048 x 2,048 11.2 / 8.4, 2,560 x
+          2,560 12.8 / 9.9, 1,024 x 4,096 15.0 / 8.3. Three shares at least (one of 768 x 768 at 32 rows 8.9, three 6.8), and up to
+          16 rows long K alone: 9 rows 768 x 768 5.9 / 6.1, 4,096 x 4,096 11.8 / 14.2, but 2,048 x 8,192 15.8 / 12.7.
+        - more rows: tiles of 64 x 64 with two to eight shares where they all have a unit at once and a share has fewer than 24 steps of
+          64 (32: 333 rows 1,024 x 4,096 14.4 / 15.2; 64: 200 rows 2,048 x 8,192 19.8 / 24.8). 128 rows 768 x 768 15.1 / 6.9, 1,024 x 4,096
+          12.8 / 10.3, 64 rows 4,096 x 4,096 18.0 / 13.9, 256 rows 2,048 x 2,048 15.9 / 12.4. From 33 rows on only where the kernel above has
+          four shares at most (39 rows 3,072 x 3,072, five: 11.5 / 11.6).
+        Tiles of 128 x 128 with shares where the library has no shares were a loss as often as a gain (640 rows 2,048 x 2,048 18.9 /
+        23.2)."""
+        key = (m, n, k, copy)
+        if key not in self._left_ways:
+            if len(self._left_ways) > 4096:
+                self._left_ways.clear()
+            self._left_ways[key] = self._choose_left(m, n, k, copy)
+        return self._left_ways[key]
+
+    def _choose_left(self, m, n, k, copy):
+        if self.dtype != torch.bfloat16 or n > self.shares_norm_width or n % 8 or k % 64 or not 9 <= m <= 768:
+            return None
+        units, columns = self.compute_units, -(-n // 64)
+        if copy and m <= 48 and units // columns >= 6:
+            shares = min(units // columns, max(k // 512, min(4, k // 256)))
+            return (0, 0, shares) if shares >= 3 and (m > 16 or k >= 3072) else None
+        if m <= (32 if units // columns < 5 else 48) or not self.tile_products:
+            return None
+        shares = min(8, units // (-(-m // 64) * columns), k // 256)
+        return (1, 1, shares) if shares >= 2 and k < 24 * 64 * shares else None
+
+    def _left(self, way, x, w, bias, residual, m, n, k, room, tile=0, shares=0):
+        """The product with its shares of K left apart (0: the tile and the shares that the product chooses itself)."""
         out = torch.empty(m, n, dtype=torch.float32, device=x.device)
         space, left = torch.empty(room, dtype=torch.float32, device=x.device), _c_int()
-        self._call("gemm", "tnx_gemm_left", way, _ptr(x), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out), m, n, k, _ptr(space), room,
+        self._call("gemm", "tnx_gemm_left", way, _ptr(x), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out), m, n, k, _ptr(space), room, tile, shares,
                    ctypes.addressof(left), _stream(),
                    work=lambda: self._product_work(m, n, k, x.element_size(), w.element_size(), 4, True))
         return out if left.value == 1 else SharesLeft(self, space, left.value, bias, residual, out)
@@ -952,6 +987,11 @@ class HipOps:
                 return self._linear_whole(self.cast(x, torch.bfloat16), tiles, bias, act, n, k)
         if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
+        if leaves and w.dtype == torch.bfloat16 and not force_tiled:
+            way = self._way_to_leave(m, n, k, tiles is not None)
+            if way is not None and (_ptr(x) | _ptr(w) | _ptr(residual)) % 16 == 0:
+                way, tile, shares = way
+                return self._left(way, self.cast(x, torch.bfloat16), w if way else tiles, bias, residual, m, n, k, shares * m * n, tile, shares)
         if self._some_rows_product(m, n, k, w, tiles, residual, out_f32, force_tiled):
             # decode batches of 33 to 128 requests, a float32 result: our kernel for some rows
             shares = max(1, min(self.compute_units // -(-n // 64), k // 512))       # as the kernel shares K out

@@ -70,11 +70,14 @@ class PreNormBlock(Block):
         return x, norm.deferred(x) if deferred else norm.forward(x, False, True)[1]
 
     def forward(self, stream: Stream, ctx, cache) -> Stream:
+        # (a norm that is deferred reads a sum that is made)
         onto = self.mixer_norm.ops.onto if self.leaves_shares else None
+        behind_mixer = onto if ctx.num_tokens > self.feed_forward_norm_rows else None
+        behind = onto if ctx.num_tokens > self.mixer_norm_rows else None
         x, h = self._normed(self.mixer_norm, stream.x, ctx.num_tokens <= self.mixer_norm_rows)
-        x = debug.tap("after_mixer", self.mixer.forward(h, ctx, cache, onto(x) if onto else x))
+        x = debug.tap("after_mixer", self.mixer.forward(h, ctx, cache, behind_mixer(x) if behind_mixer else x))
         x, h = self._normed(self.feed_forward_norm, x, ctx.num_tokens <= self.feed_forward_norm_rows)
-        return Stream(self.feed_forward.forward(h, ctx, onto(x) if onto else x), None)
+        return Stream(self.feed_forward.forward(h, ctx, behind(x) if behind else x), None)
 
 
 @register_block("post_norm")
