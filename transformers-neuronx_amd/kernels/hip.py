@@ -384,14 +384,17 @@ class SharesLeft:
         """(the sum, its norm in `dtype`)."""
         out, f32 = self.out, dtype == torch.float32
         m, n = out.shape
+        add, onto, scale, shift = _ptr(self.bias), _ptr(self.residual), _ptr(weight), _ptr(bias)
         if (self.added or n > self.ops.shares_norm_width or n % 4 or (not f32 and dtype != torch.bfloat16)
-                or any((_ptr(a) or 0) % 16 for a in (self.bias, self.residual, weight, bias))):
+                or ((add or 0) | (onto or 0) | (scale or 0) | (shift or 0)) % 16):
             return self.settled(), self.ops.layernorm(out, weight, bias, eps, dtype, False, True, center)[1]
-        self.ops._want_norm(out, weight, bias)
+        for v, name in ((weight, "norm weight"), (bias, "norm bias")):
+            if v is not None:
+                _want(v, name, torch.float32, (n,))
         h = torch.empty(m, n, dtype=dtype, device=out.device)
-        self.ops._call("elementwise", "tnx_shares_norm", _ptr(self.shares), self.count, _ptr(self.bias), _ptr(self.residual), _ptr(out),
-                       _ptr(weight), _ptr(bias), float(eps), _ptr(h) if f32 else None, None if f32 else _ptr(h), m, n,
-                       int(bool(center)), _stream(),
+        at = h.data_ptr()
+        self.ops._call("elementwise", "tnx_shares_norm", self.shares.data_ptr(), self.count, add, onto, out.data_ptr(), scale, shift, eps,
+                       at if f32 else None, None if f32 else at, m, n, 1 if center else 0, _stream(),
                        work=lambda: (f"{m}x{n}", m * n * (4 * self.count + 8 + h.element_size()), 0.0))
         self._done()
         return out, h
@@ -786,12 +789,10 @@ class HipOps:
           four shares at most (39 rows 3,072 x 3,072, five: 11.5 / 11.6).
         Tiles of 128 x 128 with shares where the library has no shares were a loss as often as a gain (640 rows 2,048 x 2,048 18.9 /
         23.2)."""
-        key = (m, n, k, copy)
-        if key not in self._left_ways:
-            if len(self._left_ways) > 4096:
-                self._left_ways.clear()
-            self._left_ways[key] = self._choose_left(m, n, k, copy)
-        return self._left_ways[key]
+        if len(self._left_ways) > 4096:
+            self._left_ways.clear()
+        self._left_ways[m, n, k, copy] = way = self._choose_left(m, n, k, copy)
+        return way
 
     def _choose_left(self, m, n, k, copy):
         if self.dtype != torch.bfloat16 or n > self.shares_norm_width or n % 8 or k % 64 or not 9 <= m <= 768:
@@ -988,7 +989,10 @@ class HipOps:
         if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
         if leaves and w.dtype == torch.bfloat16 and not force_tiled:
-            way = self._way_to_leave(m, n, k, tiles is not None)
+            copy = tiles is not None
+            way = self._left_ways.get((m, n, k, copy), 0)
+            if way == 0:
+                way = self._way_to_leave(m, n, k, copy)
             if way is not None and (_ptr(x) | _ptr(w) | _ptr(residual)) % 16 == 0:
                 way, tile, shares = way
                 return self._left(way, self.cast(x, torch.bfloat16), w if way else tiles, bias, residual, m, n, k, shares * m * n, tile, shares)
