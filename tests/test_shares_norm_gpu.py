@@ -35,6 +35,8 @@ def test_sizes(shares, tokens, width, dtype):
         norm = hip.layernorm(want, w, b, 1e-5, dtype, False, True, center)[1]
         x, h = left().normed(w, b, 1e-5, dtype, center)
         assert torch.equal(x, want) and torch.equal(h, norm) and h.dtype == dtype
+        x, h = left().normed(w, b, 1e-5, dtype, center, alone=True)
+        assert torch.equal(x, hip.layernorm(want, w, b, 1e-5, dtype, True, False, center)[0]) and torch.equal(h, norm)
         x, h = whole.normed(w, b, 1e-5, dtype, center)                          # one that was added already
         assert x is want and torch.equal(h, norm)
 
@@ -95,8 +97,8 @@ def test_ways(m, n, k, way):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
-def test_through_the_model(tmp_path, dtype):
+@pytest.mark.parametrize("dtype,before", [("bfloat16", True), ("float32", True), ("bfloat16", False), ("float32", False)])
+def test_through_the_model(tmp_path, dtype, before):
     """Prompts, a step of both kinds and recorded decode steps: the same logits, bit for bit, and sums that are looked at are made."""
     from transformers_neuronx_amd import debug
     from transformers_neuronx_amd.config.engine_config import EngineConfig
@@ -104,7 +106,7 @@ def test_through_the_model(tmp_path, dtype):
     from transformers_neuronx_amd.opt.config import OPTConfig
     from transformers_neuronx_amd.weights import write_random_model
     raw = dict(architectures=["OPTForCausalLM"], model_type="opt", vocab_size=640, hidden_size=1024, num_hidden_layers=3, num_attention_heads=16,
-               ffn_dim=4096, max_position_embeddings=512, word_embed_proj_dim=1024, do_layer_norm_before=True, activation_function="relu",
+               ffn_dim=4096, max_position_embeddings=512, word_embed_proj_dim=1024, do_layer_norm_before=before, activation_function="relu",
                enable_bias=True, layer_norm_elementwise_affine=True, init_std=0.04)
     write_random_model(OPTConfig.from_dict(raw), str(tmp_path), 3, dtype=dtype)
     logits, made = {}, []
@@ -119,7 +121,7 @@ def test_through_the_model(tmp_path, dtype):
             looked_at = runner
         else:
             runner.ops.onto = lambda x: x
-        assert all(layer.block.leaves_shares for layer in runner.model.layers)
+        assert all(layer.block.leaves_shares if before else layer.block.norms_shares for layer in runner.model.layers)
         n = 40
         runner.step([StepEntry(r, [5 + i + r for i in range(9)], []) for r in range(1, n)])
         steps = [[StepEntry(0, [5 + i % 600 for i in range(333)], [332])]]
@@ -129,7 +131,8 @@ def test_through_the_model(tmp_path, dtype):
     assert torch.equal(logits[True], logits[False])
     # (sums in another order, rounded to bfloat16 between the products)
     assert float((logits["by the rule"] - logits[False]).norm() / logits[False].norm()) < (0.02 if dtype == "bfloat16" else 1e-6)
-    assert "tnx_shares_norm" in made and "tnx_gemm_shares_sum" in made      # (the last sum is the head's, a norm of its own)
+    assert "tnx_shares_norm" in made
+    assert ("tnx_gemm_shares_sum" in made) == before             # (the last sum is the head's, which has a norm of its own)
     del made[:]
     with debug.debug_context() as kept:
         looked_at.step([StepEntry("more", [5 + i for i in range(60)], [59])])

@@ -162,13 +162,13 @@ layernorm_kernel(const float* __restrict__ x, const float* __restrict__ weight, 
 typedef __attribute__((ext_vector_type(4))) float f4;
 
 // The sum of a product's shares of K with its bias and residual, and the norm of the sum, in one launch where there were two that
-// each waited for memory. `partial` is [shares][tokens][width]; `sum` gets the row, `out_f32` or `out_bf16` its norm. A block has a
+// each waited for memory. `partial` is [shares][tokens][width]; `sum` gets the row or is null, `out_f32` and `out_bf16` its norm, one or both. A block has a
 // row, a thread four elements of it (256 PER threads), so that of few rows, too, all is asked for at once (AT_ONCE shares; more of
 // them in turns): what bounds it is that one compute unit brings a row's shares, 60 to 100 KB. They are added in their order, then
 // bias, then residual, and the statistics are made from LDS in the order of `layernorm_kernel`: the sum's and the norm's own kernels give
 // the same bits. 32 rows of 2,560 and six shares: 4.0 and 4.8 us apart, 4.8 so (5.5 with 256 threads a row, the shares in two turns);
 // prompt 1.3b of 333 tokens 2,601 / 2,534, serving 24 requests 53,878 / 53,129, before and after.
-template <int PER, int AT_ONCE, bool F32>
+template <int PER, int AT_ONCE>
 __global__ void __launch_bounds__(256 * PER)
 shares_norm_kernel(const float* __restrict__ partial, int shares, const float* __restrict__ add, const float* __restrict__ residual,
                    float* __restrict__ sum, const float* __restrict__ weight, const float* __restrict__ bias, float eps,
@@ -198,7 +198,7 @@ shares_norm_kernel(const float* __restrict__ partial, int shares, const float* _
       if (from + c < shares) v += part[c];
   }
   v = (v + ad) + on;
-  if (inside) ((f4*)sum)[own] = v;
+  if (inside && sum) ((f4*)sum)[own] = v;
   row[i] = inside ? v : none;
   // the block's sum of what threads t of four waves hold; every wave beyond the fourth makes that of a wave below again
   auto sum_of_four = [&](float x) {
@@ -231,9 +231,8 @@ shares_norm_kernel(const float* __restrict__ partial, int shares, const float* _
   const float rstd = rsqrtf(var + eps);
   if (!inside) return;
   const f4 y = ((v - mean) * rstd) * gw + gb;
-  if (F32) {
-    ((f4*)out_f32)[own] = y;
-  } else {
+  if (out_f32) ((f4*)out_f32)[own] = y;
+  if (out_bf16) {
     b4 o;
     o.x = (bf16_t)y.x; o.y = (bf16_t)y.y; o.z = (bf16_t)y.z; o.w = (bf16_t)y.w;
     ((b4*)out_bf16)[own] = o;
@@ -301,27 +300,25 @@ extern "C" int tnx_layernorm(const float* x, const float* weight, const float* b
   return 0;
 }
 
-// `center`, `weight` and `bias` as in `tnx_layernorm`; the norm goes to `out_f32` or `out_bf16`. Rows of up to 4,096 in fours, and
+// `center`, `weight` and `bias` as in `tnx_layernorm`; the norm goes to `out_f32`, `out_bf16` or both; `sum` is optional. Rows of up to 4,096 in fours, and
 // everything at multiples of 16 bytes.
 extern "C" int tnx_shares_norm(const float* partial, int shares, const float* add, const float* residual, float* sum, const float* weight,
                                const float* bias, float eps, float* out_f32, void* out_bf16, int tokens, int width, int center,
                                hipStream_t stream) {
   TNX_REQUIRE(tokens > 0 && width > 0 && width % 4 == 0 && width <= 4096 && shares > 1 && eps > 0.f, "shares_norm: bad sizes");
-  TNX_REQUIRE(partial && sum && (out_f32 == nullptr) != (out_bf16 == nullptr) && (weight != nullptr || bias == nullptr),
-              "shares_norm: one result, and a bias comes with a weight");
+  TNX_REQUIRE(partial && (out_f32 || out_bf16) && (weight != nullptr || bias == nullptr),
+              "shares_norm: a result, and a bias comes with a weight");
   TNX_REQUIRE((((uintptr_t)partial | (uintptr_t)add | (uintptr_t)residual | (uintptr_t)sum | (uintptr_t)weight | (uintptr_t)bias |
                 (uintptr_t)out_f32 | (uintptr_t)out_bf16) & 15) == 0, "shares_norm: operands must be 16-byte aligned");
-#define SHARES_NORM(PER, AT, F)                                                                                                      \
-  shares_norm_kernel<PER, AT, F><<<tokens, 256 * PER, 0, stream>>>(partial, shares, add, residual, sum, weight, bias, eps, out_f32,  \
-                                                                   (bf16_t*)out_bf16, width, center)
-#define SHARES_NORM_AT(PER, F)                                                                                 \
-  if (shares <= 2) SHARES_NORM(PER, 2, F); else if (shares <= 4) SHARES_NORM(PER, 4, F); else SHARES_NORM(PER, 8, F)
-#define SHARES_NORM_F(PER) if (out_f32) { SHARES_NORM_AT(PER, true); } else { SHARES_NORM_AT(PER, false); }
-  if (width <= 1024) { SHARES_NORM_F(1); }
-  else if (width <= 2048) { SHARES_NORM_F(2); }
-  else if (width <= 3072) { SHARES_NORM_F(3); }
-  else { SHARES_NORM_F(4); }
-#undef SHARES_NORM_F
+#define SHARES_NORM(PER, AT)                                                                                                      \
+  shares_norm_kernel<PER, AT><<<tokens, 256 * PER, 0, stream>>>(partial, shares, add, residual, sum, weight, bias, eps, out_f32,  \
+                                                                (bf16_t*)out_bf16, width, center)
+#define SHARES_NORM_AT(PER) \
+  if (shares <= 2) SHARES_NORM(PER, 2); else if (shares <= 4) SHARES_NORM(PER, 4); else SHARES_NORM(PER, 8)
+  if (width <= 1024) { SHARES_NORM_AT(1); }
+  else if (width <= 2048) { SHARES_NORM_AT(2); }
+  else if (width <= 3072) { SHARES_NORM_AT(3); }
+  else { SHARES_NORM_AT(4); }
 #undef SHARES_NORM_AT
 #undef SHARES_NORM
   TNX_CHECK_LAUNCH("shares_norm");

@@ -380,24 +380,29 @@ class SharesLeft:
             self._done()
         return self.out
 
-    def normed(self, weight, bias, eps, dtype, center):
-        """(the sum, its norm in `dtype`)."""
+    def normed(self, weight, bias, eps, dtype, center, alone=False):
+        """(the sum, its norm in `dtype`); with `alone` the sum is not kept: (its norm in float32, in `dtype`)."""
         out, f32 = self.out, dtype == torch.float32
         m, n = out.shape
         add, onto, scale, shift = _ptr(self.bias), _ptr(self.residual), _ptr(weight), _ptr(bias)
         if (self.added or n > self.ops.shares_norm_width or n % 4 or (not f32 and dtype != torch.bfloat16)
                 or ((add or 0) | (onto or 0) | (scale or 0) | (shift or 0)) % 16):
-            return self.settled(), self.ops.layernorm(out, weight, bias, eps, dtype, False, True, center)[1]
+            x, h = self.ops.layernorm(self.settled(), weight, bias, eps, dtype, alone, True, center)
+            return (x if alone else out), h
         for v, name in ((weight, "norm weight"), (bias, "norm bias")):
             if v is not None:
                 _want(v, name, torch.float32, (n,))
         h = torch.empty(m, n, dtype=dtype, device=out.device)
-        at = h.data_ptr()
-        self.ops._call("elementwise", "tnx_shares_norm", self.shares.data_ptr(), self.count, add, onto, out.data_ptr(), scale, shift, eps,
-                       at if f32 else None, None if f32 else at, m, n, 1 if center else 0, _stream(),
+        # (the product has made nothing of `out` yet: alone, the norm's float32 result lies there)
+        x = (h if f32 else out) if alone else out
+        self.ops._call("elementwise", "tnx_shares_norm", self.shares.data_ptr(), self.count, add, onto, None if alone else out.data_ptr(),
+                       scale, shift, eps, h.data_ptr() if f32 else out.data_ptr() if alone else None, None if f32 else h.data_ptr(), m, n,
+                       1 if center else 0, _stream(),
                        work=lambda: (f"{m}x{n}", m * n * (4 * self.count + 8 + h.element_size()), 0.0))
         self._done()
-        return out, h
+        if alone:
+            self.out = None                     # (nobody else may ask for the sum)
+        return x, h
 
     def _done(self):
         self.added, self.shares, self.residual = True, None, None
@@ -771,7 +776,7 @@ class HipOps:
 
     @staticmethod
     def onto(x):
-        """The residual of a product whose result goes to a norm, and to a sum behind that norm, and nowhere else."""
+        """The residual of a product whose result a norm reads next, before anyone else does."""
         return x if debug.tapping() else Onto(x)
 
     def _way_to_leave(self, m, n, k, copy):

@@ -97,6 +97,7 @@ class PostNormBlock(Block):
     # (`residual_to_product`), and an arrangement of its own around the same sums gets tensors.
     norms_between = False
     between_rows = -1              # and few are so many
+    norms_shares = False           # in steps of more, the norm's launch adds the shares of the sum's product (`HipOps.onto`)
 
     def after_load(self) -> None:
         norms, parts = (self.mixer_norm, self.feed_forward_norm), (self.mixer, self.feed_forward)
@@ -105,6 +106,7 @@ class PostNormBlock(Block):
                               and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
                               and all(_is_its_fused_form(n) for n in norms))
         self.between_rows = self.mixer_norm.ops.norm_beside_rows if self.norms_between else -1
+        self.norms_shares = self.norms_between and hasattr(self.mixer_norm.ops, "onto")
         self.in_one = _layer_parts(self, PostNormBlock) if self.norms_between else None
 
     def norms_in_one(self, before):
@@ -132,6 +134,13 @@ class PostNormBlock(Block):
                 if not hasattr(norm, "fused_form") or norm.fused_form()[2]:
                     raise ValueError("the norm behind a sum with a factor is one that only scales (rms_norm)")
 
+    def _behind(self, norm, t):
+        """(float32, compute dtype) of the norm behind a sum, of a product that may have left its shares."""
+        if self.norms_shares and hasattr(type(t), "normed"):
+            weight, bias, center, eps = norm.fused_form()
+            return t.normed(weight, bias, eps, norm.dtype, center, alone=True)
+        return norm.forward(t, True, True)
+
     def _join(self, norm, x, results):
         weight, _, _, eps = norm.fused_form()
         return self.ops.join_norm(x, self.alpha, results, weight, eps, self.dtype)
@@ -153,11 +162,10 @@ class PostNormBlock(Block):
             debug.tap("after_mixer", x)
             return Stream(*self._between(self.feed_forward_norm, self.feed_forward.forward(h, ctx, x)))
         h = stream.compute if stream.compute is not None else self.mixer_norm.ops.cast(stream.x, self.mixer_norm.dtype)
-        t = self.mixer.forward(h, ctx, cache, stream.x)
-        x, h = self.mixer_norm.forward(t, True, True)
+        onto = self.mixer_norm.ops.onto if self.norms_shares else None
+        x, h = self._behind(self.mixer_norm, self.mixer.forward(h, ctx, cache, onto(stream.x) if onto else stream.x))
         debug.tap("after_mixer", x)
-        t = self.feed_forward.forward(h, ctx, x)
-        x, h = self.feed_forward_norm.forward(t, True, True)
+        x, h = self._behind(self.feed_forward_norm, self.feed_forward.forward(h, ctx, onto(x) if onto else x))
         return Stream(x, h)
 
 
