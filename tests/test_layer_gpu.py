@@ -185,6 +185,55 @@ def test_layers_in_one_launch(case, block):
             assert float((a - b).norm() / b.norm()) <= (2e-6 if dtype == F32 else 2 * 0.005 + 2 ** -9)
 
 
+def _ready(dtype, width, inner, held, seed, layers=3, page_size=64, block="pre_norm"):
+    """Layers, and a function that runs them in one launch over caches that no launch has written: (result, pages)."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops = HipOps(dtype, DEV)
+    made = [_layer(ops, dtype, width, inner, block, "relu", True, seed + i)[0] for i in range(layers)]
+    x = (torch.randn(len(held), width, generator=torch.Generator().manual_seed(seed)) * 2.0).to(DEV)
+    steps = [_step(ops, dtype, held, width, page_size, seed, i) for i in range(layers)]
+    return ops, lambda: ops.settled(_in_one(ops, made, Stream(x, x.to(dtype)), steps).x), [p for _, c, _ in steps for p in (c.k_pages, c.v_pages)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("joined", [1, 5, 16, 40, 127])
+@pytest.mark.parametrize("dtype,width,inner,held", [(BF16, 1024, 4096, [1, 900, 64, 129, 513, 63, 10, 200]), (BF16, 640, 1152, [700, 3]),
+                                                    (F32, 1024, 4096, [65, 0, 33, 32, 300, 31, 1, 96]), (F32, 896, 3584, [300, 20])])
+def test_fewer_blocks_do_the_same(dtype, width, inner, held, joined):
+    """A launch of which only some blocks found room: tiles in several groups, K in chunks for each, several (row, head, share) a block.
+    The sums are the same ones in the same order: the same bits, in the result and in every layer's pages."""
+    ops, run, pages = _ready(dtype, width, inner, held, 7)
+    print(f"fewer {dtype} {width} {inner} {held} {joined}", flush=True)
+    want = run().clone()
+    kept = [p.clone() for p in pages]
+    ops.layer_join_most = joined
+    got = run()
+    ops.raise_if_lost()
+    assert torch.equal(got, want) and bool(torch.isfinite(want).all())
+    assert all(torch.equal(torch.nan_to_num(a), torch.nan_to_num(b)) for a, b in zip(pages, kept))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtypes", [(F32,) * 6, (BF16,) * 8, (F32, BF16) * 4])
+def test_many_launches_at_a_time(dtypes):
+    """More launches on streams of their own than have room together, each with its own engine: every one gives what it gives alone."""
+    engines = [_ready(dtype, 1024, 4096, [40 + i, 3, 65 * (i % 2)], 20 + i) for i, dtype in enumerate(dtypes)]
+    print(f"at a time {dtypes}", flush=True)
+    alone = [run().clone() for _, run, _ in engines]
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in engines]
+    results = []
+    for _ in range(12):
+        for (_, run, _), stream in zip(engines, streams):
+            with torch.cuda.stream(stream):
+                results.append(run())
+    torch.cuda.synchronize()
+    for i, got in enumerate(results):
+        assert torch.equal(got, alone[i % len(engines)]), i
+    for ops, _, _ in engines:
+        ops.raise_if_lost()
+
+
 @pytest.mark.gpu
 def test_layers_in_one_launch_through_the_model(tmp_path):
     """A model of such layers: recorded steps (the launch replayed, other steps between) give what the launches apart give, bit for bit

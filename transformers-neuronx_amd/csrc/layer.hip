@@ -10,12 +10,13 @@
 // (without them 18.4 us a layer for 16.8). us a layer, launches apart / so: bfloat16, 1,024 columns, 1 request of 100 tokens 23.1 / 16.9, 8 of
 // 100 26.5 / 20.2, 1 of 1,500 27.7 / 20.2, 8 of 2,000 41.9 / 36.6; float32 3 of 70 34.4 / 26.8, 8 of 100 45.3 / 41.3, 4 of 1,000 54.2 / 36.0.
 //
-// Waiting blocks need the blocks they wait for on the chip, those of one launch and no others. It has a block that computes for every
-// second compute unit, and a unit has room for two of the bfloat16 kernel's (512 threads of 128 registers, 74 KB of LDS) and one of
-// the float32 kernel's: as many as four and two such launches at a time leave a place free for as long as one of them is not complete,
-// and everything else that runs beside them, the blocks that fetch ahead among it, ends by itself. (Streams of one process come to
-// four hardware queues.) A wait ends after `WAIT_MOST` questions all the same, some seconds: the block then goes on with results that are
-// no numbers and says so in `failed`, and the host's next step raises it.
+// A block waits only for blocks that run beside it: the layers are shared out among those that have joined (`join`), and who joins
+// is on the chip and stays. A launch has a block that computes for every second compute unit (a unit has room for two of the bfloat16
+// kernel's, 512 threads of 128 registers and 74 KB of LDS, and one of the float32 kernel's); where other launches leave no room for all of
+// them (several engines on streams or in processes, units masked out), those that came do the work of all, and those that come later
+// end at once. Blocks that fetch ahead wait for `AHEAD_TICKS` at most and then end as well. So whatever else runs, and however many
+// such launches, every wait has its answer. It ends after `wait_most` questions all the same, some seconds: the block then goes on with
+// results that are no numbers and says so in `failed`, which the host looks at where tokens reach it.
 #include "common.h"
 
 TNX_DEFINE_ERROR_API
@@ -27,7 +28,8 @@ constexpr int MOST_ROWS = 8;
 constexpr int HD = 64;                        // the head size
 constexpr int COLS = 8;                       // columns of a product's tile: its 8 waves share K
 constexpr unsigned NOT_YET = 0xFFFFFFFFu;     // as a float, and as two bfloat16, no number, and none that a result is stored as
-constexpr int WAIT_MOST = 1 << 22;
+constexpr int CLOSED = 1 << 16;               // added to the number of blocks that asked to join, by who closes the launch to others
+constexpr long long JOIN_TICKS = 1000, AHEAD_TICKS = 20000;     // of 10 ns
 
 typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
 typedef __attribute__((ext_vector_type(2))) float f32x2;
@@ -58,6 +60,7 @@ struct Layers {
   float scale, eps;
   int rows, width, inner_width, act, center, residual_normed, first_normed;      // `first_normed` 0: the first layer's rows come as they are
   int table_width, page_shift, num_pages, page_pad, splits, chunk, layers, blocks;
+  int join_most, wait_most;      // as many blocks at most join; questions of a wait
   LayerOf of[MOST_LAYERS];
 };
 static_assert(sizeof(Layers) <= 4096, "what a launch may take");
@@ -88,6 +91,43 @@ __device__ __forceinline__ void publish(unsigned* p, unsigned v) {
 __device__ __forceinline__ void publish(unsigned* p, unsigned v, unsigned next) {
   __hip_atomic_store((unsigned long long*)p, (unsigned long long)next << 32 | v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+// Which of how many blocks this one is: the members of a launch, numbered from 0; -1: the launch goes on without it.
+struct Member {
+  int number, of;
+};
+
+// Asked by one thread. Two words behind those of the layers (-1 before the launch, as all of them): how many blocks have asked, and how
+// many have joined where not all came. All have joined once as many have asked. Who has waited so long without another having come that
+// going on with those there are would have lost no more (10 us a layer; a launch of 1 / n of the blocks takes n times as long) closes
+// the launch to others and says how many there are by then: all of those are on the chip, and whoever asks later sees that it is closed.
+__device__ __forceinline__ unsigned* gate_of(Args a) { return a->words + (size_t)a->layers * a->at.all; }
+__device__ __forceinline__ unsigned ask_in(Args a, unsigned add) {
+  return __hip_atomic_fetch_add(gate_of(a), add, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1;
+}
+__device__ __forceinline__ Member join(Args a, unsigned number) {       // `number`: what `ask_in(a, 1)` said
+  const unsigned most = a->join_most;
+  if (number >= most) return {-1, 0};                    // (also where it is closed: `CLOSED` and more)
+  unsigned came = number + 1;
+  long long since = wall_clock64();
+#pragma unroll 1
+  for (;;) {
+    const unsigned long long both = __hip_atomic_load((unsigned long long*)gate_of(a), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const unsigned asked = (unsigned)both + 1, joined = (unsigned)(both >> 32);
+    const unsigned members = asked < CLOSED && asked >= most ? most : joined;
+    // (all of them: numbered as blocks go to XCDs, for what was fetched ahead)
+    if (members != NOT_YET) return {(int)members == a->blocks ? (int)blockIdx.x : (int)number, (int)members};
+    if (asked >= CLOSED) continue;                       // (who closed it says so next)
+    const long long now = wall_clock64();
+    if (asked != came) {
+      came = asked, since = now;
+    } else if ((now - since) * came > JOIN_TICKS * a->layers * a->blocks) {
+      const unsigned all = ask_in(a, CLOSED);
+      if (all < CLOSED) __hip_atomic_store(gate_of(a) + 1, min(all, most), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+}
+
 __device__ __forceinline__ unsigned float_word(float v) {
   const unsigned u = __float_as_uint(v);
   return u == NOT_YET ? 0x7FC00000u : u;
@@ -108,11 +148,11 @@ struct Shared {
   }
 };
 
-// Asks for N x 16 bytes (`word(i)`: the first of the four words of load i) until all are there.
+// Asks for N x 16 bytes (`word(i)`: the first of the four words of load i) until all are there, `most` times at most.
 template <int N, typename Word>
-__device__ __forceinline__ void await(const Shared& from, u32x4 (&v)[N], Word word, bool& lost) {
+__device__ __forceinline__ void await(const Shared& from, u32x4 (&v)[N], Word word, int most, bool& lost) {
 #pragma unroll 1
-  for (int asked = 0; asked < WAIT_MOST; ++asked) {
+  for (int asked = 0; asked < most; ++asked) {
     asm volatile("" ::: "memory");
 #pragma unroll
     for (int i = 0; i < N; ++i) v[i] = from.four(word(i));
@@ -184,11 +224,11 @@ __device__ __forceinline__ void norm_row(Args a, const float* weight, const floa
 template <typename T, int SC, int RT>
 struct Weights {
   u32x4 v[SC][RT][Kind<T>::LOADS];
-  // steps 8 (chunk * SC + sc) + wave of tiles blockIdx.x + gridDim.x (group * RT + j); what is beyond the end reads the last again (a load
+  // steps 8 (chunk * SC + sc) + wave of tiles me.number + me.of (group * RT + j); what is beyond the end reads the last again (a load
   // that depended on anything would keep these registers from layer to layer)
-  __device__ __forceinline__ void one(const T* w, int K, int tiles, int blocks, int group, int chunk, int sc, int j) {
+  __device__ __forceinline__ void one(const T* w, int K, int tiles, Member me, int group, int chunk, int sc, int j) {
     const int tid = thread(), lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int tile = min((int)(blockIdx.x + blocks * (group * RT + j)), tiles - 1), step = min(NW * (chunk * SC + sc) + wave, K / 128 - 1);
+    const int tile = min(me.number + me.of * (group * RT + j), tiles - 1), step = min(NW * (chunk * SC + sc) + wave, K / 128 - 1);
     if constexpr (sizeof(T) == 2) {
       // rows 0-7 of the matrix instruction's operand: the tile's columns over the first half of the step's K, rows 8-15 the
       // same columns over the second
@@ -202,11 +242,11 @@ struct Weights {
       for (int l = 0; l < 4; ++l) v[sc][j][l] = *(const u32x4*)(at + 32 * l);
     }
   }
-  __device__ __forceinline__ void ask(const T* w, int K, int tiles, int blocks, int group, int chunk) {
+  __device__ __forceinline__ void ask(const T* w, int K, int tiles, Member me, int group, int chunk) {
 #pragma unroll
     for (int sc = 0; sc < SC; ++sc)
 #pragma unroll
-      for (int j = 0; j < RT; ++j) one(w, K, tiles, blocks, group, chunk, sc, j);
+      for (int j = 0; j < RT; ++j) one(w, K, tiles, me, group, chunk, sc, j);
   }
 };
 
@@ -294,27 +334,27 @@ struct Sums<float, RT, ROWS> {
 // LDS for all when it returns; `early(mine, n, m)`: what the end adds, asked for before (`first`: of the first tiles, by the caller,
 // before it waits for anything); `put(v0, v1, n, m, early)`: columns n, n + 1 of row m.
 template <int RT, typename Early>
-__device__ __forceinline__ auto of_first_tiles(Args a, int columns, Early early) {
-  const int tid = thread(), tile = blockIdx.x + a->blocks * (tid >> 5), m = (tid >> 2) & 7;
+__device__ __forceinline__ auto of_first_tiles(Args a, Member me, int columns, Early early) {
+  const int tid = thread(), tile = me.number + me.of * (tid >> 5), m = (tid >> 2) & 7;
   return early(tid < 32 * RT && tile < columns / COLS && m < a->rows, tile * COLS + 2 * (tid & 3), m);
 }
 template <typename T, int SC, int RT, int ROWS, typename First, typename Early, typename Stage, typename Put>
-__device__ __forceinline__ void product(Args a, const T* w, int K, int columns, int chunk_k, Weights<T, SC, RT>& asked, const T* rows, int pitch,
+__device__ __forceinline__ void product(Args a, Member me, const T* w, int K, int columns, int chunk_k, Weights<T, SC, RT>& asked, const T* rows, int pitch,
                                         float* red, First first, Early early, Stage stage, Put put) {
   const int tid = thread(), wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int blocks = a->blocks, tiles = columns / COLS, steps = K / 128, turns = (steps + NW * SC - 1) / (NW * SC);
+  const int tiles = columns / COLS, steps = K / 128, turns = (steps + NW * SC - 1) / (NW * SC);
   typedef Sums<T, RT, ROWS> Made;
-  if ((int)blockIdx.x >= tiles) return;
+  if (me.number >= tiles) return;
   // the thread's two columns and row of the group's tiles: RT x 8 rows x 4 pairs
   const int j = tid >> 5, m = (tid >> 2) & 7, c = 2 * (tid & 3);
 #pragma unroll 1
   for (int group = 0;; ++group) {
-    const int tile = blockIdx.x + blocks * (group * RT + j), n = tile * COLS + c;
+    const int tile = me.number + me.of * (group * RT + j), n = tile * COLS + c;
     const bool mine = tid < 32 * RT && tile < tiles && m < a->rows;
     const First extra = group == 0 ? first : early(mine, n, m);
     Made sums;
     sums.clear();
-    const bool more = (int)(blockIdx.x + blocks * (group + 1) * RT) < tiles;
+    const bool more = me.number + me.of * (group + 1) * RT < tiles;
 #pragma unroll 1
     for (int k0 = 0; k0 < K; k0 += chunk_k) {
       if (group == 0 || chunk_k < K) stage(k0);
@@ -326,8 +366,8 @@ __device__ __forceinline__ void product(Args a, const T* w, int K, int columns, 
           const int step = NW * (turn * SC + sc) + wave;
           if (step < steps) sums.add(asked, sc, rows, pitch, step * 128 - k0, a->rows);
         }
-        if (turn + 1 < turns) asked.ask(w, K, tiles, blocks, group, turn + 1);
-        else if (more) asked.ask(w, K, tiles, blocks, group + 1, 0);
+        if (turn + 1 < turns) asked.ask(w, K, tiles, me, group, turn + 1);
+        else if (more) asked.ask(w, K, tiles, me, group + 1, 0);
       }
     }
     sums.leave(red + wave * RT * 64, a->rows);
@@ -346,7 +386,8 @@ __device__ __forceinline__ void product(Args a, const T* w, int K, int columns, 
 
 // Words of `count` x 16 bytes a row into LDS, as they came.
 template <typename T>
-__device__ __forceinline__ void stage_words(const unsigned* from, int words_row, int word0, int words, int m_rows, T* rows, int pitch, bool& lost) {
+__device__ __forceinline__ void stage_words(const unsigned* from, int words_row, int word0, int words, int m_rows, T* rows, int pitch, int most,
+                                            bool& lost) {
   const Shared src(from);
   const int per_row = words / 4, all = per_row * m_rows;
   const int tid = thread();
@@ -359,7 +400,7 @@ __device__ __forceinline__ void stage_words(const unsigned* from, int words_row,
       row[i] = q / per_row, four[i] = q - row[i] * per_row;
     }
     u32x4 v[2];
-    await<2>(src, v, [&](int i) { return row[i] * words_row + word0 + 4 * four[i]; }, lost);
+    await<2>(src, v, [&](int i) { return row[i] * words_row + word0 + 4 * four[i]; }, most, lost);
 #pragma unroll
     for (int i = 0; i < 2; ++i)
       if (at + i * THREADS < all) *(u32x4*)((char*)(rows + row[i] * pitch) + 16 * four[i]) = v[i];
@@ -435,7 +476,7 @@ __device__ __forceinline__ void attend(Args a, ArgsOf of, const unsigned* words,
   if (t < end) load(t, item.page);
   const Shared mine(words + a->at.qkv + (size_t)row * (3 * a->width / 2));
   u32x4 qw[2];
-  await<2>(mine, qw, [&](int ks) { return h * (HD / 2) + 16 * ks + 4 * g; }, lost);
+  await<2>(mine, qw, [&](int ks) { return h * (HD / 2) + 16 * ks + 4 * g; }, a->wait_most, lost);
   bf16x8 qf[2];
 #pragma unroll
   for (int ks = 0; ks < 2; ++ks) qf[ks] = __builtin_bit_cast(bf16x8, qw[ks]);
@@ -499,7 +540,7 @@ __device__ __forceinline__ void attend(Args a, ArgsOf of, const unsigned* words,
     u32x4 kv[6];
     await<6>(mine, kv, [&](int i) {
       return i < 2 ? a->width / 2 + h * (HD / 2) + 16 * i + 4 * g : a->width + h * (HD / 2) + 8 * (i - 2) + 4 * (g >> 1);
-    }, lost);
+    }, a->wait_most, lost);
     float s = 0.f;
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) {
@@ -560,7 +601,7 @@ __device__ __forceinline__ void attend(Args a, ArgsOf of, const unsigned* words,
   {
     u32x4 got[1];
     const int which = min(lane >> 4, 2);
-    await<1>(mine, got, [&](int) { return which * a->width + h * HD + 4 * (lane & 15); }, lost);
+    await<1>(mine, got, [&](int) { return which * a->width + h * HD + 4 * (lane & 15); }, a->wait_most, lost);
     if (lane < 16) qs[lane] = __builtin_bit_cast(f32x4, got[0]);
     else if (own && lane < 48) ((f32x4*)sm.own)[lane - 16] = __builtin_bit_cast(f32x4, got[0]);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -677,7 +718,7 @@ __device__ __forceinline__ void stage_parts(Args a, const unsigned* words, T* ro
     const int q = min(at, all - 1), pair = q / (HD / 4), d = 4 * (q % (HD / 4)), row = pair / heads;
     const int shares = shares_of(a->cached_lens[row], a->splits);
     u32x4 got[2 * N];
-    await<2 * N>(src, got, [&](int i) { return (pair * a->splits + min(i >> 1, shares - 1)) * PART + ((i & 1) ? d : HD); }, lost);
+    await<2 * N>(src, got, [&](int i) { return (pair * a->splits + min(i >> 1, shares - 1)) * PART + ((i & 1) ? d : HD); }, a->wait_most, lost);
     float top = -INFINITY;
 #pragma unroll
     for (int s = 0; s < N; ++s) top = fmaxf(top, __uint_as_float(got[2 * s].x));
@@ -760,15 +801,19 @@ __device__ __forceinline__ void touch_cache(Args a, ArgsOf of, int first, int wa
   }
 }
 
-// Until a word is there (or for as long as a wait may be).
-__device__ __forceinline__ void until(const unsigned* p) {
-  for (int asked = 0; asked < WAIT_MOST; ++asked) {
-    if (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != NOT_YET) return;
+// Whether a word came in time.
+__device__ __forceinline__ bool until(const unsigned* p) {
+  const long long since = wall_clock64();
+  while (__hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == NOT_YET) {
+    if (wall_clock64() - since > AHEAD_TICKS) return false;
     __builtin_amdgcn_s_sleep(4);
   }
+  return true;
 }
 
 // The blocks beyond the first `blocks` run ahead of those: a matrix is fetched when what is multiplied two matrices before it is there.
+// What they fetch is a hint and the place that one holds is another block's: where the layers do not come on for 0.2 ms (the keys of 8
+// requests of 2,000 tokens in float32 take a quarter of that), they end.
 template <typename T>
 __device__ void run_ahead(Args a) {
   const int helpers = (gridDim.x - a->blocks) / 8, first = (blockIdx.x - a->blocks) / 8 * NW, waves = helpers * NW;
@@ -776,15 +821,15 @@ __device__ void run_ahead(Args a) {
   for (int l = 0; l < a->layers; ++l) {
     ArgsOf of = &a->of[l];
     const unsigned *words = a->words + (size_t)l * a->at.all, *before = words - a->at.all;
-    if (l > 0) until(before + a->at.sum);
+    if (l > 0 && !until(before + a->at.sum)) return;
     touch<T>(of->w_qkv, a->width, 3 * a->width, first, waves);
     touch_vectors(a, of, first);
     touch_cache<T>(a, of, first, waves);
-    if (l > 0) until(before + a->at.inner);
+    if (l > 0 && !until(before + a->at.inner)) return;
     touch<T>(of->w_out, a->width, a->width, first, waves);
-    if (l > 0) until(before + a->at.last);
+    if (l > 0 && !until(before + a->at.last)) return;
     touch<T>(of->w_up, a->width, a->inner_width, first, waves);
-    if (l > 0) until(words + a->at.qkv);
+    if (l > 0 && !until(words + a->at.qkv)) return;
     touch<T>(of->w_down, a->inner_width, a->width, first, waves);
   }
 }
@@ -805,6 +850,7 @@ struct Block {
   float (*stat1)[2];
   float (*stat2)[2];
   Softmax* sm;
+  Member me;
   Item mine;
   bool cut;              // some row's keys are cut into shares
   bool lost;
@@ -837,7 +883,7 @@ struct Block {
   __device__ __forceinline__ void row_words(Args a, const unsigned* from, f32x4 (&v)[PER], int wave, int lane) {
     const Shared src(from + (size_t)wave * a->width);
     u32x4 got[PER];
-    await<PER>(src, got, [&](int j) { return min(256 * j + 4 * lane, a->width - 4); }, lost);
+    await<PER>(src, got, [&](int j) { return min(256 * j + 4 * lane, a->width - 4); }, a->wait_most, lost);
 #pragma unroll
     for (int j = 0; j < PER; ++j) v[j] = __builtin_bit_cast(f32x4, got[j]);
   }
@@ -849,13 +895,13 @@ struct Block {
     ArgsOf of = &a->of[layer];
     const bool normed = layer > 0 || a->first_normed;
     Weights<T, 1, RQ> asked;
-    asked.ask((const T*)of->w_qkv, W, 3 * W / COLS, a->blocks, 0, 0);
+    asked.ask((const T*)of->w_qkv, W, 3 * W / COLS, me, 0, 0);
     auto early = [&](bool mine, int n, int m) {
       Place p{{0.f, 0.f}, -1, 0};
       if (mine) p.bias = *(const f32x2*)(of->b_qkv + n), p.page = a->token_page[m], p.off = a->token_off[m];
       return p;
     };
-    const Place first = of_first_tiles<RQ>(a, 3 * W, early);
+    const Place first = of_first_tiles<RQ>(a, me, 3 * W, early);
     norm_row<T, PER>(a, of->first_weight, of->first_bias, normed, [&](f32x4 (&v)[PER], int wave, int lane) {
       if (layer == 0) {
 #pragma unroll
@@ -865,7 +911,7 @@ struct Block {
       }
     }, rows(), W + PAD, stat1);
     __syncthreads();
-    product<T, 1, RQ, ROWS>(a, (const T*)of->w_qkv, W, 3 * W, W, asked, rows(), W + PAD, red(), first, early,
+    product<T, 1, RQ, ROWS>(a, me, (const T*)of->w_qkv, W, 3 * W, W, asked, rows(), W + PAD, red(), first, early,
       [](int) {},
       [&](float v0, float v1, int n, int m, const Place& p) {
         v0 += p.bias.x, v1 += p.bias.y;
@@ -888,15 +934,15 @@ struct Block {
   __device__ __forceinline__ void mix(Args a, int layer) {
     const int items = a->rows * (a->width / HD) * a->splits;
 #pragma unroll 1
-    for (int at = blockIdx.x; at < items; at += a->blocks) {
-      if (at != (int)blockIdx.x) mine = item_of<KEYS>(a, at);
+    for (int at = me.number; at < items; at += me.of) {
+      if (at != me.number) mine = item_of<KEYS>(a, at);
       if (mine.share < 0) continue;
       attend(a, &a->of[layer], words_of(a, layer), mine, *sm, lost, T());
       __syncthreads();
       join_waves<T>(a, words_of(a, layer), mine, cut, *sm);
       __syncthreads();
     }
-    if (items > a->blocks) mine = item_of<KEYS>(a, min((int)blockIdx.x, items - 1));
+    if (items > me.of) mine = item_of<KEYS>(a, min(me.number, items - 1));
   }
 
   // attention, the output product and the first sum (whose weights are asked for before a block attends)
@@ -905,7 +951,7 @@ struct Block {
     const int layer = again(at_layer), W = a->width;
     ArgsOf of = &a->of[layer];
     Weights<T, 1, 1> asked;
-    asked.ask((const T*)of->w_out, W, W / COLS, a->blocks, 0, 0);
+    asked.ask((const T*)of->w_out, W, W / COLS, me, 0, 0);
     auto early = [&](bool mine, int n, int m) {
       Two t{};
       if (mine) {
@@ -915,11 +961,11 @@ struct Block {
       }
       return t;
     };
-    const Two first = of_first_tiles<1>(a, W, early);
+    const Two first = of_first_tiles<1>(a, me, W, early);
     mix(a, layer);
-    product<T, 1, 1, ROWS>(a, (const T*)of->w_out, W, W, W, asked, rows(), W + PAD, red(), first, early,
+    product<T, 1, 1, ROWS>(a, me, (const T*)of->w_out, W, W, W, asked, rows(), W + PAD, red(), first, early,
       [&](int) {
-        if (!cut) stage_words<T>(words_of(a, layer) + a->at.mixed, W / WORD, 0, W / WORD, a->rows, rows(), W + PAD, lost);
+        if (!cut) stage_words<T>(words_of(a, layer) + a->at.mixed, W / WORD, 0, W / WORD, a->rows, rows(), W + PAD, a->wait_most, lost);
         else if (a->splits <= 2) stage_parts<T, 2>(a, words_of(a, layer), rows(), W + PAD, lost);
         else stage_parts<T, 8>(a, words_of(a, layer), rows(), W + PAD, lost);
         __syncthreads();
@@ -936,17 +982,17 @@ struct Block {
     const int layer = again(at_layer), W = a->width, F = a->inner_width;
     ArgsOf of = &a->of[layer];
     Weights<T, 1, RU> asked;
-    asked.ask((const T*)of->w_up, W, F / COLS, a->blocks, 0, 0);
+    asked.ask((const T*)of->w_up, W, F / COLS, me, 0, 0);
     auto early = [&](bool mine, int n, int) {
       return mine ? *(const f32x2*)(of->b_up + n) : (f32x2){0.f, 0.f};
     };
-    const f32x2 first = of_first_tiles<RU>(a, F, early);
+    const f32x2 first = of_first_tiles<RU>(a, me, F, early);
     __syncthreads();             // (the operand before is read)
     norm_row<T, PER>(a, of->second_weight, of->second_bias, true, [&](f32x4 (&v)[PER], int wave, int lane) {
       row_words(a, words_of(a, layer) + a->at.sum, v, wave, lane);
     }, rows(), W + PAD, stat2);
     __syncthreads();
-    product<T, 1, RU, ROWS>(a, (const T*)of->w_up, W, F, W, asked, rows(), W + PAD, red(), first, early,
+    product<T, 1, RU, ROWS>(a, me, (const T*)of->w_up, W, F, W, asked, rows(), W + PAD, red(), first, early,
       [](int) {},
       [&](float v0, float v1, int n, int m, f32x2 bias) {
         publish_operand(words_of(a, layer) + a->at.inner, m * F + n, apply_act(v0 + bias.x, a->act), apply_act(v1 + bias.y, a->act));
@@ -959,7 +1005,7 @@ struct Block {
     const int layer = again(at_layer), W = a->width, F = a->inner_width;
     ArgsOf of = &a->of[layer];
     Weights<T, SCD, 1> asked;
-    asked.ask((const T*)of->w_down, F, W / COLS, a->blocks, 0, 0);
+    asked.ask((const T*)of->w_down, F, W / COLS, me, 0, 0);
     const int pitch = min(a->chunk, F) + PAD;
     auto early = [&](bool mine, int n, int m) {
       Two t{};
@@ -970,11 +1016,12 @@ struct Block {
       }
       return t;
     };
-    const Two first = of_first_tiles<1>(a, W, early);
-    product<T, SCD, 1, ROWS>(a, (const T*)of->w_down, F, W, a->chunk, asked, down_rows(), pitch, red(), first, early,
+    const Two first = of_first_tiles<1>(a, me, W, early);
+    product<T, SCD, 1, ROWS>(a, me, (const T*)of->w_down, F, W, a->chunk, asked, down_rows(), pitch, red(), first, early,
       [&](int k0) {
         __syncthreads();         // (what was there is read)
-        stage_words<T>(words_of(a, layer) + a->at.inner, F / WORD, k0 / WORD, min(a->chunk, F - k0) / WORD, a->rows, down_rows(), pitch, lost);
+        stage_words<T>(words_of(a, layer) + a->at.inner, F / WORD, k0 / WORD, min(a->chunk, F - k0) / WORD, a->rows, down_rows(), pitch,
+                       a->wait_most, lost);
         __syncthreads();
       },
       [&](float v0, float v1, int n, int m, const Two& t) {
@@ -991,15 +1038,25 @@ __global__ void __launch_bounds__(THREADS, sizeof(T) == 2 ? 4 : 2) decode_layers
   extern __shared__ __attribute__((aligned(16))) char smem[];
   __shared__ float stat1[MOST_ROWS][2], stat2[MOST_ROWS][2];
   __shared__ Softmax sm;
+  __shared__ Member joined;
   Args a = (Args)__builtin_amdgcn_kernarg_segment_ptr();
   if ((int)blockIdx.x >= a->blocks) {
     run_ahead<T>(a);
     return;
   }
-  Block<T, ROWS, SCD, RQ, RU> block{smem, stat1, stat2, &sm, {}, false, false};
-  block.mine = item_of<Kind<T>::KEYS>(a, min((int)blockIdx.x, a->rows * (a->width / HD) * a->splits - 1));
+  unsigned number = 0;
+  if (threadIdx.x == 0) number = ask_in(a, 1);
+  Block<T, ROWS, SCD, RQ, RU> block{smem, stat1, stat2, &sm, {}, {}, false, false};
+  // (looked up meanwhile, as it is where all come)
+  const int items = a->rows * (a->width / HD) * a->splits;
+  block.mine = item_of<Kind<T>::KEYS>(a, min((int)blockIdx.x, items - 1));
 #pragma unroll 1
   for (int m = 0; m < a->rows; ++m) block.cut |= shares_of(a->cached_lens[m], a->splits) > 1;
+  if (threadIdx.x == 0) joined = join(a, number);
+  __syncthreads();
+  block.me = {__builtin_amdgcn_readfirstlane(joined.number), __builtin_amdgcn_readfirstlane(joined.of)};
+  if (block.me.number < 0) return;
+  if (block.me.number != (int)blockIdx.x) block.mine = item_of<Kind<T>::KEYS>(a, min(block.me.number, items - 1));
 #pragma unroll 1
   for (int layer = 0; layer < a->layers; ++layer) {
     block.project(a, layer);
@@ -1032,10 +1089,10 @@ static Places layer_places(int dtype, int rows, int width, int inner_width) {
   return p;
 }
 
-// The words of a layer's handoffs, all `NOT_YET` before the launch.
-extern "C" int tnx_decode_layer_words(int dtype, int rows, int width, int inner_width) {
-  if (rows <= 0 || rows > MOST_ROWS || width <= 0 || inner_width <= 0) return 0;
-  return layer_places(dtype, rows, width, inner_width).all;
+// The words of the layers' handoffs and, behind them, of `join`, all `NOT_YET` before the launch.
+extern "C" int tnx_decode_layer_words(int dtype, int rows, int width, int inner_width, int layers) {
+  if (rows <= 0 || rows > MOST_ROWS || width <= 0 || inner_width <= 0 || layers <= 0 || layers > MOST_LAYERS) return 0;
+  return layers * layer_places(dtype, rows, width, inner_width).all + 2;
 }
 
 template <typename T, int ROWS, int SCD, int RQ, int RU>
@@ -1055,18 +1112,20 @@ static int launch_layers(Layers& a, hipStream_t stream) {
     configured = true;
   }
   a.blocks = layer_blocks();
+  a.join_most = a.join_most ? min(a.join_most, a.blocks) : a.blocks;
   decode_layers_kernel<T, ROWS, SCD, RQ, RU><<<a.blocks + (a.blocks % 8 == 0 ? (sizeof(T) == 2 ? 32 : 96) : 0), THREADS, bytes, stream>>>(a);
   TNX_CHECK_LAUNCH("decode_layers");
   return 0;
 }
 
-// Consecutive layers; `words`: as many for each as `tnx_decode_layer_words` names.
+// Consecutive layers; `words`: as many as `tnx_decode_layer_words` names. `join_most` 0: all blocks that come.
 extern "C" int tnx_decode_layers(const Layers* layers, int dtype, hipStream_t stream) {
   Layers a = *layers;
   TNX_REQUIRE(a.rows > 0 && a.rows <= MOST_ROWS, "decode_layers: 1 to %d rows, got %d", MOST_ROWS, a.rows);
   TNX_REQUIRE(a.layers > 0 && a.layers <= MOST_LAYERS, "decode_layers: 1 to %d layers, got %d", MOST_LAYERS, a.layers);
   TNX_REQUIRE(a.width >= 128 && a.width <= 1024 && a.width % 128 == 0 && a.inner_width > 0 && a.inner_width % 128 == 0 && a.inner_width <= 4096,
               "decode_layers: widths in 128s up to 1,024, inner widths up to 4,096, got %d and %d", a.width, a.inner_width);
+  TNX_REQUIRE(a.join_most >= 0 && a.wait_most > 0, "decode_layers: blocks that join and questions of a wait, got %d and %d", a.join_most, a.wait_most);
   TNX_REQUIRE(a.page_shift >= 6 && a.page_shift < 24 && a.table_width > 0 && a.num_pages > 0, "decode_layers: pages of a power of two from 64 keys on");
   TNX_REQUIRE(a.page_pad >= 0 && a.page_pad % 8 == 0, "decode_layers: bad distance between pages");
   TNX_REQUIRE(a.x && a.out && a.token_page && a.token_off && a.cached_lens && a.table && a.failed && a.words, "decode_layers: something is missing");

@@ -222,7 +222,7 @@ _SIGNATURES = {
                            _c_ll, _c_void_p, _c_ll, _c_float, _c_int, _c_int, _c_int, _c_void_p],
     },
     "layer": {
-        "tnx_decode_layer_words": [_c_int, _c_int, _c_int, _c_int],
+        "tnx_decode_layer_words": [_c_int, _c_int, _c_int, _c_int, _c_int],
         "tnx_decode_layers": [_c_void_p, _c_int, _c_void_p],
     },
     "probe": {
@@ -422,7 +422,7 @@ class _Layers(ctypes.Structure):
     _fields_ = ([(n, _c_void_p) for n in ("x", "out", "token_page", "token_off", "cached_lens", "table", "words", "failed")]
                 + [("at", _c_int * 7), ("scale", _c_float), ("eps", _c_float)]
                 + [(n, _c_int) for n in ("rows", "width", "inner_width", "act", "center", "residual_normed", "first_normed", "table_width",
-                                         "page_shift", "num_pages", "page_pad", "splits", "chunk", "layers", "blocks")]
+                                         "page_shift", "num_pages", "page_pad", "splits", "chunk", "layers", "blocks", "join_most", "wait_most")]
                 + [("of", _LayerOf * LAYERS_MOST)])
 
 
@@ -1624,6 +1624,8 @@ class HipOps:
     # of 70, 1,024 34.4 / 26.8, 768 32.7 / 27.9, 512 24.6 / 22.2, but 256 19.4 / 21.0: what is handed on between blocks takes as long as
     # launches there. 2,048 columns 37.4 / 43.6: half of the units do not bring 100 MB of weights as quickly as all of them.
     layer_in_one = True
+    layer_join_most = 0            # so many of the launch's blocks share the work at most (0: all that find room)
+    layer_wait_most = 1 << 22      # questions of a wait, some seconds; every answer comes, from blocks that are on the chip
     layer_rows = 8
     layer_widths, layer_inner = (512, 1024), 4096
     layers_most = LAYERS_MOST
@@ -1699,7 +1701,7 @@ class HipOps:
             raise ValueError("a request is longer than its block table")
         out = torch.empty_like(x)
         # the places of the handoffs, marked as empty (by a launch of its own: whatever came before, they are)
-        words = torch.full((len(layers) * library("layer").tnx_decode_layer_words(_code(self.dtype), t, width, inner),), -1, dtype=torch.int32,
+        words = torch.full((library("layer").tnx_decode_layer_words(_code(self.dtype), t, width, inner, len(layers)),), -1, dtype=torch.int32,
                            device=x.device)
         if self._lost is None:
             self._lost = self.pinned_ints(1)
@@ -1709,6 +1711,7 @@ class HipOps:
                                                                                           view.block_table))
         args.scale, args.eps, args.center = float(p.scale), float(norms[0][1][3]), int(bool(norms[0][1][2]))
         args.rows, args.width, args.inner_width, args.act, args.layers = t, width, inner, _ACT[p.act], len(layers)
+        args.join_most, args.wait_most = self.layer_join_most, self.layer_wait_most
         args.residual_normed, args.first_normed = int(bool(residual_normed)), int(norms[0][0] is not None)
         args.table_width, args.page_shift, args.num_pages, args.page_pad = view.width, view.page_size.bit_length() - 1, num_pages, pad
 
