@@ -737,3 +737,44 @@ def test_host_loops_by_their_names(tiny_folders):
     keep = [i for i in range(cfg["vocab_size"]) if i != banned]
     torch.testing.assert_close(scores[0][0][keep], row[keep], rtol=1e-4, atol=1e-5)
     assert model.config.eos_token_id == cfg.get("eos_token_id", 2) and model.engine.logits_hook is None
+
+
+@pytest.mark.parametrize("run_ahead", [True, False])
+@pytest.mark.parametrize("void", [0, 2, 5])
+def test_tokens_of_a_void_step_are_not_handed_out(tiny_folders, run_ahead, void):
+    """A backend says that a step is void once the device has run it, the first, a middle or the last step: its tokens, and those of a
+    step running ahead, reach nobody, and the engine goes on with new requests."""
+    from transformers_neuronx_amd.kernels import LostStep
+    folder, cfg, _ = tiny_folders["A"]
+
+    def engine():
+        runner, config = _runner(folder, 256)
+        made = LLMEngine(runner, config)
+        made.run_ahead = run_ahead
+        return made
+
+    prompts, params = list(_requests(cfg["vocab_size"], [5, 9], 4).values()), SamplingParams(max_new_tokens=6, do_sample=False)
+    want = engine().generate(prompts, params)
+    late = engine()
+    ops, lost, received = late.runner.ops, [False], [0]
+
+    def receive(sent, plain=ops.receive_tokens):
+        lost[0] = received[0] == void
+        received[0] += 1
+        return plain(sent)
+
+    def raise_if_lost():
+        if lost[0]:
+            lost[0] = False
+            raise LostStep("void")
+
+    ops.receive_tokens, late.runner.raise_if_lost = receive, raise_if_lost
+    got = {0: [], 1: []}
+    with pytest.raises(LostStep):
+        for p in prompts:
+            late.add_request(p, params)
+        late.run(lambda out: got[out.req_id].append(out.token))
+    assert [got[i] for i in (0, 1)] == [w[:void] for w in want]
+    assert not late.requests and not late.has_work
+    late.runner.cache.check()
+    assert late.generate(prompts, params) == want

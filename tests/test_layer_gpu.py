@@ -264,3 +264,42 @@ def test_layers_in_one_launch_through_the_model(tmp_path):
     runner.ops._lost = (torch.ones(1, dtype=torch.int32), None)
     with pytest.raises(RuntimeError, match="waited in vain"):
         runner.step([StepEntry(1, [9], [0])])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("run_ahead", [True, False])
+@pytest.mark.parametrize("graphs", [True, False])
+def test_a_wait_that_was_given_up(tmp_path, run_ahead, graphs):
+    """Waits of one question: the launch ends, says that it is void before a token of its step is handed out, and the engine goes on
+    with launches apart."""
+    from transformers_neuronx_amd.config.engine_config import EngineConfig
+    from transformers_neuronx_amd.engine.engine import LLMEngine
+    from transformers_neuronx_amd.engine.factory import runner_from_folder
+    from transformers_neuronx_amd.kernels import LostStep
+    from transformers_neuronx_amd.opt.config import OPTConfig
+    from transformers_neuronx_amd.sampling import SamplingParams
+    from transformers_neuronx_amd.weights import write_random_model
+    raw = dict(architectures=["OPTForCausalLM"], model_type="opt", vocab_size=640, hidden_size=512, num_hidden_layers=3, num_attention_heads=8,
+               ffn_dim=1024, max_position_embeddings=256, word_embed_proj_dim=512, do_layer_norm_before=True, activation_function="relu",
+               enable_bias=True, layer_norm_elementwise_affine=True, init_std=0.2)
+    write_random_model(OPTConfig.from_dict(raw), str(tmp_path), 3, dtype="float32")
+    config = EngineConfig(dtype="float32", page_size=64, max_tokens=1024, max_num_seqs=4, device=DEV)
+    prompts, params = [[5, 6, 7, 8], [9, 10]], SamplingParams(max_new_tokens=5, do_sample=False)
+
+    def engine():
+        made = LLMEngine(runner_from_folder(str(tmp_path), config), config)
+        made.run_ahead, made.runner.use_graphs = run_ahead, graphs
+        return made
+
+    want = engine().generate(prompts, params)
+    void = engine()
+    void.runner.ops.layer_wait_most = 1
+    handed = []
+    with pytest.raises(LostStep, match="waited in vain"):
+        for p in prompts:
+            void.add_request(p, params)
+        void.run(lambda out: handed.append(out.token))
+    # the prompts' own tokens, launches apart, at most: a step ahead of their being read may be void by then
+    assert handed in ([w[0] for w in want], []) and (run_ahead or handed) and not void.has_work
+    assert not void.runner.ops.layer_in_one
+    assert void.generate(prompts, params) == want

@@ -11,6 +11,7 @@ from typing import Callable, Dict, Hashable, List, Optional, Sequence
 import torch
 
 from ..config.engine_config import EngineConfig
+from ..kernels import LostStep
 from ..sampling.params import SamplingParams
 from ..sampling.sampler import Sampler
 from .batch import StepEntry
@@ -119,10 +120,15 @@ class LLMEngine:
         return _StartedStep(runs, sampling, sent, t0)
 
     def _finish(self, step: _StartedStep) -> List[StepOutput]:
-        """Read the tokens of a started step and give them to their requests."""
+        """Read the tokens of a started step and give them to their requests. `LostStep`: there are none, and every request
+        is forgotten."""
         tokens: List[Optional[int]] = [None] * len(step.runs)
         if step.sampling:
-            it = iter(self.runner.ops.receive_tokens(step.sent))
+            try:
+                it = iter(self.runner.receive_tokens(step.sent))
+            except LostStep:
+                self.reset()               # the tokens, and the keys and values cached with them, are void
+                raise
             tokens = [next(it) if r.samples else None for r in step.runs]
         kept = self.scheduler.resolve(step.runs, tokens)
         self.scheduler.finished.clear()        # the engine reports ends through `StepOutput`; nothing piles up

@@ -51,6 +51,7 @@ def replay(lines: Iterable[str], runner, out_dir: str, out: Optional[TextIO] = N
         logits = runner.step(entries) if entries else None
         if logits is not None:
             arr = logits.detach().to(torch.float32).cpu().numpy().astype("<f4", copy=False)
+            runner.raise_if_lost()
             arr.tofile(os.path.join(out_dir, f"{step}.f32"))
         else:
             runner.ops.synchronize()

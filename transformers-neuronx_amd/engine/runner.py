@@ -106,7 +106,8 @@ class ModelRunner:
         self.kept_tokens = torch.zeros(cache.max_seqs, dtype=torch.int32, device=model.device)
         self._last_ctx: Optional[StepContext] = None
         self._staging = _Staging(ops) if hasattr(ops, "pinned_ints") else None
-        self._raise_if_lost = getattr(ops, "raise_if_lost", None)
+        # `LostStep` where what has run so far is void
+        self.raise_if_lost = getattr(ops, "raise_if_lost", lambda: None)
         # steps written to a folder for running them again alone (`engine/snapshot.py`); None: none are
         self.snapshots = snapshots_from_environment()
 
@@ -121,7 +122,7 @@ class ModelRunner:
         return self._graph_pool
 
     def _recording(self, packed: PackedStep) -> _RecordedStep:
-        key = (packed.layout(), self.model.launch_shape(packed))
+        key = (packed.layout(), self.model.launch_shape(packed), getattr(self.ops, "layer_in_one", None))
         rec = self._recorded.pop(key, None)
         if rec is None:
             while len(self._recorded) >= self.max_recordings:
@@ -176,8 +177,7 @@ class ModelRunner:
         their `want`; None when nothing is wanted (the step still runs)."""
         if not entries:
             return None
-        if self._raise_if_lost is not None:
-            self._raise_if_lost()
+        self.raise_if_lost()         # (of a step whose logits were handed out before it had run)
         taking = self.snapshots is not None and self.snapshots.wanted()
         recordable = (self.use_graphs and not debug.active() and not taking
                       and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries))
@@ -212,8 +212,14 @@ class ModelRunner:
     def keep_tokens(self, tokens: torch.Tensor):
         """Leave the tokens chosen from the last step's logits (one per wanted row, on the device) where
         the next step finds them, under the slot of each row's request, and send them to the host.
-        Returns what `ops.receive_tokens` turns into a list."""
+        Returns what `receive_tokens` turns into a list."""
         return self.ops.send_tokens(tokens, self.kept_tokens, self._last_ctx)
+
+    def receive_tokens(self, sent) -> List[int]:
+        """The tokens that `keep_tokens` sent, once they are there."""
+        tokens = self.ops.receive_tokens(sent)
+        self.raise_if_lost()
+        return tokens
 
     def finish(self, req: Hashable) -> None:
         """The request is over: its pages and its slot go back."""

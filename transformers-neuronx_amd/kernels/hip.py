@@ -11,7 +11,7 @@ from typing import Dict, Optional
 import numpy as np
 import torch
 
-from . import build
+from . import LostStep, build
 from .attention_plan import QUERY_TILE
 from .memory_plan import MEMORY_CHUNK
 from .. import debug
@@ -1725,10 +1725,13 @@ class HipOps:
         return out
 
     def raise_if_lost(self) -> None:
-        """A wait inside a launch that went on without an answer has left results that are no numbers: said here, by the host's
-        next step."""
+        """A wait inside a launch that went on without an answer has left results that are no numbers. Asked where results of a
+        step that has run reach the host; from then on layers are launches apart."""
         if self._lost is not None and int(self._lost[0][0]):
-            raise RuntimeError("a layer's launch waited in vain for blocks of its own that were not run beside it; its step's results are void")
+            self.synchronize()             # (what is under way may say the same)
+            self._lost[0].zero_()
+            self.layer_in_one = False
+            raise LostStep("a layer's launch waited in vain for blocks of its own that were not run beside it; its step's results are void")
 
     # ---------------------------------------------------------------- parts of other designs
 
