@@ -303,3 +303,32 @@ def test_a_wait_that_was_given_up(tmp_path, run_ahead, graphs):
     assert handed in ([w[0] for w in want], []) and (run_ahead or handed) and not void.has_work
     assert not void.runner.ops.layer_in_one
     assert void.generate(prompts, params) == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [BF16, F32])
+@pytest.mark.parametrize("blocks,runs", [(["post", "pre", "post", "post"], {0: 1, 1: 2, 2: 4}), (["pre", "pre", "post"], {0: 2, 2: 3}),
+                                         (["pre"] * 33, {0: 30, 30: 33}), (["post"] * 32, {0: 30, 30: 32})])
+def test_several_launches_of_layers(blocks, runs, dtype):
+    """Models whose layers are several such launches one behind the other: another arrangement, or more layers than one takes."""
+    import toy_parts
+    from transformers_neuronx_amd.cache import CacheManager
+    from transformers_neuronx_amd.engine import DecoderModel, ModelRunner
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    from transformers_neuronx_amd.weights import TensorDict, random_tensors
+    spec = toy_parts.toy_spec_blocks([b + "_norm" for b in blocks], 512)
+    logits = {}
+    for one in (True, False):
+        model, ops = DecoderModel(spec), HipOps(dtype, DEV)
+        model.load(TensorDict(random_tensors(model.param_decls(), spec.init_std, 3, dtype)), ops, dtype, DEV)
+        ops.layer_in_one, called = one, []
+        call = ops._call
+        ops._call = lambda lib, name, *a, **k: (called.append(name), call(lib, name, *a, **k))[1]
+        assert model.layers_in_one == runs
+        runner = ModelRunner(model, CacheManager(model.cache_needs(), 64, 12, 4, dtype, DEV), ops)
+        runner.step([StepEntry(r, [5 + i + r for i in range(40 + 30 * r)], []) for r in range(3)])
+        del called[:]
+        logits[one] = torch.cat([runner.step([StepEntry(r, [7 * turn + r], [0]) for r in range(3)]).float().cpu() for turn in range(3)])
+        assert called.count("tnx_decode_layers") == 3 * one * len(runs)
+    # float32 sums in another order; in bfloat16 their roundings through up to 33 layers
+    assert float((logits[True] - logits[False]).norm() / logits[False].norm()) < (0.03 if dtype == BF16 else 1e-5)

@@ -3,6 +3,7 @@ next to it: parts that say they take that get it, every other part, norm and arr
 import pytest
 import torch
 
+import toy_parts
 from transformers_neuronx_amd.kernels.reference import ReferenceOps
 from transformers_neuronx_amd.parts import FeedForward, Mixer, Stream
 from transformers_neuronx_amd.parts.block import PostNormBlock, PreNormBlock
@@ -179,6 +180,49 @@ def test_longer_steps_ask_nothing_of_a_norm_left_to_a_product(tokens, asked):
     block.after_load()
     block.forward(Stream(torch.randn(tokens, WIDTH)), Step(), None)
     assert [n.calls for n in norms] == [int(asked)] * 2
+
+
+class InOneOps(LateOps):
+    """Asks for layers in one launch as well, and takes none of them."""
+
+    layer_rows, layers_most = 8, 30
+
+    def __init__(self):
+        super().__init__()
+        self.asked = []
+
+    def layer_parts(self, attention, feed_forward):
+        return attention, feed_forward
+
+    def layers_fit(self, ctx):
+        return True
+
+    def layers_alike(self, first, block, before):
+        return True
+
+    def decode_layers(self, layers, x, norms, residual_normed, ctx, view, caches):
+        assert type(x) is torch.Tensor
+        self.asked.append(len(layers))
+
+
+@pytest.mark.parametrize("kinds,runs", [("post pre", [1, 1]), ("pre post post", [1, 2]), ("post post pre pre post", [2, 2, 1])])
+def test_runs_of_layers_behind_another_kind(kinds, runs):
+    """Layers of one launch behind a block whose last sum's norm has been left to them, where they take none: the norm is made."""
+    from transformers_neuronx_amd.engine.model import DecoderModel
+    from transformers_neuronx_amd.engine.runner import ModelRunner
+    from transformers_neuronx_amd.cache import CacheManager
+    from transformers_neuronx_amd.engine import StepEntry
+    from transformers_neuronx_amd.weights import TensorDict, random_tensors
+    spec = toy_parts.toy_spec_blocks([k + "_norm" for k in kinds.split()], 128)
+    logits = {}
+    for ops in (ReferenceOps(torch.float32, "cpu"), InOneOps()):
+        model = DecoderModel(spec)
+        model.load(TensorDict(random_tensors(model.param_decls(), spec.init_std, 3, torch.float32)), ops, torch.float32, "cpu")
+        runner = ModelRunner(model, CacheManager(model.cache_needs(), 16, 12, 4, torch.float32, "cpu"), ops)
+        runner.step([StepEntry(r, [5 + i + r for i in range(9)], []) for r in range(3)])
+        logits[type(ops)] = runner.step([StepEntry(r, [7 + r], [0]) for r in range(3)])
+    assert ops.asked == runs and ops.left > 0
+    assert torch.equal(logits[ReferenceOps], logits[InOneOps])
 
 
 def test_built_in_parts_say_so():

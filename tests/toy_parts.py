@@ -75,6 +75,22 @@ def toy_spec(width=64, heads=4, inner=96, vocab=300, positions=160, window=24, e
                      layers=layers, schedule=schedule, head=head, init_std=0.08)
 
 
+def toy_spec_blocks(blocks, width, inner=128, head=64, vocab=320, positions=160, eps=1e-5):
+    """Layers of full attention with the arrangements named, otherwise alike."""
+    norm = PartSpec("layer_norm", dict(width=width, eps=eps, affine=True))
+    parts = dict(mixer=PartSpec("attention", dict(names=QKVO, width=width, num_heads=width // head, head_size=head)), mixer_norm=norm,
+                 feed_forward=PartSpec("dense", dict(up_name="fc1", down_name="fc2", width=width, inner=inner, activation="relu", bias=True)),
+                 feed_forward_norm=norm, mixer_name="mix.", feed_forward_name="ffn.", mixer_norm_name="norm1", feed_forward_norm_name="norm2")
+    layers = tuple(LayerSpec(prefix=f"layers.{i}.", block=block, **parts) for i, block in enumerate(blocks))
+    embedding = PartSpec("token_table", dict(
+        vocab=vocab, embed_width=width, width=width, position=PartSpec("learned", dict(width=width, max_positions=positions, offset=0)),
+        table_name="embed.weight", projection_name=None, position_name="positions"))
+    head_part = PartSpec("vocab_projection", dict(vocab=vocab, embed_width=width, width=width, norm=norm, weight_name="head.weight", tied_to=None,
+                                                  projection_name=None, norm_name="final_norm"))
+    return ModelSpec(hidden_size=width, vocab_size=vocab, max_positions=positions, embedding=embedding, layers=layers,
+                     schedule=tuple(LayerCall(i) for i in range(len(layers))), head=head_part, init_std=0.08)
+
+
 def toy_plain_logits(w, tokens, width=64, heads=4, window=24, eps=1e-5):
     """The toy model on one whole sequence, from the plain functions."""
     w = {k: v.float() for k, v in w.items()}

@@ -185,8 +185,10 @@ class DecoderModel:
         for call, (layer, cid, writes) in enumerate(self.schedule):
             if call < done:
                 continue
-            if left and (call in in_one or not getattr(self.layers[layer].block, "leaves_shares", False)):
-                stream, left = self._settled(stream), False
+            block = self.layers[layer].block
+            if (left and (call in in_one or not getattr(block, "leaves_shares", False))
+                    or between and not getattr(block, "norms_between", False)):
+                stream, left, between = self._settled(stream), False, False
             if call in in_one:
                 behind = self._run_in_one(stream, call, in_one[call], ctx, caches)
                 if behind is not None:
@@ -196,9 +198,6 @@ class DecoderModel:
             cache = caches[cid] if writes else caches[cid].reader()
             state_id = self.call_state_ids[call]
             ctx.call_state = caches[state_id] if state_id is not None else None
-            block = self.layers[layer].block
-            if between and not getattr(block, "norms_between", False):
-                stream = self._settled(stream)
             stream = block.forward(stream, ctx, cache)
             between = few and getattr(block, "norms_between", False)
             left = getattr(block, "leaves_shares", False)
