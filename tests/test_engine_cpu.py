@@ -768,7 +768,7 @@ def test_tokens_of_a_void_step_are_not_handed_out(tiny_folders, run_ahead, void)
             lost[0] = False
             raise LostStep("void")
 
-    ops.receive_tokens, late.runner.raise_if_lost = receive, raise_if_lost
+    ops.receive_tokens, late.runner._raise_if_lost = receive, raise_if_lost
     got = {0: [], 1: []}
     with pytest.raises(LostStep):
         for p in prompts:
@@ -778,3 +778,59 @@ def test_tokens_of_a_void_step_are_not_handed_out(tiny_folders, run_ahead, void)
     assert not late.requests and not late.has_work
     late.runner.cache.check()
     assert late.generate(prompts, params) == want
+
+
+@pytest.mark.parametrize("run_ahead", [True, False])
+@pytest.mark.parametrize("void", [1, 2, 4])
+def test_a_void_step_found_where_the_next_begins(tiny_folders, run_ahead, void):
+    """The device has run a void step before the host begins another, which is where it is found: no token of it is handed out
+    afterwards either, by a caller that goes on with `step()`."""
+    from transformers_neuronx_amd.kernels import LostStep
+    folder, cfg, _ = tiny_folders["A"]
+
+    def engine():
+        runner, config = _runner(folder, 256)
+        made = LLMEngine(runner, config)
+        made.run_ahead = run_ahead
+        return made
+
+    prompts, params = list(_requests(cfg["vocab_size"], [5, 9], 4).values()), SamplingParams(max_new_tokens=6, do_sample=False)
+    want = engine().generate(prompts, params)
+    late = engine()
+    begun = [0]
+
+    def raise_if_lost():
+        begun[0] += 1
+        if begun[0] == at:
+            raise LostStep("void")
+
+    # asked once where a step begins and once where its tokens are there: the beginning of step `void`, counted from 0
+    at = 2 * void + (not run_ahead)
+    late.runner._raise_if_lost = raise_if_lost
+    for p in prompts:
+        late.add_request(p, params)
+    got = {0: [], 1: []}
+    with pytest.raises(LostStep):
+        late.run(lambda out: got[out.req_id].append(out.token))
+    assert [got[i] for i in (0, 1)] == [w[:void - run_ahead] for w in want]
+    assert not late.requests and not late.has_work and late.step() == []
+    late.runner.cache.check()
+    assert late.generate(prompts, params) == want
+
+
+def test_sequences_of_a_void_step_are_forgotten(tiny_folders):
+    """`step` alone, as `model(...)` calls it: the keys and values that a void step left are nobody's to go on with."""
+    from transformers_neuronx_amd.kernels import LostStep
+    folder, cfg, _ = tiny_folders["A"]
+    runner, _ = _runner(folder, 256)
+    runner.step([StepEntry("a", [5, 6, 7], [2])])
+
+    def raise_if_lost():
+        raise LostStep("void")
+
+    plain, runner._raise_if_lost = runner._raise_if_lost, raise_if_lost
+    with pytest.raises(LostStep):
+        runner.step([StepEntry("a", [8], [0])])
+    runner._raise_if_lost = plain
+    assert not runner.cache.has("a")
+    runner.cache.check()

@@ -120,15 +120,10 @@ class LLMEngine:
         return _StartedStep(runs, sampling, sent, t0)
 
     def _finish(self, step: _StartedStep) -> List[StepOutput]:
-        """Read the tokens of a started step and give them to their requests. `LostStep`: there are none, and every request
-        is forgotten."""
+        """Read the tokens of a started step and give them to their requests."""
         tokens: List[Optional[int]] = [None] * len(step.runs)
         if step.sampling:
-            try:
-                it = iter(self.runner.receive_tokens(step.sent))
-            except LostStep:
-                self.reset()               # the tokens, and the keys and values cached with them, are void
-                raise
+            it = iter(self.runner.receive_tokens(step.sent))
             tokens = [next(it) if r.samples else None for r in step.runs]
         kept = self.scheduler.resolve(step.runs, tokens)
         self.scheduler.finished.clear()        # the engine reports ends through `StepOutput`; nothing piles up
@@ -149,7 +144,15 @@ class LLMEngine:
     @torch.no_grad()
     def step(self) -> List[StepOutput]:
         """Schedule, run, sample, record: one batch of portions and decoded tokens. Returns the tokens of
-        the step it ran, or with `run_ahead` those of the step started by the call before."""
+        the step it ran, or with `run_ahead` those of the step started by the call before. `LostStep`, wherever it is found:
+        the tokens under way, and the keys and values cached with them, are void, and every request is forgotten."""
+        try:
+            return self._step()
+        except LostStep:
+            self.reset()
+            raise
+
+    def _step(self) -> List[StepOutput]:
         # a request that may not repeat its n-grams needs its last token on the host before the next is chosen
         in_step = any(q.params.no_repeat_ngram_size and not q.finished for q in self.requests.values())
         idle = self._started is None

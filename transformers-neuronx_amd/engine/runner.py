@@ -18,6 +18,7 @@ import numpy as np
 
 from ..cache.manager import CacheManager
 from .. import debug
+from ..kernels import LostStep
 from .batch import PackedStep, StepContext, StepEntry, context_from, pack_step
 from .model import DecoderModel
 from .snapshot import snapshots_from_environment
@@ -106,8 +107,7 @@ class ModelRunner:
         self.kept_tokens = torch.zeros(cache.max_seqs, dtype=torch.int32, device=model.device)
         self._last_ctx: Optional[StepContext] = None
         self._staging = _Staging(ops) if hasattr(ops, "pinned_ints") else None
-        # `LostStep` where what has run so far is void
-        self.raise_if_lost = getattr(ops, "raise_if_lost", lambda: None)
+        self._raise_if_lost = getattr(ops, "raise_if_lost", lambda: None)
         # steps written to a folder for running them again alone (`engine/snapshot.py`); None: none are
         self.snapshots = snapshots_from_environment()
 
@@ -177,7 +177,7 @@ class ModelRunner:
         their `want`; None when nothing is wanted (the step still runs)."""
         if not entries:
             return None
-        self.raise_if_lost()         # (of a step whose logits were handed out before it had run)
+        self.raise_if_lost()         # (of a step that had not run when its logits were handed out)
         taking = self.snapshots is not None and self.snapshots.wanted()
         recordable = (self.use_graphs and not debug.active() and not taking
                       and all(len(e.tokens) == 1 and list(e.want) == [0] for e in entries))
@@ -208,6 +208,14 @@ class ModelRunner:
         for e in entries:
             self.cache.advance(e.req, len(e.tokens))
         return logits if any(len(e.want) for e in entries) else None
+
+    def raise_if_lost(self) -> None:
+        """`LostStep` where what has run so far is void; the requests, whose keys and values are void with it, are forgotten."""
+        try:
+            self._raise_if_lost()
+        except LostStep:
+            self.cache.reset()
+            raise
 
     def keep_tokens(self, tokens: torch.Tensor):
         """Leave the tokens chosen from the last step's logits (one per wanted row, on the device) where
