@@ -230,3 +230,114 @@ def test_built_in_parts_say_so():
     for part in (Attention, DenseFeedForward):
         assert part.forward.residual_to_product
     assert not getattr(FeedForward.forward, "residual_to_product", False) and not getattr(Mixer.forward, "residual_to_product", False)
+
+
+class Unadded:
+    """A product's result that a norm is to read next, as the HIP backend leaves it; as `onto` makes it, a residual."""
+
+    def __init__(self, ops, x):
+        self.ops, self.x = ops, x
+
+    def settled(self):
+        return self.x
+
+    def normed(self, weight, bias, eps, dtype, center, alone=False):
+        y, h = self.ops.layernorm(self.x, weight, bias, eps, dtype, True, True, center)
+        return (y if alone else self.x), h
+
+
+class SharingOps(InOneOps):
+    """Leaves sums to the norms behind them too."""
+
+    def onto(self, x):
+        return Unadded(self, x)
+
+    def linear(self, x, w, bias=None, act=None, residual=None, **more):
+        leave = isinstance(residual, Unadded)
+        y = super().linear(x, w, bias, act=act, residual=residual.x if leave else residual, **more)
+        return Unadded(self, y) if leave else y
+
+    @staticmethod
+    def settled(x):
+        return x.x if isinstance(x, Unadded) else LateOps.settled(x)
+
+    def decode_layers(self, layers, *more):
+        super().decode_layers(layers, *more)
+        self.layers = layers
+
+
+def _toy_runner(kind, ops):
+    from transformers_neuronx_amd.engine.model import DecoderModel
+    from transformers_neuronx_amd.engine.runner import ModelRunner
+    from transformers_neuronx_amd.cache import CacheManager
+    from transformers_neuronx_amd.weights import TensorDict, random_tensors
+    spec = toy_parts.toy_spec_blocks([kind] * 3, 128)
+    model = DecoderModel(spec)
+    model.load(TensorDict(random_tensors(model.param_decls(), spec.init_std, 3, torch.float32)), ops, torch.float32, "cpu")
+    return ModelRunner(model, CacheManager(model.cache_needs(), 16, 12, 4, torch.float32, "cpu"), ops)
+
+
+def _steps(runner):
+    """A step of more rows than few, and one of few."""
+    from transformers_neuronx_amd.engine import StepEntry
+    return torch.cat([runner.step([StepEntry(r, [5 + i + r for i in range(9)], [8]) for r in range(3)]),
+                      runner.step([StepEntry(r, [7 + r], [0]) for r in range(3)])])
+
+
+@pytest.mark.parametrize("part", ["", "mixer", "feed_forward", "mixer_norm", "feed_forward_norm"])
+@pytest.mark.parametrize("kind", ["pre_norm", "post_norm"])
+@pytest.mark.parametrize("dressed", [True, False])
+def test_a_forward_put_on_an_object_is_called(kind, part, dressed):
+    """Put there after loading, on a block, a part or a norm: called in every step, with tensors; and not once it is taken away."""
+    import functools
+    want = _steps(_toy_runner(kind, ReferenceOps(torch.float32, "cpu")))
+    ops = SharingOps()
+    runner = _toy_runner(kind, ops)
+    assert torch.equal(_steps(runner), want) and ops.asked == [3]
+    block, calls = runner.model.layers[1].block, []
+    of = getattr(block, part) if part else block
+    inner = of.forward
+
+    def forward(*args, **named):
+        for a in (args[0].x if not part else args[0], *(args[-1:] if part in ("mixer", "feed_forward") else ())):
+            assert type(a) is torch.Tensor
+        out = inner(*args, **named)
+        assert not isinstance(out.x if not part else out, Unadded)
+        calls.append(1)
+        return out
+    of.forward = functools.wraps(inner)(forward) if dressed else forward
+    runner.cache.reset()
+    assert torch.equal(_steps(runner), want) and len(calls) == 2 and ops.asked == [3]
+    del of.forward
+    runner.cache.reset()
+    assert torch.equal(_steps(runner), want) and len(calls) == 2 and ops.asked == [3, 3]
+
+
+@pytest.mark.parametrize("name", ["mixer", "feed_forward"])
+def test_a_forward_put_on_a_class_before_loading_is_called(monkeypatch, name):
+    import functools
+    from transformers_neuronx_amd.parts.mixer import Attention
+    cls, calls = {"mixer": Attention, "feed_forward": DenseFeedForward}[name], []
+    inner = cls.forward
+
+    @functools.wraps(inner)
+    def forward(self, *args):
+        assert type(args[-1]) is torch.Tensor
+        calls.append(1)
+        return inner(self, *args)
+    monkeypatch.setattr(cls, "forward", forward)
+    ops = SharingOps()
+    _steps(_toy_runner("pre_norm", ops))
+    assert len(calls) == 6 and not ops.asked
+
+
+def test_layers_in_one_launch_take_the_tensors_of_the_step():
+    """Another matrix in a part's place, as `forward` would read it."""
+    ops = SharingOps()
+    runner = _toy_runner("pre_norm", ops)
+    _steps(runner)
+    mixer, ff = runner.model.layers[1].block.mixer, runner.model.layers[2].block.feed_forward
+    mixer.w_out, ff.b1, mixer.scale = mixer.w_out * 2, ff.b1 + 1, 0.5
+    runner.cache.reset()
+    _steps(runner)
+    assert ops.layers[1][0][2] is mixer.w_out and ops.layers[1][0][5] == 0.5 and ops.layers[2][1][1] is ff.b1

@@ -230,12 +230,16 @@ class DecoderModel:
         return out
 
     def _run_in_one(self, stream: Stream, begin: int, end: int, ctx, caches):
-        """The stream behind the calls from `begin` to `end`, run as one launch; None where the backend does not take the step."""
+        """The stream behind the calls from `begin` to `end`, run as one launch; None where the backend does not take the step, or a
+        block no longer is what a launch runs."""
         blocks = [self.layers[layer].block for layer, _, _ in self.schedule[begin:end]]
+        parts = [b.in_one for b in blocks]
+        if any(p is None for p in parts):
+            return None
         of_calls = [caches[cid] for _, cid, _ in self.schedule[begin:end]]
         x, first, residual_normed = blocks[0].into_one(stream)
         norms = [(first, blocks[0].norms_in_one(blocks[0])[1])] + [b.norms_in_one(before) for before, b in zip(blocks, blocks[1:])]
-        y = self.ops.decode_layers([b.in_one for b in blocks], x, norms, residual_normed, ctx, ctx.groups[of_calls[0].group], of_calls)
+        y = self.ops.decode_layers(parts, x, norms, residual_normed, ctx, ctx.groups[of_calls[0].group], of_calls)
         return None if y is None else blocks[-1].out_of_one(y)
 
     def _settled(self, stream: Stream) -> Stream:

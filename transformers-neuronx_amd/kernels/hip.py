@@ -436,6 +436,11 @@ class LayerParts:
         self.w_qkv, self.b_qkv, self.w_out, self.b_out, self.heads, self.scale = attention
         self.w_up, self.b_up, self.act, self.w_down, self.b_down = feed_forward
 
+    def alike(self, other) -> bool:
+        """Whether the two go into one launch (the other shapes follow from these)."""
+        return (self.w_qkv.shape == other.w_qkv.shape and self.w_up.shape == other.w_up.shape
+                and (self.act, self.scale) == (other.act, other.scale))
+
 
 def tile_order(w: torch.Tensor) -> torch.Tensor:
     """`w[n, k]` -> `[n/16][k/128][s][r][g][e]` with n = 16*nt + r and k = 128*kt + 32*s + 8*g + e."""
@@ -1631,8 +1636,8 @@ class HipOps:
     layers_most = LAYERS_MOST
 
     def layer_parts(self, attention, feed_forward):
-        """Asked once when a layer has its tensors: what `decode_layers` takes for it, or None where the layer is none of its
-        kind. `attention` = (w_qkv, b_qkv, w_out, b_out, heads, scale), `feed_forward` = (w_up, b_up, act, w_down, b_down)."""
+        """Asked when a layer has its tensors, and again in every step for those that it has then: what `decode_layers` takes for it,
+        or None where the layer is none of its kind. `attention` = (w_qkv, b_qkv, w_out, b_out, heads, scale), `feed_forward` = (w_up, b_up, act, w_down, b_down)."""
         p = LayerParts(attention, feed_forward)
         weights = (p.w_qkv, p.w_out, p.w_up, p.w_down)
         if not all(isinstance(w, PreparedWeight) and w.tensor.dtype == self.dtype and w.inner == w.tensor.shape[1] for w in weights):
@@ -1650,10 +1655,8 @@ class HipOps:
     @staticmethod
     def layers_alike(first, block, before) -> bool:
         """Whether `block`, behind `before`, goes into one launch with `first`: sizes, activation, scale and norms of one kind."""
-        a, b = first.in_one, block.in_one
         norms = [n for n in first.norms_in_one(first) + block.norms_in_one(before)]
-        return (a.w_qkv.shape == b.w_qkv.shape and a.w_up.shape == b.w_up.shape and (a.act, a.scale) == (b.act, b.scale)
-                and all(n[2:] == norms[0][2:] for n in norms))
+        return first.in_one.alike(block.in_one) and all(n[2:] == norms[0][2:] for n in norms)
 
     def _layer_weights(self, p):
         """The four matrices as the launch reads them, or None where one has no such copy."""
@@ -1669,7 +1672,7 @@ class HipOps:
         if not (self.layers_fit(ctx) and view.page_size >= 64 and view.page_size & (view.page_size - 1) == 0):
             return None
         width, inner = p.w_qkv.shape[1], p.w_up.shape[0]
-        if any(n is not None and n[2:] != norms[0][1][2:] for pair in norms for n in pair):
+        if any(n is not None and n[2:] != norms[0][1][2:] for pair in norms for n in pair) or not all(p.alike(q) for q in layers[1:]):
             return None
         _want(x, "x", torch.float32, (t, width))
         args = _Layers()

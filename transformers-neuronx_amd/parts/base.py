@@ -147,9 +147,17 @@ def residual_to_product(forward):
     `ops.linear` as the residual of its last product. A block behind whose sums a norm
     stands may then hand over `h` and `residual` as what `ops.norm_between` returns, and one before whose next norm nothing else reads
     the sum `residual` as `ops.onto` makes it and take a result that is no tensor yet. The mark is the function's: a subclass with
-    a `forward` of its own has tensors again unless that is marked too."""
-    forward.residual_to_product = True
+    a `forward` of its own has tensors again unless that is marked too (`hands_residual_on`)."""
+    forward.residual_to_product = forward
     return forward
+
+
+def hands_residual_on(part) -> bool:
+    """Whether `part.forward` is a function that `residual_to_product` marked, bound to this part, and not another one around it (one
+    that `functools.wraps` dresses carries the mark of what it wraps)."""
+    bound = part.forward
+    function = getattr(bound, "__func__", None)
+    return function is not None and getattr(bound, "__self__", None) is part and getattr(function, "residual_to_product", None) is function
 
 
 class Mixer(Part):
@@ -265,8 +273,14 @@ class Block(Part):
         return []
 
     # Where the backend can run this layer and its neighbours of the same kind as one launch in decode steps of few rows: what it
-    # takes for it (`ops.layer_parts`), known once the parts have their tensors. The arrangement then says what goes in and out.
+    # takes for it (`ops.layer_parts`), of the tensors that the parts have when it is asked. The arrangement then says what goes in and out.
     in_one = None
+
+    def own_forwards(self) -> bool:
+        """Whether a `forward` was put on this very block, a part or a norm of it, past its class. It is called then, with tensors,
+        and nothing is done around it; asked in every step, since it may be put there, and taken away, at any time."""
+        return ("forward" in vars(self) or "forward" in vars(self.mixer) or "forward" in vars(self.feed_forward)
+                or "forward" in vars(self.mixer_norm) or "forward" in vars(self.feed_forward_norm))
 
     def norms_in_one(self, before):
         """`Norm.fused_form` of what the layer's two halves read, where `before` is the block of the layer before in that launch."""

@@ -1,6 +1,6 @@
 """Arrangements of a layer's parts around the residual stream."""
 from .. import debug
-from .base import Block, Stream, joined_rows, register_block
+from .base import Block, Stream, hands_residual_on, joined_rows, register_block
 
 
 def _is_its_fused_form(norm) -> bool:
@@ -11,15 +11,17 @@ def _is_its_fused_form(norm) -> bool:
     return owner("fused_form") is not None and owner("forward") is owner("fused_form")
 
 
-def _layer_parts(block, kind):
-    """What the backend takes to run the layer as part of a launch of several (`Block.in_one`), or None: an arrangement of its own
-    (a subclass with another `forward`), and parts and norms that say nothing of themselves, are run part by part."""
-    ops = block.mixer_norm.ops
-    if (type(block).forward is not kind.forward or not hasattr(ops, "layer_parts")
-            or not all(_is_its_fused_form(n) for n in (block.mixer_norm, block.feed_forward_norm))):
-        return None
+def _hands_on(block) -> bool:
+    """Whether both parts do with the stream what `residual_to_product` says, and both norms are what their `fused_form` says."""
+    return (all(hands_residual_on(p) and p.first_weight() is not None for p in (block.mixer, block.feed_forward))
+            and all(_is_its_fused_form(n) for n in (block.mixer_norm, block.feed_forward_norm)))
+
+
+def _layer_parts(block):
+    """What the backend takes to run the layer as part of a launch of several (`Block.in_one`), or None: parts that say nothing of
+    themselves are run part by part. The parts' tensors are looked up in every step, as their `forward` looks them up."""
     attention, feed_forward = block.mixer.layer_form(), block.feed_forward.layer_form()
-    return ops.layer_parts(attention, feed_forward) if attention is not None and feed_forward is not None else None
+    return block.mixer_norm.ops.layer_parts(attention, feed_forward) if attention is not None and feed_forward is not None else None
 
 
 @register_block("pre_norm")
@@ -36,7 +38,16 @@ class PreNormBlock(Block):
     # Each part's last product adds the stream, and behind it stands a norm, of this block or the next: the backend may leave the
     # product's shares of K to the norm's launch (`HipOps.onto`). The block then takes a stream whose sum has not been made, and
     # leaves one.
-    leaves_shares = False
+    may_leave_shares = False
+    may_be_in_one = False
+
+    @property
+    def leaves_shares(self) -> bool:
+        return self.may_leave_shares and not self.own_forwards()
+
+    @property
+    def in_one(self):
+        return _layer_parts(self) if self.may_be_in_one and not self.own_forwards() else None
 
     def after_load(self) -> None:
         # Each norm's output goes to one part only; where that part does nothing with it but one matrix
@@ -48,11 +59,10 @@ class PreNormBlock(Block):
         self.fold_feed_forward_norm = w is not None and self.feed_forward_norm.fold_into(w)
         self.mixer_norm_rows = self.mixer_norm.defer_rows if self.fold_mixer_norm else -1
         self.feed_forward_norm_rows = self.feed_forward_norm.defer_rows if self.fold_feed_forward_norm else -1
-        self.in_one = _layer_parts(self, PreNormBlock)
-        self.leaves_shares = (hasattr(self.mixer_norm.ops, "onto") and type(self).forward is PreNormBlock.forward
-                              and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None
-                                      for p in (self.mixer, self.feed_forward))
-                              and all(_is_its_fused_form(n) for n in (self.mixer_norm, self.feed_forward_norm)))
+        # (an arrangement of its own, a subclass with another `forward`, gets tensors)
+        known = type(self).forward is PreNormBlock.forward and _hands_on(self)
+        self.may_be_in_one = known and hasattr(self.mixer_norm.ops, "layer_parts")
+        self.may_leave_shares = known and hasattr(self.mixer_norm.ops, "onto")
 
     def norms_in_one(self, before):
         return self.mixer_norm.fused_form(), self.feed_forward_norm.fused_form()
@@ -61,8 +71,8 @@ class PreNormBlock(Block):
         return stream.x, self.mixer_norm.fused_form(), False
 
     def _normed(self, norm, x, deferred):
-        """(x, its norm): `x` as a tensor, whatever the product before left of it."""
-        if self.leaves_shares and hasattr(type(x), "normed"):
+        """(x, its norm): `x` as a tensor, whatever the product before left of it (only blocks that leave shares are handed them)."""
+        if self.may_leave_shares and hasattr(type(x), "normed"):
             if not deferred:
                 weight, bias, center, eps = norm.fused_form()
                 return x.normed(weight, bias, eps, norm.dtype, center)
@@ -95,19 +105,30 @@ class PostNormBlock(Block):
     # Both parts do with the stream nothing but a product of its rows and adding it to their last product's sums, and the norms
     # are of a form that the backend's products know: in steps of few rows they norm it themselves. Parts say so
     # (`residual_to_product`), and an arrangement of its own around the same sums gets tensors.
-    norms_between = False
+    may_norm_between = False
     between_rows = -1              # and few are so many
-    norms_shares = False           # in steps of more, the norm's launch adds the shares of the sum's product (`HipOps.onto`)
+    may_norm_shares = False        # in steps of more, the norm's launch adds the shares of the sum's product (`HipOps.onto`)
+    may_be_in_one = False
+
+    @property
+    def norms_between(self) -> bool:
+        return self.may_norm_between and not self.own_forwards()
+
+    @property
+    def norms_shares(self) -> bool:
+        return self.may_norm_shares and not self.own_forwards()
+
+    @property
+    def in_one(self):
+        return _layer_parts(self) if self.may_be_in_one and not self.own_forwards() else None
 
     def after_load(self) -> None:
-        norms, parts = (self.mixer_norm, self.feed_forward_norm), (self.mixer, self.feed_forward)
-        self.norms_between = (self.alpha is None and self.has_ff and hasattr(self.mixer_norm.ops, "norm_between")
-                              and type(self).forward is PostNormBlock.forward
-                              and all(getattr(p.forward, "residual_to_product", False) and p.first_weight() is not None for p in parts)
-                              and all(_is_its_fused_form(n) for n in norms))
-        self.between_rows = self.mixer_norm.ops.norm_beside_rows if self.norms_between else -1
-        self.norms_shares = self.norms_between and hasattr(self.mixer_norm.ops, "onto")
-        self.in_one = _layer_parts(self, PostNormBlock) if self.norms_between else None
+        ops = self.mixer_norm.ops
+        self.may_norm_between = (self.alpha is None and self.has_ff and hasattr(ops, "norm_between")
+                                 and type(self).forward is PostNormBlock.forward and _hands_on(self))
+        self.between_rows = ops.norm_beside_rows if self.may_norm_between else -1
+        self.may_norm_shares = self.may_norm_between and hasattr(ops, "onto")
+        self.may_be_in_one = self.may_norm_between and hasattr(ops, "layer_parts")
 
     def norms_in_one(self, before):
         return before.feed_forward_norm.fused_form(), self.mixer_norm.fused_form()
@@ -136,7 +157,7 @@ class PostNormBlock(Block):
 
     def _behind(self, norm, t):
         """(float32, compute dtype) of the norm behind a sum, of a product that may have left its shares."""
-        if self.norms_shares and hasattr(type(t), "normed"):
+        if self.may_norm_shares and hasattr(type(t), "normed"):
             weight, bias, center, eps = norm.fused_form()
             return t.normed(weight, bias, eps, norm.dtype, center, alone=True)
         return norm.forward(t, True, True)
@@ -154,7 +175,7 @@ class PostNormBlock(Block):
             if self.has_ff:
                 x, h = self._join(self.feed_forward_norm, x, [(self.feed_forward.forward(h, ctx, None), None, None, 1.0)])
             return Stream(x, h)
-        if ctx.num_tokens <= self.between_rows:
+        if ctx.num_tokens <= self.between_rows and self.norms_between:
             x, h = stream.x, stream.compute
             if h is None:
                 h = self.mixer_norm.ops.cast(x, self.mixer_norm.dtype)

@@ -1,7 +1,7 @@
 """Feed-forward parts."""
 from typing import Dict, List
 
-from .base import FeedForward, OffersRows, register_feed_forward, residual_to_product
+from .base import FeedForward, OffersRows, hands_residual_on, register_feed_forward, residual_to_product
 from .spec import ParamDecl
 
 
@@ -49,7 +49,7 @@ class DenseFeedForward(FeedForward):
         return self.w1
 
     def layer_form(self):
-        if type(self).forward is not DenseFeedForward.forward or self.activation == "poly_norm":
+        if type(self).forward is not DenseFeedForward.forward or not hands_residual_on(self) or self.activation == "poly_norm":
             return None
         return self.w1, self.b1, self.activation, self.w2, self.b2
 

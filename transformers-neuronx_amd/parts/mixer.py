@@ -4,7 +4,7 @@ from typing import Dict, List, Optional
 
 import torch
 
-from .base import POSITIONS, CacheNeed, Mixer, OffersRows, register_mixer, residual_to_product
+from .base import POSITIONS, CacheNeed, Mixer, OffersRows, hands_residual_on, register_mixer, residual_to_product
 from .spec import ParamDecl
 
 
@@ -239,7 +239,7 @@ class Attention(OffersRows, Mixer):
         return None if self.prepared else self.w_in
 
     def layer_form(self):
-        if (type(self).forward is not Attention.forward or self.prepared or not self.own_kv or self.rotation is not None
+        if (type(self).forward is not Attention.forward or not hands_residual_on(self) or self.prepared or not self.own_kv or self.rotation is not None
                 or self.window is not None or self.defer_out or self.defer_in or self.num_kv_heads != self.num_heads or self.head_size != 64):
             return None
         return self.w_in, self.b_in, self.w_out, self.b_out, self.num_heads, self.scale
