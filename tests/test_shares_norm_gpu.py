@@ -137,3 +137,30 @@ def test_through_the_model(tmp_path, dtype, before):
     with debug.debug_context() as kept:
         looked_at.step([StepEntry("more", [5 + i for i in range(60)], [59])])
     assert "tnx_shares_norm" not in made and sum("after_mixer" in name for name in kept) == 3
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m,switches", [(256, [("tile_products", False), ("library_rows", 0)]), (32, [("some_rows", False)])])
+def test_switches_turn_for_sizes_seen_before(m, switches):
+    """Products of 2,048 x 2,048 by tiles and by rows of some number: off and on again, whatever a size's way was the last time."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    hip, g, called = HipOps(BF16, DEV), _gen(m), []
+    call = hip._call
+    hip._call = lambda lib, name, *a, **k: (called.append(name), call(lib, name, *a, **k))[1]
+    x, residual = torch.randn(m, 2048, device=DEV, generator=g).to(BF16), torch.randn(m, 2048, device=DEV, generator=g)
+    w = hip.prepare_weight((torch.randn(2048, 2048, device=DEV, generator=g) * 0.02).to(BF16))
+
+    def left():
+        del called[:]
+        hip.settled(hip.linear(x, w, None, residual=hip.onto(residual), out_f32=True))
+        return "tnx_gemm_left" in called
+    for name, value in switches:
+        kept = getattr(hip, name)
+        assert left()
+        setattr(hip, name, value)
+        assert not left() and (name != "library_rows" or called == ["tnx_gemm_bf16"])
+        setattr(hip, name, kept)
+        assert left()
+        fresh = HipOps(BF16, DEV)
+        setattr(fresh, name, value)
+        assert fresh._way_to_leave(m, 2048, 2048, True) is None

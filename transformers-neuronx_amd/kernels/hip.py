@@ -799,9 +799,15 @@ class HipOps:
           four shares at most (39 rows 3,072 x 3,072, five: 11.5 / 11.6).
         Tiles of 128 x 128 with shares where the library has no shares were a loss as often as a gain (640 rows 2,048 x 2,048 18.9 /
         23.2)."""
-        if len(self._left_ways) > 4096:
-            self._left_ways.clear()
-        self._left_ways[m, n, k, copy] = way = self._choose_left(m, n, k, copy)
+        key = (m, n, k, copy, self.compute_units, self.shares_norm_width)
+        if key not in self._left_ways:
+            if len(self._left_ways) > 4096:
+                self._left_ways.clear()
+            self._left_ways[key] = self._choose_left(m, n, k, copy)
+        way = self._left_ways[key]
+        # (what is kept are sizes' ways; the switches may turn at any time)
+        if way is not None and not (self.some_rows if way[0] == 0 else self.tile_products and 0 < self.library_rows <= m):
+            return None
         return way
 
     def _choose_left(self, m, n, k, copy):
@@ -811,7 +817,7 @@ class HipOps:
         if copy and m <= 48 and units // columns >= 6:
             shares = min(units // columns, max(k // 512, min(4, k // 256)))
             return (0, 0, shares) if shares >= 3 and (m > 16 or k >= 3072) else None
-        if m <= (32 if units // columns < 5 else 48) or not self.tile_products:
+        if m <= (32 if units // columns < 5 else 48):
             return None
         shares = min(8, units // (-(-m // 64) * columns), k // 256)
         return (1, 1, shares) if shares >= 2 and k < 24 * 64 * shares else None
@@ -999,10 +1005,7 @@ class HipOps:
         if residual is not None:
             _want(residual, "residual", torch.float32, (m, n))
         if leaves and w.dtype == torch.bfloat16 and not force_tiled:
-            copy = tiles is not None
-            way = self._left_ways.get((m, n, k, copy), 0)
-            if way == 0:
-                way = self._way_to_leave(m, n, k, copy)
+            way = self._way_to_leave(m, n, k, tiles is not None)
             if way is not None and (_ptr(x) | _ptr(w) | _ptr(residual)) % 16 == 0:
                 way, tile, shares = way
                 return self._left(way, self.cast(x, torch.bfloat16), w if way else tiles, bias, residual, m, n, k, shares * m * n, tile, shares)
