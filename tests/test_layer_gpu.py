@@ -214,6 +214,55 @@ def test_fewer_blocks_do_the_same(dtype, width, inner, held, joined):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("page_size", [256, 1024])
+@pytest.mark.parametrize("dtype,width,inner,held", [(BF16, 1024, 4096, [2047, 255, 256]), (F32, 640, 1152, [700, 0, 1023, 1024])])
+def test_larger_pages_do_the_same(dtype, width, inner, held, page_size):
+    """Where keys lie changes no sum: the bits of pages of 64."""
+    print(f"pages {dtype} {width} {inner} {held} {page_size}", flush=True)
+    results = []
+    for size in (64, page_size):
+        ops, run, _ = _ready(dtype, width, inner, held, 11, page_size=size)
+        results.append(run())
+        ops.raise_if_lost()
+    assert torch.equal(*results) and bool(torch.isfinite(results[0]).all())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", ["pre_norm", "post_norm"])
+@pytest.mark.parametrize("dtype,held", [(BF16, [70, 700, 3]), (F32, [70, 300, 3]), (F32, [1, 12, 3, 40, 65])])
+def test_rows_that_are_no_numbers(dtype, held, block):
+    """Infinities and NaN (with the bits that stand for "not yet" as well) in one request's stream, keys or values: that row is finite
+    where it is by launches apart, and the others keep their bits."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    print(f"no numbers {dtype} {held} {block}", flush=True)
+    ops, width, inf = HipOps(dtype, DEV), 1024, float("inf")
+    layers = [_layer(ops, dtype, width, 1024, block, "relu", True, 50 + i)[0] for i in range(2)]
+    clean = (torch.randn(len(held), width, generator=torch.Generator().manual_seed(5)) * 2.0).to(DEV)
+    ones = torch.full((1,), -1, dtype=torch.int32, device=DEV).view(F32)
+
+    def run(how, where, value):
+        steps, x = [_step(ops, dtype, held, width, 64, 60, i) for i in range(2)], clean.clone()
+        ctx, cache, _ = steps[0]
+        page = int(ctx.groups["full"].block_table[1, 0])
+        if where == "x":
+            x[1, 77] = value
+        elif where == "keys":
+            cache.k_pages[page, 3, 10, 5] = value
+        elif where == "values":
+            cache.v_pages[page, 3, 5, 10] = value
+        return ops.settled(how(ops, layers, Stream(x, x.to(dtype)), steps).x).clone()
+    want = run(_in_one, None, None)
+    assert bool(torch.isfinite(want).all())
+    others = [r for r in range(len(held)) if r != 1]
+    for where in ("x", "keys", "values"):
+        for value in (inf, -inf, float("nan"), ones[0]):
+            got, apart = run(_in_one, where, value), run(_chain, where, value)
+            ops.raise_if_lost()
+            assert torch.equal(got[others], want[others]), (where, value)
+            assert torch.equal(torch.isfinite(got[1]), torch.isfinite(apart[1])), (where, value)
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("dtypes", [(F32,) * 6, (BF16,) * 8, (F32, BF16) * 4])
 def test_many_launches_at_a_time(dtypes):
     """More launches on streams of their own than have room together, each with its own engine: every one gives what it gives alone."""

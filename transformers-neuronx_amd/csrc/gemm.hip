@@ -2188,7 +2188,8 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 //   36.0 (a step of 64 of 6.7b's 6,075 with tiles there, 5,897 without).
 // Up to 32 rows half a tile would be padding (32 rows 10,240 x 2,560: 17.7 / 20), and other kernels stand ready.
 // What bounds these sizes is the time a unit takes for a step of its one block (0.55 us for 128 x 128 x 64, of which the
-// matrix cores work 0.24), not memory: shares of K are the way to keep all units at it.
+// matrix cores work 0.2 and LDS 0.15; the waves wait half of it, for loads from the caches and for each other), not memory (17.1 to
+// 17.8 us for 20.4 with 333 x 6,144 x 2,048 in the last cache): shares of K are the way to keep all units at it.
 enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2 };
 static int choose_tiles(int M, int N, int K, int& shares) {
   const int units = tnx_compute_units(), steps = K / 64;
