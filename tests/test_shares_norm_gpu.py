@@ -37,6 +37,8 @@ def test_sizes(shares, tokens, width, dtype):
         assert torch.equal(x, want) and torch.equal(h, norm) and h.dtype == dtype
         x, h = left().normed(w, b, 1e-5, dtype, center, alone=True)
         assert torch.equal(x, hip.layernorm(want, w, b, 1e-5, dtype, True, False, center)[0]) and torch.equal(h, norm)
+        x, h = left().normed(w, b, torch.tensor(1e-5), dtype, center)           # (any number, as the norm's own launch takes)
+        assert torch.equal(x, want) and torch.equal(h, norm)
         x, h = whole.normed(w, b, 1e-5, dtype, center)                          # one that was added already
         assert x is want and torch.equal(h, norm)
 

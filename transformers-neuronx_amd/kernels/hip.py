@@ -396,7 +396,7 @@ class SharesLeft:
         # (the product has made nothing of `out` yet: alone, the norm's float32 result lies there)
         x = (h if f32 else out) if alone else out
         self.ops._call("elementwise", "tnx_shares_norm", self.shares.data_ptr(), self.count, add, onto, None if alone else out.data_ptr(),
-                       scale, shift, eps, h.data_ptr() if f32 else out.data_ptr() if alone else None, None if f32 else h.data_ptr(), m, n,
+                       scale, shift, float(eps), h.data_ptr() if f32 else out.data_ptr() if alone else None, None if f32 else h.data_ptr(), m, n,
                        1 if center else 0, _stream(),
                        work=lambda: (f"{m}x{n}", m * n * (4 * self.count + 8 + h.element_size()), 0.0))
         self._done()
