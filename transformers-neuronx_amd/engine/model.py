@@ -186,7 +186,8 @@ class DecoderModel:
             if call < done:
                 continue
             block = self.layers[layer].block
-            if (left and (call in in_one or not getattr(block, "leaves_shares", False))
+            leaves = getattr(block, "leaves_shares", False)
+            if (left and (call in in_one or not leaves)
                     or between and not getattr(block, "norms_between", False)):
                 stream, left, between = self._settled(stream), False, False
             if call in in_one:
@@ -200,7 +201,7 @@ class DecoderModel:
             ctx.call_state = caches[state_id] if state_id is not None else None
             stream = block.forward(stream, ctx, cache)
             between = few and getattr(block, "norms_between", False)
-            left = getattr(block, "leaves_shares", False)
+            left = leaves
             debug.tap(f"call{call}.layer{layer}", stream.x)
         if between or left:
             stream = self._settled(stream)

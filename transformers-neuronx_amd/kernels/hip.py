@@ -485,6 +485,9 @@ def _stream():
 
 
 def _want(t: torch.Tensor, name: str, dtype=None, shape=None):
+    # (asked 600 times in a prompt of 24 layers: what is wanted first, in one line, and what is not by name)
+    if t.is_cuda and t.is_contiguous() and (dtype is None or t.dtype == dtype) and (shape is None or t.shape == shape):
+        return t
     if not t.is_cuda:
         raise ValueError(f"{name} must be on the GPU")
     if not t.is_contiguous():
@@ -666,9 +669,9 @@ class HipOps:
         return out, ((cd if cd is not None else out) if want_compute else None)
 
     def cast(self, x, dtype):
-        _want(x, "x")
-        if x.dtype == dtype:
+        if x.dtype == dtype and x.is_cuda and x.is_contiguous():
             return x
+        _want(x, "x")
         out = torch.empty_like(x, dtype=dtype)
         self._call("elementwise", "tnx_cast", _ptr(x), _code(x.dtype), _ptr(out), _code(dtype), x.numel(), _stream())
         return out
@@ -799,12 +802,11 @@ class HipOps:
           four shares at most (39 rows 3,072 x 3,072, five: 11.5 / 11.6).
         Tiles of 128 x 128 with shares where the library has no shares were a loss as often as a gain (640 rows 2,048 x 2,048 18.9 /
         23.2)."""
-        key = (m, n, k, copy, self.compute_units, self.shares_norm_width)
-        if key not in self._left_ways:
+        way = self._left_ways.get((m, n, k, copy), 0)
+        if way == 0:
             if len(self._left_ways) > 4096:
                 self._left_ways.clear()
-            self._left_ways[key] = self._choose_left(m, n, k, copy)
-        way = self._left_ways[key]
+            self._left_ways[m, n, k, copy] = way = self._choose_left(m, n, k, copy)
         # (what is kept are sizes' ways; the switches may turn at any time)
         if way is not None and not (self.some_rows if way[0] == 0 else self.tile_products and 0 < self.library_rows <= m):
             return None
@@ -824,7 +826,7 @@ class HipOps:
 
     def _left(self, way, x, w, bias, residual, m, n, k, room, tile=0, shares=0):
         """The product with its shares of K left apart (0: the tile and the shares that the product chooses itself)."""
-        out = torch.empty(m, n, dtype=torch.float32, device=x.device)
+        out = torch.empty_like(residual)
         space, left = torch.empty(room, dtype=torch.float32, device=x.device), _c_int()
         self._call("gemm", "tnx_gemm_left", way, _ptr(x), _ptr(w), _ptr(bias), _ptr(residual), _ptr(out), m, n, k, _ptr(space), room, tile, shares,
                    ctypes.addressof(left), _stream(),
@@ -1251,7 +1253,12 @@ class HipOps:
     def _check_pages(self, k_pages, v_pages, num_kv, head_size, page_size):
         """The number of pages. A page's own elements lie together; from page to page there may be more than a
         page's elements, the same for keys and values (`_page_pad`: how many more)."""
-        n = k_pages.shape[0]
+        n, area = k_pages.shape[0], page_size * head_size
+        strides, apart = k_pages.stride(), k_pages.stride(0) - num_kv * area
+        if (k_pages.is_cuda and v_pages.is_cuda and k_pages.dtype == v_pages.dtype == self.dtype and apart >= 0 and apart % 8 == 0
+                and k_pages.shape == (n, num_kv, page_size, head_size) and v_pages.shape == (n, num_kv, head_size, page_size)
+                and strides == (strides[0], area, head_size, 1) and v_pages.stride() == (strides[0], area, page_size, 1)):
+            return n
         for t, name, shape in ((k_pages, "key pages", (n, num_kv, page_size, head_size)),
                                (v_pages, "value pages", (n, num_kv, head_size, page_size))):
             if not t.is_cuda or t.dtype != self.dtype:

@@ -279,8 +279,8 @@ class Block(Part):
     def own_forwards(self) -> bool:
         """Whether a `forward` was put on this very block, a part or a norm of it, past its class. It is called then, with tensors,
         and nothing is done around it; asked in every step, since it may be put there, and taken away, at any time."""
-        return ("forward" in vars(self) or "forward" in vars(self.mixer) or "forward" in vars(self.feed_forward)
-                or "forward" in vars(self.mixer_norm) or "forward" in vars(self.feed_forward_norm))
+        return ("forward" in self.__dict__ or "forward" in self.mixer.__dict__ or "forward" in self.feed_forward.__dict__
+                or "forward" in self.mixer_norm.__dict__ or "forward" in self.feed_forward_norm.__dict__)
 
     def norms_in_one(self, before):
         """`Norm.fused_form` of what the layer's two halves read, where `before` is the block of the layer before in that launch."""
