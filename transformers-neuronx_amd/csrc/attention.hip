@@ -1759,12 +1759,19 @@ extern "C" int tnx_attention_prefill_scored(const void* q, const void* k_pages, 
 // every lane), which do not queue behind the tile data; the next tile's keys are asked for as soon as this
 // tile's scores are made, its values as soon as this tile's are used (NDB <= 8; beyond that the registers
 // hold one of the two at a time).
+// STAGED (pages of 64 keys and more, head sizes that the registers are laid out for): a tile's keys and values go straight into LDS,
+// 1 KB of one run of memory an instruction and marked as read once, and the products' operands come from there. Read as the operands
+// lie, in pieces of 64 bytes, every line is asked for twice, so the mark would cost it its second half (a kernel of these reads alone, 32
+// requests of 512 tokens and 32 heads of 80: 28.0 us, 32.6 with the mark; in whole runs 28.0 and 25.3 with it, 6.6 TB/s). Straight into
+// registers / staged, us: 32 heads of 80, 32 requests of up to 720 tokens 37.0 / 31.5, 24 of 400 25.6 / 20.1, 8 of 1,500 26.2 / 22.7; of 64,
+// 24 of 112 to 412 18.9 / 15.3, 40 of 145 to 520 27.1 / 22.4; of 128, 8 of 2,050 53.8 / 46.6, 40 of 1,500 169 / 151. Where a wave has
+// one tile at most the way through LDS costs 0.2 us (3 of 100, heads of 64: 5.2 / 5.4). How many waves a block has: `HipOps._splits_for`.
 // PACK: for query heads that share their keys and values (fewer kv heads than heads). A block then takes one
 // kv head of one request, and the 16 columns hold up to 16 (8 at the largest head size) different query heads
 // of its group, so the keys and values are read once for all of them and not once a head; the maxima, sums and
 // results are a column's own throughout (a column is the lanes with the same lane % 16).
-template <int NDB, int NW, bool PACK>
-__global__ void __launch_bounds__(64 * NW, (NDB <= 8 ? 8 / NW : 1))
+template <int NDB, int NW, bool PACK, bool STAGED>
+__global__ void __launch_bounds__(64 * NW, (NDB <= 8 ? 2 : 1))
 attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
                              const bf16_t* __restrict__ v_pages, const int* __restrict__ run_start,
                              const int* __restrict__ cached_lens, const int* __restrict__ table, int table_width,
@@ -1776,8 +1783,18 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
   constexpr int DH = 16 * NDB;        // the registers are laid out for this head size; `head_size` <= DH
   constexpr bool PIPE = NDB <= 8;     // keys and values of different tiles are in registers together
   constexpr int COLS = !PACK ? 1 : NDB <= 8 ? 16 : 8;     // query heads a block takes (what LDS holds of results)
-  __shared__ float sm_o[NW][COLS][DH];
-  __shared__ float sm_m[NW][COLS], sm_l[NW][COLS];
+  static_assert(!STAGED || PIPE, "keys and values of a wave that do not fit LDS");
+  extern __shared__ __attribute__((aligned(16))) char stages[];             // STAGED: a tile's keys and values of every wave
+  float* merged;                // where the waves' results meet: the stages, when no one reads them any more
+  if constexpr (STAGED) {
+    merged = (float*)stages;
+  } else {
+    __shared__ float room[NW * COLS * (DH + 2)];
+    merged = room;
+  }
+  float(*sm_o)[COLS][DH] = (float(*)[COLS][DH])merged;
+  float(*sm_m)[COLS] = (float(*)[COLS])(merged + NW * COLS * DH);
+  float(*sm_l)[COLS] = (float(*)[COLS])(merged + NW * COLS * (DH + 1));
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r = lane & 15, g = lane >> 4;
   const int split = blockIdx.x, dz = blockIdx.z;
@@ -1837,6 +1854,52 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
     }
   };
 
+  // STAGED: a tile's keys, 64 rows of CPR chunks of 16 bytes, and its values, DH rows of 8, one run of memory each; the chunks of a row
+  // lie swizzled so that the fragments' reads of 16 rows meet few banks twice
+  constexpr int CPR = DH / 8, LOADS = DH / 8;
+  const char* k_mine = stages + wave * DH * 256;
+  const char* v_mine = k_mine + DH * 128;
+  auto k_swizzle = [](int m) {
+    return CPR == 16 ? ((m >> 3) & 3) * 4 + (m & 3) : CPR == 8 ? ((m >> 3) & 3) * 2 + ((m >> 1) & 1) : CPR == 4 ? (m >> 3) & 3 : 0;
+  };
+  unsigned koff[STAGED ? LOADS : 1], voff[STAGED ? LOADS : 1];
+  if constexpr (STAGED) {
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+      const int c = 64 * i + lane, m = c / CPR;
+      koff[i] = (unsigned)((m * CPR + ((c % CPR) ^ k_swizzle(m))) * 16);
+      const int d = c >> 3;
+      voff[i] = (unsigned)(d * page_size * 2 + ((c & 7) ^ ((d >> 1) & 7)) * 16);
+    }
+  }
+  auto stage_keys = [&](int page, int tile0) {
+    const bf16_t* kp = k_pages + (size_t)page * page_stride + (size_t)kvh * head_stride + (size_t)(tile0 & pmask) * DH;
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load_to_lds_once(kp, koff[STAGED ? i : 0], lds_offset(k_mine) + i * 1024);
+  };
+  auto stage_values = [&](int page, int tile0) {
+    const bf16_t* vp = v_pages + (size_t)page * page_stride + (size_t)kvh * head_stride + (tile0 & pmask);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) load_to_lds_once(vp, voff[STAGED ? i : 0], lds_offset(v_mine) + i * 1024);
+  };
+  auto page_of = [&](int tile0) {
+    const int key = __builtin_amdgcn_readfirstlane(min(tile0, last_key));
+    return __builtin_amdgcn_readfirstlane(min(max(tab[key >> page_shift], 0), num_pages - 1));
+  };
+  auto ask_keys = [&](int (&pg)[4], int tile0) {
+    if constexpr (STAGED) {
+      pg[0] = page_of(tile0);
+      stage_keys(pg[0], tile0);
+    } else {
+      lookup(pg, tile0);
+      load_keys(pg, tile0);
+    }
+  };
+  auto ask_values = [&](const int (&pg)[4], int tile0) {
+    if constexpr (STAGED) stage_values(pg[0], tile0);
+    else load_values(pg, tile0);
+  };
+
   int pg[4], pgn[4];
   int tile0 = 0;
   bool fetched = false;
@@ -1845,9 +1908,8 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
     // are valid whatever it turns out to be, and masked afterwards
     tile0 = split * keys_per_split + 64 * wave;
     if (64 * wave < keys_per_split) {
-      lookup(pg, tile0);
-      load_keys(pg, tile0);
-      if (PIPE) load_values(pg, tile0);
+      ask_keys(pg, tile0);
+      if (PIPE) ask_values(pg, tile0);
       fetched = true;
     }
   }
@@ -1868,13 +1930,23 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
   for (int db = 0; db < NDB; ++db) o[db] = (f32x4){0.f, 0.f, 0.f, 0.f};
 
   if (tile0 < k_end && !fetched) {
-    lookup(pg, tile0);
-    load_keys(pg, tile0);
-    if (PIPE) load_values(pg, tile0);
+    ask_keys(pg, tile0);
+    if (PIPE) ask_values(pg, tile0);
   }
   while (tile0 < k_end) {
     const int next = tile0 + 64 * NW;
     const bool more = next < k_end;
+    if constexpr (STAGED) {
+      // the keys have landed when only the values of this tile are in flight
+      asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+#pragma unroll
+      for (int kb = 0; kb < 4; ++kb) {
+        const int m = 32 * (kb >> 1) + 8 * (r >> 2) + 4 * (kb & 1) + (r & 3);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+          kf[kb][ks] = *(const bf16x8*)(k_mine + (m * CPR + (min(4 * ks + g, CPR - 1) ^ k_swizzle(m))) * 16);
+      }
+    }
     f32x4 sc[4];
 #pragma unroll
     for (int kb = 0; kb < 4; ++kb) {
@@ -1885,8 +1957,8 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
       sc[kb] = a;
     }
     if (PIPE && more) {
-      lookup(pgn, next);
-      load_keys(pgn, next);
+      if constexpr (STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the products have read the keys that were here)
+      ask_keys(pgn, next);
     }
     // sc[kb][i] of a lane is the score of key tile0 + 32 (kb / 2) + 8 g + 4 (kb % 2) + i, the same in the 16
     // lanes of a row group
@@ -1919,6 +1991,17 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
     l = l * alpha + sum;
     m = m_new;
     if (!PIPE) load_values(pg, tile0);
+    if constexpr (STAGED) {
+      if (more) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(LOADS) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int st = 0; st < 2; ++st) {
+          const int d = 16 * db + r;
+          vf[db][st] = *(const bf16x8*)(v_mine + (d * 8 + ((4 * st + g) ^ ((d >> 1) & 7))) * 16);
+        }
+    }
     if (edge) {
       // values of keys that are not the request's (beyond its end, before its window, in a page that was given
       // back) may be anything: their probabilities are zero, and they must not be NaN
@@ -1942,13 +2025,18 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
     }
     if (more) {
       if (PIPE) {
-        load_values(pgn, next);
+        if constexpr (STAGED) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        ask_values(pgn, next);
       } else {
         lookup(pg, next);
         load_keys(pg, next);
       }
     }
     tile0 = next;
+  }
+  if constexpr (STAGED) {
+    wait_for_loads();       // a first tile that turned out to be beyond the request's end lands too before what follows goes there
+    __syncthreads();
   }
   // o[db][i] of a lane is element 16 db + 4 g + i of the weighted values of its column (without PACK the same in
   // the 16 lanes of a row group)
@@ -2046,6 +2134,19 @@ __global__ void attention_decode_merge_kernel(const float* __restrict__ part_o, 
   }
 }
 
+template <int NDB, int NW, bool PACK, typename... Args>
+static int launch_decode_staged(dim3 grid, hipStream_t stream, Args... args) {
+  constexpr int bytes = NW * 16 * NDB * 256;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void*)attention_decode_mfma_kernel<NDB, NW, PACK, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "attention_decode: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  attention_decode_mfma_kernel<NDB, NW, PACK, true><<<grid, 64 * NW, bytes, stream>>>(args...);
+  return 0;
+}
+
 static int attention_decode_run(const void* q, const void* k_pages, const void* v_pages, const int* run_start,
                                 const int* cached_lens, const int* table, int table_width, int page_size,
                                 int num_pages, const int* decode_runs, int num_decode, void* out, float* part_o,
@@ -2062,7 +2163,7 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   TNX_REQUIRE(num_splits >= 1 && longest != nullptr, "attention_decode: bad split count or no length given");
   TNX_REQUIRE(num_splits == 1 || (part_o && part_ml), "attention_decode: splits need a workspace");
   TNX_REQUIRE(num_heads <= 65535 && num_decode <= 65535, "attention_decode: too many heads or requests");
-  TNX_REQUIRE(waves == 4 || (waves == 8 && head_size <= 128),
+  TNX_REQUIRE(waves == 4 || waves == 2 || (waves == 8 && head_size <= 128),
               "attention_decode: blocks have 4 waves, or 8 up to head size 128; not %d at head size %d", waves, head_size);
   if (num_decode <= 0) return 0;
   // query heads that share keys and values are taken together, up to 16 a block (8 at head sizes beyond 128)
@@ -2070,22 +2171,28 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   const bool pack = group > 1;
   const int cols = head_size <= 128 ? 16 : 8;
   dim3 grid(num_splits, pack ? num_kv * ((group + cols - 1) / cols) : num_heads, num_decode);
+  const bool staged = page_size >= 64 && (head_size == 32 || head_size == 64 || head_size == 80 || head_size == 96 || head_size == 128);
 #define MFMA_ARGS                                                                                                 \
   (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, run_start, cached_lens, table, table_width,    \
       page_shift, num_pages, decode_runs, (bf16_t*)out, part_o, part_ml, num_heads, num_kv, window, num_splits,    \
       longest, head_size, page_pad
-#define LAUNCH_MFMA(NDB)                                                                         \
-  if (waves == 8 && pack)                                                                        \
-    attention_decode_mfma_kernel<NDB, 8, true><<<grid, 512, 0, stream>>>(MFMA_ARGS);             \
-  else if (waves == 8)                                                                           \
-    attention_decode_mfma_kernel<NDB, 8, false><<<grid, 512, 0, stream>>>(MFMA_ARGS);            \
-  else if (pack)                                                                                 \
-    attention_decode_mfma_kernel<NDB, 4, true><<<grid, 256, 0, stream>>>(MFMA_ARGS);             \
-  else                                                                                           \
-    attention_decode_mfma_kernel<NDB, 4, false><<<grid, 256, 0, stream>>>(MFMA_ARGS)
-    // the registers are laid out for the next of these sizes; a smaller head repeats its last chunk there. 80 has a size
-    // of its own: laid out for 96 it reads its last sixth twice, 34.1 us against 34.8 for 32 requests of up to 700 tokens
-    // and 32 heads, 23.2 against 23.8 for 24 of them, 37.0 against 37.3 for 8 of 2,048.
+#define LAUNCH_STAGED(NDB, NW, PACK) launch_decode_staged<NDB, NW, PACK>(grid, stream, MFMA_ARGS)
+#define LAUNCH_MFMA(NDB)                                                                                                   \
+  if (staged) {                                                                                                            \
+    constexpr int MOST = NDB <= 5 ? 8 : 4;                                                                                 \
+    if (int rc = waves >= MOST ? (pack ? LAUNCH_STAGED(NDB, MOST, true) : LAUNCH_STAGED(NDB, MOST, false))                 \
+                 : waves == 4  ? (pack ? LAUNCH_STAGED(NDB, 4, true) : LAUNCH_STAGED(NDB, 4, false))                       \
+                               : (pack ? LAUNCH_STAGED(NDB, 2, true) : LAUNCH_STAGED(NDB, 2, false)))                      \
+      return rc;                                                                                                           \
+  } else if (waves == 8 && pack)                                                                                           \
+    attention_decode_mfma_kernel<NDB, 8, true, false><<<grid, 512, 0, stream>>>(MFMA_ARGS);                                \
+  else if (waves == 8)                                                                                                     \
+    attention_decode_mfma_kernel<NDB, 8, false, false><<<grid, 512, 0, stream>>>(MFMA_ARGS);                               \
+  else if (pack)                                                                                                           \
+    attention_decode_mfma_kernel<NDB, 4, true, false><<<grid, 256, 0, stream>>>(MFMA_ARGS);                                \
+  else                                                                                                                     \
+    attention_decode_mfma_kernel<NDB, 4, false, false><<<grid, 256, 0, stream>>>(MFMA_ARGS)
+    // the registers are laid out for the next of these sizes; a smaller head repeats its last chunk there. 80 has a size of its own.
     if (head_size <= 32) {
       LAUNCH_MFMA(2);
     } else if (head_size <= 64) {
@@ -2097,12 +2204,13 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
     } else if (head_size <= 128) {
       LAUNCH_MFMA(8);
     } else if (pack) {
-      attention_decode_mfma_kernel<16, 4, true><<<grid, 256, 0, stream>>>(MFMA_ARGS);
+      attention_decode_mfma_kernel<16, 4, true, false><<<grid, 256, 0, stream>>>(MFMA_ARGS);
     } else {
-      attention_decode_mfma_kernel<16, 4, false><<<grid, 256, 0, stream>>>(MFMA_ARGS);
+      attention_decode_mfma_kernel<16, 4, false, false><<<grid, 256, 0, stream>>>(MFMA_ARGS);
     }
 #undef MFMA_ARGS
 #undef LAUNCH_MFMA
+#undef LAUNCH_STAGED
   TNX_CHECK_LAUNCH("attention_decode");
   if (num_splits > 1) {
     attention_decode_merge_kernel<<<dim3(num_heads, num_decode), head_size < 64 ? 64 : head_size, 0, stream>>>(

@@ -1567,9 +1567,8 @@ class HipOps:
     prefill_direct = False            # tests set it: True, the prompt kernel that reads pages without LDS staging;
                                       # 2, the staged one with one set of four waves a block; 3, with two
     force_plain_attention = False     # tests set it to run the one-wave-per-query kernel in bfloat16 too
-    decode_waves = 4                  # waves of a decode attention block (8 is kept for head sizes up to 128)
-    decode_blocks_wanted = None       # the keys of decoding requests are split until about this many blocks run;
-                                      # None: one block a compute unit
+    decode_waves = None               # tests set it to 8: so many waves a decode attention block (head sizes up to 128)
+    decode_blocks_wanted = None       # tests set it: the keys of decoding requests are split until about this many blocks run
 
     @staticmethod
     def _decode_blocks(num_heads: int, num_kv_heads: int, head_size: int) -> int:
@@ -1581,42 +1580,46 @@ class HipOps:
         return num_kv_heads * -(-group // (16 if head_size <= 128 else 8))
 
     def _decode_splits(self, ctx, pairs: int, window: int, head_size: int = 128):
-        """(splits, waves): how many blocks share the keys of one decoding (request, head), and how many
-        waves a block has. Blocks of four waves: with the products on the matrix unit a wave keeps the
-        next tile's keys and values in flight by itself, and more waves bought nothing (measured at head
-        size 128 and a context of 2,048: one request 8 x 4 waves 15.6 us against 16.9 for 4 x 8; eight
-        requests 49.7 against 50.9; 64 requests 369 against 376).
-        No block gets less than 256 keys of the longest request (a 64-key tile a wave). Requests about as
-        long as one another are cut into as many blocks as that allows, up to 8: small blocks spread evenly
-        over the compute units whatever the number of pairs (32 heads at 2,048 tokens, tokens a second: 9
-        requests 1,582 -> 1,801, 20: 2,388 -> 2,545, 33: 3,067 -> 3,150, 128: 4,398 -> 4,487), except
-        where the pairs alone give 0.7 to 1 block a compute unit (7 and 8 requests: whole requests, 1,548
-        against 1,520 and 1,675 against 1,654) or a whole number of blocks each, within a twentieth (16, 24,
-        32, 48, 64 requests: the many small blocks and the kernel that merges them cost 2 to 3 % there and
-        have nothing to even out). Requests of very different lengths are not cut beyond what
-        gives every compute unit a block: most blocks of a short request would be empty (64 requests of 16
-        to 1,280 tokens: 6,430 tokens a second whole, 4,760 in eight blocks each). A recorded step is sized
-        by the same two facts, which are part of what it is recorded under."""
+        """(splits, waves): how many blocks share the keys of one decoding (request, head), and how many waves a block has
+        (`_splits_for`)."""
         longest = ctx.length_bound if ctx.length_bound is not None else ctx.plan_host["longest_decode"]
         fills, alike = ctx.plan_host.get("decode_shape", (0, False))
         return self._splits_for(longest, fills, alike, pairs, window, head_size)
 
     def _splits_for(self, longest: int, fills: int, alike: bool, pairs: int, window: int, head_size: int):
+        """`fills`: the blocks of 256 keys that the longest request fills now, `longest` what it may come to before a recorded step is
+        replaced. `pairs`: blocks that read whole requests. A block of four waves fills half of a unit's LDS up to heads of 80,
+        all of it beyond, where eight do not fit. us, 32 heads of 64 or 80 or (so marked) 128 where nothing else is said:
+        - the pairs leave half of the units idle, or two thirds up to heads of 80, and the keys are many: as many blocks as units share
+          them (1 request of 2,000 20.5 whole / 10.6 in eight, 2 of 128 21 / 17.1 in four, 3 of 128 26.4 / 22.3 in two; but 1 of 700
+          8.5 / 9.4, and 3 of 1,000 11.2 / 12.0 in two, since the kernel that merges costs 2);
+        - at most one block a unit: as many waves as 256 keys, twice and four times as many keep at a tile or two each (1 of 100 5.0 with two,
+          5.2 with four, 5.4 with eight; 500 9.0, 7.9, 8.1; 5 of 700 12.2, 10.6, 10.0); four where nearly all units have a block;
+        - more pairs than units, not a whole number on each, of requests about as long as one another: shares of the keys come out
+          more even (9 of 2,000 37.6 / 34.2 in four, of 128 900 32.9 / 30.3 with two waves; but 33 of 900 53.9 / 60.4). Requests of
+          unlike lengths are not cut (24 of up to 1,500 43.5 / 51.4 in two);
+        - else blocks of two waves where requests are short, of which more are on a unit at once and none waits for another's end: 24 of
+          up to 400, heads of 80 18.5 with four / 14.8, 64 of 128 72 / 51.5; 24 of 1,500 58.3 / 58.7, of 128 93.8 / 98.9."""
+        most = min(8, fills)          # shares of 256 keys now, or of what a request may come to
         if not alike:
-            fills = min(8, -(-longest // 256))
+            most = min(8, -(-longest // 256))
         if window:
-            longest = min(longest, window + 64)
-            fills = min(fills, -(-longest // 256))
-        waves = 8 if self.decode_waves == 8 and head_size <= 128 else 4
-        units = self.decode_blocks_wanted or self.compute_units
-        if self.decode_blocks_wanted:                  # told how many blocks to make (measurements and tests)
-            return max(1, min(-(-units // pairs), -(-longest // 256))), waves
-        if 0.7 * units <= pairs <= units:
-            return 1, waves
-        fill_the_chip = max(1, min(-(-units // pairs), fills))
-        if pairs > units and -(-pairs // units) * units <= 1.05 * pairs:
-            alike = False         # whole requests already come out even over the compute units
-        return (max(fill_the_chip, fills) if alike else fill_the_chip), waves
+            within = -(-min(longest, window + 64) // 256)
+            fills, most = min(fills, within), min(most, within)
+        units, wide = self.compute_units, head_size > 80
+        if self.decode_blocks_wanted or self.decode_waves == 8:     # told what to make (measurements and tests)
+            blocks = self.decode_blocks_wanted or units
+            return max(1, min(-(-blocks // pairs), -(-longest // 256))), 8 if self.decode_waves == 8 and head_size <= 128 else 4
+        shares = min(most, units // pairs)
+        if shares > (1 if wide else 2) and fills > (2 if wide else 3):
+            return shares, 4
+        if pairs <= units:
+            return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or (wide and fills > 2) else 2 if fills <= 1 else 8
+        if alike and fills >= (4 if wide else 8) and -(-pairs // units) * units > 1.05 * pairs:
+            return 4, 2 if wide else 4
+        if not wide and pairs <= 2 * units:
+            return 1, 4
+        return 1, 2 if fills <= (4 if wide else 2) else 4
 
     def attention_launch_shape(self, step, num_heads: int, window, head_size: int, num_kv_heads: Optional[int] = None):
         """What the decode attention's launch in a recorded step is sized by beyond the number of requests: the
