@@ -153,9 +153,9 @@ __device__ __forceinline__ float block_sum(float v, float* scratch) {
 }
 
 __device__ __forceinline__ float apply_act(float x, int act) {
+  // (the two that cost nothing first: the code of the others is then out of their way)
+  if (__builtin_expect(act == TNX_ACT_NONE || act == TNX_ACT_RELU, 1)) return act == TNX_ACT_RELU ? fmaxf(x, 0.f) : x;
   switch (act) {
-    case TNX_ACT_RELU:
-      return fmaxf(x, 0.f);
     case TNX_ACT_GELU:
       return 0.5f * x * (1.f + erff(x * 0.70710678118654752440f));
     case TNX_ACT_GELU_NEW: {
@@ -169,6 +169,23 @@ __device__ __forceinline__ float apply_act(float x, int act) {
     default:
       return x;
   }
+}
+
+// The activation chosen once for many elements: `f` is called with a function that has made the choice. Chosen for each of the 16 to 48
+// elements of a lane in unrolled code, those that are not used lie between those that are: kernels of 30 to 80 KB, of which a launch
+// fetches line after line from wherever the other kernels of a step have left them. Products of a prompt of 333 tokens of 1.3b, as they
+// run in a step, before / with it: 54 KB of code 22.6 / 20.6 us with ReLU, 29 KB 14.3 / 13.4 without; the prompt 2,683 / 2,574 us.
+template <int ACT>
+struct Activation {
+  __device__ __forceinline__ float operator()(float x) const { return apply_act(x, ACT); }
+};
+template <typename F>
+__device__ __forceinline__ void with_act(int act, F f) {
+  if (act == TNX_ACT_RELU) f(Activation<TNX_ACT_RELU>{});
+  else if (act == TNX_ACT_GELU) f(Activation<TNX_ACT_GELU>{});
+  else if (act == TNX_ACT_GELU_NEW) f(Activation<TNX_ACT_GELU_NEW>{});
+  else if (act == TNX_ACT_RELU2) f(Activation<TNX_ACT_RELU2>{});
+  else f(Activation<TNX_ACT_NONE>{});
 }
 
 // What a softmax's running maximum `m` and sum `l` (of exp(score - m) over the visible keys) make of the weighted

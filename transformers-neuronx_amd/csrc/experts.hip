@@ -14,20 +14,20 @@ TNX_DEFINE_ERROR_API
 
 namespace {
 
-__device__ __forceinline__ float gate_act(float x, int act) {
-  if (act == TNX_ACT_SILU) return x / (1.f + expf(-x));
-  return apply_act(x, act);
-}
-
 // What a gated expert makes of the two halves of its first product: act(g) * u; the clamped form, with
-// g' = min(g, limit) and u' = clamp(u, -limit, limit): g' sigmoid(1.702 g') (u' + 1).
-__device__ __forceinline__ float gated(float g, float u, int act, float limit) {
-  if (act == TNX_ACT_CLAMPED_SWIGLU) {
-    g = fminf(g, limit);
-    u = fminf(fmaxf(u, -limit), limit);
-    return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
-  }
-  return gate_act(g, act) * u;
+// g' = min(g, limit) and u' = clamp(u, -limit, limit): g' sigmoid(1.702 g') (u' + 1). Chosen once for many elements (`with_act`).
+template <typename F>
+__device__ __forceinline__ void with_gate(int act, float limit, F f) {
+  if (__builtin_expect(act == TNX_ACT_SILU, 1))
+    f([](float g, float u) { return g / (1.f + expf(-g)) * u; });
+  else if (act == TNX_ACT_CLAMPED_SWIGLU)
+    f([limit](float g, float u) {
+      g = fminf(g, limit);
+      u = fminf(fmaxf(u, -limit), limit);
+      return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
+    });
+  else
+    with_act(act, [&](auto activation) { f([activation](float g, float u) { return activation(g) * u; }); });
 }
 
 // ---------------------------------------------------------------- the router's choice
@@ -259,7 +259,7 @@ __global__ void __launch_bounds__(256) expert_product_kernel(ProductArgs p) {
     if (GATED) {
       float g = acc[0][r], u = acc[GATED ? 1 : 0][r];
       if (p.weight_on_input) g *= w, u *= w;
-      ((T*)p.out)[(size_t)pair * p.n + col] = from_f32<T>(gated(g, u, p.act, p.limit));
+      with_gate(p.act, p.limit, [&](auto gate) { ((T*)p.out)[(size_t)pair * p.n + col] = from_f32<T>(gate(g, u)); });
     } else if (UP) {
       ((T*)p.out)[(size_t)pair * p.n + col] = from_f32<T>(apply_act(acc[0][r], p.act));
     } else {
@@ -403,16 +403,22 @@ __global__ void __launch_bounds__(256 * PARTS) expert_product_mfma_kernel(Produc
   }
   if (pair < 0) return;
   if (!FOUND) weight = p.weights[pair];
+  if constexpr (GATED)
+    with_gate(p.act, p.limit, [&](auto gate) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = p.weight_on_input ? gate(acc[i] * weight, acc_up[i] * weight) : gate(acc[i], acc_up[i]);
+    });
+  else if constexpr (UP)
+    with_act(p.act, [&](auto activation) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) acc[i] = activation(acc[i]);
+    });
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
     const int col = col0 + 4 * g + i;        // the lane holds columns 4 g .. 4 g + 3 of pair r
     if (col >= p.n) continue;
-    if (GATED) {
-      float gt = acc[i], up = acc_up[i];
-      if (p.weight_on_input) gt *= weight, up *= weight;
-      ((bf16_t*)p.out)[(size_t)pair * p.n + col] = (bf16_t)gated(gt, up, p.act, p.limit);
-    } else if (UP) {
-      ((bf16_t*)p.out)[(size_t)pair * p.n + col] = (bf16_t)apply_act(acc[i], p.act);
+    if (UP) {
+      ((bf16_t*)p.out)[(size_t)pair * p.n + col] = (bf16_t)acc[i];
     } else {
       float y = acc[i];
       if (!p.weight_on_input) y *= weight;
@@ -509,14 +515,28 @@ __global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
   }
   t.run(smem, p.a, w, p.k / 64);
   if constexpr (GATED) {
+    with_gate(p.act, p.limit, [&](auto gate) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) t.acc[i][0][e] = gate(t.acc[i][0][e] * weight[i], t.acc[i][1][e] * weight[i]);
+    });
     t.template hand_out<bf16_t, 32>(
-        smem, [&](int i, int, int e, int, int) { return gated(t.acc[i][0][e] * weight[i], t.acc[i][1][e] * weight[i], p.act, p.limit); },
+        smem, [&](int i, int, int e, int, int) { return t.acc[i][0][e]; },
         [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((bf16_t*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
   } else if constexpr (UP) {
+    with_act(p.act, [&](auto activation) {
+#pragma unroll
+      for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+          for (int e = 0; e < 16; ++e) t.acc[i][j][e] = activation(t.acc[i][j][e]);
+    });
     t.template hand_out<bf16_t, 64>(
-        smem, [&](int i, int j, int e, int, int) { return apply_act(t.acc[i][j][e], p.act); },
+        smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
         [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((bf16_t*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
@@ -604,8 +624,10 @@ __global__ void gated_activation_kernel(const float* __restrict__ gu, T* __restr
     const float w = row_weights ? row_weights[t] : 1.f;
     const fv g = ((const fv*)gu)[at], u = ((const fv*)gu)[at + pieces];
     tv o;
+    with_gate(act, limit, [&](auto gate) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) o[e] = from_f32<T>(gated(w * g[e], w * u[e], act, limit));
+      for (int e = 0; e < V; ++e) o[e] = from_f32<T>(gate(w * g[e], w * u[e]));
+    });
     ((tv*)out)[i] = o;
   }
 }
@@ -624,8 +646,10 @@ __global__ void row_activation_kernel(const float* __restrict__ x, long long ld,
     const fv v = *(const fv*)(x + t * ld + V * c);
     const float w = row_gate ? 1.f / (1.f + expf(-row_gate[t * gate_ld])) : 1.f;
     tv o;
+    with_act(act, [&](auto activation) {
 #pragma unroll
-    for (int e = 0; e < V; ++e) o[e] = from_f32<T>(apply_act(v[e], act) * w);
+      for (int e = 0; e < V; ++e) o[e] = from_f32<T>(activation(v[e]) * w);
+    });
     ((tv*)out)[i] = o;
   }
 }

@@ -525,10 +525,34 @@ gemm_f32_parts_kernel(const float* __restrict__ x, const float* __restrict__ w, 
   for (int j = 0; j < NI; ++j)
 #pragma unroll
     for (int e = 0; e < 16; ++e) added[j][e] = bias ? bias[min(nw + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3), N - 1)] : 0.f;
-  auto value = [&](int i, int j, int e, int row, int column) {
-    const float v = mw + row < M && nw + column < N ? checked(acc[i][j][e], mw + row, nw + column) : 0.f;
-    return apply_act(v + added[j][e], act);
-  };
+  // (one question for all elements, as a rule none is: the way that is not taken stays out of the other's code)
+  float none = 0.f;
+#pragma unroll
+  for (int i = 0; i < MI; ++i)
+#pragma unroll
+    for (int j = 0; j < NI; ++j)
+#pragma unroll
+      for (int e = 0; e < 16; ++e) none += acc[i][j][e] * 0.f;
+  if (__builtin_expect(none != none, 0)) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+          const int m = mw + 32 * i + l32, n = nw + 32 * j + 8 * (e >> 2) + 4 * half + (e & 3);
+          if (m < M && n < N) acc[i][j][e] = checked(acc[i][j][e], m, n);
+        }
+  }
+  with_act(act, [&](auto activation) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) acc[i][j][e] = activation(acc[i][j][e] + added[j][e]);
+  });
+  auto value = [&](int i, int j, int e, int, int) { return acc[i][j][e]; };
   Tile<MI, NI, 2, WM, WN>::template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk, int) {
     if (mw + r >= M || nw + c >= N) return;
     const size_t o = (size_t)(mw + r) * N + nw + c;
@@ -1848,6 +1872,13 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_
   }
   wait_for_loads();             // the loads beyond the last step write to LDS: they end before the block does
   // acc[t][e] of a lane is row m = 16 t + r of the output at column 16 tile + 4 g + e
+  if (!SCATTER && shares == 1)
+    with_act(act, [&](auto activation) {
+#pragma unroll
+      for (int t = 0; t < MT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[t][e] = activation(acc[t][e] + add[e]);
+    });
   if (n < N) {
     bool fours = ((uintptr_t)out & 15) == 0;
     if constexpr (SCATTER) fours = qkv_in_fours(sc);
@@ -1864,9 +1895,7 @@ gemm_bf16_mid_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w_
           for (int e = 0; e < 4; ++e) qkv_store(v[e], v[e ^ 1], m, n + e, sc, page[t], off[t]);
         }
       } else if (shares == 1) {
-        f32x4 v = acc[t] + add;
-#pragma unroll
-        for (int e = 0; e < 4; ++e) v[e] = apply_act(v[e], act);
+        f32x4 v = acc[t];
         const size_t o = (size_t)m * N + n;
         if (residual) {
 #pragma unroll
@@ -1929,8 +1958,10 @@ gemm_mid_sum_kernel(const float* __restrict__ partial, const float* __restrict__
     for (int s = 1; s < shares; ++s) v += *(const f32x4*)(partial + (size_t)s * M * N + i);
   }
   v += add;
+  with_act(act, [&](auto activation) {
 #pragma unroll
-  for (int e = 0; e < 4; ++e) v[e] = apply_act(v[e], act);
+    for (int e = 0; e < 4; ++e) v[e] = activation(v[e]);
+  });
   store_four(v + onto, out, out_dtype, i, fours);
 }
 
@@ -2125,7 +2156,15 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_bf16_tiles_kernel(const bf1
         });
     return;
   }
-  auto value = [&](int i, int j, int e, int, int) { return apply_act(t.acc[i][j][e] + added[j][e], act); };
+  with_act(act, [&](auto activation) {
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+      for (int j = 0; j < NI; ++j)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) t.acc[i][j][e] = activation(t.acc[i][j][e] + added[j][e]);
+  });
+  auto value = [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; };
   if (out_dtype == TNX_F32) {
     t.template hand_out<float, 32 * NI>(smem, value, [&](int r, int c, f32x4 chunk, int k) {
       if (residual) chunk += onto[k];
