@@ -2198,63 +2198,62 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 }
 
 // Which products these tiles take, and with which tile and how many shares of K (0: none, the vendor library).
-// Two things count. A call of the library's takes the host some 13 us, a launch of ours 5, and a step that is not recorded is
-// bound by the host where its products take less: there the tiles win whole steps also where they take longer than the
-// library's kernel (prompts, us, with the library wherever that kernel is quicker / with the tiles: 1.3b 150 tokens 3,121 / 2,434,
-// 256 tokens 3,240 / 2,670, 2.7b 60 tokens 4,029 / 3,529, 350m 600 tokens 2,899 / 2,492). From some 30 us a product on the
-// device bounds the step, and there the quicker kernel is taken. Measured on weights that no cache holds, us, library / tiles
-// (with bias and ReLU, or the residual where a matrix is narrower than K), at 33 to 768 rows:
-//   K at least four times the columns: tiles of 128 x 128 with as many shares of K as give every unit a block. 144 rows 2,048
-//   (columns) x 8,192 (K) 24.6 / 19.8, 2,560 x 10,240 32.3 / 26.0, 4,096 x 16,384 73.8 / 48.2, 5,120 x 20,480 123 / 71; 333 rows
-//   38.3 / 26.3, 49.0 / 35.5, 83.0 / 78.8, 142 / 106; 640 rows 43.8 / 37.6, 67.0 / 60.4, -, 224 / 193. Fewer rows come here only
-//   where `gemm_bf16_mid` has no copy of the weight: 33 rows 1,024 x 4,096 11.4 / 11.2, 2,048 x 8,192 14.4 / 16.9, 2,560 x 10,240
-//   23.1 / 20.6, 4,096 x 16,384 36.6 / 39.4, 64 rows 11.4 / 11.9, 16.8 / 17.0, 27.8 / 21.5, 43.9 / 39.5. Above 128 rows K beyond
-//   4,096 has to give more than half of the units a block, and three quarters above 576 rows (4,096 x 16,384, 160 blocks: 560
-//   rows 124 / 119, 600 rows 119 / 131, 640 rows 119 / 141; 700 rows 3,072 x 12,288, 144 blocks, 88 / 98), and above 704 rows the
-//   library has a better tile: 700 and 768 rows 2,048 x 8,192 44.6 / 42.8 and 43.6 / 49.0, 5,120 x 20,480 237 / 170 and 179 / 200.
-//   A prompt of 6.7b's with 640 tokens: 11,401 us with tiles there, 10,590 without; 768 tokens 12,001 and 11,295.
-//   K up to 2,048: tiles of 64 x 64 where they make at most one and a quarter a unit, else of 128 x 128 at most one. 100 rows
-//   3,072 x 1,024 8.7 / 6.9, 6,144 x 2,048 14.1 / 13.4, 8,192 x 2,048 15.5 / 15.2; 333 rows 3,072 x 1,024 10.5 / 8.5, 6,144 x 2,048
-//   25.1 / 20.7, 8,192 x 2,048 24.0 / 21.7; 640 rows 6,144 x 2,048 24.9 / 23.5. The kernel alone is slower at 64 rows 6,144 x 2,048
-//   13.3 / 14.0 (a recorded step of 64 of 1.3b's 2,597 / 2,640) and 160 to 300 rows 17.1 / 18.6 to 16.0 / 22.5: small enough for
-//   the host to bound the step. From 2^20 elements of x on (512 rows of K 2,048: there a step of 1.3b's is 3.6 ms of kernels, what
-//   the host takes with the library) tiles of 64 x 64 are to be at most one a unit, and from there on and above 640 rows those of
-//   128 x 128 are to fill half the units: 640 rows 2,048 x 2,048 (320 and 80) 15.2 / 16.9, 3,072 x 2,048 (120 of 128 x 128) 17.7 /
-//   24.4, 700 rows 1,536 x 2,048 13.6 / 15.2, 768 rows 2,048 x 2,048 (96) 14.1 / 19.1 (a prompt of 1.3b's with 768 tokens 4,037 with
-//   them, 3,624 without); up to it one and a quarter a unit lose less than the host's 8 us (333 rows 3,072 x 2,048 16.0 / 16.4).
-//   33 to 64 rows and K up to 4,096: tiles of 64 x 64 with shares. 48 rows 3,072 x 4,096 13.4 / 12.6, 4,096 x 4,096 14.2 / 13.6, 7,680 x
-//   2,560 16.0 / 16.4, 10,240 x 2,560 21.6 / 20.8. Not from 2^25 elements on: 64 rows 12,288 x 4,096 27.9 / 31.6, 16,384 x 4,096 32.6 /
-//   36.0 (a step of 64 of 6.7b's 6,075 with tiles there, 5,897 without).
-// Up to 32 rows half a tile would be padding (32 rows 10,240 x 2,560: 17.7 / 20), and other kernels stand ready.
-// What bounds these sizes is the time a unit takes for a step of its one block (0.55 us for 128 x 128 x 64, of which the
-// matrix cores work 0.2 and LDS 0.15; the waves wait half of it, for loads from the caches and for each other), not memory (17.1 to
-// 17.8 us for 20.4 with 333 x 6,144 x 2,048 in the last cache): shares of K are the way to keep all units at it.
-enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2 };
+// A unit pulls 57 bytes a nanosecond of lines that no cache holds, 70 where half of them come from its L2 (what hits waits in line behind
+// what does not) and 135 to 160 where all do, however deep it asks; the weights of a model are in no cache. So at these sizes a tile's time
+// is the bytes that its block brings, (TM + TN) 128 a step of 64 of K, and what counts is that the tiles are small and yet go round the
+// units once. (More steps under way, K begun elsewhere by each block, a wave or loads that touch lines ahead and weights marked as
+// read once were each measured to change 2 % or nothing.) `tiles_time`, us, is that: the bytes of the fullest unit, those of all blocks, a
+// launch, and the sum of the shares. Tiles of 64 x 64 find two blocks a unit. Over 306 sizes of 33 to 768 rows it names the quickest of these
+// tiles or one 2 % slower on average; on weights that no cache holds (16 matrices and more in turn), with bias and ReLU or the residual, us,
+// the library / tiles of 64 x 64 and 128 x 128 alone / these:
+//   333 rows 6,144 (columns) x 2,048 (K) 25.0 / 20.1 / 18.7, 8,192 x 2,048 23.4 / 20.9 / 19.8, 5,120 x 4,096 28.9 / - / 27.9;
+//   200 rows 6,144 x 2,048 16.2 / 19.5 / 15.7, 8,192 x 2,048 17.7 / 20.1 / 16.2, 2,048 x 4,096 14.7 / - / 14.0;
+//   100 rows 5,120 x 4,096 22.6 / - / 16.6, 2,048 x 8,192 19.3 / 16.2 / 14.4, 4,096 x 4,096 16.8 / - / 14.0; 64 rows 2,048 x 8,192 16.6 / 14.7 / 12.2;
+//   512 rows 3,072 x 1,024 12.5 / 12.9 / 10.7, 7,680 x 2,560 31.8 / - / 28.5; 640 rows 2,048 x 4,096 25.6 / - / 23.0.
+// The library keeps (library / tiles): matrices of many columns at up to 200 rows (128 rows 10,240 x 2,560 22.8 / 24.9, 100 rows 16,384 x 4,096
+// 35.9 / 39.5; at 64 rows from 2^25 elements on), what would need more blocks than there are units (640 rows 8,192 x 2,048 26.4 / 40.8), many
+// rows of few columns with K whole (768 rows 2,048 x 2,048 15.4 / 17.8, 512 rows 2,560 x 2,560 18.0 / 19.5), and K beyond 4,096 where tiles of
+// 128 x 128 with their shares give half of the units a block or fewer, three quarters above 576 rows, or the rows are more than 704. A call of the
+// library's takes the host some 13 us, a launch of ours 5, and short prompts are not recorded: a few per cent on the device are less than that.
+// Tiles of 160 x 128 and 192 x 128, four waves and eight, were slower than the library where they would be taken (640 rows 8,192 x 2,048
+// 31.3 and 26.7, 26.1), those of 96 x 64 no quicker than the others, and those of 96 x 96 only alone (333 rows 6,144 x 2,048 17.6 for 18.7; a prompt of
+// 333 tokens of 1.3b 2,368 us with them and 2,363 without: one kernel fewer to fetch). Up to 32 rows half a tile would be padding, and other kernels stand ready.
+enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2, TILES_64x128 = 3, TILES_96x128 = 4, TILES_MOST = 4 };
+static const struct { int rows, columns; } TILE_SIZES[TILES_MOST + 1] = {{0, 0}, {64, 64}, {128, 128}, {64, 128}, {96, 128}};
+
+static float tiles_time(int tile, int M, int N, int K, int shares, int units) {
+  const int steps = K / 64, per = (steps + shares - 1) / shares;
+  shares = (steps + per - 1) / per;
+  const int rows = TILE_SIZES[tile].rows, columns = TILE_SIZES[tile].columns;
+  const long long blocks = (long long)((M + rows - 1) / rows) * ((N + columns - 1) / columns) * shares;
+  if (4 * blocks > (tile == TILES_64 && shares == 1 ? 5 : 4) * (long long)units) return INFINITY;
+  const float block = 1e-3f * per * (rows + columns);
+  const float sum = shares > 1 ? 1.6f + 1.9e-6f * shares * M * N : 0.f;
+  return 4.f + (blocks > units ? 2.16f : 1.6f) * block + 1.6e-3f * block * blocks + sum;
+}
+
 static int choose_tiles(int M, int N, int K, int& shares) {
   const int units = tnx_compute_units(), steps = K / 64;
-  const long long small = (long long)((M + 63) / 64) * ((N + 63) / 64), large = (long long)((M + 127) / 128) * ((N + 127) / 128);
-  auto share_out = [&](long long tiles) {
-    int s = (int)(units / tiles);
-    s = s < 1 ? 1 : s > 8 ? 8 : s;
-    while (s > 1 && (steps / s < 4 || (long long)s * M * N > F32_SHARES_MOST)) --s;
-    return s;
-  };
+  const long long large = (long long)((M + 127) / 128) * ((N + 127) / 128), matrix = (long long)N * K;
   shares = 1;
   if (M <= 32 || M > 768) return TILES_NONE;
-  if (K >= 4ll * N && large <= units) {
-    shares = share_out(large);
-    const long long blocks = large * shares;
-    if (K > 4096 && M > 128 && (M > 704 || 2 * blocks <= units || (M > 576 && 4 * blocks < 3 * units))) return TILES_NONE;
-    return TILES_128;
+  if (N > K && M <= 200 && matrix >= (M <= 64 ? 1ll << 25 : 3ll << 23)) return TILES_NONE;
+  if (K > 4096) {
+    if (K < 4ll * N || large > units) return TILES_NONE;
+    const long long blocks = large * min(min(8ll, units / large), max(1ll, (long long)steps / 4));
+    if (M > 128 && (M > 704 || 2 * blocks <= units || (M > 576 && 4 * blocks < 3 * units))) return TILES_NONE;
   }
-  const bool many = (long long)M * K > 1ll << 20;
-  if (K <= 2048 && 4 * small <= (many ? 4 : 5) * units) return TILES_64;
-  if (K <= 2048 && large <= units && ((M <= 640 && !many) || 2 * large > units)) return TILES_128;
-  if (M <= 64 && K <= 4096 && small <= units && (long long)N * K < 1ll << 25) {
-    shares = share_out(small);
-    return TILES_64;
-  }
-  return TILES_NONE;
+  int tile = TILES_NONE;
+  float least = INFINITY;
+  for (int t = 1; t <= TILES_MOST; ++t)
+    for (int s = 1; s <= 8 && (s == 1 || (steps / s >= 8 && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
+      const float us = tiles_time(t, M, N, K, s, units);
+      if (us < least) least = us, tile = t, shares = s;
+    }
+  if (tile != TILES_NONE) shares = (steps + (steps + shares - 1) / shares - 1) / ((steps + shares - 1) / shares);
+  // many rows of few columns, K whole
+  if (K <= 4096 && (long long)M * K > 1ll << 20 && shares == 1 && (N <= K || (N <= 3072 && 2 * large <= units))) return TILES_NONE;
+  return tile;
 }
 
 // Whether `tnx_gemm_bf16_tiles` is the way for a product (-1: it is not), and how many floats of workspace it then wants.
@@ -2275,16 +2274,21 @@ static int gemm_bf16_tiles(const void* x, const void* w, const float* bias, cons
   TNX_REQUIRE(out_dtype == TNX_F32 || (out_dtype == TNX_BF16 && residual == nullptr), "gemm_bf16_tiles: a residual beside a float32 result");
   TNX_REQUIRE(((uintptr_t)x | (uintptr_t)w | (uintptr_t)out | (uintptr_t)residual | (uintptr_t)workspace) % 16 == 0,
               "gemm_bf16_tiles: operands must be 16-byte aligned");
-  TNX_REQUIRE(tile >= 0 && tile <= TILES_128 && shares >= 0, "gemm_bf16_tiles: tiles 1 (64) and 2 (128)");
+  TNX_REQUIRE(tile >= 0 && tile <= TILES_MOST && shares >= 0, "gemm_bf16_tiles: tiles 1 to %d", TILES_MOST);
   int chosen = 1;
   if (tile == 0) tile = choose_tiles(M, N, K, chosen);
   if (shares == 0) shares = chosen;
   if (shares > K / 64) shares = K / 64;
   if (shares > 1 && (workspace == nullptr || workspace_floats < (size_t)shares * M * N)) shares = 1;
   const bf16_t *xp = (const bf16_t*)x, *wp = (const bf16_t*)w;
-  if (tile == TILES_128)
-    return launch_tiles<2, 1, 4, 2, 4>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream);
-  return launch_tiles<1, 1, 4, 2, 2>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream);
+#define TILES(MI, NI, WM, WN) return launch_tiles<MI, NI, 4, WM, WN>(xp, wp, bias, residual, out, out_dtype, act, workspace, M, N, K, shares, left, stream)
+  switch (tile) {
+    case TILES_128: TILES(2, 1, 2, 4);
+    case TILES_64x128: TILES(2, 1, 1, 4);
+    case TILES_96x128: TILES(3, 1, 1, 4);
+    default: TILES(1, 1, 2, 2);
+  }
+#undef TILES
 }
 
 extern "C" int tnx_gemm_bf16_tiles(const void* x, const void* w, const float* bias, const float* residual, void* out,
