@@ -158,6 +158,7 @@ __global__ void __launch_bounds__(1024) order_kernel(const int* __restrict__ cho
     for (int e = threadIdx.x; e < experts; e += blockDim.x)
       for (int r = 0, i = tile_at[e]; r < counts[e]; r += tile_rows, ++i) tiles[i] = make_int2(e, cursor[e] + r);
     for (int i = tiles_used + threadIdx.x; i < tile_slots; i += blockDim.x) tiles[i] = make_int2(-1, 0);
+    if (threadIdx.x == 0) tiles[tile_slots] = make_int2(tiles_used, 0);      // and behind them how many there are
     __syncthreads();                   // the cursors move from here on
   }
   for (int i = threadIdx.x; i < pairs; i += blockDim.x) {
@@ -460,37 +461,36 @@ int launch_products(const ProductArgs& p, dim3 grid, hipStream_t stream) {
 // MFMA 32x32x16 (`tiles.h`), one launch over all experts. UP_GATED: a wave takes 32 gate rows and the 32 up rows that go with
 // them, so that act(g) * u is made of its own sums; the tile makes half as many columns of `inner`. The pairs' rows are
 // gathered by the loads themselves: a lane's address in `h` is that of its pair's token. `inner` and the result lie in sorted
-// order. What bounds it is how well a unit's waves keep its matrix cores at work between their meetings (two waves a core and
-// a wave's 64 x 64 of the tile: 60 % of the time); an expert's last tile may be nearly empty, so where an expert has fewer
-// pairs the tiles are of 64.
+// order. Of long prompts what bounds it is how well a unit's waves keep its matrix cores at work between their meetings (two waves
+// a core and a wave's 64 x 64 of the tile: 60 % of the time), of short ones the bytes that a tile's block has to pull, 60 a nanosecond
+// and unit while the matrices are in no cache (128 x 256 of K 2,048: 26 us, though it be on one unit in four). An expert's last
+// tile may be nearly empty.
 // Blocks of an XCD take the tiles of one column block after the other, so that an expert's rows of the matrix are brought
 // from memory once and read again from that XCD's cache.
-// Measured at 2,048 tokens of two choices among 8 experts, a layer: 4,096 wide, inner 4,096, 543 us (760 TFLOP/s) against
-// 795 with sixteen products of the vendor library and a wait for the host between; 2,048 wide 175 against 422. With four
-// waves of 64 x 64 on 128 rows of the matrix, two blocks a unit: 632 and 207.
+// Measured for 8 experts of which a token chooses two, a layer on weights that no cache holds, us, every tile whole / the last round in
+// parts: 2,048 wide, inner 2,048: 64 tokens 75.2 / 59.9, 200 77.8 / 61.7, 396 83.0 / 75.0, 640 85.3 / 78.5, 1,024 113.8 / 106.5, 2,048 187 / 163;
+// 4,096 wide, inner 4,096: 500 251 / 244, 1,000 344 / 318, 2,048 534 / 520 (790 TFLOP/s); 64 experts of 6, 2,048 wide, inner 1,408: 500
+// 275 / 254, 2,048 438 / 410. Tiles of half or a quarter of the columns throughout are as much slower where whole ones go round the
+// units more than once (2,048 wide, 2,048 tokens, halves: 197; 4,096 wide 575 to 630).
 struct GroupedArgs {
   const bf16_t* a;          // UP: h [T, K]; DOWN: inner [sorted pairs, K]
   const bf16_t* w;          // [E, N(, 2), K]
   const int* first;         // [E + 1]
   const int* order;         // [pairs]
-  const int2* tiles;        // [slots]
+  const int2* tiles;        // [slots], then how many there are
   const float* weights;     // [pairs]; null: not on the input
   void* out;                // UP: inner, bfloat16; DOWN: float32
-  int top, n, k, act, slots;
+  int top, n, k, act, slots, units;
   float limit;
 };
 
-template <int KIND, int MI, int ST, int WN>
-__global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
+// One tile: the pairs of `tile` by the columns of the result from n0 on.
+template <int KIND, int MI, int NI, int ST, int WM, int WN>
+__device__ __forceinline__ void expert_tile(const GroupedArgs& p, char* smem, const int2 tile, const int n0) {
   constexpr bool GATED = KIND == UP_GATED, UP = KIND != DOWN;
-  typedef Tile<MI, 2, ST, 2, WN> Products;
-  extern __shared__ __attribute__((aligned(16))) char smem[];
-  const int at = by_xcd(blockIdx.x, gridDim.x);
-  const int2 tile = p.tiles[at % p.slots];
-  const int e = tile.x;
-  if (e < 0) return;
-  const int begin = tile.y, count = min(Products::TM, p.first[e + 1] - begin);
-  const int n0 = at / p.slots * (GATED ? Products::TN / 2 : Products::TN);
+  static_assert(!GATED || NI == 2, "gate rows and the up rows beside them");
+  typedef Tile<MI, NI, ST, WM, WN> Products;
+  const int e = tile.x, begin = tile.y, count = min(Products::TM, p.first[e + 1] - begin);
   Products t;
 #pragma unroll
   for (int j = 0; j < Products::LA; ++j) {
@@ -531,17 +531,17 @@ __global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
 #pragma unroll
       for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < NI; ++j)
 #pragma unroll
           for (int e = 0; e < 16; ++e) t.acc[i][j][e] = activation(t.acc[i][j][e]);
     });
-    t.template hand_out<bf16_t, 64>(
+    t.template hand_out<bf16_t, 32 * NI>(
         smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
         [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((bf16_t*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
         });
   } else {
-    t.template hand_out<float, 64>(
+    t.template hand_out<float, 32 * NI>(
         smem, [&](int i, int j, int e, int, int) { return t.acc[i][j][e]; },
         [&](int r, int c, f32x4 chunk, int) {
           if (r0 + r < count && c0 + c < p.n) *(f32x4*)((float*)p.out + (size_t)(begin + r0 + r) * p.n + c0 + c) = chunk;
@@ -549,31 +549,89 @@ __global__ void __launch_bounds__(128 * WN) expert_tiles_kernel(GroupedArgs p) {
   }
 }
 
-template <int KIND, int MI, int ST, int WN>
-int launch_tiles(const GroupedArgs& p, hipStream_t stream) {
-  typedef Tile<MI, 2, ST, 2, WN> Products;
+// Tiles of 64 pairs: four waves over 128 rows of the matrix.
+template <int KIND, int ST>
+__global__ void __launch_bounds__(256) expert_tiles_kernel(GroupedArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int at = by_xcd(blockIdx.x, gridDim.x);
+  const int2 tile = p.tiles[at % p.slots];
+  if (tile.x < 0) return;
+  expert_tile<KIND, 1, 2, ST, 2, 2>(p, smem, tile, at / p.slots * (KIND == UP_GATED ? 64 : 128));
+}
+
+// Tiles of 128 pairs: eight waves over 256 rows of the matrix, as often as these go round the units, of which each holds one
+// (144 KB). What is left over, less than one a unit, would be a whole round more for a part of the units: it goes out as halves
+// or quarters of a tile's columns where these still find a unit each. How many tiles the pairs make only the device knows, so
+// every block finds its place from their count.
+template <int KIND>
+__global__ void __launch_bounds__(512) expert_wide_tiles_kernel(GroupedArgs p) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  constexpr int COLUMNS = KIND == UP_GATED ? 128 : 256;
+  const int used = p.tiles[p.slots].x, total = used * ((p.n + COLUMNS - 1) / COLUMNS);
+  int whole = total / p.units * p.units;
+  const int left = total - whole;
+  const int pieces = 4 * left <= p.units && KIND != UP_GATED ? 4 : 2 * left <= p.units ? 2 : 1;
+  if (pieces == 1) whole = total;
+  int block = blockIdx.x;
+  if (block < whole) {
+    const int at = by_xcd(block, whole);
+    expert_tile<KIND, 2, 2, 3, 2, 4>(p, smem, p.tiles[at % used], at / used * COLUMNS);
+    return;
+  }
+  block -= whole;
+  if (pieces == 1 || block >= left * pieces) return;
+  const int piece = by_xcd(block, left * pieces), at = whole + piece / pieces;
+  const int n0 = at / used * COLUMNS + piece % pieces * (COLUMNS / pieces);
+  if (n0 >= p.n) return;
+  const int2 tile = p.tiles[at % used];
+  if constexpr (KIND != UP_GATED) {
+    if (pieces == 4) {
+      expert_tile<KIND, 1, 1, 4, 4, 2>(p, smem, tile, n0);
+      return;
+    }
+  }
+  expert_tile<KIND, 1, 2, 4, 4, 2>(p, smem, tile, n0);
+}
+
+template <int KIND>
+int launch_wide_tiles(const GroupedArgs& p, hipStream_t stream) {
+  constexpr int bytes = Tile<2, 2, 3, 2, 4>::BYTES, columns = KIND == UP_GATED ? 128 : 256;
+  static_assert(bytes >= Tile<1, 2, 4, 4, 2>::BYTES && bytes >= Tile<1, 1, 4, 4, 2>::BYTES, "room for the parts of a tile");
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)expert_tiles_kernel<KIND, MI, ST, WN>,
-                                       hipFuncAttributeMaxDynamicSharedMemorySize, Products::BYTES);
-    TNX_REQUIRE(e == hipSuccess, "expert tiles: cannot reserve %d bytes of LDS: %s", Products::BYTES, hipGetErrorString(e));
+    hipError_t e = hipFuncSetAttribute((const void*)expert_wide_tiles_kernel<KIND>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "expert tiles: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
     configured = true;
   }
-  const int columns = KIND == UP_GATED ? Products::TN / 2 : Products::TN;
-  expert_tiles_kernel<KIND, MI, ST, WN><<<(p.n + columns - 1) / columns * p.slots, 128 * WN, Products::BYTES, stream>>>(p);
+  // (whole rounds, and parts that fill one more at most)
+  const long long total = (long long)((p.n + columns - 1) / columns) * p.slots, rounds = (total + p.units - 1) / p.units;
+  expert_wide_tiles_kernel<KIND><<<(unsigned)(rounds * p.units), 512, bytes, stream>>>(p);
   TNX_CHECK_LAUNCH("expert tiles");
   return 0;
 }
 
-// Tiles of 128 pairs: eight waves over 256 of the matrix's rows, three stages (144 KB, one block a unit). Tiles of 64: four
-// waves over 128 rows; two stages, so that a unit holds three blocks, four where it has no more than one anyway (the slots
-// count an empty tile an expert too many, about half used).
+template <int KIND, int ST>
+int launch_narrow_tiles(const GroupedArgs& p, hipStream_t stream) {
+  constexpr int bytes = Tile<1, 2, ST, 2, 2>::BYTES, columns = KIND == UP_GATED ? 64 : 128;
+  static bool configured = false;
+  if (!configured) {
+    hipError_t e = hipFuncSetAttribute((const void*)expert_tiles_kernel<KIND, ST>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    TNX_REQUIRE(e == hipSuccess, "expert tiles: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
+    configured = true;
+  }
+  expert_tiles_kernel<KIND, ST><<<(p.n + columns - 1) / columns * p.slots, 256, bytes, stream>>>(p);
+  TNX_CHECK_LAUNCH("expert tiles");
+  return 0;
+}
+
+// Tiles of 64 have two stages, so that a unit holds three blocks, four where it has no more than one anyway (the slots count an
+// empty tile an expert too many, about half used).
 template <int KIND>
 int launch_tiles(const GroupedArgs& p, int tile_rows, hipStream_t stream) {
-  if (tile_rows == 128) return launch_tiles<KIND, 2, 3, 4>(p, stream);
+  if (tile_rows == 128) return launch_wide_tiles<KIND>(p, stream);
   const int columns = KIND == UP_GATED ? 64 : 128;
-  const bool deep = (long long)((p.n + columns - 1) / columns) * p.slots <= tnx_compute_units();
-  return deep ? launch_tiles<KIND, 1, 4, 2>(p, stream) : launch_tiles<KIND, 1, 2, 2>(p, stream);
+  const bool deep = (long long)((p.n + columns - 1) / columns) * p.slots <= p.units;
+  return deep ? launch_narrow_tiles<KIND, 4>(p, stream) : launch_narrow_tiles<KIND, 2>(p, stream);
 }
 
 // (`place`: the row of y that holds pair t * top + c, where the rows lie in another order; `scale`: a factor a pair.
@@ -750,7 +808,7 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
 }
 
 // The whole mixture for many pairs an expert, in bfloat16: order, the two products by tiles of `tile_rows` (64 or 128) pairs,
-// the sum. `ints`: room for experts + 1 + 2 pairs integers, then 2 (pairs / tile_rows + experts) more from a multiple of 2 on;
+// the sum. `ints`: room for experts + 1 + 2 pairs integers, then 2 (pairs / tile_rows + experts + 1) more from a multiple of 2 on;
 // `inner` [pairs, f], `y` [pairs, width]. width and f are multiples of 64.
 extern "C" int tnx_expert_grouped(const void* h, const int* chosen, const float* weights, const void* w_gate_up,
                                   const void* w_down, int* ints, void* inner, float* y, const float* residual, float* out,
@@ -775,9 +833,9 @@ extern "C" int tnx_expert_grouped(const void* h, const int* chosen, const float*
                                                                nullptr, tiles, tile_rows, slots);
   TNX_CHECK_LAUNCH("expert order");
   const GroupedArgs up{(const bf16_t*)h, (const bf16_t*)w_gate_up, first, order, tiles, weight_on_input ? weights : nullptr, inner,
-                       top, f, width, act, slots, limit};
+                       top, f, width, act, slots, tnx_compute_units(), limit};
   const GroupedArgs down{(const bf16_t*)inner, (const bf16_t*)w_down, first, order, tiles, nullptr, y, top, width, f, act, slots,
-                         limit};
+                         tnx_compute_units(), limit};
   if (int rc = ungated ? launch_tiles<UP_PLAIN>(up, tile_rows, stream) : launch_tiles<UP_GATED>(up, tile_rows, stream)) return rc;
   if (int rc = launch_tiles<DOWN>(down, tile_rows, stream)) return rc;
   launch_combine<bf16_t>(y, residual, out, tokens, top, width, place, weight_on_input ? nullptr : weights,

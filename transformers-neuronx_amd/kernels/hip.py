@@ -2574,12 +2574,15 @@ class HipOps:
         return out
 
     # From `expert_grouped_rows` (token, choice) pairs an expert on, bfloat16, sizes in 64s: the experts' products by tiles
-    # (two launches over all experts, the host reads nothing), of 128 pairs from `expert_wide_tiles` an expert on. Measured
-    # for 8 experts, two a token, us a layer, one launch of 16 pairs a tile or the library / tiles of 64 / of 128: 2,048 wide,
-    # 12 pairs an expert 57 / 67 / 77, 16: 75 / 68 / 77, 50: 132 / 73 / 82, 99: 432 / 97 / 91, 512: 422 / 205 / 175; 4,096 wide,
-    # 12: 199 / 218 / 209, 16: 218 / 216 / 208, 50: 469 / 224 / 209, 99: 449 / 283 / 220, 512: 795 / 688 / 543.
+    # (two launches over all experts, the host reads nothing), of 128 pairs from `expert_wide_tiles` an expert on and for matrices
+    # of `expert_wide_matrix` elements and more. Measured for 8 experts, two a token, us a layer, one launch of 16 pairs a tile / tiles
+    # of 64 / of 128: 2,048 wide, 12 pairs an expert 57 / 67 / -, 16: 75 / 66 / 60, 50: 132 / 70 / 62, 99: - / 88 / 75, 512: - / 199 / 163;
+    # 4,096 wide, 12: 199 / 218 / -, 16: 218 / 214 / 205, 50: 469 / 218 / 210, 512: - / 685 / 520. Small matrices find fewer tiles than
+    # units: 32 experts of 1,024 x 512, 62 pairs - / 46 / 50, 112: - / 56 / 53; 64 of 1,024 x 512, 31 pairs 59 / 61, 75: 85 / 82; 128 of 2,880 x
+    # 768, 16 pairs 291 / 291, 38: 363 / 324.
     expert_grouped_rows = 16           # 0: never (nor where `expert_library_rows` is 0: tiles of 16 pairs at any size then)
     expert_wide_tiles = 80
+    expert_wide_matrix = 1 << 21
     # Other sizes, from this many pairs an expert on, in a step that is not being recorded: the host reads where each
     # expert's pairs begin (one small copy that waits for the device) and every expert's two products go to the vendor
     # library over its own rows. Below that, and in recorded steps, one launch of ours with tiles of 16 pairs takes all
@@ -2617,12 +2620,12 @@ class HipOps:
         dev = h.device
         pairs = t * top
         out = torch.empty(t, width, dtype=torch.float32, device=dev)
-        rows = 128 if pairs >= self.expert_wide_tiles * experts else 64
+        rows = 128 if pairs >= self.expert_wide_tiles * experts or width * f >= self.expert_wide_matrix else 64
         if (self.expert_grouped_rows > 0 and self.expert_library_rows > 0 and pairs >= self.expert_grouped_rows * experts
                 and not self.expert_plain_products and h.dtype == torch.bfloat16 and width % 64 == 0 and f % 64 == 0
                 and self._tiles_reach(t, experts, top, width, f, rows)
                 and (_ptr(h) | _ptr(w_gate_up) | _ptr(w_down)) % 16 == 0 and (residual is None or _ptr(residual) % 16 == 0)):
-            ints = torch.empty(experts + 2 + 2 * pairs + 2 * (pairs // rows + experts), dtype=torch.int32, device=dev)
+            ints = torch.empty(experts + 4 + 2 * pairs + 2 * (pairs // rows + experts), dtype=torch.int32, device=dev)
             inner = torch.empty(pairs, f, dtype=h.dtype, device=dev)
             y = torch.empty(pairs, width, dtype=torch.float32, device=dev)
             self._call("experts", "tnx_expert_grouped", _ptr(h), _ptr(chosen), _ptr(weights), _ptr(w_gate_up), _ptr(w_down),
