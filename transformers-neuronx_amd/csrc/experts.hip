@@ -38,15 +38,21 @@ __device__ __forceinline__ void with_gate(int act, float limit, F f) {
 // the experts form that many equal groups of neighbours, a group ranks by its best expert, and only experts of the `keep`
 // best groups (the lower number where two are equal) take part.
 constexpr int MAX_GROUPS = 256;
-__global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z, int ld, int tokens, int experts, int top,
-                                                    int softmax, int renormalize, int* __restrict__ chosen,
-                                                    float* __restrict__ weights, const float* __restrict__ correction,
-                                                    float scale, int groups, int keep) {
-  __shared__ float best_of[4][MAX_GROUPS];        // a wave's groups: the best rank, and whether the group is kept
-  __shared__ unsigned char kept_of[4][MAX_GROUPS];
-  const int t = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
-  if (t >= tokens) return;
-  const float* row = z + (size_t)t * ld;
+struct RouteArgs {
+  int tokens, experts, top, softmax, renormalize;
+  int* chosen;
+  float* weights;
+  const float* correction;
+  float scale;
+  int groups, keep;
+};
+
+// Token t's choice from its logits `row` (global memory or LDS), by one wave; `best`, `kept`: the wave's room for the groups.
+__device__ __forceinline__ void route_token(const RouteArgs& a, const float* row, int t, float* best, unsigned char* kept) {
+  const int lane = threadIdx.x & 63, experts = a.experts, top = a.top, softmax = a.softmax, groups = a.groups, keep = a.keep;
+  int* chosen = a.chosen;
+  float* weights = a.weights;
+  const float *correction = a.correction, scale = a.scale;
   float peak = -INFINITY, total = 1.f;
   if (softmax) {
     for (int e = lane; e < experts; e += 64) peak = fmaxf(peak, row[e]);
@@ -60,8 +66,6 @@ __global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z,
   const int per = experts / groups;
   const bool grouped = keep < groups;
   if (grouped) {      // (a wave's own rows of LDS; a wave's LDS operations keep their order)
-    float* best = best_of[threadIdx.x >> 6];
-    unsigned char* kept = kept_of[threadIdx.x >> 6];
     for (int g = 0; g < groups; ++g) {
       float b = -INFINITY;
       for (int e = lane; e < per; e += 64) b = fmaxf(b, plain_rank(g * per + e));
@@ -80,7 +84,6 @@ __global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z,
       __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
   }
-  const unsigned char* kept = kept_of[threadIdx.x >> 6];
   auto rank = [&](int e) { return !grouped || kept[e / per] ? plain_rank(e) : -INFINITY; };
   float sum = 0.f;
   unsigned long long taken = 0;        // bit i: expert lane + 64 i is chosen already (a lane's own experts)
@@ -97,11 +100,11 @@ __global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z,
     const float s = correction ? score(row[first]) : score(high);
     if (lane == 0) {
       chosen[(size_t)t * top + c] = first;
-      weights[(size_t)t * top + c] = renormalize ? 0.f : s * scale;
+      weights[(size_t)t * top + c] = a.renormalize ? 0.f : s * scale;
     }
     sum += s;
   }
-  if (renormalize) {
+  if (a.renormalize) {
     // the same rounds again, now that the sum is known: each weight is written once
     taken = 0;
     for (int c = 0; c < top; ++c) {
@@ -117,6 +120,54 @@ __global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z,
       if (lane == 0) weights[(size_t)t * top + c] = (correction ? score(row[first]) : score(high)) / sum * scale;
     }
   }
+}
+
+__global__ void __launch_bounds__(256) route_kernel(const float* __restrict__ z, int ld, RouteArgs a) {
+  __shared__ float best_of[4][MAX_GROUPS];        // a wave's groups: the best rank, and whether the group is kept
+  __shared__ unsigned char kept_of[4][MAX_GROUPS];
+  const int wave = threadIdx.x >> 6, t = blockIdx.x * 4 + wave;
+  if (t < a.tokens) route_token(a, z + (size_t)t * ld, t, best_of[wave], kept_of[wave]);
+}
+
+// The router's product and the choice in one launch, a block a token: z = W_r h + bias (bfloat16 operands, exact products,
+// float32 sums of 8 to 16 elements a thread, then by tree), eight experts at a time. A launch costs 3 to 5 us here and this work a
+// fraction of it: what bounds it is the block's few readings of memory one after the other, and for many tokens the matrix, which every
+// block reads from the cache. us, a launch for the product and one for the choice / this: 8 experts, rows of 2,048, 1 token 6.2 / 4.3, 8 tokens 7.4 / 4.6,
+// 396 9.6 / 5.2, 2,048 8.2 / 8.4; rows of 4,096, 8 tokens 9.8 / 5.1, 2,048 9.7 / 10.2; 16 of 2,880, 8 tokens 9.8 / 6.8, 396 9.8 / 7.8, 2,048 11.2 / 15.1;
+// 32 of 2,048, 8 tokens 7.2 / 9.1.
+constexpr int ROUTE_PRODUCT_MOST = 16;     // experts
+__global__ void __launch_bounds__(256) route_product_kernel(const bf16_t* __restrict__ h, const bf16_t* __restrict__ w,
+                                                            const float* __restrict__ bias, int width, RouteArgs a) {
+  __shared__ float parts[4][ROUTE_PRODUCT_MOST], z[ROUTE_PRODUCT_MOST], best[ROUTE_PRODUCT_MOST];
+  __shared__ unsigned char kept[ROUTE_PRODUCT_MOST];
+  const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const bf16_t* row = h + (size_t)t * width;
+  for (int e0 = 0; e0 < a.experts; e0 += 8) {
+    float sum[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) sum[e] = 0.f;
+    for (int k = 8 * tid; k < width; k += 2048) {
+      const bf16x8 x = *(const bf16x8*)(row + k);
+      bf16x8 v[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) v[e] = *(const bf16x8*)(w + (size_t)min(e0 + e, a.experts - 1) * width + k);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+#pragma unroll
+        for (int i = 0; i < 8; ++i) sum[e] = fmaf((float)x[i], (float)v[e][i], sum[e]);
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float s = wave_sum(sum[e]);
+      if (lane == 0 && e0 + e < a.experts) parts[wave][e0 + e] = s;
+    }
+  }
+  __syncthreads();
+  if (wave) return;
+  if (lane < a.experts)
+    z[lane] = (parts[0][lane] + parts[1][lane]) + (parts[2][lane] + parts[3][lane]) + (bias ? bias[lane] : 0.f);
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  route_token(a, z, t, best, kept);
 }
 
 // ---------------------------------------------------------------- pairs in the order of their experts
@@ -741,9 +792,26 @@ extern "C" int tnx_route(const float* z, int ld, int tokens, int experts, int to
                   top <= keep * (experts / groups),
               "route: %d of %d experts in %d groups (up to %d) of which %d are kept", top, experts, groups, MAX_GROUPS, keep);
   if (tokens == 0) return 0;
-  route_kernel<<<(tokens + 3) / 4, 256, 0, stream>>>(z, ld, tokens, experts, top, softmax, renormalize, chosen, weights,
-                                                     correction, scale, groups, keep);
+  route_kernel<<<(tokens + 3) / 4, 256, 0, stream>>>(
+      z, ld, RouteArgs{tokens, experts, top, softmax, renormalize, chosen, weights, correction, scale, groups, keep});
   TNX_CHECK_LAUNCH("route");
+  return 0;
+}
+
+// The same from the rows `h` [tokens, width] and the router's matrix `w` [experts, width], bfloat16, and its bias or none.
+extern "C" int tnx_route_product(const void* h, const void* w, const float* bias, int width, int tokens, int experts, int top,
+                                 int softmax, int renormalize, int* chosen, float* weights, const float* correction, float scale,
+                                 int groups, int keep, hipStream_t stream) {
+  TNX_REQUIRE(tokens >= 0 && experts > 0 && top > 0 && top <= experts, "route_product: %d of %d experts", top, experts);
+  TNX_REQUIRE(experts <= ROUTE_PRODUCT_MOST, "route_product: up to %d experts, got %d", ROUTE_PRODUCT_MOST, experts);
+  TNX_REQUIRE(width > 0 && width % 8 == 0 && ((uintptr_t)h | (uintptr_t)w) % 16 == 0, "route_product: rows of %d, in 8s and 16-byte aligned", width);
+  TNX_REQUIRE(groups >= 1 && experts % groups == 0 && keep >= 1 && keep <= groups && top <= keep * (experts / groups),
+              "route_product: %d of %d experts in %d groups of which %d are kept", top, experts, groups, keep);
+  if (tokens == 0) return 0;
+  route_product_kernel<<<tokens, 256, 0, stream>>>(
+      (const bf16_t*)h, (const bf16_t*)w, bias, width,
+      RouteArgs{tokens, experts, top, softmax, renormalize, chosen, weights, correction, scale, groups, keep});
+  TNX_CHECK_LAUNCH("route_product");
   return 0;
 }
 

@@ -168,6 +168,8 @@ _SIGNATURES = {
     "experts": {
         "tnx_route": [_c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_float,
                       _c_int, _c_int, _c_void_p],
+        "tnx_route_product": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_void_p,
+                              _c_void_p, _c_float, _c_int, _c_int, _c_void_p],
         "tnx_expert_mixture": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                                _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                _c_int, _c_int, _c_float, _c_int, _c_int, _c_void_p],
@@ -2547,6 +2549,35 @@ class HipOps:
         count, keep = groups if groups is not None else (1, 1)
         self._call("experts", "tnx_route", _ptr(z), ld, t, experts, top, int(score == "softmax"), int(bool(renormalize)),
                    _ptr(chosen), _ptr(weights), _ptr(correction), float(scale), int(count), int(keep), _stream())
+        return chosen, weights
+
+    # A router's product and its choice are one launch up to so many experts (0: never) and so many logits of a step: beyond, the
+    # product's own kernels are quicker (`route_product_kernel` has both sides).
+    route_product_most = 16
+    route_product_logits = 8192
+
+    def route_product(self, h, w, bias, experts, top, score="sigmoid", renormalize=False, correction=None, scale=1.0, groups=None):
+        """See `ReferenceOps.route_product`."""
+        matrix = w.tensor if isinstance(w, PreparedWeight) else w
+        t, width = h.shape
+        if (experts > self.route_product_most or t * experts > self.route_product_logits or h.dtype != torch.bfloat16
+                or matrix.dtype != torch.bfloat16 or matrix.shape[1] != width or width % 8 or not (h.is_contiguous() and matrix.is_contiguous())
+                or (_ptr(h) | _ptr(matrix)) % 16):
+            return self.route(self.linear(h, w, bias, out_f32=True, f32_by_library=True)[:, :experts], top, score, renormalize, correction,
+                              scale, groups)
+        _want(h, "h")
+        if score not in ("sigmoid", "softmax"):
+            raise ValueError(f"unknown router score {score!r}")
+        if bias is not None:
+            _want(bias, "bias", torch.float32, (matrix.shape[0],))
+        if correction is not None:
+            _want(correction, "the choice's correction", torch.float32, (experts,))
+        chosen = torch.empty(t, top, dtype=torch.int32, device=h.device)
+        weights = torch.empty(t, top, dtype=torch.float32, device=h.device)
+        count, keep = groups if groups is not None else (1, 1)
+        self._call("experts", "tnx_route_product", _ptr(h), _ptr(matrix), _ptr(bias), width, t, experts, top, int(score == "softmax"),
+                   int(bool(renormalize)), _ptr(chosen), _ptr(weights), _ptr(correction), float(scale), int(count), int(keep), _stream(),
+                   work=lambda: (f"{t}x{experts}x{width}", 2.0 * width * (t + experts), 2.0 * t * experts * width))
         return chosen, weights
 
     def gated_activation(self, gate_up, activation, row_weights=None, limit=None):

@@ -869,6 +869,10 @@ class ReferenceOps:
             return g * torch.sigmoid(g) * u
         return ReferenceOps.activation(g, activation) * u
 
+    def route_product(self, h, w, bias, experts, top, score="sigmoid", renormalize=False, correction=None, scale=1.0, groups=None):
+        """`route` of the first `experts` columns of h W^T + bias."""
+        return self.route(self.linear(h, w, bias, out_f32=True)[:, :experts], top, score, renormalize, correction, scale, groups)
+
     def gated_activation(self, gate_up, activation, row_weights=None, limit=None):
         """`act(g) * u` from float32 `[T, 2 F]` = [g | u], in the compute dtype; `row_weights` `[T]`: a factor a
         row on both g and u."""

@@ -253,14 +253,16 @@ class ExpertMixture(OffersRows, FeedForward):
 
     def forward(self, h, ctx, residual, rows=None):
         ops = self.ops
-        rows = self._rows(h, rows)
-        z = rows[:, self.router_at:self.router_at + self.routed]
         more = {}
         if self.correction is not None or self.route_scale != 1.0:
             more = dict(correction=self.correction, scale=self.route_scale)
         if self.groups is not None:
             more["groups"] = self.groups
-        chosen, weights = ops.route(z, self.top, self.score, self.renormalize, **more)
+        if rows is None and self.gated:
+            chosen, weights = ops.route_product(h, self.w_in, self.b_in, self.routed, self.top, self.score, self.renormalize, **more)
+        else:
+            rows = self._rows(h, rows)
+            chosen, weights = ops.route(rows[:, self.router_at:self.router_at + self.routed], self.top, self.score, self.renormalize, **more)
         limit = dict(limit=self.limit) if self.limit is not None else {}
         if self.identity:
             limit["identity"] = self.identity
