@@ -19,7 +19,9 @@ typedef __attribute__((ext_vector_type(16))) float f32x16;
 #define TNX_ACT_RELU 1
 #define TNX_ACT_GELU 2      // 0.5 x (1 + erf(x / sqrt 2))
 #define TNX_ACT_GELU_NEW 3  // 0.5 x (1 + tanh(sqrt(2/pi) (x + 0.044715 x^3)))
-#define TNX_ACT_RELU2 5     // max(x, 0)^2  (4 is a gated expert's silu)
+#define TNX_ACT_SILU 4
+#define TNX_ACT_RELU2 5     // max(x, 0)^2
+#define TNX_ACT_CLAMPED_SWIGLU 6
 
 #define TNX_WAVE 64
 
@@ -186,6 +188,22 @@ __device__ __forceinline__ void with_act(int act, F f) {
   else if (act == TNX_ACT_GELU_NEW) f(Activation<TNX_ACT_GELU_NEW>{});
   else if (act == TNX_ACT_RELU2) f(Activation<TNX_ACT_RELU2>{});
   else f(Activation<TNX_ACT_NONE>{});
+}
+
+// What a gated expert makes of the two halves of its first product: act(g) * u; the clamped form, with
+// g' = min(g, limit) and u' = clamp(u, -limit, limit): g' sigmoid(1.702 g') (u' + 1). Chosen once for many elements (`with_act`).
+template <typename F>
+__device__ __forceinline__ void with_gate(int act, float limit, F f) {
+  if (__builtin_expect(act == TNX_ACT_SILU, 1))
+    f([](float g, float u) { return g / (1.f + expf(-g)) * u; });
+  else if (act == TNX_ACT_CLAMPED_SWIGLU)
+    f([limit](float g, float u) {
+      g = fminf(g, limit);
+      u = fminf(fmaxf(u, -limit), limit);
+      return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
+    });
+  else
+    with_act(act, [&](auto activation) { f([activation](float g, float u) { return activation(g) * u; }); });
 }
 
 // What a softmax's running maximum `m` and sum `l` (of exp(score - m) over the visible keys) make of the weighted

@@ -9,26 +9,7 @@
 
 TNX_DEFINE_ERROR_API
 
-#define TNX_ACT_SILU 4
-#define TNX_ACT_CLAMPED_SWIGLU 6
-
 namespace {
-
-// What a gated expert makes of the two halves of its first product: act(g) * u; the clamped form, with
-// g' = min(g, limit) and u' = clamp(u, -limit, limit): g' sigmoid(1.702 g') (u' + 1). Chosen once for many elements (`with_act`).
-template <typename F>
-__device__ __forceinline__ void with_gate(int act, float limit, F f) {
-  if (__builtin_expect(act == TNX_ACT_SILU, 1))
-    f([](float g, float u) { return g / (1.f + expf(-g)) * u; });
-  else if (act == TNX_ACT_CLAMPED_SWIGLU)
-    f([limit](float g, float u) {
-      g = fminf(g, limit);
-      u = fminf(fmaxf(u, -limit), limit);
-      return g / (1.f + expf(-1.702f * g)) * (u + 1.f);
-    });
-  else
-    with_act(act, [&](auto activation) { f([activation](float g, float u) { return activation(g) * u; }); });
-}
 
 // ---------------------------------------------------------------- the router's choice
 // A wave a token: `top` rounds of the largest logit (the lower number where two are equal), whose score sigmoid(z)
@@ -533,6 +514,7 @@ struct GroupedArgs {
   void* out;                // UP: inner, bfloat16; DOWN: float32
   int top, n, k, act, slots, units;
   float limit;
+  int rows;                 // where there are no experts (`first`, `order` and `tiles` null): the rows of `a`, in their own order
 };
 
 // One tile: the pairs of `tile` by the columns of the result from n0 on.
@@ -541,12 +523,12 @@ __device__ __forceinline__ void expert_tile(const GroupedArgs& p, char* smem, co
   constexpr bool GATED = KIND == UP_GATED, UP = KIND != DOWN;
   static_assert(!GATED || NI == 2, "gate rows and the up rows beside them");
   typedef Tile<MI, NI, ST, WM, WN> Products;
-  const int e = tile.x, begin = tile.y, count = min(Products::TM, p.first[e + 1] - begin);
+  const int e = tile.x, begin = tile.y, count = min(Products::TM, (p.first ? p.first[e + 1] : p.rows) - begin);
   Products t;
 #pragma unroll
   for (int j = 0; j < Products::LA; ++j) {
     const int row = Products::x_row(j), sorted = begin + min(row, count - 1);
-    t.xoff[j] = 2u * ((unsigned)(UP ? p.order[sorted] / p.top : sorted) * (unsigned)p.k + Products::k_of(row));
+    t.xoff[j] = 2u * ((unsigned)(UP && p.order ? p.order[sorted] / p.top : sorted) * (unsigned)p.k + Products::k_of(row));
   }
   const bf16_t* w = p.w + (size_t)e * (GATED ? 2 : 1) * p.n * p.k;
 #pragma unroll
@@ -618,7 +600,8 @@ template <int KIND>
 __global__ void __launch_bounds__(512) expert_wide_tiles_kernel(GroupedArgs p) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   constexpr int COLUMNS = KIND == UP_GATED ? 128 : 256;
-  const int used = p.tiles[p.slots].x, total = used * ((p.n + COLUMNS - 1) / COLUMNS);
+  auto tile = [&](int i) { return p.tiles ? p.tiles[i] : make_int2(0, 128 * i); };
+  const int used = p.tiles ? p.tiles[p.slots].x : p.slots, total = used * ((p.n + COLUMNS - 1) / COLUMNS);
   int whole = total / p.units * p.units;
   const int left = total - whole;
   const int pieces = 4 * left <= p.units && KIND != UP_GATED ? 4 : 2 * left <= p.units ? 2 : 1;
@@ -626,7 +609,7 @@ __global__ void __launch_bounds__(512) expert_wide_tiles_kernel(GroupedArgs p) {
   int block = blockIdx.x;
   if (block < whole) {
     const int at = by_xcd(block, whole);
-    expert_tile<KIND, 2, 2, 3, 2, 4>(p, smem, p.tiles[at % used], at / used * COLUMNS);
+    expert_tile<KIND, 2, 2, 3, 2, 4>(p, smem, tile(at % used), at / used * COLUMNS);
     return;
   }
   block -= whole;
@@ -634,14 +617,13 @@ __global__ void __launch_bounds__(512) expert_wide_tiles_kernel(GroupedArgs p) {
   const int piece = by_xcd(block, left * pieces), at = whole + piece / pieces;
   const int n0 = at / used * COLUMNS + piece % pieces * (COLUMNS / pieces);
   if (n0 >= p.n) return;
-  const int2 tile = p.tiles[at % used];
   if constexpr (KIND != UP_GATED) {
     if (pieces == 4) {
-      expert_tile<KIND, 1, 1, 4, 4, 2>(p, smem, tile, n0);
+      expert_tile<KIND, 1, 1, 4, 4, 2>(p, smem, tile(at % used), n0);
       return;
     }
   }
-  expert_tile<KIND, 1, 2, 4, 4, 2>(p, smem, tile, n0);
+  expert_tile<KIND, 1, 2, 4, 4, 2>(p, smem, tile(at % used), n0);
 }
 
 template <int KIND>
@@ -901,9 +883,9 @@ extern "C" int tnx_expert_grouped(const void* h, const int* chosen, const float*
                                                                nullptr, tiles, tile_rows, slots);
   TNX_CHECK_LAUNCH("expert order");
   const GroupedArgs up{(const bf16_t*)h, (const bf16_t*)w_gate_up, first, order, tiles, weight_on_input ? weights : nullptr, inner,
-                       top, f, width, act, slots, tnx_compute_units(), limit};
+                       top, f, width, act, slots, tnx_compute_units(), limit, 0};
   const GroupedArgs down{(const bf16_t*)inner, (const bf16_t*)w_down, first, order, tiles, nullptr, y, top, width, f, act, slots,
-                         tnx_compute_units(), limit};
+                         tnx_compute_units(), limit, 0};
   if (int rc = ungated ? launch_tiles<UP_PLAIN>(up, tile_rows, stream) : launch_tiles<UP_GATED>(up, tile_rows, stream)) return rc;
   if (int rc = launch_tiles<DOWN>(down, tile_rows, stream)) return rc;
   launch_combine<bf16_t>(y, residual, out, tokens, top, width, place, weight_on_input ? nullptr : weights,
@@ -935,6 +917,21 @@ extern "C" int tnx_gated_activation(const float* gate_up, void* out, int dtype, 
 #undef GATED_LAUNCH
   TNX_CHECK_LAUNCH("gated_activation");
   return 0;
+}
+
+// act(g) * u from the rows x [tokens, width] and w [2 f, width] (gate rows, then up rows), bfloat16, by the experts' tiles: the sums
+// stay in registers until both halves are there.
+extern "C" int tnx_gated_activation_tiles(const void* x, const void* w, void* out, int act, float limit, int tokens, int f, int width,
+                                          hipStream_t stream) {
+  TNX_REQUIRE(tokens >= 0 && f > 0 && width > 0 && width % 64 == 0 && f % 64 == 0, "gated_activation_tiles: sizes in 64s, got %d and %d", width, f);
+  TNX_REQUIRE((long long)tokens * width < (1ll << 31) && (long long)width * f < (1ll << 30) && (long long)tokens * f < (1ll << 31),
+              "gated_activation_tiles: operands of 4 GB or more");
+  TNX_REQUIRE(((uintptr_t)x | (uintptr_t)w | (uintptr_t)out) % 16 == 0, "gated_activation_tiles: operands must be 16-byte aligned");
+  if (tokens == 0) return 0;
+  const int slots = (tokens + 127) / 128;
+  TNX_REQUIRE((long long)slots * (f / 64 + 1) < (1ll << 31) - 1024, "gated_activation_tiles: too many tiles");
+  return launch_wide_tiles<UP_GATED>(GroupedArgs{(const bf16_t*)x, (const bf16_t*)w, nullptr, nullptr, nullptr, nullptr, out, 1, f, width, act,
+                                                 slots, tnx_compute_units(), limit, tokens}, stream);
 }
 
 // act(x) of float32 rows (`ld` apart), times sigmoid(row_gate) of its row (numbers `gate_ld` apart) or not

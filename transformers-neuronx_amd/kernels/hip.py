@@ -46,6 +46,7 @@ _SIGNATURES = {
                          _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
         "tnx_gemm_f32_parts": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
+        "tnx_gated_activation_skinny": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_float, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gemm_f32_workspace": [_c_int, _c_int, _c_int],
         "tnx_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
                           _c_int, _c_int, _c_int, _c_void_p],
@@ -178,6 +179,7 @@ _SIGNATURES = {
                                _c_int, _c_void_p],
         "tnx_row_activation": [_c_void_p, _c_ll, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_ll, _c_void_p],
         "tnx_gated_activation": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_void_p, _c_float, _c_void_p],
+        "tnx_gated_activation_tiles": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_float, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_expert_order": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p, _c_void_p, _c_void_p, _c_void_p,
                              _c_void_p, _c_void_p],
         "tnx_expert_combine": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p,
@@ -2593,6 +2595,48 @@ class HipOps:
                    _GATE_ACT[activation], _ptr(row_weights), float(limit or 0.0), _stream(),
                    work=lambda: (f"{t}x{two_f // 2}", t * two_f * 4.0 + out.numel() * out.element_size(), 0.0))
         return out
+
+    # Where a gated product makes its gates itself, without a launch for them and the float32 halves between (us, the product and
+    # a launch / this, on weights that no cache holds; f gate rows of K).
+    # Few rows, the kernel that streams the tile-ordered copy: up to 16 rows (8 rows, f 4,096 of 2,048 11.6 / 8.9, 8,192 of 4,096 28.1 / 25.1, 512 of
+    # 2,048 6.9 / 6.4), up to 32 below 2^25 elements (32 rows, 4,096 of 2,048 15.3 / 11.5, 1,024 of 1,024 8.3 / 6.7; but 8,192 of 4,096 29.6 / 33.8).
+    # Beyond 128 rows, the experts' tiles, where these and their parts find a quarter of the units and go round them once, or K is
+    # short: f 4,096 of 2,048 200 rows 20.9 / 20.3, 396 29.1 / 22.2, 1,024 50.4 / 37.3, 2,048 79.0 / 72.3; 8,192 of 4,096 200 52.6 / 43.8, 512 70.6 / 66.7, but 640
+    # 87.3 / 100 and 2,048 237 / 252; 2,816 of 1,024 200 14.5 / 12.4, 2,048 42.4 / 33.9; 1,024 of 1,024 200 8.9 / 9.8, 396 10.4 / 9.9; 512 of 2,048 640 14.1 / 14.9.
+    # Up to 128 rows the product's own kernels share K out (100 rows, 4,096 of 2,048 20.9 / 21.3, 8,192 of 4,096 40.1 / 43.6).
+    gated_skinny_most, gated_skinny_elements = 32, 1 << 25
+    gated_tiles_least, gated_tiles_share, gated_tiles_short = 129, 0.25, 2048
+
+    def _gated_way(self, m, f, k, tile_ordered):
+        """"skinny", "tiles" or None: how a gated product of m rows makes its gates itself."""
+        if m <= self.gated_skinny_most and tile_ordered and f % 16 == 0 and k % 128 == 0 and (m <= 16 or 2 * f * k < self.gated_skinny_elements):
+            return "skinny"
+        blocks = -(-m // 128) * -(-f // 128)
+        if (m >= self.gated_tiles_least and f % 64 == 0 and k % 64 == 0 and max(m * k, m * f) < 1 << 31 and k * f < 1 << 30
+                and -(-m // 128) * (f // 64 + 1) < (1 << 31) - 1024
+                and self.gated_tiles_share * self.compute_units <= (2 * blocks if 2 * blocks <= self.compute_units else blocks)
+                and (blocks <= self.compute_units or k <= self.gated_tiles_short)):
+            return "tiles"
+        return None
+
+    def gated_product(self, h, w, activation, limit=None):
+        """See `ReferenceOps.gated_product`."""
+        matrix, tiles = (w.tensor, w.tiles) if isinstance(w, PreparedWeight) else (w, None)
+        two_f, k = matrix.shape
+        if (type(h) is torch.Tensor and h.dtype == torch.bfloat16 == matrix.dtype == self.dtype and activation in _GATE_ACT
+                and h.dim() == 2 and h.shape[1] == k and h.is_contiguous() and matrix.is_contiguous()):
+            m, f = h.shape[0], two_f // 2
+            way = self._gated_way(m, f, k, tiles is not None) if two_f % 2 == 0 else None
+            skinny = way == "skinny"
+            if way and (_ptr(h) | _ptr(tiles if skinny else matrix)) % 16 == 0:
+                _want(h, "h")
+                out = torch.empty(m, f, dtype=self.dtype, device=h.device)
+                self._call("gemm" if skinny else "experts", "tnx_gated_activation_skinny" if skinny else "tnx_gated_activation_tiles",
+                           _ptr(h), _ptr(tiles if skinny else matrix), _ptr(out), _GATE_ACT[activation], float(limit or 0.0),
+                           *((m, two_f, k) if skinny else (m, f, k)), _stream(),
+                           work=lambda: (f"{m}x{two_f}x{k}", 2.0 * (two_f * k + m * k + m * f), 2.0 * m * two_f * k))
+                return out
+        return self.gated_activation(self.linear(h, w, None, out_f32=True, f32_by_library=True), activation, limit=limit)
 
     def row_activation(self, x, activation, row_gate=None):
         """See `ReferenceOps.row_activation`."""

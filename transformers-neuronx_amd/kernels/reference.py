@@ -882,6 +882,10 @@ class ReferenceOps:
             g, u = g * row_weights.float()[:, None], u * row_weights.float()[:, None]
         return self._gated(g, u, activation, limit).to(self.dtype)
 
+    def gated_product(self, h, w, activation, limit=None):
+        """`gated_activation` of h W^T, W's gate rows first."""
+        return self.gated_activation(self.linear(h, w, None, out_f32=True), activation, limit=limit)
+
     def row_activation(self, x, activation, row_gate=None):
         """`act(x)` from float32 `[T, F]`, times sigmoid(`row_gate`) of its row (float32 `[T, 1]`, rows may lie apart), in
         the compute dtype."""

@@ -95,8 +95,7 @@ class GatedFeedForward(FeedForward):
         self.w_down = ops.prepare_weight(tensors[d])
 
     def forward(self, h, ctx, residual):
-        inner = self.ops.gated_activation(self.ops.linear(h, self.w_in, None, out_f32=True, f32_by_library=True),
-                                          self.activation, **self.limit)
+        inner = self.ops.gated_product(h, self.w_in, self.activation, **self.limit)
         return self.ops.linear(inner, self.w_down, None, residual=residual, out_f32=True,
                                f32_by_library=residual is None)
 
@@ -273,8 +272,7 @@ class ExpertMixture(OffersRows, FeedForward):
             return x
         limit = dict(limit=self.shared_limit) if self.shared_limit is not None else {}
         if self.gated:
-            inner = ops.gated_activation(ops.linear(h, self.w_shared_in, None, out_f32=True, f32_by_library=True),
-                                         self.activation, **limit)
+            inner = ops.gated_product(h, self.w_shared_in, self.activation, **limit)
         else:
             gate_at = self.router_at + self.routed
             inner = ops.row_activation(rows[:, :self.shared_inner], self.activation,
