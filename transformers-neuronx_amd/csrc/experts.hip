@@ -797,6 +797,7 @@ extern "C" int tnx_route_product(const void* h, const void* w, const float* bias
   return 0;
 }
 
+// (`out` null: the pairs' weighted rows stay in `pair_rows`, for a product that adds them.)
 extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float* weights, const void* w_gate_up,
                                   const void* w_down, int* first, int* order, void* inner, float* pair_rows,
                                   const float* residual, float* out, int dtype, int tokens, int experts, int top,
@@ -807,6 +808,7 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
   TNX_REQUIRE(experts <= 4096, "expert_mixture: up to 4096 experts, got %d", experts);
   TNX_REQUIRE(dtype == TNX_F32 || dtype == TNX_BF16, "expert_mixture: dtype %d", dtype);
   const bool direct = top == 1 && !identity;
+  TNX_REQUIRE(out != nullptr || (!direct && !identity), "expert_mixture: only pairs' rows of experts with tensors are left to their reader");
   TNX_REQUIRE(direct || pair_rows != nullptr, "expert_mixture: several choices a token need room for their rows");
   TNX_REQUIRE(!identity || !weight_on_input, "expert_mixture: experts without tensors take their weight on the output");
   if (tokens == 0) return 0;
@@ -845,7 +847,7 @@ extern "C" int tnx_expert_mixture(const void* h, const int* chosen, const float*
     expert_product_kernel<bf16_t, DOWN><<<grid_down, 256, 0, stream>>>(down);
   }
   TNX_CHECK_LAUNCH("expert products");
-  if (!direct) {
+  if (!direct && out) {
     if (dtype == TNX_F32)
       launch_combine<float>(pair_rows, residual, out, tokens, top, width, nullptr, nullptr, identity ? (const float*)h : nullptr,
                             chosen, weights, experts, stream);

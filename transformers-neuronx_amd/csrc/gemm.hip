@@ -1168,11 +1168,14 @@ struct NormFold {
 // With GATED the rows of `w` are gate rows and as many up rows (N of both): a block takes a tile of either, sixteen columns of
 // act(gate) * up, which goes out in bfloat16 (`limit`: of the clamped form). A launch less: us, 8 rows, 4,096 gate rows of 2,048
 // 11.6 / 8.9, 8,192 of 4,096 28.1 / 25.1 (`HipOps._gated_way`).
-template <int MT, int WAVES, bool QKV, bool SHUF, int RT, bool NORMED = false, int NORM = NORM_NONE, int ROWS = 1, int PER = 1, bool GATED = false>
+// With PAIRS the residual is the sum of `residual` and of each row's `top` (up to four) rows of `pairs`, in their order: what a mixture
+// of experts leaves, whose launch for that sum takes 4 us of its own (a step of 4 such layers 446 us with it, 434 without).
+template <int MT, int WAVES, bool QKV, bool SHUF, int RT, bool NORMED = false, int NORM = NORM_NONE, int ROWS = 1, int PER = 1, bool GATED = false, bool PAIRS = false>
 __global__ void __launch_bounds__(WAVES * 64)
 gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__ w, const float* __restrict__ bias,
                         const float* __restrict__ residual, void* __restrict__ out, int out_dtype, int act, int M,
-                        int N, int K, QkvScatter sc, NormFold nf, NormArg<NORM> norm, float limit = 0.f) {
+                        int N, int K, QkvScatter sc, NormFold nf, NormArg<NORM> norm, float limit = 0.f,
+                        const float* __restrict__ pairs = nullptr, int top = 0) {
   static_assert(!GATED || (RT == 2 && SHUF && !QKV && !NORMED && NORM == NORM_NONE), "a tile of gate rows and one of up rows");
   static_assert(NORM == NORM_NONE || (MT == 1 && WAVES == 4 && !NORMED), "two rows a wave of four");
   __shared__ float norm_stat[NORM ? 16 : 1][2];
@@ -1206,7 +1209,8 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
   };
   constexpr bool EARLY = OUTS >= 1 && OUTS <= 4 && MT * RT * 4 % WAVES == 0;
   float add[EARLY ? OUTS : 1], onto[EARLY ? OUTS : 1], fold_c[EARLY ? OUTS : 1], fold_d[EARLY ? OUTS : 1];
-  float onto_w[EARLY ? OUTS : 1], onto_b[EARLY ? OUTS : 1];
+  float onto_w[EARLY ? OUTS : 1], onto_b[EARLY ? OUTS : 1], of_pair[PAIRS ? OUTS : 1][4];
+  static_assert(!PAIRS || EARLY, "the pairs' rows are asked for before the products");
   int page[EARLY ? OUTS : 1], off[EARLY ? OUTS : 1];
   static_assert(NORM == NORM_NONE || EARLY, "the residual is normed where it was asked for");
   if constexpr (EARLY) {
@@ -1218,6 +1222,10 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
       add[q] = bias ? bias[n] : 0.f;
       if (NORMED) fold_c[q] = nf.c[n], fold_d[q] = nf.d[n];
       onto[q] = !QKV && residual ? residual[(size_t)m * N + n] : 0.f;
+      if constexpr (PAIRS) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) of_pair[q][c] = pairs[((size_t)m * top + min(c, top - 1)) * N + n];
+      }
       if constexpr (NORM == NORM_RESIDUAL) {
         onto[q] = norm.x[(size_t)m * N + n];
         onto_w[q] = norm.weight ? norm.weight[n] : 1.f;
@@ -1441,7 +1449,13 @@ gemm_bf16_skinny_kernel(const bf16_t* __restrict__ x, const bf16_t* __restrict__
         if (bias) v += add[q];
         v = apply_act(v, act);
         if (NORM == NORM_RESIDUAL) v += (onto[q] - norm_stat[m][0]) * norm_stat[m][1] * onto_w[q] + onto_b[q];
-        else if (residual) v += onto[q];
+        else if constexpr (PAIRS) {
+          float o = onto[q];
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (c < top) o += of_pair[q][c];
+          v += o;
+        } else if (residual) v += onto[q];
         store_any(out, out_dtype, (size_t)m * N + n, v);
       } else {
         epilogue_store(v, m, n, N, bias, residual, out, out_dtype, act);
@@ -1633,6 +1647,27 @@ static int gemm_bf16_dispatch(const void* x, const void* w, const void* w_tiles,
     gemm_bf16_kernel<false><<<grid, 256, 0, stream>>>(xp, wp, bias, residual, out, out_dtype, act, M, N, K,
                                                       QkvScatter{});
   TNX_CHECK_LAUNCH("gemm_bf16");
+  return 0;
+}
+
+// x w^T + residual + each row's `top` rows of `pairs` [M top, N], float32, up to 16 rows, from the tile-ordered copy.
+extern "C" int tnx_gemm_bf16_pairs(const void* x, const void* w_tiles, const float* residual, const float* pairs, int top, float* out, int M,
+                                   int N, int K, hipStream_t stream) {
+  TNX_REQUIRE(M >= 0 && M <= 16 && N > 0 && N % 16 == 0 && K > 0 && K % 128 == 0 && top >= 1 && top <= 4,
+              "gemm_bf16_pairs: up to 16 rows of up to 4 pairs, N in 16s, K in 128s, got M=%d N=%d K=%d, %d", M, N, K, top);
+  TNX_REQUIRE(((uintptr_t)x | (uintptr_t)w_tiles) % 16 == 0, "gemm_bf16_pairs: operands must be 16-byte aligned");
+  if (M == 0) return 0;
+#define PAIRS_SKINNY(RT)                                                                                                               \
+  gemm_bf16_skinny_kernel<1, 4, false, true, RT, false, NORM_NONE, 1, 1, false, true><<<dim3((N / 16 + RT - 1) / RT), 256, 0, stream>>>( \
+      (const bf16_t*)x, (const bf16_t*)w_tiles, nullptr, residual, out, TNX_F32, TNX_ACT_NONE, M, N, K, QkvScatter{}, NormFold{},        \
+      NoNorm{}, 0.f, pairs, top)
+  switch (skinny_tiles_per_block(M, N)) {
+    case 1: PAIRS_SKINNY(1); break;
+    case 2: PAIRS_SKINNY(2); break;
+    default: PAIRS_SKINNY(3); break;
+  }
+#undef PAIRS_SKINNY
+  TNX_CHECK_LAUNCH("gemm_bf16_pairs");
   return 0;
 }
 

@@ -46,6 +46,7 @@ _SIGNATURES = {
                          _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
         "tnx_gemm_f32_parts": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                _c_int, _c_void_p, ctypes.c_size_t, _c_void_p],
+        "tnx_gemm_bf16_pairs": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gated_activation_skinny": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_float, _c_int, _c_int, _c_int, _c_void_p],
         "tnx_gemm_f32_workspace": [_c_int, _c_int, _c_int],
         "tnx_gemm_bf16": [_c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int,
@@ -364,6 +365,15 @@ class Onto:
 
     def __init__(self, x):
         self.x = x
+
+
+class PairRows:
+    """What `HipOps.expert_mixture` leaves to the product that reads it next as its residual: x + each token's `top` rows, into `out`."""
+
+    __slots__ = ("x", "rows", "top", "out")
+
+    def __init__(self, x, rows, top, out):
+        self.x, self.rows, self.top, self.out = x, rows, top, out
 
 
 class SharesLeft:
@@ -970,6 +980,24 @@ class HipOps:
                        int(force_tiled), int(bool(x.center)), _stream(), work=lambda: self._product_work(m, n, k, x_item=4))
             return out, None
 
+    def _linear_onto_pairs(self, x, w, bias, act, residual, out_f32, force_tiled, into):
+        """A product that adds what a mixture of experts left, or None where the general way has to (`_settled_pairs`)."""
+        m, n, k = x.shape[0], w.tensor.shape[0], w.tensor.shape[1]
+        if (bias is not None or act not in (None, "none") or not out_f32 or force_tiled or into is not None or w.tiles is None
+                or x.dtype != torch.bfloat16 or tuple(x.shape) != (m, k) or not x.is_contiguous() or m > 16 or n % 16 or k % 128
+                or (_ptr(x) | _ptr(w.tiles)) % 16):
+            return None
+        _want(residual.x, "residual", torch.float32, (m, n))
+        self._call("gemm", "tnx_gemm_bf16_pairs", _ptr(x), _ptr(w.tiles), _ptr(residual.x), _ptr(residual.rows), residual.top,
+                   _ptr(residual.out), m, n, k, _stream(), work=lambda: self._product_work(m, n, k, out_item=4, residual=True))
+        return residual.out
+
+    def _settled_pairs(self, pairs):
+        t, width = pairs.x.shape
+        self._call("experts", "tnx_expert_combine", _ptr(pairs.rows), None, None, _ptr(pairs.x), _ptr(pairs.out), t, pairs.top, width, None,
+                   None, 0, _stream())
+        return pairs.out
+
     def linear(self, x, w, bias=None, act=None, residual=None, out_f32=False, force_tiled=False, f32_by_library=False,
                into=None):
         """`f32_by_library`: a float32 result without a residual may come from the vendor library too (many rows);
@@ -979,6 +1007,11 @@ class HipOps:
             out, x = self._linear_of_norm(x, w, bias, act, residual.x if type(residual) is Onto else residual, out_f32, force_tiled, into)
             if out is not None:
                 return out
+        if type(residual) is PairRows:
+            out = self._linear_onto_pairs(x, w, bias, act, residual, out_f32, force_tiled, into)
+            if out is not None:
+                return out
+            residual = self._settled_pairs(residual)
         tiles, leaves = None, type(residual) is Onto
         if leaves:
             residual, leaves = residual.x, act in (None, "none") and out_f32 and into is None
@@ -2675,8 +2708,9 @@ class HipOps:
                 and (pairs // rows + experts) * (max(width, f) // 64 + 1) < 1 << 31)
 
     def expert_mixture(self, h, chosen, weights, w_gate_up, w_down, activation, weight_on, residual=None, may_wait=False,
-                       limit=None, identity=0):
-        """See `ReferenceOps.expert_mixture`. `may_wait`: the step is not being recorded, so the host may read
+                       limit=None, identity=0, before=None):
+        """See `ReferenceOps.expert_mixture`. `before`: the matrix of the product that takes the result as its residual and is all that
+        reads it: few rows are left to it as `PairRows`. `may_wait`: the step is not being recorded, so the host may read
         what the device has made. `identity`: how many experts without tensors the numbers behind the experts' stand
         for."""
         t, top = chosen.shape
@@ -2747,14 +2781,17 @@ class HipOps:
         rows = torch.empty(pairs, width, dtype=torch.float32, device=dev) if top > 1 or identity else None
         item = h.element_size()
         used = min(experts, pairs)
+        leaves = (rows is not None and residual is not None and isinstance(before, PreparedWeight) and before.tiles is not None
+                  and t <= 16 and 2 <= top <= 4 and not identity and h.dtype == self.dtype == torch.bfloat16
+                  and before.tensor.shape[0] == width and not debug.tapping())
         self._call("experts", "tnx_expert_mixture", _ptr(h), _ptr(chosen), _ptr(weights), _ptr(w_gate_up), _ptr(w_down),
-                   _ptr(ints[:experts + 1]), _ptr(ints[experts + 1:]), _ptr(inner), _ptr(rows), _ptr(residual), _ptr(out),
+                   _ptr(ints[:experts + 1]), _ptr(ints[experts + 1:]), _ptr(inner), _ptr(rows), _ptr(residual), None if leaves else _ptr(out),
                    _code(h.dtype), t, experts, top, width, f, (_ACT if ungated else _GATE_ACT)[activation],
                    int(weight_on == "input"), int(bool(self.expert_plain_products)), float(limit or 0.0), int(identity),
                    int(ungated), _stream(),
                    work=lambda: (f"{t}x{top} of {experts}", used * (2.0 if ungated else 3.0) * f * width * item + t * width * (item + 8.0),
                          (4.0 if ungated else 6.0) * t * top * f * width))
-        return out
+        return PairRows(residual, rows, top, out) if leaves else out
 
     # ---------------------------------------------------------------- output end
 

@@ -895,7 +895,7 @@ class ReferenceOps:
         return y.to(self.dtype)
 
     def expert_mixture(self, h, chosen, weights, w_gate_up, w_down, activation, weight_on, residual=None, may_wait=False,
-                       limit=None, identity=0):
+                       limit=None, identity=0, before=None):
         """float32 `residual + sum_c expert_(chosen[t, c])(h[t])` with the weights `weights[t, c]` on the expert's
         input (`weight_on="input"`: act(w g) * (w u), the float32 sums of the first product times w) or on its
         output. `w_gate_up` `[E, 2 F, D]` (gate rows, then up rows), `w_down` `[E, D, F]`. `w_gate_up` `[E, F, D]`:

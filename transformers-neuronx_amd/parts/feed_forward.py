@@ -266,6 +266,8 @@ class ExpertMixture(OffersRows, FeedForward):
         if self.identity:
             limit["identity"] = self.identity
         # (a step that is being recorded is sized by `length_bound`; any other may let the host read)
+        if self.shared_inner:
+            limit["before"] = self.w_shared_down        # the product that takes the sum as its residual
         x = ops.expert_mixture(h, chosen, weights, self.w_gate_up, self.w_down, self.activation, self.weight_on, residual,
                                may_wait=ctx is not None and ctx.length_bound is None, **limit)
         if not self.shared_inner:
