@@ -2594,17 +2594,20 @@ class HipOps:
     def route_product(self, h, w, bias, experts, top, score="sigmoid", renormalize=False, correction=None, scale=1.0, groups=None):
         """See `ReferenceOps.route_product`."""
         matrix = w.tensor if isinstance(w, PreparedWeight) else w
-        t, width = h.shape
+        (t, width), (logits, inner) = h.shape, matrix.shape
+        if not 1 <= experts <= logits:
+            raise ValueError(f"a router of {logits} rows, {experts} experts")
         if (experts > self.route_product_most or t * experts > self.route_product_logits or h.dtype != torch.bfloat16
-                or matrix.dtype != torch.bfloat16 or matrix.shape[1] != width or width % 8 or not (h.is_contiguous() and matrix.is_contiguous())
+                or matrix.dtype != torch.bfloat16 or inner != width or width % 8 or not (h.is_contiguous() and matrix.is_contiguous())
                 or (_ptr(h) | _ptr(matrix)) % 16):
             return self.route(self.linear(h, w, bias, out_f32=True, f32_by_library=True)[:, :experts], top, score, renormalize, correction,
                               scale, groups)
         _want(h, "h")
+        _want(matrix, "w")
         if score not in ("sigmoid", "softmax"):
             raise ValueError(f"unknown router score {score!r}")
         if bias is not None:
-            _want(bias, "bias", torch.float32, (matrix.shape[0],))
+            _want(bias, "bias", torch.float32, (logits,))
         if correction is not None:
             _want(correction, "the choice's correction", torch.float32, (experts,))
         chosen = torch.empty(t, top, dtype=torch.int32, device=h.device)

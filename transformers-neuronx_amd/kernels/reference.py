@@ -871,7 +871,10 @@ class ReferenceOps:
 
     def route_product(self, h, w, bias, experts, top, score="sigmoid", renormalize=False, correction=None, scale=1.0, groups=None):
         """`route` of the first `experts` columns of h W^T + bias."""
-        return self.route(self.linear(h, w, bias, out_f32=True)[:, :experts], top, score, renormalize, correction, scale, groups)
+        z = self.linear(h, w, bias, out_f32=True)
+        if not 1 <= experts <= z.shape[1]:
+            raise ValueError(f"a router of {z.shape[1]} rows, {experts} experts")
+        return self.route(z[:, :experts], top, score, renormalize, correction, scale, groups)
 
     def gated_activation(self, gate_up, activation, row_weights=None, limit=None):
         """`act(g) * u` from float32 `[T, 2 F]` = [g | u], in the compute dtype; `row_weights` `[T]`: a factor a
