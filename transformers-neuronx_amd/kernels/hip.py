@@ -2666,6 +2666,7 @@ class HipOps:
             skinny = way == "skinny"
             if way and (_ptr(h) | _ptr(tiles if skinny else matrix)) % 16 == 0:
                 _want(h, "h")
+                _want(matrix, "w")
                 out = torch.empty(m, f, dtype=self.dtype, device=h.device)
                 self._call("gemm" if skinny else "experts", "tnx_gated_activation_skinny" if skinny else "tnx_gated_activation_tiles",
                            _ptr(h), _ptr(tiles if skinny else matrix), _ptr(out), _GATE_ACT[activation], float(limit or 0.0),
