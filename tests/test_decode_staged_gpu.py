@@ -42,3 +42,24 @@ def test_the_rule_gives_launches_that_exist(head_size, window):
         assert waves in ((2, 4) if head_size > 80 else (2, 4, 8)) and 1 <= splits <= 8
         # no share without keys of the longest request's, and no more shares than units where the pairs leave some idle
         assert splits <= max(1, fills) and (splits == 1 or splits * pairs <= 256 or pairs > 256)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("hs", [64, 128])
+def test_pages_that_begin_anywhere(hs):
+    """Pages of 64 keys that do not begin on 16 bytes: the keys and values go through registers, with the same results."""
+    from test_kernels_gpu import _fill_cache_and_compare
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ctx, q, kp, vp, _ = _fill_cache_and_compare(torch.bfloat16, 2, 2, hs, 64, [1] * len(LENGTHS), [n - 1 for n in LENGTHS], None)
+
+    def moved(pages):
+        room = torch.empty(pages.numel() + 4, dtype=pages.dtype, device=DEV)
+        return room[4:].view(pages.shape).copy_(pages)
+
+    assert moved(kp).data_ptr() % 16 == 8
+    ops = HipOps(torch.bfloat16, DEV)
+    ops._splits_for = lambda *a: (2, 4)
+    view = ctx.groups["full"]
+    got = [ops.attention(q, 2, 2, hs, ctx, view, k, v).float() for k, v in ((kp, vp), (moved(kp), moved(vp)), (kp, moved(vp)))]
+    # (the same products and sums in the same order)
+    assert torch.equal(got[0], got[1]) and torch.equal(got[0], got[2])

@@ -2171,7 +2171,9 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   const bool pack = group > 1;
   const int cols = head_size <= 128 ? 16 : 8;
   dim3 grid(num_splits, pack ? num_kv * ((group + cols - 1) / cols) : num_heads, num_decode);
-  const bool staged = page_size >= 64 && (head_size == 32 || head_size == 64 || head_size == 80 || head_size == 96 || head_size == 128);
+  // (loads straight into LDS are of 16 aligned bytes; into registers they may lie anywhere)
+  const bool staged = page_size >= 64 && (head_size == 32 || head_size == 64 || head_size == 80 || head_size == 96 || head_size == 128) &&
+                      ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
 #define MFMA_ARGS                                                                                                 \
   (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, run_start, cached_lens, table, table_width,    \
       page_shift, num_pages, decode_runs, (bf16_t*)out, part_o, part_ml, num_heads, num_kv, window, num_splits,    \
