@@ -1770,7 +1770,10 @@ extern "C" int tnx_attention_prefill_scored(const void* q, const void* k_pages, 
 // kv head of one request, and the 16 columns hold up to 16 (8 at the largest head size) different query heads
 // of its group, so the keys and values are read once for all of them and not once a head; the maxima, sums and
 // results are a column's own throughout (a column is the lanes with the same lane % 16).
-template <int NDB, int NW, bool PACK, bool STAGED>
+// SHARED (a group of more than 16 heads, staged): two blocks or more read the same keys and values, so they are not marked as read once. us,
+// registers / marked / not: 24 of 700, 71 heads on 1 of 64 11.1 / 11.4 / 9.1; 8 of 2,000, 32 on 1 of 128 14.3 / 13.4 / 13.1; 64 of 2,000, 64 on 2 of 64
+// 26.1 / 26.6 / 25.3, of 128 47.0 / 47.6 / 48.5: what is left to registers at many requests is 3 to 7 %, of 108 sizes at three.
+template <int NDB, int NW, bool PACK, bool STAGED, bool SHARED = false>
 __global__ void __launch_bounds__(64 * NW, (NDB <= 8 ? 2 : 1))
 attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restrict__ k_pages,
                              const bf16_t* __restrict__ v_pages, const int* __restrict__ run_start,
@@ -1872,15 +1875,19 @@ attention_decode_mfma_kernel(const bf16_t* __restrict__ q, const bf16_t* __restr
       voff[i] = (unsigned)(d * page_size * 2 + ((c & 7) ^ ((d >> 1) & 7)) * 16);
     }
   }
+  auto stage = [](const bf16_t* p, unsigned offset, unsigned lds) {
+    if constexpr (SHARED) load_to_lds(p, offset, lds);
+    else load_to_lds_once(p, offset, lds);
+  };
   auto stage_keys = [&](int page, int tile0) {
     const bf16_t* kp = k_pages + (size_t)page * page_stride + (size_t)kvh * head_stride + (size_t)(tile0 & pmask) * DH;
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_to_lds_once(kp, koff[STAGED ? i : 0], lds_offset(k_mine) + i * 1024);
+    for (int i = 0; i < LOADS; ++i) stage(kp, koff[STAGED ? i : 0], lds_offset(k_mine) + i * 1024);
   };
   auto stage_values = [&](int page, int tile0) {
     const bf16_t* vp = v_pages + (size_t)page * page_stride + (size_t)kvh * head_stride + (tile0 & pmask);
 #pragma unroll
-    for (int i = 0; i < LOADS; ++i) load_to_lds_once(vp, voff[STAGED ? i : 0], lds_offset(v_mine) + i * 1024);
+    for (int i = 0; i < LOADS; ++i) stage(vp, voff[STAGED ? i : 0], lds_offset(v_mine) + i * 1024);
   };
   auto page_of = [&](int tile0) {
     const int key = __builtin_amdgcn_readfirstlane(min(tile0, last_key));
@@ -2134,16 +2141,16 @@ __global__ void attention_decode_merge_kernel(const float* __restrict__ part_o, 
   }
 }
 
-template <int NDB, int NW, bool PACK, typename... Args>
+template <int NDB, int NW, bool PACK, bool SHARED, typename... Args>
 static int launch_decode_staged(dim3 grid, hipStream_t stream, Args... args) {
   constexpr int bytes = NW * 16 * NDB * 256;
   static bool configured = false;
   if (!configured) {
-    hipError_t e = hipFuncSetAttribute((const void*)attention_decode_mfma_kernel<NDB, NW, PACK, true>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
+    hipError_t e = hipFuncSetAttribute((const void*)attention_decode_mfma_kernel<NDB, NW, PACK, true, SHARED>, hipFuncAttributeMaxDynamicSharedMemorySize, bytes);
     TNX_REQUIRE(e == hipSuccess, "attention_decode: cannot reserve %d bytes of LDS: %s", bytes, hipGetErrorString(e));
     configured = true;
   }
-  attention_decode_mfma_kernel<NDB, NW, PACK, true><<<grid, 64 * NW, bytes, stream>>>(args...);
+  attention_decode_mfma_kernel<NDB, NW, PACK, true, SHARED><<<grid, 64 * NW, bytes, stream>>>(args...);
   return 0;
 }
 
@@ -2170,6 +2177,7 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   const int group = num_heads / num_kv;
   const bool pack = group > 1;
   const int cols = head_size <= 128 ? 16 : 8;
+  const bool shared = group > cols;
   dim3 grid(num_splits, pack ? num_kv * ((group + cols - 1) / cols) : num_heads, num_decode);
   // (loads straight into LDS are of 16 aligned bytes; into registers they may lie anywhere)
   const bool staged = page_size >= 64 && (head_size == 32 || head_size == 64 || head_size == 80 || head_size == 96 || head_size == 128) &&
@@ -2178,13 +2186,14 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, run_start, cached_lens, table, table_width,    \
       page_shift, num_pages, decode_runs, (bf16_t*)out, part_o, part_ml, num_heads, num_kv, window, num_splits,    \
       longest, head_size, page_pad
-#define LAUNCH_STAGED(NDB, NW, PACK) launch_decode_staged<NDB, NW, PACK>(grid, stream, MFMA_ARGS)
+#define LAUNCH_STAGED(NDB, NW)                                                    \
+  (shared ? launch_decode_staged<NDB, NW, true, true>(grid, stream, MFMA_ARGS)    \
+   : pack ? launch_decode_staged<NDB, NW, true, false>(grid, stream, MFMA_ARGS)   \
+          : launch_decode_staged<NDB, NW, false, false>(grid, stream, MFMA_ARGS))
 #define LAUNCH_MFMA(NDB)                                                                                                   \
   if (staged) {                                                                                                            \
     constexpr int MOST = NDB <= 5 ? 8 : 4;                                                                                 \
-    if (int rc = waves >= MOST ? (pack ? LAUNCH_STAGED(NDB, MOST, true) : LAUNCH_STAGED(NDB, MOST, false))                 \
-                 : waves == 4  ? (pack ? LAUNCH_STAGED(NDB, 4, true) : LAUNCH_STAGED(NDB, 4, false))                       \
-                               : (pack ? LAUNCH_STAGED(NDB, 2, true) : LAUNCH_STAGED(NDB, 2, false)))                      \
+    if (int rc = waves >= MOST ? LAUNCH_STAGED(NDB, MOST) : waves == 4 ? LAUNCH_STAGED(NDB, 4) : LAUNCH_STAGED(NDB, 2))    \
       return rc;                                                                                                           \
   } else if (waves == 8 && pack)                                                                                           \
     attention_decode_mfma_kernel<NDB, 8, true, false><<<grid, 512, 0, stream>>>(MFMA_ARGS);                                \
