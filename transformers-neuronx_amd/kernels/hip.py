@@ -1625,18 +1625,21 @@ class HipOps:
 
     def _splits_for(self, longest: int, fills: int, alike: bool, pairs: int, window: int, head_size: int):
         """`fills`: the blocks of 256 keys that the longest request fills now, `longest` what it may come to before a recorded step is
-        replaced. `pairs`: blocks that read whole requests. A block of four waves fills half of a unit's LDS up to heads of 80,
-        all of it beyond, where eight do not fit. us, 32 heads of 64 or 80 or (so marked) 128 where nothing else is said:
+        replaced. `pairs`: blocks that read whole requests. A wave holds 256 bytes of LDS an element of the head: of a unit's 160 KB a
+        block of four takes 64 KB at heads of 64 and 80 at 80, so that two find room, 96 at 96 and 128 at 128, where eight do not fit. us, 32 heads of 64 or 80 or (so marked) 128 where nothing else is said:
         - the pairs leave half of the units idle, or two thirds up to heads of 80, and the keys are many: as many blocks as units share
           them (1 request of 2,000 20.5 whole / 10.6 in eight, 2 of 128 21 / 17.1 in four, 3 of 128 26.4 / 22.3 in two; but 1 of 700
           8.5 / 9.4, and 3 of 1,000 11.2 / 12.0 in two, since the kernel that merges costs 2);
         - at most one block a unit: as many waves as 256 keys, twice and four times as many keep at a tile or two each (1 of 100 5.0 with two,
-          5.2 with four, 5.4 with eight; 500 9.0, 7.9, 8.1; 5 of 700 12.2, 10.6, 10.0); four where nearly all units have a block;
+          5.2 with four, 5.4 with eight; 500 9.0, 7.9, 8.1; 5 of 700 12.2, 10.6, 10.0); four where nearly all units have a block, and where
+          the lengths are unlike until the keys are shared or, where they are not, heads of up to 80 have more than 512 keys;
         - more pairs than units, not a whole number on each, of requests about as long as one another: shares of the keys come out
           more even (9 of 2,000 37.6 / 34.2 in four, of 128 900 32.9 / 30.3 with two waves; but 33 of 900 53.9 / 60.4). Requests of
           unlike lengths are not cut (24 of up to 1,500 43.5 / 51.4 in two);
         - else blocks of two waves where requests are short, of which more are on a unit at once and none waits for another's end: 24 of
-          up to 400, heads of 80 18.5 with four / 14.8, 64 of 128 72 / 51.5; 24 of 1,500 58.3 / 58.7, of 128 93.8 / 98.9."""
+          up to 400, heads of 80 18.5 with four / 14.8, 64 of 128 72 / 51.5; 24 of 1,500 58.3 / 58.7, of 128 93.8 / 98.9.
+        Requests of unlike lengths cross one line of `fills` and no more: a recorded step is recorded again there (1.3b 5 to 9 ms, where
+        a step is 1.2 of 3 requests, 1.8 of 24), and such a batch crosses back whenever its longest request ends."""
         most = min(8, fills)          # shares of 256 keys now, or of what a request may come to
         if not alike:
             most = min(8, -(-longest // 256))
@@ -1651,6 +1654,8 @@ class HipOps:
         if shares > (1 if wide else 2) and fills > (2 if wide else 3):
             return shares, 4
         if pairs <= units:
+            if not alike:
+                return 1, 8 if not wide and shares <= 2 and fills > 2 and 10 * pairs < 7 * units else 4
             return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or (wide and fills > 2) else 2 if fills <= 1 else 8
         if alike and fills >= (4 if wide else 8) and -(-pairs // units) * units > 1.05 * pairs:
             return 4, 2 if wide else 4
@@ -1661,9 +1666,11 @@ class HipOps:
     def attention_launch_shape(self, step, num_heads: int, window, head_size: int, num_kv_heads: Optional[int] = None):
         """What the decode attention's launch in a recorded step is sized by beyond the number of requests: the
         blocks that share a request's keys (and their waves), for a `PackedStep` about to be replayed. A
-        recorded step is sized for the longest request the model allows; how requests about as long as one
-        another are cut depends on how long they are now, so a batch that grows is recorded again only when
-        that changes the launch (8 requests of 32 heads: never; 9: at every 256 keys up to eight blocks)."""
+        recorded step is sized for the longest request the model allows; how requests are cut, and how many waves
+        read them, depends on how long the longest is now, so a batch that grows is recorded again only when
+        that changes the launch: of unlike lengths once, of like ones up to seven times where their keys are
+        shared (1 request of 32 heads, at every 256 keys), never where the pairs alone are nearly a block a
+        unit (8 of 32 heads), else up to three times (`_splits_for`)."""
         n_dec = int((step.run_lens == 1).sum())
         if n_dec == 0 or self.dtype != torch.bfloat16:
             return None
