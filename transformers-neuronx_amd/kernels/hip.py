@@ -1545,8 +1545,9 @@ class HipOps:
                        _stream(), work=lambda: self._attention_work(ctx, "prompt", num_heads, num_kv_heads, head_size, window, 2))
         n_dec = ctx.plan["decode_runs"].numel()
         if n_dec:
+            staged = self._decode_staged(head_size, view.page_size) and (_ptr(k_pages) | _ptr(v_pages)) % 16 == 0
             splits, waves = self._decode_splits(ctx, n_dec * self._decode_blocks(num_heads, num_kv_heads, head_size),
-                                                window, head_size)
+                                                window, head_size, staged)
             part_o = part_ml = None
             if splits > 1:
                 part_o = torch.empty(n_dec * num_heads * splits * head_size, dtype=torch.float32, device=q.device)
@@ -1616,17 +1617,23 @@ class HipOps:
             return num_heads
         return num_kv_heads * -(-group // (16 if head_size <= 128 else 8))
 
-    def _decode_splits(self, ctx, pairs: int, window: int, head_size: int = 128):
+    @staticmethod
+    def _decode_staged(head_size: int, page_size: int) -> bool:
+        """Whether the kernel that brings keys and values straight into LDS takes pages of this kind (`attention_decode_run`)."""
+        return page_size >= 64 and head_size in (32, 64, 80, 96, 128)
+
+    def _decode_splits(self, ctx, pairs: int, window: int, head_size: int = 128, staged: bool = True):
         """(splits, waves): how many blocks share the keys of one decoding (request, head), and how many waves a block has
         (`_splits_for`)."""
         longest = ctx.length_bound if ctx.length_bound is not None else ctx.plan_host["longest_decode"]
         fills, alike = ctx.plan_host.get("decode_shape", (0, False))
-        return self._splits_for(longest, fills, alike, pairs, window, head_size)
+        return self._splits_for(longest, fills, alike, pairs, window, head_size, staged)
 
-    def _splits_for(self, longest: int, fills: int, alike: bool, pairs: int, window: int, head_size: int):
+    def _splits_for(self, longest: int, fills: int, alike: bool, pairs: int, window: int, head_size: int, staged: bool = True):
         """`fills`: the blocks of 256 keys that the longest request fills now, `longest` what it may come to before a recorded step is
         replaced. `pairs`: blocks that read whole requests. A wave holds 256 bytes of LDS an element of the head: of a unit's 160 KB a
-        block of four takes 64 KB at heads of 64 and 80 at 80, so that two find room, 96 at 96 and 128 at 128, where eight do not fit. us, 32 heads of 64 or 80 or (so marked) 128 where nothing else is said:
+        block of four takes 64 KB at heads of 64 and 80 at 80, so that two find room, 96 at 96 and 128 at 128, where eight do not fit.
+        us, 32 heads of 64 or 80 or (so marked) 128 where nothing else is said:
         - the pairs leave half of the units idle, or two thirds up to heads of 80, and the keys are many: as many blocks as units share
           them (1 request of 2,000 20.5 whole / 10.6 in eight, 2 of 128 21 / 17.1 in four, 3 of 128 26.4 / 22.3 in two; but 1 of 700
           8.5 / 9.4, and 3 of 1,000 11.2 / 12.0 in two, since the kernel that merges costs 2);
@@ -1638,30 +1645,42 @@ class HipOps:
           unlike lengths are not cut (24 of up to 1,500 43.5 / 51.4 in two);
         - else blocks of two waves where requests are short, of which more are on a unit at once and none waits for another's end: 24 of
           up to 400, heads of 80 18.5 with four / 14.8, 64 of 128 72 / 51.5; 24 of 1,500 58.3 / 58.7, of 128 93.8 / 98.9.
-        Requests of unlike lengths cross one line of `fills` and no more: a recorded step is recorded again there (1.3b 5 to 9 ms, where
-        a step is 1.2 of 3 requests, 1.8 of 24), and such a batch crosses back whenever its longest request ends."""
+        Requests of unlike lengths cross one line of `fills` and no more: a recorded step is recorded again there (1.3b 5 to 10 ms, where
+        a step is 1.2 of 3 requests, 1.8 of 24), and such a batch crosses back whenever its longest request ends.
+
+        Not `staged` (small pages, other heads): blocks have four waves or eight, and where keys are many or heads beyond 128 more shares
+        pay, whatever the pairs, since more of these blocks are on a unit and start as others end: as many as 256 keys, or, where
+        lengths are unlike, as give every unit a block. us, as above / so: pages of 16, 32 heads of 64, 3 of 2,000 15.7 / 14.0, 9 of 1,000
+        20.8 / 19.1, 33 of 1,000 54.5 / 51.5; heads of 112, 5 of 2,000 38.6 / 34.7; 16 heads of 256, 1 of 300 14.9 / 12.1; but pages of 16, heads of
+        64, 5 of 300 7.5 / 9.4, of 80, 5 of 1,000 12.1 / 15.6, 9 of 300 9.5 / 13.1."""
         most = min(8, fills)          # shares of 256 keys now, or of what a request may come to
         if not alike:
             most = min(8, -(-longest // 256))
         if window:
             within = -(-min(longest, window + 64) // 256)
             fills, most = min(fills, within), min(most, within)
-        units, wide = self.compute_units, head_size > 80
+        units, wide, two = self.compute_units, head_size > 80, 2 if staged else 4
         if self.decode_blocks_wanted or self.decode_waves == 8:     # told what to make (measurements and tests)
             blocks = self.decode_blocks_wanted or units
             return max(1, min(-(-blocks // pairs), -(-longest // 256))), 8 if self.decode_waves == 8 and head_size <= 128 else 4
+        many = fills > (2 if wide else 3)
+        if not staged and (head_size > 128 or fills > 4 or (fills == 4 and pairs > units) or (many and not alike)):
+            if 0.7 * units <= pairs <= units:
+                return 1, 4
+            few = max(1, min(-(-units // pairs), most))
+            return (few if not alike or -(-pairs // units) * units <= 1.05 * pairs and pairs > units else max(few, most)), 4
         shares = min(most, units // pairs)
-        if shares > (1 if wide else 2) and fills > (2 if wide else 3):
+        if shares > (1 if wide else 2) and many:
             return shares, 4
         if pairs <= units:
             if not alike:
-                return 1, 8 if not wide and shares <= 2 and fills > 2 and 10 * pairs < 7 * units else 4
-            return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or (wide and fills > 2) else 2 if fills <= 1 else 8
+                return 1, 8 if staged and not wide and shares <= 2 and fills > 2 and 10 * pairs < 7 * units else 4
+            return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or (wide and fills > 2) else two if fills <= 1 else 8
         if alike and fills >= (4 if wide else 8) and -(-pairs // units) * units > 1.05 * pairs:
-            return 4, 2 if wide else 4
+            return 4, two if wide else 4
         if not wide and pairs <= 2 * units:
             return 1, 4
-        return 1, 2 if fills <= (4 if wide else 2) else 4
+        return 1, two if fills <= (4 if wide else 2) else 4
 
     def attention_launch_shape(self, step, num_heads: int, window, head_size: int, num_kv_heads: Optional[int] = None):
         """What the decode attention's launch in a recorded step is sized by beyond the number of requests: the
@@ -1676,8 +1695,8 @@ class HipOps:
             return None
         fills, alike = step.plan_host.get("decode_shape", (0, False))
         blocks = self._decode_blocks(num_heads, num_kv_heads or num_heads, head_size)
-        return ("decode", blocks, head_size) + self._splits_for(step.length_bound, fills, alike, n_dec * blocks,
-                                                                int(window or 0), head_size)
+        return ("decode", blocks, head_size) + self._splits_for(step.length_bound, fills, alike, n_dec * blocks, int(window or 0),
+                                                                head_size, self._decode_staged(head_size, step.page_size))
 
     # ---------------------------------------------------------------- layers in one launch
 
