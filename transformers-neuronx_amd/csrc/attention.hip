@@ -1743,7 +1743,7 @@ extern "C" int tnx_attention_prefill_scored(const void* q, const void* k_pages, 
 // ------------------------------------------------------------------------------------------ bfloat16, decoding
 
 // One query per request over its pages, on the matrix unit. The keys of a request are split over `num_splits`
-// blocks; a block's NW waves (four or eight) take 64-key tiles in turn. Partial results (maximum, sum, weighted
+// blocks; a block's NW waves (two, four or eight) take 64-key tiles in turn. Partial results (maximum, sum, weighted
 // values, all float32) of waves meet in LDS and those of splits in a workspace that a second kernel merges. The
 // page size is a power of two here.
 // The one query of a (request, head) is the B operand of S^T = K q in all 16 of
@@ -2171,7 +2171,7 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   TNX_REQUIRE(num_splits == 1 || (part_o && part_ml), "attention_decode: splits need a workspace");
   TNX_REQUIRE(num_heads <= 65535 && num_decode <= 65535, "attention_decode: too many heads or requests");
   TNX_REQUIRE(waves == 4 || waves == 2 || (waves == 8 && head_size <= 128),
-              "attention_decode: blocks have 4 waves, or 8 up to head size 128; not %d at head size %d", waves, head_size);
+              "attention_decode: blocks have 2 or 4 waves, or 8 up to head size 128; not %d at head size %d", waves, head_size);
   if (num_decode <= 0) return 0;
   // query heads that share keys and values are taken together, up to 16 a block (8 at head sizes beyond 128)
   const int group = num_heads / num_kv;
@@ -2179,9 +2179,10 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
   const int cols = head_size <= 128 ? 16 : 8;
   const bool shared = group > cols;
   dim3 grid(num_splits, pack ? num_kv * ((group + cols - 1) / cols) : num_heads, num_decode);
-  // (loads straight into LDS are of 16 aligned bytes; into registers they may lie anywhere)
+  // (loads straight into LDS are of 16 aligned bytes; into registers they may lie anywhere. Eight waves of heads beyond 80 find no
+  // room in LDS: asked for, they read into registers. Two waves are the staging kernel's only: asked for elsewhere, they are four.)
   const bool staged = page_size >= 64 && (head_size == 32 || head_size == 64 || head_size == 80 || head_size == 96 || head_size == 128) &&
-                      ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
+                      ((uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0 && !(waves == 8 && head_size > 80);
 #define MFMA_ARGS                                                                                                 \
   (const bf16_t*)q, (const bf16_t*)k_pages, (const bf16_t*)v_pages, run_start, cached_lens, table, table_width,    \
       page_shift, num_pages, decode_runs, (bf16_t*)out, part_o, part_ml, num_heads, num_kv, window, num_splits,    \
@@ -2192,8 +2193,8 @@ static int attention_decode_run(const void* q, const void* k_pages, const void* 
           : launch_decode_staged<NDB, NW, false, false>(grid, stream, MFMA_ARGS))
 #define LAUNCH_MFMA(NDB)                                                                                                   \
   if (staged) {                                                                                                            \
-    constexpr int MOST = NDB <= 5 ? 8 : 4;                                                                                 \
-    if (int rc = waves >= MOST ? LAUNCH_STAGED(NDB, MOST) : waves == 4 ? LAUNCH_STAGED(NDB, 4) : LAUNCH_STAGED(NDB, 2))    \
+    constexpr int MOST = NDB <= 5 ? 8 : 4;     /* (eight waves come here where they find room) */                          \
+    if (int rc = waves == 8 ? LAUNCH_STAGED(NDB, MOST) : waves == 4 ? LAUNCH_STAGED(NDB, 4) : LAUNCH_STAGED(NDB, 2))       \
       return rc;                                                                                                           \
   } else if (waves == 8 && pack)                                                                                           \
     attention_decode_mfma_kernel<NDB, 8, true, false><<<grid, 512, 0, stream>>>(MFMA_ARGS);                                \
