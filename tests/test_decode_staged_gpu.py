@@ -33,6 +33,7 @@ def test_waves_and_shares_agree(heads, kv, hs, ps, window):
 @pytest.mark.parametrize("head_size", [64, 80, 128])
 @pytest.mark.parametrize("window", [0, 1024])
 def test_the_rule_gives_launches_that_exist(head_size, window):
+    """(What it answers at the sizes that were measured: `test_decode_shapes.py`.)"""
     from transformers_neuronx_amd.kernels.hip import HipOps
     ops = HipOps.__new__(HipOps)
     ops.compute_units = 256

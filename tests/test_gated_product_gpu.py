@@ -15,7 +15,7 @@ def _check(ops, m, f, k, act, limit, entry):
     call = ops._call
     ops._call = lambda module, name, *a, **kw: (ran.append(name), call(module, name, *a, **kw))[1]
     got = ops.gated_product(h, w, act, limit)
-    assert ran == [entry] and got.shape == (m, f) and got.dtype == torch.bfloat16
+    assert (ran == [entry] if entry else ran[-1] == "tnx_gated_activation") and got.shape == (m, f) and got.dtype == torch.bfloat16
     z = h.double() @ raw.double().T
     a, u = z[:, :f], z[:, f:]
     if act == "silu":
@@ -47,3 +47,16 @@ def test_tiles(m, f, k, act, limit):
     ops = HipOps(torch.bfloat16, DEV)
     ops.gated_tiles_share = 0
     _check(ops, m, f, k, act, limit, "tnx_gated_activation_tiles")
+
+
+@pytest.mark.parametrize("m,f,k,entry", [
+    (16, 4096, 4096, "skinny"), (32, 4096, 2048, "skinny"), (32, 4096, 4096, None),             # 2^25 elements, 17 rows and more
+    (33, 512, 256, None), (128, 2048, 512, None), (129, 2048, 512, "tiles"),                    # the rows between
+    (200, 1920, 192, None), (200, 1984, 192, "tiles"), (256, 2048, 64, "tiles"),                # a quarter of 256 units
+    (1100, 4096, 2048, "tiles"), (1100, 4096, 2112, None), (1100, 3584, 2112, "tiles")])        # more than one a unit, and K
+def test_either_side_of_the_lines(m, f, k, entry):
+    """The rule as it stands, at sizes where it turns, and the general way beyond."""
+    from transformers_neuronx_amd.kernels.hip import HipOps
+    ops = HipOps(torch.bfloat16, DEV)
+    ops.compute_units = 256
+    _check(ops, m, f, k, "silu", None, entry and f"tnx_gated_activation_{entry}")

@@ -19,3 +19,15 @@ def test_matrices_not_on_the_gpu_are_refused(monkeypatch):
     with pytest.raises(ValueError, match="on the GPU"):
         ops.gated_product(h, torch.zeros(2 * 8192, 64, dtype=torch.bfloat16), "silu")
     assert not calls
+
+
+def test_lines_of_the_rule():
+    """Where it turns: 2^25 elements from 17 rows on, 33 to 128 rows, a quarter of the units, more tiles than units with K beyond 2,048, and
+    sizes that the kernels do not take."""
+    way = _ops()._gated_way
+    for want, *args in [("skinny", 16, 8192, 4096, True), ("skinny", 17, 4080, 4096, True), (None, 17, 4096, 4096, True), ("skinny", 32, 4096, 2048, True),
+                        (None, 16, 8192, 4096, False), (None, 16, 4104, 4096, True), (None, 16, 4096, 4160, True), (None, 33, 512, 256, True),
+                        (None, 128, 8192, 2048, True), ("tiles", 129, 8192, 2048, True), (None, 200, 1920, 2048, True), ("tiles", 200, 1984, 2048, True),
+                        ("tiles", 1024, 4096, 4096, True), (None, 1025, 4096, 4096, True), ("tiles", 1025, 4096, 2048, True), (None, 200, 8224, 2048, True),
+                        (None, 200, 8192, 2080, True)]:
+        assert way(*args) == want, args

@@ -48,13 +48,18 @@ def test_products_that_the_rule_takes(m, n, k):
 
 
 def test_the_rule_asks_for_what_it_uses():
-    """The workspace is the shares' sums, of at least eight steps of K each, and sizes beyond the tiles' reach are refused."""
+    """The workspace is the shares' sums, and sizes beyond the tiles' reach are refused. A share has as many steps of K as come to each,
+    rounded up, eight at least; the last one has what is left, one at least (64 steps in seven shares: six of ten and one of four)."""
     from transformers_neuronx_amd.kernels.hip import library
     room = library("gemm").tnx_gemm_bf16_tiles_workspace
     for m in (33, 64, 65, 96, 100, 128, 129, 200, 333, 512, 576, 640, 705, 768):
         for n in (8, 64, 1000, 1024, 2048, 3072, 6144, 10240, 50272):
             for k in (64, 128, 1024, 2048, 2560, 4096, 8192, 16384):
                 r = room(m, n, k)
-                assert r == -1 or r % (m * n) == 0 and (r == 0 or 2 <= r // (m * n) <= 8 and k // 64 >= 8 * (r // (m * n) - 1))
+                assert r == -1 or r % (m * n) == 0
+                if r > 0:
+                    shares, steps = r // (m * n), k // 64
+                    each = -(-steps // shares)
+                    assert 2 <= shares <= 8 and each >= 8 and 1 <= steps - (shares - 1) * each <= each
     for m, n, k in ((32, 1024, 1024), (769, 1024, 1024), (100, 1001, 1024), (100, 1024, 1000), (0, 64, 64)):
         assert room(m, n, k) == -1
