@@ -2289,14 +2289,9 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 // 31.3 and 26.7, 26.1), those of 96 x 64 no quicker than the others, and those of 96 x 96 only alone (333 rows 6,144 x 2,048 17.6 for 18.7; a prompt of
 // 333 tokens of 1.3b 2,368 us with them and 2,363 without: one kernel fewer to fetch). Up to 32 rows half a tile would be padding, and other kernels stand ready.
 enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2, TILES_64x128 = 3, TILES_96x128 = 4, TILES_MOST = 4 };
-static const struct { int rows, columns; } TILE_SIZES[TILES_MOST + 1] = {{0, 0}, {64, 64}, {128, 128}, {64, 128}, {96, 128}};
 
-static float tiles_time(int tile, int M, int N, int K, int shares, int units) {
-  const int steps = K / 64, per = (steps + shares - 1) / shares;
-  shares = (steps + per - 1) / per;
-  const int rows = TILE_SIZES[tile].rows, columns = TILE_SIZES[tile].columns;
-  const long long blocks = (long long)((M + rows - 1) / rows) * ((N + columns - 1) / columns) * shares;
-  if (4 * blocks > (tile == TILES_64 && shares == 1 ? 5 : 4) * (long long)units) return INFINITY;
+// (a product whose `blocks` of `rows` by `columns` make `per` steps of 64 of K each)
+static float tiles_time(int rows, int columns, long long blocks, int M, int N, int per, int shares, int units) {
   const float block = 1e-3f * per * (rows + columns);
   const float sum = shares > 1 ? 1.6f + 1.9e-6f * shares * M * N : 0.f;
   return 4.f + (blocks > units ? 2.16f : 1.6f) * block + 1.6e-3f * block * blocks + sum;
@@ -2313,14 +2308,28 @@ static int choose_tiles(int M, int N, int K, int& shares) {
     const long long blocks = large * min(min(8ll, units / large), max(1ll, (long long)steps / 4));
     if (M > 128 && (M > 704 || 2 * blocks <= units || (M > 576 && 4 * blocks < 3 * units))) return TILES_NONE;
   }
-  int tile = TILES_NONE;
+  // (asked for every product of a prompt, whose host is what it waits for: no division twice, and none of 64 bits)
+  int tile = TILES_NONE, most = 1, per[9] = {0, steps};
+  while (most < 8 && steps >= 8 * (most + 1) && (long long)(most + 1) * M * N <= F32_SHARES_MOST) {
+    ++most;
+    per[most] = (steps + most - 1) / most;
+  }
   float least = INFINITY;
-  for (int t = 1; t <= TILES_MOST; ++t)
-    for (int s = 1; s <= 8 && (s == 1 || (steps / s >= 8 && (long long)s * M * N <= F32_SHARES_MOST)); ++s) {
-      const float us = tiles_time(t, M, N, K, s, units);
+  auto look = [&](int t, auto rows, auto columns) {
+    constexpr int TM = decltype(rows)::value, TN = decltype(columns)::value;
+    const long long tiles = (long long)((M + TM - 1) / TM) * ((N + TN - 1) / TN);
+    for (int s = 1; s <= most; ++s) {
+      if (4 * s * tiles > (t == TILES_64 && s == 1 ? 5 : 4) * units) break;
+      // (shares that leave none for the last have their steps, and with fewer of them, already been asked for)
+      if (s > 1 && per[s] * (s - 1) >= steps) continue;
+      const float us = tiles_time(TM, TN, s * tiles, M, N, per[s], s, units);
       if (us < least) least = us, tile = t, shares = s;
     }
-  if (tile != TILES_NONE) shares = (steps + (steps + shares - 1) / shares - 1) / ((steps + shares - 1) / shares);
+  };
+  look(TILES_64, std::integral_constant<int, 64>{}, std::integral_constant<int, 64>{});
+  look(TILES_128, std::integral_constant<int, 128>{}, std::integral_constant<int, 128>{});
+  look(TILES_64x128, std::integral_constant<int, 64>{}, std::integral_constant<int, 128>{});
+  look(TILES_96x128, std::integral_constant<int, 96>{}, std::integral_constant<int, 128>{});
   // many rows of few columns, K whole
   if (K <= 4096 && (long long)M * K > 1ll << 20 && shares == 1 && (N <= K || (N <= 3072 && 2 * large <= units))) return TILES_NONE;
   return tile;
