@@ -63,3 +63,12 @@ def test_the_rule_asks_for_what_it_uses():
                     assert 2 <= shares <= 8 and each >= 8 and 1 <= steps - (shares - 1) * each <= each
     for m, n, k in ((32, 1024, 1024), (769, 1024, 1024), (100, 1001, 1024), (100, 1024, 1000), (0, 64, 64)):
         assert room(m, n, k) == -1
+
+
+@pytest.mark.parametrize("m", [49, 52, 56, 64])
+def test_few_rows_of_a_matrix_that_widens_are_one_launch(m):
+    """No norm stands behind such a product to add its shares, and a prompt of so few rows waits for the host's launches."""
+    from transformers_neuronx_amd.kernels.hip import library
+    room = library("gemm").tnx_gemm_bf16_tiles_workspace
+    assert room(m, 6144, 2048) == 0 and room(m, 8192, 2048) == 0
+    assert room(m, 2048, 8192) > 0 and room(m, 2048, 2048) > 0

@@ -2290,10 +2290,10 @@ static int launch_tiles(const bf16_t* x, const bf16_t* w, const float* bias, con
 // 333 tokens of 1.3b 2,368 us with them and 2,363 without: one kernel fewer to fetch). Up to 32 rows half a tile would be padding, and other kernels stand ready.
 enum { TILES_NONE = 0, TILES_64 = 1, TILES_128 = 2, TILES_64x128 = 3, TILES_96x128 = 4, TILES_MOST = 4 };
 
-// (a product whose `blocks` of `rows` by `columns` make `per` steps of 64 of K each)
-static float tiles_time(int rows, int columns, long long blocks, int M, int N, int per, int shares, int units) {
+// (a product whose `blocks` of `rows` by `columns` make `per` steps of 64 of K each; `launch`: of the sum of the shares)
+static float tiles_time(int rows, int columns, long long blocks, int M, int N, int per, int shares, int units, float launch) {
   const float block = 1e-3f * per * (rows + columns);
-  const float sum = shares > 1 ? 1.6f + 1.9e-6f * shares * M * N : 0.f;
+  const float sum = shares > 1 ? launch + 1.9e-6f * shares * M * N : 0.f;
   return 4.f + (blocks > units ? 2.16f : 1.6f) * block + 1.6e-3f * block * blocks + sum;
 }
 
@@ -2314,6 +2314,9 @@ static int choose_tiles(int M, int N, int K, int& shares) {
     ++most;
     per[most] = (steps + most - 1) / most;
   }
+  // (behind a matrix that narrows stands a norm as a rule, whose launch adds the shares; behind one that widens the sum is a launch more for
+  // the host and the device: 64 rows 6,144 x 2,048 in two shares take 13.6 us alone for 14.2, and a prompt of 64 tokens of 1.3b 2,558 for 2,435)
+  const float launch = N > K ? 2.2f : 1.6f;
   float least = INFINITY;
   auto look = [&](int t, auto rows, auto columns) {
     constexpr int TM = decltype(rows)::value, TN = decltype(columns)::value;
@@ -2322,7 +2325,7 @@ static int choose_tiles(int M, int N, int K, int& shares) {
       if (4 * s * tiles > (t == TILES_64 && s == 1 ? 5 : 4) * units) break;
       // (shares that leave none for the last have their steps, and with fewer of them, already been asked for)
       if (s > 1 && per[s] * (s - 1) >= steps) continue;
-      const float us = tiles_time(TM, TN, s * tiles, M, N, per[s], s, units);
+      const float us = tiles_time(TM, TN, s * tiles, M, N, per[s], s, units, launch);
       if (us < least) least = us, tile = t, shares = s;
     }
   };
