@@ -52,7 +52,8 @@ def test_tiles(m, f, k, act, limit):
 @pytest.mark.parametrize("m,f,k,entry", [
     (16, 4096, 4096, "skinny"), (32, 4096, 2048, "skinny"), (32, 4096, 4096, None),             # 2^25 elements, 17 rows and more
     (33, 512, 256, None), (128, 2048, 512, None), (129, 2048, 512, "tiles"),                    # the rows between
-    (200, 1920, 192, None), (200, 1984, 192, "tiles"), (256, 2048, 64, "tiles"),                # a quarter of 256 units
+    (200, 1920, 192, None), (200, 1984, 192, "tiles"), (256, 2048, 64, "tiles"),                # a quarter of 256 units,
+    (300, 1408, 2048, None), (396, 1408, 2048, "tiles"), (256, 4096, 2560, None), (300, 2816, 2560, "tiles"),       # a third, a half
     (1100, 4096, 2048, "tiles"), (1100, 4096, 2112, None), (1100, 3584, 2112, "tiles")])        # more than one a unit, and K
 def test_either_side_of_the_lines(m, f, k, entry):
     """The rule as it stands, at sizes where it turns, and the general way beyond."""

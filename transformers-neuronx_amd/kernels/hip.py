@@ -2662,9 +2662,12 @@ class HipOps:
     # a launch / this, on weights that no cache holds; f gate rows of K).
     # Few rows, the kernel that streams the tile-ordered copy: up to 16 rows (8 rows, f 4,096 of 2,048 11.6 / 8.9, 8,192 of 4,096 28.1 / 25.1, 512 of
     # 2,048 6.9 / 6.4), up to 32 below 2^25 elements (32 rows, 4,096 of 2,048 15.3 / 11.5, 1,024 of 1,024 8.3 / 6.7; but 8,192 of 4,096 29.6 / 33.8).
-    # Beyond 128 rows, the experts' tiles, where these and their parts find a quarter of the units and go round them once, or K is
-    # short: f 4,096 of 2,048 200 rows 20.9 / 20.3, 396 29.1 / 22.2, 1,024 50.4 / 37.3, 2,048 79.0 / 72.3; 8,192 of 4,096 200 52.6 / 43.8, 512 70.6 / 66.7, but 640
-    # 87.3 / 100 and 2,048 237 / 252; 2,816 of 1,024 200 14.5 / 12.4, 2,048 42.4 / 33.9; 1,024 of 1,024 200 8.9 / 9.8, 396 10.4 / 9.9; 512 of 2,048 640 14.1 / 14.9.
+    # Beyond 128 rows, the experts' tiles, where these and their parts find a quarter of the units (a third with K beyond 1,024, more than half
+    # beyond 2,048: a unit pulls its tile's bytes no faster for standing alone, so few tiles take K's time) and go round them once, or K is
+    # short: f 4,096 of 2,048 200 rows 25.5 / 20.4, 396 33.1 / 24.7, 1,024 48.5 / 37.8, 2,048 83.0 / 76.2; 8,192 of 4,096 200 54.4 / 43.6, 512 74.7 / 69.2, but
+    # 2,048 237 / 252; 2,816 of 1,024 200 17.7 / 12.3, 2,048 43.0 / 34.4; 1,024 of 1,024 256 9.2 / 9.8, 396 11.0 / 9.9. By the part of the units found: K 2,048,
+    # 0.25 512 rows, f 1,024 16.8 / 20.5, 0.26 300, 1,408 16.5 / 18.2, 0.34 396, 1,408 20.7 / 17.7; K 4,096, 0.25 200, 2,048 26.2 / 33.9, 0.5 256, 4,096 36.9 / 40.6,
+    # 0.62 560, 2,048 40.2 / 33.0; K 2,560, 0.34 200, 2,816 24.9 / 28.0, 0.52 300 27.6 / 26.1.
     # Up to 128 rows the product's own kernels share K out (100 rows, 4,096 of 2,048 20.9 / 21.3, 8,192 of 4,096 40.1 / 43.6).
     gated_skinny_most, gated_skinny_elements = 32, 1 << 25
     gated_tiles_least, gated_tiles_share, gated_tiles_short = 129, 0.25, 2048
@@ -2676,7 +2679,8 @@ class HipOps:
         blocks = -(-m // 128) * -(-f // 128)
         if (m >= self.gated_tiles_least and f % 64 == 0 and k % 64 == 0 and max(m * k, m * f) < 1 << 31 and k * f < 1 << 30
                 and -(-m // 128) * (f // 64 + 1) < (1 << 31) - 1024
-                and self.gated_tiles_share * self.compute_units <= (2 * blocks if 2 * blocks <= self.compute_units else blocks)
+                and (self.gated_tiles_share * (1 if k <= 1024 else 1.33 if k <= 2048 else 2.04) * self.compute_units
+                     <= (2 * blocks if 2 * blocks <= self.compute_units else blocks))
                 and (blocks <= self.compute_units or k <= self.gated_tiles_short)):
             return "tiles"
         return None
