@@ -25,7 +25,7 @@ def test_growing_batches_meet_few_launches(head_size, staged, window):
 
 def test_answers_that_were_measured():
     """The launches that were the quickest of those measured, at 256 units."""
-    for want, *args in [((1, 2), 2048, 1, True, 32), ((8, 4), 2048, 8, True, 32), ((1, 8), 2048, 3, True, 160), ((1, 4), 2048, 2, True, 32),
+    for want, *args in [((1, 2), 2048, 1, True, 32), ((1, 4), 2048, 1, True, 32, 0, 80), ((1, 4), 2048, 1, True, 32, 0, 128), ((1, 2), 2048, 1, True, 768), ((8, 4), 2048, 8, True, 32), ((1, 8), 2048, 3, True, 160), ((1, 4), 2048, 2, True, 32),
                         ((4, 4), 2048, 8, True, 64, 0, 128), ((2, 4), 2048, 8, True, 96, 0, 128), ((1, 8), 2048, 4, True, 96),
                         ((4, 4), 2048, 8, True, 288), ((4, 2), 2048, 4, True, 288, 0, 128), ((1, 4), 2048, 8, False, 768),
                         ((1, 2), 2048, 2, False, 768), ((1, 2), 2048, 2, False, 768, 0, 80), ((1, 4), 2048, 6, False, 768, 0, 128),

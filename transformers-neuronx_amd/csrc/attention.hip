@@ -1765,7 +1765,7 @@ extern "C" int tnx_attention_prefill_scored(const void* q, const void* k_pages, 
 // requests of 512 tokens and 32 heads of 80: 28.0 us, 32.6 with the mark; in whole runs 28.0 and 25.3 with it, 6.6 TB/s). Straight into
 // registers / staged, us: 32 heads of 80, 32 requests of up to 720 tokens 37.0 / 31.5, 24 of 400 25.6 / 20.1, 8 of 1,500 26.2 / 22.7; of 64,
 // 24 of 112 to 412 18.9 / 15.3, 40 of 145 to 520 27.1 / 22.4; of 128, 8 of 2,050 53.8 / 46.6, 40 of 1,500 169 / 151. Where a wave has
-// one tile at most the way through LDS costs 0.2 us (3 of 100, heads of 64: 5.2 / 5.4). How many waves a block has: `HipOps._splits_for`.
+// one tile at most the way through LDS costs 0.1 to 0.6 us (3 of 60, heads of 64 4.7 / 4.8; 24 of 60, 32 on 8 of 128 6.2 / 6.7), 0.3 less from 100 keys on. How many waves a block has: `HipOps._splits_for`.
 // PACK: for query heads that share their keys and values (fewer kv heads than heads). A block then takes one
 // kv head of one request, and the 16 columns hold up to 16 (8 at the largest head size) different query heads
 // of its group, so the keys and values are read once for all of them and not once a head; the maxima, sums and

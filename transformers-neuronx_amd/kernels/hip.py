@@ -1637,8 +1637,10 @@ class HipOps:
         - the pairs leave half of the units idle, or two thirds up to heads of 80, and the keys are many: as many blocks as units share
           them (1 request of 2,000 20.5 whole / 10.6 in eight, 2 of 128 21 / 17.1 in four, 3 of 128 26.4 / 22.3 in two; but 1 of 700
           8.5 / 9.4, and 3 of 1,000 11.2 / 12.0 in two, since the kernel that merges costs 2);
-        - at most one block a unit: as many waves as 256 keys, twice and four times as many keep at a tile or two each (1 of 100 5.0 with two,
-          5.2 with four, 5.4 with eight; 500 9.0, 7.9, 8.1; 5 of 700 12.2, 10.6, 10.0); four where nearly all units have a block, and where
+        - at most one block a unit: four waves up to 512 keys, which have a tile or two each, and eight beyond where heads of up to 80 let
+          them find room (500 keys 9.0 with two, 7.9 with four, 8.1 with eight; 5 of 700 12.2, 10.6, 10.0). Up to 256 keys heads of up to 64
+          have two: a wave has one tile either way below 129 (1 of 60 4.4 with two, 4.5 with four; 128 4.1, 4.2; but 180 5.65, 4.8); wider
+          ones lose more by it beyond than they gain (80, 60 4.8, 4.95; 180 6.4, 5.35). Four where nearly all units have a block, and where
           the lengths are unlike until the keys are shared or, where they are not, heads of up to 80 have more than 512 keys;
         - more pairs than units, not a whole number on each, of requests about as long as one another: shares of the keys come out
           more even (9 of 2,000 37.6 / 34.2 in four, of 128 900 32.9 / 30.3 with two waves; but 33 of 900 53.9 / 60.4). Requests of
@@ -1675,7 +1677,7 @@ class HipOps:
         if pairs <= units:
             if not alike:
                 return 1, 8 if staged and not wide and shares <= 2 and fills > 2 and 10 * pairs < 7 * units else 4
-            return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or (wide and fills > 2) else two if fills <= 1 else 8
+            return 1, 4 if 10 * pairs >= 7 * units or fills == 2 or wide else 8 if fills > 1 else two if head_size <= 64 else 4
         if alike and fills >= (4 if wide else 8) and -(-pairs // units) * units > 1.05 * pairs:
             return 4, two if wide else 4
         if not wide and pairs <= 2 * units:
