@@ -1640,7 +1640,7 @@ class HipOps:
         - at most one block a unit: four waves up to 512 keys, which have a tile or two each, and eight beyond where heads of up to 80 let
           them find room (500 keys 9.0 with two, 7.9 with four, 8.1 with eight; 5 of 700 12.2, 10.6, 10.0). Up to 256 keys heads of up to 64
           have two: a wave has one tile either way below 129 (1 of 60 4.4 with two, 4.5 with four; 128 4.1, 4.2; but 180 5.65, 4.8); wider
-          ones lose more by it beyond than they gain (80, 60 4.8, 4.95; 180 6.4, 5.35). Four where nearly all units have a block, and where
+          ones lose more by it beyond than they gain (80, 60 5.2, 5.4; 200 6.9, 6.4; 256 6.1, 5.7). Four where nearly all units have a block, and where
           the lengths are unlike until the keys are shared or, where they are not, heads of up to 80 have more than 512 keys;
         - more pairs than units, not a whole number on each, of requests about as long as one another: shares of the keys come out
           more even (9 of 2,000 37.6 / 34.2 in four, of 128 900 32.9 / 30.3 with two waves; but 33 of 900 53.9 / 60.4). Requests of
